@@ -1,11 +1,14 @@
-"""ctypes binding of libcastle_hip.so (C ABI in include/castle_hip.h).
+"""Bindings of the native code: libcastle_hip.so (C ABI in include/castle_hip.h, through ctypes) and
+_castle_host.so (csrc/castle_host.cpp: the registered operators and the host path of a layer).
 
-The library is looked up next to this file only.  Nothing here falls back to another
-implementation: if the library is missing or a call fails, a RuntimeError is raised.
+Both are looked up next to this file only.  Nothing here falls back to another
+implementation: if one is missing or a call fails, a RuntimeError is raised.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -13,6 +16,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libcastle_hip.so")
+HOST_PATH = os.path.join(_HERE, "_castle_host.so")
 
 ABI_VERSION = 5
 DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
@@ -71,6 +75,7 @@ DECODE_DEFER = 4   # U is written on every 4th step when a castle_deferred is ha
 _VP = ctypes.POINTER(View4)
 _DP = ctypes.POINTER(Deferred)
 _lib = None
+_host = None
 _lock = threading.Lock()
 
 
@@ -132,8 +137,27 @@ def lib():
     return _lib
 
 
+def host():
+    """The extension module built from csrc/castle_host.cpp; loading it registers torch.ops.castle_hip.*"""
+    global _host
+    if _host is None:
+        lib()
+        with _lock:
+            if _host is None:
+                if not os.path.exists(HOST_PATH):
+                    raise RuntimeError(f"{HOST_PATH} not found: build it first (python -m lookahead_keys_attention_amd.build)")
+                name = __package__ + "._castle_host"
+                spec = importlib.util.spec_from_file_location(name, HOST_PATH, loader=importlib.machinery.ExtensionFileLoader(name, HOST_PATH))
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                from . import ops
+                ops._register_fakes()
+                _host = module
+    return _host
+
+
 def is_built() -> bool:
-    return os.path.exists(LIB_PATH)
+    return os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH)
 
 
 def check(code: int, what: str):

@@ -1,15 +1,16 @@
-"""Builds libcastle_hip.so (HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Builds the native code in-tree.
 
     python -m lookahead_keys_attention_amd.build
 
-No torch headers are involved: the library is plain HIP behind the C ABI declared in
-include/castle_hip.h and is loaded with ctypes.
+libcastle_hip.so   HIP kernels + C ABI for gfx950, with hipcc: plain HIP behind include/castle_hip.h, no torch headers
+_castle_host.so    csrc/castle_host.cpp, with g++ against the torch headers: operators and host path over that ABI
 """
 from __future__ import annotations
 
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -17,6 +18,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libcastle_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 SOURCES = ("castle_fwd.hip", "castle_bwd.hip", "castle_decode.hip", "castle_profile.hip", "castle_abi.hip")
+HOST_SOURCE = "castle_host.cpp"
+HOST_NAME = "_castle_host.so"
 ARCH = "gfx950"
 # packed fp32 VALU instructions stay disabled on purpose (hipcc's host pass warns that it
 # does not know the feature; that warning is harmless)
@@ -34,6 +37,15 @@ def _hipcc() -> str:
     return "hipcc"
 
 
+def _host_compiler():
+    import torch
+
+    include = os.path.join(os.path.dirname(torch.__file__), "include")
+    return ["g++", "-std=c++17", "-O2", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-I" + include,
+            "-I" + os.path.join(include, "torch", "csrc", "api", "include"), "-isystem", "/opt/rocm/include",
+            "-I" + sysconfig.get_paths()["include"]]
+
+
 def _run(cmd):
     proc = subprocess.run(cmd, capture_output=True, text=True)
     noise = "'-packed-fp32-ops' is not a recognized feature"
@@ -44,23 +56,32 @@ def _run(cmd):
 
 
 def build(verbose: bool = False, jobs: int | None = None) -> str:
-    """Compile every HIP source and link the shared library; returns its path."""
+    """Compile every source and link the two shared libraries; returns the path of the kernel library."""
     hipcc = _hipcc()
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
-    jobs = jobs or min(len(SOURCES), os.cpu_count() or 1, 8)
+    jobs = jobs or min(len(SOURCES) + 1, os.cpu_count() or 1, 8)
 
     def compile_one(src):
-        obj = os.path.join(objdir, src.replace(".hip", ".o"))
-        cmd = [hipcc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+        obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
+        cmd = _host_compiler() if src == HOST_SOURCE else [hipcc, *HIPCC_FLAGS]
+        cmd = [*cmd, "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         _run(cmd)
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        objs = list(pool.map(compile_one, SOURCES))
+        host_obj, *objs = pool.map(compile_one, (HOST_SOURCE, *SOURCES))
     link = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-fno-gpu-rdc", "-o", LIB_PATH, *objs]
+    if verbose:
+        print(" ".join(link), flush=True)
+    _run(link)
+    import torch
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    link = ["g++", "-shared", "-o", os.path.join(HERE, HOST_NAME), host_obj, "-L" + HERE, "-lcastle_hip", "-L" + torch_lib,
+            "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
     if verbose:
         print(" ".join(link), flush=True)
     _run(link)

@@ -34,10 +34,12 @@ import warnings
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import ops
 from . import _native
 
+_TENSOR_TYPES = (torch.Tensor, nn.Parameter)
 _CacheFields = namedtuple("Cache", ("U", "qu_cache", "kc_cache", "vc_cache"))
 
 
@@ -53,18 +55,44 @@ class Cache(_CacheFields):
 
     _store = None   # set on caches that live in a native capacity buffer
 
+    @classmethod
+    def _of_store(cls, store, n):
+        """The cache over the first n rows of a native store.  The views are only made when somebody
+        reads them: a decode loop hands the cache from step to step without ever looking inside."""
+        cache = tuple.__new__(cls, _NO_FIELDS)
+        cache._store, cache._n = store, n
+        return cache
+
     def _read(self):
-        raw = tuple.__getitem__(self, slice(None))
-        if self._store is None:
-            return raw
-        self._store.flush()
-        if self._store.u_half:
+        store = self._store
+        if store is None:
+            return tuple.__getitem__(self, slice(None))
+        store.flush()
+        raw = tuple(buf[:, :, : self._n] for buf in store.buffers)
+        if store.u_half:
             return (ops.decode_lookahead_keys(raw[0]),) + raw[1:]
         return raw
+
+    def _field(self, index):
+        if self._store is None:
+            return tuple.__getitem__(self, index)
+        return self._store.buffers[index][:, :, : self._n]
 
     @property
     def U(self):
         return self._read()[0]
+
+    @property
+    def qu_cache(self):
+        return self._field(1)
+
+    @property
+    def kc_cache(self):
+        return self._field(2)
+
+    @property
+    def vc_cache(self):
+        return self._field(3)
 
     def __getitem__(self, index):
         return self._read()[index]
@@ -72,14 +100,25 @@ class Cache(_CacheFields):
     def __iter__(self):
         return iter(self._read())
 
+    def __repr__(self):
+        return "Cache(U={!r}, qu_cache={!r}, kc_cache={!r}, vc_cache={!r})".format(*self._read())
+
+    def __reduce__(self):
+        return Cache, tuple(self._read())
+
+
+_NO_FIELDS = (None,) * 4
+
 
 class _CacheStore:
     """Capacity buffers behind a native cache: four (B, H, capacity, d) tensors and a row count."""
 
-    def __init__(self, B, H, d, capacity, dtype, device, U_buffer=None):
-        # U_buffer: an existing (B, H, capacity, d) tensor to adopt as the lookahead-key buffer
-        first = U_buffer if U_buffer is not None else torch.empty((B, H, capacity, d), dtype=dtype, device=device)
-        self.buffers = (first,) + tuple(torch.empty((B, H, capacity, d), dtype=dtype, device=device) for _ in range(3))
+    def __init__(self, B, H, d, capacity, dtype, device, U_buffer=None, buffers=None):
+        # U_buffer: an existing (B, H, capacity, d) tensor to adopt as the lookahead-key buffer; buffers: all four
+        if buffers is None:
+            first = U_buffer if U_buffer is not None else torch.empty((B, H, capacity, d), dtype=dtype, device=device)
+            buffers = (first,) + tuple(torch.empty((B, H, capacity, d), dtype=dtype, device=device) for _ in range(3))
+        self.buffers = tuple(buffers)
         self.capacity = capacity
         self.length = 0
         # deferred write-back of the lookahead keys: pending (ku, vu) rows, and the row count up to
@@ -93,6 +132,25 @@ class _CacheStore:
         self._geometry = (B, H, d, device)
         self._workspace = None
         self._views = None
+        self._plan = None
+
+    @property
+    def plan(self):
+        """What the native host code needs to run steps on these buffers, built once."""
+        if self._plan is None:
+            self._plan = _native.host().StepPlan(list(self.buffers), *self.rings, self.workspace, self.u_half)
+        return self._plan
+
+    def step_base(self):
+        """Row count the deferred write-back of a step starts from, -1 for a step that writes U itself."""
+        return self.base0 if ops.DEFER_LOOKAHEAD_WRITES or self.pending() > 0 else -1
+
+    def advanced(self, base):
+        """Bookkeeping behind a step taken with `base`; returns the cache of the new row count."""
+        self.length += 1
+        if base < 0:
+            self.base0 = self.length   # the step wrote the lookahead keys itself: nothing is pending
+        return Cache._of_store(self, self.length)
 
     @property
     def workspace(self):
@@ -129,10 +187,7 @@ class _CacheStore:
         self.base0 = self.length
 
     def as_cache(self) -> Cache:
-        n = self.length
-        cache = Cache(*(buf[:, :, :n] for buf in self.buffers))
-        cache._store = self
-        return cache
+        return Cache._of_store(self, self.length)
 
     def grown(self, min_capacity):
         B, H, _, d = self.buffers[0].shape
@@ -303,6 +358,19 @@ class Castle(nn.Module):
                               "inference-only); its native cache is copied out and every later step stays dense. "
                               "Decode under torch.no_grad() to keep the HIP kernels", RuntimeWarning, stacklevel=2)
             native = False
+        if native and self._plain(x):
+            if single:
+                store = self._store_for(cache, x)
+                base = store.step_base()
+                norm = self._modules["norm"]
+                y = store.plan.layer(x, norm._parameters.get("weight"), getattr(norm, "eps", None),
+                                     self._modules["to_all_qkv"]._parameters["weight"],
+                                     self._modules["combine_heads"]._parameters["weight"],
+                                     ops.SMALL_LINEAR_MAX_ROWS, store.length, base, self.scale, self.use_rotary)
+                cache = store.advanced(base)
+                return (y, cache) if return_next_cache else y
+            assert cache is None, "must be inferencing single tokens if receiving cache"
+            return self._layer_native(x, return_next_cache)
         native_step = single and native
         proj = self._project(self.to_all_qkv, x, native_step, norm=self.norm)
         if not single:
@@ -312,6 +380,46 @@ class Castle(nn.Module):
             merged, next_cache = (self._step_native if native else self._step_dense)(proj, cache)
         y = self._project(self.combine_heads, merged, native_step)
         return (y, next_cache) if return_next_cache else y
+
+    def _plain(self, x):
+        """True if the whole layer may run as one native call: unmodified projections and norm, nothing
+        hooked onto them, nothing that wants to see the operators one by one."""
+        if torch.compiler.is_compiling() or type(x) not in _TENSOR_TYPES or x.dim() != 3 or _has_any_global_hook():
+            return False
+        if ops.CHECK_RANGE or torch.is_autocast_enabled("cuda") or torch._C._are_functorch_transforms_active():
+            return False
+        if torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
+            return False
+        norm, qkv, combine = (self._modules[name] for name in ("norm", "to_all_qkv", "combine_heads"))
+        for layer in ((qkv, combine) if type(norm) is nn.Identity else (qkv, combine, norm)):
+            weight = layer._parameters.get("weight")
+            if (type(weight) is not nn.Parameter or weight.dtype != x.dtype or weight.device != x.device
+                    or layer._parameters.get("bias") is not None
+                    or layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks):
+                return False
+        return (type(qkv) is nn.Linear and type(combine) is nn.Linear and qkv.in_features == x.shape[2]
+                and type(norm) in (nn.Identity, nn.RMSNorm) and not norm._forward_hooks and not norm._forward_pre_hooks
+                and (type(norm) is nn.Identity or norm.normalized_shape == (x.shape[2],)))
+
+    def _layer_native(self, x, want_cache):
+        """The parallel pass as one native call (csrc/castle_host.cpp): norm, projection, attention core,
+        output projection and, with a cache, the rows of its buffers."""
+        B, n, _ = x.shape
+        H, d = self.heads, self.dim_head
+        norm = self._modules["norm"]
+        u_half = want_cache and x.dtype == torch.bfloat16 and ops.LOOKAHEAD_KEYS_HALF
+        flags = (ops.DEFAULT_FLAGS | (_native.FLAG_ROTARY if self.use_rotary else 0) | (_native.FLAG_U_HALF if u_half else 0))
+        y, *buffers = _native.host().layer_parallel(
+            x, norm._parameters.get("weight"), getattr(norm, "eps", None), self._modules["to_all_qkv"]._parameters["weight"],
+            self._modules["combine_heads"]._parameters["weight"], H, self.scale, flags,
+            ops.keeps_state(B, H, n, d, x.dtype), _reserve_rows(n) if want_cache else 0)
+        if not want_cache:
+            return y
+        store = _CacheStore(B, H, d, _reserve_rows(n), x.dtype, x.device, buffers=buffers)
+        store.u_half = u_half
+        store.length = store.base0 = n
+        store.scale = self.scale
+        return y, store.as_cache()
 
     @staticmethod
     def _project(layer, t, native_step, norm=None, activation=None, residual=None):
@@ -353,36 +461,28 @@ class Castle(nn.Module):
         store.scale = self.scale
         return merged, store.as_cache()
 
-    def _step_native(self, proj, cache):
-        B = proj.shape[0]
+    def _store_for(self, cache, like):
+        """The capacity buffers a single-token step on `cache` works on (like: a (B, 1, ..) tensor of the step)."""
         H, d = self.heads, self.dim_head
-        qu, ku, vu, qc, kc, vc = self._split(proj)
         store = getattr(cache, "_store", None) if cache is not None else None
         if cache is None:
-            store = _CacheStore(B, H, d, _reserve_rows(1), proj.dtype, proj.device)
+            store = _CacheStore(like.shape[0], H, d, _reserve_rows(1), like.dtype, like.device)
         elif store is None:
-            store = _CacheStore(B, H, d, _reserve_rows(cache[0].shape[-2] + 1), proj.dtype, proj.device)
+            store = _CacheStore(like.shape[0], H, d, _reserve_rows(cache[0].shape[-2] + 1), like.dtype, like.device)
             store.adopt(cache)
-        elif store.length != cache.kc_cache.shape[-2]:   # (not cache.U: reading it would write the pending keys back)
+        elif store.length != cache._n:
             raise RuntimeError("this cache was already advanced by a later decode step; the native "
                                "decode updates its cache in place, so a cache can be used once")
         store.scale = self.scale
-        t = store.length
-        if t + 1 > store.capacity:
-            store = store.grown(_reserve_rows(t + 1))
-        out = torch.empty((B, 1, H, d), dtype=proj.dtype, device=proj.device)
-        deferred = store.deferred()
-        if proj.is_contiguous() and proj.data_ptr() % 16 == 0:
-            ops.castle_decode_step_packed(store.views, store.capacity, t, proj, H, self.scale, out, store.workspace,
-                                          rotary=self.use_rotary, deferred=deferred, u_half=store.u_half)
-        else:
-            ops.castle_decode_step_hip(*store.buffers, t, qc, kc, vc, qu, ku, vu, self.scale,
-                                       out.permute(0, 2, 1, 3), store.workspace, rotary=self.use_rotary,
-                                       deferred=deferred, u_half=store.u_half)
-        if deferred is None:
-            store.base0 = t + 1   # this step wrote the lookahead keys itself: nothing is pending
-        store.length = t + 1
-        return out.view(B, 1, H * d), store.as_cache()
+        if store.length + 1 > store.capacity:
+            store = store.grown(_reserve_rows(store.length + 1))
+        return store
+
+    def _step_native(self, proj, cache):
+        store = self._store_for(cache, proj)
+        base = store.step_base()
+        out = store.plan.attend(proj, store.length, base, self.scale, self.use_rotary)
+        return out, store.advanced(base)
 
     def graph_step(self, x, store, t_device, base_device=None, residual=None):
         """The cached single-token step in the form a captured HIP graph needs: the same GPU work

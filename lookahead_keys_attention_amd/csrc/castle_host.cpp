@@ -1,0 +1,497 @@
+// Host layer between PyTorch and the C ABI of libcastle_hip.so: the registered operators
+// (torch.ops.castle_hip.*) with their autograd formulas, and the cached single-token step of a layer.
+//
+// This code is what stands between a call and its kernels, so it decides the time of every call whose
+// kernels take less than about a third of a millisecond.  The same operators written in Python
+// (torch.library.custom_op, autograd formulas, ctypes views) took 70 us of host time for a forward and
+// 150 us more for a backward pass, a cached step 71 us; here an operator costs its allocations and launches.
+#include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/utils/pybind.h>
+#include <torch/library.h>
+
+#include <optional>
+#include <tuple>
+#include <vector>
+
+#include "../../include/castle_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+int dtype_code(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kFloat: return CASTLE_F32;
+    case at::kBFloat16: return CASTLE_BF16;
+    case at::kHalf: return CASTLE_F16;
+    default: TORCH_CHECK_TYPE(false, "castle HIP kernels support float32, bfloat16 and float16, not ", t.scalar_type());
+  }
+}
+
+int64_t check(int64_t code, const char* what) {
+  TORCH_CHECK(code >= 0, what, " failed: ", castle_error_string((int)code), " (code ", code, ")");
+  return code;
+}
+
+void check_dims(int64_t d, const Tensor& t) {
+  TORCH_CHECK_VALUE(d == 16 || d == 32 || d == 64 || d == 128,
+                    "dim_head must be one of (16, 32, 64, 128) for the HIP kernels, got ", d);
+  TORCH_CHECK_VALUE(t.scalar_type() != at::kFloat || d <= 64, "float32 HIP kernels support dim_head <= 64");
+}
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+castle_view4 view4(const Tensor& t) { return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)}; }
+
+// the kernels read 16 bytes at a time along d; anything else is copied
+Tensor readable(const Tensor& t) {
+  const int64_t q = 16 / t.element_size();
+  if (t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 && t.stride(0) % q == 0 && t.stride(1) % q == 0 &&
+      t.stride(2) % q == 0)
+    return t;
+  return t.contiguous();
+}
+Tensor packed_readable(const Tensor& t) {
+  return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.contiguous();
+}
+
+Tensor bytes(int64_t n, const Tensor& like) { return at::empty({n}, like.options().dtype(at::kByte)); }
+
+struct Shape {
+  int B, H, L, d, dtype;
+};
+
+// part `i` of six of a packed (B, L, 6 H d) tensor, or the merged (B, L, H d) one (parts = 1), as a (B, H, L, d) view
+castle_view4 packed_view(const Tensor& t, const Shape& s, int parts, int i) {
+  const int64_t width = (int64_t)parts * s.H * s.d;
+  return {static_cast<char*>(t.data_ptr()) + (int64_t)i * s.H * s.d * t.element_size(), s.L * width, s.d, width};
+}
+
+// six: qc, kc, vc, qu, ku, vu.  Returns what the backward pass needs back: (workspace, state), the state
+// empty when it is not kept.
+std::tuple<Tensor, Tensor> run_fwd(const castle_view4 (&six)[6], const Shape& s, double scale, int64_t flags, const castle_view4& out,
+                                   const castle_view4& U, bool keep_state, const Tensor& like) {
+  const int64_t nbytes = check(castle_fwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_workspace_bytes");
+  const int64_t sbytes = check(castle_fwd_state_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_state_bytes");
+  Tensor ws = bytes(nbytes, like), state = bytes(sbytes, like);
+  check(castle_fwd(&six[0], &six[1], &six[2], &six[3], &six[4], &six[5], s.B, s.H, s.L, s.d, s.dtype, (float)scale, (int)flags, &out,
+                   &U, ws.data_ptr(), nbytes, state.data_ptr(), sbytes, stream_of(like)),
+        "castle_fwd");
+  if (!keep_state) state = bytes(0, like);   // the caching allocator keeps the block until the stream is done with it
+  return {ws, state};
+}
+
+// grads: dqc, dkc, dvc, dqu, dku, dvu.  The backward kernels take the operands from the copies in the forward workspace.
+void run_bwd(const castle_view4 (&six)[6], const castle_view4& out, const castle_view4& dout, const Shape& s, double scale, int64_t flags,
+             const castle_view4 (&grads)[6], const Tensor& ws, const Tensor& state) {
+  int fl = (int)flags & ~CASTLE_FLAG_U_HALF;   // describes the forward's U output only
+  if (state.numel() == 0) fl |= CASTLE_FLAG_RECOMPUTE_STATE;
+  const int64_t nbytes = check(castle_bwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype, fl), "castle_bwd_workspace_bytes");
+  Tensor bws = bytes(nbytes, ws);
+  check(castle_bwd(&six[0], &six[1], &six[2], &six[3], &six[4], &six[5], &out, &dout, s.B, s.H, s.L, s.d, s.dtype, (float)scale, fl,
+                   &grads[0], &grads[1], &grads[2], &grads[3], &grads[4], &grads[5], ws.data_ptr(), ws.numel(),
+                   state.numel() ? state.data_ptr() : nullptr, state.numel(), bws.data_ptr(), nbytes, stream_of(ws)),
+        "castle_bwd");
+}
+
+void require_gpu(const Tensor& t, const char* what) {
+  TORCH_CHECK(t.is_cuda(), what, ": the HIP kernels need tensors on the GPU (got ", t.device(), ")");
+}
+
+// ---- the operator on six (B, H, L, d) tensors ------------------------------------------------------------------
+Shape shape_of(const Tensor& q) { return {(int)q.size(0), (int)q.size(1), (int)q.size(2), (int)q.size(3), dtype_code(q)}; }
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu, const Tensor& ku,
+                                                     const Tensor& vu, double scale, bool want_U, int64_t flags, bool keep_state) {
+  require_gpu(q, "castle_attention_hip");
+  check_dims(q.size(3), q);
+  const Shape s = shape_of(q);
+  const c10::DeviceGuard guard(q.device());
+  const Tensor ops[6] = {readable(q), readable(k), readable(v), readable(qu), readable(ku), readable(vu)};
+  castle_view4 six[6];
+  for (int i = 0; i < 6; ++i) six[i] = view4(ops[i]);
+  const int64_t B = s.B, H = s.H, L = s.L, d = s.d;
+  Tensor out = at::empty({B, L, H, d}, q.options()).permute({0, 2, 1, 3});
+  Tensor U = want_U ? at::empty({B, H, L, d}, q.options()) : at::empty({0}, q.options());
+  auto [ws, state] = run_fwd(six, s, scale, flags, view4(out), want_U ? view4(U) : castle_view4{nullptr, 0, 0, 0}, keep_state, q);
+  return {out, U, ws, state};
+}
+
+Tensor attention_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu, const Tensor& ku, const Tensor& vu,
+                     const Tensor& out, const Tensor& dout, const Tensor& ws, const Tensor& state, double scale, int64_t flags) {
+  const Shape s = shape_of(q);
+  const c10::DeviceGuard guard(q.device());
+  const Tensor ops[8] = {readable(q), readable(k), readable(v), readable(qu), readable(ku), readable(vu), readable(out), readable(dout)};
+  castle_view4 six[6], grads[6];
+  for (int i = 0; i < 6; ++i) six[i] = view4(ops[i]);
+  const int64_t B = s.B, H = s.H, L = s.L, d = s.d;
+  Tensor packed = at::empty({6, B, H, L, d}, out.options());
+  for (int i = 0; i < 6; ++i)
+    grads[i] = {static_cast<char*>(packed.data_ptr()) + i * B * H * L * d * packed.element_size(), H * L * d, L * d, d};
+  run_bwd(six, view4(ops[6]), view4(ops[7]), s, scale, flags, grads, ws, state);
+  return packed;
+}
+
+// ---- the operator on the fused projection (B, L, 6 H d), order qu, ku, vu, qc, kc, vc --------------------------
+Shape packed_shape(const Tensor& proj, int64_t heads) {
+  return {(int)proj.size(0), (int)heads, (int)proj.size(1), (int)(proj.size(2) / (6 * heads)), dtype_code(proj)};
+}
+void six_of_packed(const Tensor& p, const Shape& s, castle_view4 (&six)[6]) {
+  for (int i = 0; i < 3; ++i) {
+    six[i] = packed_view(p, s, 6, 3 + i);
+    six[3 + i] = packed_view(p, s, 6, i);
+  }
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> attention_packed(const Tensor& proj, int64_t heads, double scale, bool want_U,
+                                                            int64_t row_capacity, int64_t flags, bool keep_state) {
+  // The lookahead keys come back as the first L rows of a (B, H, row_capacity, d) buffer, so that a
+  // caller can hand over the U buffer of a decode cache without copying (row_capacity >= L).
+  require_gpu(proj, "castle_attention_packed");
+  const Shape s = packed_shape(proj, heads);
+  check_dims(s.d, proj);
+  const c10::DeviceGuard guard(proj.device());
+  const Tensor p = packed_readable(proj);
+  castle_view4 six[6];
+  six_of_packed(p, s, six);
+  const int64_t B = s.B, H = s.H, L = s.L, d = s.d, cap = std::max(row_capacity, L);
+  Tensor merged = at::empty({B, L, H * d}, proj.options());
+  Tensor U = want_U ? at::empty({B, H, cap, d}, proj.options()) : at::empty({0}, proj.options());
+  auto [ws, state] = run_fwd(six, s, scale, flags, packed_view(merged, s, 1, 0),
+                             want_U ? view4(U) : castle_view4{nullptr, 0, 0, 0}, keep_state, proj);
+  return {merged, U, ws, state};
+}
+
+Tensor attention_packed_bwd(const Tensor& proj, const Tensor& merged, const Tensor& dmerged, const Tensor& ws, const Tensor& state,
+                            int64_t heads, double scale, int64_t flags) {
+  const Shape s = packed_shape(proj, heads);
+  const c10::DeviceGuard guard(proj.device());
+  const Tensor p = packed_readable(proj), dm = packed_readable(dmerged);
+  Tensor dproj = at::empty(proj.sizes(), proj.options());
+  castle_view4 six[6], grads[6];
+  six_of_packed(p, s, six);
+  six_of_packed(dproj, s, grads);
+  run_bwd(six, packed_view(merged, s, 1, 0), packed_view(dm, s, 1, 0), s, scale, flags, grads, ws, state);
+  return dproj;
+}
+
+// ---- autograd ----------------------------------------------------------------------------------------------------
+// U, the workspace and the state carry no gradient (lookahead_keys_attention_triton.py:513-515 for U), and
+// autograd does not materialise zeros for them (a fill of hundreds of MB per backward pass).  The formulas call
+// the backward operators through the dispatcher, so that they trace like any other operator.
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+bool wants_graph(std::initializer_list<Tensor> ts) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor& t : ts)
+    if (t.defined() && t.requires_grad()) return true;
+  return false;
+}
+
+template <typename F> auto op_handle(const char* name) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
+}
+
+struct AttentionFn : torch::autograd::Function<AttentionFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu,
+                               const Tensor& ku, const Tensor& vu, double scale, bool want_U, int64_t flags, bool keep_state) {
+    static const auto op = op_handle<decltype(attention)>("castle_hip::attention");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    auto [out, U, ws, state] = op.call(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state);
+    ctx->save_for_backward({q, k, v, qu, ku, vu, out, ws, state});
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["flags"] = flags;
+    ctx->mark_non_differentiable({U, ws, state});
+    ctx->set_materialize_grads(false);
+    return {out, U, ws, state};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    static const auto op = op_handle<decltype(attention_bwd)>("castle_hip::attention_bwd");
+    const auto s = ctx->get_saved_variables();
+    const Tensor dout = g[0].defined() ? g[0] : at::zeros_like(s[6]);
+    const auto d = op.call(s[0], s[1], s[2], s[3], s[4], s[5], s[6], dout, s[7], s[8], ctx->saved_data["scale"].toDouble(),
+                           ctx->saved_data["flags"].toInt()).unbind(0);
+    return {d[0], d[1], d[2], d[3], d[4], d[5], Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> attention_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu,
+                                                              const Tensor& ku, const Tensor& vu, double scale, bool want_U,
+                                                              int64_t flags, bool keep_state) {
+  if (!wants_graph({q, k, v, qu, ku, vu})) {
+    static const auto op = op_handle<decltype(attention)>("castle_hip::attention");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state);
+  }
+  auto r = AttentionFn::apply(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state);
+  return {r[0], r[1], r[2], r[3]};
+}
+
+struct AttentionPackedFn : torch::autograd::Function<AttentionPackedFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& proj, int64_t heads, double scale, bool want_U, int64_t row_capacity,
+                               int64_t flags, bool keep_state) {
+    static const auto op = op_handle<decltype(attention_packed)>("castle_hip::attention_packed");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    auto [merged, U, ws, state] = op.call(proj, heads, scale, want_U, row_capacity, flags, keep_state);
+    ctx->save_for_backward({proj, merged, ws, state});
+    ctx->saved_data["heads"] = heads;
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["flags"] = flags;
+    ctx->mark_non_differentiable({U, ws, state});
+    ctx->set_materialize_grads(false);
+    return {merged, U, ws, state};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    static const auto op = op_handle<decltype(attention_packed_bwd)>("castle_hip::attention_packed_bwd");
+    const auto s = ctx->get_saved_variables();
+    const Tensor dm = g[0].defined() ? g[0] : at::zeros_like(s[1]);
+    Tensor dproj = op.call(s[0], s[1], dm, s[2], s[3], ctx->saved_data["heads"].toInt(), ctx->saved_data["scale"].toDouble(),
+                           ctx->saved_data["flags"].toInt());
+    return {dproj, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> attention_packed_autograd(const Tensor& proj, int64_t heads, double scale, bool want_U,
+                                                                     int64_t row_capacity, int64_t flags, bool keep_state) {
+  if (!wants_graph({proj})) {
+    static const auto op = op_handle<decltype(attention_packed)>("castle_hip::attention_packed");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(proj, heads, scale, want_U, row_capacity, flags, keep_state);
+  }
+  auto r = AttentionPackedFn::apply(proj, heads, scale, want_U, row_capacity, flags, keep_state);
+  return {r[0], r[1], r[2], r[3]};
+}
+
+// ---- projections -----------------------------------------------------------------------------------------------
+// The weight gradient of a projection over many rows, dW = dY^T x, is a product with a small output
+// (out_features x in_features) and a long contraction (the rows): the GEMM the library picks leaves most of
+// the GPU idle there.  From kSplitWgradMinRows rows on it is formed as kSplitRowsInto partial products over row
+// ranges (one batched GEMM with fp32 partial results, then their sum): same rounding, 2-3 times faster at 16384 rows.
+constexpr int64_t kSplitWgradMinRows = 8192, kSplitRowsInto = 8;
+
+Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (N, K)
+  const int64_t rows = x.size(0);
+  if (x.scalar_type() != at::kFloat && rows >= kSplitWgradMinRows && rows % kSplitRowsInto == 0) {
+    const int64_t r = rows / kSplitRowsInto;
+    const Tensor a = dy.contiguous().view({kSplitRowsInto, r, dy.size(1)}).transpose(1, 2);
+    return at::bmm(a, x.contiguous().view({kSplitRowsInto, r, x.size(1)}), at::kFloat).sum(0).to(x.scalar_type());
+  }
+  return at::mm(dy.t(), x);
+}
+
+// ---- a whole layer over sequences ------------------------------------------------------------------------------
+// [RMS norm] -> fused projection -> attention core -> output projection, and its backward pass, as one
+// autograd node: the modules one by one cost more host time than the kernels of a short sequence take.
+struct LayerFn : torch::autograd::Function<LayerFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const std::optional<Tensor>& norm_w_, const Tensor& w_qkv,
+                               const Tensor& w_out, std::optional<double> eps, int64_t heads, double scale, int64_t flags, bool want_graph, bool keep_state,
+                               int64_t cache_rows) {
+    const at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor norm_w = norm_w_.value_or(Tensor());
+    const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
+    const Tensor x2 = x.reshape({B * L, dim});
+    Tensor h = x2, rstd;
+    if (norm_w.defined()) std::tie(h, rstd) = at::_fused_rms_norm(x2, {dim}, norm_w, eps);
+    const Tensor proj = at::mm(h, w_qkv.t()).view({B, L, w_qkv.size(0)});
+    const bool want_U = cache_rows > 0;
+    auto [merged, U, ws, state] = attention_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state);
+    Tensor y = at::mm(merged.view({B * L, merged.size(2)}), w_out.t()).view({B, L, w_out.size(0)});
+    variable_list out{y};
+    if (want_U) {   // the rows of the decode cache, behind U in the order of its fields: qu, kc, vc (rotated like the kernels use them)
+      const Shape s = packed_shape(proj, heads);
+      const int64_t d = s.d;
+      const int part[3] = {0, 4, 5};
+      out.push_back(U);
+      for (int i = 0; i < 3; ++i) {
+        Tensor buf = at::empty({B, heads, cache_rows, d}, proj.options());
+        if ((flags & CASTLE_FLAG_ROTARY) && part[i] != 5) {
+          const castle_view4 src = packed_view(proj, s, 6, part[i]), dst = view4(buf);
+          check(castle_rope(&src, &dst, s.B, s.H, s.L, s.d, s.dtype, 0, stream_of(proj)), "castle_rope");
+        } else {
+          buf.narrow(2, 0, L).copy_(proj.view({B, L, 6, heads, d}).select(2, part[i]).permute({0, 2, 1, 3}));
+        }
+        out.push_back(buf);
+      }
+    }
+    if (want_graph) {
+      ctx->save_for_backward({norm_w.defined() ? x2 : Tensor(), norm_w, w_qkv, w_out, h, rstd, merged, ws, state});
+      ctx->saved_data["heads"] = heads;
+      ctx->saved_data["scale"] = scale;
+      ctx->saved_data["flags"] = flags;
+      ctx->mark_non_differentiable(variable_list(out.begin() + 1, out.end()));
+      ctx->set_materialize_grads(false);
+    }
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    variable_list grads(11);
+    if (!g[0].defined()) return grads;
+    const at::NoGradGuard no_grad;   // no second derivatives, as for the operators
+    const auto s = ctx->get_saved_variables();
+    const Tensor &x2 = s[0], &norm_w = s[1], &w_qkv = s[2], &w_out = s[3], &h = s[4], &rstd = s[5], &merged = s[6], &ws = s[7], &state = s[8];
+    const c10::DeviceGuard guard(h.device());
+    const int64_t B = merged.size(0), L = merged.size(1), dim = h.size(1), heads = ctx->saved_data["heads"].toInt();
+    const Tensor dy = g[0].reshape({B * L, w_out.size(0)});
+    const size_t n = norm_w.defined() ? 1 : 0;   // needs_input_grad counts the tensors that were there
+    const bool need_x = ctx->needs_input_grad(0), need_norm = n && ctx->needs_input_grad(1);
+    const bool need_qkv = ctx->needs_input_grad(1 + n);
+    if (ctx->needs_input_grad(2 + n)) grads[3] = weight_grad(dy, merged.view({B * L, merged.size(2)}));
+    if (!need_x && !need_norm && !need_qkv) return grads;
+    const Tensor dmerged = at::mm(dy, w_out);
+    const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
+    Tensor dproj = at::empty({B, L, 6 * merged.size(2)}, merged.options());
+    castle_view4 d6[6];
+    six_of_packed(dproj, shape, d6);
+    // the backward kernels read the operand copies in the workspace: the projection itself is not kept
+    run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(),
+            ctx->saved_data["flags"].toInt(), d6, ws, state);
+    const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
+    if (need_qkv) grads[2] = weight_grad(dp2, h);
+    if (need_x || need_norm) {
+      Tensor dh = at::mm(dp2, w_qkv);
+      if (norm_w.defined()) {
+        auto [dx, dn] = at::_fused_rms_norm_backward(dh, x2, {dim}, rstd, norm_w, {need_x, need_norm});
+        if (need_norm) grads[1] = dn;
+        dh = dx;
+      }
+      if (need_x) grads[0] = dh.view({B, L, dim});
+    }
+    return grads;
+  }
+};
+
+// x (B, L, dim) -> [y], or [y, U, qu, kc, vc] with buffers of `cache_rows` rows when cache_rows > 0
+variable_list layer_parallel(const Tensor& x, const std::optional<Tensor>& norm_w, std::optional<double> eps, const Tensor& w_qkv,
+                             const Tensor& w_out, int64_t heads, double scale, int64_t flags, bool keep_state, int64_t cache_rows) {
+  const c10::DeviceGuard guard(x.device());
+  if (!wants_graph({x, norm_w.value_or(Tensor()), w_qkv, w_out}))
+    return LayerFn::forward(nullptr, x, norm_w, w_qkv, w_out, eps, heads, scale, flags, false, false, cache_rows);
+  return LayerFn::apply(x, norm_w, w_qkv, w_out, eps, heads, scale, flags, true, keep_state, cache_rows);
+}
+
+// ---- the cached single-token step ------------------------------------------------------------------------------
+// (B, 1, K) x (N, K) through the small-M kernel: see castle_small_linear_fused
+bool small_linear_ok(const Tensor& x, const Tensor& w, int64_t max_rows) {
+  return x.is_cuda() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && w.scalar_type() == x.scalar_type() &&
+         x.dim() == 3 && x.size(1) == 1 && x.size(0) <= max_rows && x.stride(2) == 1 && w.stride(1) == 1 && x.size(2) % 8 == 0 &&
+         w.size(0) % 2 == 0 && x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+}
+Tensor small_linear(const Tensor& x, const Tensor& w, const std::optional<Tensor>& norm_w, double eps, int64_t act,
+                    const std::optional<Tensor>& residual) {
+  const c10::DeviceGuard guard(x.device());
+  const int64_t B = x.size(0), N = w.size(0);
+  Tensor y = at::empty({B, 1, N}, x.options());
+  check(castle_small_linear_fused(x.data_ptr(), w.data_ptr(), y.data_ptr(), (int)B, (int)N, (int)x.size(2), x.stride(0), w.stride(0), N,
+                                  dtype_code(x), norm_w ? norm_w->data_ptr() : nullptr, (float)eps, (int)act,
+                                  residual ? residual->data_ptr() : nullptr, residual ? residual->stride(0) : 0, stream_of(x)),
+        "castle_small_linear_fused");
+  return y;
+}
+
+// The capacity buffers of one decode cache with everything a step needs to know about them
+class StepPlan {
+ public:
+  StepPlan(std::vector<Tensor> buffers, Tensor ring, Tensor gates, Tensor workspace, bool u_half)
+      : buffers_(std::move(buffers)), ring_(std::move(ring)), gates_(std::move(gates)), workspace_(std::move(workspace)) {
+    TORCH_CHECK(buffers_.size() == 4 && gates_.scalar_type() == at::kFloat && gates_.is_contiguous(), "StepPlan: unexpected buffers");
+    for (int i = 0; i < 4; ++i) views_[i] = view4(buffers_[i]);
+    s_ = shape_of(buffers_[0]);   // L = capacity
+    flags_ = u_half ? CASTLE_FLAG_U_HALF : 0;
+    deferred_ = {view4(ring_), view4(gates_), 0, nullptr};
+  }
+
+  // proj (B, 1, 6 H d) -> (B, 1, H d) at row count t.  base >= 0: deferred write-back of the lookahead keys from
+  // that row count on (see castle_deferred); base < 0: every step writes them.
+  Tensor attend(const Tensor& proj_, int64_t t, int64_t base, double scale, bool rotary) {
+    TORCH_CHECK_VALUE(t >= 0 && t < s_.L, "cache capacity ", s_.L, " cannot take row ", t);
+    const Tensor proj = packed_readable(proj_);
+    TORCH_CHECK_VALUE(proj.dim() == 3 && proj.size(0) == s_.B && proj.size(1) == 1 && proj.size(2) == 6LL * s_.H * s_.d &&
+                          proj.scalar_type() == buffers_[0].scalar_type() && proj.device() == buffers_[0].device(),
+                      "the projection does not belong to this cache");
+    const c10::DeviceGuard guard(proj.device());
+    Tensor out = at::empty({s_.B, 1, (int64_t)s_.H * s_.d}, proj.options());
+    Shape one = s_;
+    one.L = 1;
+    castle_view4 v[6];
+    six_of_packed(proj, one, v);
+    const castle_view4 vo = packed_view(out, one, 1, 0);
+    castle_deferred deferred = deferred_;
+    deferred.base = (int)base;
+    check(castle_decode_step(&views_[0], &views_[1], &views_[2], &views_[3], (int)t, s_.L, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], s_.B,
+                             s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0), &vo,
+                             base >= 0 ? &deferred : nullptr, workspace_.data_ptr(), workspace_.numel(), stream_of(proj)),
+          "castle_decode_step");
+    return out;
+  }
+
+  // the whole layer for one token: x (B, 1, dim) -> (B, 1, dim)
+  Tensor layer(const Tensor& x, const std::optional<Tensor>& norm_w, std::optional<double> eps, const Tensor& w_qkv, const Tensor& w_out,
+               int64_t max_rows, int64_t t, int64_t base, double scale, bool rotary) {
+    Tensor proj;
+    if (small_linear_ok(x, w_qkv, max_rows) && (!norm_w || (norm_w->scalar_type() == x.scalar_type() && norm_w->is_contiguous()))) {
+      const double e = eps ? *eps : x.scalar_type() == at::kHalf ? 0.0009765625 : 0.0078125;   // F.rms_norm: the type's epsilon
+      proj = small_linear(x, w_qkv, norm_w, e, CASTLE_ACT_NONE, std::nullopt);
+    } else {
+      proj = at::linear(norm_w ? at::rms_norm(x, {x.size(2)}, norm_w, eps) : x, w_qkv);
+    }
+    const Tensor merged = attend(proj, t, base, scale, rotary);
+    if (small_linear_ok(merged, w_out, max_rows)) return small_linear(merged, w_out, std::nullopt, 0., CASTLE_ACT_NONE, std::nullopt);
+    return at::linear(merged, w_out);
+  }
+
+ private:
+  std::vector<Tensor> buffers_;
+  Tensor ring_, gates_, workspace_;
+  castle_view4 views_[4];
+  castle_deferred deferred_;
+  Shape s_;
+  int flags_;
+};
+
+}  // namespace
+
+TORCH_LIBRARY(castle_hip, m) {
+  m.set_python_module("lookahead_keys_attention_amd.ops");   // the fake (meta) implementations live there
+  const std::vector<at::Tag> tags = {at::Tag::pt2_compliant_tag};
+  m.def("attention(Tensor q, Tensor k, Tensor v, Tensor qu, Tensor ku, Tensor vu, float scale, bool want_U, int flags, bool keep_state) "
+        "-> (Tensor, Tensor, Tensor, Tensor)", tags);
+  m.def("attention_bwd(Tensor q, Tensor k, Tensor v, Tensor qu, Tensor ku, Tensor vu, Tensor out, Tensor dout, Tensor ws, Tensor state, "
+        "float scale, int flags) -> Tensor", tags);
+  m.def("attention_packed(Tensor proj, int heads, float scale, bool want_U, int row_capacity, int flags, bool keep_state) "
+        "-> (Tensor, Tensor, Tensor, Tensor)", tags);
+  m.def("attention_packed_bwd(Tensor proj, Tensor merged, Tensor dmerged, Tensor ws, Tensor state, int heads, float scale, int flags) "
+        "-> Tensor", tags);
+}
+TORCH_LIBRARY_IMPL(castle_hip, CUDA, m) {
+  m.impl("attention", &attention);
+  m.impl("attention_bwd", &attention_bwd);
+  m.impl("attention_packed", &attention_packed);
+  m.impl("attention_packed_bwd", &attention_packed_bwd);
+}
+// CPU tensors: an error that says what is wrong
+TORCH_LIBRARY_IMPL(castle_hip, CPU, m) {
+  m.impl("attention", &attention);
+  m.impl("attention_packed", &attention_packed);
+}
+TORCH_LIBRARY_IMPL(castle_hip, Autograd, m) {
+  m.impl("attention", &attention_autograd);
+  m.impl("attention_packed", &attention_packed_autograd);
+}
+
+PYBIND11_MODULE(_castle_host, m) {
+  namespace py = pybind11;
+  m.attr("ABI_VERSION") = castle_abi_version();
+  using unlocked = py::call_guard<py::gil_scoped_release>;
+  m.def("layer_parallel", &layer_parallel, unlocked());
+  m.def("small_linear", &small_linear, unlocked());
+  py::class_<StepPlan>(m, "StepPlan")
+      .def(py::init<std::vector<Tensor>, Tensor, Tensor, Tensor, bool>())
+      .def("attend", &StepPlan::attend, unlocked())
+      .def("layer", &StepPlan::layer, unlocked());
+}

@@ -63,55 +63,10 @@ def _check_dims(d: int, dtype: torch.dtype):
         raise ValueError("float32 HIP kernels support dim_head <= 64")
 
 
-def _fwd_raw(qc, kc, vc, qu, ku, vu, scale, out, U, flags=0, keep_state=True):
-    """Launch castle_fwd; returns (workspace, state): the tensors the backward pass needs back.
-    `state` is an empty tensor when the caller does not keep the snapshots (`keep_state` False)."""
-    B, H, L, d = qc.shape
-    code = N.dtype_code(qc.dtype)
-    lib = N.lib()
-    nbytes = N.check(lib.castle_fwd_workspace_bytes(B, H, L, d, code), "castle_fwd_workspace_bytes")
-    sbytes = N.check(lib.castle_fwd_state_bytes(B, H, L, d, code), "castle_fwd_state_bytes")
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=qc.device)
-    state = torch.empty(sbytes, dtype=torch.uint8, device=qc.device)
-    views = [N.view4(t) for t in (qc, kc, vc, qu, ku, vu)]
-    vo = N.view4(out)
-    vU = N.view4(U) if U is not None else N.View4(None, 0, 0, 0)
-    with torch.cuda.device(qc.device):
-        rc = lib.castle_fwd(*views, B, H, L, d, code, float(scale), int(flags), vo, vU, ws.data_ptr(), nbytes,
-                            state.data_ptr(), sbytes, N.stream_ptr(qc.device))
-    N.check(rc, "castle_fwd")
-    if not keep_state:
-        state = torch.empty(0, dtype=torch.uint8, device=qc.device)   # the caching allocator keeps the block until the stream is done with it
-    if CHECK_RANGE:
-        status = range_status(ws)
-        if status:
-            raise RuntimeError(f"castle_fwd clamped values to the fp16 range (status bits {status:#x}: "
-                               "1 = input element, 2 = T' = s qc.vu entry)")
-    return ws, state
-
-
 def range_status(ws: torch.Tensor) -> int:
     """Status word the forward kernels leave at the start of their workspace (synchronises):
     bit 0 = an input element was clamped to +-65504, bit 1 = an entry of T' = s qc.vu was."""
     return int(ws[:4].view(torch.int32).item())
-
-
-def _bwd_raw(qc, kc, vc, qu, ku, vu, out, dout, scale, grads, ws, state, flags=0):
-    B, H, L, d = qc.shape
-    code = N.dtype_code(qc.dtype)
-    lib = N.lib()
-    flags &= ~N.FLAG_U_HALF   # describes the forward's U output only
-    if state.numel() == 0:
-        flags |= N.FLAG_RECOMPUTE_STATE
-    nbytes = N.check(lib.castle_bwd_workspace_bytes(B, H, L, d, code, int(flags)), "castle_bwd_workspace_bytes")
-    bws = torch.empty(nbytes, dtype=torch.uint8, device=qc.device)
-    views = [N.view4(t) for t in (qc, kc, vc, qu, ku, vu, out, dout)]
-    gviews = [N.view4(t) for t in grads]
-    with torch.cuda.device(qc.device):
-        rc = lib.castle_bwd(*views, B, H, L, d, code, float(scale), int(flags), *gviews,
-                            ws.data_ptr(), ws.numel(), state.data_ptr() if state.numel() else None, state.numel(),
-                            bws.data_ptr(), nbytes, N.stream_ptr(qc.device))
-    N.check(rc, "castle_bwd")
 
 
 def _as_readable(t: torch.Tensor) -> torch.Tensor:
@@ -119,16 +74,18 @@ def _as_readable(t: torch.Tensor) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------------------------------------
-# Registered operators (torch.library): the kernels are reachable as torch.ops.castle_hip.*, with
-# fake (meta) implementations for shape propagation / tracing and autograd formulas that call the
-# backward entry point.  The Python functions below them are what callers use.
+# Registered operators (torch.library): the kernels are reachable as torch.ops.castle_hip.*.  Their
+# implementations and autograd formulas are in csrc/castle_host.cpp (an operator written in Python
+# costs more host time than the kernels of a short sequence take); the fake (meta) implementations
+# for shape propagation / tracing are below.  The Python functions after them are what callers use.
 #
-#   castle_hip::attention         six (B,H,L,d) operands -> (out, U, workspace)
-#   castle_hip::attention_packed  (B,L,6*H*d) projection -> (merged out, workspace); U written into
-#                                 the optional (B,H,L,d) view `U_out` (a cache buffer)
+#   castle_hip::attention         six (B,H,L,d) operands -> (out, U, workspace, state)
+#   castle_hip::attention_packed  (B,L,6*H*d) projection -> (merged out, U, workspace, state); U the first L
+#                                 rows of a (B,H,row_capacity,d) buffer (a cache buffer)
 #   castle_hip::attention_bwd / attention_packed_bwd   their backward passes
 # `U` is an empty tensor when the lookahead keys are not asked for.  The workspace output is what
-# the backward pass needs back (operand copies, snapshots, log-sum-exp); it carries no gradient.
+# the backward pass needs back (operand copies, log-sum-exp), the state output the snapshots (empty
+# when they are not kept); they carry no gradient.
 def _out_like(q):
     B, H, L, d = q.shape
     return torch.empty((B, L, H, d), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3)
@@ -161,22 +118,7 @@ def _fwd_ws_bytes(B, H, L, d, dtype):
                    "castle_fwd_workspace_bytes")
 
 
-@torch.library.custom_op("castle_hip::attention", mutates_args=())
-def _attention_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, qu: torch.Tensor, ku: torch.Tensor,
-                  vu: torch.Tensor, scale: float, want_U: bool, flags: int,
-                  keep_state: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    _require_gpu(q, "castle_attention_hip")
-    B, H, L, d = q.shape
-    _check_dims(d, q.dtype)
-    ops = [_as_readable(t) for t in (q, k, v, qu, ku, vu)]
-    out = _out_like(q)
-    U = torch.empty((B, H, L, d) if want_U else (0,), dtype=q.dtype, device=q.device)
-    ws, state = _fwd_raw(*ops, scale, out, U if want_U else None, flags, keep_state)
-    return out, U, ws, state
-
-
-@_attention_op.register_fake
-def _(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state):
+def _fake_attention(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state):
     B, H, L, d = q.shape
     _check_dims(d, q.dtype)
     U = torch.empty((B, H, L, d) if want_U else (0,), dtype=q.dtype, device=q.device)
@@ -184,74 +126,11 @@ def _(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state):
     return _out_like(q), U, ws, _fake_state(B, H, L, d, q, keep_state)
 
 
-@torch.library.custom_op("castle_hip::attention_bwd", mutates_args=())
-def _attention_bwd_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, qu: torch.Tensor, ku: torch.Tensor,
-                      vu: torch.Tensor, out: torch.Tensor, dout: torch.Tensor, ws: torch.Tensor, state: torch.Tensor,
-                      scale: float, flags: int) -> torch.Tensor:
-    B, H, L, d = q.shape
-    ops = [_as_readable(t) for t in (q, k, v, qu, ku, vu)]
-    packed = torch.empty((6, B, H, L, d), dtype=out.dtype, device=out.device)
-    _bwd_raw(*ops, _as_readable(out), _as_readable(dout), scale, list(packed.unbind(0)), ws, state, flags)
-    return packed
-
-
-@_attention_bwd_op.register_fake
-def _(q, k, v, qu, ku, vu, out, dout, ws, state, scale, flags):
+def _fake_attention_bwd(q, k, v, qu, ku, vu, out, dout, ws, state, scale, flags):
     return torch.empty((6, *q.shape), dtype=out.dtype, device=out.device)
 
 
-def _attention_setup(ctx, inputs, output):
-    q, k, v, qu, ku, vu, scale, want_U, flags, keep_state = inputs
-    out, U, ws, state = output
-    ctx.save_for_backward(q, k, v, qu, ku, vu, out, ws, state)
-    ctx.scale, ctx.flags = scale, flags
-    ctx.mark_non_differentiable(U, ws, state)   # U carries no gradient (lookahead_keys_attention_triton.py:513-515)
-    # without this autograd hands the backward formula zero tensors for the unused outputs: a fill of
-    # the whole workspace and state buffers (hundreds of MB) on every backward pass
-    ctx.set_materialize_grads(False)
-
-
-def _attention_backward(ctx, dout, dU, dws, dstate):
-    q, k, v, qu, ku, vu, out, ws, state = ctx.saved_tensors
-    if dout is None:
-        dout = torch.zeros_like(out)
-    grads = torch.ops.castle_hip.attention_bwd(q, k, v, qu, ku, vu, out, dout, ws, state, ctx.scale, ctx.flags)
-    return (*grads.unbind(0), None, None, None, None)
-
-
-_attention_op.register_autograd(_attention_backward, setup_context=_attention_setup)
-
-
-def _six_views(proj, heads):
-    B, L, width = proj.shape
-    d = width // (6 * heads)
-    six = proj.view(B, L, 6, heads, d).permute(2, 0, 3, 1, 4)      # (6, B, H, L, d) views
-    return six.unbind(0)                                            # qu, ku, vu, qc, kc, vc
-
-
-def _packed_ok(t):
-    return t if (t.is_contiguous() and t.data_ptr() % 16 == 0) else t.contiguous()
-
-
-@torch.library.custom_op("castle_hip::attention_packed", mutates_args=())
-def _attention_packed_op(proj: torch.Tensor, heads: int, scale: float, want_U: bool, row_capacity: int,
-                         flags: int, keep_state: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    # The lookahead keys come back as the first L rows of a (B, H, row_capacity, d) buffer, so that a
-    # caller can hand over the U buffer of a decode cache without copying (row_capacity >= L).
-    _require_gpu(proj, "castle_attention_packed")
-    B, L, width = proj.shape
-    d = width // (6 * heads)
-    _check_dims(d, proj.dtype)
-    qu, ku, vu, qc, kc, vc = _six_views(_packed_ok(proj), heads)
-    merged = torch.empty((B, L, heads * d), dtype=proj.dtype, device=proj.device)
-    out = merged.view(B, L, heads, d).permute(0, 2, 1, 3)
-    U = torch.empty((B, heads, max(row_capacity, L), d) if want_U else (0,), dtype=proj.dtype, device=proj.device)
-    ws, state = _fwd_raw(qc, kc, vc, qu, ku, vu, scale, out, U[:, :, :L] if want_U else None, flags, keep_state)
-    return merged, U, ws, state
-
-
-@_attention_packed_op.register_fake
-def _(proj, heads, scale, want_U, row_capacity, flags, keep_state):
+def _fake_attention_packed(proj, heads, scale, want_U, row_capacity, flags, keep_state):
     B, L, width = proj.shape
     d = width // (6 * heads)
     _check_dims(d, proj.dtype)
@@ -260,43 +139,22 @@ def _(proj, heads, scale, want_U, row_capacity, flags, keep_state):
     return torch.empty((B, L, heads * d), dtype=proj.dtype, device=proj.device), U, ws, _fake_state(B, heads, L, d, proj, keep_state)
 
 
-@torch.library.custom_op("castle_hip::attention_packed_bwd", mutates_args=())
-def _attention_packed_bwd_op(proj: torch.Tensor, merged: torch.Tensor, dmerged: torch.Tensor, ws: torch.Tensor,
-                             state: torch.Tensor, heads: int, scale: float, flags: int) -> torch.Tensor:
-    B, L, width = proj.shape
-    d = width // (6 * heads)
-    qu, ku, vu, qc, kc, vc = _six_views(_packed_ok(proj), heads)
-    out = merged.view(B, L, heads, d).permute(0, 2, 1, 3)
-    dout = _packed_ok(dmerged).view(B, L, heads, d).permute(0, 2, 1, 3)
-    dproj = torch.empty((B, L, width), dtype=proj.dtype, device=proj.device)
-    dqu, dku, dvu, dqc, dkc, dvc = _six_views(dproj, heads)
-    _bwd_raw(qc, kc, vc, qu, ku, vu, out, dout, scale, (dqc, dkc, dvc, dqu, dku, dvu), ws, state, flags)
-    return dproj
-
-
-@_attention_packed_bwd_op.register_fake
-def _(proj, merged, dmerged, ws, state, heads, scale, flags):
+def _fake_attention_packed_bwd(proj, merged, dmerged, ws, state, heads, scale, flags):
     return torch.empty(proj.shape, dtype=proj.dtype, device=proj.device)
 
 
-def _packed_setup(ctx, inputs, output):
-    proj, heads, scale, want_U, row_capacity, flags, keep_state = inputs
-    merged, U, ws, state = output
-    ctx.save_for_backward(proj, merged, ws, state)
-    ctx.heads, ctx.scale, ctx.flags = heads, scale, flags
-    ctx.mark_non_differentiable(U, ws, state)
-    ctx.set_materialize_grads(False)   # see _attention_setup
+def _register_fakes():
+    """Called once, when _castle_host.so has defined the operators."""
+    for name, fake in (("attention", _fake_attention), ("attention_bwd", _fake_attention_bwd),
+                       ("attention_packed", _fake_attention_packed), ("attention_packed_bwd", _fake_attention_packed_bwd)):
+        torch.library.register_fake("castle_hip::" + name, fake)
 
 
-def _packed_backward(ctx, dmerged, dU, dws, dstate):
-    proj, merged, ws, state = ctx.saved_tensors
-    if dmerged is None:
-        dmerged = torch.zeros_like(merged)
-    dproj = torch.ops.castle_hip.attention_packed_bwd(proj, merged, dmerged, ws, state, ctx.heads, ctx.scale, ctx.flags)
-    return dproj, None, None, None, None, None, None
-
-
-_attention_packed_op.register_autograd(_packed_backward, setup_context=_packed_setup)
+def _check_range(ws):
+    status = range_status(ws)
+    if status:
+        raise RuntimeError(f"castle_fwd clamped values to the fp16 range (status bits {status:#x}: "
+                           "1 = input element, 2 = T' = s qc.vu entry)")
 
 
 def castle_attention_hip(q, k, v, qu, ku, vu, scale, return_U_for_cache=False, rotary=False):
@@ -305,8 +163,12 @@ def castle_attention_hip(q, k, v, qu, ku, vu, scale, return_U_for_cache=False, r
     flags = DEFAULT_FLAGS | (N.FLAG_ROTARY if rotary else 0)
     B, H, L, d = q.shape
     _check_dims(d, q.dtype)
-    out, U, _, _ = torch.ops.castle_hip.attention(q, k, v, qu, ku, vu, float(scale), bool(return_U_for_cache), int(flags),
-                                                  keeps_state(B, H, L, d, q.dtype))
+    if N._host is None:
+        N.host()
+    out, U, ws, _ = torch.ops.castle_hip.attention(q, k, v, qu, ku, vu, float(scale), bool(return_U_for_cache), int(flags),
+                                                   keeps_state(B, H, L, d, q.dtype))
+    if CHECK_RANGE:
+        _check_range(ws)
     return (out, U) if return_U_for_cache else out
 
 
@@ -319,9 +181,13 @@ def castle_attention_packed(proj, heads, scale, return_U_for_cache=False, row_ca
     flags = DEFAULT_FLAGS | (N.FLAG_ROTARY if rotary else 0) | (N.FLAG_U_HALF if u_half and return_U_for_cache else 0)
     B, L, width = proj.shape
     _check_dims(width // (6 * int(heads)), proj.dtype)
-    merged, U, _, _ = torch.ops.castle_hip.attention_packed(proj, int(heads), float(scale), bool(return_U_for_cache),
-                                                         int(row_capacity), int(flags),
-                                                         keeps_state(B, int(heads), L, width // (6 * int(heads)), proj.dtype))
+    if N._host is None:
+        N.host()
+    merged, U, ws, _ = torch.ops.castle_hip.attention_packed(proj, int(heads), float(scale), bool(return_U_for_cache),
+                                                             int(row_capacity), int(flags),
+                                                             keeps_state(B, int(heads), L, width // (6 * int(heads)), proj.dtype))
+    if CHECK_RANGE:
+        _check_range(ws)
     return (merged, U[:, :, : proj.shape[1]]) if return_U_for_cache else merged
 
 
@@ -408,8 +274,6 @@ def small_linear(x: torch.Tensor, weight: torch.Tensor, norm=None, activation=No
     train_triton.py:103, 164), `activation="gelu"` the erf GELU of train_triton.py:105 on the
     product, `residual` a (B, 1, N) tensor added last (train_triton.py:161-162)."""
     B, _, K = x.shape
-    n = weight.shape[0]
-    y = torch.empty((B, 1, n), dtype=x.dtype, device=x.device)
     norm_weight, eps = None, 0.0
     if norm is not None:
         norm_weight = norm.weight
@@ -418,16 +282,9 @@ def small_linear(x: torch.Tensor, weight: torch.Tensor, norm=None, activation=No
             raise ValueError("small_linear: the norm weight must be a contiguous (K,) tensor of the input type")
     if activation not in (None, "gelu"):
         raise ValueError(f"small_linear: unknown activation {activation!r}")
-    if residual is not None and (residual.shape != y.shape or residual.dtype != x.dtype or residual.stride(2) != 1):
+    if residual is not None and (residual.shape != (B, 1, weight.shape[0]) or residual.dtype != x.dtype or residual.stride(2) != 1):
         raise ValueError("small_linear: the residual must have the output's shape and type")
-    with torch.cuda.device(x.device):
-        rc = N.lib().castle_small_linear_fused(
-            x.data_ptr(), weight.data_ptr(), y.data_ptr(), B, n, K, x.stride(0), weight.stride(0), n, N.dtype_code(x.dtype),
-            norm_weight.data_ptr() if norm_weight is not None else None, eps, 1 if activation == "gelu" else 0,
-            residual.data_ptr() if residual is not None else None, residual.stride(0) if residual is not None else 0,
-            N.stream_ptr(x.device))
-    N.check(rc, "castle_small_linear_fused")
-    return y
+    return N.host().small_linear(x, weight, norm_weight, eps, 1 if activation == "gelu" else 0, residual)
 
 
 @torch.no_grad()
@@ -479,3 +336,7 @@ def castle_decode_step_packed(cache_views, capacity, t, proj, heads, scale, out,
                 workspace.data_ptr(), workspace.numel(), N.stream_ptr(proj.device))
     N.check(rc, "castle_decode_step")
     return out
+
+
+if N.is_built():
+    N.host()   # defines torch.ops.castle_hip.*
