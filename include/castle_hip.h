@@ -214,6 +214,23 @@ int castle_decode_step_static(const castle_view4* U, const castle_view4* qu_cach
                               int B, int H, int d, int dtype, float scale, int flags,
                               const castle_view4* out, const castle_deferred* deferred, void* stream);
 
+/* A whole layer for one token per sequence: y = residual + core(norm(x) w_in^T) w_out^T, the cached step with
+ * the norm and the projections around it (lookahead_keys_attention.py:95-99, 166-203, 209 with seq_len == 1) in
+ * four launches behind one call.
+ * x, y: B rows of `dim` elements; w_in (6 H d, dim), w_out (dim, H d), both row-major in the tensor type, `proj` a
+ * B x 6 H d scratch in the tensor type (order qu, ku, vu, qc, kc, vc).  norm_weight (`dim` elements), residual
+ * (B rows; may alias y) and t_device may be NULL.  dim % 8 == 0 (4 for fp32); x, w_in, w_out, proj and norm_weight
+ * 16-byte aligned with leading dimensions of whole 16-byte pieces.  The other arguments, the workspace among
+ * them, are those of castle_decode_step / castle_decode_step_device_count.  Meant for B up to a few dozen. */
+int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
+                        const castle_view4* kc_cache, const castle_view4* vc_cache,
+                        int t, const int32_t* t_device, int capacity,
+                        const void* x, int64_t ldx, int dim, const void* norm_weight, float eps,
+                        const void* w_in, int64_t ldw_in, const void* w_out, int64_t ldw_out,
+                        const void* residual, int64_t ldr, void* y, int64_t ldy, void* proj,
+                        int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
+                        void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Rotary position embedding of one tensor, out of place: out[b,h,l,:] = R(first_position + l) x[b,h,l,:]
  * (the rotation CASTLE_FLAG_ROTARY applies inside the kernels; lookahead_keys_attention.py:112).  Used to
  * fill the qu / kc rows of a decode cache after a rotary prefill. */
@@ -224,7 +241,7 @@ int castle_rope(const castle_view4* x, const castle_view4* out, int B, int H, in
  * dimensions ldx, ldw, ldy in elements; fp32 accumulation), for the few rows of a decode step: the
  * fused projection and the output projection around the cached step, which the reference runs as
  * nn.Linear on a (B, 1, dim) tensor (lookahead_keys_attention.py:99 and :209 with seq_len == 1).
- * Meant for M up to a few dozen rows (one workgroup per 32 x 32 output tile, K split over its
+ * Meant for M up to a few dozen rows (one workgroup per 16-column slice of the output, K split over its
  * waves); any M works.  K % 8 == 0, N % 2 == 0, x / w 16-byte aligned with ldx, ldw % 8 == 0. */
 int castle_small_linear(const void* x, const void* w, void* y, int M, int N, int K,
                         int64_t ldx, int64_t ldw, int64_t ldy, int dtype, void* stream);

@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "castle_decode_step_device_count",
     "castle_decode_step_static",
     "castle_decode_flush",
+    "castle_decode_layer",
     "castle_rope",
     "castle_small_linear",
     "castle_small_linear_fused",

@@ -366,7 +366,7 @@ class Castle(nn.Module):
                 y = store.plan.layer(x, norm._parameters.get("weight"), getattr(norm, "eps", None),
                                      self._modules["to_all_qkv"]._parameters["weight"],
                                      self._modules["combine_heads"]._parameters["weight"],
-                                     ops.SMALL_LINEAR_MAX_ROWS, store.length, base, self.scale, self.use_rotary)
+                                     ops.SMALL_LINEAR_MAX_ROWS, store.length, base, self.scale, self.use_rotary, None, None, None)
                 cache = store.advanced(base)
                 return (y, cache) if return_next_cache else y
             assert cache is None, "must be inferencing single tokens if receiving cache"
@@ -481,7 +481,7 @@ class Castle(nn.Module):
     def _step_native(self, proj, cache):
         store = self._store_for(cache, proj)
         base = store.step_base()
-        out = store.plan.attend(proj, store.length, base, self.scale, self.use_rotary)
+        out = store.plan.attend(proj, store.length, base, self.scale, self.use_rotary, None, None)
         return out, store.advanced(base)
 
     def graph_step(self, x, store, t_device, base_device=None, residual=None):
@@ -493,14 +493,14 @@ class Castle(nn.Module):
         keys are complete, e.g. the prefill length) switches the deferred write-back on.
         x: (B, 1, dim); store: the `_CacheStore` behind a native cache.  Returns (B, 1, dim), plus
         `residual` when one is given (added inside the output projection's launch)."""
-        B = x.shape[0]
+        if self._plain(x):
+            norm = self.norm
+            return store.plan.layer(x, getattr(norm, "weight", None), getattr(norm, "eps", None), self.to_all_qkv.weight,
+                                    self.combine_heads.weight, ops.SMALL_LINEAR_MAX_ROWS, 0, -1, self.scale, self.use_rotary, residual,
+                                    t_device, base_device)
         proj = self._project(self.to_all_qkv, x, True, norm=self.norm)
-        out = torch.empty((B, 1, self.heads, self.dim_head), dtype=proj.dtype, device=proj.device)
-        ops.castle_decode_step_packed(store.views, store.capacity, 0, proj, self.heads, self.scale, out,
-                                      store.workspace, rotary=self.use_rotary, t_device=t_device,
-                                      deferred=store.deferred(base_device) if base_device is not None else None,
-                                      u_half=store.u_half)
-        return self._project(self.combine_heads, out.view(B, 1, self.heads * self.dim_head), True, residual=residual)
+        out = store.plan.attend(proj, 0, -1, self.scale, self.use_rotary, t_device, base_device)
+        return self._project(self.combine_heads, out, True, residual=residual)
 
     # -- dense PyTorch formulation (use_triton=False) -------------------------
     def _parallel_dense(self, proj, want_cache):

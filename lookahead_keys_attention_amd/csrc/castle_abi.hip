@@ -16,7 +16,7 @@ int launch_bwd(const BwdArgs& a, int dtype, bool bf16_operands, hipStream_t stre
 int launch_decode(const DecodeArgs& a, int dtype, hipStream_t stream);
 int launch_decode_flush(const DecodeArgs& a, int dtype, hipStream_t stream);
 int launch_rope(const View4& src, const View4& dst, int B, int H, int L, int d, int dtype, int pos0, hipStream_t stream);
-int decode_pick_splits(int BH, int t);
+int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus);
 int decode_static_scratch(float** ptr);
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                         int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream);
@@ -285,14 +285,15 @@ int64_t castle_decode_workspace_bytes(int B, int H, int d, int t_max) {
   return align_up((int64_t)B * H * 64 * (d + 2) * 4, 256);
 }
 
-static int decode_step_common(const castle_view4* U, const castle_view4* qu_cache,
+// checks the arguments of a cached step and fills `a`; out may be NULL when the caller sets a.out itself
+static int decode_step_args(castle::DecodeArgs& a, const castle_view4* U, const castle_view4* qu_cache,
                               const castle_view4* kc_cache, const castle_view4* vc_cache,
                               int t, const int* t_device, int capacity,
                               const castle_view4* qc, const castle_view4* kc, const castle_view4* vc,
                               const castle_view4* qu, const castle_view4* ku, const castle_view4* vu,
                               int B, int H, int d, int dtype, float scale, int flags,
                               const castle_view4* out, const castle_deferred* deferred,
-                              void* workspace, int64_t workspace_bytes, bool static_scratch, void* stream) {
+                              void* workspace, int64_t workspace_bytes, bool static_scratch) {
   const int es = elem_size(dtype);
   if (es == 0) return CASTLE_ERR_DTYPE;
   if ((flags & CASTLE_FLAG_U_HALF) && dtype != CASTLE_BF16) return CASTLE_ERR_DTYPE;
@@ -301,9 +302,10 @@ static int decode_step_common(const castle_view4* U, const castle_view4* qu_cach
   const castle_view4* caches[] = {U, qu_cache, kc_cache, vc_cache};
   for (const castle_view4* v : caches)
     if (!view_ok(v, es, true)) return CASTLE_ERR_ARG;
-  const castle_view4* tok[] = {qc, kc, vc, qu, ku, vu, out};
+  const castle_view4* tok[] = {qc, kc, vc, qu, ku, vu};
   for (const castle_view4* v : tok)
     if (!view_ok(v, es, false)) return CASTLE_ERR_ARG;
+  if (out != nullptr && !view_ok(out, es, false)) return CASTLE_ERR_ARG;
   if (deferred != nullptr) {
     if (!view_ok(&deferred->vu_ring, es, true) || !view_ok(&deferred->gates, 4, false)) return CASTLE_ERR_ARG;
     if (deferred->base < 0 || (deferred->base_device != nullptr && reinterpret_cast<uintptr_t>(deferred->base_device) % 4 != 0))
@@ -312,7 +314,7 @@ static int decode_step_common(const castle_view4* U, const castle_view4* qu_cach
     if (t_device == nullptr && deferred->base_device == nullptr && deferred->base > t) return CASTLE_ERR_SHAPE;
   }
   // with a device-side count the split must not depend on it: sized for a full cache
-  const int splits = castle::decode_pick_splits(B * H, t_device != nullptr ? capacity : t);
+  const int splits = castle::decode_pick_splits(B * H, t_device != nullptr ? capacity : t, castle::kThreads * 16 / (d * es), device_cus());
   if (static_scratch) {
     // the per-GPU array replaces the caller's workspace; nothing is allocated on this path
     if ((int64_t)B * H * splits * (d + 2) * 4 > castle::kDecodeStaticScratchBytes) return CASTLE_ERR_SCRATCH;
@@ -324,7 +326,6 @@ static int decode_step_common(const castle_view4* U, const castle_view4* qu_cach
     return CASTLE_ERR_WORKSPACE;
   }
 
-  castle::DecodeArgs a;
   a.B = B; a.H = H; a.d = d; a.t = t; a.scale = scale;
   a.t_dev = t_device; a.capacity = capacity;
   a.rotary = (flags & CASTLE_FLAG_ROTARY) != 0;
@@ -339,7 +340,22 @@ static int decode_step_common(const castle_view4* U, const castle_view4* qu_cach
   a.pend_gate = to_view(deferred != nullptr ? &deferred->gates : nullptr);
   a.base0 = deferred != nullptr ? deferred->base : 0;
   a.base0_dev = deferred != nullptr ? deferred->base_device : nullptr;
-  return castle::launch_decode(a, dtype, static_cast<hipStream_t>(stream));
+  return CASTLE_OK;
+}
+
+static int decode_step_common(const castle_view4* U, const castle_view4* qu_cache,
+                              const castle_view4* kc_cache, const castle_view4* vc_cache,
+                              int t, const int* t_device, int capacity,
+                              const castle_view4* qc, const castle_view4* kc, const castle_view4* vc,
+                              const castle_view4* qu, const castle_view4* ku, const castle_view4* vu,
+                              int B, int H, int d, int dtype, float scale, int flags,
+                              const castle_view4* out, const castle_deferred* deferred,
+                              void* workspace, int64_t workspace_bytes, bool static_scratch, void* stream) {
+  if (out == nullptr) return CASTLE_ERR_ARG;
+  castle::DecodeArgs a;
+  const int rc = decode_step_args(a, U, qu_cache, kc_cache, vc_cache, t, t_device, capacity, qc, kc, vc, qu, ku, vu, B, H, d, dtype,
+                                  scale, flags, out, deferred, workspace, workspace_bytes, static_scratch);
+  return rc != CASTLE_OK ? rc : castle::launch_decode(a, dtype, static_cast<hipStream_t>(stream));
 }
 
 int castle_decode_step(const castle_view4* U, const castle_view4* qu_cache,
@@ -376,6 +392,39 @@ int castle_decode_step_device_count(const castle_view4* U, const castle_view4* q
   if (t_device == nullptr || reinterpret_cast<uintptr_t>(t_device) % 4 != 0) return CASTLE_ERR_ARG;
   return decode_step_common(U, qu_cache, kc_cache, vc_cache, 0, t_device, capacity, qc, kc, vc, qu, ku, vu,
                             B, H, d, dtype, scale, flags, out, deferred, workspace, workspace_bytes, false, stream);
+}
+
+int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
+                        const castle_view4* kc_cache, const castle_view4* vc_cache,
+                        int t, const int32_t* t_device, int capacity,
+                        const void* x, int64_t ldx, int dim, const void* norm_weight, float eps,
+                        const void* w_in, int64_t ldw_in, const void* w_out, int64_t ldw_out,
+                        const void* residual, int64_t ldr, void* y, int64_t ldy, void* proj,
+                        int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (B <= 0 || H <= 0 || dim <= 0 || !head_dim_ok(d) || dim % (16 / es) != 0) return CASTLE_ERR_SHAPE;
+  const void* p16[] = {x, w_in, w_out, proj};
+  for (const void* p : p16)
+    if (p == nullptr || reinterpret_cast<uintptr_t>(p) % 16 != 0) return CASTLE_ERR_ARG;
+  if (y == nullptr || reinterpret_cast<uintptr_t>(norm_weight) % 16 != 0 || (norm_weight != nullptr && !(eps >= 0.f))) return CASTLE_ERR_ARG;
+  const int q = 16 / es;
+  if (ldx % q != 0 || ldw_in % q != 0 || ldw_out % q != 0) return CASTLE_ERR_ARG;
+  if (t_device != nullptr && reinterpret_cast<uintptr_t>(t_device) % 4 != 0) return CASTLE_ERR_ARG;
+  const int inner = H * d, width = 6 * inner;
+  castle_view4 tok[6];   // qu, ku, vu, qc, kc, vc
+  for (int i = 0; i < 6; ++i) tok[i] = {static_cast<char*>(proj) + (int64_t)i * inner * es, width, d, width};
+  castle::DecodeArgs a;
+  int rc = decode_step_args(a, U, qu_cache, kc_cache, vc_cache, t_device != nullptr ? 0 : t, t_device, capacity, &tok[3], &tok[4], &tok[5],
+                            &tok[0], &tok[1], &tok[2], B, H, d, dtype, scale, flags, nullptr, deferred, workspace, workspace_bytes, false);
+  if (rc != CASTLE_OK) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  rc = castle::launch_small_linear(x, w_in, proj, B, width, dim, ldx, ldw_in, width, dtype, norm_weight, eps, CASTLE_ACT_NONE, nullptr, 0, s);
+  a.out = to_view(&tok[0]);   // the attention output goes into the scratch: its token operands are spent by then
+  if (rc == 0) rc = castle::launch_decode(a, dtype, s);
+  if (rc != 0) return rc;
+  return castle::launch_small_linear(proj, w_out, y, B, dim, inner, width, ldw_out, ldy, dtype, nullptr, 0.f, CASTLE_ACT_NONE, residual, ldr, s);
 }
 
 int castle_decode_flush(const castle_view4* U, const castle_view4* qu_cache, int t, const castle_deferred* deferred,

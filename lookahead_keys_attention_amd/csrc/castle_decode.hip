@@ -6,19 +6,15 @@
 // and for the appended row t:  U_t = 0,  x_t = s qc_t . kc_t;  out = softmax(x) V.
 // The pass is bandwidth bound: each cached element of qu, U, kc, vc is read once and U is
 // written once (5 * t * d elements per head and step).  The t rows of one (b, h) are split
-// over `splits` workgroups that each keep an online-softmax partial (acc, m, l) in fp32;
-// decode_finish_kernel merges the partials, folds in row t and appends the new rows.
+// over `splits` workgroups that each keep an online-softmax partial (acc, m, l) in fp32; the last
+// of them also takes row t and appends the new rows; decode_finish_kernel merges the partials.  (Letting
+// every workgroup of the output projection merge them while it loads its operand saves that launch and is
+// slower: 14.7 against 13.4 us for a whole layer step of one sequence, 31 against 23 us for 16.)
 #include "castle_tiles.h"
 #include "castle_params.h"
 #include "castle_profile.h"
+#include <algorithm>
 #include <mutex>
-
-#ifndef CASTLE_DEC_PF
-#define CASTLE_DEC_PF 1   // iterations of row pieces requested ahead in the stream kernel
-#endif
-#ifndef CASTLE_DEC_WGS
-#define CASTLE_DEC_WGS 640   // workgroups the stream kernel aims for
-#endif
 
 namespace castle {
 
@@ -60,10 +56,28 @@ template <typename T, int N, bool UH> __device__ __forceinline__ vec<T, N> u_pac
   }
 }
 
+// Sum over a group of LPR neighbouring lanes, in every lane.  The first steps move data inside the vector unit
+// (DPP: neighbours, halves of eight, rows of 16); a shuffle through the LDS crossbar takes several times as long,
+// and nine of them in a row per cached row are what a short step used to wait for.
+template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
+  const int x = __builtin_bit_cast(int, v);
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, true));
+}
 template <int LPR> __device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int o = 1; o < LPR; o <<= 1) v += __shfl_xor(v, o);
+  if constexpr (LPR >= 2) v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+  if constexpr (LPR >= 4) v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+  if constexpr (LPR >= 8) v = dpp_add<0x141>(v);   // row_half_mirror: lane i <- 7 - i of its eight
+  if constexpr (LPR >= 16) v = dpp_add<0x140>(v);  // row_mirror: lane i <- 15 - i of its sixteen
+  if constexpr (LPR >= 32) v += __shfl_xor(v, 16);
   return v;
+}
+
+// partial results of the split pass: the sums of all (b, h, split), then their statistics (maximum, sum of weights)
+__device__ __forceinline__ float* part_acc(const DecodeArgs& a, int bh, int split, int HD) {
+  return a.part + ((int64_t)bh * a.splits + split) * HD;
+}
+__device__ __forceinline__ float* part_stat(const DecodeArgs& a, int bh, int split, int HD) {
+  return a.part + (int64_t)a.B * a.H * a.splits * HD + ((int64_t)bh * a.splits + split) * 2;
 }
 
 // One workgroup = 4 waves; a group of LPR = d / V lanes owns one cache row per iteration.
@@ -73,20 +87,28 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
   constexpr int LPR = HD / V;                // lanes per row
   constexpr int RPI = kThreads / LPR;        // rows per workgroup iteration
   typedef vec<T, V> vt;
-  __shared__ float s_acc[kThreads / LPR][HD + 2];
+  constexpr int NW = kThreads / 64;
+  __shared__ float s_acc[NW][HD + 2];
 
   const int split = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
   int t = a.t_dev != nullptr ? *a.t_dev : a.t;
-  if (t < 0 || t >= a.capacity) t = 0;   // out of range (device-side count only): no rows, the finish kernel writes nothing
+  const bool in_range = t >= 0 && t < a.capacity;
+  if (!in_range) t = 0;   // only with a device-side count: no rows, nothing is appended
   const int tid = threadIdx.x;
   const int grp = tid / LPR, sub = tid % LPR;
-  const float c0 = a.scale, c1 = a.scale * kLog2e;
+  const float c1 = a.scale * kLog2e;
 
   // rows of this workgroup: [r0, r1), whole iterations of RPI rows
   const int per = ((t + a.splits - 1) / a.splits + RPI - 1) / RPI * RPI;
   const int r0 = split * per;
   const int r1 = min(t, r0 + per);
 
+  // deferred write-back: how many tokens are pending, and whether this step writes U
+  const bool deferred = a.pend_vu.ptr != nullptr;
+  const int base0 = a.base0_dev != nullptr ? *a.base0_dev : a.base0;
+  const int pbase = deferred ? decode_base(base0, t) : t;
+  const int np = t - pbase;                                        // 0 .. kDecodeDefer - 1
+  const bool write_u = !deferred || (t + 1) % kDecodeDefer == 0;
   float ku[V], vu[V], qc[V];
   load_f32<T, V>(view_row<T>(a.ku, b, h, 0) + sub * V, ku);
   load_f32<T, V>(view_row<T>(a.vu, b, h, 0) + sub * V, vu);
@@ -101,12 +123,7 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
     }
   }
 
-  // deferred write-back: the pending tokens' vu pieces of this lane, and whether this step writes U
-  const bool deferred = a.pend_vu.ptr != nullptr;
-  const int base0 = a.base0_dev != nullptr ? *a.base0_dev : a.base0;
-  const int pbase = deferred ? decode_base(base0, t) : t;
-  const int np = t - pbase;                                        // 0 .. kDecodeDefer - 1
-  const bool write_u = !deferred || (t + 1) % kDecodeDefer == 0;
+  // the pending tokens' vu pieces of this lane
   float pv[kDecodeDefer][V];   // indexed by ring slot; zero where no pending token sits
 #pragma unroll
   for (int sl = 0; sl < kDecodeDefer; ++sl) {
@@ -122,9 +139,41 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
   for (int e = 0; e < V; ++e) acc[e] = 0.f;
   float m = -INFINITY, l = 0.f;
 
+  // The last split that has rows takes row t too: U_t = 0, so its lookahead term is silu(0) = 0, and appends the
+  // new rows.  No workgroup of this launch reads row t or the ring slot of token t.
+  if (split == (t > 0 ? (t - 1) / per : 0) && grp == 0) {
+    float kct[V], qut[V];
+    load_f32<T, V>(view_row<T>(a.kc, b, h, 0) + sub * V, kct);
+    load_f32<T, V>(view_row<T>(a.qu, b, h, 0) + sub * V, qut);
+    load_f32<T, V>(view_row<T>(a.vc, b, h, 0) + sub * V, acc);
+    if (a.rotary) {
+#pragma unroll
+      for (int e = 0; e < V / 2; ++e) {
+        const int pair = sub * (V / 2) + e;
+        CASTLE_ROPE_PAIR(kct[2 * e], kct[2 * e + 1], (float)t, pair, HD, false);
+        CASTLE_ROPE_PAIR(qut[2 * e], qut[2 * e + 1], (float)t, pair, HD, false);
+      }
+    }
+    float dot = 0.f;
+#pragma unroll
+    for (int e = 0; e < V; ++e) dot = __builtin_fmaf(qc[e], kct[e], dot);
+    m = group_sum<LPR>(dot) * c1;
+    l = 1.f;
+    if (in_range) {
+      vt z, q, kk, v, p;
+#pragma unroll
+      for (int e = 0; e < V; ++e) { z[e] = (T)0.f; q[e] = (T)qut[e]; kk[e] = (T)kct[e]; v[e] = (T)acc[e]; p[e] = (T)vu[e]; }
+      *reinterpret_cast<vt*>(view_row<T>(a.U, b, h, t) + sub * V) = z;
+      *reinterpret_cast<vt*>(view_row<T>(a.qu_cache, b, h, t) + sub * V) = q;
+      *reinterpret_cast<vt*>(view_row<T>(a.kc_cache, b, h, t) + sub * V) = kk;
+      *reinterpret_cast<vt*>(view_row<T>(a.vc_cache, b, h, t) + sub * V) = v;
+      if (deferred) *reinterpret_cast<vt*>(view_row<T>(a.pend_vu, b, h, slot_t) + sub * V) = p;   // joins the pending sources
+    }
+  }
+
   // The row pieces of the next PF iterations are requested before the current one is processed:
   // PF + 1 times the bytes in flight per wave, which is what a latency-bound streaming loop is short of.
-  constexpr int PF = CASTLE_DEC_PF;
+  constexpr int PF = 1;
   vt nq[PF], nu[PF], nk[PF], nv[PF];
   vec<float, 4> ng[PF];
 #pragma unroll
@@ -199,28 +248,47 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
     }
     }
   }
-  (void)c0;
-  // merge the row groups of the workgroup
+  // merge the row groups of a wave in registers, then the waves through LDS
+  {
+    float M = m;
 #pragma unroll
-  for (int e = 0; e < V; ++e) s_acc[grp][sub * V + e] = acc[e];
-  if (sub == 0) { s_acc[grp][HD] = m; s_acc[grp][HD + 1] = l; }
+    for (int o = LPR; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+    const float w = m == -INFINITY ? 0.f : fast_exp2(m - M);
+    l *= w;
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] *= w;
+#pragma unroll
+    for (int o = LPR; o < 64; o <<= 1) {
+      l += __shfl_xor(l, o);
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc[e] += __shfl_xor(acc[e], o);
+    }
+    m = M;
+  }
+  const int wave = tid / 64;
+  if ((tid & 63) < LPR) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) s_acc[wave][sub * V + e] = acc[e];
+    if (sub == 0) { s_acc[wave][HD] = m; s_acc[wave][HD + 1] = l; }
+  }
   __syncthreads();
-  float* part = a.part + ((int64_t)bh * a.splits + split) * (HD + 2);
   if (tid < HD) {
     float M = -INFINITY;
-    for (int r = 0; r < RPI; ++r) M = fmaxf(M, s_acc[r][HD]);
+#pragma unroll
+    for (int r = 0; r < NW; ++r) M = fmaxf(M, s_acc[r][HD]);
     float out = 0.f, lsum = 0.f;
-    for (int r = 0; r < RPI; ++r) {
+#pragma unroll
+    for (int r = 0; r < NW; ++r) {
       const float w = (s_acc[r][HD] == -INFINITY) ? 0.f : fast_exp2(s_acc[r][HD] - M);
       out = __builtin_fmaf(w, s_acc[r][tid], out);
       lsum = __builtin_fmaf(w, s_acc[r][HD + 1], lsum);
     }
-    part[tid] = out;
-    if (tid == 0) { part[HD] = M; part[HD + 1] = lsum; }
+    part_acc(a, bh, split, HD)[tid] = out;
+    if (tid == 0) { part_stat(a, bh, split, HD)[0] = M; part_stat(a, bh, split, HD)[1] = lsum; }
   }
 }
 
-// One wave per (b, h): merge the split partials, add row t, normalise, append the new rows.
+// One wave per (b, h): merges the split partials into the attention output.
 template <typename T, int HD>
 __global__ __launch_bounds__(64) void decode_finish_kernel(DecodeArgs a) {
   constexpr int EPL = (HD + 63) / 64;   // elements per lane
@@ -228,104 +296,47 @@ __global__ __launch_bounds__(64) void decode_finish_kernel(DecodeArgs a) {
   const int lane = threadIdx.x;
   const int t = a.t_dev != nullptr ? *a.t_dev : a.t;
   if (t < 0 || t >= a.capacity) return;   // only reachable with a device-side count: the cache is full
-  const float c1 = a.scale * kLog2e;
-  const float* part = a.part + (int64_t)bh * a.splits * (HD + 2);
-  const T* qc = view_row<T>(a.qc, b, h, 0);
-  const T* kc = view_row<T>(a.kc, b, h, 0);
-  const T* vc = view_row<T>(a.vc, b, h, 0);
-  const T* qu = view_row<T>(a.qu, b, h, 0);
-
-  float dot = 0.f;
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) {
-    const int n = lane + 64 * e;
-    if (n < HD) dot = __builtin_fmaf((float)qc[n], (float)kc[n], dot);
-  }
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) dot += __shfl_xor(dot, o);
-  const float xt = dot * c1;            // row t: U_t = 0, so the lookahead term is silu(0) = 0
-
   // statistics of the partials: lane s holds split s (at most 64 splits), so the loads of all
   // splits are in flight together instead of one dependent load per loop iteration
-  const int nsplit = t > 0 ? a.splits : 0;
   float ms_l = -INFINITY, ls_l = 0.f;
-  if (lane < nsplit) {
-    ms_l = part[lane * (HD + 2) + HD];
-    ls_l = part[lane * (HD + 2) + HD + 1];
+  if (lane < a.splits) {
+    const vec<float, 2> st = *reinterpret_cast<const vec<float, 2>*>(part_stat(a, bh, lane, HD));
+    ms_l = st[0];
+    ls_l = st[1];
   }
   float M = ms_l;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
-  M = fmaxf(M, xt);
   const float w_l = (ms_l == -INFINITY) ? 0.f : fast_exp2(ms_l - M);
   float lsum = w_l * ls_l;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) lsum += __shfl_xor(lsum, o);
-  const float pt = fast_exp2(xt - M);
-  lsum += pt;
   float o[EPL];
 #pragma unroll
-  for (int e = 0; e < EPL; ++e) {
-    const int n = lane + 64 * e;
-    o[e] = n < HD ? pt * (float)vc[n] : 0.f;
-  }
+  for (int e = 0; e < EPL; ++e) o[e] = 0.f;
   constexpr int SU = 8;   // partial rows loaded per batch
-  for (int s0 = 0; s0 < nsplit; s0 += SU) {
+  for (int s0 = 0; s0 < a.splits; s0 += SU) {
     float v[SU][EPL];
 #pragma unroll
     for (int u = 0; u < SU; ++u)
 #pragma unroll
       for (int e = 0; e < EPL; ++e) {
         const int n = lane + 64 * e;
-        v[u][e] = (s0 + u < nsplit && n < HD) ? part[(s0 + u) * (HD + 2) + n] : 0.f;
+        v[u][e] = (s0 + u < a.splits && n < HD) ? part_acc(a, bh, s0 + u, HD)[n] : 0.f;
       }
 #pragma unroll
     for (int u = 0; u < SU; ++u) {
-      const float w = __shfl(w_l, (s0 + u) & 63);   // 0 for lanes beyond nsplit
+      const float w = __shfl(w_l, (s0 + u) & 63);   // 0 for lanes beyond the splits
 #pragma unroll
       for (int e = 0; e < EPL; ++e) o[e] = __builtin_fmaf(w, v[u][e], o[e]);
     }
   }
   const float inv = 1.f / lsum;
-  const bool deferred = a.pend_vu.ptr != nullptr;
-  const T* vu = view_row<T>(a.vu, b, h, 0);
-  T* pvt = deferred ? view_row<T>(a.pend_vu, b, h, t % kDecodeDefer) : nullptr;
   T* out = view_row<T>(a.out, b, h, 0);
-  T* Ut = view_row<T>(a.U, b, h, t);
-  T* qut = view_row<T>(a.qu_cache, b, h, t);
-  T* kct = view_row<T>(a.kc_cache, b, h, t);
-  T* vct = view_row<T>(a.vc_cache, b, h, t);
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
     const int n = lane + 64 * e;
-    float quv = n < HD ? (float)qu[n] : 0.f, kcv = n < HD ? (float)kc[n] : 0.f;
-    if (a.rotary) {   // element n and its pair partner n ^ 1 sit on neighbouring lanes
-      const float qup = __shfl_xor(quv, 1), kcp = __shfl_xor(kcv, 1);
-      const bool even = (n & 1) == 0;
-      float q0 = even ? quv : qup, q1 = even ? qup : quv, k0 = even ? kcv : kcp, k1 = even ? kcp : kcv;
-      CASTLE_ROPE_PAIR(q0, q1, (float)t, n / 2, HD, false);
-      CASTLE_ROPE_PAIR(k0, k1, (float)t, n / 2, HD, false);
-      quv = even ? q0 : q1;
-      kcv = even ? k0 : k1;
-    }
-    if (n < HD) {
-      out[n] = (T)(o[e] * inv);
-      Ut[n] = (T)0.f;
-      qut[n] = (T)quv;
-      kct[n] = (T)kcv;
-      vct[n] = vc[n];
-    }
-    if (deferred) {   // the new token joins the pending sources (rotated like the stream kernel uses it)
-      float vuv = n < HD ? (float)vu[n] : 0.f;
-      if (a.rotary) {
-        const float vup = __shfl_xor(vuv, 1);
-        const bool even = (n & 1) == 0;
-        float v0 = even ? vuv : vup, v1 = even ? vup : vuv;
-        CASTLE_ROPE_PAIR(v0, v1, (float)t, n / 2, HD, false);
-        vuv = even ? v0 : v1;
-      }
-      if (n < HD) pvt[n] = (T)vuv;
-    }
+    if (n < HD) out[n] = (T)(o[e] * inv);
   }
 }
 
@@ -370,7 +381,7 @@ __global__ __launch_bounds__(kThreads) void decode_flush_kernel(DecodeArgs a) {
 
 template <typename T, int HD> static int launch_decode_t(const DecodeArgs& a, hipStream_t stream) {
   const int BH = a.B * a.H;
-  if (a.t_dev != nullptr || a.t > 0) {
+  {
     ProfScope ps(kSlotDecodeStream, stream);
     if constexpr (__is_same(T, bf16_t)) {
       if (a.u_half) hipLaunchKernelGGL((decode_stream_kernel<T, HD, true>), dim3(a.splits, BH), dim3(kThreads), 0, stream, a);
@@ -476,111 +487,172 @@ int launch_rope(const View4& src, const View4& dst, int B, int H, int L, int d, 
 
 // ---------------------------------------------------------------------------
 // y[M, N] = x[M, K] w[N, K]^T for the few rows of a decode step (M = batch): the two projections
-// around the cached step (lookahead_keys_attention.py:99, 209 with seq_len == 1).  A library GEMM
-// spends most of its ~8 us here on one 32-row tile per workgroup walking K serially; this kernel
-// gives every 32 x 32 output tile to one workgroup of 8 waves that split K, so each wave issues all
-// its operand loads at once (straight from global memory, rows of x and w are K-contiguous, which is
-// the MFMA operand layout), runs a handful of MFMAs and the partial tiles are summed through LDS.
-constexpr int kLinWaves = 8;
+// around the cached step (lookahead_keys_attention.py:99, 209 with seq_len == 1).
+//
+// What bounds it is latency: a launch, one trip to memory for the weights, one reduction.  So every
+// 16-column slice of the output has a workgroup of its own (N = 512 then puts 32 CUs on the weights), its
+// waves split K so finely that all operand loads of a wave are in flight at once (straight from global
+// memory: rows of x and w are K-contiguous, which is the MFMA operand layout), and the partial tiles are
+// summed through LDS.  Against 32-column slices and 8 waves throughout, replayed from a graph, 16 rows: K 2048 ->
+// N 512 8.6 -> 5.6 us, 512 -> 3072 with the norm 5.4 -> 4.0, 512 -> 2048 with norm and GELU 5.1 -> 3.5, 512 -> 512
+// 3.5 -> 2.7 (an empty launch takes about 2).
+//
 // Optional work around the product (all of it per output row, so it costs one pass less each):
 //   norm_w   RMS normalisation of the x rows in front: y = ((x / rms(x)) * norm_w) w^T.  The weight
 //            goes into the operand, the 1 / rms factor (a per-row scalar) onto the accumulated sum;
 //            the sums of squares are collected from the fragments the product loads anyway.
 //   act      1: GELU (erf form) of the sum
 //   res      a tensor of the output's shape added at the end
-template <typename T>
-__global__ __launch_bounds__(64 * kLinWaves) void small_linear_kernel(const T* x, const T* w, T* y, int M, int N, int K,
-                                                                       int64_t ldx, int64_t ldw, int64_t ldy,
-                                                                       const T* norm_w, float eps, int act,
-                                                                       const T* res, int64_t ldr) {
-  static_assert(sizeof(T) == 2, "16-bit operands");
-  constexpr int MAXS = 8;   // 16-deep steps a wave handles per pass
-  __shared__ float red[kLinWaves][32][33];
-  __shared__ float ssq[kLinWaves][32];
-  const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
-  const int n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
-  const int steps = (K + 15) / 16;
-  const int per = (steps + kLinWaves - 1) / kLinWaves;
-  const bool row_ok = m0 + c < M, col_ok = n0 + c < N;
-  const T* xr = x + (int64_t)(m0 + c) * ldx;
-  const T* wr = w + (int64_t)(n0 + c) * ldw;
-  acc_t acc;
-  zero(acc);
-  float sq = 0.f;
-  for (int s0 = wave * per; s0 < min(steps, (wave + 1) * per); s0 += MAXS) {
-    frag<T> fa[MAXS], fb[MAXS];
+struct LinearArgs {
+  const void *x, *w;
+  void* y;
+  int M, N, K;
+  int64_t ldx, ldw, ldy;
+  const void* norm_w;
+  float eps;
+  int act;
+  const void* res;
+  int64_t ldr;
+};
+typedef vec<float, 4> acc4_t;
+__device__ __forceinline__ void mma16(acc4_t& c, const vec<bf16_t, 8>& a, const vec<bf16_t, 8>& b) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ void mma16(acc4_t& c, const vec<fp16_t, 8>& a, const vec<fp16_t, 8>& b) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+// fp32: four 4-deep products; the contraction index of slot e on lane group g is 4 g + e for both operands
+__device__ __forceinline__ void mma16(acc4_t& c, const vec<float, 4>& a, const vec<float, 4>& b) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+}
+
+// MT: 16-row tiles of a workgroup; NT: 16-column tiles; W: waves; lane l holds rows / columns l % 16, contraction piece l / 16
+template <typename T, int MT, int NT, int W>
+__global__ __launch_bounds__(64 * W) void small_linear_kernel(LinearArgs a) {
+  constexpr int V = elem_traits<T>::vec16, DEPTH = 4 * V;   // elements of a 16-byte piece, contraction depth of one step
+  constexpr int MAXS = 4;                                   // steps a wave has in flight
+  typedef vec<T, V> vt;
+  typedef vec<float, V> vf;
+  __shared__ float red[W][16 * MT][16 * NT + 1];
+  __shared__ float ssq[W][16 * MT];
+  const int lane = lane_id(), wave = wave_id(), c = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int steps = (a.K + DEPTH - 1) / DEPTH;
+  const int per = (steps + W - 1) / W;
+  const int s_end = min(steps, (wave + 1) * per);
+  const T* wr = static_cast<const T*>(a.w) + (int64_t)(n0 + c) * a.ldw;
+  const T* norm_w = static_cast<const T*>(a.norm_w);
+  acc4_t acc[MT][NT];
+  float sq[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    sq[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = acc4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int s0 = wave * per; s0 < s_end; s0 += MAXS) {
+    vt fa[MAXS][MT], fb[MAXS][NT], fg[MAXS];
 #pragma unroll
     for (int u = 0; u < MAXS; ++u) {
-      const int kk = 16 * (s0 + u) + 8 * g;
-      const bool in = s0 + u < min(steps, (wave + 1) * per) && kk < K;   // K is a multiple of 8
-      fa[u] = (in && row_ok) ? *reinterpret_cast<const frag_mem<T>*>(xr + kk) : zero_frag<T>();
-      fb[u] = (in && col_ok) ? *reinterpret_cast<const frag_mem<T>*>(wr + kk) : zero_frag<T>();
-      if (norm_w != nullptr) {
-        const frag<T> fg = in ? *reinterpret_cast<const frag_mem<T>*>(norm_w + kk) : zero_frag<T>();
-        const vec<float, 8> xv = __builtin_convertvector(fa[u], vec<float, 8>);
-        const vec<float, 8> gv = __builtin_convertvector(fg, vec<float, 8>);
+      const int kk = DEPTH * (s0 + u) + V * g;
+      const bool in = s0 + u < s_end && kk < a.K;   // K is a multiple of V
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sq = __builtin_fmaf(xv[e], xv[e], sq);
-        fa[u] = __builtin_convertvector(xv * gv, frag<T>);
+      for (int e = 0; e < V; ++e) fg[u][e] = (T)0.f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) fb[u][j][e] = (T)0.f;
+        if (in && n0 + 16 * j + c < a.N) fb[u][j] = *reinterpret_cast<const vt*>(wr + 16 * j * a.ldw + kk);
+      }
+      if (norm_w != nullptr && in) fg[u] = *reinterpret_cast<const vt*>(norm_w + kk);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const int row = m0 + 16 * i + c;
+#pragma unroll
+        for (int e = 0; e < V; ++e) fa[u][i][e] = (T)0.f;
+        if (in && row < a.M) fa[u][i] = *reinterpret_cast<const vt*>(static_cast<const T*>(a.x) + (int64_t)row * a.ldx + kk);
       }
     }
+    if (norm_w != nullptr) {
 #pragma unroll
-    for (int u = 0; u < MAXS; ++u) mma(acc, fa[u], fb[u]);
+      for (int u = 0; u < MAXS; ++u)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const vf xv = __builtin_convertvector(fa[u][i], vf), gv = __builtin_convertvector(fg[u], vf);
+#pragma unroll
+          for (int e = 0; e < V; ++e) sq[i] = __builtin_fmaf(xv[e], xv[e], sq[i]);
+          fa[u][i] = __builtin_convertvector(xv * gv, vt);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < MAXS; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) mma16(acc[i][j], fa[u][i], fb[u][j]);
   }
 #pragma unroll
-  for (int r = 0; r < 16; ++r) red[wave][acc_row(r, g)][c] = acc[r];
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][16 * i + 4 * g + r][16 * j + c] = acc[i][j][r];
   if (norm_w != nullptr) {
-    sq += __shfl_xor(sq, 32);   // the two halves of a row's 16-deep steps
-    if (g == 0) ssq[wave][c] = sq;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {   // the four contraction pieces of a row
+      sq[i] += __shfl_xor(sq[i], 16);
+      sq[i] += __shfl_xor(sq[i], 32);
+      if (g == 0) ssq[wave][16 * i + c] = sq[i];
+    }
   }
   __syncthreads();
-  // 1024 outputs, 512 threads: two neighbouring columns each
-  const int e = 2 * threadIdx.x, row = e / 32, col = e % 32;
-  float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-  for (int v = 0; v < kLinWaves; ++v) { s0 += red[v][row][col]; s1 += red[v][row][col + 1]; }
-  if (norm_w != nullptr) {
-    float t = 0.f;
+  for (int o = threadIdx.x; o < 256 * MT * NT; o += 64 * W) {
+    const int row = o / (16 * NT), col = o % (16 * NT);
+    float s = 0.f;
 #pragma unroll
-    for (int v = 0; v < kLinWaves; ++v) t += ssq[v][row];
-    const float rstd = __builtin_amdgcn_rsqf(t / (float)K + eps);
-    s0 *= rstd;
-    s1 *= rstd;
-  }
-  if (act == 1) {
-    s0 = 0.5f * s0 * (1.f + erff(s0 * 0.70710678f));
-    s1 = 0.5f * s1 * (1.f + erff(s1 * 0.70710678f));
-  }
-  if (m0 + row < M) {
-    T* dst = y + (int64_t)(m0 + row) * ldy + n0 + col;
-    const T* rsrc = res != nullptr ? res + (int64_t)(m0 + row) * ldr + n0 + col : nullptr;
-    if (n0 + col + 1 < N) {
-      if (rsrc != nullptr) {
-        const vec<T, 2> rv = *reinterpret_cast<const vec<T, 2>*>(rsrc);
-        s0 += (float)rv[0];
-        s1 += (float)rv[1];
-      }
-      vec<T, 2> o = {(T)s0, (T)s1};
-      *reinterpret_cast<vec<T, 2>*>(dst) = o;
-    } else if (n0 + col < N) {
-      if (rsrc != nullptr) s0 += (float)rsrc[0];
-      dst[0] = (T)s0;
+    for (int v = 0; v < W; ++v) s += red[v][row][col];
+    if (norm_w != nullptr) {
+      float t = 0.f;
+#pragma unroll
+      for (int v = 0; v < W; ++v) t += ssq[v][row];
+      s *= __builtin_amdgcn_rsqf(t / (float)a.K + a.eps);
+    }
+    if (a.act == 1) s = 0.5f * s * (1.f + erff(s * 0.70710678f));
+    if (m0 + row < a.M && n0 + col < a.N) {
+      if (a.res != nullptr) s += (float)static_cast<const T*>(a.res)[(int64_t)(m0 + row) * a.ldr + n0 + col];
+      static_cast<T*>(a.y)[(int64_t)(m0 + row) * a.ldy + n0 + col] = (T)s;
     }
   }
 }
+
+template <typename T> static void launch_linear_t(const LinearArgs& a, hipStream_t stream) {
+  // 16 waves when K is long enough to give each of them two steps; 32 columns per workgroup once 16 would
+  // put more than one workgroup on a CU (each of them reads all of x)
+  const int mt = a.M > 16 ? 2 : 1, gy = (a.M + 16 * mt - 1) / (16 * mt);
+  const bool wide = a.K >= 16 * 4 * elem_traits<T>::vec16 * 2;
+  const int nt = (int64_t)((a.N + 15) / 16) * gy > 256 ? 2 : 1;
+  const dim3 grid((a.N + 16 * nt - 1) / (16 * nt), gy), block(wide ? 1024 : 512);
+#define CASTLE_LINEAR(MT_, NT_, W_) hipLaunchKernelGGL((small_linear_kernel<T, MT_, NT_, W_>), grid, block, 0, stream, a)
+  if (wide) {
+    if (mt == 1) { if (nt == 1) CASTLE_LINEAR(1, 1, 16); else CASTLE_LINEAR(1, 2, 16); }
+    else { if (nt == 1) CASTLE_LINEAR(2, 1, 16); else CASTLE_LINEAR(2, 2, 16); }
+  } else {
+    if (mt == 1) { if (nt == 1) CASTLE_LINEAR(1, 1, 8); else CASTLE_LINEAR(1, 2, 8); }
+    else { if (nt == 1) CASTLE_LINEAR(2, 1, 8); else CASTLE_LINEAR(2, 2, 8); }
+  }
+#undef CASTLE_LINEAR
+}
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                         int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream) {
-  const dim3 grid((N + 31) / 32, (M + 31) / 32), block(64 * kLinWaves);
-  if (dtype == 1)
-    hipLaunchKernelGGL((small_linear_kernel<bf16_t>), grid, block, 0, stream, static_cast<const bf16_t*>(x),
-                       static_cast<const bf16_t*>(w), static_cast<bf16_t*>(y), M, N, K, ldx, ldw, ldy,
-                       static_cast<const bf16_t*>(norm_w), eps, act, static_cast<const bf16_t*>(res), ldr);
-  else if (dtype == 2)
-    hipLaunchKernelGGL((small_linear_kernel<fp16_t>), grid, block, 0, stream, static_cast<const fp16_t*>(x),
-                       static_cast<const fp16_t*>(w), static_cast<fp16_t*>(y), M, N, K, ldx, ldw, ldy,
-                       static_cast<const fp16_t*>(norm_w), eps, act, static_cast<const fp16_t*>(res), ldr);
-  else
-    return -1;
+  const LinearArgs a = {x, w, y, M, N, K, ldx, ldw, ldy, norm_w, eps, act, res, ldr};
+  switch (dtype) {
+    case 0: launch_linear_t<float>(a, stream); break;
+    case 1: launch_linear_t<bf16_t>(a, stream); break;
+    case 2: launch_linear_t<fp16_t>(a, stream); break;
+    default: return -1;
+  }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -606,15 +678,23 @@ int decode_static_scratch(float** ptr) {
   return 0;
 }
 
-// rows of one (b, h) handled per workgroup iteration, needed by the host to size `splits`
-int decode_pick_splits(int BH, int t) {
+// How many workgroups share the t rows of one (b, h).  Three workgroups fit a CU (137 registers), so a launch runs
+// in rounds of 3 CUs; a workgroup costs its iterations plus about two more for its start and end.  Fewest rounds x
+// iterations wins, at least two iterations each.  45 x 6 heads of 450 rows: 26.1 us with the 2 splits this picks, 27.6
+// with the 3 that fill a round and a straggling 5 % of the next; 16 x 8 heads of 540 rows: 16.6 us with one round,
+// 20.7 with two.
+int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus) {
   if (t <= 0) return 1;
-  int want = (CASTLE_DEC_WGS + BH - 1) / BH;           // 2-3 workgroups per CU: measured 6.3 TB/s at 512-768 workgroups, 6.0 at 2048, 4.5 at 256
-  int max_by_rows = (t + 63) / 64;          // at least 64 rows per workgroup
-  int s = want < max_by_rows ? want : max_by_rows;
-  if (s < 1) s = 1;
-  if (s > 64) s = 64;
-  return s;
+  const int64_t round = 3 * (int64_t)(cus > 0 ? cus : 256);
+  const int most = std::min(64, (t + 2 * rows_per_iteration - 1) / (2 * rows_per_iteration));
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int s = 1; s <= most; ++s) {
+    const int64_t iterations = ((t + s - 1) / s + rows_per_iteration - 1) / rows_per_iteration;
+    const int64_t cost = ((int64_t)BH * s + round - 1) / round * (iterations + 2);
+    if (cost < best_cost) { best_cost = cost; best = s; }
+  }
+  return best;
 }
 
 }  // namespace castle

@@ -375,13 +375,12 @@ variable_list layer_parallel(const Tensor& x, const std::optional<Tensor>& norm_
 }
 
 // ---- the cached single-token step ------------------------------------------------------------------------------
-// (B, 1, K) x (N, K) through the small-M kernel: see castle_small_linear_fused
-bool small_linear_ok(const Tensor& x, const Tensor& w, int64_t max_rows) {
-  return x.is_cuda() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kHalf) && w.scalar_type() == x.scalar_type() &&
-         x.dim() == 3 && x.size(1) == 1 && x.size(0) <= max_rows && x.stride(2) == 1 && w.stride(1) == 1 && x.size(2) % 8 == 0 &&
-         w.size(0) % 2 == 0 && x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0;
+// rows of a matrix that the kernels can read 16 bytes at a time
+bool rows_readable(const Tensor& t) {
+  return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) % (16 / t.element_size()) == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
+
+// (B, 1, K) x (N, K) through the small-M kernel: see castle_small_linear_fused
 Tensor small_linear(const Tensor& x, const Tensor& w, const std::optional<Tensor>& norm_w, double eps, int64_t act,
                     const std::optional<Tensor>& residual) {
   const c10::DeviceGuard guard(x.device());
@@ -407,9 +406,11 @@ class StepPlan {
   }
 
   // proj (B, 1, 6 H d) -> (B, 1, H d) at row count t.  base >= 0: deferred write-back of the lookahead keys from
-  // that row count on (see castle_deferred); base < 0: every step writes them.
-  Tensor attend(const Tensor& proj_, int64_t t, int64_t base, double scale, bool rotary) {
-    TORCH_CHECK_VALUE(t >= 0 && t < s_.L, "cache capacity ", s_.L, " cannot take row ", t);
+  // that row count on (see castle_deferred); base < 0: every step writes them.  With t_device (and base_device) the
+  // row counts are read by the kernels, as a captured graph of the step needs it.
+  Tensor attend(const Tensor& proj_, int64_t t, int64_t base, double scale, bool rotary, const std::optional<Tensor>& t_device,
+                const std::optional<Tensor>& base_device) {
+    check_count(t, t_device);
     const Tensor proj = packed_readable(proj_);
     TORCH_CHECK_VALUE(proj.dim() == 3 && proj.size(0) == s_.B && proj.size(1) == 1 && proj.size(2) == 6LL * s_.H * s_.d &&
                           proj.scalar_type() == buffers_[0].scalar_type() && proj.device() == buffers_[0].device(),
@@ -420,32 +421,69 @@ class StepPlan {
     one.L = 1;
     castle_view4 v[6];
     six_of_packed(proj, one, v);
-    const castle_view4 vo = packed_view(out, one, 1, 0);
-    castle_deferred deferred = deferred_;
-    deferred.base = (int)base;
-    check(castle_decode_step(&views_[0], &views_[1], &views_[2], &views_[3], (int)t, s_.L, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], s_.B,
-                             s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0), &vo,
-                             base >= 0 ? &deferred : nullptr, workspace_.data_ptr(), workspace_.numel(), stream_of(proj)),
+    const castle_view4 vo = packed_view(out, one, 1, 0), *c = views_;
+    castle_deferred def = deferred(base, base_device);
+    const castle_deferred* pd = base >= 0 || base_device ? &def : nullptr;
+    const int flags = flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0);
+    void* ws = workspace_.data_ptr();
+    const int64_t wb = workspace_.numel();
+    check(t_device ? castle_decode_step_device_count(c, c + 1, c + 2, c + 3, count_ptr(t_device), s_.L, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5],
+                                                     s_.B, s_.H, s_.d, s_.dtype, (float)scale, flags, &vo, pd, ws, wb, stream_of(proj))
+                   : castle_decode_step(c, c + 1, c + 2, c + 3, (int)t, s_.L, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], s_.B, s_.H, s_.d,
+                                        s_.dtype, (float)scale, flags, &vo, pd, ws, wb, stream_of(proj)),
           "castle_decode_step");
     return out;
   }
 
-  // the whole layer for one token: x (B, 1, dim) -> (B, 1, dim)
+  // the whole layer for one token: x (B, 1, dim) -> (B, 1, dim), plus `residual` if there is one
   Tensor layer(const Tensor& x, const std::optional<Tensor>& norm_w, std::optional<double> eps, const Tensor& w_qkv, const Tensor& w_out,
-               int64_t max_rows, int64_t t, int64_t base, double scale, bool rotary) {
-    Tensor proj;
-    if (small_linear_ok(x, w_qkv, max_rows) && (!norm_w || (norm_w->scalar_type() == x.scalar_type() && norm_w->is_contiguous()))) {
-      const double e = eps ? *eps : x.scalar_type() == at::kHalf ? 0.0009765625 : 0.0078125;   // F.rms_norm: the type's epsilon
-      proj = small_linear(x, w_qkv, norm_w, e, CASTLE_ACT_NONE, std::nullopt);
-    } else {
-      proj = at::linear(norm_w ? at::rms_norm(x, {x.size(2)}, norm_w, eps) : x, w_qkv);
+               int64_t max_rows, int64_t t, int64_t base, double scale, bool rotary, const std::optional<Tensor>& residual,
+               const std::optional<Tensor>& t_device, const std::optional<Tensor>& base_device) {
+    const int64_t B = s_.B, dim = x.size(-1), inner = (int64_t)s_.H * s_.d;
+    const c10::DeviceGuard guard(x.device());
+    check_count(t, t_device);
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(0) == B && x.size(1) == 1 && w_qkv.dim() == 2 && w_qkv.size(0) == 6 * inner && w_qkv.size(1) == dim &&
+                          w_out.dim() == 2 && w_out.size(1) == inner && x.scalar_type() == buffers_[0].scalar_type() && x.device() == buffers_[0].device(),
+                      "the token or the weights do not belong to this cache");
+    if (B > max_rows || w_out.size(0) != dim || !rows_readable(w_qkv) || !rows_readable(w_out)) {
+      const Tensor proj = at::linear(norm_w ? at::rms_norm(x, {dim}, norm_w, eps) : x, w_qkv);
+      const Tensor y = at::linear(attend(proj, t, base, scale, rotary, t_device, base_device), w_out);
+      return residual ? *residual + y : y;
     }
-    const Tensor merged = attend(proj, t, base, scale, rotary);
-    if (small_linear_ok(merged, w_out, max_rows)) return small_linear(merged, w_out, std::nullopt, 0., CASTLE_ACT_NONE, std::nullopt);
-    return at::linear(merged, w_out);
+    const Tensor xr = rows_readable(x.select(1, 0)) ? x : x.contiguous();
+    const Tensor nw = norm_w ? norm_w->contiguous() : Tensor();
+    const Tensor res = residual ? (residual->stride(2) == 1 ? *residual : residual->contiguous()) : Tensor();
+    // F.rms_norm without an eps takes the type's machine epsilon
+    const double e = eps ? *eps : x.scalar_type() == at::kHalf ? 0.0009765625 : x.scalar_type() == at::kBFloat16 ? 0.0078125 : 1.1920928955078125e-07;
+    Tensor proj = at::empty({B, 6 * inner}, x.options()), y = at::empty({B, 1, dim}, x.options());
+    const castle_view4* c = views_;
+    castle_deferred def = deferred(base, base_device);
+    check(castle_decode_layer(c, c + 1, c + 2, c + 3, (int)t, t_device ? count_ptr(t_device) : nullptr, s_.L, xr.data_ptr(), xr.stride(0), (int)dim,
+                              nw.defined() ? nw.data_ptr() : nullptr, (float)e, w_qkv.data_ptr(), w_qkv.stride(0), w_out.data_ptr(),
+                              w_out.stride(0), res.defined() ? res.data_ptr() : nullptr, res.defined() ? res.stride(0) : 0, y.data_ptr(), dim,
+                              proj.data_ptr(), s_.B, s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0),
+                              base >= 0 || base_device ? &def : nullptr, workspace_.data_ptr(), workspace_.numel(), stream_of(x)),
+          "castle_decode_layer");
+    return y;
   }
 
  private:
+  static const int32_t* count_ptr(const std::optional<Tensor>& t) { return static_cast<const int32_t*>(t->data_ptr()); }
+  void check_count(int64_t t, const std::optional<Tensor>& t_device) const {
+    if (t_device) {
+      TORCH_CHECK_VALUE(t_device->scalar_type() == at::kInt && t_device->numel() == 1 && t_device->device() == buffers_[0].device(),
+                        "t_device must be a one-element int32 tensor on the GPU of the step");
+      return;
+    }
+    TORCH_CHECK_VALUE(t >= 0 && t < s_.L, "cache capacity ", s_.L, " cannot take row ", t);
+  }
+  castle_deferred deferred(int64_t base, const std::optional<Tensor>& base_device) const {
+    castle_deferred r = deferred_;
+    r.base = (int)std::max<int64_t>(base, 0);
+    r.base_device = base_device ? count_ptr(base_device) : nullptr;
+    return r;
+  }
+
   std::vector<Tensor> buffers_;
   Tensor ring_, gates_, workspace_;
   castle_view4 views_[4];

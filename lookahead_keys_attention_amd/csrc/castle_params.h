@@ -110,7 +110,7 @@ struct DecodeArgs {
   View4 U, qu_cache, kc_cache, vc_cache;   // capacity buffers, row t is appended
   View4 qc, kc, vc, qu, ku, vu;            // new token, L == 1
   View4 out;                               // (B, H, 1, d)
-  float* part;      // [B*H][splits][d + 2]  partial (acc, m, l)
+  float* part;      // partial results: sums [B*H][splits][d], then statistics [B*H][splits][2] (maximum, sum of weights)
   // deferred write-back (pend_ku.ptr == nullptr: U is written every step)
   View4 pend_vu;            // (B, H, kDecodeDefer, d): row j % kDecodeDefer holds vu of token j (rotated when rotary)
   View4 pend_gate;          // (B, H, capacity, kDecodeDefer) fp32: [k][j % kDecodeDefer] = gate of row k for pending token j
