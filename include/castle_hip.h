@@ -261,6 +261,17 @@ int castle_small_linear_fused(const void* x, const void* w, void* y, int M, int 
                               const void* norm_weight, float eps, int activation,
                               const void* residual, int64_t ldr, void* stream);
 
+/* One token per row from its logits (train_triton.py:56-71): the k largest of `vocabulary` logits are kept (of
+ * equal ones the lowest indices), and the arg-max of  logit * inv_temperature - log(-log(uniform))  over them is
+ * written (both logarithms' arguments at least 1e-20); uniform: (rows, vocabulary) contiguous, or NULL for the arg-max of
+ * the logits.  token: row r goes to token[r * token_ld]; token_copy: NULL, or a second copy, contiguous. */
+int castle_sample(const void* logits, int64_t ld, const float* uniform, int rows, int vocabulary, int k, float inv_temperature,
+                  int64_t* token, int64_t token_ld, int64_t* token_copy, int dtype, void* stream);
+
+/* y[m] = table[index[m]], m < n: rows of `width` elements (whole 16-byte pieces), y contiguous.  An index outside
+ * 0 .. table_rows - 1 gives a row of zeros.  The token embedding of a step (train_triton.py:86). */
+int castle_gather_rows(const void* table, int64_t table_rows, int64_t ld, int width, const int64_t* index, int n, void* y, int dtype, void* stream);
+
 /* Per-kernel timing (no counterpart in the reference; for benchmarks).  While enabled, every
  * kernel launched by the entry points above is bracketed by a HIP event pair on its stream.
  * castle_profile_enable(on) also discards pending records.  castle_profile_read waits for the

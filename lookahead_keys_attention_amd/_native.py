@@ -44,6 +44,8 @@ EXPORTED_SYMBOLS = (
     "castle_decode_layer",
     "castle_rope",
     "castle_small_linear",
+    "castle_sample",
+    "castle_gather_rows",
     "castle_small_linear_fused",
     "castle_profile_enable",
     "castle_profile_read",

@@ -20,6 +20,9 @@ int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus);
 int decode_static_scratch(float** ptr);
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                         int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream);
+int launch_sample(const void* logits, int64_t ld, const float* u, int rows, int V, int k, float inv_temperature, int64_t* out, int64_t out_ld,
+                  int64_t* out2, int dtype, hipStream_t stream);
+int launch_gather_rows(const void* table, int64_t row_bytes, int64_t ld_bytes, int64_t rows, const int64_t* index, int n, void* y, hipStream_t stream);
 }  // namespace castle
 
 namespace {
@@ -475,6 +478,27 @@ int castle_small_linear_fused(const void* x, const void* w, void* y, int M, int 
 int castle_small_linear(const void* x, const void* w, void* y, int M, int N, int K,
                         int64_t ldx, int64_t ldw, int64_t ldy, int dtype, void* stream) {
   return castle_small_linear_fused(x, w, y, M, N, K, ldx, ldw, ldy, dtype, nullptr, 0.f, CASTLE_ACT_NONE, nullptr, 0, stream);
+}
+
+int castle_sample(const void* logits, int64_t ld, const float* uniform, int rows, int vocabulary, int k, float inv_temperature,
+                  int64_t* token, int64_t token_ld, int64_t* token_copy, int dtype, void* stream) {
+  if (elem_size(dtype) == 0) return CASTLE_ERR_DTYPE;
+  if (rows <= 0 || vocabulary <= 0 || k <= 0 || k > vocabulary) return CASTLE_ERR_SHAPE;
+  if (logits == nullptr || token == nullptr || reinterpret_cast<uintptr_t>(token) % 8 != 0 || reinterpret_cast<uintptr_t>(token_copy) % 8 != 0 ||
+      reinterpret_cast<uintptr_t>(uniform) % 4 != 0)
+    return CASTLE_ERR_ARG;
+  return castle::launch_sample(logits, ld, uniform, rows, vocabulary, k, inv_temperature, token, token_ld, token_copy, dtype,
+                               static_cast<hipStream_t>(stream));
+}
+
+int castle_gather_rows(const void* table, int64_t table_rows, int64_t ld, int width, const int64_t* index, int n, void* y, int dtype, void* stream) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (table_rows <= 0 || width <= 0 || n <= 0 || (int64_t)width * es % 16 != 0) return CASTLE_ERR_SHAPE;
+  if (table == nullptr || index == nullptr || y == nullptr || reinterpret_cast<uintptr_t>(table) % 16 != 0 || reinterpret_cast<uintptr_t>(y) % 16 != 0 ||
+      ld * es % 16 != 0 || reinterpret_cast<uintptr_t>(index) % 8 != 0)
+    return CASTLE_ERR_ARG;
+  return castle::launch_gather_rows(table, (int64_t)width * es, ld * es, table_rows, index, n, y, static_cast<hipStream_t>(stream));
 }
 
 int castle_profile_enable(int on) { return castle::profile_enable(on); }

@@ -657,6 +657,153 @@ int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int
 }
 
 // ---------------------------------------------------------------------------
+// One token per row from its logits (train_triton.py:56-71): keep the k largest, divide by the temperature, add
+// Gumbel noise formed from the uniform numbers `u`, take the arg-max.  As separate operators (a radix top-k, its sort, a
+// scatter, twice clamp / log / negate, add, arg-max) this is 15 launches and ~100 us per token around a model step of
+// ~400; here one workgroup per row finds the k-th largest value by a radix select over the row (4 rounds of 256 bins,
+// the row stays in L2) and takes the arg-max of what is at or above it in the same launch.
+constexpr int kSampleThreads = 512;
+struct SampleArgs {
+  const void* logits;
+  int64_t ld;
+  const float* u;   // [rows][V] uniform numbers; nullptr: no noise (arg-max)
+  int V, k;
+  float inv_temperature;
+  int64_t *out, out_ld;   // one token per row
+  int64_t* out2;          // optional second copy, contiguous
+};
+// order-preserving map of a float to an unsigned integer; NaN above everything
+__device__ __forceinline__ uint32_t float_order(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  return x == x ? b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u) : 0xffffffffu;
+}
+template <typename T>
+__global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleArgs a) {
+  constexpr int NW = kSampleThreads / 64;
+  __shared__ int hist[256];
+  __shared__ int s_bin, s_left, s_taken;
+  __shared__ int s_wave[NW];
+  __shared__ float s_best[NW];
+  __shared__ int s_arg[NW];
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const T* x = static_cast<const T*>(a.logits) + (int64_t)row * a.ld;
+  // the k-th largest value: digit by digit from the top, `left` of the values with the digits found so far wanted
+  uint32_t prefix = 0, mask = 0;
+  int left = a.k;
+  for (int shift = 24; shift >= 0; shift -= 8) {
+    for (int i = tid; i < 256; i += kSampleThreads) hist[i] = 0;
+    __syncthreads();
+    for (int i = tid; i < a.V; i += kSampleThreads) {
+      const uint32_t o = float_order((float)x[i]);
+      if ((o & mask) == prefix) atomicAdd(&hist[(o >> shift) & 255], 1);
+    }
+    __syncthreads();
+    if (wave == 0) {   // suffix sums of the 256 bins, four per lane, from the highest bin down
+      int h[4], sum = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { h[e] = hist[255 - (4 * lane + e)]; sum += h[e]; }
+      int above = sum;   // inclusive scan over lanes
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(above, o);
+        if (lane >= o) above += y;
+      }
+      above -= sum;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (above < left && above + h[e] >= left) { s_bin = 255 - (4 * lane + e); s_left = left - above; }
+        above += h[e];
+      }
+    }
+    __syncthreads();
+    prefix |= (uint32_t)s_bin << shift;
+    mask |= 255u << shift;
+    left = s_left;
+    __syncthreads();
+  }
+  // values above the k-th are kept, and the first `left` (in index order) of those equal to it
+  float best = -INFINITY;
+  int arg = 0x7fffffff;
+  if (tid == 0) s_taken = 0;
+  __syncthreads();
+  for (int base = 0; base < a.V; base += kSampleThreads) {
+    const int i = base + tid;
+    float v = 0.f;
+    uint32_t o = 0;
+    if (i < a.V) {
+      v = (float)x[i];
+      o = float_order(v);
+    }
+    const bool equal = i < a.V && o == prefix;
+    const unsigned long long ballot = __builtin_amdgcn_ballot_w64(equal);
+    if (lane == 0) s_wave[wave] = __builtin_popcountll(ballot);
+    __syncthreads();
+    int before = s_taken + __builtin_popcountll(ballot & ((1ull << lane) - 1));
+    for (int w = 0; w < wave; ++w) before += s_wave[w];
+    if (i < a.V && (o > prefix || (equal && before < left))) {
+      float z = v;
+      if (a.u != nullptr) {
+        const float e = -logf(fmaxf(a.u[(int64_t)row * a.V + i], 1e-20f));
+        z = v * a.inv_temperature - logf(fmaxf(e, 1e-20f));
+      }
+      if (arg == 0x7fffffff || z > best || (z != z && best == best)) { best = z; arg = i; }
+    }
+    __syncthreads();
+    if (tid == 0) {
+      int n = 0;
+      for (int w = 0; w < NW; ++w) n += s_wave[w];
+      s_taken += n;
+    }
+    __syncthreads();
+  }
+  // the largest, the lowest index among equals; a NaN counts as the largest
+  auto better = [](float v, int i, float w, int j) { return i != 0x7fffffff && (j == 0x7fffffff || (v != v ? !(w != w) || i < j : w == w && (v > w || (v == w && i < j)))); };
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float ob = __shfl_xor(best, o);
+    const int oa = __shfl_xor(arg, o);
+    if (better(ob, oa, best, arg)) { best = ob; arg = oa; }
+  }
+  if (lane == 0) { s_best[wave] = best; s_arg[wave] = arg; }
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < NW; ++w)
+      if (better(s_best[w], s_arg[w], best, arg)) { best = s_best[w]; arg = s_arg[w]; }
+    a.out[(int64_t)row * a.out_ld] = arg;
+    if (a.out2 != nullptr) a.out2[row] = arg;
+  }
+}
+
+int launch_sample(const void* logits, int64_t ld, const float* u, int rows, int V, int k, float inv_temperature, int64_t* out, int64_t out_ld,
+                  int64_t* out2, int dtype, hipStream_t stream) {
+  const SampleArgs a = {logits, ld, u, V, k, inv_temperature, out, out_ld, out2};
+  const dim3 grid(rows), block(kSampleThreads);
+  switch (dtype) {
+    case 0: hipLaunchKernelGGL((sample_kernel<float>), grid, block, 0, stream, a); break;
+    case 1: hipLaunchKernelGGL((sample_kernel<bf16_t>), grid, block, 0, stream, a); break;
+    case 2: hipLaunchKernelGGL((sample_kernel<fp16_t>), grid, block, 0, stream, a); break;
+    default: return -1;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+// y[m] = table[index[m]]: the embedding of one token per row.  One workgroup per row, 16 bytes per thread (the
+// library's gather takes 9.7 us for 16 rows of 512, this a launch).  An index outside the table writes zeros.
+__global__ __launch_bounds__(kThreads) void gather_rows_kernel(const char* table, int64_t row_bytes, int64_t ld_bytes, int64_t rows, const int64_t* index, char* y) {
+  const int64_t i = index[blockIdx.x];
+  for (int64_t o = 16 * threadIdx.x; o < row_bytes; o += 16 * kThreads) {
+    vec<float, 4> v = {0.f, 0.f, 0.f, 0.f};
+    if (i >= 0 && i < rows) v = *reinterpret_cast<const vec<float, 4>*>(table + i * ld_bytes + o);
+    *reinterpret_cast<vec<float, 4>*>(y + blockIdx.x * row_bytes + o) = v;
+  }
+}
+int launch_gather_rows(const void* table, int64_t row_bytes, int64_t ld_bytes, int64_t rows, const int64_t* index, int n, void* y, hipStream_t stream) {
+  hipLaunchKernelGGL(gather_rows_kernel, dim3(n), dim3(kThreads), 0, stream, static_cast<const char*>(table), row_bytes, ld_bytes, rows, index,
+                     static_cast<char*>(y));
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+// ---------------------------------------------------------------------------
 // Partial-result buffer of the entry point that allocates nothing: one array per GPU, part of the
 // loaded code object, alive until the process ends.  Host code never uses the array's name as an
 // address (on the host it is only a stand-in for the symbol): the device address is looked up

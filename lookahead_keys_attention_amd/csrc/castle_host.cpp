@@ -393,6 +393,33 @@ Tensor small_linear(const Tensor& x, const Tensor& w, const std::optional<Tensor
   return y;
 }
 
+// logits (B, V) -> one token per row into `token` (B,) (any stride) and, if given, `copy` (B,) contiguous
+void sample_tokens(const Tensor& logits, const std::optional<Tensor>& uniform, int64_t k, double temperature, const Tensor& token,
+                   const std::optional<Tensor>& copy) {
+  const c10::DeviceGuard guard(logits.device());
+  TORCH_CHECK_VALUE(logits.is_cuda() && logits.dim() == 2 && logits.stride(1) == 1 && token.scalar_type() == at::kLong && token.dim() == 1 &&
+                        token.size(0) == logits.size(0) && token.device() == logits.device(), "sample_tokens: unexpected logits or token tensor");
+  TORCH_CHECK_VALUE(!uniform || (uniform->is_contiguous() && uniform->scalar_type() == at::kFloat && uniform->sizes() == logits.sizes()),
+                    "sample_tokens: unexpected uniform numbers");
+  TORCH_CHECK_VALUE(!copy || (copy->is_contiguous() && copy->scalar_type() == at::kLong && copy->numel() == logits.size(0)),
+                    "sample_tokens: unexpected copy");
+  check(castle_sample(logits.data_ptr(), logits.stride(0), uniform ? static_cast<const float*>(uniform->data_ptr()) : nullptr,
+                      (int)logits.size(0), (int)logits.size(1), (int)k, 1.f / (float)temperature, static_cast<int64_t*>(token.data_ptr()),
+                      token.stride(0), copy ? static_cast<int64_t*>(copy->data_ptr()) : nullptr, dtype_code(logits), stream_of(logits)),
+        "castle_sample");
+}
+
+// embedding of one token per row: (V, K) table, (B, 1) tokens -> (B, 1, K)
+Tensor gather_rows(const Tensor& table, const Tensor& index) {
+  const c10::DeviceGuard guard(table.device());
+  if (!rows_readable(table) || table.size(1) % (16 / table.element_size()) != 0 || !index.is_contiguous()) return at::embedding(table, index);
+  Tensor y = at::empty({index.size(0), 1, table.size(1)}, table.options());
+  check(castle_gather_rows(table.data_ptr(), table.size(0), table.stride(0), (int)table.size(1), static_cast<const int64_t*>(index.data_ptr()),
+                           (int)index.numel(), y.data_ptr(), dtype_code(table), stream_of(table)),
+        "castle_gather_rows");
+  return y;
+}
+
 // The capacity buffers of one decode cache with everything a step needs to know about them
 class StepPlan {
  public:
@@ -528,6 +555,8 @@ PYBIND11_MODULE(_castle_host, m) {
   using unlocked = py::call_guard<py::gil_scoped_release>;
   m.def("layer_parallel", &layer_parallel, unlocked());
   m.def("small_linear", &small_linear, unlocked());
+  m.def("sample_tokens", &sample_tokens, unlocked());
+  m.def("gather_rows", &gather_rows, unlocked());
   py::class_<StepPlan>(m, "StepPlan")
       .def(py::init<std::vector<Tensor>, Tensor, Tensor, Tensor, bool>())
       .def("attend", &StepPlan::attend, unlocked())

@@ -141,7 +141,9 @@ class GraphedDecoder:
 
     def _step(self):
         model = self.model
-        h = model.token_emb(self.token)
+        embedding = model.token_emb
+        plain = type(embedding) is nn.Embedding and embedding.max_norm is None and not embedding._forward_hooks and not embedding._forward_pre_hooks
+        h = _native.host().gather_rows(embedding.weight, self.token) if plain else embedding(self.token)
         for (attention, feed_forward), store in zip(model.layers, self.stores):
             h = attention.graph_step(h, store, self.t_device, self.base_device, residual=h)
             h = token_feed_forward(feed_forward, h)
@@ -152,7 +154,8 @@ class GraphedDecoder:
         position: a view of the graph's output buffer, overwritten by the next call."""
         if self.length >= self.capacity:
             raise RuntimeError(f"the graph was captured for caches of {self.capacity} rows")
-        self.token.copy_(token)
+        if token is not self.token:   # (whoever wrote the token into the graph's own input hands that in)
+            self.token.copy_(token)
         self.graph.replay()
         self.length += 1
         return self.logits
@@ -247,20 +250,44 @@ class CastleLM(nn.Module):
         elif graph and not self._native_on_gpu(prompt.device):
             raise RuntimeError("graph=True needs the native kernels on a GPU")
 
+        if self._native_on_gpu(prompt.device):
+            return self._sample_native(prompt, steps, seq_len, temperature, filter_thres, generator, graph)
+
         def pick(logits):
             logits = top_k(logits[:, -1].float(), thres=filter_thres)
             if temperature == 0:
                 return logits.argmax(dim=-1, keepdim=True)
             return gumbel_sample(logits, temperature=temperature, generator=generator)
 
-        out, cache, decoder = prompt, None, None
+        out, cache = prompt, None
         for _ in range(steps):
-            if decoder is not None:
-                logits = decoder.step(out[:, -1:])
-            else:
-                step_input = out if cache is None else out[:, -1:]
-                logits, cache = self.forward(step_input, cache=cache, return_next_cache=True)
-                if graph:
-                    decoder = self._decoder_for(cache, seq_len)
+            logits, cache = self.forward(out if cache is None else out[:, -1:], cache=cache, return_next_cache=True)
             out = torch.cat((out, pick(logits)), dim=-1)
         return out[..., prompt_len:]
+
+    def _sample_native(self, prompt, steps, seq_len, temperature, filter_thres, generator, graph):
+        """`sample` with the native kernels: top-k, noise and arg-max of a token are one launch behind the
+        uniform numbers, which come from the generator exactly as `gumbel_noise` draws them; the token
+        goes straight into the graph's input."""
+        host, decoder, cache = _native.host(), None, None
+        batch = prompt.shape[0]
+        tokens = torch.empty((batch, steps), dtype=torch.long, device=prompt.device)
+        for i in range(steps):
+            if decoder is not None:
+                logits = decoder.step(decoder.token)
+            else:
+                logits, cache = self.forward(prompt if cache is None else tokens[:, i - 1:i], cache=cache, return_next_cache=True)
+                if graph:
+                    decoder = self._decoder_for(cache, seq_len)
+            logits = logits[:, -1] if logits.dtype in _native.DTYPE_CODES else logits[:, -1].float()
+            k = math.ceil((1.0 - filter_thres) * logits.shape[-1])
+            uniform = None
+            if temperature != 0:
+                uniform = torch.rand(logits.shape, dtype=torch.float32, device=logits.device, generator=generator)
+            if k < 1:   # nothing is kept: the arg-max over equal values, as the operators would have it
+                tokens[:, i] = 0
+                if decoder is not None:
+                    decoder.token.zero_()
+                continue
+            host.sample_tokens(logits, uniform, k, max(temperature, 1e-10), tokens[:, i], decoder.token if decoder is not None else None)
+        return tokens

@@ -427,6 +427,37 @@ def test_small_linear_with_norm_activation_and_residual(M, N, K, dtype, norm, ac
         assert (y.float() - mods.float()).abs().max() <= 3e-2 * max(mods.float().abs().max().item(), 1.0)
 
 
+@pytest.mark.parametrize("B,dim,Hh,d,t,dtype", [(1, 96, 1, 16, 0, torch.float32), (3, 200, 2, 32, 65, torch.bfloat16), (16, 512, 8, 64, 130, torch.float16),
+                                                (17, 264, 3, 128, 33, torch.bfloat16), (33, 1100, 3, 64, 127, torch.float32)])
+def test_layer_step_equals_its_parts(B, dim, Hh, d, t, dtype):
+    """castle_decode_layer (norm, projection, cached step, projection, residual) against the operators around
+    castle_decode_step: edges of its 16-row and 16-column tiles, ragged K, an empty cache."""
+    from lookahead_keys_attention_amd.castle import _CacheStore
+
+    g = torch.Generator(device=DEV).manual_seed(B + dim)
+    rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
+    x, norm_w = rnd(B, 1, dim), 1 + rnd(dim, std=0.2)
+    w_in, w_out, res = rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5), rnd(B, 1, dim)
+    stores = []
+    for _ in range(2):
+        store = _CacheStore(B, Hh, d, t + 9, dtype, torch.device(DEV))
+        for buf in store.buffers:
+            buf.zero_()
+        stores.append(store)
+    for i in range(4):
+        rows = rnd(B, Hh, t, d, std=0.6)
+        for store in stores:
+            store.buffers[i][:, :, :t] = rows.to(torch.float16).view(dtype) if i == 0 and store.u_half else rows
+    got = stores[0].plan.layer(x, norm_w, 1e-5, w_in, w_out, 64, t, t, d ** -0.5, True, res, None, None)
+    proj = torch.nn.functional.linear(torch.nn.functional.rms_norm(x.float(), (dim,), norm_w.float(), 1e-5).to(dtype), w_in)
+    core = stores[1].plan.attend(proj, t, t, d ** -0.5, True, None, None)
+    want = res.float() + torch.nn.functional.linear(core.float(), w_out.float())
+    assert_close(got, want.cpu().double(), dtype, "layer step", 1e-4)
+    assert torch.all(stores[0].buffers[0][:, :, t] == 0)
+    for a, b in zip(stores[0].buffers[1:], stores[1].buffers[1:]):
+        assert_close(a[:, :, t:t + 1].float(), b[:, :, t:t + 1].float().cpu().double(), dtype, "appended row", 1e-4)
+
+
 @pytest.mark.parametrize("B,Hh,t0,steps,d,dtype,rotary", [(2, 2, 0, 23, 64, torch.float32, False), (1, 2, 101, 18, 32, torch.float32, True),
                                                         (2, 2, 203, 21, 64, torch.bfloat16, False), (1, 2, 130, 9, 128, torch.bfloat16, True)])
 def test_decode_with_deferred_write_back(B, Hh, t0, steps, d, dtype, rotary):

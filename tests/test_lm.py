@@ -235,6 +235,30 @@ def test_graphed_decode_replays_match_eager_steps(dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("vocabulary,dtype", [(1, torch.float32), (255, torch.bfloat16), (512, torch.float32), (513, torch.float16), (5003, torch.bfloat16)])
+def test_sampling_kernel_picks_what_the_operators_pick(vocabulary, dtype):
+    """castle_sample against top_k + gumbel_sample with the same uniform numbers; 16-bit logits have many equal
+    values, so ties at the k-th largest occur (of equal ones the lowest indices are kept)."""
+    from lookahead_keys_attention_amd import _native
+
+    g = torch.Generator(device="cuda").manual_seed(vocabulary)
+    logits = torch.randn(7, vocabulary, device="cuda", generator=g).to(dtype)
+    for k in sorted({1, (vocabulary + 9) // 10, vocabulary}):
+        for temperature in (0.0, 0.7):
+            x = logits.float()
+            order = x.sort(dim=-1, descending=True, stable=True)
+            kept = torch.full_like(x, float("-inf")).scatter_(-1, order.indices[:, :k], order.values[:, :k])
+            u = torch.rand(x.shape, device="cuda", generator=g) if temperature else None
+            if temperature:
+                noise = -(-u.clamp(min=1e-20).log()).clamp(min=1e-20).log()
+                kept = kept / temperature + noise
+            out, copy = torch.full((7, 3), -1, device="cuda"), torch.full((7, 1), -1, device="cuda")
+            _native.host().sample_tokens(logits, u, k, max(temperature, 1e-10), out[:, 1], copy)
+            assert torch.equal(out[:, 1], kept.argmax(dim=-1)) and torch.equal(copy[:, 0], out[:, 1])
+            assert torch.all(out[:, 0] == -1) and torch.all(out[:, 2] == -1)
+
+
+@pytest.mark.gpu
 def test_sampler_reuses_its_captured_graph_for_a_new_prompt():
     model = make_lm(depth=2, dim=128, heads=2, dim_head=64, rotary=True, native=True).cuda()
     first = model.sample(tokens(2, 30, seed=3).cuda(), seq_len=50, temperature=0.0, graph=True)
