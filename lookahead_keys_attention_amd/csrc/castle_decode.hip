@@ -109,10 +109,54 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
   const int pbase = deferred ? decode_base(base0, t) : t;
   const int np = t - pbase;                                        // 0 .. kDecodeDefer - 1
   const bool write_u = !deferred || (t + 1) % kDecodeDefer == 0;
-  float ku[V], vu[V], qc[V];
-  load_f32<T, V>(view_row<T>(a.ku, b, h, 0) + sub * V, ku);
-  load_f32<T, V>(view_row<T>(a.vu, b, h, 0) + sub * V, vu);
-  load_f32<T, V>(view_row<T>(a.qc, b, h, 0) + sub * V, qc);
+  // All loads of the start go out together, the small ones first (they are waited for first): the token's pieces, the
+  // pending tokens' vu pieces, the rows of the first iteration.
+  const vt tku = *reinterpret_cast<const vt*>(view_row<T>(a.ku, b, h, 0) + sub * V);
+  const vt tvu = *reinterpret_cast<const vt*>(view_row<T>(a.vu, b, h, 0) + sub * V);
+  const vt tqc = *reinterpret_cast<const vt*>(view_row<T>(a.qc, b, h, 0) + sub * V);
+  const bool owner = split == (t > 0 ? (t - 1) / per : 0);
+  vt tkc, tqu, tvc, tpv[kDecodeDefer];
+  if (owner) {
+    tkc = *reinterpret_cast<const vt*>(view_row<T>(a.kc, b, h, 0) + sub * V);
+    tqu = *reinterpret_cast<const vt*>(view_row<T>(a.qu, b, h, 0) + sub * V);
+    tvc = *reinterpret_cast<const vt*>(view_row<T>(a.vc, b, h, 0) + sub * V);
+  }
+#pragma unroll
+  for (int sl = 0; sl < kDecodeDefer; ++sl) {
+    const int j = pbase + ((sl - pbase % kDecodeDefer + kDecodeDefer) % kDecodeDefer);   // the token that would sit in this slot
+#pragma unroll
+    for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
+    if (deferred && j < t) tpv[sl] = *reinterpret_cast<const vt*>(view_row<T>(a.pend_vu, b, h, sl) + sub * V);
+  }
+  // The row pieces of the next PF iterations are requested before the current one is processed:
+  // PF + 1 times the bytes in flight per wave, which is what a latency-bound streaming loop is short of.
+  constexpr int PF = 1;
+  vt nq[PF], nu[PF], nk[PF], nv[PF];
+  vec<float, 4> ng[PF];
+#pragma unroll
+  for (int p = 0; p < PF; ++p) ng[p] = vec<float, 4>{0.f, 0.f, 0.f, 0.f};
+  float* const gbase = deferred ? reinterpret_cast<float*>(a.pend_gate.ptr) + (int64_t)b * a.pend_gate.sb + (int64_t)h * a.pend_gate.sh : nullptr;
+  auto request = [&](int p, int k) __attribute__((always_inline)) {
+    if (k < r1) {
+      nq[p] = *reinterpret_cast<const vt*>(view_row<T>(a.qu_cache, b, h, k) + sub * V);
+      nu[p] = *reinterpret_cast<const vt*>(view_row<T>(a.U, b, h, k) + sub * V);
+      nk[p] = *reinterpret_cast<const vt*>(view_row<T>(a.kc_cache, b, h, k) + sub * V);
+      nv[p] = *reinterpret_cast<const vt*>(view_row<T>(a.vc_cache, b, h, k) + sub * V);
+      if (np > 0) ng[p] = *reinterpret_cast<const vec<float, 4>*>(gbase + (int64_t)k * kDecodeDefer);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < PF; ++p) request(p, r0 + grp + p * RPI);
+  __builtin_amdgcn_sched_barrier(0);
+  float ku[V], vu[V], qc[V], pv[kDecodeDefer][V];   // pv by ring slot: zero where no pending token sits
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+    ku[e] = (float)tku[e];
+    vu[e] = (float)tvu[e];
+    qc[e] = (float)tqc[e];
+#pragma unroll
+    for (int sl = 0; sl < kDecodeDefer; ++sl) pv[sl][e] = (float)tpv[sl][e];
+  }
   if (a.rotary) {   // the new token sits at position t
 #pragma unroll
     for (int e = 0; e < V / 2; ++e) {
@@ -121,16 +165,6 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
       CASTLE_ROPE_PAIR(vu[2 * e], vu[2 * e + 1], (float)t, pair, HD, false);
       CASTLE_ROPE_PAIR(qc[2 * e], qc[2 * e + 1], (float)t, pair, HD, false);
     }
-  }
-
-  // the pending tokens' vu pieces of this lane
-  float pv[kDecodeDefer][V];   // indexed by ring slot; zero where no pending token sits
-#pragma unroll
-  for (int sl = 0; sl < kDecodeDefer; ++sl) {
-#pragma unroll
-    for (int e = 0; e < V; ++e) pv[sl][e] = 0.f;
-    const int j = pbase + ((sl - pbase % kDecodeDefer + kDecodeDefer) % kDecodeDefer);   // the token that would sit in this slot
-    if (deferred && j < t) load_f32<T, V>(view_row<T>(a.pend_vu, b, h, sl) + sub * V, pv[sl]);
   }
   const int slot_t = t % kDecodeDefer;
 
@@ -141,11 +175,10 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
 
   // The last split that has rows takes row t too: U_t = 0, so its lookahead term is silu(0) = 0, and appends the
   // new rows.  No workgroup of this launch reads row t or the ring slot of token t.
-  if (split == (t > 0 ? (t - 1) / per : 0) && grp == 0) {
+  if (owner && grp == 0) {
     float kct[V], qut[V];
-    load_f32<T, V>(view_row<T>(a.kc, b, h, 0) + sub * V, kct);
-    load_f32<T, V>(view_row<T>(a.qu, b, h, 0) + sub * V, qut);
-    load_f32<T, V>(view_row<T>(a.vc, b, h, 0) + sub * V, acc);
+#pragma unroll
+    for (int e = 0; e < V; ++e) { kct[e] = (float)tkc[e]; qut[e] = (float)tqu[e]; acc[e] = (float)tvc[e]; }
     if (a.rotary) {
 #pragma unroll
       for (int e = 0; e < V / 2; ++e) {
@@ -171,25 +204,6 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
     }
   }
 
-  // The row pieces of the next PF iterations are requested before the current one is processed:
-  // PF + 1 times the bytes in flight per wave, which is what a latency-bound streaming loop is short of.
-  constexpr int PF = 1;
-  vt nq[PF], nu[PF], nk[PF], nv[PF];
-  vec<float, 4> ng[PF];
-#pragma unroll
-  for (int p = 0; p < PF; ++p) ng[p] = vec<float, 4>{0.f, 0.f, 0.f, 0.f};
-  float* const gbase = deferred ? reinterpret_cast<float*>(a.pend_gate.ptr) + (int64_t)b * a.pend_gate.sb + (int64_t)h * a.pend_gate.sh : nullptr;
-  auto request = [&](int p, int k) __attribute__((always_inline)) {
-    if (k < r1) {
-      nq[p] = *reinterpret_cast<const vt*>(view_row<T>(a.qu_cache, b, h, k) + sub * V);
-      nu[p] = *reinterpret_cast<const vt*>(view_row<T>(a.U, b, h, k) + sub * V);
-      nk[p] = *reinterpret_cast<const vt*>(view_row<T>(a.kc_cache, b, h, k) + sub * V);
-      nv[p] = *reinterpret_cast<const vt*>(view_row<T>(a.vc_cache, b, h, k) + sub * V);
-      if (np > 0) ng[p] = *reinterpret_cast<const vec<float, 4>*>(gbase + (int64_t)k * kDecodeDefer);
-    }
-  };
-#pragma unroll
-  for (int p = 0; p < PF; ++p) request(p, r0 + grp + p * RPI);
   for (int base = r0; base < r1; base += PF * RPI) {
 #pragma unroll
     for (int p = 0; p < PF; ++p) {
