@@ -85,8 +85,8 @@ Geometry geometry(int B, int H, int L, int d, int es, int flags = 0) {
   g.lse_bytes = align_up(BH * g.Lp * 4, 256);
   g.tblk_bytes = align_up(BH * g.Lp * kNB * es, 256);
   g.snap_bytes = align_up(BH * castle::snap_rows(g.nblk) * d * es, 256);
-  // dS / dSu tiles between the two backward kernels: the 16-bit paths use them
-  g.mat_bytes = es == 2 ? align_up(BH * g.Lp * g.Lp * es, 256) : 0;
+  // dS / dSu tiles between the two backward kernels
+  g.mat_bytes = align_up(BH * g.Lp * g.Lp * es, 256);
   // too long, or the caller asks for it: the query kernel recomputes the scores instead
   if (2 * g.mat_bytes > max_score_tile_bytes() || (flags & CASTLE_FLAG_RECOMPUTE_SCORES)) g.mat_bytes = 0;
   g.off_lse = kHeaderBytes;

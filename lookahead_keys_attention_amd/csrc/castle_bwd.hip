@@ -30,17 +30,12 @@
 #include "castle_tiles.h"
 #include "castle_params.h"
 #include "castle_profile.h"
+#include "castle_dispatch.h"
+#include "castle_narrow.h"
 
 namespace castle {
 
 extern __shared__ __attribute__((aligned(16))) unsigned char castle_smem[];
-
-template <typename T> __device__ __forceinline__ const T* head_ptr(const View4& v, int b, int h) {
-  return reinterpret_cast<const T*>(v.ptr) + (int64_t)b * v.sb + (int64_t)h * v.sh;
-}
-template <typename T> __device__ __forceinline__ T* head_ptr_mut(const View4& v, int b, int h) {
-  return reinterpret_cast<T*>(v.ptr) + (int64_t)b * v.sb + (int64_t)h * v.sh;
-}
 
 struct Carver {
   unsigned char* p;
@@ -51,34 +46,6 @@ struct Carver {
   }
 };
 constexpr int a16(int bytes) { return (bytes + 15) / 16 * 16; }
-
-// [n rows, lanes] accumulator tiles -> (row = lane index, 4 consecutive n) stores, scaled
-// Writes one gradient row held as accumulator tiles [n rows, this lane's row].  rope_pos >= 0: the
-// operand was rotated by that position before use, so its gradient is rotated back first.
-// The NT tiles are columns 32 nt0 .. 32 (nt0 + NT) - 1 of the row.
-template <typename T, int HD, int NT>   // T: element type of the destination tensor
-__device__ __forceinline__ void store_rows(T* dst_row, acc_t (&acc)[NT], float mul, int g, int rope_pos = -1, int nt0 = 0) {
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    if (rope_pos >= 0) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = 32 * (nt0 + nt) + 8 * q + 4 * g;
-        if (n < HD) {
-          CASTLE_ROPE_PAIR(acc[nt][4 * q], acc[nt][4 * q + 1], (float)rope_pos, n / 2, HD, true);
-          CASTLE_ROPE_PAIR(acc[nt][4 * q + 2], acc[nt][4 * q + 3], (float)rope_pos, n / 2 + 1, HD, true);
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[nt][r] *= mul;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = 32 * (nt0 + nt) + 8 * q + 4 * g;
-      if (n < HD) st4<T>(dst_row + n, pack4<T>(acc[nt], q));
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // delta = rowsum(dO * O); also leaves dO in the compute type, padded to Lp rows, for the other kernels
@@ -2357,7 +2324,7 @@ template <typename T, typename TI, int HD, int PART> static int configure_single
   return 0;
 }
 
-template <typename T, typename TI, int HD> static int launch_bwd_t(const BwdArgs& a, hipStream_t stream) {
+template <typename T, typename TI, int HD> static int launch_bwd_t(const BwdArgs& a, bool narrow, hipStream_t stream) {
   const int BH = a.s.B * a.s.H;
   constexpr int key_lds = bwd_key_lds_bytes<T, HD>(), query_lds = bwd_query_lds_bytes<T, HD>();
   if (key_lds > kMaxLds || query_lds > kMaxLds) return -2;
@@ -2401,6 +2368,7 @@ template <typename T, typename TI, int HD> static int launch_bwd_t(const BwdArgs
                          (int64_t)BH * a.s.L, a.amax_part, (int*)nullptr);
     hipLaunchKernelGGL((delta_kernel<T, TI, HD>), dim3((a.s.Lp + RPB - 1) / RPB, BH), block, 0, stream, a);
   }
+  if (narrow) return hipGetLastError() == hipSuccess ? 0 : -3;   // the caller launches the kernels over 32-row work items
   {
     ProfScope ps(kSlotBwdKey, stream);
     if constexpr (SPLIT) {
@@ -2451,27 +2419,16 @@ template <typename T, typename TI, int HD> static int launch_bwd_t(const BwdArgs
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-template <typename T, typename TI> static int launch_bwd_d(const BwdArgs& a, hipStream_t stream) {
-  switch (a.s.d) {
-    case 16: return launch_bwd_t<T, TI, 16>(a, stream);
-    case 32: return launch_bwd_t<T, TI, 32>(a, stream);
-    case 64: return launch_bwd_t<T, TI, 64>(a, stream);
-    case 128:
-      if constexpr (sizeof(T) == 2) return launch_bwd_t<T, TI, 128>(a, stream);
-      return -2;
-    default: return -2;
-  }
-}
-
 // bf16 tensors use fp16 MFMA operands unless bf16_operands is set (must match the forward pass,
 // whose workspace holds operands in the compute type)
 int launch_bwd(const BwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
-  switch (dtype) {
-    case 0: return launch_bwd_d<float, float>(a, stream);
-    case 1: return bf16_operands ? launch_bwd_d<bf16_t, bf16_t>(a, stream) : launch_bwd_d<fp16_t, bf16_t>(a, stream);
-    case 2: return launch_bwd_d<fp16_t, fp16_t>(a, stream);
-    default: return -1;
-  }
+  const bool narrow = a.ds_mat != nullptr && narrow_bwd(a.s, dtype);
+  const int rc = by_type(dtype, bf16_operands, [&](auto t, auto ti) {
+    using T = decltype(t); using TI = decltype(ti);
+    return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_bwd_t<T, TI, decltype(hd)::value>(a, narrow, stream); });
+  });
+  if (rc != 0 || !narrow) return rc;
+  return launch_bwd_narrow(a, dtype, bf16_operands, stream);
 }
 
 }  // namespace castle

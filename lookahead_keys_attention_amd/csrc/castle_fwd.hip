@@ -19,6 +19,9 @@
 #include "castle_tiles.h"
 #include "castle_params.h"
 #include "castle_profile.h"
+#include "castle_tqv.h"
+#include "castle_dispatch.h"
+#include "castle_narrow.h"
 
 namespace castle {
 
@@ -51,13 +54,6 @@ template <typename T, int HD> constexpr int attn_lds_bytes() {
 }
 // register prefetch of the next tile is affordable for 16-bit operands up to d = 64
 template <typename T, int HD> constexpr bool use_prefetch() { return sizeof(T) == 2; }
-
-template <typename T> __device__ __forceinline__ const T* head_ptr(const View4& v, int b, int h) {
-  return reinterpret_cast<const T*>(v.ptr) + (int64_t)b * v.sb + (int64_t)h * v.sh;
-}
-template <typename T> __device__ __forceinline__ T* head_ptr_mut(const View4& v, int b, int h) {
-  return reinterpret_cast<T*>(v.ptr) + (int64_t)b * v.sb + (int64_t)h * v.sh;
-}
 
 // ---------------------------------------------------------------------------
 // One 16-byte piece of one operand per thread; blockIdx.z selects the operand.
@@ -120,72 +116,6 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(FwdArgs a) {
   }
   T* dst = reinterpret_cast<T*>(dstv) + ((int64_t)bh * a.s.Lp + row) * HD + cv * V;
   *reinterpret_cast<vec<T, V>*>(dst) = __builtin_convertvector(f, vec<T, V>);
-}
-
-// ---------------------------------------------------------------------------
-// T' of one 64-row block, by the four waves of a workgroup (one 32x32 tile each).  These blocks have
-// no kernel of their own: they are the last workgroups of the scan launch, which reads none of them,
-// so they run in the slots the scan's tail leaves empty (its last fifth runs at under half occupancy:
-// the launch cannot end before the 64-block sweep of key group 0 does).
-template <typename T, typename TI, int HD>
-__device__ __forceinline__ void tqv_block(const FwdArgs& a, int I, int bh) {
-  constexpr int KS = HD / 16;
-  constexpr int TB = kNB / 32;
-  static_assert(TB * TB == kThreads / 64, "one 32x32 tile of the block per wave");
-  const int lane = lane_id(), c = lane & 31, g = lane >> 5;
-  const T* qc = prep_ptr<T>(a.ws.qc_p, bh, a.s.Lp, HD);   // pre-scaled by c1
-  const T* vu = prep_ptr<T>(a.ws.vu_p, bh, a.s.Lp, HD);
-  T* tb = reinterpret_cast<T*>(a.ws.t_blk) + (int64_t)bh * a.s.Lp * kNB;
-  T* ttb = reinterpret_cast<T*>(a.ws.tt_blk) + (int64_t)bh * a.s.Lp * kNB;
-  T* ttx = reinterpret_cast<T*>(a.ws.ttx_blk) + (int64_t)bh * a.s.Lp * kNB;
-  const int it = wave_id() / TB, jt = wave_id() % TB;
-  const int64_t i = (int64_t)I * kNB + 32 * it + c;   // A-operand row
-  const int64_t j = (int64_t)I * kNB + 32 * jt + c;   // B-operand row
-  // cross quarter of a pair of blocks, (Qc'_{I+1} Vu_I^T)^T for even I: same sources, the queries
-  // of the next block, no mask (every query is later).  All operand loads are issued together.
-  const bool cross = (I & 1) == 0 && I + 1 < a.s.nblk;
-  frag<T> fq[KS], fv[KS], fx[KS];
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    fq[s] = ldg_nat<T>(qc, HD, i, 16 * s + 8 * g, true);
-    fv[s] = ldg_nat<T>(vu, HD, j, 16 * s + 8 * g, true);
-    fx[s] = ldg_nat<T>(qc, HD, i + kNB, 16 * s + 8 * g, cross);
-  }
-  acc_t acc, accx;
-  zero(acc);
-  zero(accx);
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    mma(acc, fq[s], fv[s]);
-    mma(accx, fx[s], fv[s]);
-  }
-  if constexpr (__is_same(T, fp16_t)) {   // T' beyond the fp16 range is clamped (and reported in the header)
-    bool clamped = false;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float y = __builtin_amdgcn_fmed3f(acc[r], -kHalfMax, kHalfMax), yx = __builtin_amdgcn_fmed3f(accx[r], -kHalfMax, kHalfMax);
-      clamped |= (y != acc[r] && acc[r] == acc[r]) || (yx != accx[r] && accx[r] == accx[r]);
-      acc[r] = y;
-      accx[r] = yx;
-    }
-    if (clamped) atomicOr(&a.ws.hdr->status, 2);
-  }
-  // acc[r] = (Qc' Vu^T)[il = 32 it + acc_row][jl = 32 jt + c]; stored as T' = tril(.)
-  const int jl = 32 * jt + c;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int il = 32 * it + acc_row(r, g);
-    acc[r] = jl > il ? 0.f : acc[r];
-    tb[((int64_t)I * kNB + il) * kNB + jl] = (T)acc[r];
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    st4<T>(ttb + ((int64_t)I * kNB + jl) * kNB + 32 * it + 8 * q + 4 * g, pack4<T>(acc, q));
-  if (cross) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      st4<T>(ttx + ((int64_t)I * kNB + jl) * kNB + 32 * it + 8 * q + 4 * g, pack4<T>(accx, q));
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -542,48 +472,17 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, typename TI, int HD> static int launch_fwd_t(const FwdArgs& a, hipStream_t stream) {
+template <typename T, typename TI, int HD> static int launch_prep_t(const FwdArgs& a, hipStream_t stream) {
   const int BH = a.s.B * a.s.H;
-  constexpr int scan_lds = scan_lds_bytes<T, HD>(), attn_lds = attn_lds_bytes<T, HD>();
-  if (attn_lds > kMaxLds) return -2;   // this (dtype, head dim) pair does not fit the 160 KB LDS
-  static PerDeviceOnce once;
-  bool& configured = once.flag();
-  if (!configured) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, TI, HD>), hipFuncAttributeMaxDynamicSharedMemorySize, scan_lds) != hipSuccess) return -3;
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_kernel<T, TI, HD>), hipFuncAttributeMaxDynamicSharedMemorySize, attn_lds) != hipSuccess) return -3;
-    configured = true;
-  }
-  {
-    ProfScope ps(kSlotPrep, stream);
-    constexpr int PIECES_PER_ROW = HD / elem_traits<T>::vec16;
-    if constexpr (sizeof(T) == 2)
-      hipLaunchKernelGGL((amax_kernel<TI, HD>), dim3(kAmaxBlocks), dim3(kAmaxThreads), 0, stream, a.vu, a.s.H, a.s.L,
-                         (int64_t)BH * a.s.L, a.ws.amax_part, &a.ws.hdr->status);
-    hipLaunchKernelGGL((prep_kernel<T, TI, HD>), dim3((a.s.Lp * PIECES_PER_ROW + kThreads - 1) / kThreads, BH, 6), dim3(kThreads), 0, stream, a);
-  }
-  {
-    ProfScope ps(kSlotScan, stream);
-    hipLaunchKernelGGL((scan_kernel<T, TI, HD>), dim3(a.s.Lp / 128 * BH + (a.with_t ? a.s.nblk * BH : 0)), dim3(kThreads), scan_lds, stream, a);
-  }
-  {
-    ProfScope ps(kSlotAttn, stream);
-    hipLaunchKernelGGL((attn_kernel<T, TI, HD>), dim3(a.s.Lp / 128 * BH), dim3(kThreads), attn_lds, stream, a);
-  }
+  constexpr int PIECES_PER_ROW = HD / elem_traits<T>::vec16;
+  ProfScope ps(kSlotPrep, stream);
+  if constexpr (sizeof(T) == 2)
+    hipLaunchKernelGGL((amax_kernel<TI, HD>), dim3(kAmaxBlocks), dim3(kAmaxThreads), 0, stream, a.vu, a.s.H, a.s.L,
+                       (int64_t)BH * a.s.L, a.ws.amax_part, &a.ws.hdr->status);
+  hipLaunchKernelGGL((prep_kernel<T, TI, HD>), dim3((a.s.Lp * PIECES_PER_ROW + kThreads - 1) / kThreads, BH, 6), dim3(kThreads), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-template <typename T, typename TI> static int launch_fwd_d(const FwdArgs& a, hipStream_t stream) {
-  switch (a.s.d) {
-    case 16: return launch_fwd_t<T, TI, 16>(a, stream);
-    case 32: return launch_fwd_t<T, TI, 32>(a, stream);
-    case 64: return launch_fwd_t<T, TI, 64>(a, stream);
-    case 128: return launch_fwd_t<T, TI, 128>(a, stream);
-    default: return -2;
-  }
-}
-
-// The scan alone (snapshots of the lookahead state into a.ws.usnap from the operand copies the
-// forward pass left): what the backward pass runs first when the forward snapshots were not kept.
 template <typename T, typename TI, int HD> static int launch_scan_t(const FwdArgs& a, hipStream_t stream) {
   constexpr int scan_lds = scan_lds_bytes<T, HD>();
   static PerDeviceOnce once;
@@ -596,33 +495,43 @@ template <typename T, typename TI, int HD> static int launch_scan_t(const FwdArg
   hipLaunchKernelGGL((scan_kernel<T, TI, HD>), dim3(a.s.Lp / 128 * a.s.B * a.s.H + (a.with_t ? a.s.nblk * a.s.B * a.s.H : 0)), dim3(kThreads), scan_lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
-template <typename T, typename TI> static int launch_scan_d(const FwdArgs& a, hipStream_t stream) {
-  switch (a.s.d) {
-    case 16: return launch_scan_t<T, TI, 16>(a, stream);
-    case 32: return launch_scan_t<T, TI, 32>(a, stream);
-    case 64: return launch_scan_t<T, TI, 64>(a, stream);
-    case 128: return launch_scan_t<T, TI, 128>(a, stream);
-    default: return -2;
+
+template <typename T, typename TI, int HD> static int launch_attn_t(const FwdArgs& a, hipStream_t stream) {
+  constexpr int attn_lds = attn_lds_bytes<T, HD>();
+  static_assert(attn_lds <= kMaxLds, "attention kernel does not fit the LDS");
+  static PerDeviceOnce once;
+  bool& configured = once.flag();
+  if (!configured) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_kernel<T, TI, HD>), hipFuncAttributeMaxDynamicSharedMemorySize, attn_lds) != hipSuccess) return -3;
+    configured = true;
   }
-}
-int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
-  switch (dtype) {
-    case 0: return launch_scan_d<float, float>(a, stream);
-    case 1: return bf16_operands ? launch_scan_d<bf16_t, bf16_t>(a, stream) : launch_scan_d<fp16_t, bf16_t>(a, stream);
-    case 2: return launch_scan_d<fp16_t, fp16_t>(a, stream);
-    default: return -1;
-  }
+  ProfScope ps(kSlotAttn, stream);
+  hipLaunchKernelGGL((attn_kernel<T, TI, HD>), dim3(a.s.Lp / 128 * a.s.B * a.s.H), dim3(kThreads), attn_lds, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-// bf16 tensors: operands are converted to fp16 on load (exact inside the fp16 range) and every
-// operand produced inside the kernels is fp16, unless bf16_operands asks for bf16 MFMA operands.
+// The scan alone (snapshots of the lookahead state into a.ws.usnap from the operand copies the
+// forward pass left) is also what the backward pass runs first when the forward snapshots were not kept.
+int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
+  if (narrow_scan(a.s)) return launch_scan_narrow(a, dtype, bf16_operands, stream);
+  return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
+    using T = decltype(t); using TI = decltype(ti);
+    return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_scan_t<T, TI, decltype(hd)::value>(a, stream); });
+  });
+}
+
 int launch_fwd(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
-  switch (dtype) {
-    case 0: return launch_fwd_d<float, float>(a, stream);
-    case 1: return bf16_operands ? launch_fwd_d<bf16_t, bf16_t>(a, stream) : launch_fwd_d<fp16_t, bf16_t>(a, stream);
-    case 2: return launch_fwd_d<fp16_t, fp16_t>(a, stream);
-    default: return -1;
-  }
+  int rc = by_type(dtype, bf16_operands, [&](auto t, auto ti) {
+    using T = decltype(t); using TI = decltype(ti);
+    return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_prep_t<T, TI, decltype(hd)::value>(a, stream); });
+  });
+  if (rc == 0) rc = launch_scan(a, dtype, bf16_operands, stream);
+  if (rc != 0) return rc;
+  if (narrow_attn(a.s)) return launch_attn_narrow(a, dtype, bf16_operands, stream);
+  return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
+    using T = decltype(t); using TI = decltype(ti);
+    return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_attn_t<T, TI, decltype(hd)::value>(a, stream); });
+  });
 }
 
 }  // namespace castle

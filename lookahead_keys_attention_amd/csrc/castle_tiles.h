@@ -571,6 +571,41 @@ __device__ __forceinline__ vec<float, 2> rope_rot(float x0, float x1, float pos,
     (X1) = y_[1];                                                              \
   } while (0)
 
+template <typename T> __device__ __forceinline__ const T* head_ptr(const View4& v, int b, int h) {
+  return reinterpret_cast<const T*>(v.ptr) + (int64_t)b * v.sb + (int64_t)h * v.sh;
+}
+template <typename T> __device__ __forceinline__ T* head_ptr_mut(const View4& v, int b, int h) {
+  return reinterpret_cast<T*>(v.ptr) + (int64_t)b * v.sb + (int64_t)h * v.sh;
+}
+
+// [n rows, lanes] accumulator tiles -> (row = lane index, 4 consecutive n) stores, scaled
+// Writes one gradient row held as accumulator tiles [n rows, this lane's row].  rope_pos >= 0: the
+// operand was rotated by that position before use, so its gradient is rotated back first.
+// The NT tiles are columns 32 nt0 .. 32 (nt0 + NT) - 1 of the row.
+template <typename T, int HD, int NT>   // T: element type of the destination tensor
+__device__ __forceinline__ void store_rows(T* dst_row, acc_t (&acc)[NT], float mul, int g, int rope_pos = -1, int nt0 = 0) {
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    if (rope_pos >= 0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = 32 * (nt0 + nt) + 8 * q + 4 * g;
+        if (n < HD) {
+          CASTLE_ROPE_PAIR(acc[nt][4 * q], acc[nt][4 * q + 1], (float)rope_pos, n / 2, HD, true);
+          CASTLE_ROPE_PAIR(acc[nt][4 * q + 2], acc[nt][4 * q + 3], (float)rope_pos, n / 2 + 1, HD, true);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[nt][r] *= mul;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = 32 * (nt0 + nt) + 8 * q + 4 * g;
+      if (n < HD) st4<T>(dst_row + n, pack4<T>(acc[nt], q));
+    }
+  }
+}
+
 // ---- range control ------------------------------------------------------------------------
 // Partial maxima of |x| over a (B, H, L, HD) view: kAmaxBlocks workgroups, one partial each.  The
 // consumers reduce the partials themselves (amax_from_partials), so no atomics and no clearing.

@@ -84,6 +84,25 @@ def test_operator_backward(B, Hh, L, d, dtype):
             assert (leaf.grad.cpu().double() - r).abs().max() <= 1e-4, name
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,Hh,L,d", [(2, 3, 5, 64), (1, 2, 31, 32), (2, 2, 33, 64), (1, 3, 65, 16), (2, 2, 95, 128), (1, 2, 97, 64), (1, 1, 545, 128),
+                                      (1, 2, 800, 32), (10, 52, 5, 64), (8, 66, 33, 32), (10, 52, 64, 64), (8, 66, 97, 64), (4, 130, 129, 16), (4, 65, 130, 128)])
+def test_operator_at_tile_edges_with_few_and_with_many_heads(B, Hh, L, d, dtype):
+    """Few heads take the kernels over 32-row items, many (more than two workgroups of 128 rows per CU) those over 128."""
+    if dtype == torch.float32 and d == 128:
+        pytest.skip("no fp32 kernels at d = 128")
+    ops, dout = rand_ops(B, Hh, L, d, dtype, seed=5 * L + d)
+    s = d ** -0.5
+    leaves = [t.to(DEV).requires_grad_() for t in ops]
+    out, U = H().castle_attention_hip(*leaves, s, True)
+    out.backward(dout.to(DEV))
+    ref_out, ref_U = O.parallel_core(*[t.double() for t in ops], s, want_U=True)
+    assert_close(out, ref_out, dtype, "out", 1e-4)
+    assert_close(U, ref_U, dtype, "U", 1e-4)
+    for name, leaf, r in zip(NAMES, leaves, O.closed_form_grads(*[t.double() for t in ops], s, dout.double())):
+        assert_close(leaf.grad, r, dtype, name, 1e-4)
+
+
 @pytest.mark.parametrize("L,d", [(256, 64), (200, 32)])
 def test_bf16_operand_flag_forward_and_backward(L, d, monkeypatch):
     """CASTLE_FLAG_BF16_OPERANDS keeps bf16 MFMA operands (default: fp16 operands for bf16 tensors)."""
