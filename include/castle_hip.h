@@ -272,6 +272,40 @@ int castle_sample(const void* logits, int64_t ld, const float* uniform, int rows
  * 0 .. table_rows - 1 gives a row of zeros.  The token embedding of a step (train_triton.py:86). */
 int castle_gather_rows(const void* table, int64_t table_rows, int64_t ld, int width, const int64_t* index, int n, void* y, int dtype, void* stream);
 
+/* The work between the products of a transformer block (train_triton.py:102-107, 150-171; lookahead_keys_attention.py:95).
+ * All tensors: rows of `width` (or `classes`) elements in the type `dtype`, contiguous, a whole number of 16-byte pieces
+ * (at most 512 for the norm and the embedding), 16-byte aligned.
+ *
+ * castle_rms_norm: h = (s / sqrt(mean(s^2) + eps)) * weight with s = x, or s = x + delta (rounded to the type and written
+ * to `sum`) when delta != NULL.  rstd: NULL, or one float per row for the backward pass. */
+int castle_rms_norm(const void* x, const void* delta, const void* weight, void* sum, void* h, float* rstd, int64_t rows, int width, float eps,
+                    int dtype, void* stream);
+/* dx = dres + d(norm)/dx dh (dres may be NULL), dweight = sum over rows; either result may be NULL.  The workspace is
+ * only needed for dweight. */
+int64_t castle_rms_norm_bwd_workspace_bytes(int64_t rows, int width, int dtype);
+int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
+                        int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* out[i] = sum over p < parts of part[p * n + i], n % 8 == 0: partial products of a weight gradient. */
+int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream);
+
+/* Mean cross entropy (train_triton.py:166-171).  Row r of the logits belongs to the class target[(r / target_n) * target_ld +
+ * r % target_n]; rows of class -100 do not count, a class outside 0 .. classes - 1 makes the loss NaN.  loss: one element
+ * of the type; lse: one float per row and inv_count: one float, both kept for the backward pass, which multiplies by
+ * the one element of `grad`. */
+#define CASTLE_CROSS_ENTROPY_WORKSPACE 8192
+int castle_cross_entropy(const void* logits, const int64_t* target, int64_t target_n, int64_t target_ld, int64_t rows, int classes, void* loss,
+                         float* lse, float* inv_count, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+int castle_cross_entropy_bwd(const void* logits, const int64_t* target, int64_t target_n, int64_t target_ld, int64_t rows, int classes,
+                             const float* lse, const float* inv_count, const void* grad, void* dlogits, int dtype, void* stream);
+
+/* dweight[v] = sum of the dy rows whose index is v (indices addressed like `target` above), summed in a fixed order.
+ * For small vocabularies: rows * vocabulary at most 2^26, else castle_embedding_grad_workspace_bytes returns
+ * CASTLE_ERR_SHAPE. */
+int64_t castle_embedding_grad_workspace_bytes(int64_t rows, int vocabulary, int width, int dtype);
+int castle_embedding_grad(const void* dy, const int64_t* index, int64_t index_n, int64_t index_ld, int64_t rows, int vocabulary, int width,
+                          void* dweight, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Per-kernel timing (no counterpart in the reference; for benchmarks).  While enabled, every
  * kernel launched by the entry points above is bracketed by a HIP event pair on its stream.
  * castle_profile_enable(on) also discards pending records.  castle_profile_read waits for the

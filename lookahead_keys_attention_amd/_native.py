@@ -47,6 +47,14 @@ EXPORTED_SYMBOLS = (
     "castle_sample",
     "castle_gather_rows",
     "castle_small_linear_fused",
+    "castle_rms_norm",
+    "castle_rms_norm_bwd_workspace_bytes",
+    "castle_rms_norm_bwd",
+    "castle_sum_parts",
+    "castle_cross_entropy",
+    "castle_cross_entropy_bwd",
+    "castle_embedding_grad_workspace_bytes",
+    "castle_embedding_grad",
     "castle_profile_enable",
     "castle_profile_read",
 )

@@ -409,25 +409,27 @@ class Castle(nn.Module):
                 return False
         return True
 
-    def _layer_native(self, x, want_cache):
+    def _layer_native(self, x, want_cache, delta=None):
         """The parallel pass as one native call (csrc/castle_host.cpp): norm, projection, attention core,
-        output projection and, with a cache, the rows of its buffers."""
+        output projection and, with a cache, the rows of its buffers.  With `delta` the layer runs on x + delta and
+        the result is (y, x + delta), with the cache behind it: a block of a residual stream."""
         B, n, _ = x.shape
         H, d = self.heads, self.dim_head
         norm = self._modules["norm"]
         u_half = want_cache and x.dtype == torch.bfloat16 and ops.LOOKAHEAD_KEYS_HALF
         flags = (ops.DEFAULT_FLAGS | (_native.FLAG_ROTARY if self.use_rotary else 0) | (_native.FLAG_U_HALF if u_half else 0))
-        y, *buffers = _native.host().layer_parallel(
-            x, norm._parameters.get("weight"), getattr(norm, "eps", None), self._modules["to_all_qkv"]._parameters["weight"],
+        results = _native.host().layer_parallel(
+            x, delta, norm._parameters.get("weight"), getattr(norm, "eps", None), self._modules["to_all_qkv"]._parameters["weight"],
             self._modules["combine_heads"]._parameters["weight"], H, self.scale, flags,
             ops.keeps_state(B, H, n, d, x.dtype), _reserve_rows(n) if want_cache else 0)
+        outputs = 1 if delta is None else 2
         if not want_cache:
-            return y
-        store = _CacheStore(B, H, d, _reserve_rows(n), x.dtype, x.device, buffers=buffers)
+            return results[0] if delta is None else tuple(results)
+        store = _CacheStore(B, H, d, _reserve_rows(n), x.dtype, x.device, buffers=results[outputs:])
         store.u_half = u_half
         store.length = store.base0 = n
         store.scale = self.scale
-        return y, store.as_cache()
+        return (*results[:outputs], store.as_cache())
 
     @staticmethod
     def _project(layer, t, native_step, norm=None, activation=None, residual=None):

@@ -5,8 +5,10 @@
 
 #include "../../include/castle_hip.h"
 #include <stdlib.h>
+#include <initializer_list>
 #include "castle_params.h"
 #include "castle_profile.h"
+#include "castle_rows.h"
 #include "castle_tiles.h"
 
 namespace castle {
@@ -151,6 +153,8 @@ castle::FwdWorkspace carve(void* base, void* state, const Geometry& g) {
 }
 
 }  // namespace
+
+constexpr int64_t kMaxRows = (int64_t)1 << 30;   // rows of a launch: the grids stay below 2^31 workgroups
 
 extern "C" {
 
@@ -499,6 +503,108 @@ int castle_gather_rows(const void* table, int64_t table_rows, int64_t ld, int wi
       ld * es % 16 != 0 || reinterpret_cast<uintptr_t>(index) % 8 != 0)
     return CASTLE_ERR_ARG;
   return castle::launch_gather_rows(table, (int64_t)width * es, ld * es, table_rows, index, n, y, static_cast<hipStream_t>(stream));
+}
+
+static bool row_pieces_ok(int n, int es) { return n > 0 && (int64_t)n * es % 16 == 0; }
+static bool aligned16(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+  return true;
+}
+
+int castle_rms_norm(const void* x, const void* delta, const void* weight, void* sum, void* h, float* rstd, int64_t rows, int width, float eps,
+                    int dtype, void* stream) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (rows <= 0 || rows > kMaxRows || !row_pieces_ok(width, es) || (int64_t)width * es / 16 > castle::kMaxRowPieces) return CASTLE_ERR_SHAPE;
+  if (x == nullptr || weight == nullptr || h == nullptr || (delta != nullptr && sum == nullptr) || !(eps >= 0.f) ||
+      !aligned16({x, delta, weight, sum, h}) || reinterpret_cast<uintptr_t>(rstd) % 4 != 0)
+    return CASTLE_ERR_ARG;
+  const castle::NormArgs a = {x, delta, weight, sum, h, rstd, rows, width, eps};
+  return castle::launch_norm(a, dtype, static_cast<hipStream_t>(stream));
+}
+
+int64_t castle_rms_norm_bwd_workspace_bytes(int64_t rows, int width, int dtype) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (rows <= 0 || rows > kMaxRows || !row_pieces_ok(width, es) || (int64_t)width * es / 16 > castle::kMaxRowPieces) return CASTLE_ERR_SHAPE;
+  return align_up((int64_t)castle::norm_bwd_groups(rows, width, es) * width * 4, 256);
+}
+
+int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
+                        int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t need = castle_rms_norm_bwd_workspace_bytes(rows, width, dtype);
+  if (need < 0) return (int)need;
+  if (dh == nullptr || x == nullptr || weight == nullptr || rstd == nullptr || (dx == nullptr && dweight == nullptr) ||
+      !aligned16({dh, x, weight, dres, dx}) || reinterpret_cast<uintptr_t>(rstd) % 4 != 0 ||
+      reinterpret_cast<uintptr_t>(dweight) % elem_size(dtype) != 0)
+    return CASTLE_ERR_ARG;
+  if (dweight != nullptr && (workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
+  const castle::NormBwdArgs a = {dh, x, weight, dres, rstd, dx, dweight != nullptr ? static_cast<float*>(workspace) : nullptr, rows, width};
+  return castle::launch_norm_bwd(a, dweight, dtype, static_cast<hipStream_t>(stream));
+}
+
+int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream) {
+  if (elem_size(dtype) == 0) return CASTLE_ERR_DTYPE;
+  if (parts <= 0 || n <= 0 || n % 8 != 0 || n / 8 > kMaxRows) return CASTLE_ERR_SHAPE;
+  if (part == nullptr || out == nullptr || !aligned16({part, out})) return CASTLE_ERR_ARG;
+  return castle::launch_part_sum(part, parts, n, out, dtype, static_cast<hipStream_t>(stream));
+}
+
+static int cross_entropy_args(castle::CrossEntropyArgs& a, const void* logits, const int64_t* target, int64_t target_n, int64_t target_ld, int64_t rows,
+                              int classes, const float* lse, int dtype) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (rows <= 0 || rows > kMaxRows || target_n <= 0 || rows % target_n != 0 || !row_pieces_ok(classes, es)) return CASTLE_ERR_SHAPE;
+  if (logits == nullptr || target == nullptr || lse == nullptr || !aligned16({logits}) || reinterpret_cast<uintptr_t>(target) % 8 != 0 ||
+      reinterpret_cast<uintptr_t>(lse) % 4 != 0)
+    return CASTLE_ERR_ARG;
+  a = {logits, target, rows, target_n, target_ld, classes, const_cast<float*>(lse), nullptr};
+  return CASTLE_OK;
+}
+
+int castle_cross_entropy(const void* logits, const int64_t* target, int64_t target_n, int64_t target_ld, int64_t rows, int classes, void* loss,
+                         float* lse, float* inv_count, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  castle::CrossEntropyArgs a;
+  const int rc = cross_entropy_args(a, logits, target, target_n, target_ld, rows, classes, lse, dtype);
+  if (rc != CASTLE_OK) return rc;
+  if (loss == nullptr || inv_count == nullptr || reinterpret_cast<uintptr_t>(loss) % elem_size(dtype) != 0 || reinterpret_cast<uintptr_t>(inv_count) % 4 != 0)
+    return CASTLE_ERR_ARG;
+  if (workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < CASTLE_CROSS_ENTROPY_WORKSPACE) return CASTLE_ERR_WORKSPACE;
+  static_assert(CASTLE_CROSS_ENTROPY_WORKSPACE >= castle::kCrossEntropyGroups * 8, "two floats a group");
+  a.part = static_cast<float*>(workspace);
+  return castle::launch_cross_entropy(a, loss, inv_count, dtype, static_cast<hipStream_t>(stream));
+}
+
+int castle_cross_entropy_bwd(const void* logits, const int64_t* target, int64_t target_n, int64_t target_ld, int64_t rows, int classes,
+                             const float* lse, const float* inv_count, const void* grad, void* dlogits, int dtype, void* stream) {
+  castle::CrossEntropyArgs a;
+  const int rc = cross_entropy_args(a, logits, target, target_n, target_ld, rows, classes, lse, dtype);
+  if (rc != CASTLE_OK) return rc;
+  if (inv_count == nullptr || grad == nullptr || dlogits == nullptr || !aligned16({dlogits})) return CASTLE_ERR_ARG;
+  return castle::launch_cross_entropy_bwd(a, grad, inv_count, dlogits, dtype, static_cast<hipStream_t>(stream));
+}
+
+int64_t castle_embedding_grad_workspace_bytes(int64_t rows, int vocabulary, int width, int dtype) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  // every (vocabulary row, chunk) reads the token numbers of its chunk: above 2^26 of them (0.5 GB, about what the sort of
+  // the library's operator costs) this is not the way
+  if (rows <= 0 || vocabulary <= 0 || rows > kMaxRows || rows * vocabulary > (int64_t)1 << 26 || !row_pieces_ok(width, es) ||
+      (int64_t)width * es / 16 > castle::kMaxRowPieces || castle::embedding_grad_chunks(rows) > 65535)
+    return CASTLE_ERR_SHAPE;
+  return align_up((int64_t)castle::embedding_grad_chunks(rows) * vocabulary * width * 4, 256);
+}
+
+int castle_embedding_grad(const void* dy, const int64_t* index, int64_t index_n, int64_t index_ld, int64_t rows, int vocabulary, int width,
+                          void* dweight, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t need = castle_embedding_grad_workspace_bytes(rows, vocabulary, width, dtype);
+  if (need < 0) return (int)need;
+  if (index_n <= 0 || rows % index_n != 0 || (int64_t)vocabulary * width % 8 != 0) return CASTLE_ERR_SHAPE;
+  if (dy == nullptr || index == nullptr || dweight == nullptr || !aligned16({dy, dweight}) || reinterpret_cast<uintptr_t>(index) % 8 != 0) return CASTLE_ERR_ARG;
+  if (workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 256 != 0 || workspace_bytes < need) return CASTLE_ERR_WORKSPACE;
+  const castle::EmbeddingGradArgs a = {dy, index, rows, index_n, index_ld, vocabulary, width, static_cast<float*>(workspace)};
+  return castle::launch_embedding_grad(a, dweight, dtype, static_cast<hipStream_t>(stream));
 }
 
 int castle_profile_enable(int on) { return castle::profile_enable(on); }

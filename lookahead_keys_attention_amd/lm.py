@@ -20,7 +20,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from . import _native
+from . import _native, ops
 from .castle import Castle, _linear
 
 
@@ -60,6 +60,11 @@ def block_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Te
     with the two weight gradients formed in row ranges where that pays (castle._linear)."""
     norm, up, act, down = feed_forward
     return _linear(down, act(_linear(up, norm(h))))
+
+
+def _is_plain(module, kind) -> bool:
+    """True for an unmodified module of exactly this kind with no hooks on it."""
+    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
 
 
 class GraphedDecoder:
@@ -198,6 +203,8 @@ class CastleLM(nn.Module):
         (batch, n, num_tokens), plus the list of per-layer caches when return_next_cache."""
         if return_loss:
             x, target = x[:, :-1], x[:, 1:]
+        if cache is None and x.dim() == 2 and x.shape[1] > 1 and self._plain(x):
+            return self._forward_plain(x, target if return_loss else None, return_next_cache)
         h = self.token_emb(x)
         # one token per sequence, no graph to record: the few rows of every projection go through the small-M kernel
         # (only for a model whose layers run the native kernels: one built with use_triton=False stays on
@@ -216,6 +223,53 @@ class CastleLM(nn.Module):
         logits = Castle._project(self.to_logits, h, token_step, norm=self.final_norm)
         if return_loss:
             return F.cross_entropy(logits.transpose(1, 2), target)
+        return (logits, next_cache) if return_next_cache else logits
+
+    def _plain(self, x) -> bool:
+        """True if whole sequences may run as one native call per block: native layers, unmodified modules, nothing
+        hooked onto any of them."""
+        embedding, weight = self.token_emb, self.token_emb.weight
+        if (not x.is_cuda or x.dtype != torch.long or not _is_plain(embedding, nn.Embedding) or embedding.max_norm is not None
+                or embedding.padding_idx is not None or embedding.scale_grad_by_freq or embedding.sparse or weight.device != x.device
+                or weight.dtype not in _native.DTYPE_CODES or not _native.is_built()):
+            return False
+        final, logits, dtype = self.final_norm, self.to_logits, weight.dtype
+        if not (_is_plain(final, nn.RMSNorm) and _is_plain(logits, nn.Linear) and logits.bias is None and logits.weight.dtype is dtype
+                and final.weight is not None and final.weight.dtype is dtype) or not len(self.layers):
+            return False
+        like = weight.detach()[None]   # what every block gets, as far as the blocks look at it
+        for block in self.layers:
+            if not _is_plain(block, nn.ModuleList) or len(block) != 2:
+                return False
+            attention, feed_forward = block
+            if not (_is_plain(attention, Castle) and attention.use_triton and ops.kernels_support(attention.dim_head, dtype) and attention._plain(like)
+                    and _is_plain(feed_forward, nn.Sequential) and len(feed_forward) == 4):
+                return False
+            norm, up, act, down = feed_forward
+            if not (_is_plain(norm, nn.RMSNorm) and norm.weight is not None and norm.weight.dtype is dtype and _is_plain(up, nn.Linear) and up.bias is None
+                    and up.weight.dtype is dtype and _is_plain(act, nn.GELU) and act.approximate == "none" and _is_plain(down, nn.Linear)
+                    and down.bias is None and down.weight.dtype is dtype):
+                return False
+        return True
+
+    def _forward_plain(self, x, target, return_next_cache):
+        """`forward` over whole sequences, one native call per block: the sum of a residual stream is formed by the
+        norm that reads it next."""
+        host = _native.host()
+        h, delta, next_cache = host.embedding(self.token_emb.weight, x), None, []
+        for attention, feed_forward in self.layers:
+            results = attention._layer_native(h, return_next_cache, delta)
+            if return_next_cache:
+                *results, layer_next = results
+                next_cache.append(layer_next)
+            elif delta is None:
+                results = (results,)
+            attended, h = results if delta is not None else (results[0], h)
+            norm, up, _, down = feed_forward
+            delta, h = host.feed_forward(h, attended, norm.weight, norm.eps, up.weight, down.weight)
+        logits = host.head(h, delta, self.final_norm.weight, self.final_norm.eps, self.to_logits.weight)
+        if target is not None:
+            return host.cross_entropy(logits, target)
         return (logits, next_cache) if return_next_cache else logits
 
     def _decoder_for(self, cache, max_len):

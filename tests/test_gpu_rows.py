@@ -1,0 +1,105 @@
+"""Row kernels (norm with a residual sum, cross entropy, embedding gradient) against fp32 / fp64 PyTorch on the CPU."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+TOL = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}
+
+
+def host():
+    from lookahead_keys_attention_amd import _native
+
+    return _native.host()
+
+
+def close(got, ref, dtype, what):
+    got, ref = got.detach().cpu().double(), ref.detach().double()
+    assert torch.isfinite(got).all() and (got - ref).norm() <= TOL[dtype] * ref.norm() + 1e-30, (what, (got - ref).norm() / ref.norm())
+
+
+# lanes per row 16 / 32 / 64, 1 ... 8 pieces per lane, their edges, a length for the library's norm (5000)
+@pytest.mark.parametrize("dim", [8, 120, 128, 136, 256, 512, 520, 1024, 2048, 4096, 5000])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_norm_with_sum(dim, dtype):
+    g = torch.Generator().manual_seed(dim)
+    for B, L in ((1, 2), (3, 43), (2, 1500 if dim <= 512 else 60)):
+        x, delta, gy = (torch.randn(B, L, n, generator=g).to(dtype) for n in (dim, dim, 16))
+        nw, w = (1 + torch.randn(dim, generator=g) * 0.2).to(dtype), (torch.randn(16, dim, generator=g) * dim ** -0.5).to(dtype)
+        leaves = [t.to(DEV).requires_grad_() for t in (x, delta, nw, w)]
+        y = host().head(leaves[0], leaves[1], leaves[2], None, leaves[3])
+        y.backward(gy.to(DEV))
+        ref = [t.double().requires_grad_() for t in (x, delta, nw, w)]
+        s = ref[0] + ref[1]
+        yr = F.rms_norm(s + ((x + delta).double() - s).detach(), (dim,), ref[2], torch.finfo(torch.float32).eps) @ ref[3].t()
+        yr.backward(gy.double())
+        close(y, yr, dtype, "y")
+        for name, a, b in zip(("x", "delta", "norm", "w"), leaves, ref):
+            close(a.grad, b.grad, dtype, name)
+        with torch.no_grad():
+            assert torch.equal(host().head(*leaves[:3], None, leaves[3]), y)
+
+
+@pytest.mark.parametrize("classes", [8, 256, 264, 1000, 32000])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_cross_entropy(classes, dtype):
+    g = torch.Generator().manual_seed(classes)
+    for B, n in ((1, 1), (3, 37), (5, 1100 if classes <= 256 else 20)):
+        logits = (torch.randn(B, n, classes, generator=g) * 3).to(dtype)
+        target = torch.randint(0, classes, (B, n + 1), generator=g)
+        if n > 1:
+            target[0, 1] = -100
+        leaf = logits.to(DEV).requires_grad_()
+        loss = host().cross_entropy(leaf, target.to(DEV)[:, 1:])
+        (loss * 2).backward()
+        ref = logits.double().requires_grad_()
+        lr = F.cross_entropy(ref.transpose(1, 2), target[:, 1:]) if n > 1 or target[0, 1] != -100 else None
+        (lr * 2).backward()
+        close(loss, lr, dtype, "loss")
+        close(leaf.grad, ref.grad, dtype, "dlogits")
+    bad = target.clone()
+    bad[0, 2] = classes
+    assert host().cross_entropy(leaf.detach(), bad.to(DEV)[:, 1:]).isnan()
+
+
+@pytest.mark.parametrize("vocabulary,dim", [(5, 8), (256, 512), (300, 1032)])
+def test_embedding_gradient(vocabulary, dim):
+    g = torch.Generator().manual_seed(vocabulary)
+    for B, n in ((1, 1), (2, 1025), (3, 2048)):
+        w, ids = torch.randn(vocabulary, dim, generator=g).bfloat16(), torch.randint(0, vocabulary, (B, n + 1), generator=g)
+        ids[0] = 1   # one row gets most of them
+        dy = torch.randn(B, n, dim, generator=g).bfloat16()
+        leaf = w.to(DEV).requires_grad_()
+        y = host().embedding(leaf, ids.to(DEV)[:, :-1])
+        y.backward(dy.to(DEV))
+        ref = w.double().requires_grad_()
+        F.embedding(ids[:, :-1], ref).backward(dy.double())
+        assert torch.equal(y.cpu(), F.embedding(ids[:, :-1], w))
+        close(leaf.grad, ref.grad, torch.bfloat16, "dw")
+
+
+def test_language_model_blocks_equal_the_modules():
+    """The one-call-per-block path against the same model run module by module (a hook switches it off)."""
+    from lookahead_keys_attention_amd import CastleLM
+
+    torch.manual_seed(0)
+    for tie in (False, True):
+        model = CastleLM(num_tokens=64, dim=128, depth=2, heads=2, dim_head=64, tie_embedding=tie).to(DEV)
+        ids = torch.randint(0, 64, (3, 90), device=DEV)
+        results = []
+        for hooked in (False, True):
+            handle = model.layers[1][1].register_forward_hook(lambda *_: None) if hooked else None
+            assert model._plain(ids) is not hooked
+            model.zero_grad()
+            loss = model(ids, return_loss=True)
+            loss.backward()
+            with torch.no_grad():
+                logits, caches = model(ids, return_next_cache=True)
+            results.append([loss, logits, caches[1].vc_cache] + [p.grad for p in model.parameters() if p.grad is not None])
+            if handle is not None:
+                handle.remove()
+        assert len(results[0]) == len(results[1])
+        for a, b in zip(*results):
+            assert (a - b).norm() <= 1e-4 * b.norm()
