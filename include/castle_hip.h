@@ -216,7 +216,7 @@ int castle_decode_step_static(const castle_view4* U, const castle_view4* qu_cach
 
 /* A whole layer for one token per sequence: y = residual + core(norm(x) w_in^T) w_out^T, the cached step with
  * the norm and the projections around it (lookahead_keys_attention.py:95-99, 166-203, 209 with seq_len == 1) in
- * four launches behind one call.
+ * three launches behind one call.
  * x, y: B rows of `dim` elements; w_in (6 H d, dim), w_out (dim, H d), both row-major in the tensor type, `proj` a
  * B x 6 H d scratch in the tensor type (order qu, ku, vu, qc, kc, vc).  norm_weight (`dim` elements), residual
  * (B rows; may alias y) and t_device may be NULL.  dim % 8 == 0 (4 for fp32); x, w_in, w_out, proj and norm_weight

@@ -371,7 +371,10 @@ class Castle(nn.Module):
             assert cache is None, "must be inferencing single tokens if receiving cache"
             return self._layer_native(x, return_next_cache)
         native_step = single and native
-        proj = self._project(self.to_all_qkv, x, native_step, norm=self.norm)
+        norm = self.norm
+        if native and not single and torch.compiler.is_compiling() and type(norm) is nn.RMSNorm and norm.weight.dtype == x.dtype:
+            x, norm = torch.ops.castle_hip.rms_norm(x, norm.weight, norm.eps)[0], None   # what the untraced layer runs
+        proj = self._project(self.to_all_qkv, x, native_step, norm=norm)
         if not single:
             assert cache is None, "must be inferencing single tokens if receiving cache"
             merged, next_cache = (self._parallel_native if native else self._parallel_dense)(proj, return_next_cache)

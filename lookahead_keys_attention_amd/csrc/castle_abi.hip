@@ -21,7 +21,7 @@ int launch_rope(const View4& src, const View4& dst, int B, int H, int L, int d, 
 int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus);
 int decode_static_scratch(float** ptr);
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
-                        int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream);
+                        int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream, int* clear = nullptr, int clear_n = 0);
 int launch_sample(const void* logits, int64_t ld, const float* u, int rows, int V, int k, float inv_temperature, int64_t* out, int64_t out_ld,
                   int64_t* out2, int dtype, hipStream_t stream);
 int launch_gather_rows(const void* table, int64_t row_bytes, int64_t ld_bytes, int64_t rows, const int64_t* index, int n, void* y, hipStream_t stream);
@@ -289,7 +289,7 @@ int castle_bwd(const castle_view4* qc, const castle_view4* kc, const castle_view
 
 int64_t castle_decode_workspace_bytes(int B, int H, int d, int t_max) {
   if (B <= 0 || H <= 0 || !head_dim_ok(d) || t_max < 0) return CASTLE_ERR_SHAPE;
-  return align_up((int64_t)B * H * 64 * (d + 2) * 4, 256);
+  return align_up((int64_t)B * H * (64 * (d + 2) + 1) * 4, 256);   // partials of up to 64 splits, one arrival count
 }
 
 // checks the arguments of a cached step and fills `a`; out may be NULL when the caller sets a.out itself
@@ -343,6 +343,7 @@ static int decode_step_args(castle::DecodeArgs& a, const castle_view4* U, const 
   a.qu = to_view(qu); a.ku = to_view(ku); a.vu = to_view(vu);
   a.out = to_view(out);
   a.part = static_cast<float*>(workspace);
+  a.arrivals = nullptr;
   a.pend_vu = to_view(deferred != nullptr ? &deferred->vu_ring : nullptr);
   a.pend_gate = to_view(deferred != nullptr ? &deferred->gates : nullptr);
   a.base0 = deferred != nullptr ? deferred->base : 0;
@@ -427,7 +428,9 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
                             &tok[0], &tok[1], &tok[2], B, H, d, dtype, scale, flags, nullptr, deferred, workspace, workspace_bytes, false);
   if (rc != CASTLE_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  rc = castle::launch_small_linear(x, w_in, proj, B, width, dim, ldx, ldw_in, width, dtype, norm_weight, eps, CASTLE_ACT_NONE, nullptr, 0, s);
+  // the projection clears the arrival counts of the step, which then needs no launch to merge its splits
+  a.arrivals = reinterpret_cast<int*>(a.part + (int64_t)B * H * 64 * (d + 2));
+  rc = castle::launch_small_linear(x, w_in, proj, B, width, dim, ldx, ldw_in, width, dtype, norm_weight, eps, CASTLE_ACT_NONE, nullptr, 0, s, a.arrivals, B * H);
   a.out = to_view(&tok[0]);   // the attention output goes into the scratch: its token operands are spent by then
   if (rc == 0) rc = castle::launch_decode(a, dtype, s);
   if (rc != 0) return rc;

@@ -7,9 +7,10 @@
 // The pass is bandwidth bound: each cached element of qu, U, kc, vc is read once and U is
 // written once (5 * t * d elements per head and step).  The t rows of one (b, h) are split
 // over `splits` workgroups that each keep an online-softmax partial (acc, m, l) in fp32; the last
-// of them also takes row t and appends the new rows; decode_finish_kernel merges the partials.  (Letting
-// every workgroup of the output projection merge them while it loads its operand saves that launch and is
-// slower: 14.7 against 13.4 us for a whole layer step of one sequence, 31 against 23 us for 16.)
+// of them also takes row t and appends the new rows.  The partials are merged by the split that finishes last, where
+// a launch in front has cleared the arrival counts (castle_decode_layer), else by decode_finish_kernel.  (Letting
+// every workgroup of the output projection merge them while it loads its operand is slower: 14.7 against 13.4 us
+// for a whole layer step of one sequence, 31 against 23 us for 16.)
 #include "castle_tiles.h"
 #include "castle_params.h"
 #include "castle_profile.h"
@@ -79,6 +80,12 @@ __device__ __forceinline__ float* part_acc(const DecodeArgs& a, int bh, int spli
 __device__ __forceinline__ float* part_stat(const DecodeArgs& a, int bh, int split, int HD) {
   return a.part + (int64_t)a.B * a.H * a.splits * HD + ((int64_t)bh * a.splits + split) * 2;
 }
+
+// Partials cross from one XCD's L2 to another's inside a launch: stored and loaded at agent scope (write-through, no hit in a
+// stale L2), with the stores complete before the arrival is counted.  A fence would write the whole L2 back instead, dirty
+// lookahead-key rows included.
+__device__ __forceinline__ void agent_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float agent_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // One workgroup = 4 waves; a group of LPR = d / V lanes owns one cache row per iteration.
 template <typename T, int HD, bool UH>
@@ -297,8 +304,65 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
       out = __builtin_fmaf(w, s_acc[r][tid], out);
       lsum = __builtin_fmaf(w, s_acc[r][HD + 1], lsum);
     }
-    part_acc(a, bh, split, HD)[tid] = out;
-    if (tid == 0) { part_stat(a, bh, split, HD)[0] = M; part_stat(a, bh, split, HD)[1] = lsum; }
+    if (a.arrivals != nullptr && a.splits == 1) {
+      if (in_range) view_row<T>(a.out, b, h, 0)[tid] = (T)(out / lsum);
+    } else {
+      agent_store(part_acc(a, bh, split, HD) + tid, out);
+      if (tid == 0) { agent_store(part_stat(a, bh, split, HD), M); agent_store(part_stat(a, bh, split, HD) + 1, lsum); }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+  }
+  if (a.arrivals == nullptr || a.splits == 1) return;
+  __syncthreads();
+  __shared__ int s_last;
+  if (tid == 0) s_last = __hip_atomic_fetch_add(a.arrivals + bh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.splits - 1;
+  __syncthreads();
+  if (!s_last || !in_range) return;
+  // the last split: lane s of every wave holds the statistics of split s (at most 64), a wave sums every fourth partial
+  constexpr int EPL = (HD + 63) / 64;
+  const int lane = tid & 63;
+  const float ms = lane < a.splits ? agent_load(part_stat(a, bh, lane, HD)) : -INFINITY;
+  const float ls = lane < a.splits ? agent_load(part_stat(a, bh, lane, HD) + 1) : 0.f;
+  float sum[EPL];
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) sum[e] = 0.f;
+  constexpr int SU = 4;   // partials of a wave in flight
+  float wgt = 0.f, lsum = 0.f;
+  for (int s0 = wave; s0 < a.splits; s0 += SU * NW) {
+    float v[SU][EPL];
+#pragma unroll
+    for (int u = 0; u < SU; ++u)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        const int s = s0 + u * NW, n = lane + 64 * e;
+        v[u][e] = s < a.splits && n < HD ? agent_load(part_acc(a, bh, s, HD) + n) : 0.f;
+      }
+    if (s0 == wave) {   // the statistics arrive with the first partials
+      float M = ms;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+      wgt = ms == -INFINITY ? 0.f : fast_exp2(ms - M);
+      lsum = wgt * ls;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) lsum += __shfl_xor(lsum, o);
+    }
+#pragma unroll
+    for (int u = 0; u < SU; ++u) {
+      const float w = __shfl(wgt, (s0 + u * NW) & 63);   // 0 for lanes beyond the splits
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) sum[e] = __builtin_fmaf(w, v[u][e], sum[e]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < EPL; ++e)
+    if (lane + 64 * e < HD) s_acc[wave][lane + 64 * e] = sum[e];
+  if (lane == 0 && wave == 0) s_acc[0][HD] = lsum;   // wave 0 has split 0, so it has formed the sum
+  __syncthreads();
+  if (tid < HD) {
+    float o = 0.f;
+#pragma unroll
+    for (int r = 0; r < NW; ++r) o += s_acc[r][tid];
+    view_row<T>(a.out, b, h, 0)[tid] = (T)(o / s_acc[0][HD]);
   }
 }
 
@@ -404,7 +468,7 @@ template <typename T, int HD> static int launch_decode_t(const DecodeArgs& a, hi
       hipLaunchKernelGGL((decode_stream_kernel<T, HD, false>), dim3(a.splits, BH), dim3(kThreads), 0, stream, a);
     }
   }
-  {
+  if (a.arrivals == nullptr) {
     ProfScope ps(kSlotDecodeFinish, stream);
     hipLaunchKernelGGL((decode_finish_kernel<T, HD>), dim3(BH), dim3(64), 0, stream, a);
   }
@@ -527,6 +591,8 @@ struct LinearArgs {
   int act;
   const void* res;
   int64_t ldr;
+  int* clear;   // clear_n words set to zero for the launch behind this one
+  int clear_n;
 };
 typedef vec<float, 4> acc4_t;
 __device__ __forceinline__ void mma16(acc4_t& c, const vec<bf16_t, 8>& a, const vec<bf16_t, 8>& b) {
@@ -552,6 +618,8 @@ __global__ __launch_bounds__(64 * W) void small_linear_kernel(LinearArgs a) {
   __shared__ float ssq[W][16 * MT];
   const int lane = lane_id(), wave = wave_id(), c = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = threadIdx.x; i < a.clear_n; i += 64 * W) a.clear[i] = 0;
   const int steps = (a.K + DEPTH - 1) / DEPTH;
   const int per = (steps + W - 1) / W;
   const int s_end = min(steps, (wave + 1) * per);
@@ -659,8 +727,8 @@ template <typename T> static void launch_linear_t(const LinearArgs& a, hipStream
 #undef CASTLE_LINEAR
 }
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
-                        int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream) {
-  const LinearArgs a = {x, w, y, M, N, K, ldx, ldw, ldy, norm_w, eps, act, res, ldr};
+                        int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream, int* clear, int clear_n) {
+  const LinearArgs a = {x, w, y, M, N, K, ldx, ldw, ldy, norm_w, eps, act, res, ldr, clear, clear_n};
   switch (dtype) {
     case 0: launch_linear_t<float>(a, stream); break;
     case 1: launch_linear_t<bf16_t>(a, stream); break;

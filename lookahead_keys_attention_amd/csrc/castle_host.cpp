@@ -319,6 +319,46 @@ std::tuple<Tensor, Tensor> norm_rows_bwd(const Tensor& dh_, const Tensor& x, con
   return {dx, dw};
 }
 
+// The norm as a registered operator, for callers that are traced: what they record is what an untraced layer runs.
+std::tuple<Tensor, Tensor> rms_norm_op(const Tensor& x, const Tensor& weight, std::optional<double> eps) {
+  const c10::DeviceGuard guard(x.device());
+  const Normed n = norm_rows(x.reshape({-1, x.size(-1)}), Tensor(), weight, eps, true);
+  return {n.h.view(x.sizes()), n.rstd};
+}
+std::tuple<Tensor, Tensor> rms_norm_bwd_op(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight) {
+  const c10::DeviceGuard guard(x.device());
+  const int64_t D = x.size(-1);
+  auto [dx, dw] = norm_rows_bwd(dh.reshape({-1, D}), row_major(x.reshape({-1, D})), rstd, weight, Tensor(), true, true);
+  return {dx.view(x.sizes()), dw};
+}
+struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, std::optional<double> eps) {
+    static const auto op = op_handle<decltype(rms_norm_op)>("castle_hip::rms_norm");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    auto [h, rstd] = op.call(x, weight, eps);
+    ctx->save_for_backward({x, rstd, weight});
+    ctx->mark_non_differentiable({rstd});
+    ctx->set_materialize_grads(false);
+    return {h, rstd};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    static const auto op = op_handle<decltype(rms_norm_bwd_op)>("castle_hip::rms_norm_bwd");
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    const auto s = ctx->get_saved_variables();
+    auto [dx, dw] = op.call(g[0], s[0], s[1], s[2]);
+    return {dx, dw, Tensor()};
+  }
+};
+std::tuple<Tensor, Tensor> rms_norm_autograd(const Tensor& x, const Tensor& weight, std::optional<double> eps) {
+  if (!wants_graph({x, weight})) {
+    static const auto op = op_handle<decltype(rms_norm_op)>("castle_hip::rms_norm");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(x, weight, eps);
+  }
+  auto r = RmsNormFn::apply(x, weight, eps);
+  return {r[0], r[1]};
+}
+
 // ---- projections -----------------------------------------------------------------------------------------------
 // The weight gradient of a projection over many rows, dW = dY^T x, is a product with a small output
 // (out_features x in_features) and a long contraction (the rows): the GEMM the library picks leaves most of
@@ -748,12 +788,16 @@ TORCH_LIBRARY(castle_hip, m) {
         "-> (Tensor, Tensor, Tensor, Tensor)", tags);
   m.def("attention_packed_bwd(Tensor proj, Tensor merged, Tensor dmerged, Tensor ws, Tensor state, int heads, float scale, int flags) "
         "-> Tensor", tags);
+  m.def("rms_norm(Tensor x, Tensor weight, float? eps) -> (Tensor, Tensor)", tags);
+  m.def("rms_norm_bwd(Tensor dh, Tensor x, Tensor rstd, Tensor weight) -> (Tensor, Tensor)", tags);
 }
 TORCH_LIBRARY_IMPL(castle_hip, CUDA, m) {
   m.impl("attention", &attention);
   m.impl("attention_bwd", &attention_bwd);
   m.impl("attention_packed", &attention_packed);
   m.impl("attention_packed_bwd", &attention_packed_bwd);
+  m.impl("rms_norm", &rms_norm_op);
+  m.impl("rms_norm_bwd", &rms_norm_bwd_op);
 }
 // CPU tensors: an error that says what is wrong
 TORCH_LIBRARY_IMPL(castle_hip, CPU, m) {
@@ -763,6 +807,7 @@ TORCH_LIBRARY_IMPL(castle_hip, CPU, m) {
 TORCH_LIBRARY_IMPL(castle_hip, Autograd, m) {
   m.impl("attention", &attention_autograd);
   m.impl("attention_packed", &attention_packed_autograd);
+  m.impl("rms_norm", &rms_norm_autograd);
 }
 
 PYBIND11_MODULE(_castle_host, m) {

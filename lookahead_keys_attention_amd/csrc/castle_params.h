@@ -110,6 +110,7 @@ struct DecodeArgs {
   View4 U, qu_cache, kc_cache, vc_cache;   // capacity buffers, row t is appended
   View4 qc, kc, vc, qu, ku, vu;            // new token, L == 1
   View4 out;                               // (B, H, 1, d)
+  int* arrivals;    // [B*H] zero before the launch: the last split of a (b, h) to finish merges the partials; nullptr: a launch of its own does
   float* part;      // partial results: sums [B*H][splits][d], then statistics [B*H][splits][2] (maximum, sum of weights)
   // deferred write-back (pend_ku.ptr == nullptr: U is written every step)
   View4 pend_vu;            // (B, H, kDecodeDefer, d): row j % kDecodeDefer holds vu of token j (rotated when rotary)
