@@ -16,6 +16,7 @@
 #include "castle_profile.h"
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace castle {
 
@@ -87,22 +88,34 @@ __device__ __forceinline__ float* part_stat(const DecodeArgs& a, int bh, int spl
 __device__ __forceinline__ void agent_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float agent_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// One workgroup = 4 waves; a group of LPR = d / V lanes owns one cache row per iteration.
+// A group of LPR = d / V lanes owns one cache row per iteration.  (Workgroups of 16 waves, so that a head needs no
+// split and no merge, are slower throughout: 23.1 against 21.7 us for a layer step of 16 x 8 heads of 540 rows.)
+//
+// On three of four steps no lookahead key is written, and then none is formed either: qc . U_k of the completed key is
+// qc . U_k of the stored one plus a gate times qc . vu for every pending token, which is one number per token and
+// head.  (180 vector instructions per row and lane with the completed key in registers, 110 without: at 16 x 8 heads x
+// 540 rows they took as long as the memory.)
 template <typename T, int HD, bool UH>
-__global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a) {
   constexpr int V = elem_traits<T>::vec16;   // elements per 16-byte lane load
   constexpr int LPR = HD / V;                // lanes per row
   constexpr int RPI = kThreads / LPR;        // rows per workgroup iteration
-  typedef vec<T, V> vt;
   constexpr int NW = kThreads / 64;
+  typedef vec<T, V> vt;
   __shared__ float s_acc[NW][HD + 2];
+  __shared__ float s_vu[kDecodeDefer + 1][HD];   // vu of the pending tokens by ring slot and of the new one, for steps that write U
 
   const int split = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
+  const int tid = threadIdx.x;
+  const int grp = tid / LPR, sub = tid % LPR;
+  // All loads of the start go out together, the small ones first (they are waited for first): the token's pieces,
+  // which do not need the row count, then the pending tokens' vu pieces and the rows of the first iteration.
+  const vt tku = *reinterpret_cast<const vt*>(view_row<T>(a.ku, b, h, 0) + sub * V);
+  const vt tvu = *reinterpret_cast<const vt*>(view_row<T>(a.vu, b, h, 0) + sub * V);
+  const vt tqc = *reinterpret_cast<const vt*>(view_row<T>(a.qc, b, h, 0) + sub * V);
   int t = a.t_dev != nullptr ? *a.t_dev : a.t;
   const bool in_range = t >= 0 && t < a.capacity;
   if (!in_range) t = 0;   // only with a device-side count: no rows, nothing is appended
-  const int tid = threadIdx.x;
-  const int grp = tid / LPR, sub = tid % LPR;
   const float c1 = a.scale * kLog2e;
 
   // rows of this workgroup: [r0, r1), whole iterations of RPI rows
@@ -116,11 +129,6 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
   const int pbase = deferred ? decode_base(base0, t) : t;
   const int np = t - pbase;                                        // 0 .. kDecodeDefer - 1
   const bool write_u = !deferred || (t + 1) % kDecodeDefer == 0;
-  // All loads of the start go out together, the small ones first (they are waited for first): the token's pieces, the
-  // pending tokens' vu pieces, the rows of the first iteration.
-  const vt tku = *reinterpret_cast<const vt*>(view_row<T>(a.ku, b, h, 0) + sub * V);
-  const vt tvu = *reinterpret_cast<const vt*>(view_row<T>(a.vu, b, h, 0) + sub * V);
-  const vt tqc = *reinterpret_cast<const vt*>(view_row<T>(a.qc, b, h, 0) + sub * V);
   const bool owner = split == (t > 0 ? (t - 1) / per : 0);
   vt tkc, tqu, tvc, tpv[kDecodeDefer];
   if (owner) {
@@ -128,146 +136,170 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
     tqu = *reinterpret_cast<const vt*>(view_row<T>(a.qu, b, h, 0) + sub * V);
     tvc = *reinterpret_cast<const vt*>(view_row<T>(a.vc, b, h, 0) + sub * V);
   }
+  int pend_j[kDecodeDefer];   // the token in a ring slot, or -1: a row k has a gate for token j if k < j
 #pragma unroll
   for (int sl = 0; sl < kDecodeDefer; ++sl) {
     const int j = pbase + ((sl - pbase % kDecodeDefer + kDecodeDefer) % kDecodeDefer);   // the token that would sit in this slot
+    pend_j[sl] = deferred && j < t ? j : -1;
 #pragma unroll
     for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
-    if (deferred && j < t) tpv[sl] = *reinterpret_cast<const vt*>(view_row<T>(a.pend_vu, b, h, sl) + sub * V);
+    if (pend_j[sl] >= 0) tpv[sl] = *reinterpret_cast<const vt*>(view_row<T>(a.pend_vu, b, h, sl) + sub * V);
   }
-  // The row pieces of the next PF iterations are requested before the current one is processed:
-  // PF + 1 times the bytes in flight per wave, which is what a latency-bound streaming loop is short of.
-  constexpr int PF = 1;
-  vt nq[PF], nu[PF], nk[PF], nv[PF];
-  vec<float, 4> ng[PF];
-#pragma unroll
-  for (int p = 0; p < PF; ++p) ng[p] = vec<float, 4>{0.f, 0.f, 0.f, 0.f};
+  // The row pieces of the next iteration are requested before the current one is processed.
+  vt nq, nu, nk, nv;
+  vec<float, 4> ng = {0.f, 0.f, 0.f, 0.f};
   float* const gbase = deferred ? reinterpret_cast<float*>(a.pend_gate.ptr) + (int64_t)b * a.pend_gate.sb + (int64_t)h * a.pend_gate.sh : nullptr;
-  auto request = [&](int p, int k) __attribute__((always_inline)) {
+  auto request = [&](int k) __attribute__((always_inline)) {
     if (k < r1) {
-      nq[p] = *reinterpret_cast<const vt*>(view_row<T>(a.qu_cache, b, h, k) + sub * V);
-      nu[p] = *reinterpret_cast<const vt*>(view_row<T>(a.U, b, h, k) + sub * V);
-      nk[p] = *reinterpret_cast<const vt*>(view_row<T>(a.kc_cache, b, h, k) + sub * V);
-      nv[p] = *reinterpret_cast<const vt*>(view_row<T>(a.vc_cache, b, h, k) + sub * V);
-      if (np > 0) ng[p] = *reinterpret_cast<const vec<float, 4>*>(gbase + (int64_t)k * kDecodeDefer);
+      nq = *reinterpret_cast<const vt*>(view_row<T>(a.qu_cache, b, h, k) + sub * V);
+      nu = *reinterpret_cast<const vt*>(view_row<T>(a.U, b, h, k) + sub * V);
+      nk = *reinterpret_cast<const vt*>(view_row<T>(a.kc_cache, b, h, k) + sub * V);
+      nv = *reinterpret_cast<const vt*>(view_row<T>(a.vc_cache, b, h, k) + sub * V);
+      if (np > 0) ng = *reinterpret_cast<const vec<float, 4>*>(gbase + (int64_t)k * kDecodeDefer);
     }
   };
-#pragma unroll
-  for (int p = 0; p < PF; ++p) request(p, r0 + grp + p * RPI);
+  request(r0 + grp);
   __builtin_amdgcn_sched_barrier(0);
-  float ku[V], vu[V], qc[V], pv[kDecodeDefer][V];   // pv by ring slot: zero where no pending token sits
-#pragma unroll
-  for (int e = 0; e < V; ++e) {
-    ku[e] = (float)tku[e];
-    vu[e] = (float)tvu[e];
-    qc[e] = (float)tqc[e];
-#pragma unroll
-    for (int sl = 0; sl < kDecodeDefer; ++sl) pv[sl][e] = (float)tpv[sl][e];
-  }
-  if (a.rotary) {   // the new token sits at position t
-#pragma unroll
-    for (int e = 0; e < V / 2; ++e) {
-      const int pair = sub * (V / 2) + e;
-      CASTLE_ROPE_PAIR(ku[2 * e], ku[2 * e + 1], (float)t, pair, HD, false);
-      CASTLE_ROPE_PAIR(vu[2 * e], vu[2 * e + 1], (float)t, pair, HD, false);
-      CASTLE_ROPE_PAIR(qc[2 * e], qc[2 * e + 1], (float)t, pair, HD, false);
-    }
-  }
+  float ku[V], qc[V], acc[V], m = -INFINITY, l = 0.f;   // ku, qc times c1: products come out in log2 units
+  float cvu[kDecodeDefer], cvu_t;                       // c1 qc . vu of the pending tokens and of the new one
   const int slot_t = t % kDecodeDefer;
-
-  float acc[V];
+  {
+    float vu[V];
 #pragma unroll
-  for (int e = 0; e < V; ++e) acc[e] = 0.f;
-  float m = -INFINITY, l = 0.f;
-
-  // The last split that has rows takes row t too: U_t = 0, so its lookahead term is silu(0) = 0, and appends the
-  // new rows.  No workgroup of this launch reads row t or the ring slot of token t.
-  if (owner && grp == 0) {
-    float kct[V], qut[V];
-#pragma unroll
-    for (int e = 0; e < V; ++e) { kct[e] = (float)tkc[e]; qut[e] = (float)tqu[e]; acc[e] = (float)tvc[e]; }
-    if (a.rotary) {
+    for (int e = 0; e < V; ++e) {
+      ku[e] = (float)tku[e];
+      vu[e] = (float)tvu[e];
+      qc[e] = (float)tqc[e];
+      acc[e] = 0.f;
+    }
+    if (a.rotary) {   // the new token sits at position t
 #pragma unroll
       for (int e = 0; e < V / 2; ++e) {
         const int pair = sub * (V / 2) + e;
-        CASTLE_ROPE_PAIR(kct[2 * e], kct[2 * e + 1], (float)t, pair, HD, false);
-        CASTLE_ROPE_PAIR(qut[2 * e], qut[2 * e + 1], (float)t, pair, HD, false);
+        CASTLE_ROPE_PAIR(ku[2 * e], ku[2 * e + 1], (float)t, pair, HD, false);
+        CASTLE_ROPE_PAIR(vu[2 * e], vu[2 * e + 1], (float)t, pair, HD, false);
+        CASTLE_ROPE_PAIR(qc[2 * e], qc[2 * e + 1], (float)t, pair, HD, false);
       }
     }
-    float dot = 0.f;
+    cvu_t = 0.f;
 #pragma unroll
-    for (int e = 0; e < V; ++e) dot = __builtin_fmaf(qc[e], kct[e], dot);
-    m = group_sum<LPR>(dot) * c1;
-    l = 1.f;
-    if (in_range) {
-      vt z, q, kk, v, p;
+    for (int e = 0; e < V; ++e) {
+      ku[e] *= c1;
+      qc[e] *= c1;
+      cvu_t = __builtin_fmaf(qc[e], vu[e], cvu_t);
+    }
+    cvu_t = group_sum<LPR>(cvu_t);
 #pragma unroll
-      for (int e = 0; e < V; ++e) { z[e] = (T)0.f; q[e] = (T)qut[e]; kk[e] = (T)kct[e]; v[e] = (T)acc[e]; p[e] = (T)vu[e]; }
-      *reinterpret_cast<vt*>(view_row<T>(a.U, b, h, t) + sub * V) = z;
-      *reinterpret_cast<vt*>(view_row<T>(a.qu_cache, b, h, t) + sub * V) = q;
-      *reinterpret_cast<vt*>(view_row<T>(a.kc_cache, b, h, t) + sub * V) = kk;
-      *reinterpret_cast<vt*>(view_row<T>(a.vc_cache, b, h, t) + sub * V) = v;
-      if (deferred) *reinterpret_cast<vt*>(view_row<T>(a.pend_vu, b, h, slot_t) + sub * V) = p;   // joins the pending sources
+    for (int sl = 0; sl < kDecodeDefer; ++sl) {
+      float c = 0.f;
+#pragma unroll
+      for (int e = 0; e < V; ++e) c = __builtin_fmaf(qc[e], (float)tpv[sl][e], c);
+      cvu[sl] = group_sum<LPR>(c);
+    }
+    if (write_u && grp == 0) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+#pragma unroll
+        for (int sl = 0; sl < kDecodeDefer; ++sl) s_vu[sl][sub * V + e] = (float)tpv[sl][e];
+        s_vu[kDecodeDefer][sub * V + e] = vu[e];
+      }
+    }
+    // The last split that has rows takes row t too: U_t = 0, so its lookahead term is silu(0) = 0, and appends the
+    // new rows.  No workgroup of this launch reads row t or the ring slot of token t.
+    if (owner && grp == 0) {
+      float kct[V], qut[V];
+#pragma unroll
+      for (int e = 0; e < V; ++e) { kct[e] = (float)tkc[e]; qut[e] = (float)tqu[e]; acc[e] = (float)tvc[e]; }
+      if (a.rotary) {
+#pragma unroll
+        for (int e = 0; e < V / 2; ++e) {
+          const int pair = sub * (V / 2) + e;
+          CASTLE_ROPE_PAIR(kct[2 * e], kct[2 * e + 1], (float)t, pair, HD, false);
+          CASTLE_ROPE_PAIR(qut[2 * e], qut[2 * e + 1], (float)t, pair, HD, false);
+        }
+      }
+      float dot = 0.f;
+#pragma unroll
+      for (int e = 0; e < V; ++e) dot = __builtin_fmaf(qc[e], kct[e], dot);
+      m = group_sum<LPR>(dot);
+      l = 1.f;
+      if (in_range) {
+        vt z, q, kk, v, p;
+#pragma unroll
+        for (int e = 0; e < V; ++e) { z[e] = (T)0.f; q[e] = (T)qut[e]; kk[e] = (T)kct[e]; v[e] = (T)acc[e]; p[e] = (T)vu[e]; }
+        *reinterpret_cast<vt*>(view_row<T>(a.U, b, h, t) + sub * V) = z;
+        *reinterpret_cast<vt*>(view_row<T>(a.qu_cache, b, h, t) + sub * V) = q;
+        *reinterpret_cast<vt*>(view_row<T>(a.kc_cache, b, h, t) + sub * V) = kk;
+        *reinterpret_cast<vt*>(view_row<T>(a.vc_cache, b, h, t) + sub * V) = v;
+        if (deferred) *reinterpret_cast<vt*>(view_row<T>(a.pend_vu, b, h, slot_t) + sub * V) = p;   // joins the pending sources
+      }
     }
   }
 
-  for (int base = r0; base < r1; base += PF * RPI) {
-#pragma unroll
-    for (int p = 0; p < PF; ++p) {
-    const int k = base + p * RPI + grp;
-    const vt cq = nq[p], cu = nu[p], ck = nk[p], cv = nv[p];
-    const vec<float, 4> g4 = ng[p];
-    request(p, k + PF * RPI);
-    if (k < r1) {
-      float quk[V], uk[V], kck[V], vck[V];
-      T* urow = view_row<T>(a.U, b, h, k) + sub * V;
-#pragma unroll
-      for (int e = 0; e < V; ++e) { quk[e] = (float)cq[e]; kck[e] = (float)ck[e]; vck[e] = (float)cv[e]; }
-      u_unpack<T, V, UH>(cu, uk);
-      // pending sources j > k first (none unless the write-back is deferred): their gates were
-      // formed by the steps that appended them and wait in the row's side array
-      float* grow = deferred ? gbase + (int64_t)k * kDecodeDefer : nullptr;
-      if (np > 0) {
-#pragma unroll
-        for (int sl = 0; sl < kDecodeDefer; ++sl) {
-          const int j = pbase + ((sl - pbase % kDecodeDefer + kDecodeDefer) % kDecodeDefer);
-          const float gj = (j < t && j > k) ? g4[sl] : 0.f;   // rows appended inside the window have no gate for earlier tokens
-#pragma unroll
-          for (int e = 0; e < V; ++e) uk[e] = __builtin_fmaf(gj, pv[sl][e], uk[e]);
-        }
-      }
-      float dg = 0.f;
-#pragma unroll
-      for (int e = 0; e < V; ++e) dg = __builtin_fmaf(quk[e], ku[e], dg);
-      dg = group_sum<LPR>(dg);
-      const float gate = sigmoid_l2(dg * c1);
-#pragma unroll
-      for (int e = 0; e < V; ++e) uk[e] = __builtin_fmaf(gate, vu[e], uk[e]);
-      if (write_u) {
-        // the lookahead key as later steps will see it: the stored (rounded) one when it is written now
-        const vt unew = u_pack<T, V, UH>(uk);
-        *reinterpret_cast<vt*>(urow) = unew;
-        u_unpack<T, V, UH>(unew, uk);
-      } else if (sub == 0) {
-        grow[slot_t] = gate;   // the new token stays pending: its gate for this row
-      }
-      float dsu = 0.f, dsc = 0.f;
+  auto rows = [&](auto writes) __attribute__((always_inline)) {
+    for (int k = r0 + grp; k < r1; k += RPI) {
+      const vt cq = nq, cu = nu, ck = nk, cv = nv;
+      const vec<float, 4> g4 = ng;
+      request(k + RPI);
+      float dg = 0.f, dsc = 0.f, dsu = 0.f;
 #pragma unroll
       for (int e = 0; e < V; ++e) {
-        dsu = __builtin_fmaf(qc[e], uk[e], dsu);
-        dsc = __builtin_fmaf(qc[e], kck[e], dsc);
+        dg = __builtin_fmaf((float)cq[e], ku[e], dg);
+        dsc = __builtin_fmaf((float)ck[e], qc[e], dsc);
       }
-      dsu = group_sum<LPR>(dsu);
-      dsc = group_sum<LPR>(dsc);
-      const float x = (dsc - dsu * sigmoid_l2(dsu * c1)) * c1;   // score in log2 units
+      const float gate = sigmoid_l2(group_sum<LPR>(dg));
+      // pending sources j > k first (none unless the write-back is deferred): their gates were formed by the steps
+      // that appended them and wait in the row's side array (rows appended inside the window have none for earlier tokens)
+      float gj[kDecodeDefer];
+#pragma unroll
+      for (int sl = 0; sl < kDecodeDefer; ++sl) gj[sl] = k < pend_j[sl] ? g4[sl] : 0.f;
+      if constexpr (decltype(writes)::value) {
+        float uk[V];
+        u_unpack<T, V, UH>(cu, uk);
+        asm volatile("" ::: "memory");   // s_vu is read again for every row: held in registers it would cost 40 of them
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+#pragma unroll
+          for (int sl = 0; sl < kDecodeDefer; ++sl) uk[e] = __builtin_fmaf(gj[sl], s_vu[sl][sub * V + e], uk[e]);
+          uk[e] = __builtin_fmaf(gate, s_vu[kDecodeDefer][sub * V + e], uk[e]);
+        }
+        // the lookahead key as later steps will see it: the stored (rounded) one
+        const vt unew = u_pack<T, V, UH>(uk);
+        *reinterpret_cast<vt*>(view_row<T>(a.U, b, h, k) + sub * V) = unew;
+        u_unpack<T, V, UH>(unew, uk);
+#pragma unroll
+        for (int e = 0; e < V; ++e) dsu = __builtin_fmaf(qc[e], uk[e], dsu);
+        dsu = group_sum<LPR>(dsu);
+      } else {
+        if constexpr (UH) {
+          const vec<fp16_t, V> u = __builtin_bit_cast(vec<fp16_t, V>, cu);
+#pragma unroll
+          for (int e = 0; e < V; ++e) dsu = __builtin_fmaf((float)u[e], qc[e], dsu);
+          dsu = group_sum<LPR>(dsu) * kUHalfUnscale;
+        } else {
+#pragma unroll
+          for (int e = 0; e < V; ++e) dsu = __builtin_fmaf((float)cu[e], qc[e], dsu);
+          dsu = group_sum<LPR>(dsu);
+        }
+#pragma unroll
+        for (int sl = 0; sl < kDecodeDefer; ++sl) dsu = __builtin_fmaf(gj[sl], cvu[sl], dsu);
+        dsu = __builtin_fmaf(gate, cvu_t, dsu);
+        if (sub == 0) gbase[(int64_t)k * kDecodeDefer + slot_t] = gate;   // the new token stays pending: its gate for this row
+      }
+      const float x = group_sum<LPR>(dsc) - dsu * sigmoid_l2(dsu);   // score in log2 units
       const float mn = fmaxf(m, x);
       const float al = fast_exp2(m - mn), p_ = fast_exp2(x - mn);
       l = l * al + p_;
 #pragma unroll
-      for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(p_, vck[e], acc[e] * al);
+      for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(p_, (float)cv[e], acc[e] * al);
       m = mn;
     }
-    }
+  };
+  if (write_u) {
+    __syncthreads();   // s_vu
+    rows(std::true_type());
+  } else {
+    rows(std::false_type());
   }
   // merge the row groups of a wave in registers, then the waves through LDS
   {
@@ -304,7 +336,7 @@ __global__ __launch_bounds__(kThreads) void decode_stream_kernel(DecodeArgs a) {
       out = __builtin_fmaf(w, s_acc[r][tid], out);
       lsum = __builtin_fmaf(w, s_acc[r][HD + 1], lsum);
     }
-    if (a.arrivals != nullptr && a.splits == 1) {
+    if (a.splits == 1) {
       if (in_range) view_row<T>(a.out, b, h, 0)[tid] = (T)(out / lsum);
     } else {
       agent_store(part_acc(a, bh, split, HD) + tid, out);
@@ -458,19 +490,18 @@ __global__ __launch_bounds__(kThreads) void decode_flush_kernel(DecodeArgs a) {
 }
 
 template <typename T, int HD> static int launch_decode_t(const DecodeArgs& a, hipStream_t stream) {
-  const int BH = a.B * a.H;
   {
     ProfScope ps(kSlotDecodeStream, stream);
     if constexpr (__is_same(T, bf16_t)) {
-      if (a.u_half) hipLaunchKernelGGL((decode_stream_kernel<T, HD, true>), dim3(a.splits, BH), dim3(kThreads), 0, stream, a);
-      else hipLaunchKernelGGL((decode_stream_kernel<T, HD, false>), dim3(a.splits, BH), dim3(kThreads), 0, stream, a);
+      if (a.u_half) hipLaunchKernelGGL((decode_stream_kernel<T, HD, true>), dim3(a.splits, a.B * a.H), dim3(kThreads), 0, stream, a);
+      else hipLaunchKernelGGL((decode_stream_kernel<T, HD, false>), dim3(a.splits, a.B * a.H), dim3(kThreads), 0, stream, a);
     } else {
-      hipLaunchKernelGGL((decode_stream_kernel<T, HD, false>), dim3(a.splits, BH), dim3(kThreads), 0, stream, a);
+      hipLaunchKernelGGL((decode_stream_kernel<T, HD, false>), dim3(a.splits, a.B * a.H), dim3(kThreads), 0, stream, a);
     }
   }
-  if (a.arrivals == nullptr) {
+  if (a.splits > 1 && a.arrivals == nullptr) {
     ProfScope ps(kSlotDecodeFinish, stream);
-    hipLaunchKernelGGL((decode_finish_kernel<T, HD>), dim3(BH), dim3(64), 0, stream, a);
+    hipLaunchKernelGGL((decode_finish_kernel<T, HD>), dim3(a.B * a.H), dim3(64), 0, stream, a);
   }
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
@@ -907,8 +938,8 @@ int decode_static_scratch(float** ptr) {
   return 0;
 }
 
-// How many workgroups share the t rows of one (b, h).  Three workgroups fit a CU (137 registers), so a launch runs
-// in rounds of 3 CUs; a workgroup costs its iterations plus about two more for its start and end.  Fewest rounds x
+// How many workgroups share the t rows of one (b, h).  Three workgroups a CU keep the memory busy (a
+// fourth fits, and is not faster), so a launch runs in rounds of 3 CUs; a workgroup costs its iterations plus about two more for its start and end.  Fewest rounds x
 // iterations wins, at least two iterations each.  45 x 6 heads of 450 rows: 26.1 us with the 2 splits this picks, 27.6
 // with the 3 that fill a round and a straggling 5 % of the next; 16 x 8 heads of 540 rows: 16.6 us with one round,
 // 20.7 with two.
