@@ -286,6 +286,20 @@ int64_t castle_rms_norm_bwd_workspace_bytes(int64_t rows, int width, int dtype);
 int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
                         int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* c[M, N] = the product of two matrices over K, in the type `dtype` with fp32 sums: the projections of a layer and their
+ * gradients over hundreds to thousands of rows (nn.Linear at lookahead_keys_attention.py:75, 80, 99, 209).  An operand
+ * is contraction-contiguous (a: M rows of K, b: N rows of K) or, with its flag set, free-contiguous (K rows of M or N); a
+ * free-contiguous a needs a free-contiguous b.  Rows are whole 16-byte pieces, as are leading dimensions and N.
+ * epilogue: CASTLE_GEMM_GELU also writes gelu(c) (erf form) to aux, CASTLE_GEMM_GELU_SLOPE multiplies the product by the
+ * derivative of gelu at aux; aux has c's shape and leading dimension.  A workspace of castle_gemm_workspace_bytes
+ * (0 when the contraction is not split; then ldc may exceed N). */
+#define CASTLE_GEMM_PLAIN 0
+#define CASTLE_GEMM_GELU 1
+#define CASTLE_GEMM_GELU_SLOPE 2
+int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue);
+int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
+                int M, int N, int K, int dtype, int epilogue, void* aux, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* out[i] = sum over p < parts of part[p * n + i], n % 8 == 0: partial products of a weight gradient. */
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream);
 

@@ -47,6 +47,8 @@ EXPORTED_SYMBOLS = (
     "castle_sample",
     "castle_gather_rows",
     "castle_small_linear_fused",
+    "castle_gemm_workspace_bytes",
+    "castle_gemm",
     "castle_rms_norm",
     "castle_rms_norm_bwd_workspace_bytes",
     "castle_rms_norm_bwd",

@@ -371,10 +371,15 @@ class Castle(nn.Module):
             assert cache is None, "must be inferencing single tokens if receiving cache"
             return self._layer_native(x, return_next_cache)
         native_step = single and native
-        norm = self.norm
-        if native and not single and torch.compiler.is_compiling() and type(norm) is nn.RMSNorm and norm.weight.dtype == x.dtype:
-            x, norm = torch.ops.castle_hip.rms_norm(x, norm.weight, norm.eps)[0], None   # what the untraced layer runs
-        proj = self._project(self.to_all_qkv, x, native_step, norm=norm)
+        if native and not single and torch.compiler.is_compiling() and self._traceable(x):
+            # the operators of this library, one by one: what the untraced layer runs
+            assert cache is None, "must be inferencing single tokens if receiving cache"
+            if type(self.norm) is nn.RMSNorm:
+                x = torch.ops.castle_hip.rms_norm(x, self.norm.weight, self.norm.eps)[0]
+            merged, next_cache = self._parallel_native(torch.ops.castle_hip.linear(x, self.to_all_qkv.weight), return_next_cache)
+            y = torch.ops.castle_hip.linear(merged, self.combine_heads.weight)
+            return (y, next_cache) if return_next_cache else y
+        proj = self._project(self.to_all_qkv, x, native_step, norm=self.norm)
         if not single:
             assert cache is None, "must be inferencing single tokens if receiving cache"
             merged, next_cache = (self._parallel_native if native else self._parallel_dense)(proj, return_next_cache)
@@ -411,6 +416,13 @@ class Castle(nn.Module):
                     or layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks):
                 return False
         return True
+
+    def _traceable(self, x):
+        """`_plain` as far as a tracing compiler can follow it."""
+        norm = self.norm
+        return (type(norm) is nn.Identity or type(norm) is nn.RMSNorm and norm.weight.dtype == x.dtype) and all(
+            type(layer) is nn.Linear and layer.bias is None and layer.weight.dtype == x.dtype for layer in (self.to_all_qkv, self.combine_heads)
+        ) and not torch.is_autocast_enabled("cuda")
 
     def _layer_native(self, x, want_cache, delta=None):
         """The parallel pass as one native call (csrc/castle_host.cpp): norm, projection, attention core,

@@ -7,6 +7,7 @@
 #include <stdlib.h>
 #include <initializer_list>
 #include "castle_params.h"
+#include "castle_gemm.h"
 #include "castle_profile.h"
 #include "castle_rows.h"
 #include "castle_tiles.h"
@@ -545,6 +546,32 @@ int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const
   if (dweight != nullptr && (workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
   const castle::NormBwdArgs a = {dh, x, weight, dres, rstd, dx, dweight != nullptr ? static_cast<float*>(workspace) : nullptr, rows, width};
   return castle::launch_norm_bwd(a, dweight, dtype, static_cast<hipStream_t>(stream));
+}
+
+int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (M <= 0 || N <= 0 || K <= 0 || N % (16 / es) != 0 || (int64_t)(M / 64 + 1) * (N / 64 + 1) > (int64_t)1 << 30) return CASTLE_ERR_SHAPE;
+  return align_up(castle::gemm_workspace(M, N, K, es, epilogue != CASTLE_GEMM_PLAIN), 256);
+}
+
+int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
+                int M, int N, int K, int dtype, int epilogue, void* aux, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t need = castle_gemm_workspace_bytes(M, N, K, dtype, epilogue);
+  if (need < 0) return (int)need;
+  static_assert(CASTLE_GEMM_PLAIN == castle::kGemmPlain && CASTLE_GEMM_GELU == castle::kGemmGelu && CASTLE_GEMM_GELU_SLOPE == castle::kGemmGeluSlope, "");
+  const int v = 16 / elem_size(dtype);
+  const int a_row = a_free_contiguous ? M : K, b_row = b_free_contiguous ? N : K;
+  if (a_row % v != 0 || b_row % v != 0 || lda < a_row || ldb < b_row || ldc < N || lda % v != 0 || ldb % v != 0 || ldc % v != 0 ||
+      (a_free_contiguous && !b_free_contiguous))
+    return CASTLE_ERR_SHAPE;
+  if (epilogue < CASTLE_GEMM_PLAIN || epilogue > CASTLE_GEMM_GELU_SLOPE || a == nullptr || b == nullptr || c == nullptr ||
+      (epilogue != CASTLE_GEMM_PLAIN && aux == nullptr) || !aligned16({a, b, c, aux}))
+    return CASTLE_ERR_ARG;
+  if (need > 0 && (ldc != N || (int64_t)M * N % 8 != 0)) return CASTLE_ERR_SHAPE;
+  if (need > 0 && (workspace == nullptr || !aligned16({workspace}) || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
+  const castle::GemmArgs args = {a, b, c, aux, M, N, K, lda, ldb, ldc, epilogue, 0, nullptr};
+  return castle::launch_gemm(args, !a_free_contiguous, !b_free_contiguous, dtype, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
 }
 
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream) {

@@ -1,0 +1,22 @@
+// Launcher of castle_gemm.hip.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace castle {
+
+enum { kGemmPlain = 0, kGemmGelu = 1, kGemmGeluSlope = 2 };
+struct GemmArgs {
+  const void *a, *b;   // contraction-contiguous: [free][ld], else [contraction][ld]
+  void* c;             // [M][ldc]; a product that is split over the contraction needs ldc == N
+  void* aux;           // kGemmGelu: gelu(c) goes here; kGemmGeluSlope: c is multiplied by the derivative of gelu at it; ldc rows
+  int M, N, K;
+  int64_t lda, ldb, ldc;
+  int epilogue;
+  int k_per_split;
+  float* part;
+};
+int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue);
+int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream);
+
+}  // namespace castle

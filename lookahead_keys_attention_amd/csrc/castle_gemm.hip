@@ -1,0 +1,244 @@
+// Products of a layer's projections over some hundreds to some thousands of rows:
+//   forward          y[R, N]  = x[R, K] w[N, K]^T          both operands contraction-contiguous
+//   input gradient   dx[R, K] = dy[R, N] w[N, K]           the second one stored [contraction][free]
+//   weight gradient  dw[N, K] = dy[R, N]^T x[R, K]         both stored [contraction][free]
+//
+// Why own kernels: a call of the library's product costs 18 us of host time, more than the whole product takes on the GPU
+// up to about 5 GFLOP, and its weight gradient walks all rows in one chain per output tile (1536 x 256 from 3000
+// rows: 30 us).  A launch here costs 4 us of host time, the rows of a weight gradient are split over workgroups, and GELU
+// and its derivative ride on the store.
+//
+// Four waves share a BM x BN tile of the output (2 x 2 quarters).  What bounds these sizes is latency: few workgroups on
+// a CU and a short contraction.  So the pieces of two steps of the contraction are in flight in registers while a third
+// is in LDS (two buffers, one barrier a step).  Operands stored [contraction][free] are copied as they are and
+// read with transpose reads.
+#include "castle_tiles.h"
+#include "castle_dispatch.h"
+#include "castle_gemm.h"
+#include <algorithm>
+#include "castle_rows.h"
+
+namespace castle {
+namespace {
+
+__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678f)); }
+__device__ __forceinline__ float gelu_slope(float x) {
+  return 0.5f * (1.f + erff(x * 0.70710678f)) + x * 0.3989422804f * fast_exp2(-0.5f * kLog2e * x * x);
+}
+
+// A tile of FREE rows / columns and BK steps of the contraction: global -> registers -> LDS -> operand fragments.
+// KC: the operand is contraction-contiguous (LDS [FREE][BK]), else stored [contraction][free] (LDS [BK][FREE]).
+template <typename T, bool KC, int FREE, int BK> struct Operand {
+  static constexpr int V = elem_traits<T>::vec16;
+  static constexpr int COLS = KC ? BK : FREE, ROWS = KC ? FREE : BK, VPR = COLS / V, N = ROWS * VPR / kThreads;
+  static constexpr int LD = KC ? lds_ld<T>(COLS) : lds_ld_tr<T>(COLS), ELEMS = ROWS * LD;
+  static_assert(ROWS * VPR % kThreads == 0, "a whole number of pieces per thread");
+  typedef vec<T, V> vt;
+  // where the pieces of this thread are, in elements from the operand's start: one addition per piece and step (formed
+  // from row and column each time they took longer than the products).  Pieces beyond the free end read another row's
+  // data: those outputs are not stored.
+  int at[N];
+  vt r[2][N];
+  static __device__ __forceinline__ int row_of(int j) { return (threadIdx.x + j * kThreads) / VPR; }
+  static __device__ __forceinline__ int col_of(int j) { return (threadIdx.x + j * kThreads) % VPR * V; }
+  __device__ __forceinline__ void start(int ld, int free0, int free_end, int k0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int f = free0 + (KC ? row_of(j) : col_of(j)), k = k0 + (KC ? col_of(j) : row_of(j));
+      at[j] = KC ? min(f, free_end - 1) * ld + k : k * ld + (f < free_end ? f : 0);
+    }
+  }
+  __device__ __forceinline__ void load(int slot, const T* p, int ld, int k, int k_end) {
+    if (k + BK <= k_end) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) r[slot][j] = *reinterpret_cast<const vt*>(p + at[j]);
+    } else {   // the last step: zeros behind the contraction's end
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) r[slot][j][e] = (T)0.f;
+        if (k + (KC ? col_of(j) : row_of(j)) < k_end) r[slot][j] = *reinterpret_cast<const vt*>(p + at[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) at[j] += KC ? BK : BK * ld;
+  }
+  __device__ __forceinline__ void store(int slot, T* lds) const {
+#pragma unroll
+    for (int j = 0; j < N; ++j) *reinterpret_cast<vt*>(lds + row_of(j) * LD + col_of(j)) = r[slot][j];
+  }
+  static __device__ __forceinline__ frag<T> read(const T* lds, int free0, int k0, int c, int g) {
+    if constexpr (KC) return ld_nat<T>(lds, LD, free0 + c, k0 + 8 * g);
+    else return ld_free<T, false>(lds, LD, free0, FREE, k0, c, g);
+  }
+};
+
+template <typename T, bool AK, bool BKC, int BM, int BN, int BK>
+__global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmArgs a) {
+  constexpr int WM = BM / 64, WN = BN / 64;   // 32-wide pieces of a wave's quarter
+  typedef Operand<T, AK, BM, BK> OpA;
+  typedef Operand<T, BKC, BN, BK> OpB;
+  constexpr int V = elem_traits<T>::vec16, LDC = BN + V;
+  constexpr int kStage = 2 * (OpA::ELEMS + OpB::ELEMS), kOut = BM * LDC;
+  __shared__ __attribute__((aligned(16))) T smem[kStage > kOut ? kStage : kOut];
+  const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
+  const int tiles_n = (a.N + BN - 1) / BN;
+  const int m0 = blockIdx.x / tiles_n * BM, n0 = blockIdx.x % tiles_n * BN;
+  const int wm = wave / 2 * (BM / 2), wn = wave % 2 * (BN / 2);
+  const int k0 = blockIdx.y * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split);
+  const int steps = (k_end - k0 + BK - 1) / BK;
+  const T *pa = static_cast<const T*>(a.a), *pb = static_cast<const T*>(a.b);
+  OpA ra;
+  OpB rb;
+  ra.start((int)a.lda, m0, a.M, k0);
+  rb.start((int)a.ldb, n0, a.N, k0);
+  acc_t acc[WM][WN];
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j) zero(acc[i][j]);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {   // (a second step beyond the end loads zeros)
+    ra.load(p, pa, (int)a.lda, k0 + p * BK, k_end);
+    rb.load(p, pb, (int)a.ldb, k0 + p * BK, k_end);
+  }
+  auto step = [&](auto parity, int it) __attribute__((always_inline)) {
+    constexpr int p = decltype(parity)::value;
+    T* la = smem + p * (OpA::ELEMS + OpB::ELEMS);
+    T* lb = la + OpA::ELEMS;
+    ra.store(p, la);
+    rb.store(p, lb);
+    if (it + 2 < steps) {
+      ra.load(p, pa, (int)a.lda, k0 + (it + 2) * BK, k_end);
+      rb.load(p, pb, (int)a.ldb, k0 + (it + 2) * BK, k_end);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < BK / 16; ++s) {
+      frag<T> fa[WM], fb[WN];
+#pragma unroll
+      for (int i = 0; i < WM; ++i) fa[i] = OpA::read(la, wm + 32 * i, 16 * s, c, g);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) fb[j] = OpB::read(lb, wn + 32 * j, 16 * s, c, g);
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) mma(acc[i][j], fa[i], fb[j]);
+    }
+  };
+  for (int it = 0; it < steps; it += 2) {
+    step(std::integral_constant<int, 0>(), it);
+    if (it + 1 < steps) step(std::integral_constant<int, 1>(), it + 1);
+  }
+  if (a.part != nullptr) {   // partial product of this range of the contraction
+    float* part = a.part + (int64_t)blockIdx.y * a.M * a.N;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = m0 + wm + 32 * i + acc_row(r, g), n = n0 + wn + 32 * j + c;
+          if (m < a.M && n < a.N) part[(int64_t)m * a.N + n] = acc[i][j][r];
+        }
+    return;
+  }
+  // through LDS to whole rows
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < WM; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) smem[(wm + 32 * i + acc_row(r, g)) * LDC + wn + 32 * j + c] = (T)acc[i][j][r];
+  __syncthreads();
+  typedef vec<T, V> vt;
+  typedef vec<float, V> vf;
+  for (int i = threadIdx.x; i < BM * (BN / V); i += kThreads) {
+    const int row = i / (BN / V), col = i % (BN / V) * V, m = m0 + row, n = n0 + col;
+    if (m >= a.M || n >= a.N) continue;
+    vt x = *reinterpret_cast<const vt*>(smem + row * LDC + col);
+    const int64_t at = (int64_t)m * a.ldc + n;
+    if (a.epilogue == kGemmGeluSlope) {
+      vf f = __builtin_convertvector(x, vf);
+      const vf u = __builtin_convertvector(*reinterpret_cast<const vt*>(static_cast<const T*>(a.aux) + at), vf);
+#pragma unroll
+      for (int e = 0; e < V; ++e) f[e] *= gelu_slope(u[e]);
+      x = __builtin_convertvector(f, vt);
+    }
+    *reinterpret_cast<vt*>(static_cast<T*>(a.c) + at) = x;
+    if (a.epilogue == kGemmGelu) {
+      vf f = __builtin_convertvector(x, vf);
+#pragma unroll
+      for (int e = 0; e < V; ++e) f[e] = gelu(f[e]);
+      *reinterpret_cast<vt*>(static_cast<T*>(a.aux) + at) = __builtin_convertvector(f, vt);
+    }
+  }
+}
+
+// Tile and number of ranges of the contraction, from what a launch takes (us, measured over 96 ... 5916 rows, outputs of
+// 128 ... 3072 columns and contractions of 128 ... 5916): 2.3, and per step of a workgroup 0.42 (64 x 64) or 0.95
+// (128 x 128) when it has a CU to itself, 0.32 or 0.9 when the CU has others; fp32 0.75 and 0.62.  A split adds a
+// second launch, 2.5, and its partial results, written and read.  3000 rows, 1536 x 256 out: 24.2 us in one range, 14.4 in the
+// four that this picks; the same product forward: 8.4 on 64 x 64 tiles, 9.5 on 128 x 128; 5916 rows of 512 -> 2048: 30.6
+// and 23.2.
+struct Plan {
+  int tile, splits;
+};
+Plan plan(int M, int N, int K, bool can_split, int elem_size) {
+  Plan best = {64, 1};
+  double best_cost = 1e30;
+  for (int tile = 64; tile <= (elem_size == 2 ? 128 : 64); tile += 64) {
+    const double alone = elem_size == 4 ? 0.75 : tile == 64 ? 0.42 : 0.95, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.32 : 0.9;
+    const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
+    const int steps = (K * elem_size + 127) / 128;   // 128 bytes of the contraction a step
+    for (int s = 1; s <= (can_split ? std::min(16, (steps + 1) / 2) : 1); ++s) {
+      const int64_t per_cu = (tiles * s + 255) / 256, n = (steps + s - 1) / s;
+      double cost = per_cu == 1 ? n * alone : per_cu * n * shared;
+      if (s > 1) cost += 2.5 + (double)s * M * N * 8 / 4e6;
+      if (cost < best_cost) { best_cost = cost; best = {tile, s}; }
+    }
+  }
+  return best;
+}
+constexpr int kStep16 = 64, kStep32 = 32;   // contraction steps in LDS, 16-bit and fp32
+
+template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
+  constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
+  const int tiles = ((a.M + p.tile - 1) / p.tile) * ((a.N + p.tile - 1) / p.tile);
+  const dim3 grid(tiles, p.splits);
+  if constexpr (sizeof(T) == 2) {
+    if (p.tile == 128) {
+      hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK>), grid, dim3(kThreads), 0, stream, a);
+      return hipGetLastError() == hipSuccess ? 0 : -3;
+    }
+  }
+  hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK>), grid, dim3(kThreads), 0, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+}  // namespace
+
+int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue) {
+  const Plan p = plan(M, N, K, !epilogue, elem_size);
+  return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
+}
+
+int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream) {
+  const int es = dtype == 0 ? 4 : 2, step = dtype == 0 ? kStep32 : kStep16;
+  Plan p = plan(a.M, a.N, a.K, a.epilogue == kGemmPlain, es);
+  a.k_per_split = ((a.K + p.splits - 1) / p.splits + step - 1) / step * step;
+  p.splits = (a.K + a.k_per_split - 1) / a.k_per_split;   // rounding up may leave the last ones empty
+  a.part = p.splits > 1 ? workspace : nullptr;
+  const int rc = by_type(dtype, true, [&](auto t, auto) {
+    using T = decltype(t);
+    if (a_kc && b_kc) return launch_t<T, true, true>(a, p, stream);
+    if (a_kc) return launch_t<T, true, false>(a, p, stream);
+    if (!b_kc) return launch_t<T, false, false>(a, p, stream);
+    return -2;
+  });
+  if (rc != 0 || a.part == nullptr) return rc;
+  return launch_part_sum(a.part, p.splits, (int64_t)a.M * a.N, a.c, dtype, stream);
+}
+
+}  // namespace castle

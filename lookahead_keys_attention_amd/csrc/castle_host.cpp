@@ -359,7 +359,45 @@ std::tuple<Tensor, Tensor> rms_norm_autograd(const Tensor& x, const Tensor& weig
   return {r[0], r[1]};
 }
 
+// a (M, K), or (K, M) with a_t; b (N, K), or (K, N) with b_t -> (M, N); rows contiguous up to a leading dimension
+bool product_rows(const Tensor& t) {
+  return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) % (16 / t.element_size()) == 0 && t.size(1) % (16 / t.element_size()) == 0 && aligned16(t);
+}
+Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux) {
+  const c10::DeviceGuard guard(a.device());
+  TORCH_CHECK_VALUE(product_rows(a) && product_rows(b), "product: unexpected operands");
+  const int64_t M = a.size(a_t ? 1 : 0), K = a.size(a_t ? 0 : 1), N = b.size(b_t ? 1 : 0);
+  TORCH_CHECK_VALUE(b.size(b_t ? 0 : 1) == K && b.device() == a.device() && b.scalar_type() == a.scalar_type(), "product: operands do not match");
+  const int dtype = dtype_code(a);
+  const int64_t nbytes = check(castle_gemm_workspace_bytes((int)M, (int)N, (int)K, dtype, (int)epilogue), "castle_gemm_workspace_bytes");
+  Tensor c = at::empty({M, N}, a.options()), ws = nbytes ? bytes(nbytes, a) : Tensor();
+  TORCH_CHECK_VALUE(!aux || (aux->is_contiguous() && aux->sizes() == c.sizes() && aux->scalar_type() == c.scalar_type() && aux->device() == c.device()),
+                    "product: unexpected second tensor");
+  check(castle_gemm(a.data_ptr(), a.stride(0), a_t, b.data_ptr(), b.stride(0), b_t, c.data_ptr(), N, (int)M, (int)N, (int)K, dtype, (int)epilogue,
+                    aux ? aux->data_ptr() : nullptr, nbytes ? ws.data_ptr() : nullptr, nbytes, stream_of(a)),
+        "castle_gemm");
+  return c;
+}
+
 // ---- projections -----------------------------------------------------------------------------------------------
+// Own products where a call is short: the library's costs 18 us of host time, one here 4.  On the GPU they are level or
+// ahead up to the sizes below (us, own / library: 5916 rows 512 -> 2048 forward 23 / 33, 8192 rows 29 / 22; input gradient
+// of 1000 rows x 3072 x 512 15 / 16, 5916 x 2048 x 512 28 / 23; weight gradient of 3000 rows, 1536 x 256, 14 / 27, of
+// 5916, 2048 x 512, 32 / 41; fp32 is behind in all but the smallest, whose time is the host's).
+bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16, double most_32) {
+  return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
+}
+constexpr double kOwnForward = 14e9, kOwnInputGrad = 4e9, kOwnWeightGrad = 40e9, kOwn32 = 4e8;
+
+Tensor project(const Tensor& x, const Tensor& w) {   // (R, K), (N, K) -> (R, N)
+  if (own_product(x, w, x.size(0), w.size(0), x.size(1), kOwnForward, kOwn32)) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
+  return at::mm(x, w.t());
+}
+Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R, K)
+  if (own_product(dy, w, dy.size(0), w.size(0), w.size(1), kOwnInputGrad, kOwn32)) return product(dy, false, w, true, CASTLE_GEMM_PLAIN, std::nullopt);
+  return at::mm(dy, w);
+}
+
 // The weight gradient of a projection over many rows, dW = dY^T x, is a product with a small output
 // (out_features x in_features) and a long contraction (the rows): the GEMM the library picks leaves most of
 // the GPU idle there.  From kSplitWgradMinRows rows on it is formed as kSplitRowsInto partial products over row
@@ -377,7 +415,43 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (
           "castle_sum_parts");
     return dw;
   }
+  if (own_product(dy, x, rows, N, K, kOwnWeightGrad, kOwn32)) return product(dy, true, x, true, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(dy.t(), x);
+}
+
+// A projection as a registered operator, for callers that are traced.
+Tensor linear_op(const Tensor& x, const Tensor& weight) {
+  const c10::DeviceGuard guard(x.device());
+  std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = weight.size(0);
+  return project(x.reshape({-1, x.size(-1)}), weight).view(shape);
+}
+std::tuple<Tensor, Tensor> linear_bwd_op(const Tensor& dy_, const Tensor& x, const Tensor& weight) {
+  const c10::DeviceGuard guard(x.device());
+  const Tensor dy = dy_.reshape({-1, weight.size(0)});
+  return {input_grad(dy, weight).view(x.sizes()), weight_grad(dy, x.reshape({-1, x.size(-1)}))};
+}
+struct LinearFn : torch::autograd::Function<LinearFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight) {
+    static const auto op = op_handle<decltype(linear_op)>("castle_hip::linear");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    ctx->save_for_backward({x, weight});
+    return op.call(x, weight);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    static const auto op = op_handle<decltype(linear_bwd_op)>("castle_hip::linear_bwd");
+    const auto s = ctx->get_saved_variables();
+    auto [dx, dw] = op.call(g[0], s[0], s[1]);
+    return {dx, dw};
+  }
+};
+Tensor linear_autograd(const Tensor& x, const Tensor& weight) {
+  if (!wants_graph({x, weight})) {
+    static const auto op = op_handle<decltype(linear_op)>("castle_hip::linear");
+    const at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(x, weight);
+  }
+  return LinearFn::apply(x, weight);
 }
 
 // ---- a whole layer over sequences ------------------------------------------------------------------------------
@@ -392,10 +466,10 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const Tensor norm_w = norm_w_.value_or(Tensor());
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
     const Normed n = norm_rows(x.reshape({B * L, dim}), delta ? delta->reshape({B * L, dim}) : Tensor(), norm_w, eps, want_graph);
-    const Tensor proj = at::mm(n.h, w_qkv.t()).view({B, L, w_qkv.size(0)});
+    const Tensor proj = project(n.h, w_qkv).view({B, L, w_qkv.size(0)});
     const bool want_U = cache_rows > 0;
     auto [merged, U, ws, state] = attention_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state);
-    variable_list out{at::mm(merged.view({B * L, merged.size(2)}), w_out.t()).view({B, L, w_out.size(0)})};
+    variable_list out{project(merged.view({B * L, merged.size(2)}), w_out).view({B, L, w_out.size(0)})};
     if (delta) out.push_back(n.sum.view({B, L, dim}));
     const size_t results = out.size();
     if (want_U) {   // the rows of the decode cache, behind U in the order of its fields: qu, kc, vc (rotated like the kernels use them)
@@ -445,7 +519,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const bool need_norm = nn && ctx->needs_input_grad(1 + nd), need_qkv = ctx->needs_input_grad(1 + nd + nn);
     if (ctx->needs_input_grad(2 + nd + nn)) grads[4] = weight_grad(dy, merged.view({B * L, merged.size(2)}));
     if (!need_x && !need_norm && !need_qkv) return grads;
-    const Tensor dmerged = at::mm(dy, w_out);
+    const Tensor dmerged = input_grad(dy, w_out);
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
     Tensor dproj = at::empty({B, L, 6 * merged.size(2)}, merged.options());
     castle_view4 d6[6];
@@ -456,7 +530,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
     if (need_qkv) grads[3] = weight_grad(dp2, h);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(at::mm(dp2, w_qkv), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({B * L, dim}) : Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(input_grad(dp2, w_qkv), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({B * L, dim}) : Tensor(), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = dx.view({B, L, dim});
       if (has_delta) grads[1] = grads[0];
@@ -482,8 +556,15 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const at::AutoDispatchBelowADInplaceOrView below;
     const int64_t R = x.numel() / x.size(-1);
     const Normed n = norm_rows(x.reshape({R, x.size(-1)}), delta.reshape({R, x.size(-1)}), norm_w, eps, want_graph);
-    const Tensor up = at::mm(n.h, w_up.t()), act = at::gelu(up);
-    Tensor y = at::mm(act, w_down.t()).view(x.sizes());
+    Tensor up, act;
+    if (own_product(n.h, w_up, R, w_up.size(0), w_up.size(1), kOwnForward, kOwn32)) {   // GELU on the way out
+      act = at::empty({R, w_up.size(0)}, n.h.options());
+      up = product(n.h, false, w_up, false, CASTLE_GEMM_GELU, act);
+    } else {
+      up = at::mm(n.h, w_up.t());
+      act = at::gelu(up);
+    }
+    Tensor y = project(act, w_down).view(x.sizes());
     if (want_graph) {
       ctx->save_for_backward({n.sum, norm_w, w_up, w_down, n.h, n.rstd, up, act});
       ctx->set_materialize_grads(false);
@@ -506,10 +587,12 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const Tensor dy = g[0].reshape({R, dim});
     if (ctx->needs_input_grad(4)) grads[4] = weight_grad(dy, act);
     if (!need_x && !need_norm && !need_up) return grads;
-    const Tensor dup = at::gelu_backward(at::mm(dy, w_down), up);
+    const Tensor dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnInputGrad, kOwn32)
+                           ? product(dy, false, w_down, true, CASTLE_GEMM_GELU_SLOPE, up)
+                           : at::gelu_backward(at::mm(dy, w_down), up);
     if (need_up) grads[3] = weight_grad(dup, h);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(at::mm(dup, w_up), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({R, dim}) : Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(input_grad(dup, w_up), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({R, dim}) : Tensor(), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = grads[1] = dx.view(g[0].sizes());
     }
@@ -531,7 +614,7 @@ struct HeadFn : torch::autograd::Function<HeadFn> {
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
     const Normed n = norm_rows(x.reshape({B * L, dim}), delta.reshape({B * L, dim}), norm_w, eps, want_graph);
     if (want_graph) ctx->save_for_backward({n.sum, norm_w, w, n.h, n.rstd});
-    return at::mm(n.h, w.t()).view({B, L, w.size(0)});
+    return project(n.h, w).view({B, L, w.size(0)});
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     variable_list grads(6);
@@ -543,7 +626,7 @@ struct HeadFn : torch::autograd::Function<HeadFn> {
     const bool need_x = ctx->needs_input_grad(0) || ctx->needs_input_grad(1), need_norm = ctx->needs_input_grad(2);
     if (ctx->needs_input_grad(3)) grads[3] = weight_grad(dy, h);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(at::mm(dy, w), sum, rstd, norm_w, Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(input_grad(dy, w), sum, rstd, norm_w, Tensor(), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = grads[1] = dx.view({g[0].size(0), g[0].size(1), sum.size(1)});
     }
@@ -790,6 +873,8 @@ TORCH_LIBRARY(castle_hip, m) {
         "-> Tensor", tags);
   m.def("rms_norm(Tensor x, Tensor weight, float? eps) -> (Tensor, Tensor)", tags);
   m.def("rms_norm_bwd(Tensor dh, Tensor x, Tensor rstd, Tensor weight) -> (Tensor, Tensor)", tags);
+  m.def("linear(Tensor x, Tensor weight) -> Tensor", tags);
+  m.def("linear_bwd(Tensor dy, Tensor x, Tensor weight) -> (Tensor, Tensor)", tags);
 }
 TORCH_LIBRARY_IMPL(castle_hip, CUDA, m) {
   m.impl("attention", &attention);
@@ -798,6 +883,8 @@ TORCH_LIBRARY_IMPL(castle_hip, CUDA, m) {
   m.impl("attention_packed_bwd", &attention_packed_bwd);
   m.impl("rms_norm", &rms_norm_op);
   m.impl("rms_norm_bwd", &rms_norm_bwd_op);
+  m.impl("linear", &linear_op);
+  m.impl("linear_bwd", &linear_bwd_op);
 }
 // CPU tensors: an error that says what is wrong
 TORCH_LIBRARY_IMPL(castle_hip, CPU, m) {
@@ -808,6 +895,7 @@ TORCH_LIBRARY_IMPL(castle_hip, Autograd, m) {
   m.impl("attention", &attention_autograd);
   m.impl("attention_packed", &attention_packed_autograd);
   m.impl("rms_norm", &rms_norm_autograd);
+  m.impl("linear", &linear_autograd);
 }
 
 PYBIND11_MODULE(_castle_host, m) {
@@ -815,6 +903,7 @@ PYBIND11_MODULE(_castle_host, m) {
   m.attr("ABI_VERSION") = castle_abi_version();
   using unlocked = py::call_guard<py::gil_scoped_release>;
   m.def("layer_parallel", &layer_parallel, unlocked());
+  m.def("product", &product, unlocked());
   m.def("feed_forward", &feed_forward, unlocked());
   m.def("head", &head, unlocked());
   m.def("cross_entropy", &cross_entropy, unlocked());

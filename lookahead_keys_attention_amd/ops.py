@@ -83,7 +83,8 @@ def _as_readable(t: torch.Tensor) -> torch.Tensor:
 #   castle_hip::attention_packed  (B,L,6*H*d) projection -> (merged out, U, workspace, state); U the first L
 #                                 rows of a (B,H,row_capacity,d) buffer (a cache buffer)
 #   castle_hip::rms_norm          rows, weight -> (normalised rows, their factors): the norm of a layer that is traced
-#   castle_hip::attention_bwd / attention_packed_bwd / rms_norm_bwd   their backward passes
+#   castle_hip::linear            rows, weight -> rows weight^T: its projections
+#   castle_hip::attention_bwd / attention_packed_bwd / rms_norm_bwd / linear_bwd   their backward passes
 # `U` is an empty tensor when the lookahead keys are not asked for.  The workspace output is what
 # the backward pass needs back (operand copies, log-sum-exp), the state output the snapshots (empty
 # when they are not kept); they carry no gradient.
@@ -154,11 +155,20 @@ def _fake_rms_norm_bwd(dh, x, rstd, weight):
     return torch.empty(x.shape, dtype=x.dtype, device=x.device), torch.empty_like(weight)
 
 
+def _fake_linear(x, weight):
+    return torch.empty((*x.shape[:-1], weight.shape[0]), dtype=x.dtype, device=x.device)
+
+
+def _fake_linear_bwd(dy, x, weight):
+    return torch.empty(x.shape, dtype=x.dtype, device=x.device), torch.empty_like(weight)
+
+
 def _register_fakes():
     """Called once, when _castle_host.so has defined the operators."""
     for name, fake in (("attention", _fake_attention), ("attention_bwd", _fake_attention_bwd),
                        ("attention_packed", _fake_attention_packed), ("attention_packed_bwd", _fake_attention_packed_bwd),
-                       ("rms_norm", _fake_rms_norm), ("rms_norm_bwd", _fake_rms_norm_bwd)):
+                       ("rms_norm", _fake_rms_norm), ("rms_norm_bwd", _fake_rms_norm_bwd),
+                       ("linear", _fake_linear), ("linear_bwd", _fake_linear_bwd)):
         torch.library.register_fake("castle_hip::" + name, fake)
 
 

@@ -103,3 +103,32 @@ def test_language_model_blocks_equal_the_modules():
         assert len(results[0]) == len(results[1])
         for a, b in zip(*results):
             assert (a - b).norm() <= 1e-4 * b.norm()
+
+
+# tiles of 64 and 128 with remainders in every direction, contractions of less than a step, ranges of the contraction
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 8), (63, 72, 40), (65, 128, 200), (96, 768, 128), (257, 1536, 264), (1003, 256, 2048), (3000, 520, 512),
+                                      (4500, 2048, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_products(rows, n, k, dtype):
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w, dy = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((rows, k), (n, k), (rows, n)))
+    tol = {torch.float32: 1e-5, torch.bfloat16: 4e-3, torch.float16: 6e-4}[dtype]
+
+    def check(got, ref, what):
+        assert torch.isfinite(got).all() and (got.double() - ref).norm() <= tol * ref.norm(), (what, (got.double() - ref).norm() / ref.norm())
+
+    wide = torch.full((rows, k + 16), 3.0, device=DEV, dtype=dtype)
+    wide[:, :k] = x   # rows of a wider tensor
+    ref = x.double() @ w.double().t()
+    check(host().product(wide[:, :k], False, w, False, 0, None), ref, "forward")
+    check(host().product(dy, False, w, True, 0, None), dy.double() @ w.double(), "input gradient")
+    if n % 8 == 0:
+        check(host().product(dy, True, x, True, 0, None), dy.double().t() @ x.double(), "weight gradient")
+    act = torch.empty(rows, n, device=DEV, dtype=dtype)
+    up = host().product(x, False, w, False, 1, act)
+    assert torch.equal(up, host().product(x, False, w, False, 2, torch.full_like(act, 30.0)))   # the slope is 1 there
+    check(act, F.gelu(up.double()), "gelu")
+    u = torch.randn(rows, k, generator=g, device=DEV).to(dtype)
+    plain = dy.double() @ w.double()
+    slope = torch.autograd.functional.vjp(F.gelu, u.double(), torch.ones_like(plain))[1]
+    check(host().product(dy, False, w, True, 2, u), plain * slope, "slope")
