@@ -478,6 +478,15 @@ __device__ __forceinline__ void work_item(int BH, int& rank, int& bh) {
   bh = blockIdx.x % BH;
 }
 
+// The same for a kernel of which two workgroups fit a CU, `n` ranks in all.  Workgroups are handed out one per CU first, then a
+// second each.  When every one of them is resident at once, nothing is handed out later to level the load: CU k has
+// items k and k + cus, and in the order above the long rows of both bands meet.  So the second band runs the other way.
+__device__ __forceinline__ void work_item_paired(int BH, int n, int cus, int& rank, int& bh) {
+  work_item(BH, rank, bh);
+  const int first = cus / BH;   // ranks of the first band
+  if (n * BH <= 2 * cus && rank >= first) rank = first + n - 1 - rank;
+}
+
 // ---- state snapshots -------------------------------------------------------------------
 // A snapshot holds one state row (HD values) per key.  Keys are grouped by 32 ("snapshot
 // tile", 32*HD elements, tiles in key order); inside a tile the 16-byte pieces (V values of one
