@@ -271,7 +271,8 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
 
   prio_by_band(blockIdx.x, a.s.cus);
   int rank, bh;
-  work_item_paired(a.s.B * a.s.H, a.s.Lp / 128, a.s.cus, rank, bh);
+  if ((int)gridDim.x <= 2 * a.s.cus) work_item_snake(a.s.B * a.s.H, a.s.Lp / 128, a.s.cus, rank, bh);
+  else work_item(a.s.B * a.s.H, rank, bh);
   const int qb = a.s.Lp / 128 - 1 - rank;   // the last query block sees the most keys
   const int b = bh / a.s.H, h = bh % a.s.H;
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;

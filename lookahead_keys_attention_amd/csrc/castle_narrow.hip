@@ -160,6 +160,10 @@ template <int HD, int W> constexpr int reduce_bytes() { return W * narrow_nt<HD>
 constexpr int max2(int a, int b) { return a > b ? a : b; }
 // two waves per SIMD where the fragments of 16-bit operands leave room for it
 template <typename T, int HD> constexpr int narrow_waves() { return sizeof(T) == 2 && HD <= 64 ? 2 : 1; }
+template <typename T, int HD> __device__ __forceinline__ void narrow_item(int BH, int n, int cus, int& rank, int& bh) {
+  if constexpr (narrow_waves<T, HD>() == 2) work_item_snake(BH, n, cus, rank, bh);
+  else work_item(BH, rank, bh);
+}
 
 // ---------------------------------------------------------------------------
 template <typename T, int HD, int W> constexpr int scan_narrow_lds() { return max2((2 * W + 1) * wave_tile_bytes<T, HD>(), reduce_bytes<HD, W>()); }
@@ -178,7 +182,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
     }
   }
   int kt, bh;   // key tile 0 sweeps every source block
-  work_item(BH, kt, bh);
+  narrow_item<T, HD>(BH, ntile, a.s.cus, kt, bh);
   const int b = bh / a.s.H, h = bh % a.s.H;
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
   const float c1 = a.s.scale * kLog2e;
@@ -301,7 +305,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void attn_narrow_k
   constexpr int KS = HD / 16, NT = narrow_nt<HD>(), LD = lds_ld_tr<T>(HD);
   const int L = a.s.L, BH = a.s.B * a.s.H, ntile = (L + 31) / 32;
   int rank, bh;
-  work_item(BH, rank, bh);
+  narrow_item<T, HD>(BH, ntile, a.s.cus, rank, bh);
   const int it = ntile - 1 - rank;   // the last queries see the most keys
   const int b = bh / a.s.H, h = bh % a.s.H;
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
@@ -487,7 +491,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
   constexpr bool STAGES = sizeof(T) == 2 && HD == 64;   // two waves per SIMD just fit: 17 spilled registers instead of 41
   const int L = a.s.L, BH = a.s.B * a.s.H, nblk = (L + kNB - 1) / kNB;
   int kt, bh;   // key tile 0 meets every query
-  work_item(BH, kt, bh);
+  narrow_item<T, HD>(BH, (L + 31) / 32, a.s.cus, kt, bh);
   const int b = bh / a.s.H, h = bh % a.s.H;
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
   const float c0 = a.s.scale, c1 = a.s.scale * kLog2e;
@@ -760,7 +764,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
   constexpr bool STAGES = sizeof(T) == 2;   // d = 64: 31 spilled registers instead of 77
   const int L = a.s.L, BH = a.s.B * a.s.H, ntile = (L + 31) / 32, nblk = (L + kNB - 1) / kNB;
   int rank, bh;
-  work_item(BH, rank, bh);
+  narrow_item<T, HD>(BH, ntile, a.s.cus, rank, bh);
   const int it = ntile - 1 - rank;   // the last rows meet the most keys
   const int b = bh / a.s.H, h = bh % a.s.H;
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
@@ -999,30 +1003,41 @@ template <typename T, typename TI, int HD, int W> static int attn_narrow(const F
   hipLaunchKernelGGL((attn_narrow_kernel<T, TI, HD, W>), dim3((a.s.L + 31) / 32 * a.s.B * a.s.H), dim3(64 * W), lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
-template <typename T, typename TI, int HD, int W> static int bwd_narrow(const BwdArgs& a, hipStream_t stream) {
-  constexpr int key_lds = key_narrow_lds<T, HD, W>(), query_lds = query_narrow_lds<T, HD, W>();
+template <typename T, typename TI, int HD, int W> static int bwd_narrow(const BwdArgs& a, hipStream_t stream) {   // W: waves of the key kernel
+  constexpr int key_lds = key_narrow_lds<T, HD, W>(), query_lds = query_narrow_lds<T, HD, 4>();
   static_assert(key_lds <= kMaxLds && query_lds <= kMaxLds);
   static PerDeviceOnce once;
   bool& configured = once.flag();
-  if (!configured) configured = raise_lds(&key_narrow_kernel<T, TI, HD, W>, key_lds) && raise_lds(&query_narrow_kernel<T, TI, HD, W>, query_lds);
+  if (!configured) configured = raise_lds(&key_narrow_kernel<T, TI, HD, W>, key_lds) && raise_lds(&query_narrow_kernel<T, TI, HD, 4>, query_lds);
   if (!configured) return -3;
-  const dim3 grid((a.s.L + 31) / 32 * a.s.B * a.s.H), block(64 * W);
+  const dim3 grid((a.s.L + 31) / 32 * a.s.B * a.s.H);
   {
     ProfScope ps(kSlotBwdKey, stream);
-    hipLaunchKernelGGL((key_narrow_kernel<T, TI, HD, W>), grid, block, key_lds, stream, a);
+    hipLaunchKernelGGL((key_narrow_kernel<T, TI, HD, W>), grid, dim3(64 * W), key_lds, stream, a);
   }
   {
     ProfScope ps(kSlotBwdQuery, stream);
-    hipLaunchKernelGGL((query_narrow_kernel<T, TI, HD, W>), grid, block, query_lds, stream, a);
+    hipLaunchKernelGGL((query_narrow_kernel<T, TI, HD, 4>), grid, dim3(256), query_lds, stream, a);
   }
   return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+// Eight waves on an item instead of four while that leaves no CU a second workgroup to run (16-bit, d <= 64: two waves fit a
+// SIMD) and the walk is long enough to share: 1 head x 8000 rows, us with 4 / 8: scan 79 / 63, attn 105 / 84, key 294 / 224;
+// 4 x 2500: 31 / 27, 40 / 34, 102 / 81.  Level at 10 tiles, slower at 4.  (The query kernel gains nothing: 169 / 166, 67 / 75.)
+template <typename T, int HD> bool eight_waves(const CoreShape& s) {
+  const int64_t tiles = (s.L + 31) / 32;
+  return sizeof(T) == 2 && HD <= 64 && tiles >= 16 && tiles * s.B * s.H <= kNarrowCus * 5 / 4;
 }
 
 int launch_scan_narrow(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
   return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
     return by_head_dim<T>(a.s.d, [&](auto hd) {
-      return scan_narrow<T, TI, decltype(hd)::value, 4>(a, stream);
+      constexpr int HD = decltype(hd)::value;
+      if constexpr (narrow_waves<T, HD>() == 2)
+        if (eight_waves<T, HD>(a.s)) return scan_narrow<T, TI, HD, 8>(a, stream);
+      return scan_narrow<T, TI, HD, 4>(a, stream);
     });
   });
 }
@@ -1030,7 +1045,10 @@ int launch_attn_narrow(const FwdArgs& a, int dtype, bool bf16_operands, hipStrea
   return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
     return by_head_dim<T>(a.s.d, [&](auto hd) {
-      return attn_narrow<T, TI, decltype(hd)::value, 4>(a, stream);
+      constexpr int HD = decltype(hd)::value;
+      if constexpr (narrow_waves<T, HD>() == 2)
+        if (eight_waves<T, HD>(a.s)) return attn_narrow<T, TI, HD, 8>(a, stream);
+      return attn_narrow<T, TI, HD, 4>(a, stream);
     });
   });
 }
@@ -1038,7 +1056,10 @@ int launch_bwd_narrow(const BwdArgs& a, int dtype, bool bf16_operands, hipStream
   return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
     return by_head_dim<T>(a.s.d, [&](auto hd) {
-      return bwd_narrow<T, TI, decltype(hd)::value, 4>(a, stream);
+      constexpr int HD = decltype(hd)::value;
+      if constexpr (narrow_waves<T, HD>() == 2)
+        if (eight_waves<T, HD>(a.s)) return bwd_narrow<T, TI, HD, 8>(a, stream);
+      return bwd_narrow<T, TI, HD, 4>(a, stream);
     });
   });
 }

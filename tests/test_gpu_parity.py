@@ -103,6 +103,12 @@ def test_operator_at_tile_edges_with_few_and_with_many_heads(B, Hh, L, d, dtype)
         assert_close(leaf.grad, r, dtype, name, 1e-4)
 
 
+@pytest.mark.parametrize("B,Hh,L,d", [(1, 1, 481, 64), (1, 1, 513, 64), (2, 3, 545, 32), (1, 5, 1024, 16), (1, 9, 1025, 64), (1, 1, 2049, 64)])
+def test_operator_with_long_walks_shared_by_eight_waves(B, Hh, L, d):
+    """Few heads of many rows, at both ends of the range of that choice and with segments of unequal length."""
+    test_operator_at_tile_edges_with_few_and_with_many_heads(B, Hh, L, d, torch.bfloat16)
+
+
 @pytest.mark.parametrize("L,d", [(256, 64), (200, 32)])
 def test_bf16_operand_flag_forward_and_backward(L, d, monkeypatch):
     """CASTLE_FLAG_BF16_OPERANDS keeps bf16 MFMA operands (default: fp16 operands for bf16 tensors)."""
