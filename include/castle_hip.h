@@ -237,6 +237,11 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
 int castle_rope(const castle_view4* x, const castle_view4* out, int B, int H, int L, int d, int dtype,
                 int first_position, void* stream);
 
+/* The first L rows of a decode cache after a parallel pass (lookahead_keys_attention.py:26, 205-214): qu, kc and vc copied
+ * into its buffers, qu and kc rotated by their position under CASTLE_FLAG_ROTARY. */
+int castle_cache_rows(const castle_view4* qu, const castle_view4* kc, const castle_view4* vc, const castle_view4* qu_cache,
+                      const castle_view4* kc_cache, const castle_view4* vc_cache, int B, int H, int L, int d, int dtype, int flags, void* stream);
+
 /* y[M, N] = x[M, K] w[N, K]^T, all three row-major in the 16-bit element type `dtype` (leading
  * dimensions ldx, ldw, ldy in elements; fp32 accumulation), for the few rows of a decode step: the
  * fused projection and the output projection around the cached step, which the reference runs as

@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "castle_decode_flush",
     "castle_decode_layer",
     "castle_rope",
+    "castle_cache_rows",
     "castle_small_linear",
     "castle_sample",
     "castle_gather_rows",

@@ -18,6 +18,7 @@ int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t str
 int launch_bwd(const BwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_decode(const DecodeArgs& a, int dtype, hipStream_t stream);
 int launch_decode_flush(const DecodeArgs& a, int dtype, hipStream_t stream);
+int launch_cache_rows(const View4 (&src)[3], const View4 (&dst)[3], int B, int H, int L, int d, int dtype, int rotary, hipStream_t stream);
 int launch_rope(const View4& src, const View4& dst, int B, int H, int L, int d, int dtype, int pos0, hipStream_t stream);
 int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus);
 int decode_static_scratch(float** ptr);
@@ -464,6 +465,18 @@ int castle_rope(const castle_view4* x, const castle_view4* out, int B, int H, in
   if (B <= 0 || H <= 0 || L <= 0 || first_position < 0 || !head_dim_ok(d) || (int64_t)B * H > 65535) return CASTLE_ERR_SHAPE;
   if (!view_ok(x, es, true) || !view_ok(out, es, true)) return CASTLE_ERR_ARG;
   return castle::launch_rope(to_view(x), to_view(out), B, H, L, d, dtype, first_position, static_cast<hipStream_t>(stream));
+}
+
+int castle_cache_rows(const castle_view4* qu, const castle_view4* kc, const castle_view4* vc, const castle_view4* qu_cache,
+                      const castle_view4* kc_cache, const castle_view4* vc_cache, int B, int H, int L, int d, int dtype, int flags, void* stream) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (B <= 0 || H <= 0 || L <= 0 || !head_dim_ok(d) || (int64_t)B * H > 65535) return CASTLE_ERR_SHAPE;
+  const castle_view4* all[] = {qu, kc, vc, qu_cache, kc_cache, vc_cache};
+  for (const castle_view4* v : all)
+    if (!view_ok(v, es, true)) return CASTLE_ERR_ARG;
+  const castle::View4 src[3] = {to_view(qu), to_view(kc), to_view(vc)}, dst[3] = {to_view(qu_cache), to_view(kc_cache), to_view(vc_cache)};
+  return castle::launch_cache_rows(src, dst, B, H, L, d, dtype, (flags & CASTLE_FLAG_ROTARY) != 0, static_cast<hipStream_t>(stream));
 }
 
 int castle_small_linear_fused(const void* x, const void* w, void* y, int M, int N, int K,

@@ -572,6 +572,52 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(View4 src, View4 dst, in
   *reinterpret_cast<vec<T, V>*>(view_row<T>(dst, b, h, row) + cv * V) = __builtin_convertvector(f, vec<T, V>);
 }
 
+// The rows of a decode cache from a projection, one launch for its three copied tensors: qu and kc (rotated by their position
+// if asked for) and vc.
+struct CacheRowsArgs {
+  View4 src[3], dst[3];
+  int H, L, rotary;
+};
+template <typename T, int HD>
+__global__ __launch_bounds__(kThreads) void cache_rows_kernel(CacheRowsArgs a) {
+  constexpr int V = elem_traits<T>::vec16;
+  constexpr int VPR = HD / V;
+  const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H, part = blockIdx.z;
+  const int64_t piece = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const int64_t row = piece / VPR;
+  const int cv = (int)(piece % VPR);
+  if (row >= a.L) return;
+  vec<T, V> x = *reinterpret_cast<const vec<T, V>*>(view_row<T>(a.src[part], b, h, row) + cv * V);
+  if (a.rotary && part != 2) {
+    vec<float, V> f = __builtin_convertvector(x, vec<float, V>);
+#pragma unroll
+    for (int e = 0; e < V / 2; ++e) CASTLE_ROPE_PAIR(f[2 * e], f[2 * e + 1], (float)row, cv * (V / 2) + e, HD, false);
+    x = __builtin_convertvector(f, vec<T, V>);
+  }
+  *reinterpret_cast<vec<T, V>*>(view_row<T>(a.dst[part], b, h, row) + cv * V) = x;
+}
+template <typename T> static int launch_cache_rows_d(const CacheRowsArgs& a, int B, int d, hipStream_t stream) {
+  const int pieces_per_row = d / elem_traits<T>::vec16;
+  const dim3 grid((unsigned)(((int64_t)a.L * pieces_per_row + kThreads - 1) / kThreads), B * a.H, 3);
+  switch (d) {
+    case 16: hipLaunchKernelGGL((cache_rows_kernel<T, 16>), grid, dim3(kThreads), 0, stream, a); break;
+    case 32: hipLaunchKernelGGL((cache_rows_kernel<T, 32>), grid, dim3(kThreads), 0, stream, a); break;
+    case 64: hipLaunchKernelGGL((cache_rows_kernel<T, 64>), grid, dim3(kThreads), 0, stream, a); break;
+    case 128: hipLaunchKernelGGL((cache_rows_kernel<T, 128>), grid, dim3(kThreads), 0, stream, a); break;
+    default: return -2;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+int launch_cache_rows(const View4 (&src)[3], const View4 (&dst)[3], int B, int H, int L, int d, int dtype, int rotary, hipStream_t stream) {
+  const CacheRowsArgs a = {{src[0], src[1], src[2]}, {dst[0], dst[1], dst[2]}, H, L, rotary};
+  switch (dtype) {
+    case 0: return launch_cache_rows_d<float>(a, B, d, stream);
+    case 1: return launch_cache_rows_d<bf16_t>(a, B, d, stream);
+    case 2: return launch_cache_rows_d<fp16_t>(a, B, d, stream);
+    default: return -1;
+  }
+}
+
 template <typename T> static int launch_rope_d(const View4& src, const View4& dst, int B, int H, int L, int d, int pos0, hipStream_t stream) {
   const int pieces_per_row = d / elem_traits<T>::vec16;
   const dim3 grid((unsigned)(((int64_t)L * pieces_per_row + kThreads - 1) / kThreads), B * H);
@@ -622,6 +668,7 @@ struct LinearArgs {
   int act;
   const void* res;
   int64_t ldr;
+  int rows, cols;   // of the output that a workgroup takes: at most 16 MT, 16 NT
   int* clear;   // clear_n words set to zero for the launch behind this one
   int clear_n;
 };
@@ -648,7 +695,8 @@ __global__ __launch_bounds__(64 * W) void small_linear_kernel(LinearArgs a) {
   __shared__ float red[W][16 * MT][16 * NT + 1];
   __shared__ float ssq[W][16 * MT];
   const int lane = lane_id(), wave = wave_id(), c = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int n0 = blockIdx.x * a.cols, m0 = blockIdx.y * a.rows;
+  const int n_end = min(a.N, n0 + a.cols), m_end = min(a.M, m0 + a.rows);
   if (blockIdx.x == 0 && blockIdx.y == 0)
     for (int i = threadIdx.x; i < a.clear_n; i += 64 * W) a.clear[i] = 0;
   const int steps = (a.K + DEPTH - 1) / DEPTH;
@@ -676,7 +724,7 @@ __global__ __launch_bounds__(64 * W) void small_linear_kernel(LinearArgs a) {
       for (int j = 0; j < NT; ++j) {
 #pragma unroll
         for (int e = 0; e < V; ++e) fb[u][j][e] = (T)0.f;
-        if (in && n0 + 16 * j + c < a.N) fb[u][j] = *reinterpret_cast<const vt*>(wr + 16 * j * a.ldw + kk);
+        if (in && n0 + 16 * j + c < n_end) fb[u][j] = *reinterpret_cast<const vt*>(wr + 16 * j * a.ldw + kk);
       }
       if (norm_w != nullptr && in) fg[u] = *reinterpret_cast<const vt*>(norm_w + kk);
 #pragma unroll
@@ -684,7 +732,7 @@ __global__ __launch_bounds__(64 * W) void small_linear_kernel(LinearArgs a) {
         const int row = m0 + 16 * i + c;
 #pragma unroll
         for (int e = 0; e < V; ++e) fa[u][i][e] = (T)0.f;
-        if (in && row < a.M) fa[u][i] = *reinterpret_cast<const vt*>(static_cast<const T*>(a.x) + (int64_t)row * a.ldx + kk);
+        if (in && row < m_end) fa[u][i] = *reinterpret_cast<const vt*>(static_cast<const T*>(a.x) + (int64_t)row * a.ldx + kk);
       }
     }
     if (norm_w != nullptr) {
@@ -733,20 +781,27 @@ __global__ __launch_bounds__(64 * W) void small_linear_kernel(LinearArgs a) {
       s *= __builtin_amdgcn_rsqf(t / (float)a.K + a.eps);
     }
     if (a.act == 1) s = 0.5f * s * (1.f + erff(s * 0.70710678f));
-    if (m0 + row < a.M && n0 + col < a.N) {
+    if (m0 + row < m_end && n0 + col < n_end) {
       if (a.res != nullptr) s += (float)static_cast<const T*>(a.res)[(int64_t)(m0 + row) * a.ldr + n0 + col];
       static_cast<T*>(a.y)[(int64_t)(m0 + row) * a.ldy + n0 + col] = (T)s;
     }
   }
 }
 
-template <typename T> static void launch_linear_t(const LinearArgs& a, hipStream_t stream) {
-  // 16 waves when K is long enough to give each of them two steps; 32 columns per workgroup once 16 would
-  // put more than one workgroup on a CU (each of them reads all of x)
-  const int mt = a.M > 16 ? 2 : 1, gy = (a.M + 16 * mt - 1) / (16 * mt);
+template <typename T> static void launch_linear_t(LinearArgs a, hipStream_t stream) {
+  // 16 waves when K is long enough to give each of them two steps
   const bool wide = a.K >= 16 * 4 * elem_traits<T>::vec16 * 2;
-  const int nt = (int64_t)((a.N + 15) / 16) * gy > 256 ? 2 : 1;
-  const dim3 grid((a.N + 16 * nt - 1) / (16 * nt), gy), block(wide ? 1024 : 512);
+  // Rows x columns of a workgroup: a CU draws about 40 bytes per ns, so what counts is the rows of x plus the columns of w
+  // that the busiest CU reads.  Parts of a 16 x 16 matrix tile stay empty for it: K 2048 -> N 512 with 16 rows takes
+  // 32 CUs of 128 KB as 16 x 16, 128 CUs of 64 KB as 8 x 8.
+  int64_t best = INT64_MAX;
+  for (int r = 8; r <= 32; r *= 2)
+    for (int c = 8; c <= 32; c *= 2) {
+      const int64_t groups = (int64_t)((a.M + r - 1) / r) * ((a.N + c - 1) / c), cost = (groups + 255) / 256 * (std::min(r, a.M) + c) * 1024 + groups / 64;
+      if (cost < best) { best = cost; a.rows = r; a.cols = c; }
+    }
+  const int mt = a.rows > 16 ? 2 : 1, nt = a.cols > 16 ? 2 : 1;
+  const dim3 grid((a.N + a.cols - 1) / a.cols, (a.M + a.rows - 1) / a.rows), block(wide ? 1024 : 512);
 #define CASTLE_LINEAR(MT_, NT_, W_) hipLaunchKernelGGL((small_linear_kernel<T, MT_, NT_, W_>), grid, block, 0, stream, a)
   if (wide) {
     if (mt == 1) { if (nt == 1) CASTLE_LINEAR(1, 1, 16); else CASTLE_LINEAR(1, 2, 16); }
@@ -759,7 +814,7 @@ template <typename T> static void launch_linear_t(const LinearArgs& a, hipStream
 }
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                         int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream, int* clear, int clear_n) {
-  const LinearArgs a = {x, w, y, M, N, K, ldx, ldw, ldy, norm_w, eps, act, res, ldr, clear, clear_n};
+  const LinearArgs a = {x, w, y, M, N, K, ldx, ldw, ldy, norm_w, eps, act, res, ldr, 0, 0, clear, clear_n};
   switch (dtype) {
     case 0: launch_linear_t<float>(a, stream); break;
     case 1: launch_linear_t<bf16_t>(a, stream); break;

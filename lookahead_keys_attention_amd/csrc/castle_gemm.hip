@@ -82,8 +82,12 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
   constexpr int kStage = 2 * (OpA::ELEMS + OpB::ELEMS), kOut = BM * LDC;
   __shared__ __attribute__((aligned(16))) T smem[kStage > kOut ? kStage : kOut];
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
-  const int tiles_n = (a.N + BN - 1) / BN;
-  const int m0 = blockIdx.x / tiles_n * BM, n0 = blockIdx.x % tiles_n * BN;
+  // Workgroups go round the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the tiles, so the rows of
+  // `a` are read by one XCD, not by all (input gradient of 3000 rows x 1536 x 256: 13.5 -> 11.1 us).
+  const int tiles_n = (a.N + BN - 1) / BN, tiles = (a.M + BM - 1) / BM * tiles_n;
+  const int tile = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+  if (tile >= tiles) return;
+  const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
   const int wm = wave / 2 * (BM / 2), wn = wave % 2 * (BN / 2);
   const int k0 = blockIdx.y * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split);
   const int steps = (k_end - k0 + BK - 1) / BK;
@@ -206,7 +210,7 @@ constexpr int kStep16 = 64, kStep32 = 32;   // contraction steps in LDS, 16-bit 
 template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
   constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
   const int tiles = ((a.M + p.tile - 1) / p.tile) * ((a.N + p.tile - 1) / p.tile);
-  const dim3 grid(tiles, p.splits);
+  const dim3 grid((tiles + 7) / 8 * 8, p.splits);
   if constexpr (sizeof(T) == 2) {
     if (p.tile == 128) {
       hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK>), grid, dim3(kThreads), 0, stream, a);

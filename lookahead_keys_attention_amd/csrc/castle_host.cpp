@@ -474,19 +474,16 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const size_t results = out.size();
     if (want_U) {   // the rows of the decode cache, behind U in the order of its fields: qu, kc, vc (rotated like the kernels use them)
       const Shape s = packed_shape(proj, heads);
-      const int64_t d = s.d;
       const int part[3] = {0, 4, 5};
+      castle_view4 src[3], dst[3];
       out.push_back(U);
       for (int i = 0; i < 3; ++i) {
-        Tensor buf = at::empty({B, heads, cache_rows, d}, proj.options());
-        if ((flags & CASTLE_FLAG_ROTARY) && part[i] != 5) {
-          const castle_view4 src = packed_view(proj, s, 6, part[i]), dst = view4(buf);
-          check(castle_rope(&src, &dst, s.B, s.H, s.L, s.d, s.dtype, 0, stream_of(proj)), "castle_rope");
-        } else {
-          buf.narrow(2, 0, L).copy_(proj.view({B, L, 6, heads, d}).select(2, part[i]).permute({0, 2, 1, 3}));
-        }
-        out.push_back(buf);
+        out.push_back(at::empty({B, heads, cache_rows, s.d}, proj.options()));
+        src[i] = packed_view(proj, s, 6, part[i]);
+        dst[i] = view4(out.back());
       }
+      check(castle_cache_rows(&src[0], &src[1], &src[2], &dst[0], &dst[1], &dst[2], s.B, s.H, s.L, s.d, s.dtype, (int)flags & CASTLE_FLAG_ROTARY,
+                              stream_of(proj)), "castle_cache_rows");
     }
     if (want_graph) {
       ctx->save_for_backward({norm_w.defined() ? n.sum : Tensor(), norm_w, w_qkv, w_out, n.h, n.rstd, merged, ws, state});
