@@ -21,9 +21,31 @@
 namespace castle {
 namespace {
 
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678f)); }
-__device__ __forceinline__ float gelu_slope(float x) {
-  return 0.5f * (1.f + erff(x * 0.70710678f)) + x * 0.3989422804f * fast_exp2(-0.5f * kLog2e * x * x);
+// Phi(x) = erfc(-x / sqrt 2) / 2.  For 16-bit outputs from the Chebyshev fit of Numerical Recipes (erfcc, fractional error
+// below 1.2e-7 everywhere); the library's erff takes three times the instructions, which a store of 16384 x 2048 felt
+// with 8 us.
+template <typename T> __device__ __forceinline__ float normal_cdf(float x) {
+  if constexpr (sizeof(T) == 4) {
+    return 0.5f * (1.f + erff(x * 0.70710678f));
+  } else {
+    const float z = fabsf(x) * 0.70710678f, t = fast_rcp(__builtin_fmaf(0.5f, z, 1.f));
+    float p = 0.17087277f;
+    p = __builtin_fmaf(p, t, -0.82215223f);
+    p = __builtin_fmaf(p, t, 1.48851587f);
+    p = __builtin_fmaf(p, t, -1.13520398f);
+    p = __builtin_fmaf(p, t, 0.27886807f);
+    p = __builtin_fmaf(p, t, -0.18628806f);
+    p = __builtin_fmaf(p, t, 0.09678418f);
+    p = __builtin_fmaf(p, t, 0.37409196f);
+    p = __builtin_fmaf(p, t, 1.00002368f);
+    p = __builtin_fmaf(p, t, -1.26551223f);
+    const float e = 0.5f * t * fast_exp2(kLog2e * (p - z * z));
+    return x < 0.f ? e : 1.f - e;
+  }
+}
+template <typename T> __device__ __forceinline__ float gelu(float x) { return x * normal_cdf<T>(x); }
+template <typename T> __device__ __forceinline__ float gelu_slope(float x) {
+  return normal_cdf<T>(x) + x * 0.3989422804f * fast_exp2(-0.5f * kLog2e * x * x);
 }
 
 // A tile of FREE rows / columns and BK steps of the contraction: global -> registers -> LDS -> operand fragments.
@@ -83,29 +105,28 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
   __shared__ __attribute__((aligned(16))) T smem[kStage > kOut ? kStage : kOut];
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
   // Workgroups go round the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the tiles, so the rows of
-  // `a` are read by one XCD, not by all (input gradient of 3000 rows x 1536 x 256: 13.5 -> 11.1 us).
+  // `a` are read by one XCD, not by all (input gradient of 3000 rows x 1536 x 256: 13.5 -> 11.1 us).  A workgroup takes
+  // several tiles where there are more than the CUs hold: the first steps of the next are requested before the
+  // output of the last is written.
   const int tiles_n = (a.N + BN - 1) / BN, tiles = (a.M + BM - 1) / BM * tiles_n;
-  const int tile = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
-  if (tile >= tiles) return;
-  const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
+  const int share = (tiles + 7) / 8, first = blockIdx.x % 8 * share, last = min(tiles, first + share);
   const int wm = wave / 2 * (BM / 2), wn = wave % 2 * (BN / 2);
   const int k0 = blockIdx.y * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split);
   const int steps = (k_end - k0 + BK - 1) / BK;
   const T *pa = static_cast<const T*>(a.a), *pb = static_cast<const T*>(a.b);
   OpA ra;
   OpB rb;
-  ra.start((int)a.lda, m0, a.M, k0);
-  rb.start((int)a.ldb, n0, a.N, k0);
-  acc_t acc[WM][WN];
+  acc_t acc[WM][WN];   // [n rows, m lanes]
+  int tile = first + blockIdx.x / 8;
+  auto request = [&]() __attribute__((always_inline)) {
+    ra.start((int)a.lda, tile / tiles_n * BM, a.M, k0);
+    rb.start((int)a.ldb, tile % tiles_n * BN, a.N, k0);
 #pragma unroll
-  for (int i = 0; i < WM; ++i)
-#pragma unroll
-    for (int j = 0; j < WN; ++j) zero(acc[i][j]);
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {   // (a second step beyond the end loads zeros)
-    ra.load(p, pa, (int)a.lda, k0 + p * BK, k_end);
-    rb.load(p, pb, (int)a.ldb, k0 + p * BK, k_end);
-  }
+    for (int p = 0; p < 2; ++p) {   // (a second step beyond the end loads zeros)
+      ra.load(p, pa, (int)a.lda, k0 + p * BK, k_end);
+      rb.load(p, pb, (int)a.ldb, k0 + p * BK, k_end);
+    }
+  };
   auto step = [&](auto parity, int it) __attribute__((always_inline)) {
     constexpr int p = decltype(parity)::value;
     T* la = smem + p * (OpA::ELEMS + OpB::ELEMS);
@@ -127,56 +148,68 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int j = 0; j < WN; ++j) mma(acc[i][j], fa[i], fb[j]);
+        for (int j = 0; j < WN; ++j) mma(acc[i][j], fb[j], fa[i]);
     }
   };
-  for (int it = 0; it < steps; it += 2) {
-    step(std::integral_constant<int, 0>(), it);
-    if (it + 1 < steps) step(std::integral_constant<int, 1>(), it + 1);
-  }
-  if (a.part != nullptr) {   // partial product of this range of the contraction
-    float* part = a.part + (int64_t)blockIdx.y * a.M * a.N;
+  if (tile < last) request();
+  while (tile < last) {
+    const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j) zero(acc[i][j]);
+    for (int it = 0; it < steps; it += 2) {
+      step(std::integral_constant<int, 0>(), it);
+      if (it + 1 < steps) step(std::integral_constant<int, 1>(), it + 1);
+    }
+    tile += gridDim.x / 8;
+    if (tile < last) request();
+    if (a.part != nullptr) {   // partial product of this range of the contraction
+      float* part = a.part + (int64_t)blockIdx.y * a.M * a.N;
+#pragma unroll
+      for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int m = m0 + wm + 32 * i + c, n = n0 + wn + 32 * j + 8 * q + 4 * g;
+            if (m < a.M && n < a.N) *reinterpret_cast<vec<float, 4>*>(part + (int64_t)m * a.N + n) = pack4<float>(acc[i][j], q);
+          }
+      __syncthreads();   // the operands of the last step are dead
+      continue;
+    }
+    // through LDS to whole rows
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
       for (int j = 0; j < WN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + wm + 32 * i + acc_row(r, g), n = n0 + wn + 32 * j + c;
-          if (m < a.M && n < a.N) part[(int64_t)m * a.N + n] = acc[i][j][r];
-        }
-    return;
-  }
-  // through LDS to whole rows
-  __syncthreads();
+        for (int q = 0; q < 4; ++q) st4<T>(smem + (wm + 32 * i + c) * LDC + wn + 32 * j + 8 * q + 4 * g, pack4<T>(acc[i][j], q));
+    __syncthreads();
+    typedef vec<T, V> vt;
+    typedef vec<float, V> vf;
+    for (int i = threadIdx.x; i < BM * (BN / V); i += kThreads) {
+      const int row = i / (BN / V), col = i % (BN / V) * V, m = m0 + row, n = n0 + col;
+      if (m >= a.M || n >= a.N) continue;
+      vt x = *reinterpret_cast<const vt*>(smem + row * LDC + col);
+      const int64_t at = (int64_t)m * a.ldc + n;
+      if (a.epilogue == kGemmGeluSlope) {
+        vf f = __builtin_convertvector(x, vf);
+        const vf u = __builtin_convertvector(*reinterpret_cast<const vt*>(static_cast<const T*>(a.aux) + at), vf);
 #pragma unroll
-  for (int i = 0; i < WM; ++i)
+        for (int e = 0; e < V; ++e) f[e] *= gelu_slope<T>(u[e]);
+        x = __builtin_convertvector(f, vt);
+      }
+      *reinterpret_cast<vt*>(static_cast<T*>(a.c) + at) = x;
+      if (a.epilogue == kGemmGelu) {
+        vf f = __builtin_convertvector(x, vf);
 #pragma unroll
-    for (int j = 0; j < WN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) smem[(wm + 32 * i + acc_row(r, g)) * LDC + wn + 32 * j + c] = (T)acc[i][j][r];
-  __syncthreads();
-  typedef vec<T, V> vt;
-  typedef vec<float, V> vf;
-  for (int i = threadIdx.x; i < BM * (BN / V); i += kThreads) {
-    const int row = i / (BN / V), col = i % (BN / V) * V, m = m0 + row, n = n0 + col;
-    if (m >= a.M || n >= a.N) continue;
-    vt x = *reinterpret_cast<const vt*>(smem + row * LDC + col);
-    const int64_t at = (int64_t)m * a.ldc + n;
-    if (a.epilogue == kGemmGeluSlope) {
-      vf f = __builtin_convertvector(x, vf);
-      const vf u = __builtin_convertvector(*reinterpret_cast<const vt*>(static_cast<const T*>(a.aux) + at), vf);
-#pragma unroll
-      for (int e = 0; e < V; ++e) f[e] *= gelu_slope(u[e]);
-      x = __builtin_convertvector(f, vt);
+        for (int e = 0; e < V; ++e) f[e] = gelu<T>(f[e]);
+        *reinterpret_cast<vt*>(static_cast<T*>(a.aux) + at) = __builtin_convertvector(f, vt);
+      }
     }
-    *reinterpret_cast<vt*>(static_cast<T*>(a.c) + at) = x;
-    if (a.epilogue == kGemmGelu) {
-      vf f = __builtin_convertvector(x, vf);
-#pragma unroll
-      for (int e = 0; e < V; ++e) f[e] = gelu(f[e]);
-      *reinterpret_cast<vt*>(static_cast<T*>(a.aux) + at) = __builtin_convertvector(f, vt);
-    }
+    __syncthreads();
   }
 }
 
@@ -210,7 +243,8 @@ constexpr int kStep16 = 64, kStep32 = 32;   // contraction steps in LDS, 16-bit 
 template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
   constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
   const int tiles = ((a.M + p.tile - 1) / p.tile) * ((a.N + p.tile - 1) / p.tile);
-  const dim3 grid((tiles + 7) / 8 * 8, p.splits);
+  // at most what the CUs hold at once: two workgroups of 128 x 128 tiles or four of 64 x 64
+  const dim3 grid(std::min((tiles + 7) / 8 * 8, p.tile == 128 ? 512 : 1024), p.splits);
   if constexpr (sizeof(T) == 2) {
     if (p.tile == 128) {
       hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK>), grid, dim3(kThreads), 0, stream, a);

@@ -388,6 +388,7 @@ bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int6
   return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
 }
 constexpr double kOwnForward = 14e9, kOwnInputGrad = 4e9, kOwnWeightGrad = 40e9, kOwn32 = 4e8;
+constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 70 / 83
 
 Tensor project(const Tensor& x, const Tensor& w) {   // (R, K), (N, K) -> (R, N)
   if (own_product(x, w, x.size(0), w.size(0), x.size(1), kOwnForward, kOwn32)) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
@@ -584,7 +585,7 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const Tensor dy = g[0].reshape({R, dim});
     if (ctx->needs_input_grad(4)) grads[4] = weight_grad(dy, act);
     if (!need_x && !need_norm && !need_up) return grads;
-    const Tensor dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnInputGrad, kOwn32)
+    const Tensor dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnGeluSlope, kOwn32)
                            ? product(dy, false, w_down, true, CASTLE_GEMM_GELU_SLOPE, up)
                            : at::gelu_backward(at::mm(dy, w_down), up);
     if (need_up) grads[3] = weight_grad(dup, h);
