@@ -60,6 +60,9 @@ extern "C" {
  * hundred steps, in this format to an eighth of that, for the same bytes.  Every entry point that
  * touches one U buffer must get the same setting; a reader converts with  U = 64 * (fp16 bits). */
 #define CASTLE_FLAG_U_HALF 16
+/* Cached step only: the caches that are read until this one's next step exceed the last-level cache, so its rows are not
+ * kept there (set by itself for a host-side row count whose cache alone is that large).  Results are the same. */
+#define CASTLE_FLAG_READ_ONCE 32
 
 /* error codes */
 #define CASTLE_OK 0

@@ -339,6 +339,8 @@ static int decode_step_args(castle::DecodeArgs& a, const castle_view4* U, const 
   a.t_dev = t_device; a.capacity = capacity;
   a.rotary = (flags & CASTLE_FLAG_ROTARY) != 0;
   a.u_half = (flags & CASTLE_FLAG_U_HALF) != 0;
+  // the cache alone, where its size is known: 36 x 8 heads x 2080 rows (307 MB) 71 us a layer step, 78 read once; 42 x 8 (358 MB) 90, 86
+  a.read_once = (flags & CASTLE_FLAG_READ_ONCE) != 0 || (t_device == nullptr && 4LL * B * H * t * d * es > 320000000);
   a.splits = splits;
   a.U = to_view(U); a.qu_cache = to_view(qu_cache); a.kc_cache = to_view(kc_cache); a.vc_cache = to_view(vc_cache);
   a.qc = to_view(qc); a.kc = to_view(kc); a.vc = to_view(vc);

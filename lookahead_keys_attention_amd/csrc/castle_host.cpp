@@ -799,6 +799,9 @@ class StepPlan {
     return out;
   }
 
+  // the steps of this cache are part of a loop over more cached rows than the last-level cache holds
+  void read_once(bool on) { flags_ = on ? flags_ | CASTLE_FLAG_READ_ONCE : flags_ & ~CASTLE_FLAG_READ_ONCE; }
+
   // the whole layer for one token: x (B, 1, dim) -> (B, 1, dim), plus `residual` if there is one
   Tensor layer(const Tensor& x, const std::optional<Tensor>& norm_w, std::optional<double> eps, const Tensor& w_qkv, const Tensor& w_out,
                int64_t max_rows, int64_t t, int64_t base, double scale, bool rotary, const std::optional<Tensor>& residual,
@@ -912,5 +915,6 @@ PYBIND11_MODULE(_castle_host, m) {
   py::class_<StepPlan>(m, "StepPlan")
       .def(py::init<std::vector<Tensor>, Tensor, Tensor, Tensor, bool>())
       .def("attend", &StepPlan::attend, unlocked())
+      .def("read_once", &StepPlan::read_once)
       .def("layer", &StepPlan::layer, unlocked());
 }

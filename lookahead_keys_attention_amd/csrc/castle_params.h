@@ -106,6 +106,7 @@ struct DecodeArgs {
   int splits;       // partitions of the t rows per (b, h)
   float scale;
   int rotary;       // 1: the new token's qc, kc, qu, ku, vu are rotated by position t
+  int read_once;    // 1: the cached rows are not expected in any cache by the next step, nor kept for it
   int u_half;       // 1: the U buffer is in the half-precision cache format (kUHalfScale)
   View4 U, qu_cache, kc_cache, vc_cache;   // capacity buffers, row t is appended
   View4 qc, kc, vc, qu, ku, vu;            // new token, L == 1

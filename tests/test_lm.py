@@ -368,3 +368,19 @@ def test_token_feed_forward_equals_the_block_on_the_cpu():
     assert torch.allclose(got, model.to_logits(model.final_norm(h)), atol=1e-6)
     assert torch.allclose(Castle._project(feed_forward[1], h, False, norm=torch.nn.Identity(), activation="gelu", residual=None),
                           torch.nn.functional.gelu(feed_forward[1](h)), atol=1e-6)
+
+
+@pytest.mark.gpu
+def test_sampling_is_the_same_when_the_cached_rows_are_read_once(monkeypatch):
+    """READ_ONCE_BYTES only decides how the rows are loaded (CASTLE_FLAG_READ_ONCE)."""
+    from lookahead_keys_attention_amd import lm
+
+    torch.manual_seed(3)
+    model = CastleLM(num_tokens=VOCAB, dim=128, depth=2, heads=2, dim_head=64, use_triton=True).cuda().bfloat16()
+    prompt = tokens(3, 70).cuda()
+    results = []
+    for limit in (1 << 60, 0):
+        monkeypatch.setattr(lm, "READ_ONCE_BYTES", limit)
+        model.release_decoder()
+        results.append(model.sample(prompt, 90, generator=torch.Generator(device="cuda").manual_seed(5), graph=True))
+    assert torch.equal(*results)
