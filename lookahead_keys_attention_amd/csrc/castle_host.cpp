@@ -401,18 +401,22 @@ Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R
 
 // The weight gradient of a projection over many rows, dW = dY^T x, is a product with a small output
 // (out_features x in_features) and a long contraction (the rows): the GEMM the library picks leaves most of
-// the GPU idle there.  From kSplitWgradMinRows rows on it is formed as kSplitRowsInto partial products over row
-// ranges (one batched GEMM with fp32 partial results, then their sum): same rounding, 2-3 times faster at 16384 rows.
-constexpr int64_t kSplitWgradMinRows = 8192, kSplitRowsInto = 8;
+// the GPU idle there.  From kSplitWgradMinRows rows on it is formed as partial products over row ranges (one batched GEMM
+// with fp32 partial results, then their sum; same rounding), as many as make about 256 tiles of 256 x 256: 16384 rows,
+// us as one product / with 2, 4, 8 ranges and their sum: 3072 x 512 123 / 80, 64, 63; 2048 x 2048 153 / 137, 139, 161;
+// 6144 x 1024 214 / 187, 200, 231; 12288 x 2048 890 / 931, 884, 1000.
+constexpr int64_t kSplitWgradMinRows = 8192;
 
 Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (N, K)
   const int64_t rows = x.size(0), N = dy.size(1), K = x.size(1);
-  if (x.scalar_type() != at::kFloat && rows >= kSplitWgradMinRows && rows % kSplitRowsInto == 0 && N * K % 8 == 0) {
-    const int64_t r = rows / kSplitRowsInto;
-    const Tensor a = dy.contiguous().view({kSplitRowsInto, r, N}).transpose(1, 2);
-    const Tensor part = at::bmm(a, x.contiguous().view({kSplitRowsInto, r, K}), at::kFloat).contiguous();
+  const int64_t tiles = ((N + 255) / 256) * ((K + 255) / 256), parts = tiles >= 192 ? 1 : tiles >= 96 ? 2 : tiles >= 48 ? 4 : 8;
+  if (x.scalar_type() != at::kFloat && rows >= kSplitWgradMinRows && rows % parts == 0 && N * K % 8 == 0) {
+    if (parts == 1) return at::mm(dy.t(), x);
+    const int64_t r = rows / parts;
+    const Tensor a = dy.contiguous().view({parts, r, N}).transpose(1, 2);
+    const Tensor part = at::bmm(a, x.contiguous().view({parts, r, K}), at::kFloat).contiguous();
     Tensor dw = at::empty({N, K}, x.options());
-    check(castle_sum_parts(static_cast<const float*>(part.data_ptr()), (int)kSplitRowsInto, N * K, dw.data_ptr(), dtype_code(x), stream_of(x)),
+    check(castle_sum_parts(static_cast<const float*>(part.data_ptr()), (int)parts, N * K, dw.data_ptr(), dtype_code(x), stream_of(x)),
           "castle_sum_parts");
     return dw;
   }
