@@ -63,6 +63,12 @@ extern "C" {
 /* Cached step only: the caches that are read until this one's next step exceed the last-level cache, so its rows are not
  * kept there (set by itself for a host-side row count whose cache alone is that large).  Results are the same. */
 #define CASTLE_FLAG_READ_ONCE 32
+/* castle_fwd: the CASTLE_AMAX_PARTIALS floats at byte 256 of the workspace hold partial maxima of |vu| and the word at its start
+ * is 0; castle_bwd: the same place of the backward workspace holds partial maxima of |dout| (castle_gemm leaves them
+ * there): a launch and a pass less.  Ignored for fp32. */
+#define CASTLE_FLAG_AMAX_READY 64
+#define CASTLE_AMAX_PARTIALS 256
+#define CASTLE_AMAX_OFFSET 256
 
 /* error codes */
 #define CASTLE_OK 0
@@ -305,8 +311,16 @@ int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const
 #define CASTLE_GEMM_GELU 1
 #define CASTLE_GEMM_GELU_SLOPE 2
 int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue);
+/* amax != NULL: CASTLE_AMAX_PARTIALS partial maxima of |c| over `columns` columns from `column` on (whole 16-byte pieces), for
+ * CASTLE_FLAG_AMAX_READY; status, if not NULL, is set to 0.  Only where castle_gemm_amax_ok says so. */
+typedef struct castle_amax {
+  float* partials;
+  int* status;
+  int32_t column, columns;
+} castle_amax;
+int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns);
 int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
-                int M, int N, int K, int dtype, int epilogue, void* aux, void* workspace, int64_t workspace_bytes, void* stream);
+                int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* out[i] = sum over p < parts of part[p * n + i], n % 8 == 0: partial products of a weight gradient. */
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream);

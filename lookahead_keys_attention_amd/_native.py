@@ -49,6 +49,7 @@ EXPORTED_SYMBOLS = (
     "castle_gather_rows",
     "castle_small_linear_fused",
     "castle_gemm_workspace_bytes",
+    "castle_gemm_amax_ok",
     "castle_gemm",
     "castle_rms_norm",
     "castle_rms_norm_bwd_workspace_bytes",

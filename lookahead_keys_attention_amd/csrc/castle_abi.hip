@@ -218,6 +218,7 @@ int castle_fwd(const castle_view4* qc, const castle_view4* kc, const castle_view
   a.U = to_view(want_U ? U : nullptr);
   a.u_half = (flags & CASTLE_FLAG_U_HALF) != 0;
   a.ws = carve(workspace, state, g);
+  a.amax_ready = (flags & CASTLE_FLAG_AMAX_READY) != 0;
   return castle::launch_fwd(a, dtype, (flags & CASTLE_FLAG_BF16_OPERANDS) != 0, static_cast<hipStream_t>(stream));
 }
 
@@ -269,6 +270,7 @@ int castle_bwd(const castle_view4* qc, const castle_view4* kc, const castle_view
   a.ws = carve(const_cast<void*>(fwd_workspace), state, g);
   a.bhdr = reinterpret_cast<castle::BwdHeader*>(bw);
   a.amax_part = reinterpret_cast<float*>(bw + 256);
+  a.amax_ready = (flags & CASTLE_FLAG_AMAX_READY) != 0;
   bw += kHeaderBytes;
   a.gsnap = bw;
   a.delta = reinterpret_cast<float*>(bw + g.snap_bytes);
@@ -570,11 +572,17 @@ int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue
   return align_up(castle::gemm_workspace(M, N, K, es, epilogue != CASTLE_GEMM_PLAIN), 256);
 }
 
+int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns) {
+  const int es = elem_size(dtype);
+  if (es == 0 || M <= 0 || N <= 0 || K <= 0 || column < 0 || columns <= 0 || column + columns > N || column % (16 / es) != 0 || columns % (16 / es) != 0) return 0;
+  return castle::gemm_amax_ok(M, N, K, es, column, column + columns);
+}
+
 int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
-                int M, int N, int K, int dtype, int epilogue, void* aux, void* workspace, int64_t workspace_bytes, void* stream) {
+                int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream) {
   const int64_t need = castle_gemm_workspace_bytes(M, N, K, dtype, epilogue);
   if (need < 0) return (int)need;
-  static_assert(CASTLE_GEMM_PLAIN == castle::kGemmPlain && CASTLE_GEMM_GELU == castle::kGemmGelu && CASTLE_GEMM_GELU_SLOPE == castle::kGemmGeluSlope, "");
+  static_assert(CASTLE_AMAX_PARTIALS == castle::kAmaxBlocks && CASTLE_GEMM_PLAIN == castle::kGemmPlain && CASTLE_GEMM_GELU == castle::kGemmGelu && CASTLE_GEMM_GELU_SLOPE == castle::kGemmGeluSlope, "");
   const int v = 16 / elem_size(dtype);
   const int a_row = a_free_contiguous ? M : K, b_row = b_free_contiguous ? N : K;
   if (a_row % v != 0 || b_row % v != 0 || lda < a_row || ldb < b_row || ldc < N || lda % v != 0 || ldb % v != 0 || ldc % v != 0 ||
@@ -585,7 +593,15 @@ int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b
     return CASTLE_ERR_ARG;
   if (need > 0 && (ldc != N || (int64_t)M * N % 8 != 0)) return CASTLE_ERR_SHAPE;
   if (need > 0 && (workspace == nullptr || !aligned16({workspace}) || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
-  const castle::GemmArgs args = {a, b, c, aux, M, N, K, lda, ldb, ldc, epilogue, 0, nullptr};
+  castle::GemmArgs args = {a, b, c, aux, M, N, K, lda, ldb, ldc, epilogue, 0, nullptr, nullptr, nullptr, 0, 1};
+  if (amax != nullptr) {
+    if (!castle_gemm_amax_ok(M, N, K, dtype, amax->column, amax->columns)) return CASTLE_ERR_SHAPE;
+    if (amax->partials == nullptr || reinterpret_cast<uintptr_t>(amax->partials) % 4 != 0 || reinterpret_cast<uintptr_t>(amax->status) % 4 != 0) return CASTLE_ERR_ARG;
+    args.amax = amax->partials;
+    args.amax_status = amax->status;
+    args.amax_from = amax->column;
+    args.amax_to = amax->column + amax->columns;
+  }
   return castle::launch_gemm(args, !a_free_contiguous, !b_free_contiguous, dtype, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
 }
 

@@ -2363,9 +2363,11 @@ template <typename T, typename TI, int HD> static int launch_bwd_t(const BwdArgs
   const dim3 grid(a.s.Lp / 128 * BH), block(kThreads);
   {
     ProfScope ps(kSlotDelta, stream);
-    if constexpr (sizeof(T) == 2)
-      hipLaunchKernelGGL((amax_kernel<TI, HD>), dim3(kAmaxBlocks), dim3(kAmaxThreads), 0, stream, a.dout, a.s.H, a.s.L,
-                         (int64_t)BH * a.s.L, a.amax_part, (int*)nullptr);
+    if constexpr (sizeof(T) == 2) {
+      if (!a.amax_ready)
+        hipLaunchKernelGGL((amax_kernel<TI, HD>), dim3(kAmaxBlocks), dim3(kAmaxThreads), 0, stream, a.dout, a.s.H, a.s.L,
+                           (int64_t)BH * a.s.L, a.amax_part, (int*)nullptr);
+    }
     hipLaunchKernelGGL((delta_kernel<T, TI, HD>), dim3((a.s.Lp + RPB - 1) / RPB, BH), block, 0, stream, a);
   }
   if (narrow) return hipGetLastError() == hipSuccess ? 0 : -3;   // the caller launches the kernels over 32-row work items

@@ -477,9 +477,11 @@ template <typename T, typename TI, int HD> static int launch_prep_t(const FwdArg
   const int BH = a.s.B * a.s.H;
   constexpr int PIECES_PER_ROW = HD / elem_traits<T>::vec16;
   ProfScope ps(kSlotPrep, stream);
-  if constexpr (sizeof(T) == 2)
-    hipLaunchKernelGGL((amax_kernel<TI, HD>), dim3(kAmaxBlocks), dim3(kAmaxThreads), 0, stream, a.vu, a.s.H, a.s.L,
-                       (int64_t)BH * a.s.L, a.ws.amax_part, &a.ws.hdr->status);
+  if constexpr (sizeof(T) == 2) {
+    if (!a.amax_ready)
+      hipLaunchKernelGGL((amax_kernel<TI, HD>), dim3(kAmaxBlocks), dim3(kAmaxThreads), 0, stream, a.vu, a.s.H, a.s.L,
+                         (int64_t)BH * a.s.L, a.ws.amax_part, &a.ws.hdr->status);
+  }
   hipLaunchKernelGGL((prep_kernel<T, TI, HD>), dim3((a.s.Lp * PIECES_PER_ROW + kThreads - 1) / kThreads, BH, 6), dim3(kThreads), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

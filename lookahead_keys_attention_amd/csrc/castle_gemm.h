@@ -15,7 +15,13 @@ struct GemmArgs {
   int epilogue;
   int k_per_split;
   float* part;
+  // largest |c| of the columns amax_from .. amax_to - 1 (a whole number of 16-byte pieces): one partial maximum per tile of them,
+  // zeros in the other slots of the kAmaxBlocks at `amax`
+  float* amax;
+  int* amax_status;   // set to 0 if not nullptr
+  int amax_from, amax_to;
 };
+bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to);
 int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue);
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream);
 

@@ -151,6 +151,11 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
         for (int j = 0; j < WN; ++j) mma(acc[i][j], fb[j], fa[i]);
     }
   };
+  const int amax_tile = a.amax_from / BN, amax_tiles = (a.amax_to - 1) / BN + 1 - amax_tile;   // of a row of tiles
+  if (a.amax != nullptr && blockIdx.x == 0) {
+    for (int i = (a.M + BM - 1) / BM * amax_tiles + threadIdx.x; i < kAmaxBlocks; i += kThreads) a.amax[i] = 0.f;
+    if (threadIdx.x == 0 && a.amax_status != nullptr) *a.amax_status = 0;
+  }
   if (tile < last) request();
   while (tile < last) {
     const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
@@ -189,6 +194,7 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
     __syncthreads();
     typedef vec<T, V> vt;
     typedef vec<float, V> vf;
+    float most = 0.f;
     for (int i = threadIdx.x; i < BM * (BN / V); i += kThreads) {
       const int row = i / (BN / V), col = i % (BN / V) * V, m = m0 + row, n = n0 + col;
       if (m >= a.M || n >= a.N) continue;
@@ -202,11 +208,29 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
         x = __builtin_convertvector(f, vt);
       }
       *reinterpret_cast<vt*>(static_cast<T*>(a.c) + at) = x;
+      if (a.amax != nullptr && n >= a.amax_from && n < a.amax_to) {
+        const vf f = __builtin_convertvector(x, vf);
+#pragma unroll
+        for (int e = 0; e < V; ++e) most = fmaxf(most, fabsf(f[e]));   // fmaxf drops NaNs
+      }
       if (a.epilogue == kGemmGelu) {
         vf f = __builtin_convertvector(x, vf);
 #pragma unroll
         for (int e = 0; e < V; ++e) f[e] = gelu<T>(f[e]);
         *reinterpret_cast<vt*>(static_cast<T*>(a.aux) + at) = __builtin_convertvector(f, vt);
+      }
+    }
+    const int slot = n0 / BN - amax_tile;
+    if (a.amax != nullptr && slot >= 0 && slot < amax_tiles) {
+      __shared__ float s_most[kThreads / 64];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) most = fmaxf(most, __shfl_xor(most, o));
+      if (lane == 0) s_most[wave] = most;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < kThreads / 64; ++w) most = fmaxf(most, s_most[w]);
+        a.amax[m0 / BM * amax_tiles + slot] = fminf(most, 3.0e38f);   // an infinite value counts as the largest finite one
       }
     }
     __syncthreads();
@@ -260,6 +284,13 @@ template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p,
 int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue) {
   const Plan p = plan(M, N, K, !epilogue, elem_size);
   return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
+}
+
+// the maximum is taken on the store: not for a contraction in ranges, nor for more tiles than there are slots
+bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to) {
+  const Plan p = plan(M, N, K, true, elem_size);
+  const int per_row = (amax_to - 1) / p.tile + 1 - amax_from / p.tile;
+  return p.splits == 1 && (int64_t)((M + p.tile - 1) / p.tile) * per_row <= kAmaxBlocks;
 }
 
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream) {

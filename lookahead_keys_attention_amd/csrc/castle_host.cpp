@@ -74,10 +74,12 @@ castle_view4 packed_view(const Tensor& t, const Shape& s, int parts, int i) {
 // six: qc, kc, vc, qu, ku, vu.  Returns what the backward pass needs back: (workspace, state), the state
 // empty when it is not kept.
 std::tuple<Tensor, Tensor> run_fwd(const castle_view4 (&six)[6], const Shape& s, double scale, int64_t flags, const castle_view4& out,
-                                   const castle_view4& U, bool keep_state, const Tensor& like) {
+                                   const castle_view4& U, bool keep_state, const Tensor& like, const Tensor& prepared = Tensor()) {
+  // prepared: a workspace that holds the partial maxima of |vu| already
   const int64_t nbytes = check(castle_fwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_workspace_bytes");
   const int64_t sbytes = check(castle_fwd_state_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_state_bytes");
-  Tensor ws = bytes(nbytes, like), state = bytes(sbytes, like);
+  Tensor ws = prepared.defined() ? prepared : bytes(nbytes, like), state = bytes(sbytes, like);
+  if (prepared.defined()) flags |= CASTLE_FLAG_AMAX_READY;
   check(castle_fwd(&six[0], &six[1], &six[2], &six[3], &six[4], &six[5], s.B, s.H, s.L, s.d, s.dtype, (float)scale, (int)flags, &out,
                    &U, ws.data_ptr(), nbytes, state.data_ptr(), sbytes, stream_of(like)),
         "castle_fwd");
@@ -85,13 +87,21 @@ std::tuple<Tensor, Tensor> run_fwd(const castle_view4 (&six)[6], const Shape& s,
   return {ws, state};
 }
 
+int bwd_flags(int64_t flags, const Tensor& state) {
+  return ((int)flags & ~CASTLE_FLAG_U_HALF) | (state.numel() == 0 ? CASTLE_FLAG_RECOMPUTE_STATE : 0);   // U_HALF describes the forward's U output only
+}
+int64_t bwd_workspace_bytes(const Shape& s, int64_t flags, const Tensor& state) {
+  return check(castle_bwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype, bwd_flags(flags, state)), "castle_bwd_workspace_bytes");
+}
+
 // grads: dqc, dkc, dvc, dqu, dku, dvu.  The backward kernels take the operands from the copies in the forward workspace.
 void run_bwd(const castle_view4 (&six)[6], const castle_view4& out, const castle_view4& dout, const Shape& s, double scale, int64_t flags,
-             const castle_view4 (&grads)[6], const Tensor& ws, const Tensor& state) {
-  int fl = (int)flags & ~CASTLE_FLAG_U_HALF;   // describes the forward's U output only
-  if (state.numel() == 0) fl |= CASTLE_FLAG_RECOMPUTE_STATE;
-  const int64_t nbytes = check(castle_bwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype, fl), "castle_bwd_workspace_bytes");
-  Tensor bws = bytes(nbytes, ws);
+             const castle_view4 (&grads)[6], const Tensor& ws, const Tensor& state, const Tensor& prepared = Tensor()) {
+  // prepared: a backward workspace that holds the partial maxima of |dout| already
+  int fl = bwd_flags(flags, state);
+  const int64_t nbytes = bwd_workspace_bytes(s, flags, state);
+  Tensor bws = prepared.defined() ? prepared : bytes(nbytes, ws);
+  if (prepared.defined()) fl |= CASTLE_FLAG_AMAX_READY;
   check(castle_bwd(&six[0], &six[1], &six[2], &six[3], &six[4], &six[5], &out, &dout, s.B, s.H, s.L, s.d, s.dtype, (float)scale, fl,
                    &grads[0], &grads[1], &grads[2], &grads[3], &grads[4], &grads[5], ws.data_ptr(), ws.numel(),
                    state.numel() ? state.data_ptr() : nullptr, state.numel(), bws.data_ptr(), nbytes, stream_of(ws)),
@@ -147,8 +157,8 @@ void six_of_packed(const Tensor& p, const Shape& s, castle_view4 (&six)[6]) {
   }
 }
 
-std::tuple<Tensor, Tensor, Tensor, Tensor> attention_packed(const Tensor& proj, int64_t heads, double scale, bool want_U,
-                                                            int64_t row_capacity, int64_t flags, bool keep_state) {
+std::tuple<Tensor, Tensor, Tensor, Tensor> run_packed(const Tensor& proj, int64_t heads, double scale, bool want_U,
+                                                            int64_t row_capacity, int64_t flags, bool keep_state, const Tensor& prepared) {
   // The lookahead keys come back as the first L rows of a (B, H, row_capacity, d) buffer, so that a
   // caller can hand over the U buffer of a decode cache without copying (row_capacity >= L).
   require_gpu(proj, "castle_attention_packed");
@@ -162,8 +172,13 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> attention_packed(const Tensor& proj, 
   Tensor merged = at::empty({B, L, H * d}, proj.options());
   Tensor U = want_U ? at::empty({B, H, cap, d}, proj.options()) : at::empty({0}, proj.options());
   auto [ws, state] = run_fwd(six, s, scale, flags, packed_view(merged, s, 1, 0),
-                             want_U ? view4(U) : castle_view4{nullptr, 0, 0, 0}, keep_state, proj);
+                             want_U ? view4(U) : castle_view4{nullptr, 0, 0, 0}, keep_state, proj, prepared);
   return {merged, U, ws, state};
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> attention_packed(const Tensor& proj, int64_t heads, double scale, bool want_U,
+                                                            int64_t row_capacity, int64_t flags, bool keep_state) {
+  return run_packed(proj, heads, scale, want_U, row_capacity, flags, keep_state, Tensor());
 }
 
 Tensor attention_packed_bwd(const Tensor& proj, const Tensor& merged, const Tensor& dmerged, const Tensor& ws, const Tensor& state,
@@ -363,7 +378,7 @@ std::tuple<Tensor, Tensor> rms_norm_autograd(const Tensor& x, const Tensor& weig
 bool product_rows(const Tensor& t) {
   return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) % (16 / t.element_size()) == 0 && t.size(1) % (16 / t.element_size()) == 0 && aligned16(t);
 }
-Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux) {
+Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux, const castle_amax* amax = nullptr) {
   const c10::DeviceGuard guard(a.device());
   TORCH_CHECK_VALUE(product_rows(a) && product_rows(b), "product: unexpected operands");
   const int64_t M = a.size(a_t ? 1 : 0), K = a.size(a_t ? 0 : 1), N = b.size(b_t ? 1 : 0);
@@ -374,7 +389,7 @@ Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epi
   TORCH_CHECK_VALUE(!aux || (aux->is_contiguous() && aux->sizes() == c.sizes() && aux->scalar_type() == c.scalar_type() && aux->device() == c.device()),
                     "product: unexpected second tensor");
   check(castle_gemm(a.data_ptr(), a.stride(0), a_t, b.data_ptr(), b.stride(0), b_t, c.data_ptr(), N, (int)M, (int)N, (int)K, dtype, (int)epilogue,
-                    aux ? aux->data_ptr() : nullptr, nbytes ? ws.data_ptr() : nullptr, nbytes, stream_of(a)),
+                    aux ? aux->data_ptr() : nullptr, amax, nbytes ? ws.data_ptr() : nullptr, nbytes, stream_of(a)),
         "castle_gemm");
   return c;
 }
@@ -390,9 +405,35 @@ bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int6
 constexpr double kOwnForward = 14e9, kOwnInputGrad = 4e9, kOwnWeightGrad = 40e9, kOwn32 = 4e8;
 constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 70 / 83
 
+// The attention kernels behind a product begin with the largest element of some of its columns (vu of a fused projection, all
+// of the gradient of the merged heads): an own product leaves the partial maxima where they look for them, in the
+// workspace that is then handed on (`prepared`; undefined when there are none: fp32, the library's product, a split contraction).
+struct Maxima {
+  Tensor prepared;
+  castle_amax where;
+  const castle_amax* get() const { return prepared.defined() ? &where : nullptr; }
+};
+Maxima maxima(const Tensor& like, int64_t rows, int64_t n, int64_t k, int64_t column, int64_t columns, int64_t nbytes, bool status) {
+  Maxima m;
+  if (like.scalar_type() == at::kFloat || !castle_gemm_amax_ok((int)rows, (int)n, (int)k, dtype_code(like), (int)column, (int)columns)) return m;
+  m.prepared = bytes(nbytes, like);
+  char* p = static_cast<char*>(m.prepared.data_ptr());
+  m.where = {reinterpret_cast<float*>(p + CASTLE_AMAX_OFFSET), status ? reinterpret_cast<int*>(p) : nullptr, (int32_t)column, (int32_t)columns};
+  return m;
+}
+
 Tensor project(const Tensor& x, const Tensor& w) {   // (R, K), (N, K) -> (R, N)
   if (own_product(x, w, x.size(0), w.size(0), x.size(1), kOwnForward, kOwn32)) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(x, w.t());
+}
+// the fused projection, with the maxima of its vu part
+Tensor project_packed(const Tensor& x, const Tensor& w, const Shape& s, Tensor& prepared) {
+  if (!own_product(x, w, x.size(0), w.size(0), x.size(1), kOwnForward, kOwn32)) return at::mm(x, w.t());
+  const int64_t part = (int64_t)s.H * s.d;
+  const Maxima m = maxima(x, x.size(0), w.size(0), x.size(1), 2 * part, part,
+                          check(castle_fwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_workspace_bytes"), true);
+  prepared = m.prepared;
+  return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
 }
 Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R, K)
   if (own_product(dy, w, dy.size(0), w.size(0), w.size(1), kOwnInputGrad, kOwn32)) return product(dy, false, w, true, CASTLE_GEMM_PLAIN, std::nullopt);
@@ -471,9 +512,11 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const Tensor norm_w = norm_w_.value_or(Tensor());
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
     const Normed n = norm_rows(x.reshape({B * L, dim}), delta ? delta->reshape({B * L, dim}) : Tensor(), norm_w, eps, want_graph);
-    const Tensor proj = project(n.h, w_qkv).view({B, L, w_qkv.size(0)});
+    check_dims(w_qkv.size(0) / (6 * heads), n.h);
+    Tensor prepared;
+    const Tensor proj = project_packed(n.h, w_qkv, {(int)B, (int)heads, (int)L, (int)(w_qkv.size(0) / (6 * heads)), dtype_code(n.h)}, prepared).view({B, L, w_qkv.size(0)});
     const bool want_U = cache_rows > 0;
-    auto [merged, U, ws, state] = attention_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state);
+    auto [merged, U, ws, state] = run_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state, prepared);
     variable_list out{project(merged.view({B * L, merged.size(2)}), w_out).view({B, L, w_out.size(0)})};
     if (delta) out.push_back(n.sum.view({B, L, dim}));
     const size_t results = out.size();
@@ -521,14 +564,22 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const bool need_norm = nn && ctx->needs_input_grad(1 + nd), need_qkv = ctx->needs_input_grad(1 + nd + nn);
     if (ctx->needs_input_grad(2 + nd + nn)) grads[4] = weight_grad(dy, merged.view({B * L, merged.size(2)}));
     if (!need_x && !need_norm && !need_qkv) return grads;
-    const Tensor dmerged = input_grad(dy, w_out);
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
+    const int64_t flags = ctx->saved_data["flags"].toInt();
+    Tensor dmerged, prepared;
+    if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), kOwnInputGrad, kOwn32)) {
+      const Maxima m = maxima(dy, B * L, w_out.size(1), w_out.size(0), 0, w_out.size(1), bwd_workspace_bytes(shape, flags, state), false);
+      prepared = m.prepared;
+      dmerged = product(dy, false, w_out, true, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
+    } else {
+      dmerged = at::mm(dy, w_out);
+    }
     Tensor dproj = at::empty({B, L, 6 * merged.size(2)}, merged.options());
     castle_view4 d6[6];
     six_of_packed(dproj, shape, d6);
     // the backward kernels read the operand copies in the workspace: the projection itself is not kept
-    run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(),
-            ctx->saved_data["flags"].toInt(), d6, ws, state);
+    run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(), flags, d6, ws,
+            state, prepared);
     const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
     if (need_qkv) grads[3] = weight_grad(dp2, h);
     if (need_x || need_norm) {
@@ -908,7 +959,9 @@ PYBIND11_MODULE(_castle_host, m) {
   m.attr("ABI_VERSION") = castle_abi_version();
   using unlocked = py::call_guard<py::gil_scoped_release>;
   m.def("layer_parallel", &layer_parallel, unlocked());
-  m.def("product", &product, unlocked());
+  m.def("product", [](const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux) {
+    return product(a, a_t, b, b_t, epilogue, aux);
+  }, unlocked());
   m.def("feed_forward", &feed_forward, unlocked());
   m.def("head", &head, unlocked());
   m.def("cross_entropy", &cross_entropy, unlocked());

@@ -58,6 +58,7 @@ struct FwdArgs {
   View4 U;        // ptr == nullptr when the final lookahead keys are not wanted
   FwdWorkspace ws;
   int with_t = 1; // the scan launch also fills the T' blocks (0 when only the snapshots are recomputed for a backward pass)
+  int amax_ready = 0;   // the partial maxima of |vu| and the status word are in the workspace already
   int u_half = 0; // U is written in the half-precision cache format (see kUHalfScale) instead of the tensor type
 };
 
@@ -68,6 +69,7 @@ struct BwdArgs {
   FwdWorkspace ws;
   BwdHeader* bhdr;
   float* amax_part;   // [kAmaxBlocks] partial maxima of |dO|
+  int amax_ready = 0; // they are there already
   void* gsnap;    // [B*H][snap_rows(nblk)][d]  reverse state at block ends
   float* delta;   // [B*H][Lp]  rowsum(dO * O)
   // Score-gradient tiles handed from the key-stationary to the query-stationary kernel (16-bit

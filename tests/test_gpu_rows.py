@@ -132,3 +132,32 @@ def test_products(rows, n, k, dtype):
     plain = dy.double() @ w.double()
     slope = torch.autograd.functional.vjp(F.gelu, u.double(), torch.ones_like(plain))[1]
     check(host().product(dy, False, w, True, 2, u), plain * slope, "slope")
+
+
+@pytest.mark.parametrize("rows,n,k,column,columns", [(1, 64, 64, 8, 16), (130, 576, 128, 192, 96), (1000, 1536, 256, 512, 256), (2048, 512, 256, 0, 512),
+                                                     (5000, 3072, 512, 1024, 512)])
+def test_product_leaves_partial_maxima(rows, n, k, column, columns):
+    """The largest element of some columns, taken on the store: column ranges inside, across and at the ends of tiles."""
+    import ctypes
+
+    from lookahead_keys_attention_amd import _native as N
+
+    class Amax(ctypes.Structure):
+        _fields_ = [("partials", ctypes.c_void_p), ("status", ctypes.c_void_p), ("column", ctypes.c_int32), ("columns", ctypes.c_int32)]
+
+    lib = N.lib()
+    vp, i, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    lib.castle_gemm.argtypes = [vp, i64, i, vp, i64, i, vp, i64, i, i, i, i, i, vp, ctypes.POINTER(Amax), vp, i64, vp]
+    assert lib.castle_gemm_amax_ok(rows, n, k, 1, column, columns)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w = (torch.randn(*s, generator=g, device=DEV).bfloat16() for s in ((rows, k), (n, k)))
+    c, part = torch.empty(rows, n, device=DEV, dtype=torch.bfloat16), torch.full((257,), -1.0, device=DEV)
+    for r, col in ((0, column), (rows - 1, column + columns - 1), (rows // 2, column + columns // 2)):
+        w[col] += 3 * x[r] / x[r].norm() * k ** 0.5   # the largest element sits there, and one just outside must not count
+        if column > 0:
+            w[column - 1] += 9 * x[r]
+        amax = Amax(part.data_ptr(), part[256:].data_ptr(), column, columns)
+        N.check(lib.castle_gemm(x.data_ptr(), k, 0, w.data_ptr(), k, 0, c.data_ptr(), n, rows, n, k, 1, 0, None, ctypes.byref(amax), None, 0,
+                                N.stream_ptr(x.device)), "castle_gemm")
+        torch.cuda.synchronize()
+        assert part[:256].max() == c[:, column:column + columns].float().abs().max() and part[:256].min() >= 0 and part[256:].view(torch.int32).item() == 0
