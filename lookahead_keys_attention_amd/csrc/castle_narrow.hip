@@ -480,7 +480,8 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void attn_narrow_k
 
 // ---------------------------------------------------------------------------
 // shared rows of the keys (-c1 Qu, Kc, Vc); two operand tiles and a tile of T' rows per wave
-template <typename T, int HD> constexpr int key_narrow_wave_bytes() { return 2 * wave_tile_bytes<T, HD>() + t_tile_bytes<T>(); }
+// and the row sums of a block (-log2 normaliser, -delta)
+template <typename T, int HD> constexpr int key_narrow_wave_bytes() { return 2 * wave_tile_bytes<T, HD>() + t_tile_bytes<T>() + 2 * kNB * 4; }
 template <typename T, int HD, int W> constexpr int key_narrow_lds() {
   return 3 * wave_tile_bytes<T, HD>() + max2(W * key_narrow_wave_bytes<T, HD>(), reduce_bytes<HD, W>());
 }
@@ -504,6 +505,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
   T* s_a = reinterpret_cast<T*>(work + wave * key_narrow_wave_bytes<T, HD>());
   T* s_b = s_a + 32 * LD;
   T* s_t = s_b + 32 * LD;
+  float* s_sum = reinterpret_cast<float*>(s_t + 32 * LDT);
   float* red = reinterpret_cast<float*>(work);
   const T* qc = prep_ptr<T>(a.ws.qc_p, bh, a.s.Lp, HD);
   const T* ku = prep_ptr<T>(a.ws.ku_p, bh, a.s.Lp, HD);
@@ -554,9 +556,23 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
     acc_t dvc[NT], dkc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) { zero(dvc[nt]); zero(dkc[nt]); }
-    if (lo < hi) pa.load(ku + (int64_t)lo * kNB * HD);
+    // one row of the block per lane, a block ahead: loaded where a tile needs them, they were waited for twice a block
+    // (12 heads x 1000 rows: 50.9 -> 48.1 us)
+    float nl = 0.f, nd = 0.f;
+    auto sums = [&](int I) __attribute__((always_inline)) {
+      nl = lse[I * kNB + lane];
+      nd = delta[I * kNB + lane];
+    };
+    if (lo < hi) {
+      pa.load(ku + (int64_t)lo * kNB * HD);
+      sums(lo);
+    }
     __syncthreads();   // the shared rows are there
     for (int I = lo; I < hi; ++I) {
+      const bool there = I * kNB + lane < L;
+      s_sum[lane] = there ? -nl * kLog2e : -INFINITY;
+      s_sum[kNB + lane] = there ? -nd : 0.f;
+      sums(min(I + 1, nblk - 1));
       frag<T> fub[KS], fa[2][2];
       load_snap32<T, HD>(fub, I > Iw ? usnap + (usnap_off(I) + kw0) * HD : ku, c, g);
 #pragma unroll
@@ -582,18 +598,17 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
       }
 #pragma unroll
       for (int itl = 0; itl < 2; ++itl) {
-        const int it = 2 * I + itl, i0 = 32 * it;
+        const int it = 2 * I + itl;
         acc_t sc, su, dp;   // [i rows, k lanes]; sc starts from -lse, dp from -delta of its row
         zero(su);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int r0 = i0 + 8 * q + 4 * g;
-          const vec<float, 4> nl = *reinterpret_cast<const vec<float, 4>*>(lse + r0);
-          const vec<float, 4> nd = *reinterpret_cast<const vec<float, 4>*>(delta + r0);
+          const vec<float, 4> l4 = *reinterpret_cast<const vec<float, 4>*>(s_sum + 32 * itl + 8 * q + 4 * g);
+          const vec<float, 4> d4 = *reinterpret_cast<const vec<float, 4>*>(s_sum + kNB + 32 * itl + 8 * q + 4 * g);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            sc[4 * q + e] = r0 + e < L ? -nl[e] * kLog2e : -INFINITY;
-            dp[4 * q + e] = r0 + e < L ? -nd[e] : 0.f;
+            sc[4 * q + e] = l4[e];
+            dp[4 * q + e] = d4[e];
           }
         }
         wave_lds_order<STAGES>();
@@ -819,17 +834,32 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
   zero(own);
   zero(far);
 
-  for (int kt = wave; kt <= it; kt += W) {
-    const int Kb = kt >> 1;
-    Flat32<T, HD> pq, pk;   // Kc and the state are requested later, where registers get free
+  // What a key tile begins with is requested at the end of the one before, where registers get free (Kc and the state: in the
+  // middle of their own): 8 heads x 2000 rows 58.3 -> 55.0 us, 2 x 3000 71.7 -> 67.5.  Not with one wave per SIMD (d = 128
+  // 72.6 -> 84, fp32 118 -> 122: the registers then move between the two files).
+  constexpr bool EARLY = narrow_waves<T, HD>() == 2;
+  Flat32<T, HD> pq;
+  frag<T> og[KS], fds[2], fdsu[2], fdsn[2];
+  auto request = [&](int kt) __attribute__((always_inline)) {
     pq.load(qu + (int64_t)kt * 32 * HD);
-    frag<T> og[KS], ou[KS], fds[2], fdsu[2], fdsn[2];
     load_snap32<T, HD>(og, has_g ? gsnap + (int64_t)kt * 32 * HD : kc, c, g);
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
       fds[s2] = *reinterpret_cast<const frag_mem<T>*>(ds_mat + kt * tile_row + s2 * 512);
       fdsu[s2] = *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + s2 * 512);
-      fdsn[s2] = next ? *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + 1024 + s2 * 512) : zero_frag<T>();
+      if constexpr (EARLY) fdsn[s2] = *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + (next ? 1024 : 0) + s2 * 512);
+      else fdsn[s2] = next ? *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + 1024 + s2 * 512) : zero_frag<T>();
+    }
+  };
+  if constexpr (EARLY) request(min(wave, it));
+  for (int kt = wave; kt <= it; kt += W) {
+    const int Kb = kt >> 1;
+    if constexpr (!EARLY) request(kt);
+    Flat32<T, HD> pk;
+    frag<T> ou[KS];
+    if (EARLY && !next) {
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) fdsn[s2] = zero_frag<T>();
     }
     wave_lds_order<STAGES>();
     pq.store(s_x);
@@ -914,6 +944,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
       }
     }
     wave_lds_order<STAGES>();
+    if constexpr (EARLY) request(min(kt + W, it));   // unconditional: the last iteration repeats a tile
     if (Kb >= I) {
 #pragma unroll
       for (int s = 0; s < KS; ++s) ou[s] = zero_frag<T>();
@@ -942,10 +973,10 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
 #pragma unroll
   for (int q = 0; q < 4; ++q) st4<T>(s_ds + c * LDX + 8 * q + 4 * g, pack4<T>(own, q));
   // the Qc' rows of the tile; a second tile: the first tile's Vu rows (for dqc), a first tile: the second tile's Qc' rows
-  Flat32<T, HD> pq, pk;
-  pq.load(qc + (int64_t)it * 32 * HD);
+  Flat32<T, HD> pi, pk;
+  pi.load(qc + (int64_t)it * 32 * HD);
   pk.load(half == 1 ? vu + (int64_t)I * kNB * HD : qc + (int64_t)min(it + 1, a.s.Lp / 32 - 1) * 32 * HD);
-  pq.store(s_y);
+  pi.store(s_y);
   pk.store(s_x);
   wave_lds_order<STAGES>();
 #pragma unroll
