@@ -877,13 +877,15 @@ class StepPlan {
     const Tensor res = residual ? (residual->stride(2) == 1 ? *residual : residual->contiguous()) : Tensor();
     // the step's own default: the type's machine epsilon
     const double e = eps ? *eps : x.scalar_type() == at::kHalf ? 0.0009765625 : x.scalar_type() == at::kBFloat16 ? 0.0078125 : 1.1920928955078125e-07;
-    Tensor proj = at::empty({B, 6 * inner}, x.options()), y = at::empty({B, 1, dim}, x.options());
+    // the projection is scratch of the step like the workspace: kept with it, an allocation costs more than a microsecond
+    if (!proj_.defined()) proj_ = at::empty({B, 6 * inner}, x.options().requires_grad(false));
+    Tensor y = at::empty({B, 1, dim}, x.options());
     const castle_view4* c = views_;
     castle_deferred def = deferred(base, base_device);
     check(castle_decode_layer(c, c + 1, c + 2, c + 3, (int)t, t_device ? count_ptr(t_device) : nullptr, s_.L, xr.data_ptr(), xr.stride(0), (int)dim,
                               nw.defined() ? nw.data_ptr() : nullptr, (float)e, w_qkv.data_ptr(), w_qkv.stride(0), w_out.data_ptr(),
                               w_out.stride(0), res.defined() ? res.data_ptr() : nullptr, res.defined() ? res.stride(0) : 0, y.data_ptr(), dim,
-                              proj.data_ptr(), s_.B, s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0),
+                              proj_.data_ptr(), s_.B, s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0),
                               base >= 0 || base_device ? &def : nullptr, workspace_.data_ptr(), workspace_.numel(), stream_of(x)),
           "castle_decode_layer");
     return y;
@@ -907,7 +909,7 @@ class StepPlan {
   }
 
   std::vector<Tensor> buffers_;
-  Tensor ring_, gates_, workspace_;
+  Tensor ring_, gates_, workspace_, proj_;
   castle_view4 views_[4];
   castle_deferred deferred_;
   Shape s_;
