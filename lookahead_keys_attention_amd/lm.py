@@ -14,6 +14,8 @@ default to the reference's choice (both on, train_triton.py:99-100).
 """
 from __future__ import annotations
 
+import contextlib
+import gc
 import math
 
 import torch
@@ -70,6 +72,20 @@ def _is_plain(module, kind) -> bool:
     return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
 
 
+@contextlib.contextmanager
+def _no_collection():
+    """Python's cyclic garbage collector waits.  A model and the decoder kept from its last `sample` call hold each
+    other, so the graph of a dropped model is destroyed by a collection; the destructor synchronises the device, which a
+    capture forbids, and an error in a destructor ends the process."""
+    enabled = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if enabled:
+            gc.enable()
+
+
 class GraphedDecoder:
     """One captured HIP graph of a whole single-token step of a `CastleLM` on the native path.
 
@@ -114,7 +130,7 @@ class GraphedDecoder:
                 self._step()
         torch.cuda.current_stream(device).wait_stream(side)
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph), torch.no_grad():
+        with _no_collection(), torch.cuda.graph(self.graph), torch.no_grad():
             self.logits = self._step()
             self.t_device += 1
         self._set_counters()

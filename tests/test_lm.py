@@ -384,3 +384,38 @@ def test_sampling_is_the_same_when_the_cached_rows_are_read_once(monkeypatch):
         model.release_decoder()
         results.append(model.sample(prompt, 90, generator=torch.Generator(device="cuda").manual_seed(5), graph=True))
     assert torch.equal(*results)
+
+
+def test_no_collection_runs_while_a_graph_is_captured():
+    """A dropped model and its kept decoder are cyclic garbage; its graph must not be destroyed inside another capture."""
+    import gc
+    import weakref
+
+    from lookahead_keys_attention_amd.lm import _no_collection
+
+    class Graph:
+        pass
+
+    gc.collect()
+    model, kept = Graph(), Graph()
+    kept.model, model.kept = model, kept
+    graph = weakref.ref(kept)
+    threshold = gc.get_threshold()
+    gc.set_threshold(1, 1000, 1000)   # every few objects a collection of the young ones
+    try:
+        with _no_collection():
+            del model, kept
+            junk = [[] for _ in range(5000)]
+            assert graph() is not None
+        assert gc.isenabled()
+        junk = [[] for _ in range(5000)]   # noqa: F841  (allocations, so that a collection is due)
+        assert graph() is None
+    finally:
+        gc.set_threshold(*threshold)
+    gc.disable()
+    try:
+        with _no_collection():
+            pass
+        assert not gc.isenabled()   # a program that runs without the collector keeps running without it
+    finally:
+        gc.enable()
