@@ -315,16 +315,16 @@ Normed norm_rows(const Tensor& x_, const Tensor& delta_, const Tensor& w_, std::
         "castle_rms_norm");
   return {sum, h, rstd};
 }
-// dh -> (dres + gradient of the rows, gradient of the weight); x, rstd as norm_rows left them
-std::tuple<Tensor, Tensor> norm_rows_bwd(const Tensor& dh_, const Tensor& x, const Tensor& rstd, const Tensor& w_, const Tensor& dres_, bool need_x,
+// dh -> (dres + gradient of the rows, gradient of the weight); rstd as norm_rows left it
+std::tuple<Tensor, Tensor> norm_rows_bwd(const Tensor& dh_, const Tensor& x_, const Tensor& rstd, const Tensor& w_, const Tensor& dres_, bool need_x,
                                          bool need_w) {
   if (!w_.defined()) return {dres_.defined() ? dres_ + dh_ : dh_, Tensor()};
-  const int64_t R = x.size(0), D = x.size(1);
+  const int64_t R = x_.size(0), D = x_.size(1);
   if (rstd.dim() != 1) {
-    auto [dx, dw] = at::_fused_rms_norm_backward(dh_, x, {D}, rstd, w_, {need_x, need_w});
+    auto [dx, dw] = at::_fused_rms_norm_backward(dh_, x_, {D}, rstd, w_, {need_x, need_w});
     return {need_x && dres_.defined() ? dres_ + dx : dx, dw};
   }
-  const Tensor dh = row_major(dh_), w = row_major(w_), dres = need_x && dres_.defined() ? row_major(dres_) : Tensor();
+  const Tensor x = row_major(x_), dh = row_major(dh_), w = row_major(w_), dres = need_x && dres_.defined() ? row_major(dres_) : Tensor();
   const int64_t nbytes = need_w ? castle_rms_norm_bwd_workspace_bytes(R, (int)D, dtype_code(x)) : 0;
   Tensor dx = need_x ? at::empty_like(x) : Tensor(), dw = need_w ? at::empty_like(w) : Tensor(), ws = need_w ? bytes(nbytes, x) : Tensor();
   check(castle_rms_norm_bwd(dh.data_ptr(), x.data_ptr(), w.data_ptr(), static_cast<const float*>(rstd.data_ptr()), dres.defined() ? dres.data_ptr() : nullptr,
@@ -343,7 +343,7 @@ std::tuple<Tensor, Tensor> rms_norm_op(const Tensor& x, const Tensor& weight, st
 std::tuple<Tensor, Tensor> rms_norm_bwd_op(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight) {
   const c10::DeviceGuard guard(x.device());
   const int64_t D = x.size(-1);
-  auto [dx, dw] = norm_rows_bwd(dh.reshape({-1, D}), row_major(x.reshape({-1, D})), rstd, weight, Tensor(), true, true);
+  auto [dx, dw] = norm_rows_bwd(dh.reshape({-1, D}), x.reshape({-1, D}), rstd, weight, Tensor(), true, true);
   return {dx.view(x.sizes()), dw};
 }
 struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
@@ -534,7 +534,15 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
                               stream_of(proj)), "castle_cache_rows");
     }
     if (want_graph) {
-      ctx->save_for_backward({norm_w.defined() ? n.sum : Tensor(), norm_w, w_qkv, w_out, n.h, n.rstd, merged, ws, state});
+      // The layer's input itself is saved, not the rows that are a view of it: a view made below ADInplaceOrView has a
+      // version of its own, so a change of the input in place would go unnoticed.  And only what the gradients asked for read:
+      // anything else may be changed.
+      const bool below = x.requires_grad() || (delta && delta->requires_grad()) || (norm_w.defined() && norm_w.requires_grad());
+      const bool need_qkv = w_qkv.requires_grad();
+      auto keep = [&](bool needed, const Tensor& t) { return !needed ? Tensor() : t.defined() && t.is_alias_of(x) ? x : t; };
+      ctx->save_for_backward({keep(below && norm_w.defined(), n.sum), keep(below, norm_w), keep(below, w_qkv), keep(below || need_qkv, w_out),
+                              keep(need_qkv, n.h), n.rstd, merged, ws, state});
+      ctx->saved_data["dim"] = dim;
       ctx->saved_data["heads"] = heads;
       ctx->saved_data["scale"] = scale;
       ctx->saved_data["flags"] = flags;
@@ -556,11 +564,12 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     }
     const at::NoGradGuard no_grad;   // no second derivatives, as for the operators
     const auto s = ctx->get_saved_variables();
-    const Tensor &sum = s[0], &norm_w = s[1], &w_qkv = s[2], &w_out = s[3], &h = s[4], &rstd = s[5], &merged = s[6], &ws = s[7], &state = s[8];
-    const c10::DeviceGuard guard(h.device());
-    const int64_t B = merged.size(0), L = merged.size(1), dim = h.size(1), heads = ctx->saved_data["heads"].toInt();
-    const Tensor dy = g[0].reshape({B * L, w_out.size(0)});
-    const size_t nn = norm_w.defined() ? 1 : 0;
+    const Tensor &norm_w = s[1], &w_qkv = s[2], &w_out = s[3], &rstd = s[5], &merged = s[6], &ws = s[7], &state = s[8];
+    const c10::DeviceGuard guard(merged.device());
+    const int64_t B = merged.size(0), L = merged.size(1), dim = ctx->saved_data["dim"].toInt(), heads = ctx->saved_data["heads"].toInt();
+    const Tensor dy = g[0].reshape({B * L, g[0].size(2)});
+    auto rows = [&](const Tensor& t) { return t.defined() ? t.reshape({B * L, dim}) : t; };
+    const size_t nn = rstd.defined() ? 1 : 0;
     const bool need_norm = nn && ctx->needs_input_grad(1 + nd), need_qkv = ctx->needs_input_grad(1 + nd + nn);
     if (ctx->needs_input_grad(2 + nd + nn)) grads[4] = weight_grad(dy, merged.view({B * L, merged.size(2)}));
     if (!need_x && !need_norm && !need_qkv) return grads;
@@ -581,9 +590,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(), flags, d6, ws,
             state, prepared);
     const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
-    if (need_qkv) grads[3] = weight_grad(dp2, h);
+    if (need_qkv) grads[3] = weight_grad(dp2, rows(s[4]));
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(input_grad(dp2, w_qkv), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({B * L, dim}) : Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(input_grad(dp2, w_qkv), rows(s[0]), rstd, norm_w, rows(dsum), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = dx.view({B, L, dim});
       if (has_delta) grads[1] = grads[0];

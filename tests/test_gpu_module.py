@@ -183,6 +183,33 @@ def test_projection_over_many_rows_forms_its_weight_gradient_in_row_ranges():
         assert C._linear(layer, x).grad_fn is None
 
 
+@pytest.mark.parametrize("prenorm", [False, True])
+def test_input_changed_in_place_before_the_backward_pass(prenorm):
+    """A layer's input is read by its backward pass: one that was changed in place is an error, as for the modules
+    one by one, where a gradient needs it, and no error where none does."""
+    m = make(64, 2, 32, prenorm=prenorm)
+    for wide in (False, True):   # rows of the input itself, and of a wider tensor
+        h = torch.randn(2, 40, 80 if wide else 64, device=DEV)[..., :64]
+        y = m(h)
+        h += y.detach()
+        if prenorm and wide:   # (the norm works on a copy of such rows)
+            y.sum().backward()
+            continue
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.sum().backward()
+    m.to_all_qkv.weight.requires_grad_(False)
+    leaf = torch.randn(2, 40, 64, device=DEV, requires_grad=True)
+    want, = torch.autograd.grad(m(leaf).sum(), leaf)
+    h = leaf * 1
+    y = m(h)
+    h += 1
+    if prenorm:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.sum().backward()
+    else:   # no gradient reads the input of a frozen projection
+        assert torch.equal(torch.autograd.grad(y.sum(), leaf)[0], want)
+
+
 def test_multi_token_with_cache_is_rejected():
     m = make(32, 2, 16)
     x = torch.randn(1, 4, 32).to(DEV)
