@@ -10,6 +10,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
 
@@ -208,6 +209,26 @@ bool wants_graph(std::initializer_list<Tensor> ts) {
   return false;
 }
 
+// The gradients have no derivatives of their own.  Where a graph of the backward pass is recorded (create_graph) they hang on a
+// node that raises when somebody differentiates them: as constants, a penalty on them would add nothing, without a word.
+variable_list no_second_derivatives(const variable_list& grads) {
+  variable_list alias;
+  alias.reserve(grads.size());
+  for (const Tensor& t : grads) alias.push_back(t.defined() ? t.detach().set_requires_grad(true) : t);
+  const auto raises = std::make_shared<torch::autograd::DelayedError>(
+      "trying to differentiate twice through the CASTLE kernels: their gradients have no derivatives (Castle(use_triton=False) is "
+      "differentiable any number of times)", (int64_t)grads.size());
+  return (*raises)(std::move(alias));
+}
+template <typename F> variable_list once_differentiable(F&& gradients) {
+  variable_list grads;
+  {
+    const at::NoGradGuard no_grad;
+    grads = gradients();
+  }
+  return at::GradMode::is_enabled() ? no_second_derivatives(grads) : grads;
+}
+
 template <typename F> auto op_handle(const char* name) {
   return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
 }
@@ -234,6 +255,15 @@ struct AttentionFn : torch::autograd::Function<AttentionFn> {
     return {d[0], d[1], d[2], d[3], d[4], d[5], Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
+
+Tensor attention_bwd_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu, const Tensor& ku, const Tensor& vu,
+                              const Tensor& out, const Tensor& dout, const Tensor& ws, const Tensor& state, double scale, int64_t flags) {
+  static const auto op = op_handle<decltype(attention_bwd)>("castle_hip::attention_bwd");
+  const bool graph = at::GradMode::is_enabled() && wants_graph({q, k, v, qu, ku, vu, out, dout});
+  const at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor d = op.call(q, k, v, qu, ku, vu, out, dout, ws, state, scale, flags);
+  return graph ? no_second_derivatives({d})[0] : d;
+}
 
 std::tuple<Tensor, Tensor, Tensor, Tensor> attention_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu,
                                                               const Tensor& ku, const Tensor& vu, double scale, bool want_U,
@@ -270,6 +300,15 @@ struct AttentionPackedFn : torch::autograd::Function<AttentionPackedFn> {
     return {dproj, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
+
+Tensor attention_packed_bwd_autograd(const Tensor& proj, const Tensor& merged, const Tensor& dmerged, const Tensor& ws, const Tensor& state,
+                                     int64_t heads, double scale, int64_t flags) {
+  static const auto op = op_handle<decltype(attention_packed_bwd)>("castle_hip::attention_packed_bwd");
+  const bool graph = at::GradMode::is_enabled() && wants_graph({proj, merged, dmerged});
+  const at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor d = op.call(proj, merged, dmerged, ws, state, heads, scale, flags);
+  return graph ? no_second_derivatives({d})[0] : d;
+}
 
 std::tuple<Tensor, Tensor, Tensor, Tensor> attention_packed_autograd(const Tensor& proj, int64_t heads, double scale, bool want_U,
                                                                      int64_t row_capacity, int64_t flags, bool keep_state) {
@@ -364,6 +403,15 @@ struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
     return {dx, dw, Tensor()};
   }
 };
+std::tuple<Tensor, Tensor> rms_norm_bwd_autograd(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight) {
+  static const auto op = op_handle<decltype(rms_norm_bwd_op)>("castle_hip::rms_norm_bwd");
+  const bool graph = at::GradMode::is_enabled() && wants_graph({dh, x, weight});
+  const at::AutoDispatchBelowADInplaceOrView below;
+  const auto [dx, dw] = op.call(dh, x, rstd, weight);
+  if (!graph) return {dx, dw};
+  const auto r = no_second_derivatives({dx, dw});
+  return {r[0], r[1]};
+}
 std::tuple<Tensor, Tensor> rms_norm_autograd(const Tensor& x, const Tensor& weight, std::optional<double> eps) {
   if (!wants_graph({x, weight})) {
     static const auto op = op_handle<decltype(rms_norm_op)>("castle_hip::rms_norm");
@@ -491,6 +539,15 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
     return {dx, dw};
   }
 };
+std::tuple<Tensor, Tensor> linear_bwd_autograd(const Tensor& dy, const Tensor& x, const Tensor& weight) {
+  static const auto op = op_handle<decltype(linear_bwd_op)>("castle_hip::linear_bwd");
+  const bool graph = at::GradMode::is_enabled() && wants_graph({dy, x, weight});
+  const at::AutoDispatchBelowADInplaceOrView below;
+  const auto [dx, dw] = op.call(dy, x, weight);
+  if (!graph) return {dx, dw};
+  const auto r = no_second_derivatives({dx, dw});
+  return {r[0], r[1]};
+}
 Tensor linear_autograd(const Tensor& x, const Tensor& weight) {
   if (!wants_graph({x, weight})) {
     static const auto op = op_handle<decltype(linear_op)>("castle_hip::linear");
@@ -553,16 +610,17 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    if (g[0].defined()) return once_differentiable([&] { return gradients(ctx, g); });
+    variable_list grads(12);
+    if (ctx->saved_data["delta"].toBool() && g[1].defined()) grads[0] = grads[1] = g[1];
+    return grads;
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& g) {
     variable_list grads(12);
     const bool has_delta = ctx->saved_data["delta"].toBool();
     const Tensor dsum = has_delta ? g[1] : Tensor();
     const size_t nd = has_delta ? 1 : 0;   // needs_input_grad counts the tensors that were there
     const bool need_x = ctx->needs_input_grad(0) || (has_delta && ctx->needs_input_grad(1));
-    if (!g[0].defined()) {
-      if (dsum.defined()) grads[0] = grads[1] = dsum;
-      return grads;
-    }
-    const at::NoGradGuard no_grad;   // no second derivatives, as for the operators
     const auto s = ctx->get_saved_variables();
     const Tensor &norm_w = s[1], &w_qkv = s[2], &w_out = s[3], &rstd = s[5], &merged = s[6], &ws = s[7], &state = s[8];
     const c10::DeviceGuard guard(merged.device());
@@ -634,14 +692,15 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     return {y, n.sum.view(x.sizes())};
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    if (g[0].defined()) return once_differentiable([&] { return gradients(ctx, g); });
+    variable_list grads(7);
+    if (g[1].defined()) grads[0] = grads[1] = g[1];
+    return grads;
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& g) {
     variable_list grads(7);
     const Tensor dsum = g[1];
     const bool need_x = ctx->needs_input_grad(0) || ctx->needs_input_grad(1), need_norm = ctx->needs_input_grad(2), need_up = ctx->needs_input_grad(3);
-    if (!g[0].defined()) {
-      if (dsum.defined()) grads[0] = grads[1] = dsum;
-      return grads;
-    }
-    const at::NoGradGuard no_grad;
     const auto s = ctx->get_saved_variables();
     const Tensor &sum = s[0], &norm_w = s[1], &w_up = s[2], &w_down = s[3], &h = s[4], &rstd = s[5], &up = s[6], &act = s[7];
     const c10::DeviceGuard guard(h.device());
@@ -679,8 +738,10 @@ struct HeadFn : torch::autograd::Function<HeadFn> {
     return project(n.h, w).view({B, L, w.size(0)});
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return once_differentiable([&] { return gradients(ctx, g); });
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& g) {
     variable_list grads(6);
-    const at::NoGradGuard no_grad;
     const auto s = ctx->get_saved_variables();
     const Tensor &sum = s[0], &norm_w = s[1], &w = s[2], &h = s[3], &rstd = s[4];
     const c10::DeviceGuard guard(h.device());
@@ -722,7 +783,9 @@ struct CrossEntropyFn : torch::autograd::Function<CrossEntropyFn> {
     return loss;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
-    const at::NoGradGuard no_grad;
+    return once_differentiable([&] { return gradients(ctx, g); });
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& g) {
     const auto s = ctx->get_saved_variables();
     const Tensor &logits = s[0], &target = s[1], &lse = s[2], &inv = s[3];
     const c10::DeviceGuard guard(logits.device());
@@ -754,7 +817,9 @@ struct EmbeddingFn : torch::autograd::Function<EmbeddingFn> {
     return at::embedding(weight, index);
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
-    const at::NoGradGuard no_grad;
+    return once_differentiable([&] { return gradients(ctx, g); });
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& g) {
     const Tensor index = token_rows(ctx->get_saved_variables()[0]);
     const c10::DeviceGuard guard(index.device());
     const int64_t V = ctx->saved_data["vocabulary"].toInt(), D = g[0].size(-1), R = index.numel();
@@ -961,8 +1026,12 @@ TORCH_LIBRARY_IMPL(castle_hip, CPU, m) {
 TORCH_LIBRARY_IMPL(castle_hip, Autograd, m) {
   m.impl("attention", &attention_autograd);
   m.impl("attention_packed", &attention_packed_autograd);
+  m.impl("attention_bwd", &attention_bwd_autograd);
+  m.impl("attention_packed_bwd", &attention_packed_bwd_autograd);
   m.impl("rms_norm", &rms_norm_autograd);
+  m.impl("rms_norm_bwd", &rms_norm_bwd_autograd);
   m.impl("linear", &linear_autograd);
+  m.impl("linear_bwd", &linear_bwd_autograd);
 }
 
 PYBIND11_MODULE(_castle_host, m) {

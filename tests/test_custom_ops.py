@@ -43,6 +43,32 @@ def test_fake_tensor_forward_and_backward_of_the_six_operand_operator():
             assert (state.numel() > 0) == keep
 
 
+def _twice(y, leaf):
+    """Differentiates a gradient of y: the penalty's share must not silently be zero."""
+    grad, = torch.autograd.grad(y.square().sum(), leaf, create_graph=True)
+    with pytest.raises(RuntimeError, match="differentiate twice"):
+        (y.sum() + grad.square().sum()).backward()
+
+
+def test_second_derivatives_of_the_operators_raise():
+    with FakeTensorMode():
+        six = [torch.empty(2, 2, 40, 32, requires_grad=True) for _ in range(6)]
+        for leaf in (six[0], six[5]):
+            _twice(ops.castle_attention_hip(*six, 0.125), leaf)
+        proj = torch.empty(2, 40, 6 * 2 * 32, requires_grad=True)
+        _twice(ops.castle_attention_packed(proj, 2, 0.125), proj)
+        x, w, nw = (torch.empty(*s, requires_grad=True) for s in ((2, 40, 64), (48, 64), (64,)))
+        for leaf in (x, nw):
+            _twice(torch.ops.castle_hip.rms_norm(x, nw, None)[0], leaf)
+        for leaf in (x, w):
+            _twice(torch.ops.castle_hip.linear(x, w), leaf)
+        # a graph that nobody differentiates is no error, and without one nothing hangs on the gradients
+        y = torch.ops.castle_hip.linear(x, w)
+        assert torch.autograd.grad(y.sum(), x, create_graph=True)[0].requires_grad
+        y = torch.ops.castle_hip.linear(x, w)
+        assert not torch.autograd.grad(y.sum(), x)[0].requires_grad
+
+
 def test_fake_tensor_trace_of_the_module():
     """Castle.forward traces without a GPU: projection -> registered operator -> output projection,
     forward and backward, for the parallel pass with and without the cache."""

@@ -210,6 +210,18 @@ def test_input_changed_in_place_before_the_backward_pass(prenorm):
         assert torch.equal(torch.autograd.grad(y.sum(), leaf)[0], want)
 
 
+@pytest.mark.parametrize("prenorm", [False, True])
+def test_second_derivatives_of_a_layer_raise(prenorm):
+    m = make(64, 2, 32, prenorm=prenorm)
+    x = torch.randn(2, 40, 64, device=DEV, requires_grad=True)
+    for leaf in (x, m.to_all_qkv.weight, m.combine_heads.weight):
+        y = m(x)
+        first, = torch.autograd.grad(y.square().sum(), leaf, create_graph=True)
+        with pytest.raises(RuntimeError, match="differentiate twice"):
+            (y.sum() + first.square().sum()).backward()
+        assert torch.equal(first, torch.autograd.grad(m(x).square().sum(), leaf)[0])
+
+
 def test_multi_token_with_cache_is_rejected():
     m = make(32, 2, 16)
     x = torch.randn(1, 4, 32).to(DEV)

@@ -105,6 +105,22 @@ def test_language_model_blocks_equal_the_modules():
             assert (a - b).norm() <= 1e-4 * b.norm()
 
 
+def test_second_derivatives_of_the_language_model_blocks_raise():
+    """Every parameter's gradient: embedding, attention, feed-forward, head and loss are nodes of their own."""
+    from lookahead_keys_attention_amd import CastleLM
+
+    torch.manual_seed(0)
+    model = CastleLM(num_tokens=64, dim=64, depth=2, heads=2, dim_head=32).to(DEV)
+    ids = torch.randint(0, 64, (2, 40), device=DEV)
+    assert model._plain(ids)
+    for name, p in model.named_parameters():
+        if p.requires_grad:
+            loss = model(ids, return_loss=True)
+            grad, = torch.autograd.grad(loss, p, create_graph=True)
+            with pytest.raises(RuntimeError, match="differentiate twice"):
+                (loss + grad.square().sum()).backward()
+
+
 # tiles of 64 and 128 with remainders in every direction, contractions of less than a step, ranges of the contraction
 @pytest.mark.parametrize("rows,n,k", [(1, 8, 8), (63, 72, 40), (65, 128, 200), (96, 768, 128), (257, 1536, 264), (1003, 256, 2048), (3000, 520, 512),
                                       (4500, 2048, 512)])
