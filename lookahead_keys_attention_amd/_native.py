@@ -48,6 +48,7 @@ EXPORTED_SYMBOLS = (
     "castle_sample",
     "castle_gather_rows",
     "castle_small_linear_fused",
+    "castle_gemm_operand_ok",
     "castle_gemm_workspace_bytes",
     "castle_gemm_amax_ok",
     "castle_gemm",

@@ -578,6 +578,9 @@ int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns)
   return castle::gemm_amax_ok(M, N, K, es, column, column + columns);
 }
 
+// The kernel forms element offsets in 32 bits and runs ahead of the last row by up to three steps of the contraction.
+int castle_gemm_operand_ok(int64_t rows, int64_t ld) { return rows >= 0 && ld >= 0 && ld < (int64_t)1 << 31 && rows < (int64_t)1 << 31 && (rows + 192) * ld < (int64_t)1 << 31; }
+
 int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
                 int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream) {
   const int64_t need = castle_gemm_workspace_bytes(M, N, K, dtype, epilogue);
@@ -585,6 +588,7 @@ int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b
   static_assert(CASTLE_AMAX_PARTIALS == castle::kAmaxBlocks && CASTLE_GEMM_PLAIN == castle::kGemmPlain && CASTLE_GEMM_GELU == castle::kGemmGelu && CASTLE_GEMM_GELU_SLOPE == castle::kGemmGeluSlope, "");
   const int v = 16 / elem_size(dtype);
   const int a_row = a_free_contiguous ? M : K, b_row = b_free_contiguous ? N : K;
+  if (!castle_gemm_operand_ok(a_free_contiguous ? K : M, lda) || !castle_gemm_operand_ok(b_free_contiguous ? K : N, ldb)) return CASTLE_ERR_SHAPE;
   if (a_row % v != 0 || b_row % v != 0 || lda < a_row || ldb < b_row || ldc < N || lda % v != 0 || ldb % v != 0 || ldc % v != 0 ||
       (a_free_contiguous && !b_free_contiguous))
     return CASTLE_ERR_SHAPE;

@@ -107,6 +107,24 @@ def test_small_linear_and_static_step_validate_on_the_host(lib):
     assert lib.castle_decode_step(v, v, v, v, 8, 8, v, v, v, v, v, v, 1, 1, 128, 1, 0.1, 0, v, None, 4096, 1 << 30, None) == -2
 
 
+def test_products_refuse_operands_beyond_32_bit_offsets(lib):
+    vp, i, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    lib.castle_gemm.argtypes = [vp, i64, i, vp, i64, i, vp, i64, i, i, i, i, i, vp, vp, vp, i64, vp]
+    lib.castle_gemm_operand_ok.argtypes = [i64, i64]
+
+    def gemm(lda, a_t, ldb, b_t, M=40000, N=64, K=64):
+        return lib.castle_gemm(4096, lda, a_t, 4096, ldb, b_t, 4096, N, M, N, K, 1, 0, None, None, 4096, 1 << 40, None)
+
+    for ld in (65536, 1 << 31, (1 << 32) + 64, 1 << 40):   # 40000 rows of 65536: 2.6e9 elements; the others do not fit 32 bits themselves
+        assert gemm(ld, 0, 64, 0) == -2
+        assert gemm(64, 0, ld, 0, M=64, N=40000) == -2
+        assert gemm(64, 0, ld, 1, M=64, K=40000) == -2
+        assert gemm(ld, 1, 64, 1, M=64, K=40000) == -2
+        assert not lib.castle_gemm_operand_ok(40000, ld)
+    # the last element at 2^31 and just inside, three steps of the contraction ahead
+    assert lib.castle_gemm_operand_ok(32767 - 192, 65536) and not lib.castle_gemm_operand_ok(32768 - 192, 65536)
+
+
 def test_check_raises_with_message(lib):
     with pytest.raises(RuntimeError, match="unsupported shape"):
         N.check(-2, "castle_fwd")

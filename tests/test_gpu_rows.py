@@ -150,6 +150,26 @@ def test_products(rows, n, k, dtype):
     check(host().product(dy, False, w, True, 2, u), plain * slope, "slope")
 
 
+def test_projection_of_rows_beyond_32_bit_offsets():
+    """Rows that lie further apart than the products' offsets reach: 40000 of them, 65536 elements apart."""
+    from lookahead_keys_attention_amd import Castle
+
+    torch.manual_seed(0)
+    model = Castle(64, heads=1, dim_head=16, use_triton=True).to(DEV).bfloat16()
+    wide = torch.empty(8, 5000, 65536, device=DEV, dtype=torch.bfloat16)
+    x = wide[..., :64]
+    x.copy_(torch.randn(8, 5000, 64, device=DEV))
+    with pytest.raises(ValueError):
+        host().product(x.flatten(0, 1), False, model.to_all_qkv.weight.detach(), False, 0, None)
+    results = []
+    for rows in (x, x.contiguous()):
+        leaf = rows.detach().requires_grad_()
+        y = model(leaf)
+        results.append([y, *torch.autograd.grad(y.float().square().sum(), [leaf, *model.parameters()])])
+    for a, b in zip(*results):   # (the library's products and the kernels' order their sums differently)
+        assert (a - b).float().norm() <= 1e-2 * b.float().norm()
+
+
 @pytest.mark.parametrize("rows,n,k,column,columns", [(1, 64, 64, 8, 16), (130, 576, 128, 192, 96), (1000, 1536, 256, 512, 256), (2048, 512, 256, 0, 512),
                                                      (5000, 3072, 512, 1024, 512)])
 def test_product_leaves_partial_maxima(rows, n, k, column, columns):
