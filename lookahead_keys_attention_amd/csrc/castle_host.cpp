@@ -422,10 +422,10 @@ std::tuple<Tensor, Tensor> rms_norm_autograd(const Tensor& x, const Tensor& weig
   return {r[0], r[1]};
 }
 
-// a (M, K), or (K, M) with a_t; b (N, K), or (K, N) with b_t -> (M, N); rows contiguous up to a leading dimension, the last
-// element within reach of the kernel's 32-bit offsets
+// a (M, K), or (K, M) with a_t; b (N, K), or (K, N) with b_t -> (M, N); rows contiguous up to a leading dimension (not
+// repeated or overlapping ones), the last element within reach of the kernel's 32-bit offsets
 bool product_rows(const Tensor& t) {
-  return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) % (16 / t.element_size()) == 0 && t.size(1) % (16 / t.element_size()) == 0 && aligned16(t) &&
+  return t.dim() == 2 && t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % (16 / t.element_size()) == 0 && t.size(1) % (16 / t.element_size()) == 0 && aligned16(t) &&
          castle_gemm_operand_ok(t.size(0), t.stride(0));
 }
 Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux, const castle_amax* amax = nullptr) {

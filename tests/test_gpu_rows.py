@@ -170,6 +170,26 @@ def test_projection_of_rows_beyond_32_bit_offsets():
         assert (a - b).float().norm() <= 1e-2 * b.float().norm()
 
 
+def test_rows_that_overlap_in_memory():
+    """Inputs and output gradients whose rows are one row repeated (stride 0), or windows of one row: a sum over the
+    sequence hands such gradients back."""
+    from lookahead_keys_attention_amd import Castle
+
+    torch.manual_seed(0)
+    line = torch.randn(1, 1, 64 + 8 * 39, device=DEV)
+    for prenorm in (False, True):
+        model = Castle(64, heads=2, dim_head=32, use_triton=True, prenorm=prenorm).to(DEV)
+        for x in (line[..., :64].expand(2, 40, 64), line[0].unfold(1, 64, 8), torch.randn(1, 40, 64, device=DEV)):
+            for pool in (lambda y: y.sum(dim=1), lambda y: y.sum(dim=(0, 1))):
+                results = []
+                for rows in (x, x.contiguous()):
+                    y = model(rows)
+                    pooled = pool(y) if rows is x else pool(y * 1)   # (the product's gradient is contiguous)
+                    results.append([y, *torch.autograd.grad(pooled.square().sum(), model.parameters())])
+                for a, b in zip(*results):   # (other products, so other orders of the 32-bit sums)
+                    assert (a - b).norm() <= 1e-4 * b.norm()
+
+
 @pytest.mark.parametrize("rows,n,k,column,columns", [(1, 64, 64, 8, 16), (130, 576, 128, 192, 96), (1000, 1536, 256, 512, 256), (2048, 512, 256, 0, 512),
                                                      (5000, 3072, 512, 1024, 512)])
 def test_product_leaves_partial_maxima(rows, n, k, column, columns):
