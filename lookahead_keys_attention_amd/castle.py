@@ -243,10 +243,17 @@ class _ManyRowLinear(torch.autograd.Function):
         return dx, dw
 
 
+def _unmodified(module, kind) -> bool:
+    """True for a module of exactly this kind that runs its class's forward and nothing else: nothing hooked onto it, no
+    `forward` of its own (offloading, adapters and quantisation wrappers replace it on the instance)."""
+    return type(module) is kind and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+
+
 def _linear(layer, t):
     """layer(t) for a bias-free nn.Linear, through _ManyRowLinear where its weight gradient pays."""
     rows = t.numel() // t.shape[-1] if t.shape[-1] else 0
-    if (t.is_cuda and layer.bias is None and t.dtype in (torch.bfloat16, torch.float16) and layer.weight.dtype == t.dtype
+    if (t.is_cuda and _unmodified(layer, nn.Linear) and layer.bias is None and t.dtype in (torch.bfloat16, torch.float16) and layer.weight.dtype == t.dtype
             and rows >= SPLIT_WGRAD_MIN_ROWS and rows % SPLIT_ROWS_INTO == 0 and t.is_contiguous()
             and torch.is_grad_enabled() and layer.weight.requires_grad):
         return _ManyRowLinear.apply(t, layer.weight)
@@ -389,8 +396,8 @@ class Castle(nn.Module):
         return (y, next_cache) if return_next_cache else y
 
     def _plain(self, x):
-        """True if the whole layer may run as one native call: unmodified projections and norm, nothing
-        hooked onto them, nothing that wants to see the operators one by one."""
+        """True if the whole layer may run as one native call: unmodified projections and norm, nothing that
+        wants to see the operators one by one."""
         # (this runs on every call: a cached step of one sequence takes about 15 us in all)
         kind = type(x)
         if (kind is not torch.Tensor and kind is not nn.Parameter) or x.dim() != 3 or ops.CHECK_RANGE or _has_any_global_hook():
@@ -400,29 +407,27 @@ class Castle(nn.Module):
             return False
         modules, dtype, device, dim = self._modules, x.dtype, x.device, x.shape[2]
         norm, qkv, combine = modules["norm"], modules["to_all_qkv"], modules["combine_heads"]
-        if type(norm) is nn.RMSNorm:
+        if _unmodified(norm, nn.RMSNorm):
             weight = norm._parameters["weight"]
-            if (type(weight) is not nn.Parameter or weight.dtype is not dtype or weight.device != device or norm.normalized_shape != (dim,)
-                    or norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks):
+            if type(weight) is not nn.Parameter or weight.dtype is not dtype or weight.device != device or norm.normalized_shape != (dim,):
                 return False
-        elif type(norm) is not nn.Identity or norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks:
+        elif not _unmodified(norm, nn.Identity):
             return False
-        if type(qkv) is not nn.Linear or type(combine) is not nn.Linear or qkv.in_features != dim:
+        if not (_unmodified(qkv, nn.Linear) and _unmodified(combine, nn.Linear)) or qkv.in_features != dim:
             return False
         for layer in (qkv, combine):
             params = layer._parameters
             weight = params.get("weight")
-            if (type(weight) is not nn.Parameter or weight.dtype is not dtype or weight.device != device or params.get("bias") is not None
-                    or layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks):
+            if type(weight) is not nn.Parameter or weight.dtype is not dtype or weight.device != device or params.get("bias") is not None:
                 return False
         return True
 
     def _traceable(self, x):
         """`_plain` as far as a tracing compiler can follow it."""
         norm = self.norm
-        return (type(norm) is nn.Identity or type(norm) is nn.RMSNorm and norm.weight.dtype == x.dtype) and all(
-            type(layer) is nn.Linear and layer.bias is None and layer.weight.dtype == x.dtype for layer in (self.to_all_qkv, self.combine_heads)
-        ) and not torch.is_autocast_enabled("cuda")
+        return (_unmodified(norm, nn.Identity) or _unmodified(norm, nn.RMSNorm) and norm.weight is not None and norm.weight.dtype == x.dtype) and all(
+            _unmodified(layer, nn.Linear) and layer.bias is None and layer.weight.dtype == x.dtype for layer in (self.to_all_qkv, self.combine_heads)
+        ) and not _has_any_global_hook() and not torch.is_autocast_enabled("cuda")
 
     def _layer_native(self, x, want_cache, delta=None):
         """The parallel pass as one native call (csrc/castle_host.cpp): norm, projection, attention core,
@@ -452,9 +457,10 @@ class Castle(nn.Module):
         nn.Identity) in front, GELU (`activation="gelu"`) and a residual behind.  On the native
         single-token step the few rows go through the library's own small-M kernel, which does all
         of it in one launch (inference only); otherwise the layers themselves run."""
-        if isinstance(norm, nn.Identity):
+        if norm is not None and _unmodified(norm, nn.Identity):
             norm = None
-        if native_step and ops.small_linear_ok(t, layer.weight) and (norm is None or isinstance(norm, nn.RMSNorm)):
+        if (native_step and _unmodified(layer, nn.Linear) and layer.bias is None and (norm is None or _unmodified(norm, nn.RMSNorm))
+                and ops.small_linear_ok(t, layer.weight)):
             return ops.small_linear(t, layer.weight, norm=norm, activation=activation, residual=residual)
         y = _linear(layer, t if norm is None else norm(t))
         if activation == "gelu":

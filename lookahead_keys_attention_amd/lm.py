@@ -23,7 +23,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from . import _native, ops
-from .castle import Castle, _linear
+from .castle import Castle, _linear, _unmodified
 
 
 READ_ONCE_BYTES = 320_000_000
@@ -51,10 +51,17 @@ def top_k(logits: torch.Tensor, thres: float = 0.9) -> torch.Tensor:
     return torch.full_like(logits, float("-inf")).scatter_(-1, index, values)
 
 
+def _is_block(feed_forward) -> bool:
+    """True if the block may be taken apart: [norm, linear, erf GELU, linear] and nothing that wants to see a call of it."""
+    return _unmodified(feed_forward, nn.Sequential) and len(feed_forward) == 4 and _unmodified(feed_forward[2], nn.GELU) and feed_forward[2].approximate == "none"
+
+
 def token_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Tensor:
     """h + feed_forward(h) for a single-token step (inference), the block being [norm, linear,
     GELU, linear]: two launches of the small-M linear kernel (norm and GELU ride on the first, the
     residual on the second) when it can take them (16-bit GPU tensors), the layers themselves otherwise."""
+    if not _is_block(feed_forward):
+        return h + feed_forward(h)
     norm, up, act, down = feed_forward
     hidden = Castle._project(up, h, True, norm=norm, activation="gelu")
     return Castle._project(down, hidden, True, residual=h)
@@ -63,13 +70,10 @@ def token_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Te
 def block_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Tensor:
     """feed_forward(h) for the block [norm, linear, GELU, linear] over many rows: the layers themselves,
     with the two weight gradients formed in row ranges where that pays (castle._linear)."""
+    if not _is_block(feed_forward):
+        return feed_forward(h)
     norm, up, act, down = feed_forward
     return _linear(down, act(_linear(up, norm(h))))
-
-
-def _is_plain(module, kind) -> bool:
-    """True for an unmodified module of exactly this kind with no hooks on it."""
-    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
 
 
 @contextlib.contextmanager
@@ -140,14 +144,15 @@ class GraphedDecoder:
         self.counters.copy_(torch.tensor([self.length, self.base0], dtype=torch.int32), non_blocking=False)
 
     def _signature(self):
-        """What the captured graph has baked in: the addresses of the weights it reads."""
-        return tuple(p.data_ptr() for p in self.model.parameters())
+        """What the captured graph has baked in: the addresses of the weights it reads.  None (never the same again) for a
+        model with modules that run something of their own."""
+        return tuple(p.data_ptr() for p in self.model.parameters()) if self.model._unmodified() else None
 
     def fits(self, caches, max_len: int) -> bool:
         """True if `load(caches)` can reuse this graph for a generation of up to max_len rows."""
         first = getattr(caches[0], "_store", None)
         mine = self.stores[0].buffers[0]
-        return (first is not None and max_len <= self.capacity and self.signature == self._signature()
+        return (first is not None and max_len <= self.capacity and self.signature is not None and self.signature == self._signature()
                 and first.buffers[0].shape[:2] == mine.shape[:2] and first.buffers[0].shape[3] == mine.shape[3]
                 and first.buffers[0].dtype == mine.dtype and first.buffers[0].device == mine.device
                 and first.u_half == self.stores[0].u_half)
@@ -171,7 +176,7 @@ class GraphedDecoder:
     def _step(self):
         model = self.model
         embedding = model.token_emb
-        plain = type(embedding) is nn.Embedding and embedding.max_norm is None and not embedding._forward_hooks and not embedding._forward_pre_hooks
+        plain = _unmodified(embedding, nn.Embedding) and embedding.max_norm is None
         h = _native.host().gather_rows(embedding.weight, self.token) if plain else embedding(self.token)
         for (attention, feed_forward), store in zip(model.layers, self.stores):
             h = attention.graph_step(h, store, self.t_device, self.base_device, residual=h)
@@ -253,26 +258,25 @@ class CastleLM(nn.Module):
         """True if whole sequences may run as one native call per block: native layers, unmodified modules, nothing
         hooked onto any of them."""
         embedding, weight = self.token_emb, self.token_emb.weight
-        if (not x.is_cuda or x.dtype != torch.long or not _is_plain(embedding, nn.Embedding) or embedding.max_norm is not None
+        if (not x.is_cuda or x.dtype != torch.long or not _unmodified(embedding, nn.Embedding) or embedding.max_norm is not None
                 or embedding.padding_idx is not None or embedding.scale_grad_by_freq or embedding.sparse or weight.device != x.device
                 or weight.dtype not in _native.DTYPE_CODES or not _native.is_built()):
             return False
         final, logits, dtype = self.final_norm, self.to_logits, weight.dtype
-        if not (_is_plain(final, nn.RMSNorm) and _is_plain(logits, nn.Linear) and logits.bias is None and logits.weight.dtype is dtype
+        if not (_unmodified(final, nn.RMSNorm) and _unmodified(logits, nn.Linear) and logits.bias is None and logits.weight.dtype is dtype
                 and final.weight is not None and final.weight.dtype is dtype) or not len(self.layers):
             return False
         like = weight.detach()[None]   # what every block gets, as far as the blocks look at it
         for block in self.layers:
-            if not _is_plain(block, nn.ModuleList) or len(block) != 2:
+            if not _unmodified(block, nn.ModuleList) or len(block) != 2:
                 return False
             attention, feed_forward = block
-            if not (_is_plain(attention, Castle) and attention.use_triton and ops.kernels_support(attention.dim_head, dtype) and attention._plain(like)
-                    and _is_plain(feed_forward, nn.Sequential) and len(feed_forward) == 4):
+            if not (_unmodified(attention, Castle) and attention.use_triton and ops.kernels_support(attention.dim_head, dtype) and attention._plain(like)
+                    and _is_block(feed_forward)):
                 return False
-            norm, up, act, down = feed_forward
-            if not (_is_plain(norm, nn.RMSNorm) and norm.weight is not None and norm.weight.dtype is dtype and _is_plain(up, nn.Linear) and up.bias is None
-                    and up.weight.dtype is dtype and _is_plain(act, nn.GELU) and act.approximate == "none" and _is_plain(down, nn.Linear)
-                    and down.bias is None and down.weight.dtype is dtype):
+            norm, up, _, down = feed_forward
+            if not (_unmodified(norm, nn.RMSNorm) and norm.weight is not None and norm.weight.dtype is dtype and _unmodified(up, nn.Linear) and up.bias is None
+                    and up.weight.dtype is dtype and _unmodified(down, nn.Linear) and down.bias is None and down.weight.dtype is dtype):
                 return False
         return True
 
@@ -311,6 +315,10 @@ class CastleLM(nn.Module):
         """Drops the graph (and the cache buffers it was captured on) kept from the last `sample` call."""
         self.__dict__.pop("_kept_decoder", None)
 
+    def _unmodified(self) -> bool:
+        """True if a replayed graph of a token step does what a call of every module would: no hooks, no replaced `forward`."""
+        return all(_unmodified(module, type(module)) for module in self.modules())
+
     def _native_on_gpu(self, device) -> bool:
         return device.type == "cuda" and _native.is_built() and all(attention.use_triton for attention, _ in self.layers)
 
@@ -320,11 +328,12 @@ class CastleLM(nn.Module):
         The prompt goes through the parallel path once; afterwards each step feeds the last token
         and the per-layer caches.  temperature = 0 picks the arg-max (no noise).
         graph: replay the token steps as one captured HIP graph (`GraphedDecoder`).  None = when
-        the model runs the native kernels on a GPU and more than a few steps follow; True insists."""
+        the model runs the native kernels on a GPU, its modules are unmodified (no hooks, which a replay would not
+        run) and more than a few steps follow; True insists."""
         prompt_len = prompt.shape[-1]
         steps = max(0, seq_len - prompt_len)
         if graph is None:
-            graph = self._native_on_gpu(prompt.device) and steps > 8
+            graph = self._native_on_gpu(prompt.device) and steps > 8 and self._unmodified()
         elif graph and not self._native_on_gpu(prompt.device):
             raise RuntimeError("graph=True needs the native kernels on a GPU")
 

@@ -222,6 +222,33 @@ def test_second_derivatives_of_a_layer_raise(prenorm):
         assert torch.equal(first, torch.autograd.grad(m(x).square().sum(), leaf)[0])
 
 
+@pytest.mark.parametrize("name", ["norm", "to_all_qkv", "combine_heads"])
+def test_replaced_forward_and_traced_hooks_run(name):
+    m = make(64, 2, 32, prenorm=True)
+    x = torch.randn(2, 40, 64, device=DEV)
+    layer, calls = getattr(m, name), []
+    original = layer.forward
+
+    def halved(t):
+        calls.append(t.shape)
+        return original(t) * 0.5
+
+    with torch.no_grad():
+        layer.forward = halved
+        y, cache = m(x, return_next_cache=True)
+        step, _ = m(x[:, :1], cache=cache)
+        del layer.forward
+        assert len(calls) == 2
+        handle = layer.register_forward_hook(lambda module, args, out: out * 0.5)
+        assert (m(x) - y).norm() <= 1e-5 * y.norm()
+        compiled = torch.compile(m, backend="aot_eager")(x)
+        assert (compiled - y).norm() <= 1e-5 * y.norm()
+        handle.remove()
+        layer.weight.mul_(0.5)   # the same in the weights
+        y2, cache = m(x, return_next_cache=True)
+        assert (y - y2).norm() <= 1e-5 * y2.norm() and (step - m(x[:, :1], cache=cache)[0]).norm() <= 1e-5 * step.norm()
+
+
 def test_multi_token_with_cache_is_rejected():
     m = make(32, 2, 16)
     x = torch.randn(1, 4, 32).to(DEV)

@@ -105,6 +105,31 @@ def test_language_model_blocks_equal_the_modules():
             assert (a - b).norm() <= 1e-4 * b.norm()
 
 
+def test_replaced_forward_in_a_language_model_runs():
+    from lookahead_keys_attention_amd import CastleLM
+
+    torch.manual_seed(0)
+    model = CastleLM(num_tokens=64, dim=64, depth=2, heads=2, dim_head=32).to(DEV)
+    ids = torch.randint(0, 64, (2, 40), device=DEV)
+    attention, feed_forward = model.layers[1]
+    for module in (model.token_emb, attention, attention.norm, feed_forward, feed_forward[0], feed_forward[1], feed_forward[2], feed_forward[3],
+                   model.final_norm, model.to_logits):
+        assert model._plain(ids)
+        calls, original = [], module.forward
+
+        def counted(*args, **kwargs):
+            calls.append(1)
+            return original(*args, **kwargs)
+
+        module.forward = counted
+        assert not model._plain(ids)
+        model(ids, return_loss=True)
+        assert len(calls) == 1
+        model.sample(ids[:, :6], 6 + 12)   # a prompt, eleven steps
+        assert len(calls) == 1 + 12
+        del module.forward
+
+
 def test_second_derivatives_of_the_language_model_blocks_raise():
     """Every parameter's gradient: embedding, attention, feed-forward, head and loss are nodes of their own."""
     from lookahead_keys_attention_amd import CastleLM

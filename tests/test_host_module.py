@@ -134,3 +134,37 @@ def test_single_token_call_is_differentiable_when_grad_is_needed():
     y, _ = m(x[:, 2:], cache=cache)
     y.sum().backward()
     assert m.to_all_qkv.weight.grad is not None and m.to_all_qkv.weight.grad.abs().sum() > 0
+
+
+def test_layer_with_a_changed_module_is_not_taken_as_one_call():
+    """Hooks and a `forward` set on the instance must run: such a layer goes through its modules, untraced and traced."""
+    m = Castle(32, heads=2, dim_head=16, use_triton=True, prenorm=True)
+    x = torch.randn(1, 4, 32)
+
+    class Traced(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.m = m
+
+        def forward(self, x):
+            return x + 1, self.m._traceable(x)
+
+    def taken():
+        torch._dynamo.reset()
+        plain = m._plain(x)
+        assert plain == m._traceable(x) == torch.compile(Traced(), backend="eager", fullgraph=True)(x)[1]
+        return plain
+
+    assert taken()
+    for layer in (m.norm, m.to_all_qkv, m.combine_heads):
+        for register in (layer.register_forward_hook, layer.register_forward_pre_hook, layer.register_full_backward_hook):
+            handle = register(lambda *_: None)
+            assert not taken()
+            handle.remove()
+        layer.forward = type(layer).forward.__get__(layer)
+        assert not taken()
+        del layer.forward
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *_: None)
+    assert not m._plain(x) and not m._traceable(x)
+    handle.remove()
+    assert taken()
