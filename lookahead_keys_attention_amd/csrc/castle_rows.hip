@@ -196,11 +196,11 @@ template <typename T> __global__ __launch_bounds__(kThreads) void ce_kernel(Cros
       for (int e = 0; e < V; ++e) mn = fmaxf(mn, v[e]);
       s *= m == -INFINITY ? 0.f : fast_exp2((m - mn) * kLog2e);
 #pragma unroll
-      for (int e = 0; e < V; ++e) s += mn == -INFINITY ? 0.f : fast_exp2((v[e] - mn) * kLog2e);
+      for (int e = 0; e < V; ++e) s += mn == -INFINITY ? v[e] != v[e] ? NAN : 0.f : fast_exp2((v[e] - mn) * kLog2e);   // (fmaxf drops NaNs)
       m = mn;
     }
     const float M = row_max<64>(m);
-    const float lse = M + logf(row_sum<64>(m == -INFINITY ? 0.f : s * fast_exp2((m - M) * kLog2e)));
+    const float lse = M + logf(row_sum<64>(m == -INFINITY ? s : s * fast_exp2((m - M) * kLog2e)));   // (nothing seen but -inf: 0, or NaN)
     if (lane == 0) a.lse[row] = lse;
     if (t == -100) continue;
     sum += t >= 0 && t < a.V ? lse - (float)x[t] : NAN;

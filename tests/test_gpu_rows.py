@@ -64,6 +64,37 @@ def test_cross_entropy(classes, dtype):
     assert host().cross_entropy(leaf.detach(), bad.to(DEV)[:, 1:]).isnan()
 
 
+@pytest.mark.parametrize("classes", [8, 256, 1000])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_cross_entropy_of_nan_and_infinite_logits(classes, dtype):
+    """One NaN, an aligned 16-byte piece of them, a whole row; infinities of either sign: like the library on the CPU."""
+    piece, inf, nan = 16 // dtype.itemsize, float("inf"), float("nan")
+    g = torch.Generator().manual_seed(classes)
+    base, target = torch.randn(1, 5, classes, generator=g).to(dtype), torch.randint(0, classes, (1, 5), generator=g)
+    last = classes - piece
+    for where, value in ((slice(0, 1), nan), (slice(0, piece), nan), (slice(last, classes), nan), (slice(0, classes), nan), (slice(0, piece), -inf),
+                         (slice(0, classes), -inf), (slice(0, 1), inf), (slice(0, classes), inf)):
+        logits = base.clone()
+        logits[0, 2, where] = value
+        if value == -inf and classes > piece:
+            target[0, 2] = last   # (a class that is not among them)
+        leaf, ref = logits.to(DEV).requires_grad_(), logits.double().requires_grad_()
+        loss, want = host().cross_entropy(leaf, target.to(DEV)), F.cross_entropy(ref.transpose(1, 2), target)
+        assert loss.isnan() == want.isnan().to(DEV) and (want.isnan() or (loss.cpu().double() - want).abs() <= TOL[dtype] * want.abs())
+        loss.backward()
+        want.backward()
+        assert torch.equal(leaf.grad.isnan().cpu(), ref.grad.isnan())
+        finite = ~ref.grad.isnan()
+        close(leaf.grad.cpu()[finite], ref.grad[finite], dtype, "dlogits")
+        # a row that does not count brings nothing in
+        target_without = target.clone()
+        target_without[0, 2] = -100
+        leaf.grad = None
+        loss = host().cross_entropy(leaf, target_without.to(DEV))
+        loss.backward()
+        assert loss.isfinite() and leaf.grad.isfinite().all() and not leaf.grad[0, 2].any()
+
+
 @pytest.mark.parametrize("vocabulary,dim", [(5, 8), (256, 512), (300, 1032)])
 def test_embedding_gradient(vocabulary, dim):
     g = torch.Generator().manual_seed(vocabulary)
