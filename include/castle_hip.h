@@ -328,7 +328,7 @@ int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream);
 
 /* Mean cross entropy (train_triton.py:166-171).  Row r of the logits belongs to the class target[(r / target_n) * target_ld +
- * r % target_n]; rows of class -100 do not count, a class outside 0 .. classes - 1 makes the loss NaN.  loss: one element
+ * r % target_n]; rows of class -100 do not count, a class outside 0 .. classes - 1 makes the loss and the row's gradient NaN.  loss: one element
  * of the type; lse: one float per row and inv_count: one float, both kept for the backward pass, which multiplies by
  * the one element of `grad`. */
 #define CASTLE_CROSS_ENTROPY_WORKSPACE 8192

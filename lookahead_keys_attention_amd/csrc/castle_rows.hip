@@ -174,7 +174,7 @@ template <typename T> __global__ __launch_bounds__(kThreads) void part_sum_kerne
 }
 
 // Mean cross entropy of rows of logits against class numbers (torch's default ignore_index -100 does not count; a class
-// outside 0 .. V - 1 makes the loss NaN).  One wave per row; lse of every row is kept for the backward pass.  16384 x 256
+// outside 0 .. V - 1 makes the loss and its row's gradient NaN).  One wave per row; lse of every row is kept for the backward pass.  16384 x 256
 // bf16 in the layout the logits come in: under 10 us each way (190 and 176 us as operators on the transposed logits).
 __device__ __forceinline__ int64_t target_of(const CrossEntropyArgs& a, int64_t row) { return a.target[row / a.n * a.target_ld + row % a.n]; }
 
@@ -237,12 +237,13 @@ template <typename T> __global__ __launch_bounds__(kThreads) void ce_bwd_kernel(
   const int64_t row = (int64_t)blockIdx.x * kRowWaves + wave_id();
   if (row >= a.rows) return;
   const int64_t t = target_of(a, row), at = row * a.V;
-  const float g = t == -100 ? 0.f : (float)*grad * *inv_count, lse = a.lse[row];
+  const bool counts = t != -100;
+  const float g = t >= 0 && t < a.V ? (float)*grad * *inv_count : NAN, lse = a.lse[row];
   for (int i = lane; i < pieces; i += 64) {
     const vf v = __builtin_convertvector(*reinterpret_cast<const vt*>(static_cast<const T*>(a.logits) + at + i * V), vf);
     vf d;
 #pragma unroll
-    for (int e = 0; e < V; ++e) d[e] = g == 0.f ? 0.f : g * (fast_exp2((v[e] - lse) * kLog2e) - (t == i * V + e ? 1.f : 0.f));
+    for (int e = 0; e < V; ++e) d[e] = !counts ? 0.f : g * (fast_exp2((v[e] - lse) * kLog2e) - (t == i * V + e ? 1.f : 0.f));
     *reinterpret_cast<vt*>(dlogits + at + i * V) = __builtin_convertvector(d, vt);
   }
 }

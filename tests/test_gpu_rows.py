@@ -95,6 +95,15 @@ def test_cross_entropy_of_nan_and_infinite_logits(classes, dtype):
         assert loss.isfinite() and leaf.grad.isfinite().all() and not leaf.grad[0, 2].any()
 
 
+def test_cross_entropy_of_a_class_out_of_range():
+    logits = torch.randn(2, 3, 264, device=DEV).requires_grad_()
+    for bad in (264, -1, 1 << 40, -(1 << 40)):
+        target = torch.tensor([[1, 2, 3], [4, bad, -100]], device=DEV)
+        loss = host().cross_entropy(logits, target)
+        grad, = torch.autograd.grad(loss, logits)
+        assert loss.isnan() and grad[1, 1].isnan().all() and grad[0].isfinite().all() and not grad[1, 2].any()
+
+
 @pytest.mark.parametrize("vocabulary,dim", [(5, 8), (256, 512), (300, 1032)])
 def test_embedding_gradient(vocabulary, dim):
     g = torch.Generator().manual_seed(vocabulary)
