@@ -27,6 +27,11 @@ from .castle import Castle, _linear, _unmodified
 
 
 READ_ONCE_BYTES = 320_000_000
+# The sampling kernel gives a row of logits to one workgroup, the operators below spread it over the GPU: up to this
+# vocabulary the kernel is ahead at any number of rows (us per token with the random numbers, kernel / operators, 1 row and
+# 64, logits of one leading digit last: 256 11 / 72 and 12 / 72; 8192 35 / 95 and 39 / 131; 20480 80 / 101 and 82 / 145,
+# 88 / 102; 28672 107 / 103 and 110 / 168, 122 / 102; 131072 462 / 108 and 533 / 777).
+SAMPLER_MAX_VOCABULARY = 20480
 
 
 # -- sampling helpers (train_triton.py:56-71) ------------------------------------------------
@@ -49,6 +54,14 @@ def top_k(logits: torch.Tensor, thres: float = 0.9) -> torch.Tensor:
     k = math.ceil((1.0 - thres) * logits.shape[-1])
     values, index = logits.topk(k, dim=-1)
     return torch.full_like(logits, float("-inf")).scatter_(-1, index, values)
+
+
+def pick_token(logits, temperature, filter_thres, generator=None):
+    """(batch, n, vocabulary) logits -> (batch, 1) tokens from the last position; temperature = 0 picks the arg-max."""
+    logits = top_k(logits[:, -1].float(), thres=filter_thres)
+    if temperature == 0:
+        return logits.argmax(dim=-1, keepdim=True)
+    return gumbel_sample(logits, temperature=temperature, generator=generator)
 
 
 def _is_block(feed_forward) -> bool:
@@ -340,21 +353,15 @@ class CastleLM(nn.Module):
         if self._native_on_gpu(prompt.device):
             return self._sample_native(prompt, steps, seq_len, temperature, filter_thres, generator, graph)
 
-        def pick(logits):
-            logits = top_k(logits[:, -1].float(), thres=filter_thres)
-            if temperature == 0:
-                return logits.argmax(dim=-1, keepdim=True)
-            return gumbel_sample(logits, temperature=temperature, generator=generator)
-
         out, cache = prompt, None
         for _ in range(steps):
             logits, cache = self.forward(out if cache is None else out[:, -1:], cache=cache, return_next_cache=True)
-            out = torch.cat((out, pick(logits)), dim=-1)
+            out = torch.cat((out, pick_token(logits, temperature, filter_thres, generator)), dim=-1)
         return out[..., prompt_len:]
 
     def _sample_native(self, prompt, steps, seq_len, temperature, filter_thres, generator, graph):
-        """`sample` with the native kernels: top-k, noise and arg-max of a token are one launch behind the
-        uniform numbers, which come from the generator exactly as `gumbel_noise` draws them; the token
+        """`sample` with the native kernels: top-k, noise and arg-max of a token are one launch (the operators for
+        large vocabularies) behind the uniform numbers, which come from the generator exactly as `gumbel_noise` draws them; the token
         goes straight into the graph's input."""
         host, decoder, cache = _native.host(), None, None
         batch = prompt.shape[0]
@@ -366,6 +373,11 @@ class CastleLM(nn.Module):
                 logits, cache = self.forward(prompt if cache is None else tokens[:, i - 1:i], cache=cache, return_next_cache=True)
                 if graph:
                     decoder = self._decoder_for(cache, seq_len)
+            if logits.shape[-1] > SAMPLER_MAX_VOCABULARY:
+                tokens[:, i:i + 1] = pick_token(logits, temperature, filter_thres, generator)
+                if decoder is not None:
+                    decoder.token.copy_(tokens[:, i:i + 1])
+                continue
             logits = logits[:, -1] if logits.dtype in _native.DTYPE_CODES else logits[:, -1].float()
             k = math.ceil((1.0 - filter_thres) * logits.shape[-1])
             uniform = None

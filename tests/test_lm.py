@@ -259,6 +259,23 @@ def test_sampling_kernel_picks_what_the_operators_pick(vocabulary, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("temperature", [0, 0.7])
+def test_sampling_with_the_operators_of_large_vocabularies(monkeypatch, temperature):
+    """Beyond SAMPLER_MAX_VOCABULARY the operators pick: the same tokens, with and without a graph."""
+    from lookahead_keys_attention_amd import lm
+
+    torch.manual_seed(4)
+    model = lm.CastleLM(num_tokens=300, dim=64, depth=1, dim_head=32, heads=2).to("cuda").eval()
+    prompt = torch.randint(0, 300, (3, 9), device="cuda")
+    picked = []
+    for limit in (lm.SAMPLER_MAX_VOCABULARY, 299):
+        monkeypatch.setattr(lm, "SAMPLER_MAX_VOCABULARY", limit)
+        for graph in (False, True):
+            picked.append(model.sample(prompt, 9 + 14, temperature=temperature, graph=graph, generator=torch.Generator(device="cuda").manual_seed(2)))
+    assert all(torch.equal(picked[0], p) for p in picked[1:]) and picked[0].unique().numel() > 3
+
+
+@pytest.mark.gpu
 def test_sampler_reuses_its_captured_graph_for_a_new_prompt():
     model = make_lm(depth=2, dim=128, heads=2, dim_head=64, rotary=True, native=True).cuda()
     first = model.sample(tokens(2, 30, seed=3).cuda(), seq_len=50, temperature=0.0, graph=True)
