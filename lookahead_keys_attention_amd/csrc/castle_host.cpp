@@ -379,11 +379,13 @@ std::tuple<Tensor, Tensor> rms_norm_op(const Tensor& x, const Tensor& weight, st
   const Normed n = norm_rows(x.reshape({-1, x.size(-1)}), Tensor(), weight, eps, true);
   return {n.h.view(x.sizes()), n.rstd};
 }
-std::tuple<Tensor, Tensor> rms_norm_bwd_op(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight) {
+// (a gradient that is not asked for, of a frozen weight for instance, comes back empty)
+std::tuple<Tensor, Tensor> rms_norm_bwd_op(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight, bool need_x, bool need_w) {
   const c10::DeviceGuard guard(x.device());
   const int64_t D = x.size(-1);
-  auto [dx, dw] = norm_rows_bwd(dh.reshape({-1, D}), x.reshape({-1, D}), rstd, weight, Tensor(), true, true);
-  return {dx.view(x.sizes()), dw};
+  if (!need_x && !need_w) return {at::empty({0}, x.options()), at::empty({0}, weight.options())};
+  auto [dx, dw] = norm_rows_bwd(dh.reshape({-1, D}), x.reshape({-1, D}), rstd, weight, Tensor(), need_x, need_w);
+  return {need_x ? dx.view(x.sizes()) : at::empty({0}, x.options()), need_w ? dw : at::empty({0}, weight.options())};
 }
 struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, std::optional<double> eps) {
@@ -399,15 +401,16 @@ struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
     static const auto op = op_handle<decltype(rms_norm_bwd_op)>("castle_hip::rms_norm_bwd");
     if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
     const auto s = ctx->get_saved_variables();
-    auto [dx, dw] = op.call(g[0], s[0], s[1], s[2]);
-    return {dx, dw, Tensor()};
+    const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
+    auto [dx, dw] = op.call(g[0], s[0], s[1], s[2], need_x, need_w);
+    return {need_x ? dx : Tensor(), need_w ? dw : Tensor(), Tensor()};
   }
 };
-std::tuple<Tensor, Tensor> rms_norm_bwd_autograd(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight) {
+std::tuple<Tensor, Tensor> rms_norm_bwd_autograd(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight, bool need_x, bool need_w) {
   static const auto op = op_handle<decltype(rms_norm_bwd_op)>("castle_hip::rms_norm_bwd");
   const bool graph = at::GradMode::is_enabled() && wants_graph({dh, x, weight});
   const at::AutoDispatchBelowADInplaceOrView below;
-  const auto [dx, dw] = op.call(dh, x, rstd, weight);
+  const auto [dx, dw] = op.call(dh, x, rstd, weight, need_x, need_w);
   if (!graph) return {dx, dw};
   const auto r = no_second_derivatives({dx, dw});
   return {r[0], r[1]};
@@ -522,10 +525,11 @@ Tensor linear_op(const Tensor& x, const Tensor& weight) {
   shape.back() = weight.size(0);
   return project(x.reshape({-1, x.size(-1)}), weight).view(shape);
 }
-std::tuple<Tensor, Tensor> linear_bwd_op(const Tensor& dy_, const Tensor& x, const Tensor& weight) {
+std::tuple<Tensor, Tensor> linear_bwd_op(const Tensor& dy_, const Tensor& x, const Tensor& weight, bool need_x, bool need_w) {
   const c10::DeviceGuard guard(x.device());
   const Tensor dy = dy_.reshape({-1, weight.size(0)});
-  return {input_grad(dy, weight).view(x.sizes()), weight_grad(dy, x.reshape({-1, x.size(-1)}))};
+  return {need_x ? input_grad(dy, weight).view(x.sizes()) : at::empty({0}, x.options()),
+          need_w ? weight_grad(dy, x.reshape({-1, x.size(-1)})) : at::empty({0}, weight.options())};
 }
 struct LinearFn : torch::autograd::Function<LinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight) {
@@ -537,15 +541,16 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     static const auto op = op_handle<decltype(linear_bwd_op)>("castle_hip::linear_bwd");
     const auto s = ctx->get_saved_variables();
-    auto [dx, dw] = op.call(g[0], s[0], s[1]);
-    return {dx, dw};
+    const bool need_x = ctx->needs_input_grad(0), need_w = ctx->needs_input_grad(1);
+    auto [dx, dw] = op.call(g[0], s[0], s[1], need_x, need_w);
+    return {need_x ? dx : Tensor(), need_w ? dw : Tensor()};
   }
 };
-std::tuple<Tensor, Tensor> linear_bwd_autograd(const Tensor& dy, const Tensor& x, const Tensor& weight) {
+std::tuple<Tensor, Tensor> linear_bwd_autograd(const Tensor& dy, const Tensor& x, const Tensor& weight, bool need_x, bool need_w) {
   static const auto op = op_handle<decltype(linear_bwd_op)>("castle_hip::linear_bwd");
   const bool graph = at::GradMode::is_enabled() && wants_graph({dy, x, weight});
   const at::AutoDispatchBelowADInplaceOrView below;
-  const auto [dx, dw] = op.call(dy, x, weight);
+  const auto [dx, dw] = op.call(dy, x, weight, need_x, need_w);
   if (!graph) return {dx, dw};
   const auto r = no_second_derivatives({dx, dw});
   return {r[0], r[1]};
@@ -1006,9 +1011,9 @@ TORCH_LIBRARY(castle_hip, m) {
   m.def("attention_packed_bwd(Tensor proj, Tensor merged, Tensor dmerged, Tensor ws, Tensor state, int heads, float scale, int flags) "
         "-> Tensor", tags);
   m.def("rms_norm(Tensor x, Tensor weight, float? eps) -> (Tensor, Tensor)", tags);
-  m.def("rms_norm_bwd(Tensor dh, Tensor x, Tensor rstd, Tensor weight) -> (Tensor, Tensor)", tags);
+  m.def("rms_norm_bwd(Tensor dh, Tensor x, Tensor rstd, Tensor weight, bool need_x=True, bool need_w=True) -> (Tensor, Tensor)", tags);
   m.def("linear(Tensor x, Tensor weight) -> Tensor", tags);
-  m.def("linear_bwd(Tensor dy, Tensor x, Tensor weight) -> (Tensor, Tensor)", tags);
+  m.def("linear_bwd(Tensor dy, Tensor x, Tensor weight, bool need_x=True, bool need_w=True) -> (Tensor, Tensor)", tags);
 }
 TORCH_LIBRARY_IMPL(castle_hip, CUDA, m) {
   m.impl("attention", &attention);

@@ -84,7 +84,8 @@ def _as_readable(t: torch.Tensor) -> torch.Tensor:
 #                                 rows of a (B,H,row_capacity,d) buffer (a cache buffer)
 #   castle_hip::rms_norm          rows, weight -> (normalised rows, their factors): the norm of a layer that is traced
 #   castle_hip::linear            rows, weight -> rows weight^T: its projections
-#   castle_hip::attention_bwd / attention_packed_bwd / rms_norm_bwd / linear_bwd   their backward passes
+#   castle_hip::attention_bwd / attention_packed_bwd / rms_norm_bwd / linear_bwd   their backward passes (of the last
+#                                 two: a gradient that is not asked for comes back empty)
 # `U` is an empty tensor when the lookahead keys are not asked for.  The workspace output is what
 # the backward pass needs back (operand copies, log-sum-exp), the state output the snapshots (empty
 # when they are not kept); they carry no gradient.
@@ -151,16 +152,21 @@ def _fake_rms_norm(x, weight, eps):
     return torch.empty(x.shape, dtype=x.dtype, device=x.device), torch.empty((rows,) if native else (rows, 1), dtype=torch.float32, device=x.device)
 
 
-def _fake_rms_norm_bwd(dh, x, rstd, weight):
-    return torch.empty(x.shape, dtype=x.dtype, device=x.device), torch.empty_like(weight)
+def _fake_gradients(x, weight, need_x, need_w):
+    return (torch.empty(x.shape if need_x else (0,), dtype=x.dtype, device=x.device),
+            torch.empty(weight.shape if need_w else (0,), dtype=weight.dtype, device=weight.device))
+
+
+def _fake_rms_norm_bwd(dh, x, rstd, weight, need_x=True, need_w=True):
+    return _fake_gradients(x, weight, need_x, need_w)
 
 
 def _fake_linear(x, weight):
     return torch.empty((*x.shape[:-1], weight.shape[0]), dtype=x.dtype, device=x.device)
 
 
-def _fake_linear_bwd(dy, x, weight):
-    return torch.empty(x.shape, dtype=x.dtype, device=x.device), torch.empty_like(weight)
+def _fake_linear_bwd(dy, x, weight, need_x=True, need_w=True):
+    return _fake_gradients(x, weight, need_x, need_w)
 
 
 def _register_fakes():

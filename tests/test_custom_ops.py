@@ -69,6 +69,31 @@ def test_second_derivatives_of_the_operators_raise():
         assert not torch.autograd.grad(y.sum(), x)[0].requires_grad
 
 
+def test_frozen_weights_cost_no_gradient_of_theirs():
+    """The traced norm and projections form the gradients that are asked for, as the modules do."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    asked = {}
+
+    class Record(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func.namespace == "castle_hip" and func._opname.endswith("_bwd"):
+                asked[func._opname] = [a for a in args if isinstance(a, bool)]
+            return func(*args, **(kwargs or {}))
+
+    with FakeTensorMode(), Record():
+        for of_x in (False, True):
+            for of_w in (False, True):
+                if of_x or of_w:
+                    x, w, nw = (torch.empty(*s, requires_grad=r) for s, r in (((2, 40, 64), of_x), ((48, 64), of_w), ((64,), of_w)))
+                    asked.clear()
+                    (torch.ops.castle_hip.linear(x, w).sum() + torch.ops.castle_hip.rms_norm(x, nw, None)[0].sum()).backward()
+                    for name in ("linear_bwd", "rms_norm_bwd"):   # (trailing arguments at their default are not among `args`)
+                        assert (asked[name] + [True, True])[:2] == [of_x, of_w]
+                    assert [t.grad is not None for t in (x, w, nw)] == [of_x, of_w, of_w]
+                    assert all(t.grad is None or t.grad.shape == t.shape for t in (x, w, nw))
+
+
 def test_fake_tensor_trace_of_the_module():
     """Castle.forward traces without a GPU: projection -> registered operator -> output projection,
     forward and backward, for the parallel pass with and without the cache."""
@@ -116,3 +141,23 @@ def test_compiled_module_equals_eager_on_the_gpu():
     assert torch.equal(yc, y)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_compiled_module_with_frozen_weights_equals_eager_on_the_gpu():
+    torch.manual_seed(0)
+    m = Castle(64, heads=2, dim_head=32, use_triton=True, prenorm=True).to("cuda")
+    x = torch.randn(2, 70, 64, device="cuda", requires_grad=True)
+    for frozen in (m.to_all_qkv.weight, m.combine_heads.weight, m.norm.weight, x):
+        frozen.requires_grad_(False)
+        torch._dynamo.reset()
+        results = []
+        for f in (m, torch.compile(m, backend="aot_eager", fullgraph=True)):
+            m.zero_grad()
+            x.grad = None
+            f(x).square().sum().backward()
+            results.append([t.grad for t in (x, *m.parameters())])
+        frozen.requires_grad_(True)
+        for a, b in zip(*results):
+            assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+        assert sum(a is None for a in results[0]) == 1
