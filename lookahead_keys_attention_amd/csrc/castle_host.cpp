@@ -7,6 +7,7 @@
 // 150 us more for a backward pass, a cached step 71 us; here an operator costs its allocations and launches.
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -925,6 +926,7 @@ class StepPlan {
     castle_deferred def = deferred(base, base_device);
     const castle_deferred* pd = base >= 0 || base_device ? &def : nullptr;
     const int flags = flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0);
+    used_on_current_stream();
     void* ws = workspace_.data_ptr();
     const int64_t wb = workspace_.numel();
     check(t_device ? castle_decode_step_device_count(c, c + 1, c + 2, c + 3, count_ptr(t_device), s_.L, &v[0], &v[1], &v[2], &v[3], &v[4], &v[5],
@@ -960,6 +962,7 @@ class StepPlan {
     const double e = eps ? *eps : x.scalar_type() == at::kHalf ? 0.0009765625 : x.scalar_type() == at::kBFloat16 ? 0.0078125 : 1.1920928955078125e-07;
     // the projection is scratch of the step like the workspace: kept with it, an allocation costs more than a microsecond
     if (!proj_.defined()) proj_ = at::empty({B, 6 * inner}, x.options().requires_grad(false));
+    used_on_current_stream();
     Tensor y = at::empty({B, 1, dim}, x.options());
     const castle_view4* c = views_;
     castle_deferred def = deferred(base, base_device);
@@ -973,6 +976,17 @@ class StepPlan {
   }
 
  private:
+  // What the steps work on was allocated on the stream of the prompt or of the first step; the allocator has to know of every other
+  // stream that uses it, or it hands the memory of a dropped cache out again before a step on that stream is through.
+  void used_on_current_stream() {
+    const c10::Stream stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(buffers_[0].get_device()).unwrap();
+    if (stream_ && *stream_ == stream && recorded_proj_ == proj_.defined()) return;
+    for (const Tensor& t : buffers_) t.record_stream(stream);
+    for (const Tensor* t : {&ring_, &gates_, &workspace_, &proj_})
+      if (t->defined()) t->record_stream(stream);
+    stream_ = stream;
+    recorded_proj_ = proj_.defined();
+  }
   static const int32_t* count_ptr(const std::optional<Tensor>& t) { return static_cast<const int32_t*>(t->data_ptr()); }
   void check_count(int64_t t, const std::optional<Tensor>& t_device) const {
     if (t_device) {
@@ -991,6 +1005,8 @@ class StepPlan {
 
   std::vector<Tensor> buffers_;
   Tensor ring_, gates_, workspace_, proj_;
+  std::optional<c10::Stream> stream_;   // of the last step
+  bool recorded_proj_ = false;
   castle_view4 views_[4];
   castle_deferred deferred_;
   Shape s_;

@@ -249,6 +249,35 @@ def test_replaced_forward_and_traced_hooks_run(name):
         assert (y - y2).norm() <= 1e-5 * y2.norm() and (step - m(x[:, :1], cache=cache)[0]).norm() <= 1e-5 * step.norm()
 
 
+def test_memory_of_a_dropped_cache_waits_for_a_step_on_another_stream():
+    m = make(256, 4, 64, dtype=torch.bfloat16).eval()
+    x = torch.randn(2, 70, 256, device=DEV).bfloat16()
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        _, cache = m(x, return_next_cache=True)
+        _, cache = m(x[:, :1], cache=cache)   # the step's scratch is allocated here
+        want, _ = m(x[:, 1:2], cache=m(x[:, :1], cache=m(x, return_next_cache=True)[1])[1])
+        store = cache._store
+        kept = [*store.buffers, *store.rings, store.workspace]
+        taken = {t.data_ptr() for t in kept}
+        sizes = [t.numel() * t.element_size() for t in kept]
+        projection = 2 * 6 * 4 * 64 * 2
+        torch.cuda.synchronize()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(20_000_000)   # (cycles of a clock of 100 MHz)
+            got, cache = m(x[:, 1:2], cache=cache)
+        del cache, store, kept
+        fresh = [torch.empty(n, dtype=torch.uint8, device=DEV) for n in sizes]
+        stats = torch.cuda.memory_stats()
+        busy = not side.query()
+        pending = stats["active_bytes.all.current"] - stats["allocated_bytes.all.current"]
+    assert busy, "the step on the other stream was through before the check"
+    assert not taken & {t.data_ptr() for t in fresh} and pending >= sum(sizes) + projection
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
 def test_multi_token_with_cache_is_rejected():
     m = make(32, 2, 16)
     x = torch.randn(1, 4, 32).to(DEV)
