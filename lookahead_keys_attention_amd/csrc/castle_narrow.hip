@@ -220,7 +220,10 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
     }
     for (int jt = first; jt < last; ++jt) {
       const int I = jt >> 1;
-      if (keep && I > Kb && (jt == first || !(jt & 1))) store_snap_tile<T, HD, NT>(snap + (usnap_off(I) + kw0) * HD, st, c, g);
+      if (keep && I > Kb && (jt == first || !(jt & 1))) {
+        settle();
+        store_snap_tile<T, HD, NT>(snap + (usnap_off(I) + kw0) * HD, st, c, g);
+      }
       wave_lds_order<>();
       pk.store(s_ku);
       pv.store(s_vu);
@@ -250,6 +253,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
   if (seg < nblk - Kb) {   // more than one part: the sums of the parts in front of this wave's
     if (hi < nblk) sweep(false);
     float* red = reinterpret_cast<float*>(castle_smem);
+    settle();
     __syncthreads();   // the tiles are dead
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -269,6 +273,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
   }
   if (lo >= hi) return;
   sweep(true);
+  settle();
   if (hi == nblk && a.U.ptr != nullptr && k < L) {
     TI* dst = head_ptr_mut<TI>(a.U, b, h) + (int64_t)k * a.U.sl;
     const float su_mul = a.ws.hdr->su_mul;   // the state was built from vu * vu_scale
@@ -466,6 +471,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void attn_narrow_k
     lt += mw == -INFINITY ? 0.f : fast_exp2(mw - M) * s_stat[(w * 64 + lane) * 2 + 1];
   }
   const float wt = m == -INFINITY ? 0.f : fast_exp2(m - M) / lt;
+  settle();
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
