@@ -246,8 +246,9 @@ class _ManyRowLinear(torch.autograd.Function):
 def _unmodified(module, kind) -> bool:
     """True for a module of exactly this kind that runs its class's forward and nothing else: nothing hooked onto it, no
     `forward` of its own (offloading, adapters and quantisation wrappers replace it on the instance)."""
-    return type(module) is kind and "forward" not in module.__dict__ and not (
-        module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+    own = module.__dict__
+    return type(module) is kind and not ("forward" in own or own["_forward_hooks"] or own["_forward_pre_hooks"]
+                                         or own["_backward_hooks"] or own["_backward_pre_hooks"])
 
 
 def _linear(layer, t):
