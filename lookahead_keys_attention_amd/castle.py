@@ -209,19 +209,14 @@ class _CacheStore:
         self.length = self.base0 = t
 
 
-# The weight gradient of a projection over many rows, dW = dY^T x, is a product with a small
-# output (out_features x in_features) and a long contraction (the rows): the GEMM the library picks
-# leaves most of the GPU idle there (one tile per output block walking all rows serially).  Above this
-# row count it is formed as SPLIT_ROWS_INTO partial products over row ranges (one batched GEMM with
-# fp32 partial results, then their sum): same rounding as the single product (fp32 accumulation, one
-# rounding at the end), 2-3 times faster at 16384 rows.
+# From this many rows on the weight gradient of a projection is formed like a whole layer's (weight_grad in
+# csrc/castle_host.cpp: as partial products over row ranges where the output alone would leave the GPU idle).
 SPLIT_WGRAD_MIN_ROWS = 8192
-SPLIT_ROWS_INTO = 8
 
 
 class _ManyRowLinear(torch.autograd.Function):
     """x @ weight.T (the bias-free nn.Linear of lookahead_keys_attention.py:75, 80) whose backward forms
-    the weight gradient in row ranges; forward and input gradient are the library GEMMs."""
+    the weight gradient by the rule of a whole layer; forward and input gradient are the library GEMMs."""
 
     @staticmethod
     def forward(ctx, x, weight):
@@ -236,10 +231,8 @@ class _ManyRowLinear(torch.autograd.Function):
             dx = dy @ weight
         if ctx.needs_input_grad[1]:
             x2, dy2 = x.reshape(-1, x.shape[-1]), dy.reshape(-1, dy.shape[-1])
-            rows, parts = x2.shape[0], SPLIT_ROWS_INTO
-            partial = torch.bmm(dy2.view(parts, rows // parts, -1).transpose(1, 2), x2.view(parts, rows // parts, -1),
-                                out_dtype=torch.float32)
-            dw = partial.sum(0).to(weight.dtype)
+            # (a graph of the backward pass wants operators that have derivatives)
+            dw = dy2.t() @ x2 if torch.is_grad_enabled() else _native.host().weight_grad(dy2, x2)
         return dx, dw
 
 
@@ -255,7 +248,7 @@ def _linear(layer, t):
     """layer(t) for a bias-free nn.Linear, through _ManyRowLinear where its weight gradient pays."""
     rows = t.numel() // t.shape[-1] if t.shape[-1] else 0
     if (t.is_cuda and _unmodified(layer, nn.Linear) and layer.bias is None and t.dtype in (torch.bfloat16, torch.float16) and layer.weight.dtype == t.dtype
-            and rows >= SPLIT_WGRAD_MIN_ROWS and rows % SPLIT_ROWS_INTO == 0 and t.is_contiguous()
+            and rows >= SPLIT_WGRAD_MIN_ROWS and t.is_contiguous()
             and torch.is_grad_enabled() and layer.weight.requires_grad):
         return _ManyRowLinear.apply(t, layer.weight)
     return layer(t)

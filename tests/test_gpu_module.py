@@ -183,6 +183,30 @@ def test_projection_over_many_rows_forms_its_weight_gradient_in_row_ranges():
         assert C._linear(layer, x).grad_fn is None
 
 
+# outputs of 8, 4, 2 ranges and of one product; rows that do not divide
+@pytest.mark.parametrize("rows,n,k", [(8192, 1536, 256), (8192, 2048, 2048), (8192, 6144, 1024), (8192, 6144, 2048), (8203, 512, 512)])
+def test_a_hooked_layer_forms_its_weight_gradients_like_a_plain_one(rows, n, k):
+    from lookahead_keys_attention_amd import _native, castle as C
+
+    torch.manual_seed(6)
+    layer = torch.nn.Linear(k, n, bias=False).to(DEV).bfloat16()
+    x = torch.randn(1, rows, k, device=DEV).bfloat16()
+    gy = torch.randn(1, rows, n, device=DEV).bfloat16()
+    y = C._linear(layer, x)
+    assert "ManyRowLinear" in type(y.grad_fn).__name__
+    y.backward(gy)
+    assert torch.equal(layer.weight.grad, _native.host().weight_grad(gy[0], x[0]))
+    ref = gy[0].float().t() @ x[0].float()
+    assert (layer.weight.grad.float() - ref).norm() <= 4e-3 * ref.norm()   # one rounding to bf16
+    handle = layer.register_forward_hook(lambda *_: None)   # on the projection itself: the module runs
+    assert "ManyRowLinear" not in type(C._linear(layer, x).grad_fn).__name__
+    handle.remove()
+    # with a graph of the backward pass the gradient has derivatives
+    leaf = x[:, :, :].clone().requires_grad_()
+    dw, = torch.autograd.grad(C._linear(layer, leaf).sum(), layer.weight, create_graph=True)
+    assert torch.autograd.grad(dw.sum(), leaf)[0].eq(n).all()
+
+
 @pytest.mark.parametrize("prenorm", [False, True])
 def test_input_changed_in_place_before_the_backward_pass(prenorm):
     """A layer's input is read by its backward pass: one that was changed in place is an error, as for the modules
