@@ -958,8 +958,7 @@ class StepPlan {
     const Tensor xr = rows_readable(x.select(1, 0)) ? x : x.contiguous();
     const Tensor nw = norm_w ? norm_w->contiguous() : Tensor();
     const Tensor res = residual ? (residual->stride(2) == 1 ? *residual : residual->contiguous()) : Tensor();
-    // the step's own default: the type's machine epsilon
-    const double e = eps ? *eps : x.scalar_type() == at::kHalf ? 0.0009765625 : x.scalar_type() == at::kBFloat16 ? 0.0078125 : 1.1920928955078125e-07;
+    const double e = norm_eps(eps);
     // the projection is scratch of the step like the workspace: kept with it, an allocation costs more than a microsecond
     if (!proj_.defined()) proj_ = at::empty({B, 6 * inner}, x.options().requires_grad(false));
     used_on_current_stream();

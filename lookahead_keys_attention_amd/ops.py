@@ -305,7 +305,7 @@ def small_linear(x: torch.Tensor, weight: torch.Tensor, norm=None, activation=No
     norm_weight, eps = None, 0.0
     if norm is not None:
         norm_weight = norm.weight
-        eps = norm.eps if norm.eps is not None else torch.finfo(x.dtype).eps   # what F.rms_norm uses for eps=None
+        eps = norm.eps if norm.eps is not None else torch.finfo(torch.float32).eps   # of the 32-bit sums, as F.rms_norm does
         if norm_weight.dtype != x.dtype or norm_weight.numel() != K or not norm_weight.is_contiguous():
             raise ValueError("small_linear: the norm weight must be a contiguous (K,) tensor of the input type")
     if activation not in (None, "gelu"):

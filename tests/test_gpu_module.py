@@ -234,6 +234,27 @@ def test_input_changed_in_place_before_the_backward_pass(prenorm):
         assert torch.equal(torch.autograd.grad(y.sum(), leaf)[0], want)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2e-2), (torch.float16, 4e-3)])
+def test_step_and_parallel_pass_normalise_small_rows_alike(dtype, tol):
+    """A norm without an eps of its own adds that of the 32-bit sums, whatever the type of the rows: with rows of 0.05 the
+    type's epsilon would be three times their mean square.  (Tolerance: the types' roundings, as for the other steps.)"""
+    from lookahead_keys_attention_amd import CastleLM
+
+    m = make(128, 2, 64, dtype=dtype, prenorm=True).eval()
+    x = torch.randn(2, 40, 128, generator=torch.Generator().manual_seed(8)).to(DEV).to(dtype)
+    ids = torch.randint(0, 64, (2, 40), generator=torch.Generator().manual_seed(9)).to(DEV)
+    lm = CastleLM(num_tokens=64, dim=128, depth=2, dim_head=64, heads=2).to(DEV).to(dtype).eval()
+    with torch.no_grad():
+        lm.token_emb.weight.mul_(0.02)
+        for p in (lm.layers[0][0].combine_heads, lm.layers[0][1][3], lm.layers[1][0].combine_heads, lm.layers[1][1][3]):
+            p.weight.mul_(0.02)   # the residual stream stays small
+        for model, rows in ((m, x), (m, x * 0.05), (lm, ids)):
+            want = model(rows)[:, -1]
+            _, cache = model(rows[:, :39], return_next_cache=True)
+            got = model(rows[:, 39:], cache=cache, return_next_cache=True)[0][:, 0]
+            assert (got - want).double().norm() <= tol * want.double().norm()
+
+
 @pytest.mark.parametrize("prenorm", [False, True])
 def test_second_derivatives_of_a_layer_raise(prenorm):
     m = make(64, 2, 32, prenorm=prenorm)

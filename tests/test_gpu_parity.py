@@ -420,7 +420,7 @@ def test_small_linear_matches_fp64_matmul(M, N, K, dtype):
 def test_small_linear_with_norm_activation_and_residual(M, N, K, dtype, norm, act, res):
     """castle_small_linear_fused: RMS normalisation in front, erf GELU and a residual behind, in one
     launch, against the same chain in fp64 on the same 16-bit values (nn.RMSNorm with eps=None takes
-    the type's machine epsilon; the norm weight multiplies the normalised row)."""
+    the machine epsilon of its 32-bit sums; the norm weight multiplies the normalised row)."""
     g = torch.Generator().manual_seed(M + N + K)
     x = (torch.randn(M, 1, K, generator=g) * 1.7).to(dtype).to(DEV)
     w = (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype).to(DEV)
@@ -432,7 +432,7 @@ def test_small_linear_with_norm_activation_and_residual(M, N, K, dtype, norm, ac
     y = H().small_linear(x, w, norm=layer, activation=act, residual=r)
     ref = x.double()
     if norm:
-        eps = torch.finfo(dtype).eps
+        eps = torch.finfo(torch.float32).eps
         ref = ref * torch.rsqrt(ref.pow(2).mean(-1, keepdim=True) + eps) * layer.weight.double()
     ref = ref @ w.double().T
     if act == "gelu":
