@@ -61,6 +61,11 @@ Tensor packed_readable(const Tensor& t) {
   return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.contiguous();
 }
 
+// The kernels have no formula for a tangent (forward-mode derivatives); a result without one would stand for a derivative of zero.
+void no_tangent(const Tensor& t) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!t._fw_grad(0).defined(), "the CASTLE kernels have no forward-mode derivatives (Castle(use_triton=False) has)");
+}
+
 Tensor bytes(int64_t n, const Tensor& like) { return at::empty({n}, like.options().dtype(at::kByte)); }
 
 struct Shape {
@@ -203,11 +208,15 @@ Tensor attention_packed_bwd(const Tensor& proj, const Tensor& merged, const Tens
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
+// Whether a call records a graph.
 bool wants_graph(std::initializer_list<Tensor> ts) {
-  if (!at::GradMode::is_enabled()) return false;
-  for (const Tensor& t : ts)
-    if (t.defined() && t.requires_grad()) return true;
-  return false;
+  bool graph = false;
+  for (const Tensor& t : ts) {
+    if (!t.defined()) continue;
+    no_tangent(t);
+    graph = graph || t.requires_grad();
+  }
+  return graph && at::GradMode::is_enabled();
 }
 
 // The gradients have no derivatives of their own.  Where a graph of the backward pass is recorded (create_graph) they hang on a
@@ -260,7 +269,7 @@ struct AttentionFn : torch::autograd::Function<AttentionFn> {
 Tensor attention_bwd_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu, const Tensor& ku, const Tensor& vu,
                               const Tensor& out, const Tensor& dout, const Tensor& ws, const Tensor& state, double scale, int64_t flags) {
   static const auto op = op_handle<decltype(attention_bwd)>("castle_hip::attention_bwd");
-  const bool graph = at::GradMode::is_enabled() && wants_graph({q, k, v, qu, ku, vu, out, dout});
+  const bool graph = wants_graph({q, k, v, qu, ku, vu, out, dout});
   const at::AutoDispatchBelowADInplaceOrView below;
   const Tensor d = op.call(q, k, v, qu, ku, vu, out, dout, ws, state, scale, flags);
   return graph ? no_second_derivatives({d})[0] : d;
@@ -305,7 +314,7 @@ struct AttentionPackedFn : torch::autograd::Function<AttentionPackedFn> {
 Tensor attention_packed_bwd_autograd(const Tensor& proj, const Tensor& merged, const Tensor& dmerged, const Tensor& ws, const Tensor& state,
                                      int64_t heads, double scale, int64_t flags) {
   static const auto op = op_handle<decltype(attention_packed_bwd)>("castle_hip::attention_packed_bwd");
-  const bool graph = at::GradMode::is_enabled() && wants_graph({proj, merged, dmerged});
+  const bool graph = wants_graph({proj, merged, dmerged});
   const at::AutoDispatchBelowADInplaceOrView below;
   const Tensor d = op.call(proj, merged, dmerged, ws, state, heads, scale, flags);
   return graph ? no_second_derivatives({d})[0] : d;
@@ -409,7 +418,7 @@ struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
 };
 std::tuple<Tensor, Tensor> rms_norm_bwd_autograd(const Tensor& dh, const Tensor& x, const Tensor& rstd, const Tensor& weight, bool need_x, bool need_w) {
   static const auto op = op_handle<decltype(rms_norm_bwd_op)>("castle_hip::rms_norm_bwd");
-  const bool graph = at::GradMode::is_enabled() && wants_graph({dh, x, weight});
+  const bool graph = wants_graph({dh, x, weight});
   const at::AutoDispatchBelowADInplaceOrView below;
   const auto [dx, dw] = op.call(dh, x, rstd, weight, need_x, need_w);
   if (!graph) return {dx, dw};
@@ -549,7 +558,7 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
 };
 std::tuple<Tensor, Tensor> linear_bwd_autograd(const Tensor& dy, const Tensor& x, const Tensor& weight, bool need_x, bool need_w) {
   static const auto op = op_handle<decltype(linear_bwd_op)>("castle_hip::linear_bwd");
-  const bool graph = at::GradMode::is_enabled() && wants_graph({dy, x, weight});
+  const bool graph = wants_graph({dy, x, weight});
   const at::AutoDispatchBelowADInplaceOrView below;
   const auto [dx, dw] = op.call(dy, x, weight, need_x, need_w);
   if (!graph) return {dx, dw};
@@ -858,6 +867,7 @@ bool rows_readable(const Tensor& t) {
 Tensor small_linear(const Tensor& x, const Tensor& w, const std::optional<Tensor>& norm_w, double eps, int64_t act,
                     const std::optional<Tensor>& residual) {
   const c10::DeviceGuard guard(x.device());
+  no_tangent(x);
   const int64_t B = x.size(0), N = w.size(0);
   Tensor y = at::empty({B, 1, N}, x.options());
   check(castle_small_linear_fused(x.data_ptr(), w.data_ptr(), y.data_ptr(), (int)B, (int)N, (int)x.size(2), x.stride(0), w.stride(0), N,
@@ -912,6 +922,7 @@ class StepPlan {
   Tensor attend(const Tensor& proj_, int64_t t, int64_t base, double scale, bool rotary, const std::optional<Tensor>& t_device,
                 const std::optional<Tensor>& base_device) {
     check_count(t, t_device);
+    no_tangent(proj_);
     const Tensor proj = packed_readable(proj_);
     TORCH_CHECK_VALUE(proj.dim() == 3 && proj.size(0) == s_.B && proj.size(1) == 1 && proj.size(2) == 6LL * s_.H * s_.d &&
                           proj.scalar_type() == buffers_[0].scalar_type() && proj.device() == buffers_[0].device(),
@@ -947,6 +958,7 @@ class StepPlan {
     const int64_t B = s_.B, dim = x.size(-1), inner = (int64_t)s_.H * s_.d;
     const c10::DeviceGuard guard(x.device());
     check_count(t, t_device);
+    no_tangent(x);
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(0) == B && x.size(1) == 1 && w_qkv.dim() == 2 && w_qkv.size(0) == 6 * inner && w_qkv.size(1) == dim &&
                           w_out.dim() == 2 && w_out.size(1) == inner && x.scalar_type() == buffers_[0].scalar_type() && x.device() == buffers_[0].device(),
                       "the token or the weights do not belong to this cache");

@@ -69,6 +69,25 @@ def test_second_derivatives_of_the_operators_raise():
         assert not torch.autograd.grad(y.sum(), x)[0].requires_grad
 
 
+def test_forward_mode_derivatives_raise():
+    """Without a gradient to record as with one: a result without its tangent would claim a derivative of zero."""
+    from torch.autograd import forward_ad
+
+    with FakeTensorMode(), forward_ad.dual_level():
+        for recorded in (False, True):
+            def dual(*shape):
+                t = torch.empty(*shape, requires_grad=recorded)
+                return forward_ad.make_dual(t, torch.empty(*shape))
+
+            plain = [torch.empty(2, 2, 40, 32) for _ in range(5)]
+            for call in (lambda: ops.castle_attention_hip(*plain, dual(2, 2, 40, 32), 0.125),
+                         lambda: ops.castle_attention_packed(dual(2, 40, 6 * 2 * 32), 2, 0.125),
+                         lambda: torch.ops.castle_hip.rms_norm(dual(2, 40, 64), torch.empty(64), None),
+                         lambda: torch.ops.castle_hip.linear(torch.empty(2, 40, 64), dual(48, 64))):
+                with pytest.raises(NotImplementedError, match="forward-mode"):
+                    call()
+
+
 def test_frozen_weights_cost_no_gradient_of_theirs():
     """The traced norm and projections form the gradients that are asked for, as the modules do."""
     from torch.utils._python_dispatch import TorchDispatchMode

@@ -323,6 +323,16 @@ def test_memory_of_a_dropped_cache_waits_for_a_step_on_another_stream():
     assert torch.equal(got, want)
 
 
+def test_forward_mode_derivatives_of_a_layer_raise():
+    from torch.autograd import forward_ad
+
+    m = make(64, 2, 32).requires_grad_(False)
+    x = torch.randn(2, 40, 64, device=DEV)
+    for rows in (x, x[:, :1]):   # the parallel pass, a cached step
+        with forward_ad.dual_level(), pytest.raises(NotImplementedError, match="forward-mode"):
+            m(forward_ad.make_dual(rows, torch.ones_like(rows)))
+
+
 def test_multi_token_with_cache_is_rejected():
     m = make(32, 2, 16)
     x = torch.randn(1, 4, 32).to(DEV)
