@@ -118,6 +118,8 @@ class GraphedDecoder:
         stores = [getattr(c, "_store", None) for c in caches]
         if len(stores) != len(model.layers) or any(st is None for st in stores):
             raise RuntimeError("GraphedDecoder needs the native caches of every layer (use_triton=True on a GPU)")
+        if not all(_unmodified(attention, Castle) for attention, _ in model.layers):
+            raise RuntimeError("GraphedDecoder captures the attention layers' own step: hooks or a `forward` set on them would not run")
         lengths = {st.length for st in stores}
         if len(lengths) != 1:
             raise RuntimeError("the layer caches disagree about their length")
@@ -157,15 +159,14 @@ class GraphedDecoder:
         self.counters.copy_(torch.tensor([self.length, self.base0], dtype=torch.int32), non_blocking=False)
 
     def _signature(self):
-        """What the captured graph has baked in: the addresses of the weights it reads.  None (never the same again) for a
-        model with modules that run something of their own."""
-        return tuple(p.data_ptr() for p in self.model.parameters()) if self.model._unmodified() else None
+        """What the captured graph has baked in: the addresses of the weights it reads."""
+        return tuple(p.data_ptr() for p in self.model.parameters())
 
     def fits(self, caches, max_len: int) -> bool:
         """True if `load(caches)` can reuse this graph for a generation of up to max_len rows."""
         first = getattr(caches[0], "_store", None)
         mine = self.stores[0].buffers[0]
-        return (first is not None and max_len <= self.capacity and self.signature is not None and self.signature == self._signature()
+        return (first is not None and max_len <= self.capacity and self.signature == self._signature()
                 and first.buffers[0].shape[:2] == mine.shape[:2] and first.buffers[0].shape[3] == mine.shape[3]
                 and first.buffers[0].dtype == mine.dtype and first.buffers[0].device == mine.device
                 and first.u_half == self.stores[0].u_half)
@@ -313,15 +314,17 @@ class CastleLM(nn.Module):
             return host.cross_entropy(logits, target)
         return (logits, next_cache) if return_next_cache else logits
 
-    def _decoder_for(self, cache, max_len):
+    def _decoder_for(self, cache, max_len, keep=True):
         """A GraphedDecoder positioned on `cache`: the one kept from an earlier call when its graph
-        still fits (same weights, batch, type; enough rows), else a newly captured one."""
+        still fits (same weights, batch, type; enough rows), else a newly captured one.  keep=False: captured for this
+        call alone (what hooks or a replaced `forward` did meanwhile is not for other calls)."""
         kept = self.__dict__.get("_kept_decoder")
-        if kept is not None and kept.fits(cache, max_len):
+        if keep and kept is not None and kept.fits(cache, max_len):
             kept.load(cache)
             return kept
         decoder = GraphedDecoder(self, cache, max_len)
-        self.__dict__["_kept_decoder"] = decoder   # not a module attribute: never part of the state
+        if keep:
+            self.__dict__["_kept_decoder"] = decoder   # not a module attribute: never part of the state
         return decoder
 
     def release_decoder(self):
@@ -330,7 +333,12 @@ class CastleLM(nn.Module):
 
     def _unmodified(self) -> bool:
         """True if a replayed graph of a token step does what a call of every module would: no hooks, no replaced `forward`."""
-        return all(_unmodified(module, type(module)) for module in self.modules())
+        modules = [self]
+        for module in modules:   # (a shared module twice is no harm; `self.modules()` takes three times as long)
+            if not _unmodified(module, type(module)):
+                return False
+            modules += [child for child in module._modules.values() if child is not None]
+        return True
 
     def _native_on_gpu(self, device) -> bool:
         return device.type == "cuda" and _native.is_built() and all(attention.use_triton for attention, _ in self.layers)
@@ -345,13 +353,10 @@ class CastleLM(nn.Module):
         run) and more than a few steps follow; True insists."""
         prompt_len = prompt.shape[-1]
         steps = max(0, seq_len - prompt_len)
-        if graph is None:
-            graph = self._native_on_gpu(prompt.device) and steps > 8 and self._unmodified()
-        elif graph and not self._native_on_gpu(prompt.device):
-            raise RuntimeError("graph=True needs the native kernels on a GPU")
-
         if self._native_on_gpu(prompt.device):
             return self._sample_native(prompt, steps, seq_len, temperature, filter_thres, generator, graph)
+        if graph:
+            raise RuntimeError("graph=True needs the native kernels on a GPU")
 
         out, cache = prompt, None
         for _ in range(steps):
@@ -371,8 +376,10 @@ class CastleLM(nn.Module):
                 logits = decoder.step(decoder.token)
             else:
                 logits, cache = self.forward(prompt if cache is None else tokens[:, i - 1:i], cache=cache, return_next_cache=True)
-                if graph:
-                    decoder = self._decoder_for(cache, seq_len)
+                if i == 0 and (graph or graph is None and steps > 8):   # (looked into while the GPU works on the prompt)
+                    unmodified = self._unmodified()
+                    if unmodified or graph:
+                        decoder = self._decoder_for(cache, seq_len, unmodified)
             if logits.shape[-1] > SAMPLER_MAX_VOCABULARY:
                 tokens[:, i:i + 1] = pick_token(logits, temperature, filter_thres, generator)
                 if decoder is not None:

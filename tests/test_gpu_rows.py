@@ -167,7 +167,16 @@ def test_replaced_forward_in_a_language_model_runs():
         assert len(calls) == 1
         model.sample(ids[:, :6], 6 + 12)   # a prompt, eleven steps
         assert len(calls) == 1 + 12
+        kept = model.__dict__.get("_kept_decoder")
+        if module is attention:
+            with pytest.raises(RuntimeError, match="would not run"):
+                model.sample(ids[:, :6], 6 + 12, graph=True)
+        else:   # insisted on: what the module does is captured, for this call
+            model.sample(ids[:, :6], 6 + 12, graph=True)
+            assert len(calls) > 1 + 12 and model.__dict__.get("_kept_decoder") is kept
         del module.forward
+        model.sample(ids[:, :6], 6 + 12)
+        assert model._kept_decoder is not None and (kept is None or model._kept_decoder is kept)
 
 
 def test_second_derivatives_of_the_language_model_blocks_raise():
