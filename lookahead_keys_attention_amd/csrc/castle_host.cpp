@@ -7,7 +7,7 @@
 // 150 us more for a backward pass, a cached step 71 us; here an operator costs its allocations and launches.
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
-#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -990,11 +990,14 @@ class StepPlan {
   // What the steps work on was allocated on the stream of the prompt or of the first step; the allocator has to know of every other
   // stream that uses it, or it hands the memory of a dropped cache out again before a step on that stream is through.
   void used_on_current_stream() {
-    const c10::Stream stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(buffers_[0].get_device()).unwrap();
+    const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(buffers_[0].get_device());
     if (stream_ && *stream_ == stream && recorded_proj_ == proj_.defined()) return;
-    for (const Tensor& t : buffers_) t.record_stream(stream);
-    for (const Tensor* t : {&ring_, &gates_, &workspace_, &proj_})
-      if (t->defined()) t->record_stream(stream);
+    // (straight to the allocator: record_stream costs a microsecond a tensor)
+    auto record = [&](const Tensor& t) {
+      if (t.defined()) c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::recordStreamMasqueradingAsCUDA(t.storage().data_ptr(), stream);
+    };
+    for (const Tensor& t : buffers_) record(t);
+    for (const Tensor* t : {&ring_, &gates_, &workspace_, &proj_}) record(*t);
     stream_ = stream;
     recorded_proj_ = proj_.defined();
   }
@@ -1016,7 +1019,7 @@ class StepPlan {
 
   std::vector<Tensor> buffers_;
   Tensor ring_, gates_, workspace_, proj_;
-  std::optional<c10::Stream> stream_;   // of the last step
+  std::optional<c10::hip::HIPStreamMasqueradingAsCUDA> stream_;   // of the last step
   bool recorded_proj_ = false;
   castle_view4 views_[4];
   castle_deferred deferred_;
