@@ -332,7 +332,7 @@ class Castle(nn.Module):
 
     # -- forward ------------------------------------------------------------
     def forward(self, x, cache=None, return_next_cache=None):
-        n = x.shape[1]
+        n = x.size(1)
         single = n == 1
         if return_next_cache is None:
             return_next_cache = single
@@ -399,20 +399,27 @@ class Castle(nn.Module):
         if (torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda") or torch._C._are_functorch_transforms_active()
                 or torch._C._len_torch_dispatch_stack()):
             return False
-        modules, dtype, device, dim = self._modules, x.dtype, x.device, x.shape[2]
+        modules, dtype, device, dim = self._modules, x.dtype, x.device, x.size(2)
         norm, qkv, combine = modules["norm"], modules["to_all_qkv"], modules["combine_heads"]
-        if _unmodified(norm, nn.RMSNorm):
-            weight = norm._parameters["weight"]
-            if type(weight) is not nn.Parameter or weight.dtype is not dtype or weight.device != device or norm.normalized_shape != (dim,):
+        kind = type(norm)
+        if kind is nn.RMSNorm:
+            if norm.normalized_shape != (dim,):
                 return False
-        elif not _unmodified(norm, nn.Identity):
+        elif kind is not nn.Identity:
             return False
-        if not (_unmodified(qkv, nn.Linear) and _unmodified(combine, nn.Linear)) or qkv.in_features != dim:
+        if type(qkv) is not nn.Linear or type(combine) is not nn.Linear or qkv.in_features != dim:
             return False
-        for layer in (qkv, combine):
-            params = layer._parameters
+        for layer in (norm, qkv, combine):   # (`_unmodified` in line: its calls took 0.2 us)
+            own = layer.__dict__
+            if "forward" in own or own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]:
+                return False
+            params = own["_parameters"]
             weight = params.get("weight")
-            if type(weight) is not nn.Parameter or weight.dtype is not dtype or weight.device != device or params.get("bias") is not None:
+            if type(weight) is not nn.Parameter:
+                if layer is norm and kind is nn.Identity:
+                    continue
+                return False
+            if weight.dtype is not dtype or weight.device != device or params.get("bias") is not None:
                 return False
         return True
 
