@@ -236,7 +236,8 @@ template <typename F> variable_list once_differentiable(F&& gradients) {
     const at::NoGradGuard no_grad;
     grads = gradients();
   }
-  return at::GradMode::is_enabled() ? no_second_derivatives(grads) : grads;
+  if (at::GradMode::is_enabled()) return no_second_derivatives(grads);
+  return grads;
 }
 
 template <typename F> auto op_handle(const char* name) {
@@ -616,11 +617,9 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
       auto keep = [&](bool needed, const Tensor& t) { return !needed ? Tensor() : t.defined() && t.is_alias_of(x) ? x : t; };
       ctx->save_for_backward({keep(below && norm_w.defined(), n.sum), keep(below, norm_w), keep(below, w_qkv), keep(below || need_qkv, w_out),
                               keep(need_qkv, n.h), n.rstd, merged, ws, state});
-      ctx->saved_data["dim"] = dim;
       ctx->saved_data["heads"] = heads;
       ctx->saved_data["scale"] = scale;
       ctx->saved_data["flags"] = flags;
-      ctx->saved_data["delta"] = delta.has_value();
       ctx->mark_non_differentiable(variable_list(out.begin() + results, out.end()));
       ctx->set_materialize_grads(false);
     }
@@ -629,21 +628,23 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     if (g[0].defined()) return once_differentiable([&] { return gradients(ctx, g); });
     variable_list grads(12);
-    if (ctx->saved_data["delta"].toBool() && g[1].defined()) grads[0] = grads[1] = g[1];
+    if (has_delta(g) && g[1].defined()) grads[0] = grads[1] = g[1];
     return grads;
   }
+  // the results are y, the sum if there is a delta, and four cache tensors if they are asked for
+  static bool has_delta(const variable_list& g) { return g.size() % 4 == 2; }
   static variable_list gradients(AutogradContext* ctx, const variable_list& g) {
     variable_list grads(12);
-    const bool has_delta = ctx->saved_data["delta"].toBool();
+    const bool has_delta = LayerFn::has_delta(g);
     const Tensor dsum = has_delta ? g[1] : Tensor();
     const size_t nd = has_delta ? 1 : 0;   // needs_input_grad counts the tensors that were there
     const bool need_x = ctx->needs_input_grad(0) || (has_delta && ctx->needs_input_grad(1));
     const auto s = ctx->get_saved_variables();
     const Tensor &norm_w = s[1], &w_qkv = s[2], &w_out = s[3], &rstd = s[5], &merged = s[6], &ws = s[7], &state = s[8];
     const c10::DeviceGuard guard(merged.device());
-    const int64_t B = merged.size(0), L = merged.size(1), dim = ctx->saved_data["dim"].toInt(), heads = ctx->saved_data["heads"].toInt();
+    const int64_t B = merged.size(0), L = merged.size(1), heads = ctx->saved_data["heads"].toInt();
     const Tensor dy = g[0].reshape({B * L, g[0].size(2)});
-    auto rows = [&](const Tensor& t) { return t.defined() ? t.reshape({B * L, dim}) : t; };
+    auto rows = [&](const Tensor& t) { return t.defined() && t.dim() == 3 ? t.reshape({B * L, t.size(2)}) : t; };
     const size_t nn = rstd.defined() ? 1 : 0;
     const bool need_norm = nn && ctx->needs_input_grad(1 + nd), need_qkv = ctx->needs_input_grad(1 + nd + nn);
     if (ctx->needs_input_grad(2 + nd + nn)) grads[4] = weight_grad(dy, merged.view({B * L, merged.size(2)}));
@@ -669,7 +670,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     if (need_x || need_norm) {
       auto [dx, dn] = norm_rows_bwd(input_grad(dp2, w_qkv), rows(s[0]), rstd, norm_w, rows(dsum), need_x, need_norm);
       if (need_norm) grads[2] = dn;
-      if (need_x) grads[0] = dx.view({B, L, dim});
+      if (need_x) grads[0] = dx.view({B, L, dx.size(1)});
       if (has_delta) grads[1] = grads[0];
     }
     return grads;

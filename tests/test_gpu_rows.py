@@ -145,6 +145,21 @@ def test_language_model_blocks_equal_the_modules():
             assert (a - b).norm() <= 1e-4 * b.norm()
 
 
+def test_gradients_beside_caches_equal_those_without():
+    """The nodes' outputs are y, the running sum and the rows of a cache, in any combination."""
+    from lookahead_keys_attention_amd import CastleLM
+
+    torch.manual_seed(0)
+    model = CastleLM(num_tokens=64, dim=64, depth=2, heads=2, dim_head=32).to(DEV)
+    ids = torch.randint(0, 64, (2, 40), device=DEV)
+    params = [p for p in model.parameters() if p.requires_grad]
+    results = []
+    for cached in (False, True):
+        out = model(ids, return_next_cache=cached)
+        results.append(torch.autograd.grad((out[0] if cached else out).square().sum(), params))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 def test_replaced_forward_in_a_language_model_runs():
     from lookahead_keys_attention_amd import CastleLM
 
