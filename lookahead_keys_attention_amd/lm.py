@@ -64,6 +64,11 @@ def pick_token(logits, temperature, filter_thres, generator=None):
     return gumbel_sample(logits, temperature=temperature, generator=generator)
 
 
+def _runs_castle_forward(attention) -> bool:
+    """True for a `Castle`, or a subclass of it, whose call does what `Castle.forward` does and nothing else."""
+    return _unmodified(attention, type(attention)) and type(attention).forward is Castle.forward
+
+
 def _is_block(feed_forward) -> bool:
     """True if the block may be taken apart: [norm, linear, erf GELU, linear] and nothing that wants to see a call of it."""
     return _unmodified(feed_forward, nn.Sequential) and len(feed_forward) == 4 and _unmodified(feed_forward[2], nn.GELU) and feed_forward[2].approximate == "none"
@@ -118,7 +123,7 @@ class GraphedDecoder:
         stores = [getattr(c, "_store", None) for c in caches]
         if len(stores) != len(model.layers) or any(st is None for st in stores):
             raise RuntimeError("GraphedDecoder needs the native caches of every layer (use_triton=True on a GPU)")
-        if not all(_unmodified(attention, Castle) for attention, _ in model.layers):
+        if not all(_runs_castle_forward(attention) for attention, _ in model.layers):
             raise RuntimeError("GraphedDecoder captures the attention layers' own step: hooks or a `forward` set on them would not run")
         lengths = {st.length for st in stores}
         if len(lengths) != 1:
@@ -338,7 +343,7 @@ class CastleLM(nn.Module):
             if not _unmodified(module, type(module)):
                 return False
             modules += [child for child in module._modules.values() if child is not None]
-        return True
+        return all(_runs_castle_forward(attention) for attention, _ in self.layers)
 
     def _native_on_gpu(self, device) -> bool:
         return device.type == "cuda" and _native.is_built() and all(attention.use_triton for attention, _ in self.layers)

@@ -194,6 +194,32 @@ def test_replaced_forward_in_a_language_model_runs():
         assert model._kept_decoder is not None and (kept is None or model._kept_decoder is kept)
 
 
+def test_subclasses_of_the_attention_layer_in_a_sampled_model():
+    """One that leaves `forward` alone is captured like the layer itself; one that has its own is stepped."""
+    from lookahead_keys_attention_amd import Castle, CastleLM
+
+    class Named(Castle):
+        pass
+
+    class Counted(Castle):
+        calls = 0
+
+        def forward(self, *args, **kwargs):
+            Counted.calls += 1
+            return super().forward(*args, **kwargs)
+
+    torch.manual_seed(0)
+    model = CastleLM(num_tokens=64, dim=64, depth=2, heads=2, dim_head=32).to(DEV)
+    ids = torch.randint(0, 64, (2, 6), device=DEV)
+    want = model.sample(ids, 6 + 12, temperature=0)
+    for kind, kept in ((Named, True), (Counted, False)):
+        model.release_decoder()
+        model.layers[1][0].__class__ = kind
+        assert torch.equal(model.sample(ids, 6 + 12, temperature=0), want)
+        assert ("_kept_decoder" in model.__dict__) == kept
+    assert Counted.calls == 12
+
+
 def test_second_derivatives_of_the_language_model_blocks_raise():
     """Every parameter's gradient: embedding, attention, feed-forward, head and loss are nodes of their own."""
     from lookahead_keys_attention_amd import CastleLM
