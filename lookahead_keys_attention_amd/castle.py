@@ -230,9 +230,10 @@ class _ManyRowLinear(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx = dy @ weight
         if ctx.needs_input_grad[1]:
-            x2, dy2 = x.reshape(-1, x.shape[-1]), dy.reshape(-1, dy.shape[-1])
-            # (a graph of the backward pass wants operators that have derivatives)
-            dw = dy2.t() @ x2 if torch.is_grad_enabled() else _native.host().weight_grad(dy2, x2)
+            if torch.is_grad_enabled():   # a graph of the backward pass wants operators that have derivatives
+                dw = dy.reshape(-1, dy.shape[-1]).t() @ x.reshape(-1, x.shape[-1])
+            else:
+                dw = torch.ops.castle_hip.linear_bwd(dy, x, weight, False, True)[1]
         return dx, dw
 
 
@@ -244,10 +245,11 @@ def _unmodified(module, kind) -> bool:
                                          or own["_backward_hooks"] or own["_backward_pre_hooks"])
 
 
-def _linear(layer, t):
-    """layer(t) for a bias-free nn.Linear, through _ManyRowLinear where its weight gradient pays."""
+def _linear(layer, t, native=True):
+    """layer(t) for a bias-free nn.Linear, through _ManyRowLinear where its weight gradient pays.  native=False: the layer
+    itself (of a module built with use_triton=False, which may stand where the library is not built)."""
     rows = t.numel() // t.shape[-1] if t.shape[-1] else 0
-    if (t.is_cuda and _unmodified(layer, nn.Linear) and layer.bias is None and t.dtype in (torch.bfloat16, torch.float16) and layer.weight.dtype == t.dtype
+    if (native and t.is_cuda and _unmodified(layer, nn.Linear) and layer.bias is None and t.dtype in (torch.bfloat16, torch.float16) and layer.weight.dtype == t.dtype
             and rows >= SPLIT_WGRAD_MIN_ROWS and t.is_contiguous()
             and torch.is_grad_enabled() and layer.weight.requires_grad):
         return _ManyRowLinear.apply(t, layer.weight)
@@ -380,13 +382,13 @@ class Castle(nn.Module):
             merged, next_cache = self._parallel_native(torch.ops.castle_hip.linear(x, self.to_all_qkv.weight), return_next_cache)
             y = torch.ops.castle_hip.linear(merged, self.combine_heads.weight)
             return (y, next_cache) if return_next_cache else y
-        proj = self._project(self.to_all_qkv, x, native_step, norm=self.norm)
+        proj = self._project(self.to_all_qkv, x, native_step, norm=self.norm, native=native)
         if not single:
             assert cache is None, "must be inferencing single tokens if receiving cache"
             merged, next_cache = (self._parallel_native if native else self._parallel_dense)(proj, return_next_cache)
         else:
             merged, next_cache = (self._step_native if native else self._step_dense)(proj, cache)
-        y = self._project(self.combine_heads, merged, native_step)
+        y = self._project(self.combine_heads, merged, native_step, native=native)
         return (y, next_cache) if return_next_cache else y
 
     def _plain(self, x):
@@ -453,7 +455,7 @@ class Castle(nn.Module):
         return (*results[:outputs], store.as_cache())
 
     @staticmethod
-    def _project(layer, t, native_step, norm=None, activation=None, residual=None):
+    def _project(layer, t, native_step, norm=None, activation=None, residual=None, native=True):
         """A bias-free projection with what surrounds it in a block: `norm` (an nn.RMSNorm or
         nn.Identity) in front, GELU (`activation="gelu"`) and a residual behind.  On the native
         single-token step the few rows go through the library's own small-M kernel, which does all
@@ -463,7 +465,7 @@ class Castle(nn.Module):
         if (native_step and _unmodified(layer, nn.Linear) and layer.bias is None and (norm is None or _unmodified(norm, nn.RMSNorm))
                 and ops.small_linear_ok(t, layer.weight)):
             return ops.small_linear(t, layer.weight, norm=norm, activation=activation, residual=residual)
-        y = _linear(layer, t if norm is None else norm(t))
+        y = _linear(layer, t if norm is None else norm(t), native)
         if activation == "gelu":
             y = F.gelu(y)
         return y if residual is None else residual + y

@@ -1080,10 +1080,6 @@ PYBIND11_MODULE(_castle_host, m) {
   m.def("product", [](const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux) {
     return product(a, a_t, b, b_t, epilogue, aux);
   }, unlocked());
-  m.def("weight_grad", [](const Tensor& dy, const Tensor& x) {
-    const c10::DeviceGuard guard(x.device());
-    return weight_grad(dy, x);
-  }, unlocked());
   m.def("feed_forward", &feed_forward, unlocked());
   m.def("head", &head, unlocked());
   m.def("cross_entropy", &cross_entropy, unlocked());

@@ -85,10 +85,10 @@ def token_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Te
     return Castle._project(down, hidden, True, residual=h)
 
 
-def block_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Tensor:
-    """feed_forward(h) for the block [norm, linear, GELU, linear] over many rows: the layers themselves,
+def block_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor, native: bool = True) -> torch.Tensor:
+    """feed_forward(h) for the block [norm, linear, GELU, linear] over many rows: the layers themselves; of a native model
     with the two weight gradients formed in row ranges where that pays (castle._linear)."""
-    if not _is_block(feed_forward):
+    if not (native and _is_block(feed_forward)):
         return feed_forward(h)
     norm, up, act, down = feed_forward
     return _linear(down, act(_linear(up, norm(h))))
@@ -257,7 +257,8 @@ class CastleLM(nn.Module):
         # one token per sequence, no graph to record: the few rows of every projection go through the small-M kernel
         # (only for a model whose layers run the native kernels: one built with use_triton=False stays on
         # the PyTorch layers throughout, so it remains an independent baseline for the native one)
-        token_step = h.shape[1] == 1 and not torch.is_grad_enabled() and self._native_on_gpu(h.device)
+        native = self._native_on_gpu(h.device)
+        token_step = h.shape[1] == 1 and not torch.is_grad_enabled() and native
         next_cache = []
         for index, (attention, feed_forward) in enumerate(self.layers):
             layer_cache = cache[index] if cache is not None and index < len(cache) else None
@@ -267,8 +268,8 @@ class CastleLM(nn.Module):
             else:
                 attended = attention(h, cache=layer_cache, return_next_cache=False)
             h = h + attended
-            h = token_feed_forward(feed_forward, h) if token_step else h + block_feed_forward(feed_forward, h)
-        logits = Castle._project(self.to_logits, h, token_step, norm=self.final_norm)
+            h = token_feed_forward(feed_forward, h) if token_step else h + block_feed_forward(feed_forward, h, native)
+        logits = Castle._project(self.to_logits, h, token_step, norm=self.final_norm, native=native)
         if return_loss:
             return F.cross_entropy(logits.transpose(1, 2), target)
         return (logits, next_cache) if return_next_cache else logits

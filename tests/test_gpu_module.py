@@ -186,7 +186,7 @@ def test_projection_over_many_rows_forms_its_weight_gradient_in_row_ranges():
 # outputs of 8, 4, 2 ranges and of one product; rows that do not divide
 @pytest.mark.parametrize("rows,n,k", [(8192, 1536, 256), (8192, 2048, 2048), (8192, 6144, 1024), (8192, 6144, 2048), (8203, 512, 512)])
 def test_a_hooked_layer_forms_its_weight_gradients_like_a_plain_one(rows, n, k):
-    from lookahead_keys_attention_amd import _native, castle as C
+    from lookahead_keys_attention_amd import castle as C
 
     torch.manual_seed(6)
     layer = torch.nn.Linear(k, n, bias=False).to(DEV).bfloat16()
@@ -195,16 +195,38 @@ def test_a_hooked_layer_forms_its_weight_gradients_like_a_plain_one(rows, n, k):
     y = C._linear(layer, x)
     assert "ManyRowLinear" in type(y.grad_fn).__name__
     y.backward(gy)
-    assert torch.equal(layer.weight.grad, _native.host().weight_grad(gy[0], x[0]))
+    assert torch.equal(layer.weight.grad, torch.ops.castle_hip.linear_bwd(gy, x, layer.weight.detach(), False, True)[1])
     ref = gy[0].float().t() @ x[0].float()
     assert (layer.weight.grad.float() - ref).norm() <= 4e-3 * ref.norm()   # one rounding to bf16
     handle = layer.register_forward_hook(lambda *_: None)   # on the projection itself: the module runs
     assert "ManyRowLinear" not in type(C._linear(layer, x).grad_fn).__name__
     handle.remove()
+    # traced: a norm that is hooked keeps the layer from being taken apart into the library's operators
+    norm = torch.nn.RMSNorm(k).to(DEV).bfloat16()
+    norm.register_forward_hook(lambda *_: None)
+    want = torch.autograd.grad(C._linear(layer, norm(x)), layer.weight, gy)[0]
+    torch._dynamo.reset()
+    traced = torch.compile(lambda t: C._linear(layer, norm(t)), backend="aot_eager", fullgraph=True)
+    assert torch.equal(torch.autograd.grad(traced(x), layer.weight, gy)[0], want)
     # with a graph of the backward pass the gradient has derivatives
     leaf = x[:, :, :].clone().requires_grad_()
     dw, = torch.autograd.grad(C._linear(layer, leaf).sum(), layer.weight, create_graph=True)
     assert torch.autograd.grad(dw.sum(), leaf)[0].eq(n).all()
+
+
+def test_dense_modules_over_many_rows_use_no_native_operator():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from lookahead_keys_attention_amd import CastleLM
+
+    class NoNative(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            assert func.namespace != "castle_hip", func
+            return func(*args, **(kwargs or {}))
+
+    model = CastleLM(num_tokens=64, dim=32, depth=1, dim_head=16, heads=2, use_triton=False).to(DEV).bfloat16()
+    with NoNative():
+        model(torch.zeros(512, 17, dtype=torch.long, device=DEV), return_loss=True).backward()
 
 
 @pytest.mark.parametrize("prenorm", [False, True])
