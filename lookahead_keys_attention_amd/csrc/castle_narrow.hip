@@ -25,7 +25,10 @@
 // may be skipped by a branch.  Where such a branch jumps over a run of loads, the compiler (ROCm 7.2) counts the
 // loads as waiting time on both ways, and on the taken one the first registers are read before they are written
 // (seen in the scan at d = 128: three accumulator registers of the last tile).  So the loads of a next tile are
-// unconditional (the last iteration repeats a tile), and conditional products come before unconditional ones.
+// unconditional (the last iteration repeats a tile), and conditional products come before unconditional ones.  Where sums over
+// waves or stores follow a loop of products, settle() stands in front of the first read; not where a barrier and reads of
+// LDS stand between anyway (the weights of the attention's partial results), nor where nothing can be skipped (a snapshot
+// at the top of the next iteration).
 //
 // Definitions, units and range control are those of castle_fwd.hip and castle_bwd.hip.  Rows beyond the sequence are
 // not visited (only what a partly filled tile of 32 holds).
@@ -220,10 +223,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
     }
     for (int jt = first; jt < last; ++jt) {
       const int I = jt >> 1;
-      if (keep && I > Kb && (jt == first || !(jt & 1))) {
-        settle();
-        store_snap_tile<T, HD, NT>(snap + (usnap_off(I) + kw0) * HD, st, c, g);
-      }
+      if (keep && I > Kb && (jt == first || !(jt & 1))) store_snap_tile<T, HD, NT>(snap + (usnap_off(I) + kw0) * HD, st, c, g);
       wave_lds_order<>();
       pk.store(s_ku);
       pv.store(s_vu);
@@ -471,7 +471,6 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void attn_narrow_k
     lt += mw == -INFINITY ? 0.f : fast_exp2(mw - M) * s_stat[(w * 64 + lane) * 2 + 1];
   }
   const float wt = m == -INFINITY ? 0.f : fast_exp2(m - M) / lt;
-  settle();
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
