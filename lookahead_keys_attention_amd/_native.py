@@ -173,7 +173,7 @@ def host():
 
 
 def is_built() -> bool:
-    return os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH)
+    return _host is not None or os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH)   # (asked in every token step)
 
 
 def check(code: int, what: str):

@@ -69,18 +69,23 @@ def _runs_castle_forward(attention) -> bool:
     return _unmodified(attention, type(attention)) and type(attention).forward is Castle.forward
 
 
-def _is_block(feed_forward) -> bool:
-    """True if the block may be taken apart: [norm, linear, erf GELU, linear] and nothing that wants to see a call of it."""
-    return _unmodified(feed_forward, nn.Sequential) and len(feed_forward) == 4 and _unmodified(feed_forward[2], nn.GELU) and feed_forward[2].approximate == "none"
+def _block_parts(feed_forward):
+    """(norm, linear, GELU, linear) of a block that may be taken apart: these four, the erf GELU, and nothing that wants to see a
+    call of the block or of the GELU; None otherwise."""
+    if not _unmodified(feed_forward, nn.Sequential):
+        return None
+    parts = tuple(feed_forward._modules.values())
+    return parts if len(parts) == 4 and _unmodified(parts[2], nn.GELU) and parts[2].approximate == "none" else None
 
 
 def token_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Tensor:
     """h + feed_forward(h) for a single-token step (inference), the block being [norm, linear,
     GELU, linear]: two launches of the small-M linear kernel (norm and GELU ride on the first, the
     residual on the second) when it can take them (16-bit GPU tensors), the layers themselves otherwise."""
-    if not _is_block(feed_forward):
+    parts = _block_parts(feed_forward)
+    if parts is None:
         return h + feed_forward(h)
-    norm, up, act, down = feed_forward
+    norm, up, _, down = parts
     hidden = Castle._project(up, h, True, norm=norm, activation="gelu")
     return Castle._project(down, hidden, True, residual=h)
 
@@ -88,9 +93,10 @@ def token_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor) -> torch.Te
 def block_feed_forward(feed_forward: nn.Sequential, h: torch.Tensor, native: bool = True) -> torch.Tensor:
     """feed_forward(h) for the block [norm, linear, GELU, linear] over many rows: the layers themselves; of a native model
     with the two weight gradients formed in row ranges where that pays (castle._linear)."""
-    if not (native and _is_block(feed_forward)):
+    parts = _block_parts(feed_forward) if native else None
+    if parts is None:
         return feed_forward(h)
-    norm, up, act, down = feed_forward
+    norm, up, act, down = parts
     return _linear(down, act(_linear(up, norm(h))))
 
 
@@ -292,7 +298,7 @@ class CastleLM(nn.Module):
                 return False
             attention, feed_forward = block
             if not (_unmodified(attention, Castle) and attention.use_triton and ops.kernels_support(attention.dim_head, dtype) and attention._plain(like)
-                    and _is_block(feed_forward)):
+                    and _block_parts(feed_forward) is not None):
                 return False
             norm, up, _, down = feed_forward
             if not (_unmodified(norm, nn.RMSNorm) and norm.weight is not None and norm.weight.dtype is dtype and _unmodified(up, nn.Linear) and up.bias is None
