@@ -240,6 +240,21 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
                         int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
                         void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same in one launch for a few sequences with the row count from the host (up to 10 MB of cached rows), where the host's
+ * work for three launches is what a step waits for; otherwise in three.  `control`: castle_decode_layer_control_bytes bytes,
+ * 256-byte aligned, zeroed once before the first such call and then left to these calls (NULL: three launches); calls that share it
+ * must not overlap, as they must not on one cache.  Workgroups of the launch wait for each other's results, never for one that has not
+ * started: the waits end whatever else runs on the GPU. */
+int64_t castle_decode_layer_control_bytes(int B, int H, int d, int dtype);
+int castle_decode_layer_once(const castle_view4* U, const castle_view4* qu_cache,
+                             const castle_view4* kc_cache, const castle_view4* vc_cache,
+                             int t, const int32_t* t_device, int capacity,
+                             const void* x, int64_t ldx, int dim, const void* norm_weight, float eps,
+                             const void* w_in, int64_t ldw_in, const void* w_out, int64_t ldw_out,
+                             const void* residual, int64_t ldr, void* y, int64_t ldy, void* proj,
+                             int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
+                             void* workspace, int64_t workspace_bytes, void* control, int64_t control_bytes, void* stream);
+
 /* Rotary position embedding of one tensor, out of place: out[b,h,l,:] = R(first_position + l) x[b,h,l,:]
  * (the rotation CASTLE_FLAG_ROTARY applies inside the kernels; lookahead_keys_attention.py:112).  Used to
  * fill the qu / kc rows of a decode cache after a rotary prefill. */

@@ -42,6 +42,8 @@ EXPORTED_SYMBOLS = (
     "castle_decode_step_static",
     "castle_decode_flush",
     "castle_decode_layer",
+    "castle_decode_layer_control_bytes",
+    "castle_decode_layer_once",
     "castle_rope",
     "castle_cache_rows",
     "castle_small_linear",

@@ -22,6 +22,8 @@ int launch_cache_rows(const View4 (&src)[3], const View4 (&dst)[3], int B, int H
 int launch_rope(const View4& src, const View4& dst, int B, int H, int L, int d, int dtype, int pos0, hipStream_t stream);
 int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus);
 int decode_static_scratch(float** ptr);
+int64_t decode_layer_control_bytes(int B, int H, int d, int es);
+int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, int dtype, int cus, hipStream_t stream);
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                         int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream, int* clear = nullptr, int clear_n = 0);
 int launch_sample(const void* logits, int64_t ld, const float* u, int rows, int V, int k, float inv_temperature, int64_t* out, int64_t out_ld,
@@ -408,14 +410,21 @@ int castle_decode_step_device_count(const castle_view4* U, const castle_view4* q
                             B, H, d, dtype, scale, flags, out, deferred, workspace, workspace_bytes, false, stream);
 }
 
-int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
+int64_t castle_decode_layer_control_bytes(int B, int H, int d, int dtype) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (B <= 0 || H <= 0 || !head_dim_ok(d) || (int64_t)B * H > 65535) return CASTLE_ERR_SHAPE;
+  return align_up(castle::decode_layer_control_bytes(B, H, d, es), 256);
+}
+
+static int decode_layer_common(const castle_view4* U, const castle_view4* qu_cache,
                         const castle_view4* kc_cache, const castle_view4* vc_cache,
                         int t, const int32_t* t_device, int capacity,
                         const void* x, int64_t ldx, int dim, const void* norm_weight, float eps,
                         const void* w_in, int64_t ldw_in, const void* w_out, int64_t ldw_out,
                         const void* residual, int64_t ldr, void* y, int64_t ldy, void* proj,
                         int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
-                        void* workspace, int64_t workspace_bytes, void* stream) {
+                        void* workspace, int64_t workspace_bytes, void* control, int64_t control_bytes, void* stream) {
   const int es = elem_size(dtype);
   if (es == 0) return CASTLE_ERR_DTYPE;
   if (B <= 0 || H <= 0 || dim <= 0 || !head_dim_ok(d) || dim % (16 / es) != 0) return CASTLE_ERR_SHAPE;
@@ -434,6 +443,13 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
                             &tok[0], &tok[1], &tok[2], B, H, d, dtype, scale, flags, nullptr, deferred, workspace, workspace_bytes, false);
   if (rc != CASTLE_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (control != nullptr) {
+    if (reinterpret_cast<uintptr_t>(control) % 256 != 0 || control_bytes < castle_decode_layer_control_bytes(B, H, d, dtype)) return CASTLE_ERR_WORKSPACE;
+    const castle::DecodeLinear in = {x, w_in, nullptr, B, width, dim, ldx, ldw_in, 0, norm_weight, eps, nullptr, 0};
+    const castle::DecodeLinear out = {nullptr, w_out, y, B, dim, inner, 0, ldw_out, ldy, nullptr, 0.f, residual, ldr};
+    rc = castle::launch_decode_layer(a, in, out, control, dtype, device_cus(), s);
+    if (rc != 1) return rc;
+  }
   // the projection clears the arrival counts of the step, which then needs no launch to merge its splits
   a.arrivals = reinterpret_cast<int*>(a.part + (int64_t)B * H * 64 * (d + 2));
   rc = castle::launch_small_linear(x, w_in, proj, B, width, dim, ldx, ldw_in, width, dtype, norm_weight, eps, CASTLE_ACT_NONE, nullptr, 0, s, a.arrivals, B * H);
@@ -441,6 +457,30 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
   if (rc == 0) rc = castle::launch_decode(a, dtype, s);
   if (rc != 0) return rc;
   return castle::launch_small_linear(proj, w_out, y, B, dim, inner, width, ldw_out, ldy, dtype, nullptr, 0.f, CASTLE_ACT_NONE, residual, ldr, s);
+}
+
+int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
+                        const castle_view4* kc_cache, const castle_view4* vc_cache,
+                        int t, const int32_t* t_device, int capacity,
+                        const void* x, int64_t ldx, int dim, const void* norm_weight, float eps,
+                        const void* w_in, int64_t ldw_in, const void* w_out, int64_t ldw_out,
+                        const void* residual, int64_t ldr, void* y, int64_t ldy, void* proj,
+                        int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
+                        void* workspace, int64_t workspace_bytes, void* stream) {
+  return decode_layer_common(U, qu_cache, kc_cache, vc_cache, t, t_device, capacity, x, ldx, dim, norm_weight, eps, w_in, ldw_in, w_out, ldw_out,
+                             residual, ldr, y, ldy, proj, B, H, d, dtype, scale, flags, deferred, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+int castle_decode_layer_once(const castle_view4* U, const castle_view4* qu_cache,
+                        const castle_view4* kc_cache, const castle_view4* vc_cache,
+                        int t, const int32_t* t_device, int capacity,
+                        const void* x, int64_t ldx, int dim, const void* norm_weight, float eps,
+                        const void* w_in, int64_t ldw_in, const void* w_out, int64_t ldw_out,
+                        const void* residual, int64_t ldr, void* y, int64_t ldy, void* proj,
+                        int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
+                        void* workspace, int64_t workspace_bytes, void* control, int64_t control_bytes, void* stream) {
+  return decode_layer_common(U, qu_cache, kc_cache, vc_cache, t, t_device, capacity, x, ldx, dim, norm_weight, eps, w_in, ldw_in, w_out, ldw_out,
+                             residual, ldr, y, ldy, proj, B, H, d, dtype, scale, flags, deferred, workspace, workspace_bytes, control, control_bytes, stream);
 }
 
 int castle_decode_flush(const castle_view4* U, const castle_view4* qu_cache, int t, const castle_deferred* deferred,

@@ -88,6 +88,59 @@ __device__ __forceinline__ float* part_stat(const DecodeArgs& a, int bh, int spl
 __device__ __forceinline__ void agent_store(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float agent_load(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+// Results that cross from one job of a launch to another without a wait for the memory in between: 8-byte words of four
+// payload bytes and the tag of the launch, stored and loaded at agent scope.  A word that carries the tag is there, whole.
+struct TokenWords {
+  const uint64_t* proj = nullptr;   // [B][6][H][d] in words
+  uint64_t* merged = nullptr;       // [B][H][d]
+  uint64_t* part = nullptr;         // [B][H][splits][d + 2]: sums, maximum, sum of weights, a float each
+  uint32_t tag = 0;
+};
+// LDS of the early rows: by iteration and tensor (qu, U, kc, vc, gates) 1 KB per wave
+constexpr int kEarly = 2;
+constexpr int kEarlyTensor = kThreads * 16, kEarlyIteration = 5 * kEarlyTensor;
+extern __shared__ __attribute__((aligned(16))) unsigned char castle_early[];
+__device__ __forceinline__ unsigned char* early_rows(int n, int lane) { return castle_early + n * kEarlyIteration + wave_id() * 1024 + lane * 16; }
+// 16 bytes per lane from memory to consecutive places in LDS
+template <bool ONCE> __device__ __forceinline__ void load_lds16(const void* from, unsigned char* to) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from, (__attribute__((address_space(3))) void*)to, 16, 0, ONCE ? 2 : 0);
+}
+template <typename T> constexpr int kPerWord = 4 / (int)sizeof(T);
+__device__ __forceinline__ void store_word(uint64_t* p, uint32_t payload, uint32_t tag) {
+  __hip_atomic_store(p, (uint64_t)tag << 32 | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// element i of a row of words from lane i (of consecutive lanes); 16-bit elements leave in pairs
+template <typename T> __device__ __forceinline__ void put_word(uint64_t* row, int i, float v, uint32_t tag) {
+  if constexpr (sizeof(T) == 4) {
+    store_word(row + i, __builtin_bit_cast(uint32_t, v), tag);
+  } else {
+    const float w = __shfl_xor(v, 1);
+    if (i % 2 == 0) store_word(row + i / 2, __builtin_bit_cast(uint32_t, vec<T, 2>{(T)v, (T)w}), tag);
+  }
+}
+// N 16-byte pieces (four words each) per lane, zeros for a null pointer.  False if after some patience a word of the wave's lanes
+// still does not carry the tag.
+constexpr int kPatience = 64;   // polls, of about a microsecond
+template <typename T, int N> __device__ __forceinline__ bool wait_words(const uint64_t* const (&p)[N], uint32_t tag, vec<T, elem_traits<T>::vec16> (&x)[N]) {
+  for (int polls = 0; polls < kPatience; ++polls) {
+    bool there = true;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      uint64_t w[4] = {};
+      if (p[n] != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = __hip_atomic_load(p[n] + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) there = there && (uint32_t)(w[e] >> 32) == tag;
+      }
+      x[n] = __builtin_bit_cast(vec<T, elem_traits<T>::vec16>, vec<uint32_t, 4>{(uint32_t)w[0], (uint32_t)w[1], (uint32_t)w[2], (uint32_t)w[3]});
+    }
+    if (__builtin_amdgcn_ballot_w64(!there) == 0) return true;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return false;
+}
+
 // A group of LPR = d / V lanes owns one cache row per iteration.  (Workgroups of 16 waves, so that a head needs no
 // split and no merge, are slower throughout: 23.1 against 21.7 us for a layer step of 16 x 8 heads of 540 rows.)
 //
@@ -95,31 +148,40 @@ __device__ __forceinline__ float agent_load(const float* p) { return __hip_atomi
 // qc . U_k of the stored one plus a gate times qc . vu for every pending token, which is one number per token and
 // head.  (180 vector instructions per row and lane with the completed key in registers, 110 without: at 16 x 8 heads x
 // 540 rows they took as long as the memory.)
-template <typename T, int HD, bool UH, bool ONCE>
-__global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a) {
+//
+// WORDS: a job of a launch that does the whole layer step (decode_layer_kernel below).  The token's pieces come as tagged
+// words, waited for behind the requests for the first rows, and the output leaves as such; ready(whether they came) says
+// whether the job goes on (if not, nothing has been written).
+template <typename T, int HD, bool UH, bool ONCE, bool WORDS, typename G, typename F>
+__device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int bh, const TokenWords& words, G&& begin, F&& ready) {
   constexpr int V = elem_traits<T>::vec16;   // elements per 16-byte lane load
   constexpr int LPR = HD / V;                // lanes per row
   constexpr int RPI = kThreads / LPR;        // rows per workgroup iteration
   constexpr int NW = kThreads / 64;
   typedef vec<T, V> vt;
-  __shared__ float s_acc[NW][HD + 2];
+  __shared__ float s_acc[NW + (WORDS ? 1 : 0)][HD + 2];
   __shared__ float s_vu[kDecodeDefer + 1][HD];   // vu of the pending tokens by ring slot and of the new one, for steps that write U
 
-  const int split = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
+  const int b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x;
   const int grp = tid / LPR, sub = tid % LPR;
   // All loads of the start go out together, the small ones first (they are waited for first): the token's pieces,
   // which do not need the row count, then the pending tokens' vu pieces and the rows of the first iteration.
-  const vt tku = *reinterpret_cast<const vt*>(view_row<T>(a.ku, b, h, 0) + sub * V);
-  const vt tvu = *reinterpret_cast<const vt*>(view_row<T>(a.vu, b, h, 0) + sub * V);
-  const vt tqc = *reinterpret_cast<const vt*>(view_row<T>(a.qc, b, h, 0) + sub * V);
+  vt tku, tvu, tqc;
+  if constexpr (!WORDS) {
+    tku = *reinterpret_cast<const vt*>(view_row<T>(a.ku, b, h, 0) + sub * V);
+    tvu = *reinterpret_cast<const vt*>(view_row<T>(a.vu, b, h, 0) + sub * V);
+    tqc = *reinterpret_cast<const vt*>(view_row<T>(a.qc, b, h, 0) + sub * V);
+  }
   int t = a.t_dev != nullptr ? *a.t_dev : a.t;
   const bool in_range = t >= 0 && t < a.capacity;
   if (!in_range) t = 0;   // only with a device-side count: no rows, nothing is appended
   const float c1 = a.scale * kLog2e;
 
-  // rows of this workgroup: [r0, r1), whole iterations of RPI rows
-  const int per = ((t + a.splits - 1) / a.splits + RPI - 1) / RPI * RPI;
+  // rows of this workgroup: [r0, r1), whole iterations of RPI rows.  With WORDS the last split has none (unless it is the only
+  // one): it has the appended row to see to, and the partial results of the others.
+  const int with_rows = WORDS && a.splits > 1 ? a.splits - 1 : a.splits;
+  const int per = ((t + with_rows - 1) / with_rows + RPI - 1) / RPI * RPI;
   const int r0 = split * per;
   const int r1 = min(t, r0 + per);
 
@@ -129,9 +191,9 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
   const int pbase = deferred ? decode_base(base0, t) : t;
   const int np = t - pbase;                                        // 0 .. kDecodeDefer - 1
   const bool write_u = !deferred || (t + 1) % kDecodeDefer == 0;
-  const bool owner = split == (t > 0 ? (t - 1) / per : 0);
+  const bool owner = split == (WORDS ? a.splits - 1 : t > 0 ? (t - 1) / per : 0);
   vt tkc, tqu, tvc, tpv[kDecodeDefer];
-  if (owner) {
+  if (!WORDS && owner) {
     tkc = *reinterpret_cast<const vt*>(view_row<T>(a.kc, b, h, 0) + sub * V);
     tqu = *reinterpret_cast<const vt*>(view_row<T>(a.qu, b, h, 0) + sub * V);
     tvc = *reinterpret_cast<const vt*>(view_row<T>(a.vc, b, h, 0) + sub * V);
@@ -145,9 +207,12 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
     for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
     if (pend_j[sl] >= 0) tpv[sl] = *reinterpret_cast<const vt*>(view_row<T>(a.pend_vu, b, h, sl) + sub * V);
   }
-  // The row pieces of the next iteration are requested before the current one is processed.
+  // The row pieces of the next iteration are requested before the current one is processed.  While the token is
+  // still being projected (WORDS) those of the first `early` iterations are on their way too, straight into LDS: a lane reads
+  // back what it asked for.
   vt nq, nu, nk, nv;
   vec<float, 4> ng = {0.f, 0.f, 0.f, 0.f};
+  constexpr int early = WORDS ? kEarly : 0;
   float* const gbase = deferred ? reinterpret_cast<float*>(a.pend_gate.ptr) + (int64_t)b * a.pend_gate.sb + (int64_t)h * a.pend_gate.sh : nullptr;
   // ONCE: past what the last-level cache (256 MB) holds of the loop this step belongs to, keeping rows in it only drives out the
   // weights and what else could stay (a layer step of 16 x 8 heads x 540 rows, one of 12 layers: 21.8 -> 19.9 us; with 6
@@ -165,8 +230,32 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
       if (np > 0) ng = read(reinterpret_cast<const vec<float, 4>*>(gbase + (int64_t)k * kDecodeDefer));
     }
   };
-  request(r0 + grp);
+  if constexpr (WORDS) {
+    for (int n = 0; n < early; ++n) {
+      const int k = r0 + grp + n * RPI;
+      if (k < r1) {
+        unsigned char* const to = early_rows(n, 0);
+        load_lds16<ONCE>(view_row<T>(a.qu_cache, b, h, k) + sub * V, to);
+        load_lds16<ONCE>(view_row<T>(a.U, b, h, k) + sub * V, to + kEarlyTensor);
+        load_lds16<ONCE>(view_row<T>(a.kc_cache, b, h, k) + sub * V, to + 2 * kEarlyTensor);
+        load_lds16<ONCE>(view_row<T>(a.vc_cache, b, h, k) + sub * V, to + 3 * kEarlyTensor);
+        if (np > 0) load_lds16<ONCE>(gbase + (int64_t)k * kDecodeDefer, to + 4 * kEarlyTensor);
+      }
+    }
+  }
+  request(r0 + grp + early * RPI);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (WORDS) {
+    begin();
+    const uint64_t* w = words.proj + ((int64_t)b * 6 * a.H + h) * (HD / kPerWord<T>) + sub * 4;   // parts qu, ku, vu, qc, kc, vc
+    const int64_t part = (int64_t)a.H * (HD / kPerWord<T>);
+    vt got[6];
+    const uint64_t* const need[6] = {w + part, w + 2 * part, w + 3 * part, owner ? w + 4 * part : nullptr, owner ? w : nullptr, owner ? w + 5 * part : nullptr};
+    if (!ready(wait_words<T>(need, words.tag, got))) return false;
+    tku = got[0]; tvu = got[1]; tqc = got[2];
+    if (owner) { tkc = got[3]; tqu = got[4]; tvc = got[5]; }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the early rows are in LDS (requested in front of the words, they came first)
+  }
   float ku[V], qc[V], acc[V], m = -INFINITY, l = 0.f;   // ku, qc times c1: products come out in log2 units
   float cvu[kDecodeDefer], cvu_t;                       // c1 qc . vu of the pending tokens and of the new one
   const int slot_t = t % kDecodeDefer;
@@ -244,10 +333,20 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
   }
 
   auto rows = [&](auto writes) __attribute__((always_inline)) {
-    for (int k = r0 + grp; k < r1; k += RPI) {
-      const vt cq = nq, cu = nu, ck = nk, cv = nv;
-      const vec<float, 4> g4 = ng;
-      request(k + RPI);
+    int n = 0;
+    for (int k = r0 + grp; k < r1; k += RPI, ++n) {
+      vt cq = nq, cu = nu, ck = nk, cv = nv;
+      vec<float, 4> g4 = ng;
+      if (WORDS && n < early) {
+        const unsigned char* const from = early_rows(n, lane_id());
+        cq = *reinterpret_cast<const vt*>(from);
+        cu = *reinterpret_cast<const vt*>(from + kEarlyTensor);
+        ck = *reinterpret_cast<const vt*>(from + 2 * kEarlyTensor);
+        cv = *reinterpret_cast<const vt*>(from + 3 * kEarlyTensor);
+        g4 = *reinterpret_cast<const vec<float, 4>*>(from + 4 * kEarlyTensor);   // (not looked at without pending tokens)
+      } else {
+        request(k + RPI);
+      }
       float dg = 0.f, dsc = 0.f, dsu = 0.f;
 #pragma unroll
       for (int e = 0; e < V; ++e) {
@@ -332,17 +431,92 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
     if (sub == 0) { s_acc[wave][HD] = m; s_acc[wave][HD + 1] = l; }
   }
   __syncthreads();
+  float out = 0.f, M = -INFINITY, lsum = 0.f;
   if (tid < HD) {
-    float M = -INFINITY;
 #pragma unroll
     for (int r = 0; r < NW; ++r) M = fmaxf(M, s_acc[r][HD]);
-    float out = 0.f, lsum = 0.f;
 #pragma unroll
     for (int r = 0; r < NW; ++r) {
       const float w = (s_acc[r][HD] == -INFINITY) ? 0.f : fast_exp2(s_acc[r][HD] - M);
       out = __builtin_fmaf(w, s_acc[r][tid], out);
       lsum = __builtin_fmaf(w, s_acc[r][HD + 1], lsum);
     }
+  }
+  constexpr int EPL = (HD + 63) / 64;
+  const int lane = tid & 63;
+  if constexpr (WORDS) {
+    uint64_t* const row = words.merged + (int64_t)bh * (HD / kPerWord<T>);
+    if (a.splits == 1) {
+      if (tid < HD) put_word<T>(row, tid, out / lsum, words.tag);
+      return true;
+    }
+    uint64_t* const parts = words.part + (int64_t)bh * a.splits * (HD + 2);
+    if (split < a.splits - 1) {
+      uint64_t* const p = parts + (int64_t)split * (HD + 2);
+      if (tid < HD) store_word(p + tid, __builtin_bit_cast(uint32_t, out), words.tag);
+      if (tid < 2) store_word(p + HD + tid, __builtin_bit_cast(uint32_t, tid == 0 ? M : lsum), words.tag);
+      return true;
+    }
+    // The last split's workgroup waits for the others (jobs in front of it) and merges: wave w takes every NW-th partial.
+    constexpr int SU = 4;   // of them in flight
+    float m_w = -INFINITY, l_w = 0.f, a_w[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) a_w[e] = 0.f;
+    for (int s0 = wave; s0 < a.splits - 1; s0 += SU * NW) {
+      float v[SU][EPL + 2];
+      while (true) {
+        bool there = true;
+#pragma unroll
+        for (int u = 0; u < SU; ++u) {
+          const int s = s0 + u * NW;
+          v[u][EPL] = -INFINITY;
+          if (s < a.splits - 1) {
+#pragma unroll
+            for (int e = 0; e < EPL + 2; ++e) {
+              const int n = e < EPL ? lane + 64 * e : HD + e - EPL;
+              if (n >= HD + 2) continue;   // (lanes beyond a short row read the statistics once more)
+              const uint64_t w = __hip_atomic_load(parts + (int64_t)s * (HD + 2) + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              there = there && (uint32_t)(w >> 32) == words.tag;
+              v[u][e] = __builtin_bit_cast(float, (uint32_t)w);
+            }
+          }
+        }
+        if (__builtin_amdgcn_ballot_w64(!there) == 0) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+#pragma unroll
+      for (int u = 0; u < SU; ++u) {
+        if (v[u][EPL] == -INFINITY) continue;   // not there, or without rows
+        const float mn = fmaxf(m_w, v[u][EPL]), wo = fast_exp2(m_w - mn), wn = fast_exp2(v[u][EPL] - mn);
+        l_w = l_w * wo + wn * v[u][EPL + 1];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) a_w[e] = a_w[e] * wo + wn * v[u][e];
+        m_w = mn;
+      }
+    }
+    __syncthreads();   // s_acc is read
+#pragma unroll
+    for (int e = 0; e < EPL; ++e)
+      if (lane + 64 * e < HD) s_acc[wave][lane + 64 * e] = a_w[e];
+    if (lane == 0) { s_acc[wave][HD] = m_w; s_acc[wave][HD + 1] = l_w; }
+    if (tid < HD) s_acc[NW][tid] = out;
+    if (tid == 0) { s_acc[NW][HD] = M; s_acc[NW][HD + 1] = lsum; }
+    __syncthreads();
+    if (tid < HD) {
+      float top = -INFINITY, o = 0.f, l_all = 0.f;
+#pragma unroll
+      for (int r = 0; r <= NW; ++r) top = fmaxf(top, s_acc[r][HD]);
+#pragma unroll
+      for (int r = 0; r <= NW; ++r) {
+        const float w = s_acc[r][HD] == -INFINITY ? 0.f : fast_exp2(s_acc[r][HD] - top);
+        o = __builtin_fmaf(w, s_acc[r][tid], o);
+        l_all = __builtin_fmaf(w, s_acc[r][HD + 1], l_all);
+      }
+      put_word<T>(row, tid, o / l_all, words.tag);
+    }
+    return true;
+  }
+  if (tid < HD) {
     if (a.splits == 1) {
       if (in_range) view_row<T>(a.out, b, h, 0)[tid] = (T)(out / lsum);
     } else {
@@ -351,22 +525,21 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
   }
-  if (a.arrivals == nullptr || a.splits == 1) return;
+  if (a.arrivals == nullptr || a.splits == 1) return true;
   __syncthreads();
   __shared__ int s_last;
   if (tid == 0) s_last = __hip_atomic_fetch_add(a.arrivals + bh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.splits - 1;
   __syncthreads();
-  if (!s_last || !in_range) return;
+  if (!s_last || !in_range) return true;
   // the last split: lane s of every wave holds the statistics of split s (at most 64), a wave sums every fourth partial
-  constexpr int EPL = (HD + 63) / 64;
-  const int lane = tid & 63;
   const float ms = lane < a.splits ? agent_load(part_stat(a, bh, lane, HD)) : -INFINITY;
   const float ls = lane < a.splits ? agent_load(part_stat(a, bh, lane, HD) + 1) : 0.f;
   float sum[EPL];
 #pragma unroll
   for (int e = 0; e < EPL; ++e) sum[e] = 0.f;
   constexpr int SU = 4;   // partials of a wave in flight
-  float wgt = 0.f, lsum = 0.f;
+  float wgt = 0.f;
+  lsum = 0.f;
   for (int s0 = wave; s0 < a.splits; s0 += SU * NW) {
     float v[SU][EPL];
 #pragma unroll
@@ -377,7 +550,7 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
         v[u][e] = s < a.splits && n < HD ? agent_load(part_acc(a, bh, s, HD) + n) : 0.f;
       }
     if (s0 == wave) {   // the statistics arrive with the first partials
-      float M = ms;
+      M = ms;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
       wgt = ms == -INFINITY ? 0.f : fast_exp2(ms - M);
@@ -403,6 +576,11 @@ __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a
     for (int r = 0; r < NW; ++r) o += s_acc[r][tid];
     view_row<T>(a.out, b, h, 0)[tid] = (T)(o / s_acc[0][HD]);
   }
+  return true;
+}
+template <typename T, int HD, bool UH, bool ONCE>
+__global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a) {
+  stream_job<T, HD, UH, ONCE, false>(a, blockIdx.x, blockIdx.y, TokenWords(), [] {}, [] { return true; });
 }
 
 // One wave per (b, h): merges the split partials into the attention output.
@@ -834,6 +1012,338 @@ int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int
     default: return -1;
   }
   return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+// ---------------------------------------------------------------------------
+// The whole layer step in one launch: jobs for the tiles of the projection, for the splits of the streaming pass and for the
+// tiles of the output projection, one workgroup each, in that order.
+//
+// What bounds it is trips to memory, one after the other: arguments, weights, reduction (3.1 us until the projection is
+// stored), the words of the token (2), rows and their sums (3), the partial results (2), the words of the output and the last product
+// (2.5).  The streaming jobs have requested their rows and the output jobs hold their weights by the time the projection is
+// done; a word takes 0.6 us from its store to a load that sees it, and a poll about one.
+//
+// Waiting inside a launch ends only if what is waited for runs.  Nothing is assumed about the order in which workgroups
+// start: every job is claimed before it writes anything (one word per job), jobs wait for jobs in front of them only, for a
+// bounded time, and a workgroup that has waited in vain claims and runs what nobody has claimed in front of its own job, first to
+// last, before it tries its own again.  The first of the unfinished jobs finds all it needs, so there is always one that
+// ends.  (The last split waits for the others without a bound, but only once all of them are claimed.)  A workgroup whose job was
+// taken leaves.  The last workgroup to leave moves the tag on, so that no launch can take words or claims of another for
+// its own.
+constexpr int kExitGroups = 32, kLine = 32;   // words of a 128-byte line
+constexpr int kLayerJobs = 2048;
+constexpr int kLayerGroups = 3;   // workgroups of a CU
+// Up to this many bytes of cached rows, and with the row count from the host: a step that the host launches is bound by it with
+// three launches (16 us of host work, more than the kernels take), one launch takes 12 to 14 (us a step, three / one:
+// 1 x 8 heads of 300 rows 16.1 / 12.9, 1 x 2 of 1000 16.6 / 13.5, 4 x 8 of 300 16.0 / 14.4, 16 x 4 of 300 16.3 / 15.2, level
+// at 8 x 8 of 300 and 1 x 16 of 300 with 12 MB of weights, 8 x 8 of 1000 19.3 / 20.9).  Replayed from a graph the hand-over inside a launch
+// costs what a launch does (29.1 / 29.2 with feed-forward at 1 x 8 heads of 300 rows, 36.5 / 37.6 at 16 x 8).
+constexpr int64_t kLayerCacheBytes = 10 << 20;
+constexpr int kTries = 1 << 19;   // of a job whose operands do not come: some tens of seconds, where something else is broken
+struct LayerArgs {
+  DecodeArgs d;
+  LinearArgs in, out;
+  uint32_t* control;   // tag of the last launch; workgroups gone, in all and by group, a line each; claims
+  uint64_t *proj, *merged, *part;
+  int n_in, n_stream, n_out, in_cols, out_cols;   // jobs; column tiles of the two products
+};
+constexpr int kGone = kLine, kGoneGroup = 2 * kLine, kClaims = kGoneGroup + kExitGroups * kLine;
+
+__device__ __forceinline__ uint32_t agent_word(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// true if the job was free
+__device__ __forceinline__ bool claim_job(uint32_t* claims, int job, uint32_t tag) {
+  return __hip_atomic_exchange(claims + job, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != tag;
+}
+// by each wave: n jobs (at most 64) are claimed
+__device__ __forceinline__ bool jobs_claimed(const uint32_t* claims, int n, uint32_t tag) {
+  const bool open = lane_id() < n && agent_word(claims + min(lane_id(), n - 1)) != tag;
+  return __builtin_amdgcn_ballot_w64(open) == 0;
+}
+// by one wave: claims the first free one of the first n jobs, -1 if there is none
+__device__ __forceinline__ int take_job(uint32_t* claims, int n, uint32_t tag) {
+  for (int base = 0; base < n; base += 64) {
+    const int i = base + lane_id();
+    unsigned long long open = __builtin_amdgcn_ballot_w64(i < n && agent_word(claims + min(i, n - 1)) != tag);
+    while (open != 0) {
+      const int job = base + __builtin_ctzll(open);
+      int got = 0;
+      if (lane_id() == 0) got = claim_job(claims, job, tag);
+      if (__builtin_amdgcn_readfirstlane(got)) return job;
+      open &= open - 1;
+    }
+  }
+  return -1;
+}
+
+struct LinearLds {
+  float red[kThreads / 64][16][17];
+  float ssq[kThreads / 64][16];
+};
+__device__ __forceinline__ LinearLds& linear_lds() {
+  __shared__ LinearLds lds;
+  return lds;
+}
+// One 16 x 16 tile (or part of one) of y = x w^T, the K split over the waves as in small_linear_kernel.  WORDS_IN: x comes as words, else
+// y leaves as words.  ready(whether the words came): a barrier that says whether the result may be written.
+template <typename T, bool WORDS_IN, typename G, typename F>
+__device__ __forceinline__ bool linear_job(const LinearArgs& a, int tile, int col_tiles, const uint64_t* xw, uint64_t* yw, uint32_t tag, G&& begin, F&& ready) {
+  constexpr int V = elem_traits<T>::vec16, DEPTH = 4 * V, MAXS = 4, W = kThreads / 64;
+  typedef vec<T, V> vt;
+  typedef vec<float, V> vf;
+  auto& red = linear_lds().red;
+  auto& ssq = linear_lds().ssq;
+  const int lane = lane_id(), wave = wave_id(), c = lane & 15, g = lane >> 4;
+  const int n0 = tile % col_tiles * a.cols, m0 = tile / col_tiles * a.rows;
+  const int n_end = min(a.N, n0 + a.cols), m_end = min(a.M, m0 + a.rows), row = m0 + c;
+  const int steps = (a.K + DEPTH - 1) / DEPTH;
+  const int per = (steps + W - 1) / W;
+  const int s_end = min(steps, (wave + 1) * per);
+  const T* wr = static_cast<const T*>(a.w) + (int64_t)(n0 + c) * a.ldw;
+  const T* norm_w = static_cast<const T*>(a.norm_w);
+  acc4_t acc = {0.f, 0.f, 0.f, 0.f};
+  float sq = 0.f;
+  vt fb[MAXS];
+  auto weights = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < MAXS; ++u) {
+      const int kk = DEPTH * (s0 + u) + V * g;
+#pragma unroll
+      for (int e = 0; e < V; ++e) fb[u][e] = (T)0.f;
+      if (s0 + u < s_end && kk < a.K && n0 + c < n_end) fb[u] = *reinterpret_cast<const vt*>(wr + kk);   // K is a multiple of V
+    }
+  };
+  weights(wave * per);
+  if constexpr (WORDS_IN) begin();
+  bool came = true;
+  for (int s0 = wave * per; s0 < s_end; s0 += MAXS) {
+    vt fa[MAXS], fg[MAXS];
+    if constexpr (WORDS_IN) {
+      // the first piece until it is there, then the others together: polling all of them would take 32 KB a round
+      auto at = [&](int u) __attribute__((always_inline)) {
+        const int kk = DEPTH * (s0 + u) + V * g;
+        return s0 + u < s_end && kk < a.K && row < m_end ? xw + ((int64_t)row * a.K + kk) / kPerWord<T> : nullptr;
+      };
+      const uint64_t* const first[1] = {at(0)};
+      const uint64_t* const rest[MAXS - 1] = {at(1), at(2), at(3)};
+      vt x0[1], xr[MAXS - 1];
+      came = came && wait_words<T>(first, tag, x0) && wait_words<T>(rest, tag, xr);
+      fa[0] = x0[0];
+#pragma unroll
+      for (int u = 1; u < MAXS; ++u) fa[u] = xr[u - 1];
+    } else {
+#pragma unroll
+      for (int u = 0; u < MAXS; ++u) {
+        const int kk = DEPTH * (s0 + u) + V * g;
+        const bool in = s0 + u < s_end && kk < a.K;
+#pragma unroll
+        for (int e = 0; e < V; ++e) { fa[u][e] = (T)0.f; fg[u][e] = (T)0.f; }
+        if (in && norm_w != nullptr) fg[u] = *reinterpret_cast<const vt*>(norm_w + kk);
+        if (in && row < m_end) fa[u] = *reinterpret_cast<const vt*>(static_cast<const T*>(a.x) + (int64_t)row * a.ldx + kk);
+      }
+      begin();
+      if (norm_w != nullptr) {
+#pragma unroll
+        for (int u = 0; u < MAXS; ++u) {
+          const vf xv = __builtin_convertvector(fa[u], vf), gv = __builtin_convertvector(fg[u], vf);
+#pragma unroll
+          for (int e = 0; e < V; ++e) sq = __builtin_fmaf(xv[e], xv[e], sq);
+          fa[u] = __builtin_convertvector(xv * gv, vt);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < MAXS; ++u) mma16(acc, fa[u], fb[u]);
+    weights(s0 + MAXS);
+  }
+  asm volatile("s_nop 15" ::: "memory");   // the loop may end right behind a product
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[wave][4 * g + r][c] = acc[r];
+  if (!WORDS_IN && norm_w != nullptr) {   // the four contraction pieces of a row
+    sq += __shfl_xor(sq, 16);
+    sq += __shfl_xor(sq, 32);
+    if (g == 0) ssq[wave][c] = sq;
+  }
+  if (!ready(came)) return false;
+  constexpr int E = WORDS_IN ? 1 : kPerWord<T>;   // columns of a thread
+  const int o = threadIdx.x;
+  if (o < 256 / E) {
+    const int rr = o / (16 / E), col = o % (16 / E) * E;
+    float s[E];
+    float scale = 1.f;
+    if (!WORDS_IN && norm_w != nullptr) {
+      float t = 0.f;
+#pragma unroll
+      for (int v = 0; v < W; ++v) t += ssq[v][rr];
+      scale = __builtin_amdgcn_rsqf(t / (float)a.K + a.eps);
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      s[e] = 0.f;
+#pragma unroll
+      for (int v = 0; v < W; ++v) s[e] += red[v][rr][col + e];
+      if (!WORDS_IN && norm_w != nullptr) s[e] *= scale;
+    }
+    if (m0 + rr < m_end && n0 + col < n_end) {
+      if constexpr (WORDS_IN) {
+        if (a.res != nullptr) s[0] += (float)static_cast<const T*>(a.res)[(int64_t)(m0 + rr) * a.ldr + n0 + col];
+        static_cast<T*>(a.y)[(int64_t)(m0 + rr) * a.ldy + n0 + col] = (T)s[0];
+      } else {
+        uint32_t payload;
+        if constexpr (E == 2) payload = __builtin_bit_cast(uint32_t, vec<T, 2>{(T)s[0], (T)s[1]});
+        else payload = __builtin_bit_cast(uint32_t, s[0]);
+        store_word(yw + ((int64_t)(m0 + rr) * a.N + n0 + col) / kPerWord<T>, payload, tag);
+      }
+    }
+  }
+  return true;
+}
+
+template <typename T, int HD, bool UH>
+__global__ __launch_bounds__(kThreads, kLayerGroups) void decode_layer_kernel(LayerArgs args) {
+  __shared__ int s_mine, s_came[kThreads / 64], s_job;
+  const int own = blockIdx.x;
+  uint32_t* const claims = args.control + kClaims;
+  const uint32_t tag = args.control[0] + 1;
+  bool claimed = false, mine = true;   // mine, of thread 0: the claim's answer
+  // behind the first loads of a job: the tag is there by then, and the answer when the loads are
+  auto begin = [&] __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (!claimed && threadIdx.x == 0) mine = claim_job(claims, own, tag);
+    claimed = true;
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  enum { kTaken, kGo, kLater };   // another workgroup has the job; it may go on; something it needs is missing
+  int answer = kGo;
+  auto agree = [&](bool came) __attribute__((always_inline)) {
+    if (threadIdx.x == 0) s_mine = mine;
+    if (lane_id() == 0) s_came[wave_id()] = came;
+    __syncthreads();
+    bool all = true;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) all = all && s_came[w];
+    answer = __builtin_amdgcn_readfirstlane(!s_mine ? kTaken : all ? kGo : kLater);
+    return answer == kGo;
+  };
+  auto run = [&](const LayerArgs& f, int job) __attribute__((always_inline)) {
+    const int stream = job - f.n_in, out = stream - f.n_stream;
+    if (stream < 0) {
+      linear_job<T, false>(f.in, job, f.in_cols, nullptr, f.proj, tag, begin, agree);
+    } else if (out < 0) {
+      const int split = stream % f.d.splits;
+      const TokenWords words = {f.proj, f.merged, f.part, tag};
+      stream_job<T, HD, UH, false, true>(f.d, split, stream / f.d.splits, words, begin, [&](bool came) {
+        // the last split waits for the others' partial results when its own rows are done: they have to be claimed by now
+        if (split == f.d.splits - 1) came = came && jobs_claimed(claims + job - split, split, tag);
+        return agree(came);
+      });
+    } else {
+      linear_job<T, true>(f.out, out, f.out_cols, f.merged, nullptr, tag, begin, agree);
+    }
+  };
+  run(args, own);
+  int job = own;
+  for (int tries = 0; (job != own || answer == kLater) && tries < kTries; ++tries) {
+    // The arguments are read where a job needs them: read ahead of the loop, 160 scalar and 80 vector registers spill.
+    const __attribute__((address_space(4))) LayerArgs* kernarg = (const __attribute__((address_space(4))) LayerArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kernarg));
+    __syncthreads();   // what the last job kept in LDS is read
+    if (job == own || answer != kLater) {   // (a job once taken is run until it is done)
+      if (wave_id() == 0) {
+        const int j = take_job(claims, own, tag);
+        if (threadIdx.x == 0) s_job = j;
+      }
+      __syncthreads();
+      job = __builtin_amdgcn_readfirstlane(s_job);
+      if (job < 0) job = own;
+    }
+    run(*(const LayerArgs*)kernarg, job);
+  }
+  if (threadIdx.x == 0) {
+    const int groups = min(kExitGroups, (int)gridDim.x), g = blockIdx.x % kExitGroups;
+    const int members = ((int)gridDim.x - g + kExitGroups - 1) / kExitGroups;
+    uint32_t* const gone = args.control + kGoneGroup + g * kLine;
+    auto add = [](uint32_t* p) { return (int)__hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    auto set = [](uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    if (add(gone) == members - 1) {
+      set(gone, 0);
+      if (add(args.control + kGone) == groups - 1) {
+        set(args.control + kGone, 0);
+        set(args.control, tag);
+      }
+    }
+  }
+}
+
+static int64_t word_count(int64_t elements, int es) { return elements * es / 4; }
+int64_t decode_layer_control_bytes(int B, int H, int d, int es) {
+  return (kClaims + kLayerJobs) * 4 + 8 * (word_count((int64_t)B * 6 * H * d, es) + word_count((int64_t)B * H * d, es) + (int64_t)kLayerJobs * (d + 2));
+}
+
+// Rows x columns (at most 16 x 16) of a job: small ones while that leaves no CU a second
+static void pick_job_tile(LinearArgs& a) {
+  a.rows = a.cols = 16;
+  for (int r = 8; r <= 16; r *= 2)
+    for (int c = 8; c <= 16; c *= 2) {
+      const int64_t groups = (int64_t)((a.M + r - 1) / r) * ((a.N + c - 1) / c);
+      if (groups <= 128 && std::min(r, a.M) + c < std::min(a.rows, a.M) + a.cols) { a.rows = r; a.cols = c; }
+    }
+}
+template <typename T, int HD> static int launch_layer_t(const LayerArgs& f, hipStream_t stream) {
+  ProfScope ps(kSlotDecodeStream, stream);
+  const dim3 grid(f.n_in + f.n_stream + f.n_out), block(kThreads);
+  constexpr int lds = kEarly * kEarlyIteration;
+  if constexpr (__is_same(T, bf16_t)) {
+    if (f.d.u_half) hipLaunchKernelGGL((decode_layer_kernel<T, HD, true>), grid, block, lds, stream, f);
+    else hipLaunchKernelGGL((decode_layer_kernel<T, HD, false>), grid, block, lds, stream, f);
+  } else {
+    hipLaunchKernelGGL((decode_layer_kernel<T, HD, false>), grid, block, lds, stream, f);
+  }
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+template <typename T> static int launch_layer_d(const LayerArgs& f, hipStream_t stream) {
+  switch (f.d.d) {
+    case 16: return launch_layer_t<T, 16>(f, stream);
+    case 32: return launch_layer_t<T, 32>(f, stream);
+    case 64: return launch_layer_t<T, 64>(f, stream);
+    case 128: return launch_layer_t<T, 128>(f, stream);
+    default: return -2;
+  }
+}
+
+// 1: the step does not fit one launch (more workgroups than the GPU holds at once).
+int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, int dtype, int cus, hipStream_t stream) {
+  const int es = dtype == 0 ? 4 : 2;
+  LayerArgs f = {};
+  f.d = d;
+  f.in = {in.x, in.w, nullptr, in.M, in.N, in.K, in.ldx, in.ldw, 0, in.norm_w, in.eps, 0, nullptr, 0, 0, 0, nullptr, 0};
+  f.out = {nullptr, out.w, out.y, out.M, out.N, out.K, 0, out.ldw, out.ldy, nullptr, 0.f, 0, out.res, out.ldr, 0, 0, nullptr, 0};
+  pick_job_tile(f.in);
+  pick_job_tile(f.out);
+  f.in_cols = (in.N + f.in.cols - 1) / f.in.cols;
+  f.out_cols = (out.N + f.out.cols - 1) / f.out.cols;
+  const int64_t n_in = (int64_t)f.in_cols * ((in.M + f.in.rows - 1) / f.in.rows), n_out = (int64_t)f.out_cols * ((out.M + f.out.rows - 1) / f.out.rows);
+  const int64_t BH = (int64_t)d.B * d.H;
+  const int rows = kThreads * 16 / (d.d * es) * (kEarly + 1);   // of a split: what it requests ahead of the token
+  f.d.splits = d.t * (kEarly + 1) <= rows ? 1 : (d.t + rows - 1) / rows + 1;
+  if (d.t_dev != nullptr || 4 * BH * d.t * d.d * es > kLayerCacheBytes || f.d.splits > 64 || n_in + BH * f.d.splits > kLayerGroups * (int64_t)cus ||
+      n_in + BH * f.d.splits + n_out > kLayerJobs)
+    return 1;
+  f.n_in = (int)n_in;
+  f.n_out = (int)n_out;
+  f.n_stream = (int)BH * f.d.splits;
+  char* p = static_cast<char*>(control);
+  f.control = reinterpret_cast<uint32_t*>(p);
+  p += (kClaims + kLayerJobs) * 4;
+  f.proj = reinterpret_cast<uint64_t*>(p);
+  f.merged = f.proj + word_count((int64_t)d.B * in.N, es);
+  f.part = f.merged + word_count((int64_t)d.B * out.K, es);
+  switch (dtype) {
+    case 0: return launch_layer_d<float>(f, stream);
+    case 1: return launch_layer_d<bf16_t>(f, stream);
+    case 2: return launch_layer_d<fp16_t>(f, stream);
+    default: return -1;
+  }
 }
 
 // ---------------------------------------------------------------------------

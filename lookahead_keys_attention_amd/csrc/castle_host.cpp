@@ -974,16 +974,21 @@ class StepPlan {
     const double e = norm_eps(eps);
     // the projection is scratch of the step like the workspace: kept with it, an allocation costs more than a microsecond
     if (!proj_.defined()) proj_ = at::empty({B, 6 * inner}, x.options().requires_grad(false));
+    if (!control_.defined() && !t_device) {   // for the step as one launch
+      const int64_t n = check(castle_decode_layer_control_bytes(s_.B, s_.H, s_.d, s_.dtype), "castle_decode_layer_control_bytes");
+      control_ = at::zeros({n}, x.options().dtype(at::kByte).requires_grad(false));
+    }
     used_on_current_stream();
     Tensor y = at::empty({B, 1, dim}, x.options());
     const castle_view4* c = views_;
     castle_deferred def = deferred(base, base_device);
-    check(castle_decode_layer(c, c + 1, c + 2, c + 3, (int)t, t_device ? count_ptr(t_device) : nullptr, s_.L, xr.data_ptr(), xr.stride(0), (int)dim,
+    check(castle_decode_layer_once(c, c + 1, c + 2, c + 3, (int)t, t_device ? count_ptr(t_device) : nullptr, s_.L, xr.data_ptr(), xr.stride(0), (int)dim,
                               nw.defined() ? nw.data_ptr() : nullptr, (float)e, w_qkv.data_ptr(), w_qkv.stride(0), w_out.data_ptr(),
                               w_out.stride(0), res.defined() ? res.data_ptr() : nullptr, res.defined() ? res.stride(0) : 0, y.data_ptr(), dim,
                               proj_.data_ptr(), s_.B, s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0),
-                              base >= 0 || base_device ? &def : nullptr, workspace_.data_ptr(), workspace_.numel(), stream_of(x)),
-          "castle_decode_layer");
+                              base >= 0 || base_device ? &def : nullptr, workspace_.data_ptr(), workspace_.numel(), t_device ? nullptr : control_.data_ptr(),
+                                   t_device ? 0 : control_.numel(), stream_of(x)),
+          "castle_decode_layer_once");
     return y;
   }
 
@@ -992,15 +997,16 @@ class StepPlan {
   // stream that uses it, or it hands the memory of a dropped cache out again before a step on that stream is through.
   void used_on_current_stream() {
     const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(buffers_[0].get_device());
-    if (stream_ && *stream_ == stream && recorded_proj_ == proj_.defined()) return;
+    if (stream_ && *stream_ == stream && recorded_proj_ == proj_.defined() && recorded_control_ == control_.defined()) return;
     // (straight to the allocator: record_stream costs a microsecond a tensor)
     auto record = [&](const Tensor& t) {
       if (t.defined()) c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::recordStreamMasqueradingAsCUDA(t.storage().data_ptr(), stream);
     };
     for (const Tensor& t : buffers_) record(t);
-    for (const Tensor* t : {&ring_, &gates_, &workspace_, &proj_}) record(*t);
+    for (const Tensor* t : {&ring_, &gates_, &workspace_, &proj_, &control_}) record(*t);
     stream_ = stream;
     recorded_proj_ = proj_.defined();
+    recorded_control_ = control_.defined();
   }
   static const int32_t* count_ptr(const std::optional<Tensor>& t) { return static_cast<const int32_t*>(t->data_ptr()); }
   void check_count(int64_t t, const std::optional<Tensor>& t_device) const {
@@ -1019,9 +1025,9 @@ class StepPlan {
   }
 
   std::vector<Tensor> buffers_;
-  Tensor ring_, gates_, workspace_, proj_;
+  Tensor ring_, gates_, workspace_, proj_, control_;
   std::optional<c10::hip::HIPStreamMasqueradingAsCUDA> stream_;   // of the last step
-  bool recorded_proj_ = false;
+  bool recorded_proj_ = false, recorded_control_ = false;
   castle_view4 views_[4];
   castle_deferred deferred_;
   Shape s_;

@@ -121,6 +121,17 @@ struct DecodeArgs {
   int base0;                // rows of U are complete up to source base0 - 1 at least (e.g. the prefill length)
   const int* base0_dev;     // the same from device memory (graph replay): base0_dev[0]
 };
+// one of the two products around a cached step of a whole layer
+struct DecodeLinear {
+  const void *x, *w;
+  void* y;
+  int M, N, K;
+  int64_t ldx, ldw, ldy;
+  const void* norm_w;
+  float eps;
+  const void* res;
+  int64_t ldr;
+};
 // first source not yet folded into the stored lookahead keys when the cache holds t rows
 __host__ __device__ inline int decode_base(int base0, int t) {
   const int b = t - t % kDecodeDefer;

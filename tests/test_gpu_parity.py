@@ -483,6 +483,60 @@ def test_layer_step_equals_its_parts(B, dim, Hh, d, t, dtype):
         assert_close(a[:, :, t:t + 1].float(), b[:, :, t:t + 1].float().cpu().double(), dtype, "appended row", 1e-4)
 
 
+@pytest.mark.parametrize("B,dim,Hh,d,t0,dtype,rotary", [(1, 96, 1, 16, 0, torch.float32, True), (2, 512, 3, 64, 30, torch.bfloat16, True), (3, 200, 2, 32, 189, torch.float16, False),
+                                                       (17, 264, 2, 64, 94, torch.bfloat16, False), (1, 136, 2, 128, 93, torch.bfloat16, True), (2, 1100, 2, 64, 700, torch.float32, False)])
+def test_layer_step_in_one_launch_equals_three(B, dim, Hh, d, t0, dtype, rotary):
+    """castle_decode_layer_once with its control words against castle_decode_layer over consecutive steps on caches of their own: around
+    whole iterations of a split (32 rows at d = 64 and 16 bit, three to a split) and with the write-back every fourth step.  Both
+    round the projection and the attention output to the tensor type, so what differs is the order of 32-bit sums; a value of a 16-bit
+    tensor in between may then round the other way: two roundings of 2^-8 (bf16) through the output projection and the store."""
+    import ctypes
+
+    from lookahead_keys_attention_amd import _native as N, ops
+    from lookahead_keys_attention_amd.castle import _CacheStore
+
+    lib, steps = ctypes.CDLL(N.LIB_PATH), 9
+    lib.castle_decode_layer_control_bytes.restype = ctypes.c_int64
+    g = torch.Generator(device=DEV).manual_seed(B + dim)
+    rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
+    norm_w, res = 1 + rnd(dim, std=0.2), rnd(B, 1, dim)
+    w_in, w_out = rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5)
+    code, u_half = N.DTYPE_CODES[dtype], dtype == torch.bfloat16
+    control = torch.zeros(lib.castle_decode_layer_control_bytes(B, Hh, d, code), dtype=torch.uint8, device=DEV)
+    stores = [_CacheStore(B, Hh, d, t0 + steps, dtype, torch.device(DEV)) for _ in range(2)]
+    for i in range(4):
+        rows = rnd(B, Hh, t0, d, std=0.6)
+        for store in stores:
+            store.buffers[i].zero_()
+            store.buffers[i][:, :, :t0] = rows.to(torch.float16).view(dtype) if i == 0 and u_half else rows
+    proj = torch.empty(B, 6 * Hh * d, dtype=dtype, device=DEV)
+    flags = (N.FLAG_ROTARY if rotary else 0) | (N.FLAG_U_HALF if u_half else 0)
+    vp, i64 = ctypes.c_void_p, ctypes.c_int64
+    for step in range(steps):
+        x, ys = rnd(B, 1, dim), []
+        for store, words in zip(stores, (control, None)):
+            y = torch.empty(B, 1, dim, dtype=dtype, device=DEV)
+            views = [ctypes.byref(v) for v in store.views]
+            deferred = ops.make_deferred(store.rings[0], store.rings[1], t0)
+            rc = lib.castle_decode_layer_once(
+                *views, t0 + step, None, t0 + steps, vp(x.data_ptr()), i64(dim), dim, vp(norm_w.data_ptr()), ctypes.c_float(1e-5), vp(w_in.data_ptr()), i64(dim),
+                vp(w_out.data_ptr()), i64(Hh * d), vp(res.data_ptr()), i64(dim), vp(y.data_ptr()), i64(dim), vp(proj.data_ptr()), B, Hh, d, code,
+                ctypes.c_float(d ** -0.5), flags, ctypes.byref(deferred), vp(store.workspace.data_ptr()), i64(store.workspace.numel()),
+                vp(words.data_ptr() if words is not None else None), i64(words.numel() if words is not None else 0),
+                vp(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0
+            ys.append(y.double())
+        scale = ys[1].abs().max().item()
+        assert (ys[0] - ys[1]).abs().max().item() <= scale * {torch.float32: 1e-4, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype], step
+    for a, b in zip(stores[0].buffers[1:], stores[1].buffers[1:]):
+        assert_close(a.float(), b.float().cpu().double(), dtype, "cached rows", 1e-4)
+    if u_half:
+        a, b = (store.buffers[0].view(torch.float16).float() for store in stores)
+    else:
+        a, b = (store.buffers[0].float() for store in stores)
+    assert_close(a, b.cpu().double(), dtype, "lookahead keys", 1e-4)
+
+
 @pytest.mark.parametrize("B,Hh,t0,steps,d,dtype,rotary", [(2, 2, 0, 23, 64, torch.float32, False), (1, 2, 101, 18, 32, torch.float32, True),
                                                         (2, 2, 203, 21, 64, torch.bfloat16, False), (1, 2, 130, 9, 128, torch.bfloat16, True)])
 def test_decode_with_deferred_write_back(B, Hh, t0, steps, d, dtype, rotary):
