@@ -50,7 +50,7 @@ template <typename T> __device__ __forceinline__ float gelu_slope(float x) {
 
 // A tile of FREE rows / columns and BK steps of the contraction: global -> registers -> LDS -> operand fragments.
 // KC: the operand is contraction-contiguous (LDS [FREE][BK]), else stored [contraction][free] (LDS [BK][FREE]).
-template <typename T, bool KC, int FREE, int BK> struct Operand {
+template <typename T, bool KC, int FREE, int BK, int G> struct Operand {
   static constexpr int V = elem_traits<T>::vec16;
   static constexpr int COLS = KC ? BK : FREE, ROWS = KC ? FREE : BK, VPR = COLS / V, N = ROWS * VPR / kThreads;
   static constexpr int LD = KC ? lds_ld<T>(COLS) : lds_ld_tr<T>(COLS), ELEMS = ROWS * LD;
@@ -61,8 +61,8 @@ template <typename T, bool KC, int FREE, int BK> struct Operand {
   // data: those outputs are not stored.
   int at[N];
   vt r[2][N];
-  static __device__ __forceinline__ int row_of(int j) { return (threadIdx.x + j * kThreads) / VPR; }
-  static __device__ __forceinline__ int col_of(int j) { return (threadIdx.x + j * kThreads) % VPR * V; }
+  static __device__ __forceinline__ int row_of(int j) { return (threadIdx.x % kThreads + j * kThreads) / VPR; }
+  static __device__ __forceinline__ int col_of(int j) { return (threadIdx.x % kThreads + j * kThreads) % VPR * V; }
   __device__ __forceinline__ void start(int ld, int free0, int free_end, int k0) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -83,7 +83,7 @@ template <typename T, bool KC, int FREE, int BK> struct Operand {
       }
     }
 #pragma unroll
-    for (int j = 0; j < N; ++j) at[j] += KC ? BK : BK * ld;
+    for (int j = 0; j < N; ++j) at[j] += KC ? G * BK : G * BK * ld;
   }
   __device__ __forceinline__ void store(int slot, T* lds) const {
 #pragma unroll
@@ -95,15 +95,17 @@ template <typename T, bool KC, int FREE, int BK> struct Operand {
   }
 };
 
-template <typename T, bool AK, bool BKC, int BM, int BN, int BK>
-__global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmArgs a) {
+// G: groups of four waves.  Two take alternate steps of the contraction for the same tile, each in LDS of its own, and are summed at
+// the end: where the tiles leave a CU one workgroup, a second wave per SIMD works while the first waits for LDS and barrier.
+template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G>
+__global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(GemmArgs a) {
   constexpr int WM = BM / 64, WN = BN / 64;   // 32-wide pieces of a wave's quarter
-  typedef Operand<T, AK, BM, BK> OpA;
-  typedef Operand<T, BKC, BN, BK> OpB;
+  typedef Operand<T, AK, BM, BK, G> OpA;
+  typedef Operand<T, BKC, BN, BK, G> OpB;
   constexpr int V = elem_traits<T>::vec16, LDC = BN + V;
   constexpr int kStage = 2 * (OpA::ELEMS + OpB::ELEMS), kOut = BM * LDC;
-  __shared__ __attribute__((aligned(16))) T smem[kStage > kOut ? kStage : kOut];
-  const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
+  __shared__ __attribute__((aligned(16))) T smem[G * kStage > kOut ? G * kStage : kOut];
+  const int lane = lane_id(), wave = wave_id() % 4, group = wave_id() / 4, c = lane & 31, g = lane >> 5;
   // Workgroups go round the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the tiles, so the rows of
   // `a` are read by one XCD, not by all (input gradient of 3000 rows x 1536 x 256: 13.5 -> 11.1 us).  A workgroup takes
   // several tiles where there are more than the CUs hold: the first steps of the next are requested before the
@@ -112,30 +114,31 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
   const int share = (tiles + 7) / 8, first = blockIdx.x % 8 * share, last = min(tiles, first + share);
   const int wm = wave / 2 * (BM / 2), wn = wave % 2 * (BN / 2);
   const int k0 = blockIdx.y * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split);
-  const int steps = (k_end - k0 + BK - 1) / BK;
+  const int steps = ((k_end - k0 + BK - 1) / BK + G - 1) / G;   // of a group: its steps are G BK apart
+  T* const stage = smem + group * kStage;
   const T *pa = static_cast<const T*>(a.a), *pb = static_cast<const T*>(a.b);
   OpA ra;
   OpB rb;
   acc_t acc[WM][WN];   // [n rows, m lanes]
   int tile = first + blockIdx.x / 8;
   auto request = [&]() __attribute__((always_inline)) {
-    ra.start((int)a.lda, tile / tiles_n * BM, a.M, k0);
-    rb.start((int)a.ldb, tile % tiles_n * BN, a.N, k0);
+    ra.start((int)a.lda, tile / tiles_n * BM, a.M, k0 + group * BK);
+    rb.start((int)a.ldb, tile % tiles_n * BN, a.N, k0 + group * BK);
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {   // (a second step beyond the end loads zeros)
-      ra.load(p, pa, (int)a.lda, k0 + p * BK, k_end);
-      rb.load(p, pb, (int)a.ldb, k0 + p * BK, k_end);
+    for (int p = 0; p < 2; ++p) {   // (a step beyond the end loads zeros)
+      ra.load(p, pa, (int)a.lda, k0 + (p * G + group) * BK, k_end);
+      rb.load(p, pb, (int)a.ldb, k0 + (p * G + group) * BK, k_end);
     }
   };
   auto step = [&](auto parity, int it) __attribute__((always_inline)) {
     constexpr int p = decltype(parity)::value;
-    T* la = smem + p * (OpA::ELEMS + OpB::ELEMS);
+    T* la = stage + p * (OpA::ELEMS + OpB::ELEMS);
     T* lb = la + OpA::ELEMS;
     ra.store(p, la);
     rb.store(p, lb);
     if (it + 2 < steps) {
-      ra.load(p, pa, (int)a.lda, k0 + (it + 2) * BK, k_end);
-      rb.load(p, pb, (int)a.ldb, k0 + (it + 2) * BK, k_end);
+      ra.load(p, pa, (int)a.lda, k0 + ((it + 2) * G + group) * BK, k_end);
+      rb.load(p, pb, (int)a.ldb, k0 + ((it + 2) * G + group) * BK, k_end);
     }
     __syncthreads();
 #pragma unroll
@@ -153,7 +156,7 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
   };
   const int amax_tile = a.amax_from / BN, amax_tiles = (a.amax_to - 1) / BN + 1 - amax_tile;   // of a row of tiles
   if (a.amax != nullptr && blockIdx.x == 0) {
-    for (int i = (a.M + BM - 1) / BM * amax_tiles + threadIdx.x; i < kAmaxBlocks; i += kThreads) a.amax[i] = 0.f;
+    for (int i = (a.M + BM - 1) / BM * amax_tiles + threadIdx.x; i < kAmaxBlocks; i += kThreads * G) a.amax[i] = 0.f;
     if (threadIdx.x == 0 && a.amax_status != nullptr) *a.amax_status = 0;
   }
   if (tile < last) request();
@@ -167,6 +170,31 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
       step(std::integral_constant<int, 0>(), it);
       if (it + 1 < steps) step(std::integral_constant<int, 1>(), it + 1);
     }
+    if constexpr (G == 2) {
+      typedef vec<float, 4> v4;
+      static_assert(kThreads * WM * WN * 64 <= (int)sizeof(smem), "one group's sums");
+      v4* sums = reinterpret_cast<v4*>(smem);
+      asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");   // the loop may end right behind a product
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();   // the operands of the last step are dead
+      if (group == 1) {
+#pragma unroll
+        for (int i = 0; i < WM * WN; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sums[(i * 4 + q) * kThreads + threadIdx.x % kThreads] = pack4<float>(acc[i / WN][i % WN], q);
+      }
+      __syncthreads();
+      if (group == 0) {
+#pragma unroll
+        for (int i = 0; i < WM * WN; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const v4 other = sums[(i * 4 + q) * kThreads + threadIdx.x];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i / WN][i % WN][4 * q + e] += other[e];
+          }
+      }
+    }
     tile += gridDim.x / 8;
     if (tile < last) request();
     if (a.part != nullptr) {   // partial product of this range of the contraction
@@ -178,13 +206,14 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const int m = m0 + wm + 32 * i + c, n = n0 + wn + 32 * j + 8 * q + 4 * g;
-            if (m < a.M && n < a.N) *reinterpret_cast<vec<float, 4>*>(part + (int64_t)m * a.N + n) = pack4<float>(acc[i][j], q);
+            if (group == 0 && m < a.M && n < a.N) *reinterpret_cast<vec<float, 4>*>(part + (int64_t)m * a.N + n) = pack4<float>(acc[i][j], q);
           }
       __syncthreads();   // the operands of the last step are dead
       continue;
     }
     // through LDS to whole rows
     __syncthreads();
+    if (group == 0)
 #pragma unroll
     for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -195,7 +224,7 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
     typedef vec<T, V> vt;
     typedef vec<float, V> vf;
     float most = 0.f;
-    for (int i = threadIdx.x; i < BM * (BN / V); i += kThreads) {
+    for (int i = threadIdx.x; i < BM * (BN / V); i += kThreads * G) {
       const int row = i / (BN / V), col = i % (BN / V) * V, m = m0 + row, n = n0 + col;
       if (m >= a.M || n >= a.N) continue;
       vt x = *reinterpret_cast<const vt*>(smem + row * LDC + col);
@@ -222,14 +251,14 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
     }
     const int slot = n0 / BN - amax_tile;
     if (a.amax != nullptr && slot >= 0 && slot < amax_tiles) {
-      __shared__ float s_most[kThreads / 64];
+      __shared__ float s_most[G * kThreads / 64];
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) most = fmaxf(most, __shfl_xor(most, o));
-      if (lane == 0) s_most[wave] = most;
+      if (lane == 0) s_most[wave_id()] = most;
       __syncthreads();
       if (threadIdx.x == 0) {
 #pragma unroll
-        for (int w = 1; w < kThreads / 64; ++w) most = fmaxf(most, s_most[w]);
+        for (int w = 1; w < G * kThreads / 64; ++w) most = fmaxf(most, s_most[w]);
         a.amax[m0 / BM * amax_tiles + slot] = fminf(most, 3.0e38f);   // an infinite value counts as the largest finite one
       }
     }
@@ -237,27 +266,30 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 4) void gemm_kernel(GemmA
   }
 }
 
-// Tile and number of ranges of the contraction, from what a launch takes (us, measured over 96 ... 5916 rows, outputs of
-// 128 ... 3072 columns and contractions of 128 ... 5916): 2.3, and per step of a workgroup 0.42 (64 x 64) or 0.95
-// (128 x 128) when it has a CU to itself, 0.32 or 0.9 when the CU has others; fp32 0.75 and 0.62.  A split adds a
-// second launch, 2.5, and its partial results, written and read.  3000 rows, 1536 x 256 out: 24.2 us in one range, 14.4 in the
-// four that this picks; the same product forward: 8.4 on 64 x 64 tiles, 9.5 on 128 x 128; 5916 rows of 512 -> 2048: 30.6
-// and 23.2.
+// Tile, number of ranges of the contraction and groups of a workgroup, from what a launch takes (us, measured over 96 ... 5916 rows,
+// outputs of 128 ... 3072 columns and contractions of 128 ... 5916): 2.3, and per step of a workgroup 0.42 (64 x 64) or 0.95
+// (128 x 128) when it has a CU to itself, 0.32 or 0.9 when the CU has others; fp32 0.78 and 0.62.  A second group takes a step of a
+// workgroup that has a CU to itself to 0.30, fp32 0.66, for 0.3 at the end (one range, one group / two: 3000 rows of 1536 -> 256
+// 12.7 / 9.9, 256 rows of fp32 512 -> 3072 15.1 / 13.1; level at two workgroups a CU, behind from three on: 3000 rows of 256 -> 1536 8.7
+// / 11.3).  A split adds a second launch, 2.5, and its partial results, written and read.  Weight gradient of 3000 rows, 1536 x
+// 256 out: 22.6 us in one range, 14.1 in two of two groups; 3000 rows 256 -> 1536 forward: 8.4 on 64 x 64 tiles, 9.5 on 128 x 128;
+// 5916 rows of 512 -> 2048: 30.6 and 23.2.
 struct Plan {
-  int tile, splits;
+  int tile, splits, groups;
 };
 Plan plan(int M, int N, int K, bool can_split, int elem_size) {
-  Plan best = {64, 1};
+  Plan best = {64, 1, 1};
   double best_cost = 1e30;
   for (int tile = 64; tile <= (elem_size == 2 ? 128 : 64); tile += 64) {
-    const double alone = elem_size == 4 ? 0.75 : tile == 64 ? 0.42 : 0.95, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.32 : 0.9;
+    const double alone = elem_size == 4 ? 0.78 : tile == 64 ? 0.42 : 0.95, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.32 : 0.9;
     const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
     const int steps = (K * elem_size + 127) / 128;   // 128 bytes of the contraction a step
     for (int s = 1; s <= (can_split ? std::min(16, (steps + 1) / 2) : 1); ++s) {
       const int64_t per_cu = (tiles * s + 255) / 256, n = (steps + s - 1) / s;
-      double cost = per_cu == 1 ? n * alone : per_cu * n * shared;
+      const int groups = tile == 64 && per_cu == 1 && n >= 4 ? 2 : 1;
+      double cost = groups == 2 ? 0.3 + n * (elem_size == 4 ? 0.66 : 0.30) : per_cu == 1 ? n * alone : per_cu * n * shared;
       if (s > 1) cost += 2.5 + (double)s * M * N * 8 / 4e6;
-      if (cost < best_cost) { best_cost = cost; best = {tile, s}; }
+      if (cost < best_cost) { best_cost = cost; best = {tile, s, groups}; }
     }
   }
   return best;
@@ -271,11 +303,12 @@ template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p,
   const dim3 grid(std::min((tiles + 7) / 8 * 8, p.tile == 128 ? 512 : 1024), p.splits);
   if constexpr (sizeof(T) == 2) {
     if (p.tile == 128) {
-      hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK>), grid, dim3(kThreads), 0, stream, a);
+      hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK, 1>), grid, dim3(kThreads), 0, stream, a);
       return hipGetLastError() == hipSuccess ? 0 : -3;
     }
   }
-  hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK>), grid, dim3(kThreads), 0, stream, a);
+  if (p.groups == 2) hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK, 2>), grid, dim3(2 * kThreads), 0, stream, a);
+  else hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK, 1>), grid, dim3(kThreads), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

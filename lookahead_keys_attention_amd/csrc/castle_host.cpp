@@ -462,11 +462,12 @@ Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epi
 // Own products where a call is short: the library's costs 18 us of host time, one here 4.  On the GPU they are level or
 // ahead up to the sizes below (us, own / library: 5916 rows 512 -> 2048 forward 23 / 33, 8192 rows 29 / 22; input gradient
 // of 1000 rows x 3072 x 512 15 / 16, 5916 x 2048 x 512 28 / 23; weight gradient of 3000 rows, 1536 x 256, 14 / 27, of
-// 5916, 2048 x 512, 32 / 41; fp32 is behind in all but the smallest, whose time is the host's).
+// 5916, 2048 x 512, 32 / 41).  In fp32 they are level up to the size below (256 rows, 512 <-> 3072: forward 13 / 13, input gradient 16 / 12,
+// weight gradient 15 / 16), where a layer's time is the host's; 2048 rows 60 / 53, 64 / 49, 72 / 55.
 bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16, double most_32) {
   return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
 }
-constexpr double kOwnForward = 14e9, kOwnInputGrad = 4e9, kOwnWeightGrad = 40e9, kOwn32 = 4e8;
+constexpr double kOwnForward = 14e9, kOwnInputGrad = 4e9, kOwnWeightGrad = 40e9, kOwn32 = 1e9;
 constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 70 / 83
 
 // The attention kernels behind a product begin with the largest element of some of its columns (vu of a fused projection, all

@@ -265,6 +265,16 @@ def test_products(rows, n, k, dtype):
     check(host().product(dy, False, w, True, 2, u), plain * slope, "slope")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,n,k", [(65, 72, 264), (130, 264, 328), (192, 64, 1000), (320, 512, 136)])
+def test_products_of_two_groups(rows, n, k, dtype):
+    """One tile a CU and a contraction of four steps and more: even and odd numbers of steps, a last one that is partly filled, one that
+    only the first group has."""
+    test_products(rows, n, k, dtype)
+    if dtype == torch.bfloat16 and n >= 64 and k >= 256:
+        test_product_leaves_partial_maxima(rows, n, k, 8, n - 16)
+
+
 def test_projection_of_rows_beyond_32_bit_offsets():
     """Rows that lie further apart than the products' offsets reach: 40000 of them, 65536 elements apart."""
     from lookahead_keys_attention_amd import Castle
