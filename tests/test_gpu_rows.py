@@ -271,7 +271,7 @@ def test_products_of_two_groups(rows, n, k, dtype):
     """One tile a CU and a contraction of four steps and more: even and odd numbers of steps, a last one that is partly filled, one that
     only the first group has."""
     test_products(rows, n, k, dtype)
-    if dtype == torch.bfloat16 and n >= 64 and k >= 256:
+    if dtype == torch.bfloat16 and 256 <= k < 512:   # (a longer contraction is split, and its maxima are not taken)
         test_product_leaves_partial_maxima(rows, n, k, 8, n - 16)
 
 
