@@ -74,6 +74,24 @@ template <int LPR> __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// Folds a value over the lanes that sit at the same place of the wave's groups of LPR lanes, in every lane, inside the vector unit
+// too: rotations of a row of 16, then exchanges of rows and of halves.  (Shuffles through LDS, 30 of them, took 0.3 us.)
+template <int LPR, typename Op> __device__ __forceinline__ float fold_groups(float v, Op&& op) {
+  auto turned = [&](auto ctrl) __attribute__((always_inline)) {
+    const int x = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  if constexpr (LPR <= 2) v = op(v, turned(std::integral_constant<int, 0x122>()));   // row_ror:2
+  if constexpr (LPR <= 4) v = op(v, turned(std::integral_constant<int, 0x124>()));   // row_ror:4
+  if constexpr (LPR <= 8) v = op(v, turned(std::integral_constant<int, 0x128>()));   // row_ror:8
+  if constexpr (LPR <= 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+    v = op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+  }
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  return op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
 // partial results of the split pass: the sums of all (b, h, split), then their statistics (maximum, sum of weights)
 __device__ __forceinline__ float* part_acc(const DecodeArgs& a, int bh, int split, int HD) {
   return a.part + ((int64_t)bh * a.splits + split) * HD;
@@ -152,7 +170,10 @@ template <typename T, int N> __device__ __forceinline__ bool wait_words(const ui
 // WORDS: a job of a launch that does the whole layer step (decode_layer_kernel below).  The token's pieces come as tagged
 // words, waited for behind the requests for the first rows, and the output leaves as such; ready(whether they came) says
 // whether the job goes on (if not, nothing has been written).
-template <typename T, int HD, bool UH, bool ONCE, bool WORDS, typename G, typename F>
+//
+// ALIKE: the six token views have strides in common, and so have the four caches.  Formed for each view by itself, the addresses
+// were 350 scalar instructions in front of the first request, most of a microsecond.
+template <typename T, int HD, bool UH, bool ONCE, bool WORDS, bool ALIKE, typename G, typename F>
 __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int bh, const TokenWords& words, G&& begin, F&& ready) {
   constexpr int V = elem_traits<T>::vec16;   // elements per 16-byte lane load
   constexpr int LPR = HD / V;                // lanes per row
@@ -165,48 +186,45 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
   const int b = bh / a.H, h = bh % a.H;
   const int tid = threadIdx.x;
   const int grp = tid / LPR, sub = tid % LPR;
-  // All loads of the start go out together, the small ones first (they are waited for first): the token's pieces,
-  // which do not need the row count, then the pending tokens' vu pieces and the rows of the first iteration.
+  // the counts of a replayed graph: on their way while the requests below are formed
+  int t = a.t_dev != nullptr ? *a.t_dev : a.t;
+  const int base0 = a.base0_dev != nullptr ? *a.base0_dev : a.base0;
+  const int64_t tok_at = (int64_t)b * a.ku.sb + (int64_t)h * a.ku.sh, cache_at = (int64_t)b * a.U.sb + (int64_t)h * a.U.sh;
+  auto tok = [&](const View4& v) __attribute__((always_inline)) {   // this lane's piece of the token
+    return reinterpret_cast<const vt*>((ALIKE ? reinterpret_cast<T*>(v.ptr) + tok_at : view_row<T>(v, b, h, 0)) + sub * V);
+  };
+  auto cached = [&](const View4& v, int k) __attribute__((always_inline)) {   // and of a cached row
+    return reinterpret_cast<vt*>((ALIKE ? reinterpret_cast<T*>(v.ptr) + cache_at + (int64_t)k * a.U.sl : view_row<T>(v, b, h, k)) + sub * V);
+  };
+  // All loads of the start go out together, the small ones first (they are waited for first): the token's pieces and the whole ring
+  // of pending vu pieces, which do not need the row count, then the rows of the first iteration.
   vt tku, tvu, tqc;
   if constexpr (!WORDS) {
-    tku = *reinterpret_cast<const vt*>(view_row<T>(a.ku, b, h, 0) + sub * V);
-    tvu = *reinterpret_cast<const vt*>(view_row<T>(a.vu, b, h, 0) + sub * V);
-    tqc = *reinterpret_cast<const vt*>(view_row<T>(a.qc, b, h, 0) + sub * V);
+    tku = *tok(a.ku);
+    tvu = *tok(a.vu);
+    tqc = *tok(a.qc);
   }
-  int t = a.t_dev != nullptr ? *a.t_dev : a.t;
+  const bool deferred = a.pend_vu.ptr != nullptr;
+  vt tpv[kDecodeDefer];
+#pragma unroll
+  for (int sl = 0; sl < kDecodeDefer; ++sl) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
+    if (deferred) tpv[sl] = *reinterpret_cast<const vt*>(view_row<T>(a.pend_vu, b, h, sl) + sub * V);
+  }
   const bool in_range = t >= 0 && t < a.capacity;
   if (!in_range) t = 0;   // only with a device-side count: no rows, nothing is appended
-  const float c1 = a.scale * kLog2e;
-
   // rows of this workgroup: [r0, r1), whole iterations of RPI rows.  With WORDS the last split has none (unless it is the only
   // one): it has the appended row to see to, and the partial results of the others.
   const int with_rows = WORDS && a.splits > 1 ? a.splits - 1 : a.splits;
   const int per = ((t + with_rows - 1) / with_rows + RPI - 1) / RPI * RPI;
   const int r0 = split * per;
   const int r1 = min(t, r0 + per);
-
   // deferred write-back: how many tokens are pending, and whether this step writes U
-  const bool deferred = a.pend_vu.ptr != nullptr;
-  const int base0 = a.base0_dev != nullptr ? *a.base0_dev : a.base0;
   const int pbase = deferred ? decode_base(base0, t) : t;
   const int np = t - pbase;                                        // 0 .. kDecodeDefer - 1
   const bool write_u = !deferred || (t + 1) % kDecodeDefer == 0;
-  const bool owner = split == (WORDS ? a.splits - 1 : t > 0 ? (t - 1) / per : 0);
-  vt tkc, tqu, tvc, tpv[kDecodeDefer];
-  if (!WORDS && owner) {
-    tkc = *reinterpret_cast<const vt*>(view_row<T>(a.kc, b, h, 0) + sub * V);
-    tqu = *reinterpret_cast<const vt*>(view_row<T>(a.qu, b, h, 0) + sub * V);
-    tvc = *reinterpret_cast<const vt*>(view_row<T>(a.vc, b, h, 0) + sub * V);
-  }
-  int pend_j[kDecodeDefer];   // the token in a ring slot, or -1: a row k has a gate for token j if k < j
-#pragma unroll
-  for (int sl = 0; sl < kDecodeDefer; ++sl) {
-    const int j = pbase + ((sl - pbase % kDecodeDefer + kDecodeDefer) % kDecodeDefer);   // the token that would sit in this slot
-    pend_j[sl] = deferred && j < t ? j : -1;
-#pragma unroll
-    for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
-    if (pend_j[sl] >= 0) tpv[sl] = *reinterpret_cast<const vt*>(view_row<T>(a.pend_vu, b, h, sl) + sub * V);
-  }
+  const bool owner = split == (WORDS ? a.splits - 1 : t > 0 ? (t - 1) / per : 0);   // of the appended row
   // The row pieces of the next iteration are requested before the current one is processed.  While the token is
   // still being projected (WORDS) those of the first `early` iterations are on their way too, straight into LDS: a lane reads
   // back what it asked for.
@@ -223,10 +241,10 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
   };
   auto request = [&](int k) __attribute__((always_inline)) {
     if (k < r1) {
-      nq = read(reinterpret_cast<const vt*>(view_row<T>(a.qu_cache, b, h, k) + sub * V));
-      nu = read(reinterpret_cast<const vt*>(view_row<T>(a.U, b, h, k) + sub * V));
-      nk = read(reinterpret_cast<const vt*>(view_row<T>(a.kc_cache, b, h, k) + sub * V));
-      nv = read(reinterpret_cast<const vt*>(view_row<T>(a.vc_cache, b, h, k) + sub * V));
+      nq = read(cached(a.qu_cache, k));
+      nu = read(cached(a.U, k));
+      nk = read(cached(a.kc_cache, k));
+      nv = read(cached(a.vc_cache, k));
       if (np > 0) ng = read(reinterpret_cast<const vec<float, 4>*>(gbase + (int64_t)k * kDecodeDefer));
     }
   };
@@ -235,16 +253,24 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
       const int k = r0 + grp + n * RPI;
       if (k < r1) {
         unsigned char* const to = early_rows(n, 0);
-        load_lds16<ONCE>(view_row<T>(a.qu_cache, b, h, k) + sub * V, to);
-        load_lds16<ONCE>(view_row<T>(a.U, b, h, k) + sub * V, to + kEarlyTensor);
-        load_lds16<ONCE>(view_row<T>(a.kc_cache, b, h, k) + sub * V, to + 2 * kEarlyTensor);
-        load_lds16<ONCE>(view_row<T>(a.vc_cache, b, h, k) + sub * V, to + 3 * kEarlyTensor);
+        load_lds16<ONCE>(cached(a.qu_cache, k), to);
+        load_lds16<ONCE>(cached(a.U, k), to + kEarlyTensor);
+        load_lds16<ONCE>(cached(a.kc_cache, k), to + 2 * kEarlyTensor);
+        load_lds16<ONCE>(cached(a.vc_cache, k), to + 3 * kEarlyTensor);
         if (np > 0) load_lds16<ONCE>(gbase + (int64_t)k * kDecodeDefer, to + 4 * kEarlyTensor);
       }
     }
   }
   request(r0 + grp + early * RPI);
   __builtin_amdgcn_sched_barrier(0);
+  const float c1 = a.scale * kLog2e;
+  vt tkc, tqu, tvc;
+  int pend_j[kDecodeDefer];   // the token in a ring slot, or -1: a row k has a gate for token j if k < j
+#pragma unroll
+  for (int sl = 0; sl < kDecodeDefer; ++sl) {
+    const int j = pbase + ((sl - pbase % kDecodeDefer + kDecodeDefer) % kDecodeDefer);   // the token that would sit in this slot
+    pend_j[sl] = deferred && j < t ? j : -1;
+  }
   if constexpr (WORDS) {
     begin();
     const uint64_t* w = words.proj + ((int64_t)b * 6 * a.H + h) * (HD / kPerWord<T>) + sub * 4;   // parts qu, ku, vu, qc, kc, vc
@@ -256,6 +282,12 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
     if (owner) { tkc = got[3]; tqu = got[4]; tvc = got[5]; }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the early rows are in LDS (requested in front of the words, they came first)
   }
+#pragma unroll
+  for (int sl = 0; sl < kDecodeDefer; ++sl)
+    if (pend_j[sl] < 0) {   // whatever an empty slot holds
+#pragma unroll
+      for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
+    }
   float ku[V], qc[V], acc[V], m = -INFINITY, l = 0.f;   // ku, qc times c1: products come out in log2 units
   float cvu[kDecodeDefer], cvu_t;                       // c1 qc . vu of the pending tokens and of the new one
   const int slot_t = t % kDecodeDefer;
@@ -300,36 +332,6 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
         s_vu[kDecodeDefer][sub * V + e] = vu[e];
       }
     }
-    // The last split that has rows takes row t too: U_t = 0, so its lookahead term is silu(0) = 0, and appends the
-    // new rows.  No workgroup of this launch reads row t or the ring slot of token t.
-    if (owner && grp == 0) {
-      float kct[V], qut[V];
-#pragma unroll
-      for (int e = 0; e < V; ++e) { kct[e] = (float)tkc[e]; qut[e] = (float)tqu[e]; acc[e] = (float)tvc[e]; }
-      if (a.rotary) {
-#pragma unroll
-        for (int e = 0; e < V / 2; ++e) {
-          const int pair = sub * (V / 2) + e;
-          CASTLE_ROPE_PAIR(kct[2 * e], kct[2 * e + 1], (float)t, pair, HD, false);
-          CASTLE_ROPE_PAIR(qut[2 * e], qut[2 * e + 1], (float)t, pair, HD, false);
-        }
-      }
-      float dot = 0.f;
-#pragma unroll
-      for (int e = 0; e < V; ++e) dot = __builtin_fmaf(qc[e], kct[e], dot);
-      m = group_sum<LPR>(dot);
-      l = 1.f;
-      if (in_range) {
-        vt z, q, kk, v, p;
-#pragma unroll
-        for (int e = 0; e < V; ++e) { z[e] = (T)0.f; q[e] = (T)qut[e]; kk[e] = (T)kct[e]; v[e] = (T)acc[e]; p[e] = (T)vu[e]; }
-        *reinterpret_cast<vt*>(view_row<T>(a.U, b, h, t) + sub * V) = z;
-        *reinterpret_cast<vt*>(view_row<T>(a.qu_cache, b, h, t) + sub * V) = q;
-        *reinterpret_cast<vt*>(view_row<T>(a.kc_cache, b, h, t) + sub * V) = kk;
-        *reinterpret_cast<vt*>(view_row<T>(a.vc_cache, b, h, t) + sub * V) = v;
-        if (deferred) *reinterpret_cast<vt*>(view_row<T>(a.pend_vu, b, h, slot_t) + sub * V) = p;   // joins the pending sources
-      }
-    }
   }
 
   auto rows = [&](auto writes) __attribute__((always_inline)) {
@@ -371,7 +373,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
         }
         // the lookahead key as later steps will see it: the stored (rounded) one
         const vt unew = u_pack<T, V, UH>(uk);
-        *reinterpret_cast<vt*>(view_row<T>(a.U, b, h, k) + sub * V) = unew;
+        *cached(a.U, k) = unew;
         u_unpack<T, V, UH>(unew, uk);
 #pragma unroll
         for (int e = 0; e < V; ++e) dsu = __builtin_fmaf(qc[e], uk[e], dsu);
@@ -407,21 +409,56 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
   } else {
     rows(std::false_type());
   }
+  // The owner takes row t too: U_t = 0, so its lookahead term is silu(0) = 0, and appends the new rows.  No workgroup of this
+  // launch looks at row t or the ring slot of token t.
+  if (owner && grp == 0) {
+    if constexpr (!WORDS) {
+      tkc = *tok(a.kc);
+      tqu = *tok(a.qu);
+      tvc = *tok(a.vc);
+    }
+    float kct[V], qut[V], vut[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) { kct[e] = (float)tkc[e]; qut[e] = (float)tqu[e]; vut[e] = (float)tvu[e]; }
+    if (a.rotary) {
+#pragma unroll
+      for (int e = 0; e < V / 2; ++e) {
+        const int pair = sub * (V / 2) + e;
+        CASTLE_ROPE_PAIR(kct[2 * e], kct[2 * e + 1], (float)t, pair, HD, false);
+        CASTLE_ROPE_PAIR(qut[2 * e], qut[2 * e + 1], (float)t, pair, HD, false);
+        CASTLE_ROPE_PAIR(vut[2 * e], vut[2 * e + 1], (float)t, pair, HD, false);
+      }
+    }
+    float x = 0.f;
+#pragma unroll
+    for (int e = 0; e < V; ++e) x = __builtin_fmaf(qc[e], kct[e], x);
+    x = group_sum<LPR>(x);
+    const float mn = fmaxf(m, x);
+    const float al = fast_exp2(m - mn), p_ = fast_exp2(x - mn);
+    l = l * al + p_;
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = __builtin_fmaf(p_, (float)tvc[e], acc[e] * al);
+    m = mn;
+    if (in_range) {
+      vt z, q, kk, p;
+#pragma unroll
+      for (int e = 0; e < V; ++e) { z[e] = (T)0.f; q[e] = (T)qut[e]; kk[e] = (T)kct[e]; p[e] = (T)vut[e]; }
+      *cached(a.U, t) = z;
+      *cached(a.qu_cache, t) = q;
+      *cached(a.kc_cache, t) = kk;
+      *cached(a.vc_cache, t) = tvc;
+      if (deferred) *reinterpret_cast<vt*>(view_row<T>(a.pend_vu, b, h, slot_t) + sub * V) = p;   // joins the pending sources
+    }
+  }
   // merge the row groups of a wave in registers, then the waves through LDS
   {
-    float M = m;
-#pragma unroll
-    for (int o = LPR; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o));
+    const auto largest = [](float x, float y) { return fmaxf(x, y); };
+    const auto sum = [](float x, float y) { return x + y; };
+    const float M = fold_groups<LPR>(m, largest);
     const float w = m == -INFINITY ? 0.f : fast_exp2(m - M);
-    l *= w;
+    l = fold_groups<LPR>(l * w, sum);
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[e] *= w;
-#pragma unroll
-    for (int o = LPR; o < 64; o <<= 1) {
-      l += __shfl_xor(l, o);
-#pragma unroll
-      for (int e = 0; e < V; ++e) acc[e] += __shfl_xor(acc[e], o);
-    }
+    for (int e = 0; e < V; ++e) acc[e] = fold_groups<LPR>(acc[e] * w, sum);
     m = M;
   }
   const int wave = tid / 64;
@@ -578,9 +615,9 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
   }
   return true;
 }
-template <typename T, int HD, bool UH, bool ONCE>
+template <typename T, int HD, bool UH, bool ONCE, bool ALIKE>
 __global__ __launch_bounds__(kThreads, 4) void decode_stream_kernel(DecodeArgs a) {
-  stream_job<T, HD, UH, ONCE, false>(a, blockIdx.x, blockIdx.y, TokenWords(), [] {}, [] { return true; });
+  stream_job<T, HD, UH, ONCE, false, ALIKE>(a, blockIdx.x, blockIdx.y, TokenWords(), [] {}, [] { return true; });
 }
 
 // One wave per (b, h): merges the split partials into the attention output.
@@ -674,10 +711,16 @@ __global__ __launch_bounds__(kThreads) void decode_flush_kernel(DecodeArgs a) {
   }
 }
 
+static bool views_alike(const DecodeArgs& a) {
+  auto same = [](const View4& v, const View4& w, bool rows) { return v.sb == w.sb && v.sh == w.sh && (!rows || v.sl == w.sl); };
+  return same(a.kc_cache, a.U, true) && same(a.vc_cache, a.U, true) && same(a.qu_cache, a.U, true) && same(a.qc, a.ku, false) && same(a.kc, a.ku, false) &&
+         same(a.vc, a.ku, false) && same(a.qu, a.ku, false) && same(a.vu, a.ku, false);
+}
 template <typename T, int HD, bool UH> static void launch_stream(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid(a.splits, a.B * a.H);
-  if (a.read_once) hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, true>), grid, dim3(kThreads), 0, stream, a);
-  else hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, false>), grid, dim3(kThreads), 0, stream, a);
+  if (!views_alike(a)) hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, false, false>), grid, dim3(kThreads), 0, stream, a);
+  else if (a.read_once) hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, true, true>), grid, dim3(kThreads), 0, stream, a);
+  else hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, false, true>), grid, dim3(kThreads), 0, stream, a);
 }
 template <typename T, int HD> static int launch_decode_t(const DecodeArgs& a, hipStream_t stream) {
   {
@@ -1232,7 +1275,7 @@ __global__ __launch_bounds__(kThreads, kLayerGroups) void decode_layer_kernel(La
     } else if (out < 0) {
       const int split = stream % f.d.splits;
       const TokenWords words = {f.proj, f.merged, f.part, tag};
-      stream_job<T, HD, UH, false, true>(f.d, split, stream / f.d.splits, words, begin, [&](bool came) {
+      stream_job<T, HD, UH, false, true, true>(f.d, split, stream / f.d.splits, words, begin, [&](bool came) {
         // the last split waits for the others' partial results when its own rows are done: they have to be claimed by now
         if (split == f.d.splits - 1) came = came && jobs_claimed(claims + job - split, split, tag);
         return agree(came);
@@ -1326,7 +1369,7 @@ int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const Decod
   const int64_t BH = (int64_t)d.B * d.H;
   const int rows = kThreads * 16 / (d.d * es) * (kEarly + 1);   // of a split: what it requests ahead of the token
   f.d.splits = d.t * (kEarly + 1) <= rows ? 1 : (d.t + rows - 1) / rows + 1;
-  if (d.t_dev != nullptr || 4 * BH * d.t * d.d * es > kLayerCacheBytes || f.d.splits > 64 || n_in + BH * f.d.splits > kLayerGroups * (int64_t)cus ||
+  if (d.t_dev != nullptr || !views_alike(d) || 4 * BH * d.t * d.d * es > kLayerCacheBytes || f.d.splits > 64 || n_in + BH * f.d.splits > kLayerGroups * (int64_t)cus ||
       n_in + BH * f.d.splits + n_out > kLayerJobs)
     return 1;
   f.n_in = (int)n_in;

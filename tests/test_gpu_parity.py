@@ -396,6 +396,47 @@ def test_decode_steps(B, Hh, t0, steps, d, dtype):
     assert torch.equal(bufs[3][:, :, :L].cpu(), ops[2])
 
 
+@pytest.mark.parametrize("Hh,d,dtype,t", [(3, 64, torch.bfloat16, 0), (3, 64, torch.bfloat16, 65), (2, 16, torch.float16, 300), (2, 128, torch.float16, 47), (1, 32, torch.float32, 130)])
+def test_decode_step_ignores_what_lies_beyond_the_count(Hh, d, dtype, t):
+    """The whole ring is read before the row count is known: NaN in every row and ring slot that holds nothing changes no bit, with the count from the host and from the device, and caches whose strides differ give the same bits."""
+    from lookahead_keys_attention_amd import _native as N
+    from lookahead_keys_attention_amd.castle import _CacheStore
+
+    B, cap = 2, t + 130
+    g = torch.Generator(device=DEV).manual_seed(t + d)
+    rnd = lambda *shape: (torch.randn(*shape, generator=g, device=DEV) * 0.6).to(dtype)
+    rows, steps = [rnd(B, Hh, t, d) for _ in range(4)], [[rnd(B, Hh, 1, d) for _ in range(6)] for _ in range(3)]
+    results = []
+    for kind in ("zero", "nan", "device", "strides"):
+        store = _CacheStore(B, Hh, d, cap, dtype, torch.device(DEV))
+        fill = 0.0 if kind == "zero" else float("nan")
+        caches = [torch.full((B, Hh, cap, d + (16 * i if kind == "strides" else 0)), fill, dtype=dtype, device=DEV)[..., :d] for i in range(4)]
+        for cache, row in zip(caches, rows):
+            cache[:, :, :t] = row
+        for extra in store.rings:
+            extra.fill_(fill)
+        outs = []
+        for i, token in enumerate(steps):
+            out = torch.empty(B, Hh, 1, d, dtype=dtype, device=DEV)
+            deferred = H().make_deferred(store.rings[0], store.rings[1], t)
+            if kind == "device":
+                count = torch.tensor([t + i], dtype=torch.int32, device=DEV)
+                N.check(N.lib().castle_decode_step_device_count(*[N.view4(c) for c in caches], count.data_ptr(), cap, *[N.view4(x) for x in token], B, Hh, d,
+                                                                N.dtype_code(dtype), d ** -0.5, N.FLAG_ROTARY, N.view4(out), deferred, store.workspace.data_ptr(),
+                                                                store.workspace.numel(), N.stream_ptr(out.device)), "castle_decode_step_device_count")
+            else:
+                H().castle_decode_step_hip(*caches, t + i, *token, d ** -0.5, out, store.workspace, rotary=True, deferred=deferred)
+            outs.append(out)
+        results.append((torch.cat(outs, 2), torch.stack([c[:, :, :t + 3] for c in caches])))
+    for out, cached in results:
+        assert torch.isfinite(out.float()).all()
+    for (out, cached), kind in zip(results[1:], ("nan", "device", "strides")):
+        if kind == "device":   # (its splits are those of a full cache: sums in another order, roundings of the results)
+            assert_close(out.float(), results[0][0].cpu().double(), dtype, kind, 1e-5)
+        else:
+            assert torch.equal(out, results[0][0]) and torch.equal(cached, results[0][1]), kind
+
+
 @pytest.mark.parametrize("M,N,K,dtype", [(32, 3072, 512, torch.bfloat16), (32, 512, 512, torch.bfloat16), (1, 96, 32, torch.float16),
                                          (5, 6 * 2 * 16, 40, torch.bfloat16), (64, 130, 264, torch.float16), (33, 64, 2048, torch.bfloat16)])
 def test_small_linear_matches_fp64_matmul(M, N, K, dtype):
