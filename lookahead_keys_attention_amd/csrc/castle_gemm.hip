@@ -266,42 +266,353 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
   }
 }
 
-// Tile, number of ranges of the contraction and groups of a workgroup, from what a launch takes (us, measured over 96 ... 5916 rows,
-// outputs of 128 ... 3072 columns and contractions of 128 ... 5916): 2.3, and per step of a workgroup 0.42 (64 x 64) or 0.95
-// (128 x 128) when it has a CU to itself, 0.32 or 0.9 when the CU has others; fp32 0.78 and 0.62.  A second group takes a step of a
-// workgroup that has a CU to itself to 0.30, fp32 0.66, for 0.3 at the end (one range, one group / two: 3000 rows of 1536 -> 256
-// 12.7 / 9.9, 256 rows of fp32 512 -> 3072 15.1 / 13.1; level at two workgroups a CU, behind from three on: 3000 rows of 256 -> 1536 8.7
-// / 11.3).  A split adds a second launch, 2.5, and its partial results, written and read.  Weight gradient of 3000 rows, 1536 x
-// 256 out: 22.6 us in one range, 14.1 in two of two groups; 3000 rows 256 -> 1536 forward: 8.4 on 64 x 64 tiles, 9.5 on 128 x 128;
-// 5916 rows of 512 -> 2048: 30.6 and 23.2.
-struct Plan {
-  int tile, splits, groups;
+// ---- large products of 16-bit operands -----------------------------------------------------------------------------------------
+// 256 x 128 or 256 x 256 of the output per workgroup of eight waves, one workgroup per CU.  What bounds a step of the contraction (64) is
+// the way from L2 into the CU, about 29 bytes a clock (256 x 128: 48 KB in 0.70 us with the products left out, 0.55 us for the products
+// without it, 0.75 together), so larger tiles, which read less for each product: 0.75 ... 1.0 us a step for 256 x 128, 1.4 ... 1.6 for
+// 256 x 256, where 128 x 128 tiles of gemm_kernel take 0.6.  The steps go straight from memory to LDS, into three buffers (two of 256 x
+// 256), the next ones on their way while one is multiplied, over the end of a tile too; the stores of a tile are not waited for.
+// 16384 rows, us, gemm_kernel / here / the library (outputs not in a cache): 512 -> 2048 59 / 43 / 45, with gelu 80 / 64 / 76; 512 -> 3072
+// 86 / 61 / 66; 512 -> 512 18 / 16 / 20; 8192 rows of 512 -> 3072 46 / 36 / 51, 3072 -> 512 49 / 44 / 39.
+// 16-byte pieces go to LDS in the order of the lanes, so rows cannot be padded: a piece takes another place in its row instead, such that
+// the lanes of a read spread over all banks (contraction-contiguous: piece p of row r at p ^ (r / 2 % 8); else the pieces of row k
+// at p ^ 4 (k % 4)).
+constexpr int kWideM = 256, kWideK = 64, kWideThreads = 512;
+template <int BN> struct Wide {
+  static constexpr int kStages = BN == 256 ? 2 : 3;
+  static constexpr int kStage = (kWideM + BN) * kWideK * 2;   // bytes
+  static constexpr int kLoads = kStage / 1024 / (kWideThreads / 64);   // of a wave and step, 1 KB each
+  // where a wave turns 32 rows of its outputs, 4 KB: behind the buffers if there is room, else in the one of the last step
+  static constexpr bool kOwnTurn = BN == 256;
+  static constexpr int kLds = kStages * kStage + (kOwnTurn ? 4096 * kWideThreads / 64 : 4 * kWideThreads / 64);   // and a maximum of each wave
 };
-Plan plan(int M, int N, int K, bool can_split, int elem_size) {
+
+// the compiler waits for every load in flight at each read of LDS if it knows of loads into it: it is not told
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory", "m0");
+}
+template <typename T, bool KC, int FREE> struct WideOperand {
+  static constexpr int N = FREE / 64;   // loads of a wave
+  const T* at;
+  uint32_t off[N];   // bytes
+  __device__ __forceinline__ void start(const T* p, int64_t ld, int free0, int free_end, int k0) {
+    const int lane = lane_id(), first = wave_id() * N;
+    at = KC ? p + free0 * ld + k0 : p + k0 * ld + free0;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      if constexpr (KC) {
+        const int row = 8 * (first + q) + (lane >> 3), piece = (lane & 7) ^ (row >> 1 & 7);
+        off[q] = 2 * (uint32_t)((int)ld * min(row, free_end - 1 - free0) + 8 * piece);
+      } else {
+        constexpr int PIECES = FREE / 8, ROWS = 64 / PIECES;
+        const int k = ROWS * (first + q) + lane / PIECES, piece = lane % PIECES ^ 4 * (k & 3);
+        off[q] = 2 * (uint32_t)(k * (int)ld + (free0 + 8 * piece < free_end ? 8 * piece : 0));
+      }
+    }
+  }
+  __device__ __forceinline__ void load(int64_t ld, uint32_t lds) {
+#pragma unroll
+    for (int q = 0; q < N; ++q) load_to_lds(at, off[q], lds + 1024 * (wave_id() * N + q));
+    at += KC ? kWideK : kWideK * ld;
+  }
+  // operand fragments of the wave's 32 W columns from free0, 16 contraction steps from 16 s
+  template <int W> static __device__ __forceinline__ void read(const T* lds, frag<T> (&f)[W], int free0, int s, int c, int g) {
+    if constexpr (KC) {
+      const T* p = lds + (free0 + c) * kWideK + 8 * ((2 * s + g) ^ (c >> 1 & 7));
+#pragma unroll
+      for (int i = 0; i < W; ++i) f[i] = *reinterpret_cast<const frag<T>*>(p + 32 * kWideK * i);
+    } else {
+      const int lp = c & 15, k = 16 * s + 8 * g + (lp >> 2);
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        const T* p = lds + k * FREE + 32 * ((free0 / 32 + i) ^ (lp >> 2)) + 16 * (c >> 4) + 4 * (lp & 3);
+        const vec<T, 4> lo = lds_tr4<T>(p), hi = lds_tr4<T>(p + 4 * FREE);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { f[i][e] = lo[e]; f[i][4 + e] = hi[e]; }
+      }
+    }
+  }
+};
+extern __shared__ __attribute__((aligned(16))) unsigned char castle_wide[];
+
+// FUSED: with gelu or its derivative on the store (kernels of their own: the code of a plain store stays short)
+template <typename T, bool AK, bool BKC, int BN, bool FUSED> __global__ __launch_bounds__(kWideThreads, 2) void gemm_wide_kernel(GemmArgs a) {
+  typedef Wide<BN> W;
+  constexpr int WN = BN / 64;   // 32-wide pieces of a wave
+  typedef WideOperand<T, AK, kWideM> OpA;
+  typedef WideOperand<T, BKC, BN> OpB;
+  typedef vec<T, 8> vt;
+  typedef vec<float, 8> vf;
+  const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
+  // Tiles in the order of an XCD's L2: all rows of eight columns of tiles (2048 output columns), then those of the next.
+  constexpr int kBand = 2048 / BN;
+  const int tiles_m = (a.M + kWideM - 1) / kWideM, tiles_n = (a.N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+  auto place = [&](int t, int& m0, int& n0) __attribute__((always_inline)) {
+    const int band = t / (tiles_m * kBand), rest = t - band * tiles_m * kBand, width = min(kBand, tiles_n - band * kBand);
+    m0 = rest / width * kWideM;
+    n0 = (band * kBand + rest % width) * BN;
+  };
+  const int share = (tiles + 7) / 8, first = blockIdx.x % 8 * share, last = min(tiles, first + share), stride = gridDim.x / 8;
+  const int wm = wave / 2 * 64, wn = wave % 2 * (BN / 2);
+  const int k0 = blockIdx.y * a.k_per_split, steps = (min(a.K, k0 + a.k_per_split) - k0) / kWideK;
+  const int amax_tile = a.amax_from / BN, amax_tiles = (a.amax_to - 1) / BN + 1 - amax_tile;   // of a row of tiles
+  if (a.amax != nullptr && blockIdx.x == 0) {
+    for (int i = (a.M + kWideM - 1) / kWideM * amax_tiles + threadIdx.x; i < kAmaxBlocks; i += kWideThreads) a.amax[i] = 0.f;
+    if (threadIdx.x == 0 && a.amax_status != nullptr) *a.amax_status = 0;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)castle_wide;
+  int tile = first + blockIdx.x / 8;
+  if (tile >= last) return;
+  // the step that is requested next runs ahead of the one that is multiplied, into the next tile
+  OpA ra;
+  OpB rb;
+  int next_tile = tile, next_step = 0, ahead = 0;   // ahead: steps requested and not waited for
+  auto start = [&]() __attribute__((always_inline)) {
+    int m0, n0;
+    place(next_tile, m0, n0);
+    ra.start(static_cast<const T*>(a.a), a.lda, m0, a.M, k0);
+    rb.start(static_cast<const T*>(a.b), a.ldb, n0, a.N, k0);
+  };
+  auto request = [&](int buffer) __attribute__((always_inline)) {
+    if (next_tile >= last) return;
+    ++ahead;
+    ra.load(a.lda, lds0 + buffer);
+    rb.load(a.ldb, lds0 + buffer + kWideM * kWideK * 2);
+    if (++next_step == steps) {
+      next_step = 0;
+      next_tile += stride;
+      if (next_tile < last) start();
+    }
+  };
+  start();
+  request(0);
+  request(W::kStage);
+  if constexpr (W::kStages == 3) request(2 * W::kStage);
+  // The step behind the current one is in LDS, from every wave, and all have read the current one.  Waits are for all but the last so many
+  // requests; the stores of a tile that lies inside the output are counted (STORES more), so they are not waited for.
+  constexpr int STORES = 4 * WN;
+  int stores = 0;   // 1: the stores of the tile before are behind the pieces that are waited for, 2: as many again
+  auto arrive = [&]() __attribute__((always_inline)) {
+    auto wait = [&](auto n) __attribute__((always_inline)) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(n)::value) : "memory");
+    };
+    const int newer = ahead - 1;   // steps
+    if (newer > 1) wait(std::integral_constant<int, 2 * W::kLoads>());
+    else if (newer == 1) {
+      if (stores == 2) wait(std::integral_constant<int, W::kLoads + 2 * STORES>());
+      else if (stores == 1) wait(std::integral_constant<int, W::kLoads + STORES>());
+      else wait(std::integral_constant<int, W::kLoads>());
+    } else {
+      if (stores == 2) wait(std::integral_constant<int, 2 * STORES>());
+      else if (stores == 1) wait(std::integral_constant<int, STORES>());
+      else wait(std::integral_constant<int, 0>());
+    }
+    stores = 0;
+    --ahead;
+  };
+  int buffer = 0;
+  frag<T> fa[2][2], fb[2][WN];
+  auto read = [&](int slot, int s) __attribute__((always_inline)) {
+    const T* la = reinterpret_cast<const T*>(castle_wide + buffer);
+    OpA::read(la, fa[slot], wm, s, c, g);
+    OpB::read(la + kWideM * kWideK, fb[slot], wn, s, c, g);
+    __builtin_amdgcn_sched_barrier(0);   // these reads, then the products of the fragments before
+  };
+  arrive();
+  read(0, 0);
+  while (tile < last) {
+    int m0, n0;
+    place(tile, m0, n0);
+    acc_t acc[2][WN];   // [n rows, m lanes]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < WN; ++j) zero(acc[i][j]);
+    auto multiply = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) mma(acc[i][j], fb[slot][j], fa[slot][i]);
+    };
+    int done = 0;   // buffer of the step that ends
+    for (int it = 0; it < steps; ++it) {
+#pragma unroll
+      for (int s = 0; s < kWideK / 16 - 1; ++s) {
+        read(1 - s % 2, s + 1);
+        multiply(s % 2);
+      }
+      arrive();
+      done = buffer;
+      buffer = buffer == (W::kStages - 1) * W::kStage ? 0 : buffer + W::kStage;
+      if (it + 1 < steps) request(done);
+      read(0, 0);   // (behind the last step of all: what is there, for nothing)
+      multiply(1);
+    }
+    asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");   // the loop may end right behind a product
+    __builtin_amdgcn_sched_barrier(0);
+    tile += stride;
+    const bool inside = m0 + kWideM <= a.M && n0 + BN <= a.N;
+    if (a.part != nullptr) {   // partial product of this range of the contraction
+      request(done);
+      float* part = a.part + (int64_t)blockIdx.y * a.M * a.N;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int m = m0 + wm + 32 * i + c, n = n0 + wn + 32 * j + 8 * q + 4 * g;
+            if (m < a.M && n < a.N) *reinterpret_cast<vec<float, 4>*>(part + (int64_t)m * a.N + n) = pack4<float>(acc[i][j], q);
+          }
+      if (inside) stores = 2;
+      continue;
+    }
+    // to whole rows through the buffer of the last step, each wave in the part that it fills next; pieces placed as above
+    static_assert(OpA::N * 1024 == 32 * 64 * 2, "32 rows of each wave");
+    if constexpr (W::kOwnTurn) request(done);
+    T* out = reinterpret_cast<T*>(castle_wide + (W::kOwnTurn ? W::kStages * W::kStage : done) + wave * 4096);
+    float most = 0.f;
+    // the second operand of the slope is on its way a piece ahead
+    vt u[2][4];
+    auto fetch = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + wm + 32 * (h % 2) + 8 * r + (lane >> 3), n = n0 + wn + 64 * (h / 2) + 8 * (lane & 7);
+        u[h % 2][r] = *reinterpret_cast<const vt*>(static_cast<const T*>(a.aux) + (int64_t)min(m, a.M - 1) * a.ldc + (n < a.N ? n : 0));
+      }
+    };
+    const bool slope = FUSED && a.epilogue == kGemmGeluSlope, gelu_too = FUSED && a.epilogue == kGemmGelu;
+    if (slope) fetch(0);
+#pragma unroll
+    for (int h = 0; h < WN; ++h) {   // 32 x 64 of the wave's part
+      const int i = h % 2, half = h / 2;
+      if (slope && h + 1 < WN) fetch(h + 1);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) st4<T>(out + c * 64 + 8 * ((4 * j + q) ^ (c >> 1 & 7)) + 4 * g, pack4<T>(acc[i][2 * half + j], q));
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 8 * r + (lane >> 3), m = m0 + wm + 32 * i + row, n = n0 + wn + 64 * half + 8 * (lane & 7);
+        vt x = *reinterpret_cast<const vt*>(out + row * 64 + 8 * ((lane & 7) ^ (row >> 1 & 7)));
+        if (m >= a.M || n >= a.N) continue;
+        const int64_t at = (int64_t)m * a.ldc + n;
+        if (slope) {
+          vf f = __builtin_convertvector(x, vf);
+          const vf v = __builtin_convertvector(u[i][r], vf);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] *= gelu_slope<T>(v[e]);
+          x = __builtin_convertvector(f, vt);
+        }
+        *reinterpret_cast<vt*>(static_cast<T*>(a.c) + at) = x;
+        if (a.amax != nullptr && n >= a.amax_from && n < a.amax_to) {
+          const vf f = __builtin_convertvector(x, vf);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(f[e]));   // fmaxf drops NaNs
+        }
+        if (gelu_too) {
+          vf f = __builtin_convertvector(x, vf);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) f[e] = gelu<T>(f[e]);
+          *reinterpret_cast<vt*>(static_cast<T*>(a.aux) + at) = __builtin_convertvector(f, vt);
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if constexpr (!W::kOwnTurn) request(done);
+    if (inside) stores = gelu_too ? 2 : 1;
+    const int slot = n0 / BN - amax_tile;
+    if (a.amax != nullptr && slot >= 0 && slot < amax_tiles) {
+      constexpr int kApart = W::kOwnTurn ? 1024 : 1;   // in the wave's own part
+      float* s_most = reinterpret_cast<float*>(castle_wide + W::kStages * W::kStage);
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) most = fmaxf(most, __shfl_xor(most, o));
+      if (lane == 0) s_most[wave * kApart] = most;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < kWideThreads / 64; ++w) most = fmaxf(most, s_most[w * kApart]);
+        a.amax[m0 / kWideM * amax_tiles + slot] = fminf(most, 3.0e38f);   // an infinite value counts as the largest finite one
+      }
+    }
+  }
+}
+
+// Tile, number of ranges of the contraction and groups of a workgroup, from what a launch takes (us, measured over 96 ... 16384 rows,
+// outputs of 128 ... 3072 columns and contractions of 128 ... 16384, with outputs that no cache holds): 2.3, and for each tile of a CU
+// so much a step and at its end, more at the end where gelu or its derivative rides on the store.  A second group takes a step of a
+// workgroup of 64 x 64 that has a CU to itself from 0.42 to 0.36, fp32 from 0.78 to 0.66, for 0.3 at the end (one range, one group / two:
+// 3000 rows of 1536 -> 256 12.7 / 9.9, 256 rows of fp32 512 -> 3072 15.1 / 13.1); at two workgroups a CU it gains where the contraction is
+// long (3000 rows of 3072 -> 512 29 / 26, of 512 -> 512 level), behind from three on.  A split adds a second launch, 2.5, and its partial
+// results, written and read.  Weight gradient of 3000 rows, 1536 x 256 out: 22.6 us in one range, 14.1 in two of two groups; 3008 rows
+// 512 -> 2048 17.6 on 64 x 64, 16.6 on 128 x 128, 14.2 on 256 x 128; 4096 rows 512 -> 3072 31.8, 26.2, 24.9 and 21.8 on 256 x 256.
+struct Plan {
+  int tile, splits, groups;   // tile: 64, 128, or columns of a tile of 256 rows + 256
+  int rows() const { return std::min(tile, kWideM); }
+  int columns() const { return tile > kWideM ? tile - kWideM : tile; }
+  int tiles(int M, int N) const { return ((M + rows() - 1) / rows()) * ((N + columns() - 1) / columns()); }
+};
+Plan plan(int M, int N, int K, bool plain, int elem_size) {
   Plan best = {64, 1, 1};
   double best_cost = 1e30;
+  auto take = [&](double cost, const Plan& p) {
+    if (cost < best_cost) { best_cost = cost; best = p; }
+  };
   for (int tile = 64; tile <= (elem_size == 2 ? 128 : 64); tile += 64) {
-    const double alone = elem_size == 4 ? 0.78 : tile == 64 ? 0.42 : 0.95, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.32 : 0.9;
+    const double alone = elem_size == 4 ? 0.78 : tile == 64 ? 0.42 : 0.85, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.29 : 0.6;
+    const double end = elem_size == 4 ? 0 : tile == 64 ? 0.25 : 2.3, fused = plain ? 0 : tile == 64 ? 0.5 : 2.6;
     const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
     const int steps = (K * elem_size + 127) / 128;   // 128 bytes of the contraction a step
-    for (int s = 1; s <= (can_split ? std::min(16, (steps + 1) / 2) : 1); ++s) {
+    for (int s = 1; s <= (plain ? std::min(16, (steps + 1) / 2) : 1); ++s) {
       const int64_t per_cu = (tiles * s + 255) / 256, n = (steps + s - 1) / s;
-      const int groups = tile == 64 && per_cu == 1 && n >= 4 ? 2 : 1;
-      double cost = groups == 2 ? 0.3 + n * (elem_size == 4 ? 0.66 : 0.30) : per_cu == 1 ? n * alone : per_cu * n * shared;
+      const int groups = tile == 64 && (per_cu == 1 ? n >= 4 : elem_size == 2 && s == 1 && per_cu == 2 && n >= 12) ? 2 : 1;
+      double cost = groups == 2 ? 0.3 + n * (elem_size == 4 ? 0.66 : per_cu == 1 ? 0.36 : 0.55) : per_cu == 1 ? n * alone + end : per_cu * (n * shared + end);
       if (s > 1) cost += 2.5 + (double)s * M * N * 8 / 4e6;
-      if (cost < best_cost) { best_cost = cost; best = {tile, s, groups}; }
+      take(cost + (per_cu == 1 ? 2 : per_cu) * fused, {tile, s, groups});
+    }
+  }
+  if (elem_size == 2 && K % kWideK == 0) {
+    for (int columns = 128; columns <= 256; columns += 128) {
+      const double start = columns == 128 ? 1.6 : 2.6, end = columns == 128 ? (plain ? 3 : 8.8) : plain ? 6.5 : 16.5;
+      const int64_t tiles = (int64_t)((M + kWideM - 1) / kWideM) * ((N + columns - 1) / columns);
+      const int steps = K / kWideK;
+      for (int s = 1; s <= (plain ? std::min(16, steps / 4) : 1); ++s) {
+        const int64_t per_cu = (tiles * s + 255) / 256, n = (steps + s - 1) / s;
+        const double busy = std::min(1., tiles * s / 256.), step = columns == 128 ? 0.75 + 0.27 * busy : 1.2 + 0.36 * busy;
+        take(start + per_cu * (n * step + end) + (s > 1 ? 2.5 + (double)s * M * N * 8 / 6e6 : 0), {kWideM + columns, s, 1});
+      }
     }
   }
   return best;
 }
 constexpr int kStep16 = 64, kStep32 = 32;   // contraction steps in LDS, 16-bit and fp32
 
+template <typename T, bool AK, bool BKC, int BN, bool FUSED> int launch_wide(const GemmArgs& a, const Plan& p, hipStream_t stream) {
+  static PerDeviceOnce once;
+  bool& configured = once.flag();
+  if (!configured) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<T, AK, BKC, BN, FUSED>), hipFuncAttributeMaxDynamicSharedMemorySize, Wide<BN>::kLds) != hipSuccess) return -3;
+    configured = true;
+  }
+  hipLaunchKernelGGL((gemm_wide_kernel<T, AK, BKC, BN, FUSED>), dim3(std::min((p.tiles(a.M, a.N) + 7) / 8 * 8, 256), p.splits), dim3(kWideThreads), Wide<BN>::kLds, stream, a);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
 template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
   constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
-  const int tiles = ((a.M + p.tile - 1) / p.tile) * ((a.N + p.tile - 1) / p.tile);
+  const int tiles = p.tiles(a.M, a.N);
   // at most what the CUs hold at once: two workgroups of 128 x 128 tiles or four of 64 x 64
   const dim3 grid(std::min((tiles + 7) / 8 * 8, p.tile == 128 ? 512 : 1024), p.splits);
   if constexpr (sizeof(T) == 2) {
+    if (p.tile > kWideM) {
+      const bool plain = a.epilogue == kGemmPlain;
+      if (p.columns() == 128) return plain ? launch_wide<T, AK, BKC, 128, false>(a, p, stream) : launch_wide<T, AK, BKC, 128, true>(a, p, stream);
+      return plain ? launch_wide<T, AK, BKC, 256, false>(a, p, stream) : launch_wide<T, AK, BKC, 256, true>(a, p, stream);
+    }
     if (p.tile == 128) {
       hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK, 1>), grid, dim3(kThreads), 0, stream, a);
       return hipGetLastError() == hipSuccess ? 0 : -3;
@@ -322,13 +633,13 @@ int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue) {
 // the maximum is taken on the store: not for a contraction in ranges, nor for more tiles than there are slots
 bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to) {
   const Plan p = plan(M, N, K, true, elem_size);
-  const int per_row = (amax_to - 1) / p.tile + 1 - amax_from / p.tile;
-  return p.splits == 1 && (int64_t)((M + p.tile - 1) / p.tile) * per_row <= kAmaxBlocks;
+  const int per_row = (amax_to - 1) / p.columns() + 1 - amax_from / p.columns();
+  return p.splits == 1 && (int64_t)((M + p.rows() - 1) / p.rows()) * per_row <= kAmaxBlocks;
 }
 
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream) {
   const int es = dtype == 0 ? 4 : 2, step = dtype == 0 ? kStep32 : kStep16;
-  Plan p = plan(a.M, a.N, a.K, a.epilogue == kGemmPlain, es);
+  Plan p = plan(a.M, a.N, a.K, a.epilogue == kGemmPlain || a.amax != nullptr, es);   // (the slots of the maxima follow from the plain plan)
   a.k_per_split = ((a.K + p.splits - 1) / p.splits + step - 1) / step * step;
   p.splits = (a.K + a.k_per_split - 1) / a.k_per_split;   // rounding up may leave the last ones empty
   a.part = p.splits > 1 ? workspace : nullptr;

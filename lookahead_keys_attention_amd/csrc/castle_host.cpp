@@ -460,15 +460,19 @@ Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epi
 
 // ---- projections -----------------------------------------------------------------------------------------------
 // Own products where a call is short: the library's costs 18 us of host time, one here 4.  On the GPU they are level or
-// ahead up to the sizes below (us, own / library: 5916 rows 512 -> 2048 forward 23 / 33, 8192 rows 29 / 22; input gradient
-// of 1000 rows x 3072 x 512 15 / 16, 5916 x 2048 x 512 28 / 23; weight gradient of 3000 rows, 1536 x 256, 14 / 27, of
-// 5916, 2048 x 512, 32 / 41).  In fp32 they are level up to the size below (256 rows, 512 <-> 3072: forward 13 / 13, input gradient 16 / 12,
+// ahead up to the sizes below (us, own / library: input gradient of 1000 rows x 3072 x 512 15 / 16, 4096 x 3072 x 512 31 / 31, 8192 x 3072 x
+// 512 44 / 39; weight gradient of 3000 rows, 1536 x 256, 14 / 27, of 4096, 3072 x 512, 31 / 41; forward of 4096 rows 1024 -> 3072 34 / 30).  Up
+// to a contraction of 512 they are ahead at every size measured: a tile's start and end weigh more there than its steps, and the
+// store takes gelu and the maxima along (16384 rows 512 -> 2048 43 / 45, 512 -> 3072 61 / 66, 512 -> 512 16 / 20, its input gradient 16 / 19).
+// In fp32 they are level up to the size below (256 rows, 512 <-> 3072: forward 13 / 13, input gradient 16 / 12,
 // weight gradient 15 / 16), where a layer's time is the host's; 2048 rows 60 / 53, 64 / 49, 72 / 55.
 bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16, double most_32) {
   return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
 }
-constexpr double kOwnForward = 14e9, kOwnInputGrad = 4e9, kOwnWeightGrad = 40e9, kOwn32 = 1e9;
-constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 70 / 83
+double own_forward(int64_t k) { return k <= 512 && k % 64 == 0 ? 64e9 : 14e9; }   // (other contractions have no tiles of 256 rows)
+double own_input_grad(int64_t k) { return k <= 512 && k % 64 == 0 ? 64e9 : 4e9; }
+constexpr double kOwnWeightGrad = 40e9, kOwn32 = 1e9;
+constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 73 / 91
 
 // The attention kernels behind a product begin with the largest element of some of its columns (vu of a fused projection, all
 // of the gradient of the merged heads): an own product leaves the partial maxima where they look for them, in the
@@ -488,12 +492,12 @@ Maxima maxima(const Tensor& like, int64_t rows, int64_t n, int64_t k, int64_t co
 }
 
 Tensor project(const Tensor& x, const Tensor& w) {   // (R, K), (N, K) -> (R, N)
-  if (own_product(x, w, x.size(0), w.size(0), x.size(1), kOwnForward, kOwn32)) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
+  if (own_product(x, w, x.size(0), w.size(0), x.size(1), own_forward(x.size(1)), kOwn32)) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(x, w.t());
 }
 // the fused projection, with the maxima of its vu part
 Tensor project_packed(const Tensor& x, const Tensor& w, const Shape& s, Tensor& prepared) {
-  if (!own_product(x, w, x.size(0), w.size(0), x.size(1), kOwnForward, kOwn32)) return at::mm(x, w.t());
+  if (!own_product(x, w, x.size(0), w.size(0), x.size(1), own_forward(x.size(1)), kOwn32)) return at::mm(x, w.t());
   const int64_t part = (int64_t)s.H * s.d;
   const Maxima m = maxima(x, x.size(0), w.size(0), x.size(1), 2 * part, part,
                           check(castle_fwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_workspace_bytes"), true);
@@ -501,7 +505,7 @@ Tensor project_packed(const Tensor& x, const Tensor& w, const Shape& s, Tensor& 
   return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
 }
 Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R, K)
-  if (own_product(dy, w, dy.size(0), w.size(0), w.size(1), kOwnInputGrad, kOwn32)) return product(dy, false, w, true, CASTLE_GEMM_PLAIN, std::nullopt);
+  if (own_product(dy, w, dy.size(0), w.size(0), w.size(1), own_input_grad(w.size(0)), kOwn32)) return product(dy, false, w, true, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(dy, w);
 }
 
@@ -653,7 +657,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
     const int64_t flags = ctx->saved_data["flags"].toInt();
     Tensor dmerged, prepared;
-    if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), kOwnInputGrad, kOwn32)) {
+    if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)), kOwn32)) {
       const Maxima m = maxima(dy, B * L, w_out.size(1), w_out.size(0), 0, w_out.size(1), bwd_workspace_bytes(shape, flags, state), false);
       prepared = m.prepared;
       dmerged = product(dy, false, w_out, true, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
@@ -696,7 +700,7 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const int64_t R = x.numel() / x.size(-1);
     const Normed n = norm_rows(x.reshape({R, x.size(-1)}), delta.reshape({R, x.size(-1)}), norm_w, eps, want_graph);
     Tensor up, act;
-    if (own_product(n.h, w_up, R, w_up.size(0), w_up.size(1), kOwnForward, kOwn32)) {   // GELU on the way out
+    if (own_product(n.h, w_up, R, w_up.size(0), w_up.size(1), own_forward(w_up.size(1)), kOwn32)) {   // GELU on the way out
       act = at::empty({R, w_up.size(0)}, n.h.options());
       up = product(n.h, false, w_up, false, CASTLE_GEMM_GELU, act);
     } else {

@@ -275,6 +275,17 @@ def test_products_of_two_groups(rows, n, k, dtype):
         test_product_leaves_partial_maxima(rows, n, k, 8, n - 16)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,n,k", [(2112, 3136, 512), (2112, 512, 3136), (8136, 2040, 512), (8136, 512, 2040), (8136, 2040, 320), (4160, 3136, 448),
+                                      (2112, 6144, 1024)])
+def test_products_of_wide_tiles(rows, n, k, dtype):
+    """Tiles of 256 x 128 and 256 x 256 in each layout: last ones of 64 rows and columns and of odd eights, even and odd numbers of steps,
+    one tile a CU and several, ranges of the contraction."""
+    test_products(rows, n, k, dtype)
+    if dtype == torch.bfloat16 and n > k:
+        test_product_leaves_partial_maxima(rows, n, k, 520, 256)
+
+
 def test_projection_of_rows_beyond_32_bit_offsets():
     """Rows that lie further apart than the products' offsets reach: 40000 of them, 65536 elements apart."""
     from lookahead_keys_attention_amd import Castle
