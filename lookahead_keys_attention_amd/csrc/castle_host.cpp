@@ -463,14 +463,15 @@ Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epi
 // ahead up to the sizes below (us, own / library: input gradient of 1000 rows x 3072 x 512 15 / 16, 4096 x 3072 x 512 31 / 31, 8192 x 3072 x
 // 512 44 / 39; weight gradient of 3000 rows, 1536 x 256, 14 / 27, of 4096, 3072 x 512, 31 / 41; forward of 4096 rows 1024 -> 3072 34 / 30).  Up
 // to a contraction of 512 they are ahead at every size measured: a tile's start and end weigh more there than its steps, and the
-// store takes gelu and the maxima along (16384 rows 512 -> 2048 43 / 45, 512 -> 3072 61 / 66, 512 -> 512 16 / 20, its input gradient 16 / 19).
+// store takes gelu and the maxima along (16384 rows 512 -> 2048 43 / 45, 512 -> 3072 61 / 66, 512 -> 512 16 / 20, its input gradient 16 / 19;
+// 65536 rows, both projections of a layer: 45 us less than the library's).
 // In fp32 they are level up to the size below (256 rows, 512 <-> 3072: forward 13 / 13, input gradient 16 / 12,
 // weight gradient 15 / 16), where a layer's time is the host's; 2048 rows 60 / 53, 64 / 49, 72 / 55.
 bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16, double most_32) {
   return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
 }
-double own_forward(int64_t k) { return k <= 512 && k % 64 == 0 ? 64e9 : 14e9; }   // (other contractions have no tiles of 256 rows)
-double own_input_grad(int64_t k) { return k <= 512 && k % 64 == 0 ? 64e9 : 4e9; }
+double own_forward(int64_t k) { return k <= 512 && k % 64 == 0 ? 260e9 : 14e9; }   // (other contractions have no tiles of 256 rows)
+double own_input_grad(int64_t k) { return k <= 512 && k % 64 == 0 ? 260e9 : 4e9; }
 constexpr double kOwnWeightGrad = 40e9, kOwn32 = 1e9;
 constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 73 / 91
 
