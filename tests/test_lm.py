@@ -259,6 +259,30 @@ def test_sampling_kernel_picks_what_the_operators_pick(vocabulary, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("vocabulary", [1, 64, 65, 256, 257, 512])
+def test_sampling_of_one_wave_equals_that_of_many(vocabulary, dtype):
+    """Small vocabularies against the same rows with -inf behind them, which the kernel for large ones takes: equal values, both zeros,
+    infinities and NaN among the logits."""
+    from lookahead_keys_attention_amd import _native
+
+    g = torch.Generator(device="cuda").manual_seed(vocabulary)
+    logits = (4 * torch.randn(32, vocabulary, device="cuda", generator=g)).round().div(4).to(dtype)
+    special = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0, -0.0], device="cuda", dtype=dtype)
+    at = torch.rand(logits.shape, device="cuda", generator=g) < torch.linspace(0, 1, 32, device="cuda")[:, None]
+    logits = torch.where(at, special[torch.randint(0, 5, logits.shape, device="cuda", generator=g)], logits)
+    wide = torch.full((32, 600), float("-inf"), device="cuda", dtype=dtype)
+    wide[:, :vocabulary] = logits
+    u = torch.rand(wide.shape, device="cuda", generator=g)
+    for k in sorted({1, (vocabulary + 9) // 10, vocabulary}):
+        for noise in (False, True):
+            few, many = (torch.full((32,), -1, device="cuda") for _ in range(2))
+            _native.host().sample_tokens(logits, u[:, :vocabulary].contiguous() if noise else None, k, 0.7, few, None)
+            _native.host().sample_tokens(wide, u if noise else None, k, 0.7, many, None)
+            assert torch.equal(few, many), (k, noise)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("temperature", [0, 0.7])
 def test_sampling_with_the_operators_of_large_vocabularies(monkeypatch, temperature):
     """Beyond SAMPLER_MAX_VOCABULARY the operators pick: the same tokens, with and without a graph."""
