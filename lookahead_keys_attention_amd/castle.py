@@ -432,15 +432,24 @@ class Castle(nn.Module):
             _unmodified(layer, nn.Linear) and layer.bias is None and layer.weight.dtype == x.dtype for layer in (self.to_all_qkv, self.combine_heads)
         ) and not _has_any_global_hook() and not torch.is_autocast_enabled("cuda")
 
-    def _layer_native(self, x, want_cache, delta=None):
+    def _layer_native(self, x, want_cache, delta=None, store=None):
         """The parallel pass as one native call (csrc/castle_host.cpp): norm, projection, attention core,
         output projection and, with a cache, the rows of its buffers.  With `delta` the layer runs on x + delta and
-        the result is (y, x + delta), with the cache behind it: a block of a residual stream."""
+        the result is (y, x + delta), with the cache behind it: a block of a residual stream.  `store`: the cache goes into
+        its buffers (inference only)."""
         B, n, _ = x.shape
         H, d = self.heads, self.dim_head
         norm = self._modules["norm"]
         u_half = want_cache and x.dtype == torch.bfloat16 and ops.LOOKAHEAD_KEYS_HALF
         flags = (ops.DEFAULT_FLAGS | (_native.FLAG_ROTARY if self.use_rotary else 0) | (_native.FLAG_U_HALF if u_half else 0))
+        if store is not None:
+            results = _native.host().layer_prefill(
+                x, delta, norm._parameters.get("weight"), getattr(norm, "eps", None), self._modules["to_all_qkv"]._parameters["weight"],
+                self._modules["combine_heads"]._parameters["weight"], H, self.scale, flags, list(store.buffers))
+            store.u_half = u_half
+            store.length = store.base0 = n
+            store.scale = self.scale
+            return (*results, store.as_cache())
         results = _native.host().layer_parallel(
             x, delta, norm._parameters.get("weight"), getattr(norm, "eps", None), self._modules["to_all_qkv"]._parameters["weight"],
             self._modules["combine_heads"]._parameters["weight"], H, self.scale, flags,

@@ -165,8 +165,9 @@ void six_of_packed(const Tensor& p, const Shape& s, castle_view4 (&six)[6]) {
 }
 
 std::tuple<Tensor, Tensor, Tensor, Tensor> run_packed(const Tensor& proj, int64_t heads, double scale, bool want_U,
-                                                            int64_t row_capacity, int64_t flags, bool keep_state, const Tensor& prepared) {
-  // The lookahead keys come back as the first L rows of a (B, H, row_capacity, d) buffer, so that a
+                                                            int64_t row_capacity, int64_t flags, bool keep_state, const Tensor& prepared,
+                                                            const Tensor& U_buffer = Tensor()) {
+  // The lookahead keys come back as the first L rows of a (B, H, row_capacity, d) buffer, `U_buffer` if there is one, so that a
   // caller can hand over the U buffer of a decode cache without copying (row_capacity >= L).
   require_gpu(proj, "castle_attention_packed");
   const Shape s = packed_shape(proj, heads);
@@ -177,7 +178,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> run_packed(const Tensor& proj, int64_
   six_of_packed(p, s, six);
   const int64_t B = s.B, H = s.H, L = s.L, d = s.d, cap = std::max(row_capacity, L);
   Tensor merged = at::empty({B, L, H * d}, proj.options());
-  Tensor U = want_U ? at::empty({B, H, cap, d}, proj.options()) : at::empty({0}, proj.options());
+  Tensor U = U_buffer.defined() ? U_buffer : want_U ? at::empty({B, H, cap, d}, proj.options()) : at::empty({0}, proj.options());
   auto [ws, state] = run_fwd(six, s, scale, flags, packed_view(merged, s, 1, 0),
                              want_U ? view4(U) : castle_view4{nullptr, 0, 0, 0}, keep_state, proj, prepared);
   return {merged, U, ws, state};
@@ -588,7 +589,7 @@ Tensor linear_autograd(const Tensor& x, const Tensor& weight) {
 struct LayerFn : torch::autograd::Function<LayerFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const std::optional<Tensor>& delta, const std::optional<Tensor>& norm_w_,
                                const Tensor& w_qkv, const Tensor& w_out, std::optional<double> eps, int64_t heads, double scale, int64_t flags,
-                               bool want_graph, bool keep_state, int64_t cache_rows) {
+                               bool want_graph, bool keep_state, int64_t cache_rows, const std::vector<Tensor>& into = {}) {
     const at::AutoDispatchBelowADInplaceOrView below;
     const Tensor norm_w = norm_w_.value_or(Tensor());
     const int64_t B = x.size(0), L = x.size(1), dim = x.size(2);
@@ -597,7 +598,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     Tensor prepared;
     const Tensor proj = project_packed(n.h, w_qkv, {(int)B, (int)heads, (int)L, (int)(w_qkv.size(0) / (6 * heads)), dtype_code(n.h)}, prepared).view({B, L, w_qkv.size(0)});
     const bool want_U = cache_rows > 0;
-    auto [merged, U, ws, state] = run_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state, prepared);
+    auto [merged, U, ws, state] = run_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state, prepared, into.empty() ? Tensor() : into[0]);
     variable_list out{project(merged.view({B * L, merged.size(2)}), w_out).view({B, L, w_out.size(0)})};
     if (delta) out.push_back(n.sum.view({B, L, dim}));
     const size_t results = out.size();
@@ -607,7 +608,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
       castle_view4 src[3], dst[3];
       out.push_back(U);
       for (int i = 0; i < 3; ++i) {
-        out.push_back(at::empty({B, heads, cache_rows, s.d}, proj.options()));
+        out.push_back(into.empty() ? at::empty({B, heads, cache_rows, s.d}, proj.options()) : into[i + 1]);
         src[i] = packed_view(proj, s, 6, part[i]);
         dst[i] = view4(out.back());
       }
@@ -690,6 +691,21 @@ variable_list layer_parallel(const Tensor& x, const std::optional<Tensor>& delta
   if (!wants_graph({x, delta.value_or(Tensor()), norm_w.value_or(Tensor()), w_qkv, w_out}))
     return LayerFn::forward(nullptr, x, delta, norm_w, w_qkv, w_out, eps, heads, scale, flags, false, false, cache_rows);
   return LayerFn::apply(x, delta, norm_w, w_qkv, w_out, eps, heads, scale, flags, true, keep_state, cache_rows);
+}
+
+// The same into the four buffers of a decode cache that is there already, without a graph -> [y, x + delta if there is a delta]
+variable_list layer_prefill(const Tensor& x, const std::optional<Tensor>& delta, const std::optional<Tensor>& norm_w, std::optional<double> eps,
+                            const Tensor& w_qkv, const Tensor& w_out, int64_t heads, double scale, int64_t flags, const std::vector<Tensor>& buffers) {
+  const c10::DeviceGuard guard(x.device());
+  TORCH_CHECK_VALUE(buffers.size() == 4 && x.dim() == 3 && !wants_graph({x, delta.value_or(Tensor()), norm_w.value_or(Tensor()), w_qkv, w_out}),
+                    "layer_prefill: four buffers, and no gradients");
+  const int64_t d = w_qkv.size(0) / (6 * heads), rows = buffers[0].dim() == 4 ? buffers[0].size(2) : 0;
+  for (const Tensor& t : buffers)
+    TORCH_CHECK_VALUE(t.is_contiguous() && t.sizes() == at::IntArrayRef({x.size(0), heads, rows, d}) && rows >= x.size(1) && t.scalar_type() == x.scalar_type() &&
+                      t.device() == x.device(), "layer_prefill: unexpected buffers");
+  auto out = LayerFn::forward(nullptr, x, delta, norm_w, w_qkv, w_out, eps, heads, scale, flags, false, false, rows, buffers);
+  out.resize(delta ? 2 : 1);
+  return out;
 }
 
 // ---- the other blocks of a language model over sequences ---------------------------------------------------------
@@ -1089,6 +1105,7 @@ PYBIND11_MODULE(_castle_host, m) {
   m.attr("ABI_VERSION") = castle_abi_version();
   using unlocked = py::call_guard<py::gil_scoped_release>;
   m.def("layer_parallel", &layer_parallel, unlocked());
+  m.def("layer_prefill", &layer_prefill, unlocked());
   m.def("product", [](const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epilogue, const std::optional<Tensor>& aux) {
     return product(a, a_t, b, b_t, epilogue, aux);
   }, unlocked());

@@ -320,6 +320,50 @@ def test_sampler_reuses_its_captured_graph_for_a_new_prompt():
 
 
 @pytest.mark.gpu
+def test_prompts_go_into_the_buffers_of_the_kept_decoder():
+    """A later prompt's caches are written where the kept graph reads them: other lengths and batches, new weights, an eager call and a
+    replaced `forward` in between; what a decoder of its own would pick."""
+    from lookahead_keys_attention_amd import _native
+
+    model = make_lm(depth=2, dim=128, heads=2, dim_head=64, rotary=True, native=True).cuda()
+
+    def check(batch, n, steps=20, reused=True):
+        kept = model.__dict__.get("_kept_decoder")
+        held = [buf.data_ptr() for st in kept.stores for buf in st.buffers] if kept is not None else None
+        prompt = tokens(batch, n, seed=n).cuda()
+        got = model.sample(prompt, seq_len=n + steps, temperature=0.0)
+        now = model._kept_decoder
+        assert ([buf.data_ptr() for st in now.stores for buf in st.buffers] == held) == reused
+        assert (now is kept) == (reused and kept.signature == now.signature)
+        mine = model._kept_decoder
+        model.release_decoder()
+        assert torch.equal(got, model.sample(prompt, seq_len=n + steps, temperature=0.0))
+        model.__dict__["_kept_decoder"] = mine
+
+    check(2, 30, reused=False)
+    check(2, 30)
+    check(2, 7)
+    check(2, 200, steps=100)
+    check(3, 30, reused=False)
+    model.sample(tokens(3, 9, seed=1).cuda(), seq_len=13)   # steps without a graph, in buffers of their own
+    check(3, 31)
+    with torch.no_grad():   # new weights: the graph goes, the buffers stay
+        model.to_logits.weight = torch.nn.Parameter(model.to_logits.weight.flip(0).clone())
+    prompt = tokens(3, 12, seed=2).cuda()
+    before = model._kept_decoder
+    got = model.sample(prompt, seq_len=30, temperature=0.0)
+    assert model._kept_decoder is not before and torch.equal(got, model.sample(prompt, seq_len=30, temperature=0.0, graph=False))
+    check(3, 18)
+    attention, norm = model.layers[0][0], model.layers[0][0].norm
+    x, buffers = torch.randn(3, 10, 128, device="cuda"), list(model._kept_decoder.stores[0].buffers)
+    for wrong in (buffers[:3], [b[:, :, :9] for b in buffers], [b[:2] for b in buffers], [b.half() for b in buffers]):
+        with torch.no_grad(), pytest.raises(ValueError):
+            _native.host().layer_prefill(x, None, norm.weight, norm.eps, attention.to_all_qkv.weight, attention.combine_heads.weight, 2, 0.125, 0, wrong)
+    with pytest.raises(ValueError):
+        _native.host().layer_prefill(x, None, norm.weight, norm.eps, attention.to_all_qkv.weight, attention.combine_heads.weight, 2, 0.125, 0, buffers)
+
+
+@pytest.mark.gpu
 def test_decode_step_with_an_out_of_range_device_count_writes_nothing():
     from lookahead_keys_attention_amd import ops
     from lookahead_keys_attention_amd.castle import _CacheStore
