@@ -339,6 +339,19 @@ int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns)
 int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
                 int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same of normalised rows, castle_rms_norm without a summand and castle_gemm of two contraction-contiguous operands in one launch: c
+ * = (a / sqrt(mean(a^2) + eps) * weight, rounded to the type) b^T.  h (M rows of K) and rstd (M floats) keep the normalised rows and their
+ * factors, or are NULL; rstd needs h.  For few rows: only where castle_gemm_norm_ok says so. */
+typedef struct castle_gemm_norm {
+  const void* weight;
+  float eps;
+  void* h;
+  float* rstd;
+} castle_gemm_norm;
+int castle_gemm_norm_ok(int M, int N, int K, int dtype);
+int castle_gemm_of_norm(const void* a, int64_t lda, const castle_gemm_norm* norm, const void* b, int64_t ldb, void* c, int64_t ldc, int M, int N, int K,
+                        int dtype, const castle_amax* amax, void* stream);
+
 /* out[i] = sum over p < parts of part[p * n + i], n % 8 == 0: partial products of a weight gradient. */
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream);
 

@@ -54,6 +54,8 @@ EXPORTED_SYMBOLS = (
     "castle_gemm_workspace_bytes",
     "castle_gemm_amax_ok",
     "castle_gemm",
+    "castle_gemm_norm_ok",
+    "castle_gemm_of_norm",
     "castle_rms_norm",
     "castle_rms_norm_bwd_workspace_bytes",
     "castle_rms_norm_bwd",

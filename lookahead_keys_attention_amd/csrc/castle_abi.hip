@@ -621,7 +621,12 @@ int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns)
 // The kernel forms element offsets in 32 bits and runs ahead of the last row by up to three steps of the contraction.
 int castle_gemm_operand_ok(int64_t rows, int64_t ld) { return rows >= 0 && ld >= 0 && ld < (int64_t)1 << 31 && rows < (int64_t)1 << 31 && (rows + 192) * ld < (int64_t)1 << 31; }
 
-int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
+int castle_gemm_norm_ok(int M, int N, int K, int dtype) {
+  const int es = elem_size(dtype);
+  return es != 0 && M > 0 && N > 0 && K > 0 && K % (16 / es) == 0 && N % (16 / es) == 0 && castle::gemm_norm_ok(M, N, K, es) ? 1 : 0;
+}
+
+static int gemm_common(const castle_gemm_norm* norm, const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
                 int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream) {
   const int64_t need = castle_gemm_workspace_bytes(M, N, K, dtype, epilogue);
   if (need < 0) return (int)need;
@@ -637,7 +642,17 @@ int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b
     return CASTLE_ERR_ARG;
   if (need > 0 && (ldc != N || (int64_t)M * N % 8 != 0)) return CASTLE_ERR_SHAPE;
   if (need > 0 && (workspace == nullptr || !aligned16({workspace}) || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
-  castle::GemmArgs args = {a, b, c, aux, M, N, K, lda, ldb, ldc, epilogue, 0, nullptr, nullptr, nullptr, 0, 1};
+  castle::GemmArgs args = {a, b, c, aux, M, N, K, lda, ldb, ldc, epilogue, 0, nullptr, nullptr, nullptr, 0, 1, nullptr, 0.f, nullptr, nullptr};
+  if (norm != nullptr) {
+    if (!castle_gemm_norm_ok(M, N, K, dtype) || a_free_contiguous || b_free_contiguous || epilogue != CASTLE_GEMM_PLAIN) return CASTLE_ERR_SHAPE;
+    if (norm->weight == nullptr || !(norm->eps >= 0.f) || !aligned16({norm->h}) || reinterpret_cast<uintptr_t>(norm->weight) % elem_size(dtype) != 0 ||
+        reinterpret_cast<uintptr_t>(norm->rstd) % 4 != 0 || (norm->rstd != nullptr && norm->h == nullptr))
+      return CASTLE_ERR_ARG;
+    args.norm_w = norm->weight;
+    args.eps = norm->eps;
+    args.h = norm->h;
+    args.rstd = norm->rstd;
+  }
   if (amax != nullptr) {
     if (!castle_gemm_amax_ok(M, N, K, dtype, amax->column, amax->columns)) return CASTLE_ERR_SHAPE;
     if (amax->partials == nullptr || reinterpret_cast<uintptr_t>(amax->partials) % 4 != 0 || reinterpret_cast<uintptr_t>(amax->status) % 4 != 0) return CASTLE_ERR_ARG;
@@ -647,6 +662,16 @@ int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b
     args.amax_to = amax->column + amax->columns;
   }
   return castle::launch_gemm(args, !a_free_contiguous, !b_free_contiguous, dtype, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+}
+
+int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
+                int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream) {
+  return gemm_common(nullptr, a, lda, a_free_contiguous, b, ldb, b_free_contiguous, c, ldc, M, N, K, dtype, epilogue, aux, amax, workspace, workspace_bytes, stream);
+}
+int castle_gemm_of_norm(const void* a, int64_t lda, const castle_gemm_norm* norm, const void* b, int64_t ldb, void* c, int64_t ldc, int M, int N, int K,
+                        int dtype, const castle_amax* amax, void* stream) {
+  if (norm == nullptr) return CASTLE_ERR_ARG;
+  return gemm_common(norm, a, lda, 0, b, ldb, 0, c, ldc, M, N, K, dtype, CASTLE_GEMM_PLAIN, nullptr, amax, nullptr, 0, stream);
 }
 
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream) {

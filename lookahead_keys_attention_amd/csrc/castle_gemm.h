@@ -20,7 +20,14 @@ struct GemmArgs {
   float* amax;
   int* amax_status;   // set to 0 if not nullptr
   int amax_from, amax_to;
+  // rows of `a` are normalised on their way: a / sqrt(mean(a^2) + eps) * norm_w, kept in h (ld K) and their factors in rstd if not nullptr
+  const void* norm_w;
+  float eps;
+  void* h;
+  float* rstd;
 };
+constexpr int kNormBytes = 2048;   // longest row that a product normalises
+bool gemm_norm_ok(int M, int N, int K, int elem_size);
 bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to);
 int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue);
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream);

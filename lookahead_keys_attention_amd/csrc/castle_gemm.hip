@@ -97,7 +97,9 @@ template <typename T, bool KC, int FREE, int BK, int G> struct Operand {
 
 // G: groups of four waves.  Two take alternate steps of the contraction for the same tile, each in LDS of its own, and are summed at
 // the end: where the tiles leave a CU one workgroup, a second wave per SIMD works while the first waits for LDS and barrier.
-template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G>
+// NORM: the rows of `a` are normalised between memory and LDS, one tile per workgroup.  Every workgroup reads its 64 rows once for
+// their factors, with the first steps already on their way; that beats a launch in front of the product where the GPU is nearly empty.
+template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G, bool NORM = false>
 __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(GemmArgs a) {
   constexpr int WM = BM / 64, WN = BN / 64;   // 32-wide pieces of a wave's quarter
   typedef Operand<T, AK, BM, BK, G> OpA;
@@ -130,10 +132,25 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
       rb.load(p, pb, (int)a.ldb, k0 + (p * G + group) * BK, k_end);
     }
   };
+  __shared__ __attribute__((aligned(16))) float s_norm[NORM ? kNormBytes / (int)sizeof(T) : 4], s_factor[NORM ? BM : 1];
+  const int m_first = tile / tiles_n * BM;
+  const bool norm_keeps = NORM && a.h != nullptr && tile % tiles_n == 0;   // (the first column of tiles stores what all of them form)
   auto step = [&](auto parity, int it) __attribute__((always_inline)) {
     constexpr int p = decltype(parity)::value;
     T* la = stage + p * (OpA::ELEMS + OpB::ELEMS);
     T* lb = la + OpA::ELEMS;
+    if constexpr (NORM) {
+      const int k = k0 + (it * G + group) * BK;
+#pragma unroll
+      for (int j = 0; j < OpA::N; ++j) {
+        const int row = OpA::row_of(j), col = k + OpA::col_of(j);
+        typedef vec<float, V> vf;
+        if (col < a.K) {
+          ra.r[p][j] = __builtin_convertvector(__builtin_convertvector(ra.r[p][j], vf) * s_factor[row] * *reinterpret_cast<const vf*>(s_norm + col), vec<T, V>);
+          if (norm_keeps && m_first + row < a.M) *reinterpret_cast<vec<T, V>*>(static_cast<T*>(a.h) + (int64_t)(m_first + row) * a.K + col) = ra.r[p][j];
+        }
+      }
+    }
     ra.store(p, la);
     rb.store(p, lb);
     if (it + 2 < steps) {
@@ -160,6 +177,31 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
     if (threadIdx.x == 0 && a.amax_status != nullptr) *a.amax_status = 0;
   }
   if (tile < last) request();
+  if constexpr (NORM) {
+    if (tile < last) {
+      constexpr int LPR = kThreads * G / BM;   // lanes of a row
+      static_assert(64 % LPR == 0, "a row in one wave");
+      typedef vec<float, V> vf;
+      const int row = threadIdx.x / LPR, sub = threadIdx.x % LPR;
+      const T* x = pa + (int64_t)min(m_first + row, a.M - 1) * a.lda;
+      float ssq = 0.f;
+#pragma unroll 4
+      for (int i = sub; i < a.K / V; i += LPR) {
+        const vf v = __builtin_convertvector(*reinterpret_cast<const vec<T, V>*>(x + i * V), vf);
+#pragma unroll
+        for (int e = 0; e < V; ++e) ssq = __builtin_fmaf(v[e], v[e], ssq);
+      }
+      for (int i = threadIdx.x; i < a.K; i += kThreads * G) s_norm[i] = (float)static_cast<const T*>(a.norm_w)[i];
+#pragma unroll
+      for (int o = 1; o < LPR; o <<= 1) ssq += __shfl_xor(ssq, o);
+      const float r = 1.f / sqrtf(ssq / (float)a.K + a.eps);
+      if (sub == 0) {
+        s_factor[row] = r;
+        if (norm_keeps && a.rstd != nullptr && m_first + row < a.M) a.rstd[m_first + row] = r;
+      }
+      __syncthreads();
+    }
+  }
   while (tile < last) {
     const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
 #pragma unroll
@@ -637,14 +679,27 @@ bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to
   return p.splits == 1 && (int64_t)((M + p.rows() - 1) / p.rows()) * per_row <= kAmaxBlocks;
 }
 
+// One tile per workgroup and a CU for each, so that a row is read for its factor where it costs nothing else.
+bool gemm_norm_ok(int M, int N, int K, int elem_size) {
+  return K * elem_size <= kNormBytes && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 256 && plan(M, N, K, true, elem_size).splits == 1;
+}
+
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream) {
   const int es = dtype == 0 ? 4 : 2, step = dtype == 0 ? kStep32 : kStep16;
   Plan p = plan(a.M, a.N, a.K, a.epilogue == kGemmPlain || a.amax != nullptr, es);   // (the slots of the maxima follow from the plain plan)
   a.k_per_split = ((a.K + p.splits - 1) / p.splits + step - 1) / step * step;
   p.splits = (a.K + a.k_per_split - 1) / a.k_per_split;   // rounding up may leave the last ones empty
   a.part = p.splits > 1 ? workspace : nullptr;
+  if (a.norm_w != nullptr) p = {64, 1, (a.K + step - 1) / step >= 4 ? 2 : 1};
   const int rc = by_type(dtype, true, [&](auto t, auto) {
     using T = decltype(t);
+    if (a.norm_w != nullptr) {
+      constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
+      const dim3 grid((p.tiles(a.M, a.N) + 7) / 8 * 8);
+      if (p.groups == 2) hipLaunchKernelGGL((gemm_kernel<T, true, true, 64, 64, BK, 2, true>), grid, dim3(2 * kThreads), 0, stream, a);
+      else hipLaunchKernelGGL((gemm_kernel<T, true, true, 64, 64, BK, 1, true>), grid, dim3(kThreads), 0, stream, a);
+      return hipGetLastError() == hipSuccess ? 0 : -3;
+    }
     if (a_kc && b_kc) return launch_t<T, true, true>(a, p, stream);
     if (a_kc) return launch_t<T, true, false>(a, p, stream);
     if (!b_kc) return launch_t<T, false, false>(a, p, stream);

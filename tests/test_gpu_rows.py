@@ -286,6 +286,49 @@ def test_products_of_wide_tiles(rows, n, k, dtype):
         test_product_leaves_partial_maxima(rows, n, k, 520, 256)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 8), (63, 72, 40), (96, 768, 128), (65, 264, 264), (130, 1536, 512), (200, 136, 456), (1000, 640, 1000)])
+def test_product_of_normalised_rows(rows, n, k, dtype):
+    """Norm and product in one launch, with and without what a backward pass reads: remainders in every direction, one group of waves and two."""
+    import ctypes
+
+    from lookahead_keys_attention_amd import _native as N
+
+    class Norm(ctypes.Structure):
+        _fields_ = [("weight", ctypes.c_void_p), ("eps", ctypes.c_float), ("h", ctypes.c_void_p), ("rstd", ctypes.c_void_p)]
+
+    lib, code = N.lib(), N.DTYPE_CODES[dtype]
+    vp, i, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64
+    lib.castle_gemm_of_norm.argtypes = [vp, i64, ctypes.POINTER(Norm), vp, i64, vp, i64, i, i, i, i, vp, vp]
+    if not lib.castle_gemm_norm_ok(rows, n, k, code):
+        assert dtype is torch.float32   # a row too long, or a contraction that is better split
+        return
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, w, weight = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((rows, k + 8), (n, k), (k,)))
+    x = (x * torch.logspace(-3, 2, rows, device=DEV)[:, None]).to(dtype)
+    bits = {torch.float32: 24, torch.bfloat16: 8, torch.float16: 11}[dtype]
+    factor = (x[:, :k].double().square().mean(dim=-1) + 1e-6).rsqrt()
+    rows_ref = x[:, :k].double() * factor[:, None] * weight.double()
+    out = []
+    for keep in (True, False):
+        c, h, rstd = torch.full((rows, n + 8), 7.0, device=DEV, dtype=dtype), torch.full((rows, k), 7.0, device=DEV, dtype=dtype), torch.full((rows,), 7.0, device=DEV)
+        norm = Norm(weight.data_ptr(), 1e-6, h.data_ptr() if keep else None, rstd.data_ptr() if keep else None)
+        N.check(lib.castle_gemm_of_norm(x.data_ptr(), k + 8, ctypes.byref(norm), w.data_ptr(), k, c.data_ptr(), n + 8, rows, n, k, code, None,
+                                        N.stream_ptr(x.device)), "castle_gemm_of_norm")
+        torch.cuda.synchronize()
+        out.append(c)
+        assert torch.all(c[:, n:] == 7)
+        if keep:
+            # (the factor: k squares and k sums of 2^-24 each, at most; halved by the root)
+            assert torch.all((rstd.double() - factor).abs() <= (k + 4) * 2.0 ** -24 * factor)
+            small = 2.0 ** -24 if dtype is torch.float16 else 0.0   # half of the smallest step
+            assert torch.all((h.double() - rows_ref).abs() <= (2.0 ** -bits + (k + 8) * 2.0 ** -24) * rows_ref.abs() + small)
+            ref = h.double() @ w.double().t()
+    assert torch.equal(out[0], out[1])
+    bound = (k + 4) * 2.0 ** -24 * (rows_ref.abs() @ w.double().abs().t()) + 2.0 ** -bits * ref.abs() + (2.0 ** -24 if dtype is torch.float16 else 0.0)
+    assert torch.all((out[0][:, :n].double() - ref).abs() <= 1.01 * bound)
+
+
 def test_projection_of_rows_beyond_32_bit_offsets():
     """Rows that lie further apart than the products' offsets reach: 40000 of them, 65536 elements apart."""
     from lookahead_keys_attention_amd import Castle
