@@ -248,8 +248,12 @@ __global__ __launch_bounds__(kThreads, (scan_waves_per_simd<T, HD>())) void scan
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, typename TI, int HD>
-__global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(FwdArgs a) {
+// G: groups of four waves.  Two take alternate chunks of the keys of the same rows, each in LDS of its own, and are merged at the end: a
+// workgroup with a CU to itself then has the two waves per SIMD that the kernel needs, from its first chunk to its last.  Where the longest
+// row block is the time (d = 128; forward pass, one group / two: 2 x 16 heads x 2048 rows 276 / 264 us, 1 x 16 x 4096 482 / 458, 6 x 16 x 333 81 /
+// 75); a GPU that is full anyway does the same work faster in separate workgroups (3 x 16 x 2048 378 / 408).
+template <typename T, typename TI, int HD, int G>
+__global__ __launch_bounds__(kThreads * G, sizeof(T) == 2 ? 2 : 1) void attn_kernel(FwdArgs a) {
   constexpr int KS = HD / 16;
   constexpr int HDP = HD < 32 ? 32 : HD;
   constexpr int NT = HDP / 32;
@@ -260,7 +264,8 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
   constexpr int LDK = lds_ld_tr<T>(HD), LDV = lds_ld_chain<T>(kNB), LDA = lds_ld<T>(QB);
   constexpr bool PF = use_prefetch<T, HD>();
   constexpr bool TRV = sizeof(T) == 2;
-  T* s_kc = reinterpret_cast<T*>(castle_smem);   // [CK][LDK]
+  const int tid = G == 1 ? threadIdx.x : threadIdx.x % kThreads, group = G == 1 ? 0 : wave_id() / 4;
+  T* s_kc = reinterpret_cast<T*>(castle_smem + group * attn_lds_bytes<T, HD>());   // [CK][LDK]
   T* s_qu = s_kc + CK * LDK;                     // [CK][LDK]
   T* s_ub0 = s_qu + CK * LDK;                    // [NBLK_Q][CK][LDK]
   T* s_vct = s_ub0 + NBLK_Q * CK * LDK;          // fp32: [HDP][LDV] (transposed); 16-bit: [CK][LDK]
@@ -269,13 +274,12 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
   constexpr int LDT = lds_ld<T>(kNB);
   T* s_t = s_a + CK * LDA;                                    // [QB][LDT], only if TL
 
-  prio_by_band(blockIdx.x, a.s.cus);
+  if (G == 1) prio_by_band(blockIdx.x, a.s.cus);
   int rank, bh;
-  if ((int)gridDim.x <= 2 * a.s.cus) work_item_snake(a.s.B * a.s.H, a.s.Lp / 128, a.s.cus, rank, bh);
-  else work_item(a.s.B * a.s.H, rank, bh);
+  work_item(a.s.B * a.s.H, rank, bh);
   const int qb = a.s.Lp / 128 - 1 - rank;   // the last query block sees the most keys
   const int b = bh / a.s.H, h = bh % a.s.H;
-  const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
+  const int lane = lane_id(), wave = G == 1 ? wave_id() : wave_id() % 4, c = lane & 31, g = lane >> 5;
   const int L = a.s.L;
   const float c1 = a.s.scale * kLog2e;
   const float su_mul = a.ws.hdr->su_mul;   // Su = su_mul * (the product built from vu * vu_scale)
@@ -322,26 +326,26 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
   SnapStage<T, CK, HD> pub[NBLK_Q];
   auto load_chunk = [&](int ck) __attribute__((always_inline)) {   // chunk ck = keys [ck*CK, ck*CK + CK)
     const int Kb = ck * CK / kNB;
-    pkc.load_flat(kc + (int64_t)ck * CK * HD);
-    if (TRV) pvr.load_flat(vc + (int64_t)ck * CK * HD);
+    pkc.load_flat(kc + (int64_t)ck * CK * HD, tid);
+    if (TRV) pvr.load_flat(vc + (int64_t)ck * CK * HD, tid);
     else pvc.load(vc, HD, (int64_t)ck * CK, kNoRowLimit);
-    pqu.load_flat(qu + (int64_t)ck * CK * HD);
+    pqu.load_flat(qu + (int64_t)ck * CK * HD, tid);
 #pragma unroll
     for (int q = 0; q < NBLK_Q; ++q) {
       const int blk = Ifirst + q;
-      if (Kb < blk && blk < a.s.nblk) pub[q].load(snap + (usnap_off(blk) + (int64_t)ck * CK) * HD);
+      if (Kb < blk && blk < a.s.nblk) pub[q].load(snap + (usnap_off(blk) + (int64_t)ck * CK) * HD, tid);
     }
   };
   auto store_chunk = [&](int ck) __attribute__((always_inline)) {
     const int Kb = ck * CK / kNB;
-    pkc.store(s_kc, LDK);
-    if (TRV) pvr.store(s_vct, LDK);
+    pkc.store(s_kc, LDK, tid);
+    if (TRV) pvr.store(s_vct, LDK, tid);
     else pvc.store(s_vct, LDV);
-    pqu.store(s_qu, LDK);
+    pqu.store(s_qu, LDK, tid);
 #pragma unroll
     for (int q = 0; q < NBLK_Q; ++q) {
       const int blk = Ifirst + q;
-      if (Kb < blk && blk < a.s.nblk) pub[q].store(s_ub0 + q * CK * LDK, LDK);
+      if (Kb < blk && blk < a.s.nblk) pub[q].store(s_ub0 + q * CK * LDK, LDK, tid);
     }
   };
 
@@ -352,15 +356,15 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
 #pragma unroll
   for (int s = 0; s < kNB / 16; ++s)
     if (!TL) asm volatile("" : "+v"(ft[s]));
-  if (PF) load_chunk(0);
-  for (int ck = 0; ck < nchunks; ++ck) {
-    const int Kb = ck * CK / kNB;
+  if (PF && group < nchunks) load_chunk(group);
+  for (int it = 0; it < nchunks; it += G) {
+    const int ck = it + group, Kb = ck * CK / kNB;
     __syncthreads();
     if (!PF) load_chunk(ck);
-    store_chunk(ck);
-    if (PF && ck + 1 < nchunks) load_chunk(ck + 1);   // in flight while this chunk is processed
+    if (G == 1 || ck < nchunks) store_chunk(ck);
+    if (PF && ck + G < nchunks) load_chunk(ck + G);   // in flight while this chunk is processed
     __syncthreads();
-    const bool active = Kb <= Iw;
+    const bool active = Kb <= Iw && (G == 1 || ck < nchunks);
     if (active) {
       // gate tile for this wave's 32 source rows: A^T[j rows, k lanes]
 #pragma unroll
@@ -454,6 +458,31 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 2 ? 2 : 1) void attn_kernel(
       }
     }
   }
+  if constexpr (G == 2) {
+    static_assert(kThreads * (16 * NT + 2) * 4 <= 2 * attn_lds_bytes<T, HD>(), "one group's sums");
+    float* sums = reinterpret_cast<float*>(castle_smem);
+    asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");   // the loop may end right behind a product
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    if (group == 1) {
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[(16 * nt + r) * kThreads + tid] = o[nt][r];
+      sums[16 * NT * kThreads + tid] = m;
+      sums[(16 * NT + 1) * kThreads + tid] = l;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    // a row always has a key in the first chunk; the second group may have none: maximum -inf, sums 0
+    const float m1 = sums[16 * NT * kThreads + tid], both = fmaxf(m, m1), f0 = fast_exp2(m - both), f1 = fast_exp2(m1 - both);
+    l = l * f0 + sums[(16 * NT + 1) * kThreads + tid] * f1;
+    m = both;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[nt][r] = o[nt][r] * f0 + sums[(16 * nt + r) * kThreads + tid] * f1;
+  }
   const float lt = l + __shfl_xor(l, 32);
   if (i < L) {
     const float inv = 1.f / lt;
@@ -502,14 +531,26 @@ template <typename T, typename TI, int HD> static int launch_scan_t(const FwdArg
 template <typename T, typename TI, int HD> static int launch_attn_t(const FwdArgs& a, hipStream_t stream) {
   constexpr int attn_lds = attn_lds_bytes<T, HD>();
   static_assert(attn_lds <= kMaxLds, "attention kernel does not fit the LDS");
+  constexpr bool PAIRS = sizeof(T) == 2 && HD == 128;
   static PerDeviceOnce once;
   bool& configured = once.flag();
   if (!configured) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_kernel<T, TI, HD>), hipFuncAttributeMaxDynamicSharedMemorySize, attn_lds) != hipSuccess) return -3;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_kernel<T, TI, HD, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, attn_lds) != hipSuccess) return -3;
+    if constexpr (PAIRS) {
+      static_assert(2 * attn_lds <= kMaxLds, "two groups do not fit the LDS");
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_kernel<T, TI, HD, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, 2 * attn_lds) != hipSuccess) return -3;
+    }
     configured = true;
   }
   ProfScope ps(kSlotAttn, stream);
-  hipLaunchKernelGGL((attn_kernel<T, TI, HD>), dim3(a.s.Lp / 128 * a.s.B * a.s.H), dim3(kThreads), attn_lds, stream, a);
+  const dim3 grid(a.s.Lp / 128 * a.s.B * a.s.H);
+  if constexpr (PAIRS) {
+    if ((int)grid.x <= 2 * a.s.cus) {   // as far as the longest row blocks and not their sum bound the launch
+      hipLaunchKernelGGL((attn_kernel<T, TI, HD, 2>), grid, dim3(2 * kThreads), 2 * attn_lds, stream, a);
+      return hipGetLastError() == hipSuccess ? 0 : -3;
+    }
+  }
+  hipLaunchKernelGGL((attn_kernel<T, TI, HD, 1>), grid, dim3(kThreads), attn_lds, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

@@ -481,7 +481,7 @@ __device__ __forceinline__ void work_item(int BH, int& rank, int& bh) {
 // The same for a kernel of which two or more workgroups fit a CU, `n` ranks in all, when all or most of them are resident at
 // once: nothing is handed out later to level the load.  Workgroups are handed out one per CU first, then a second
 // each: CU k has items k and k + cus, and in the order above the long rows of both bands meet.  So every second band
-// runs the other way.  (d = 128 attention, 2 x 16 heads x 2048 rows: 206 -> 185 us; key_narrow, 8 heads x 2000 rows: 97 -> 87.)
+// runs the other way.  (key_narrow, 8 heads x 2000 rows: 97 -> 87 us.)
 __device__ __forceinline__ void work_item_snake(int BH, int n, int cus, int& rank, int& bh) {
   work_item(BH, rank, bh);
   const int band = cus / BH;   // ranks of a band

@@ -109,6 +109,23 @@ def test_operator_with_long_walks_shared_by_eight_waves(B, Hh, L, d):
     test_operator_at_tile_edges_with_few_and_with_many_heads(B, Hh, L, d, torch.bfloat16)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hh,L", [(300, 1), (257, 33), (512, 96), (257, 128), (130, 129), (100, 352), (40, 1000)])
+def test_wide_heads_by_two_groups_of_waves(Hh, L, dtype):
+    """d = 128 at one and two row blocks a CU, where two groups of waves share the keys of a row, against the same heads among others: one
+    chunk, odd and even numbers of them, a last one that only the first group has."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    six = [torch.randn(1, Hh, L, 128, generator=g, device="cuda").to(dtype) for _ in range(6)]
+    blocks = Hh * ((L + 127) // 128)
+    assert 256 < blocks <= 512
+    few = H().castle_attention_hip(*six, 128 ** -0.5)
+    many = H().castle_attention_hip(*(t.repeat(512 // blocks + 1, 1, 1, 1) for t in six), 128 ** -0.5)
+    # both round their sums of at most the largest value, of weights rounded to fp16 behind maxima of their own
+    bits = 8 if dtype == torch.bfloat16 else 11
+    bound = 2.0 ** -(bits - 1) * many[0].float().abs() + 2.0 ** -9 * six[2].float().abs().max()
+    assert torch.isfinite(few).all() and torch.all((few[0].float() - many[0].float()).abs() <= bound)
+
+
 @pytest.mark.parametrize("L,d", [(256, 64), (200, 32)])
 def test_bf16_operand_flag_forward_and_backward(L, d, monkeypatch):
     """CASTLE_FLAG_BF16_OPERANDS keeps bf16 MFMA operands (default: fp16 operands for bf16 tensors)."""
