@@ -1632,10 +1632,10 @@ template <typename T, int HD> constexpr int bwd_query2_lds_bytes() {
 template <typename T, bool CHAINED>
 struct TileStage {
   vec<T, 8> r;
-  __device__ __forceinline__ void load(const T* src) {
+  template <bool SCALAR = true> __device__ __forceinline__ void load(const T* src) {
     const int slab = threadIdx.x >> 6, l = threadIdx.x & 63;       // slab = 2 * tile + s2
     const int g = (l >> 4) & 1, k = (l & 15) + 16 * (l >> 5);
-    r = __builtin_nontemporal_load(reinterpret_cast<const frag_mem<T>*>(src + slab * 512 + k * 16 + g * 8));   // read once
+    r = load_once_at<frag_mem<T>, SCALAR>(src, (slab * 512 + k * 16 + g * 8) * (int)sizeof(T));
   }
   __device__ __forceinline__ void store(T* dst) const {
     const int slab = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -1748,11 +1748,11 @@ __global__ __launch_bounds__(2 * kThreads, 2) void bwd_query2_kernel(BwdArgs a) 
     SnapStage<T, kCK, HD> pu;
 #define CASTLE_BQ2_LOAD_A(K0)                                                            \
   do {                                                                                   \
-    pkc.load_flat(kc + (int64_t)(K0) * HD, tid);                                         \
-    pqu.load_flat(qu + (int64_t)(K0) * HD, tid);                                         \
-    if ((K0) / kNB < blk0) pu.load(usnap + (usnap_off(blk0) + (K0)) * HD, tid);          \
-    pds.load(dsm + (int64_t)((K0) / 32) * tile_row);                                     \
-    pdsu.load(dsum + (int64_t)((K0) / 32) * tile_row);                                   \
+    pkc.template load_flat<false>(kc + (int64_t)(K0) * HD, tid);                                         \
+    pqu.template load_flat<false>(qu + (int64_t)(K0) * HD, tid);                                         \
+    if ((K0) / kNB < blk0) pu.template load<false>(usnap + (usnap_off(blk0) + (K0)) * HD, tid);          \
+    pds.template load<false>(dsm + (int64_t)((K0) / 32) * tile_row);                                     \
+    pdsu.template load<false>(dsum + (int64_t)((K0) / 32) * tile_row);                                   \
   } while (0)
     CASTLE_BQ2_LOAD_A(0);
     for (int k0 = 0; k0 < kend; k0 += kCK) {
@@ -1839,8 +1839,8 @@ __global__ __launch_bounds__(2 * kThreads, 2) void bwd_query2_kernel(BwdArgs a) 
     __syncthreads();   // e1: chunk tiles dead
     {
       RowStage<T, T, QB, HD, 2 * kThreads> st;
-      st.load_flat(vu + (int64_t)qb * QB * HD); st.store(e_vu, LDK);
-      st.load_flat(qc + (int64_t)qb * QB * HD); st.store(e_qc, LDK);
+      st.template load_flat<false>(vu + (int64_t)qb * QB * HD); st.store(e_vu, LDK);
+      st.template load_flat<false>(qc + (int64_t)qb * QB * HD); st.store(e_qc, LDK);
     }
     __syncthreads();   // e2: epilogue tiles and dT shared
     if (i < L) store_rows<TI, HD, NT>(head_ptr_mut<TI>(a.dku, b, h) + (int64_t)i * a.dku.sl, dku, c0 * kLn2 * gun, g, a.s.rotary ? i : -1);
@@ -1858,9 +1858,9 @@ __global__ __launch_bounds__(2 * kThreads, 2) void bwd_query2_kernel(BwdArgs a) 
     SnapStage<T, kCK, HD> pg;
 #define CASTLE_BQ2_LOAD_B(K0)                                                                             \
   do {                                                                                                    \
-    if (has_g) pg.load(gsnap + (gsnap_off(blk1) + (K0)) * HD, tid);                                       \
-    pds.load(dsm + (int64_t)((K0) / 32) * tile_row);                                                      \
-    pdsu.load(dsum + (int64_t)((K0) / 32) * tile_row);                                                    \
+    if (has_g) pg.template load<false>(gsnap + (gsnap_off(blk1) + (K0)) * HD, tid);                                       \
+    pds.template load<false>(dsm + (int64_t)((K0) / 32) * tile_row);                                                      \
+    pdsu.template load<false>(dsum + (int64_t)((K0) / 32) * tile_row);                                                    \
   } while (0)
     CASTLE_BQ2_LOAD_B(0);
     for (int k0 = 0; k0 < kend; k0 += kCK) {
@@ -1920,8 +1920,8 @@ __global__ __launch_bounds__(2 * kThreads, 2) void bwd_query2_kernel(BwdArgs a) 
     __syncthreads();   // e1
     {
       RowStage<T, T, QB, HD, 2 * kThreads> st;
-      st.load_flat(vu + (int64_t)qb * QB * HD); st.store(e_vu, LDK);
-      st.load_flat(qc + (int64_t)qb * QB * HD); st.store(e_qc, LDK);
+      st.template load_flat<false>(vu + (int64_t)qb * QB * HD); st.store(e_vu, LDK);
+      st.template load_flat<false>(qc + (int64_t)qb * QB * HD); st.store(e_qc, LDK);
     }
     // dT^T[j rows, i lanes] masked to j <= i, shared as dT[i][j] for the source-side product
 #pragma unroll
@@ -2201,10 +2201,10 @@ __global__ __launch_bounds__(2 * kThreads, 2) void bwd_queryw_kernel(BwdArgs a) 
 #define CASTLE_BQW_LOAD_B(K0)                                                          \
   do {                                                                                 \
     if ((K0) / kNB < blk0) pu.load(usnap + (usnap_off(blk0) + (K0)) * HD, tid);        \
-    if (has_g) pg.load(gsnap + (gsnap_off(blk1) + (K0)) * HD, tid);                    \
     pds.load(dsm + (int64_t)((K0) / 32) * tile_row);                                   \
     pdsu.load(dsum + (int64_t)((K0) / 32) * tile_row);                                 \
   } while (0)
+    if (has_g) pg.load(gsnap + gsnap_off(blk1) * HD, tid);
     CASTLE_BQW_LOAD_B(0);
     for (int k0 = 0; k0 < kend; k0 += kCK) {
       const int Kb = k0 / kNB;
@@ -2224,21 +2224,24 @@ __global__ __launch_bounds__(2 * kThreads, 2) void bwd_queryw_kernel(BwdArgs a) 
           const frag<T> bds = ld_free<T, false>(s_ds, LDD, jw, 1 << 30, 16 * s2, c, g);
 #pragma unroll
           for (int n0 = 0; n0 < NT; n0 += 2) {
-            frag<T> okt[2], out[2];
+            frag<T> o2[2];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              okt[u] = ld_free<T, false>(s_kc, LDK, 32 * (n0 + u), HD, 16 * s2, c, g);
-              out[u] = ld_free<T, false>(s_ub, LDK, 32 * (n0 + u), HD, 16 * s2, c, g);
-            }
+            for (int u = 0; u < 2; ++u) o2[u] = ld_free<T, false>(s_kc, LDK, 32 * (n0 + u), HD, 16 * s2, c, g);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              mma(dqc[n0 + u], okt[u], bds);
-              if (Kb < blk0) mma(dqc[n0 + u], out[u], bdsu[s2]);
+            for (int u = 0; u < 2; ++u) mma(dqc[n0 + u], o2[u], bds);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) o2[u] = ld_free<T, false>(s_ub, LDK, 32 * (n0 + u), HD, 16 * s2, c, g);
+            if (Kb < blk0) {
+#pragma unroll
+              for (int u = 0; u < 2; ++u) mma(dqc[n0 + u], o2[u], bdsu[s2]);
             }
           }
         }
       }
+      // requested with the others it did not fit the registers: the spilled piece was waited for on the spot, between the barriers
+      // (with the scalar bases and the smaller batches above: 1 x 16 heads x 16384 rows 22.05 -> 21.70 ms, 2 x 16 x 2048 771 -> 756 us in all)
+      if (has_g && k0 + kCK < kend) pg.load(gsnap + (gsnap_off(blk1) + k0 + kCK) * HD, tid);
       if (!live) continue;
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {   // two small batches of operand fragments: this role is at the register limit

@@ -60,13 +60,20 @@ template <bool STAGES = false> __device__ __forceinline__ void wave_lds_order() 
 // load covers 1 KB of consecutive addresses.  (MFMA fragments straight from global memory touch 32 lines per
 // load; a CU works through those one after the other, which made it the bottleneck of these kernels: the key kernel at
 // 3 x 4 heads of 1000 rows took 68 us that way.)
-template <typename T, int COLS> struct Flat32 {
+// SCALAR: see load_at
+template <typename T, int COLS, bool SCALAR = true> struct Flat32 {
   static constexpr int V = elem_traits<T>::vec16, VPR = COLS / V, N = 32 * VPR / 64, LD = lds_ld_tr<T>(COLS);
   vec<T, V> r[N];
   __device__ __forceinline__ void load(const T* rows) {
-    const int lane = lane_id();
+    if constexpr (SCALAR) {
+      const global_bytes base = scalar_base(rows);
+      const uint32_t at = lane_offset(lane_id() * 16);
 #pragma unroll
-    for (int n = 0; n < N; ++n) r[n] = *reinterpret_cast<const vec<T, V>*>(rows + (lane + 64 * n) * V);
+      for (int n = 0; n < N; ++n) r[n] = *(const __attribute__((address_space(1))) vec<T, V>*)(base + at + 1024 * n);
+    } else {
+#pragma unroll
+      for (int n = 0; n < N; ++n) r[n] = *reinterpret_cast<const vec<T, V>*>(rows + (lane_id() + 64 * n) * V);
+    }
   }
   __device__ __forceinline__ void store(T* tile, float mul) const {
     const int lane = lane_id();
@@ -200,7 +207,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
 
   frag<T> fq[KS];   // -c1 Qu rows of the keys
   if (wave == 0) {
-    Flat32<T, HD> f;
+    Flat32<T, HD, HD >= 64> f;
     f.load(qu + (int64_t)kw0 * HD);
     f.store(s_qu, -c1);
   }
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void scan_narrow_k
   auto sweep = [&](bool keep) __attribute__((always_inline)) {
     // source tiles of 32 rows, two per block; the rows of the next one are requested while one is worked on
     const int first = max(2 * lo, kt), last = min(2 * hi, ntile);
-    Flat32<T, HD> pk, pv;
+    Flat32<T, HD, HD >= 64> pk, pv;
     if (first < last) {
       pk.load(ku + (int64_t)first * 32 * HD);
       pv.load(vu + (int64_t)first * 32 * HD);
@@ -333,11 +340,11 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void attn_narrow_k
 
   for (int t = wave; t < 4; t += W) {
     if (t < 3) {
-      Flat32<T, HD> f;
+      Flat32<T, HD, HD >= 64> f;
       f.load(t == 0 ? qc + (int64_t)it * 32 * HD : ku + ((int64_t)I * kNB + 32 * (t - 1)) * HD);
       f.store(s_rows + t * 32 * LD, t == 0 ? 1.f : -c1);
     } else {
-      Flat32<T, kNB> f;
+      Flat32<T, kNB, HD >= 64> f;
       f.load(tb + (int64_t)it * 32 * kNB);
       f.store(s_t);
     }
@@ -359,7 +366,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void attn_narrow_k
   for (int nt = 0; nt < NT; ++nt) zero(o[nt]);
   float m = -INFINITY, l = 0.f;
 
-  Flat32<T, HD> pq, pk, pv;
+  Flat32<T, HD, HD >= 64> pq, pk, pv;
   frag<T> nu[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) nu[s] = zero_frag<T>();
@@ -494,7 +501,8 @@ template <typename T, int HD, int W> constexpr int key_narrow_lds() {
 template <typename T, typename TI, int HD, int W>
 __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_kernel(BwdArgs a) {
   constexpr int KS = HD / 16, NT = narrow_nt<HD>(), LD = lds_ld_tr<T>(HD), LDT = kLdT64<T>;
-  constexpr bool STAGES = sizeof(T) == 2 && HD == 64;   // two waves per SIMD just fit: 17 spilled registers instead of 41
+  constexpr bool SB = sizeof(T) == 4 || HD >= 64;   // scalar bases where the registers are short (d = 32, 32 heads x 777: 41.9 us without, 43.8 with)
+  constexpr bool STAGES = sizeof(T) == 2 && HD == 64;   // two waves per SIMD just fit
   const int L = a.s.L, BH = a.s.B * a.s.H, nblk = (L + kNB - 1) / kNB;
   int kt, bh;   // key tile 0 meets every query
   narrow_item<T, HD>(BH, (L + 31) / 32, a.s.cus, kt, bh);
@@ -521,14 +529,15 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
   const T* usnap = reinterpret_cast<const T*>(a.ws.usnap) + (int64_t)bh * snap_rows(a.s.nblk) * HD;
   T* gsnap = reinterpret_cast<T*>(a.gsnap) + (int64_t)bh * snap_rows(a.s.nblk) * HD;
   // dS / dSu tiles of these keys: element (key k, chained slot) of query tile it at it * 1024 + s2 * 512 + k * 16 + g * 8
-  const int64_t tile0 = (int64_t)bh * a.s.Lp * a.s.Lp + (int64_t)kt * (a.s.Lp / 32) * 1024 + c * 16 + g * 8;
+  const int64_t tile0 = (int64_t)bh * a.s.Lp * a.s.Lp + (int64_t)kt * (a.s.Lp / 32) * 1024;
+  const uint32_t tile_at = (c * 16 + g * 8) * (int)sizeof(T);
   T* ds_mat = reinterpret_cast<T*>(a.ds_mat) + tile0;
   T* dsu_mat = reinterpret_cast<T*>(a.dsu_mat) + tile0;
   const float* lse = a.ws.lse + (int64_t)bh * a.s.Lp;
   const float* delta = a.delta + (int64_t)bh * a.s.Lp;
 
   for (int t = wave; t < 3; t += W) {
-    Flat32<T, HD> f;
+    Flat32<T, HD, SB> f;
     f.load(prep_ptr<T>(t == 0 ? a.ws.qu_p : t == 1 ? a.ws.kc_p : a.ws.vc_p, bh, a.s.Lp, HD) + (int64_t)kw0 * HD);
     f.store(s_qu + t * 32 * LD, t == 0 ? -c1 : 1.f);
   }
@@ -550,8 +559,8 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
     }
   };
   // the next tiles, requested one step ahead
-  Flat32<T, HD> pa, pb;
-  Flat32<T, kNB> pt;
+  Flat32<T, HD, SB> pa, pb;
+  Flat32<T, kNB, SB> pt;
 
   acc_t G[NT];   // [n rows, k lanes]
 #pragma unroll
@@ -565,8 +574,8 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
     // (12 heads x 1000 rows: 50.9 -> 48.1 us)
     float nl = 0.f, nd = 0.f;
     auto sums = [&](int I) __attribute__((always_inline)) {
-      nl = lse[I * kNB + lane];
-      nd = delta[I * kNB + lane];
+      nl = load_at<float, SB>(lse + I * kNB, 4 * lane);
+      nd = load_at<float, SB>(delta + I * kNB, 4 * lane);
     };
     if (lo < hi) {
       pa.load(ku + (int64_t)lo * kNB * HD);
@@ -624,7 +633,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
         if (itl == 0) {
           pa.load(qc + ((int64_t)I * kNB + 32) * HD);
           pb.load(dout + ((int64_t)I * kNB + 32) * HD);
-          pt.load(tb + ((int64_t)I * kNB + 32) * kNB);
+          if (!STAGES) pt.load(tb + ((int64_t)I * kNB + 32) * kNB);
         } else {
           pa.load(ku + (int64_t)min(I + 1, nblk - 1) * kNB * HD);
         }
@@ -659,11 +668,14 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
           ds[r] = dsv;
           dsu[r] = -dsv * sp * su_mul;
         }
+        // (requested with the other two it is what does not fit the registers, and a spilled piece is waited for on the spot: 3 x 4 heads of 1000
+        // rows, layer with its gradients 186 -> 179 us, with the scalar bases)
+        if (STAGES && itl == 0) pt.load(tb + ((int64_t)I * kNB + 32) * kNB);
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
           const frag<T> fp = chain<T>(sc, s2), fds = chain<T>(ds, s2), fdsu = chain<T>(dsu, s2);
-          *reinterpret_cast<frag_mem<T>*>(ds_mat + (int64_t)it * 1024 + s2 * 512) = fds;   // whole lines per store
-          *reinterpret_cast<frag_mem<T>*>(dsu_mat + (int64_t)it * 1024 + s2 * 512) = fdsu;
+          store_at<frag_mem<T>, SB>(ds_mat + (int64_t)it * 1024 + s2 * 512, tile_at, fds);   // whole lines per store
+          store_at<frag_mem<T>, SB>(dsu_mat + (int64_t)it * 1024 + s2 * 512, tile_at, fdsu);
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) {
             const frag<T> qt = ld_free<T, true>(s_a, LD, 32 * nt, HD, 16 * s2, c, g);
@@ -717,7 +729,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
 #pragma unroll
     for (int itl = 0; itl < 2; ++itl)
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) fdsu[itl][s2] = *reinterpret_cast<const frag_mem<T>*>(dsu_mat + (int64_t)(2 * I + itl) * 1024 + s2 * 512);
+      for (int s2 = 0; s2 < 2; ++s2) fdsu[itl][s2] = load_at<frag_mem<T>, SB>(dsu_mat + (int64_t)(2 * I + itl) * 1024 + s2 * 512, tile_at);
     settle();
     if (I <= nblk - 2) store_snap_tile<T, HD, NT>(gsnap + (gsnap_off(I) + kw0) * HD, G, c, g);
 #pragma unroll
@@ -781,7 +793,8 @@ template <typename T, int HD, int W> constexpr int query_narrow_lds() {
 template <typename T, typename TI, int HD, int W>
 __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_kernel(BwdArgs a) {
   constexpr int KS = HD / 16, NT = narrow_nt<HD>(), LD = lds_ld_tr<T>(HD), LDX = kLdX<T>;
-  constexpr bool STAGES = sizeof(T) == 2;   // d = 64: 31 spilled registers instead of 77
+  constexpr bool SB = sizeof(T) == 4 || HD >= 64;   // scalar bases where the registers are short (d = 32, 32 heads x 777: 28.7 us without, 29.5 with)
+  constexpr bool STAGES = sizeof(T) == 2;   // d = 64: 13 spilled registers, none in the loop
   const int L = a.s.L, BH = a.s.B * a.s.H, ntile = (L + 31) / 32, nblk = (L + kNB - 1) / kNB;
   int rank, bh;
   narrow_item<T, HD>(BH, ntile, a.s.cus, rank, bh);
@@ -813,17 +826,18 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
   const T* ttb = reinterpret_cast<const T*>(a.ws.tt_blk) + (int64_t)bh * a.s.Lp * kNB;
   const T* usnap = reinterpret_cast<const T*>(a.ws.usnap) + (int64_t)bh * snap_rows(a.s.nblk) * HD + usnap_off(I) * HD;
   const T* gsnap = reinterpret_cast<const T*>(a.gsnap) + (int64_t)bh * snap_rows(a.s.nblk) * HD + (has_g ? gsnap_off(I) * HD : 0);
-  const T* ds_mat = reinterpret_cast<const T*>(a.ds_mat) + (int64_t)bh * a.s.Lp * a.s.Lp + (int64_t)it * 1024 + c * 16 + g * 8;
-  const T* dsu_mat = reinterpret_cast<const T*>(a.dsu_mat) + (int64_t)bh * a.s.Lp * a.s.Lp + (int64_t)it * 1024 + c * 16 + g * 8;
+  const T* ds_mat = reinterpret_cast<const T*>(a.ds_mat) + (int64_t)bh * a.s.Lp * a.s.Lp + (int64_t)it * 1024;
+  const T* dsu_mat = reinterpret_cast<const T*>(a.dsu_mat) + (int64_t)bh * a.s.Lp * a.s.Lp + (int64_t)it * 1024;
+  const uint32_t tile_at = (c * 16 + g * 8) * (int)sizeof(T);
   const int64_t tile_row = (int64_t)(a.s.Lp / 32) * 1024;   // between the tiles of consecutive key tiles
 
   for (int t = wave; t < 4; t += W) {
     if (t < 3) {
-      Flat32<T, HD> f;
+      Flat32<T, HD, SB> f;
       f.load(t == 0 ? ku + (int64_t)it * 32 * HD : t == 1 ? vu + (int64_t)it * 32 * HD : ku + (int64_t)I * kNB * HD);
       f.store(s_ku + t * 32 * LD, t == 1 ? 1.f : -c1);
     } else {
-      Flat32<T, kNB> f;
+      Flat32<T, kNB, SB> f;
       f.load(ttb + (int64_t)it * 32 * kNB);
       f.store(s_tt);
     }
@@ -843,24 +857,24 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
   // middle of their own): 8 heads x 2000 rows 58.3 -> 55.0 us, 2 x 3000 71.7 -> 67.5.  Not with one wave per SIMD (d = 128
   // 72.6 -> 84, fp32 118 -> 122: the registers then move between the two files).
   constexpr bool EARLY = narrow_waves<T, HD>() == 2;
-  Flat32<T, HD> pq;
+  Flat32<T, HD, SB> pq;
   frag<T> og[KS], fds[2], fdsu[2], fdsn[2];
   auto request = [&](int kt) __attribute__((always_inline)) {
     pq.load(qu + (int64_t)kt * 32 * HD);
     load_snap32<T, HD>(og, has_g ? gsnap + (int64_t)kt * 32 * HD : kc, c, g);
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      fds[s2] = *reinterpret_cast<const frag_mem<T>*>(ds_mat + kt * tile_row + s2 * 512);
-      fdsu[s2] = *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + s2 * 512);
-      if constexpr (EARLY) fdsn[s2] = *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + (next ? 1024 : 0) + s2 * 512);
-      else fdsn[s2] = next ? *reinterpret_cast<const frag_mem<T>*>(dsu_mat + kt * tile_row + 1024 + s2 * 512) : zero_frag<T>();
+      fds[s2] = load_at<frag_mem<T>, SB>(ds_mat + kt * tile_row + s2 * 512, tile_at);
+      fdsu[s2] = load_at<frag_mem<T>, SB>(dsu_mat + kt * tile_row + s2 * 512, tile_at);
+      if constexpr (EARLY) fdsn[s2] = load_at<frag_mem<T>, SB>(dsu_mat + kt * tile_row + (next ? 1024 : 0) + s2 * 512, tile_at);
+      else fdsn[s2] = next ? load_at<frag_mem<T>, SB>(dsu_mat + kt * tile_row + 1024 + s2 * 512, tile_at) : zero_frag<T>();
     }
   };
   if constexpr (EARLY) request(min(wave, it));
   for (int kt = wave; kt <= it; kt += W) {
     const int Kb = kt >> 1;
     if constexpr (!EARLY) request(kt);
-    Flat32<T, HD> pk;
+    Flat32<T, HD, SB> pk;
     frag<T> ou[KS];
     if (EARLY && !next) {
 #pragma unroll
@@ -978,7 +992,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void query_narrow_
 #pragma unroll
   for (int q = 0; q < 4; ++q) st4<T>(s_ds + c * LDX + 8 * q + 4 * g, pack4<T>(own, q));
   // the Qc' rows of the tile; a second tile: the first tile's Vu rows (for dqc), a first tile: the second tile's Qc' rows
-  Flat32<T, HD> pi, pk;
+  Flat32<T, HD, SB> pi, pk;
   pi.load(qc + (int64_t)it * 32 * HD);
   pk.load(half == 1 ? vu + (int64_t)I * kNB * HD : qc + (int64_t)min(it + 1, a.s.Lp / 32 - 1) * 32 * HD);
   pi.store(s_y);

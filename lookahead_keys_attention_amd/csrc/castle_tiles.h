@@ -176,6 +176,34 @@ __device__ __forceinline__ frag<T> ldg_nat(const TI* base, int64_t row_stride, i
   return cvt_vec<T, TI, 8>(*reinterpret_cast<const frag_mem<TI>*>(base + row * row_stride + col));
 }
 
+// An element at an offset per lane (bytes) from a base that is the same for the wave: base in scalar registers, offset in one vector
+// register (SCALAR; without it as the compiler likes it, where nothing spills).  Left to itself the compiler keeps a 64-bit address, or the offset widened to 64 bits, in vector registers for every array
+// that a loop walks, and spills; a reload of one, or a spill of what was requested ahead, then waits for all loads in flight, as the
+// counter of loads is one.
+typedef __attribute__((address_space(1))) unsigned char* global_bytes;
+__device__ __forceinline__ global_bytes scalar_base(const void* p) {
+  uint64_t u = reinterpret_cast<uint64_t>(p);
+  u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)u);
+  asm("" : "+s"(u));
+  return (global_bytes)u;
+}
+__device__ __forceinline__ uint32_t lane_offset(uint32_t bytes) {
+  asm("" : "+v"(bytes));   // widened where it is used, not ahead of the loop
+  return bytes;
+}
+template <typename U, bool SCALAR = true> __device__ __forceinline__ U load_at(const void* base, uint32_t offset) {
+  if constexpr (!SCALAR) return *reinterpret_cast<const U*>(static_cast<const char*>(base) + offset);
+  else return *(const __attribute__((address_space(1))) U*)(scalar_base(base) + lane_offset(offset));
+}
+template <typename U, bool SCALAR = true> __device__ __forceinline__ U load_once_at(const void* base, uint32_t offset) {
+  if constexpr (!SCALAR) return __builtin_nontemporal_load(reinterpret_cast<const U*>(static_cast<const char*>(base) + offset));
+  else return __builtin_nontemporal_load((const __attribute__((address_space(1))) U*)(scalar_base(base) + lane_offset(offset)));
+}
+template <typename U, bool SCALAR = true> __device__ __forceinline__ void store_at(void* base, uint32_t offset, U v) {
+  if constexpr (!SCALAR) *reinterpret_cast<U*>(static_cast<char*>(base) + offset) = v;
+  else *(__attribute__((address_space(1))) U*)(scalar_base(base) + lane_offset(offset)) = v;
+}
+
 // ---- global -> LDS staging -------------------------------------------------
 // Copies a ROWS x COLS tile whose first row is global row `row0`; rows >= `row_end` are
 // zero-filled.  dst is row-major with leading dimension lds_ld<T>(COLS).
@@ -281,12 +309,12 @@ struct RowStage {
   }
   // Same for a tile whose ROWS rows of COLS elements are contiguous in memory and all exist (the
   // operand copies in the compute type): piece v of the tile sits at tile + v * V.
-  __device__ __forceinline__ void load_flat(const TI* tile, int tid = threadIdx.x) {
+  template <bool SCALAR = true> __device__ __forceinline__ void load_flat(const TI* tile, int tid = threadIdx.x) {
     static_assert(TOTAL % THREADS == 0 || TOTAL < THREADS, "tile must split evenly over the threads");
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       const int v = tid + n * THREADS;
-      if (TOTAL >= THREADS || v < TOTAL) r[n] = *reinterpret_cast<const vec<TI, V>*>(tile + v * V);
+      if (TOTAL >= THREADS || v < TOTAL) r[n] = load_at<vec<TI, V>, SCALAR>(tile + n * THREADS * V, tid * 16);
     }
   }
   __device__ __forceinline__ void store(T* dst, int ld, int tid = threadIdx.x) const {
@@ -542,11 +570,11 @@ struct SnapStage {
   vec<T, V> r[N];
 
   // src: first element of the first tile (the tiles of consecutive key groups are contiguous)
-  __device__ __forceinline__ void load(const T* src, int tid = threadIdx.x) {
+  template <bool SCALAR = true> __device__ __forceinline__ void load(const T* src, int tid = threadIdx.x) {
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       const int v = tid + n * kThreads;
-      if (v < TOTAL) r[n] = __builtin_nontemporal_load(reinterpret_cast<const vec<T, V>*>(src + (int64_t)v * V));   // read once
+      if (v < TOTAL) r[n] = load_once_at<vec<T, V>, SCALAR>(src + n * kThreads * V, tid * 16);
     }
   }
   __device__ __forceinline__ void store(T* dst, int ld, int tid = threadIdx.x) const {
