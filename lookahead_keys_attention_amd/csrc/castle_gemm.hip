@@ -184,13 +184,34 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
       typedef vec<float, V> vf;
       const int row = threadIdx.x / LPR, sub = threadIdx.x % LPR;
       const T* x = pa + (int64_t)min(m_first + row, a.M - 1) * a.lda;
-      float ssq = 0.f;
-#pragma unroll 4
-      for (int i = sub; i < a.K / V; i += LPR) {
-        const vf v = __builtin_convertvector(*reinterpret_cast<const vec<T, V>*>(x + i * V), vf);
+      // summed in the order of the norm by itself (16, 32 or 64 lanes to a row, added in pairs), PER of whose lanes a lane here stands for:
+      // the layer gives the same bits by either way
+      const int pieces = a.K / V;
+      auto sum_of = [&](auto per, int lanes) __attribute__((always_inline)) {
+        constexpr int PER = decltype(per)::value;
+        float sum[PER];
 #pragma unroll
-        for (int e = 0; e < V; ++e) ssq = __builtin_fmaf(v[e], v[e], ssq);
-      }
+        for (int v = 0; v < PER; ++v) sum[v] = 0.f;
+        for (int first = 0; first < pieces; first += lanes) {
+#pragma unroll
+          for (int v = 0; v < PER; ++v) {
+            const int i = first + sub * PER + v;
+            const vf f = __builtin_convertvector(*reinterpret_cast<const vec<T, V>*>(x + (i < pieces ? i : 0) * V), vf);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+              const float g = i < pieces ? f[e] : 0.f;
+              sum[v] = __builtin_fmaf(g, g, sum[v]);
+            }
+          }
+        }
+#pragma unroll
+        for (int o = 1; o < PER; o <<= 1)
+#pragma unroll
+          for (int v = 0; v < PER; v += 2 * o) sum[v] += sum[v + o];
+        return sum[0];
+      };
+      float ssq = pieces <= 16 ? sum_of(std::integral_constant<int, 16 / LPR>(), 16)
+                               : pieces <= 32 ? sum_of(std::integral_constant<int, 32 / LPR>(), 32) : sum_of(std::integral_constant<int, 64 / LPR>(), 64);
       for (int i = threadIdx.x; i < a.K; i += kThreads * G) s_norm[i] = (float)static_cast<const T*>(a.norm_w)[i];
 #pragma unroll
       for (int o = 1; o < LPR; o <<= 1) ssq += __shfl_xor(ssq, o);
@@ -679,9 +700,12 @@ bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to
   return p.splits == 1 && (int64_t)((M + p.rows() - 1) / p.rows()) * per_row <= kAmaxBlocks;
 }
 
-// One tile per workgroup and a CU for each, so that a row is read for its factor where it costs nothing else.
+// One tile per workgroup and a CU for each, so that a row is read for its factor where it costs nothing else; tile and groups of the product
+// by itself, for the same bits.
 bool gemm_norm_ok(int M, int N, int K, int elem_size) {
-  return K * elem_size <= kNormBytes && (int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 256 && plan(M, N, K, true, elem_size).splits == 1;
+  if ((int64_t)K * elem_size > kNormBytes) return false;
+  const Plan p = plan(M, N, K, true, elem_size);
+  return p.tile == 64 && p.splits == 1 && p.tiles(M, N) <= 256;
 }
 
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream) {
@@ -690,7 +714,6 @@ int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, h
   a.k_per_split = ((a.K + p.splits - 1) / p.splits + step - 1) / step * step;
   p.splits = (a.K + a.k_per_split - 1) / a.k_per_split;   // rounding up may leave the last ones empty
   a.part = p.splits > 1 ? workspace : nullptr;
-  if (a.norm_w != nullptr) p = {64, 1, (a.K + step - 1) / step >= 4 ? 2 : 1};
   const int rc = by_type(dtype, true, [&](auto t, auto) {
     using T = decltype(t);
     if (a.norm_w != nullptr) {

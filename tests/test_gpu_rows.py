@@ -287,7 +287,7 @@ def test_products_of_wide_tiles(rows, n, k, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
-@pytest.mark.parametrize("rows,n,k", [(1, 8, 8), (63, 72, 40), (96, 768, 128), (65, 264, 264), (130, 1536, 512), (200, 136, 456), (1000, 640, 1000)])
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 8), (63, 72, 40), (96, 768, 128), (65, 264, 264), (130, 1536, 512), (200, 136, 456), (1000, 640, 1000), (70, 128, 248)])
 def test_product_of_normalised_rows(rows, n, k, dtype):
     """Norm and product in one launch, with and without what a backward pass reads: remainders in every direction, one group of waves and two."""
     import ctypes
@@ -324,6 +324,8 @@ def test_product_of_normalised_rows(rows, n, k, dtype):
             small = 2.0 ** -24 if dtype is torch.float16 else 0.0   # half of the smallest step
             assert torch.all((h.double() - rows_ref).abs() <= (2.0 ** -bits + (k + 8) * 2.0 ** -24) * rows_ref.abs() + small)
             ref = h.double() @ w.double().t()
+            alone = torch.ops.castle_hip.rms_norm(x[:, :k].contiguous(), weight, 1e-6)   # the same bits as the norm by itself
+            assert torch.equal(h, alone[0]) and torch.equal(rstd, alone[1])
     assert torch.equal(out[0], out[1])
     bound = (k + 4) * 2.0 ** -24 * (rows_ref.abs() @ w.double().abs().t()) + 2.0 ** -bits * ref.abs() + (2.0 ** -24 if dtype is torch.float16 else 0.0)
     assert torch.all((out[0][:, :n].double() - ref).abs() <= 1.01 * bound)
