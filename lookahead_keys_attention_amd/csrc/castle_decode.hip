@@ -93,6 +93,11 @@ template <int LPR, typename Op> __device__ __forceinline__ float fold_groups(flo
   return op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
+// Running maxima of the streaming pass start here and not at -inf: a score of -inf then has weight 0 wherever it stands (exp2(-inf - -inf) would be a
+// NaN), and a row, a wave or a split without a maximum is one with sums of 0, or of NaN where all its scores are NaN, which the merges carry on like any
+// other (by a maximum of -inf they could not tell the two).
+constexpr float kLowest = -__FLT_MAX__;
+
 // partial results of the split pass: the sums of all (b, h, split), then their statistics (maximum, sum of weights)
 __device__ __forceinline__ float* part_acc(const DecodeArgs& a, int bh, int split, int HD) {
   return a.part + ((int64_t)bh * a.splits + split) * HD;
@@ -289,7 +294,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
 #pragma unroll
       for (int e = 0; e < V; ++e) tpv[sl][e] = (T)0.f;
     }
-  float ku[V], qc[V], acc[V], m = -INFINITY, l = 0.f;   // ku, qc times c1: products come out in log2 units
+  float ku[V], qc[V], acc[V], m = kLowest, l = 0.f;   // ku, qc times c1: products come out in log2 units
   float cvu[kDecodeDefer], cvu_t;                       // c1 qc . vu of the pending tokens and of the new one
   const int slot_t = t % kDecodeDefer;
   {
@@ -456,7 +461,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
     const auto largest = [](float x, float y) { return fmaxf(x, y); };
     const auto sum = [](float x, float y) { return x + y; };
     const float M = fold_groups<LPR>(m, largest);
-    const float w = m == -INFINITY ? 0.f : fast_exp2(m - M);
+    const float w = fast_exp2(m - M);
     l = fold_groups<LPR>(l * w, sum);
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = fold_groups<LPR>(acc[e] * w, sum);
@@ -469,13 +474,13 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
     if (sub == 0) { s_acc[wave][HD] = m; s_acc[wave][HD + 1] = l; }
   }
   __syncthreads();
-  float out = 0.f, M = -INFINITY, lsum = 0.f;
+  float out = 0.f, M = kLowest, lsum = 0.f;
   if (tid < HD) {
 #pragma unroll
     for (int r = 0; r < NW; ++r) M = fmaxf(M, s_acc[r][HD]);
 #pragma unroll
     for (int r = 0; r < NW; ++r) {
-      const float w = (s_acc[r][HD] == -INFINITY) ? 0.f : fast_exp2(s_acc[r][HD] - M);
+      const float w = fast_exp2(s_acc[r][HD] - M);
       out = __builtin_fmaf(w, s_acc[r][tid], out);
       lsum = __builtin_fmaf(w, s_acc[r][HD + 1], lsum);
     }
@@ -497,7 +502,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
     }
     // The last split's workgroup waits for the others (jobs in front of it) and merges: wave w takes every NW-th partial.
     constexpr int SU = 4;   // of them in flight
-    float m_w = -INFINITY, l_w = 0.f, a_w[EPL];
+    float m_w = kLowest, l_w = 0.f, a_w[EPL];
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a_w[e] = 0.f;
     for (int s0 = wave; s0 < a.splits - 1; s0 += SU * NW) {
@@ -507,7 +512,8 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
           const int s = s0 + u * NW;
-          v[u][EPL] = -INFINITY;
+#pragma unroll
+          for (int e = 0; e < EPL + 2; ++e) v[u][e] = e == EPL ? kLowest : 0.f;   // beyond the splits: nothing to add
           if (s < a.splits - 1) {
 #pragma unroll
             for (int e = 0; e < EPL + 2; ++e) {
@@ -524,7 +530,6 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
       }
 #pragma unroll
       for (int u = 0; u < SU; ++u) {
-        if (v[u][EPL] == -INFINITY) continue;   // not there, or without rows
         const float mn = fmaxf(m_w, v[u][EPL]), wo = fast_exp2(m_w - mn), wn = fast_exp2(v[u][EPL] - mn);
         l_w = l_w * wo + wn * v[u][EPL + 1];
 #pragma unroll
@@ -541,12 +546,12 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
     if (tid == 0) { s_acc[NW][HD] = M; s_acc[NW][HD + 1] = lsum; }
     __syncthreads();
     if (tid < HD) {
-      float top = -INFINITY, o = 0.f, l_all = 0.f;
+      float top = kLowest, o = 0.f, l_all = 0.f;
 #pragma unroll
       for (int r = 0; r <= NW; ++r) top = fmaxf(top, s_acc[r][HD]);
 #pragma unroll
       for (int r = 0; r <= NW; ++r) {
-        const float w = s_acc[r][HD] == -INFINITY ? 0.f : fast_exp2(s_acc[r][HD] - top);
+        const float w = fast_exp2(s_acc[r][HD] - top);
         o = __builtin_fmaf(w, s_acc[r][tid], o);
         l_all = __builtin_fmaf(w, s_acc[r][HD + 1], l_all);
       }

@@ -541,6 +541,99 @@ def test_layer_step_equals_its_parts(B, dim, Hh, d, t, dtype):
         assert_close(a[:, :, t:t + 1].float(), b[:, :, t:t + 1].float().cpu().double(), dtype, "appended row", 1e-4)
 
 
+class LayerSteps:
+    """castle_decode_layer_once over consecutive steps on a cache of its own: with control words (one launch) or without (three)."""
+
+    def __init__(self, B, dim, Hh, d, dtype, rows, capacity, w_in, w_out, norm_w, once, rotary=False, deferred=True):
+        import ctypes
+
+        from lookahead_keys_attention_amd import _native as N
+        from lookahead_keys_attention_amd.castle import _CacheStore
+
+        self.lib = ctypes.CDLL(N.LIB_PATH)
+        self.lib.castle_decode_layer_control_bytes.restype = ctypes.c_int64
+        self.B, self.dim, self.Hh, self.d, self.dtype, self.capacity, self.deferred = B, dim, Hh, d, dtype, capacity, deferred
+        self.code, self.u_half = N.DTYPE_CODES[dtype], dtype == torch.bfloat16
+        self.flags = (N.FLAG_ROTARY if rotary else 0) | (N.FLAG_U_HALF if self.u_half else 0)
+        self.w_in, self.w_out, self.norm_w = w_in, w_out, norm_w
+        self.t0 = self.t = rows[0].shape[2]
+        self.store = _CacheStore(B, Hh, d, capacity, dtype, torch.device(DEV))
+        for i, row in enumerate(rows):
+            self.store.buffers[i].zero_()
+            self.store.buffers[i][:, :, :self.t0] = row.to(torch.float16).view(dtype) if i == 0 and self.u_half else row
+        nbytes = self.lib.castle_decode_layer_control_bytes(B, Hh, d, self.code)
+        self.control = torch.zeros(nbytes, dtype=torch.uint8, device=DEV) if once else None
+        self.proj = torch.empty(B, 6 * Hh * d, dtype=dtype, device=DEV)
+
+    def step(self, x, residual=None, flags=0):
+        import ctypes
+
+        from lookahead_keys_attention_amd import ops
+
+        vp, i64, store = ctypes.c_void_p, ctypes.c_int64, self.store
+        ptr = lambda t: vp(t.data_ptr() if t is not None else None)
+        y = torch.empty(self.B, 1, self.dim, dtype=self.dtype, device=DEV)
+        inner = self.Hh * self.d
+        pending = ops.make_deferred(store.rings[0], store.rings[1], self.t0) if self.deferred else None
+        rc = self.lib.castle_decode_layer_once(
+            *[ctypes.byref(v) for v in store.views], self.t, None, self.capacity, ptr(x), i64(self.dim), self.dim, ptr(self.norm_w), ctypes.c_float(1e-5),
+            ptr(self.w_in), i64(self.dim), ptr(self.w_out), i64(inner), ptr(residual), i64(self.dim), ptr(y), i64(self.dim), ptr(self.proj), self.B, self.Hh,
+            self.d, self.code, ctypes.c_float(self.d ** -0.5), self.flags | flags, ctypes.byref(pending) if pending is not None else None, ptr(store.workspace),
+            i64(store.workspace.numel()), ptr(self.control), i64(self.control.numel() if self.control is not None else 0),
+            vp(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        self.t += 1
+        return y
+
+
+@pytest.mark.parametrize("t", [1, 40, 96, 300])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_layer_step_in_one_launch_passes_nan_on(dtype, t):
+    """A token of NaN makes this and every later output of its sequence NaN, with one split and with several, as in three launches: the partial
+    results of splits whose scores are all NaN count.  The other sequence stays finite."""
+    B, dim, Hh, d, steps = 2, 128, 2, 64, 7
+    g = torch.Generator(device=DEV).manual_seed(t)
+    rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
+    rows, w_in, w_out = [rnd(B, Hh, t, d, std=0.6) for _ in range(4)], rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5)
+    one, three = (LayerSteps(B, dim, Hh, d, dtype, rows, t + steps, w_in, w_out, None, once) for once in (True, False))
+    for step in range(steps):
+        x = rnd(B, 1, dim)
+        if step == 1:
+            x[0] = float("nan")
+        a, b = one.step(x), three.step(x)
+        assert torch.equal(a.isnan(), b.isnan()), step
+        assert a[0].isnan().all() == (step >= 1) and a[1].isfinite().all(), step
+        assert_close(a[1], b[1].cpu(), dtype, "the other sequence", 1e-4)
+
+
+@pytest.mark.parametrize("t", [1, 40, 300])
+def test_layer_step_with_a_score_of_minus_infinity(t):
+    """A token whose own score overflows to -inf has no weight among the others, whichever workgroup adds it; cached rows whose scores do have none either."""
+    B, dim, Hh, d = 1, 64, 2, 16
+    dtype, inner = torch.float32, 2 * 16
+    g = torch.Generator(device=DEV).manual_seed(t)
+    rnd = lambda *shape, std=1.0: torch.randn(*shape, generator=g, device=DEV) * std
+    rows, w_in, w_out = [rnd(B, Hh, t, d, std=0.6) for _ in range(4)], rnd(6 * inner, dim, std=dim ** -0.5), rnd(dim, inner, std=inner ** -0.5)
+    w_in[:, 0] = 0
+    w_in[3 * inner:4 * inner, 0], w_in[4 * inner:5 * inner, 0] = -1e20, 1e20   # qc and kc of a token whose first element is one
+    for low in (False, True):
+        if low and t > 1:   # every other cached row too: -1e20 times 1e20
+            rows[2][:, :, ::2] = 1e20
+        one, three = (LayerSteps(B, dim, Hh, d, dtype, rows, t + 2, w_in, w_out, None, once) for once in (True, False))
+        x = rnd(B, 1, dim)
+        x[:, :, 0] = 1
+        a, b = one.step(x), three.step(x)
+        # the largest finite score has all the weight: scores lie 1e19 apart
+        proj = torch.nn.functional.linear(x.double(), w_in.double())[0, 0].view(6, Hh, d)
+        gate = torch.sigmoid(rows[1][0].double() @ proj[1].unsqueeze(-1) * d ** -0.5)
+        su = ((rows[0][0].double() + gate * proj[2].unsqueeze(1)) @ proj[3].unsqueeze(-1))[..., 0] * d ** -0.5
+        score = (rows[2][0].double() @ proj[3].unsqueeze(-1))[..., 0] * d ** -0.5 - su * torch.sigmoid(su)
+        value = torch.stack([rows[3][0, h, score[h].argmax()] for h in range(Hh)]).double()
+        want = (value.reshape(-1) @ w_out.double().t()).cpu()
+        for y in (a, b):
+            assert_close(y[0, 0], want, dtype, "layer step", 1e-4)
+
+
 @pytest.mark.parametrize("B,dim,Hh,d,t0,dtype,rotary", [(1, 96, 1, 16, 0, torch.float32, True), (2, 512, 3, 64, 30, torch.bfloat16, True), (3, 200, 2, 32, 189, torch.float16, False),
                                                        (17, 264, 2, 64, 94, torch.bfloat16, False), (1, 136, 2, 128, 93, torch.bfloat16, True), (2, 1100, 2, 64, 700, torch.float32, False)])
 def test_layer_step_in_one_launch_equals_three(B, dim, Hh, d, t0, dtype, rotary):
