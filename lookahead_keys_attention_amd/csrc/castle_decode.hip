@@ -93,11 +93,6 @@ template <int LPR, typename Op> __device__ __forceinline__ float fold_groups(flo
   return op(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
-// Running maxima of the streaming pass start here and not at -inf: a score of -inf then has weight 0 wherever it stands (exp2(-inf - -inf) would be a
-// NaN), and a row, a wave or a split without a maximum is one with sums of 0, or of NaN where all its scores are NaN, which the merges carry on like any
-// other (by a maximum of -inf they could not tell the two).
-constexpr float kLowest = -__FLT_MAX__;
-
 // partial results of the split pass: the sums of all (b, h, split), then their statistics (maximum, sum of weights)
 __device__ __forceinline__ float* part_acc(const DecodeArgs& a, int bh, int split, int HD) {
   return a.part + ((int64_t)bh * a.splits + split) * HD;

@@ -315,7 +315,7 @@ __global__ __launch_bounds__(kThreads * G, sizeof(T) == 2 ? 2 : 1) void attn_ker
   acc_t o[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) zero(o[nt]);
-  float m = -INFINITY, l = 0.f;
+  float m = kLowest, l = 0.f;
   if (!TRV && HDP > HD) lds_zero(s_vct + HD * LDV, (HDP - HD) * LDV);
 
   int nchunks = (qb * QB + QB) / CK;
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(kThreads * G, sizeof(T) == 2 ? 2 : 1) void attn_ker
     }
     __syncthreads();
     if (group == 1) return;
-    // a row always has a key in the first chunk; the second group may have none: maximum -inf, sums 0
+    // (a group without a key of this row, or with scores of -inf only: the lowest maximum, sums 0)
     const float m1 = sums[16 * NT * kThreads + tid], both = fmaxf(m, m1), f0 = fast_exp2(m - both), f1 = fast_exp2(m1 - both);
     l = l * f0 + sums[(16 * NT + 1) * kThreads + tid] * f1;
     m = both;

@@ -176,6 +176,11 @@ __device__ __forceinline__ frag<T> ldg_nat(const TI* base, int64_t row_stride, i
   return cvt_vec<T, TI, 8>(*reinterpret_cast<const frag_mem<TI>*>(base + row * row_stride + col));
 }
 
+// Running maxima of scores that are merged later start here and not at -inf: a score of -inf then has weight 0 wherever it stands (exp2(-inf - -inf) would
+// be a NaN), and a row, a wave or a split without a maximum is one with sums of 0, or of NaN where all its scores are NaN, which a merge carries on like
+// any other (by a maximum of -inf it could not tell the two).
+constexpr float kLowest = -__FLT_MAX__;
+
 // An element at an offset per lane (bytes) from a base that is the same for the wave: base in scalar registers, offset in one vector
 // register (SCALAR; without it as the compiler likes it, where nothing spills).  Left to itself the compiler keeps a 64-bit address, or the offset widened to 64 bits, in vector registers for every array
 // that a loop walks, and spills; a reload of one, or a spill of what was requested ahead, then waits for all loads in flight, as the

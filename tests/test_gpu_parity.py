@@ -126,6 +126,28 @@ def test_wide_heads_by_two_groups_of_waves(Hh, L, dtype):
     assert torch.isfinite(few).all() and torch.all((few[0].float() - many[0].float()).abs() <= bound)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("first,last", [(32, 128), (0, 64), (64, 320)])
+def test_wide_heads_with_scores_of_minus_infinity(first, last, dtype):
+    """Keys whose scores are -inf have no weight, also where one of two groups of waves sees nothing else at first: what many heads, by one group, and
+    the oracle give without them."""
+    Hh, L, d = 100, 352, 128
+    g = torch.Generator(device="cuda").manual_seed(first)
+    six = [torch.randn(1, Hh, L, d, generator=g, device="cuda").to(dtype) for _ in range(6)]
+    six[0][..., 0] = six[0][..., 0].abs() + 0.1
+    six[1][:, :, first:last, 0] = float("-inf")
+    few = H().castle_attention_hip(*six, d ** -0.5)
+    many = H().castle_attention_hip(*(t.repeat(2, 1, 1, 1) for t in six), d ** -0.5)[:1]
+    seen = slice(last if first == 0 else 0, L)   # (a row that sees no other key has no result)
+    ref = O.parallel_core(*[t[:, :1].cpu().double() for t in six], d ** -0.5, want_U=False)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    for out in (few, many):
+        assert torch.isfinite(out[:, :, seen]).all()
+        if first == 0 and dtype is torch.float16:   # (bf16 rows are saturated on their way to fp16)
+            assert out[:, :, :last].isnan().all()
+        assert_close(out[:, :1, seen], ref[:, :, seen], dtype, "out", 1e-3)
+
+
 @pytest.mark.parametrize("L,d", [(256, 64), (200, 32)])
 def test_bf16_operand_flag_forward_and_backward(L, d, monkeypatch):
     """CASTLE_FLAG_BF16_OPERANDS keeps bf16 MFMA operands (default: fp16 operands for bf16 tensors)."""
