@@ -240,11 +240,12 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
                         int B, int H, int d, int dtype, float scale, int flags, const castle_deferred* deferred,
                         void* workspace, int64_t workspace_bytes, void* stream);
 
-/* The same in one launch for a few sequences with the row count from the host (up to 10 MB of cached rows), where the host's
- * work for three launches is what a step waits for; otherwise in three.  `control`: castle_decode_layer_control_bytes bytes,
- * 256-byte aligned, zeroed once before the first such call and then left to these calls (NULL: three launches); calls that share it
- * must not overlap, as they must not on one cache.  Workgroups of the launch wait for each other's results, never for one that has not
- * started: the waits end whatever else runs on the GPU. */
+/* The same in one launch where the host's work for three is what a step waits for: a few sequences, the row count from the host, up to 10 MB
+ * of cached rows, caches of equal strides, and the sizes for which castle_decode_layer_once_ok says 1; otherwise in three.  `control`:
+ * castle_decode_layer_control_bytes bytes, 256-byte aligned, zeroed once before the first such call and then left to these calls (NULL: three
+ * launches); calls that share it must not overlap, as they must not on one cache.  Workgroups of the launch wait for each other's results, never for
+ * one that has not started: the waits end whatever else runs on the GPU. */
+int castle_decode_layer_once_ok(int B, int H, int d, int dtype, int t, int dim);
 int64_t castle_decode_layer_control_bytes(int B, int H, int d, int dtype);
 int castle_decode_layer_once(const castle_view4* U, const castle_view4* qu_cache,
                              const castle_view4* kc_cache, const castle_view4* vc_cache,

@@ -44,6 +44,7 @@ EXPORTED_SYMBOLS = (
     "castle_decode_layer",
     "castle_decode_layer_control_bytes",
     "castle_decode_layer_once",
+    "castle_decode_layer_once_ok",
     "castle_rope",
     "castle_cache_rows",
     "castle_small_linear",

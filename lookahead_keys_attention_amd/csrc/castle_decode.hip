@@ -1077,12 +1077,24 @@ int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int
 constexpr int kExitGroups = 32, kLine = 32;   // words of a 128-byte line
 constexpr int kLayerJobs = 2048;
 constexpr int kLayerGroups = 3;   // workgroups of a CU
-// Up to this many bytes of cached rows, and with the row count from the host: a step that the host launches is bound by it with
-// three launches (16 us of host work, more than the kernels take), one launch takes 12 to 14 (us a step, three / one:
-// 1 x 8 heads of 300 rows 16.1 / 12.9, 1 x 2 of 1000 16.6 / 13.5, 4 x 8 of 300 16.0 / 14.4, 16 x 4 of 300 16.3 / 15.2, level
-// at 8 x 8 of 300 and 1 x 16 of 300 with 12 MB of weights, 8 x 8 of 1000 19.3 / 20.9).  Replayed from a graph the hand-over inside a launch
-// costs what a launch does (29.1 / 29.2 with feed-forward at 1 x 8 heads of 300 rows, 36.5 / 37.6 at 16 x 8).
-constexpr int64_t kLayerCacheBytes = 10 << 20;
+// Which steps: what one launch saves is the host's work for two more, 15 to 16 us a step with three whatever shorter kernels take; what it costs
+// are the hand-overs and the smaller workgroups of the products (us a step, three / one; heads of 64 elements with 300 rows and a layer of width 512,
+// 16 bit, if nothing else is said).  Ahead or level: 1 x 8 heads 16.3 / 13.0, 1 x 16 15.8 / 15.3, 4 x 8 15.6 / 13.9, 8 x 8 15.5 / 15.0, 16 x 4 15.6 / 14.6,
+// 64 x 2 heads of 32 with 100 rows 15.5 / 14.1, 1 x 2 with 2500 rows 15.4 / 14.6; width 256 1 x 4 15.4 / 12.8, 16 x 4 with 100 rows 16.0 / 13.2, fp32 1 x 4 15.3 / 14.0,
+// 1 x 4 with 900 rows 15.0 / 14.8, 1 x 5 15.1 / 14.9.  Not where
+// - the contraction of the projection is longer than what the four waves of a job request at once, since every further round is a trip to
+//   memory: width 768 4 x 12 15.7 / 16.5, 1024 8 x 16 16.3 / 20.3, 2048 16 x 4 15.6 / 20.9, 4096 1 x 4 15.8 / 21.3, fp32 512 1 x 8 15.6 / 17.2;
+// - many jobs come before the output projection (layer_front): 8 x 16 with 40 rows 15.7 / 18.0, 16 x 8 with 100 15.8 / 16.2, 64 x 4 with 40
+//   15.6 / 16.3, 1 x 32 16.0 / 16.5, fp32 width 256 1 x 5 with 600 rows 15.0 / 15.4, with 900 14.8 / 15.9, 1 x 16 16.7 / 20.5;
+// - the merge of a head takes more than two rounds: 1 x 1 of 128 with 2900 rows 15.2 / 20.3, fp32 1 x 2 with 2500 15.1 / 17.5;
+// - the cached rows take longer to read than the launches: 8 x 8 heads of 1000 rows 19.3 / 20.9;
+// - the row count is on the device: replayed from a graph, a hand-over inside a launch costs what a launch does (29.1 / 29.2 with feed-forward at 1 x 8
+//   heads of 300 rows, 36.5 / 37.6 at 16 x 8).
+constexpr int kLayerRound = 1024;                               // bytes of the contraction
+constexpr int kLayerFront16 = 512, kLayerFront32 = 176;         // jobs before the output projection: two a CU in 16 bit, two thirds of one in fp32
+constexpr int kLayerSplits = 33;                                // 32 partial results, and the last split's own
+constexpr int64_t kLayerCacheBytes = 10 << 20;                  // of cached rows
+constexpr int layer_front(int es) { return es == 2 ? kLayerFront16 : kLayerFront32; }
 constexpr int kTries = 1 << 19;   // of a job whose operands do not come: some tens of seconds, where something else is broken
 struct LayerArgs {
   DecodeArgs d;
@@ -1321,7 +1333,7 @@ __global__ __launch_bounds__(kThreads, kLayerGroups) void decode_layer_kernel(La
 
 static int64_t word_count(int64_t elements, int es) { return elements * es / 4; }
 int64_t decode_layer_control_bytes(int B, int H, int d, int es) {
-  return (kClaims + kLayerJobs) * 4 + 8 * (word_count((int64_t)B * 6 * H * d, es) + word_count((int64_t)B * H * d, es) + (int64_t)kLayerJobs * (d + 2));
+  return (kClaims + kLayerJobs) * 4 + 8 * (word_count((int64_t)B * 6 * H * d, es) + word_count((int64_t)B * H * d, es) + (int64_t)layer_front(es) * (d + 2));
 }
 
 // Rows x columns (at most 16 x 16) of a job: small ones while that leaves no CU a second
@@ -1355,27 +1367,41 @@ template <typename T> static int launch_layer_d(const LayerArgs& f, hipStream_t 
   }
 }
 
-// 1: the step does not fit one launch (more workgroups than the GPU holds at once).
-int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, int dtype, int cus, hipStream_t stream) {
+// Tiles, splits and jobs of a step whose sizes are in d, in and out; false if it does not go in one launch (see kLayerRound).
+static bool layer_jobs(LayerArgs& f, int es) {
+  pick_job_tile(f.in);
+  pick_job_tile(f.out);
+  f.in_cols = (f.in.N + f.in.cols - 1) / f.in.cols;
+  f.out_cols = (f.out.N + f.out.cols - 1) / f.out.cols;
+  const int64_t n_in = (int64_t)f.in_cols * ((f.in.M + f.in.rows - 1) / f.in.rows), n_out = (int64_t)f.out_cols * ((f.out.M + f.out.rows - 1) / f.out.rows);
+  const int64_t BH = (int64_t)f.d.B * f.d.H;
+  const int rows = kThreads * 16 / (f.d.d * es) * (kEarly + 1);   // of a split: what it requests ahead of the token
+  f.d.splits = (int64_t)f.d.t * (kEarly + 1) <= rows ? 1 : (f.d.t + rows - 1) / rows + 1;
+  if ((int64_t)f.in.K * es > kLayerRound || 4 * BH * f.d.t * f.d.d * es > kLayerCacheBytes || f.d.splits > kLayerSplits || n_in + BH * f.d.splits > layer_front(es) ||
+      n_in + BH * f.d.splits + n_out > kLayerJobs)
+    return false;
+  f.n_in = (int)n_in;
+  f.n_out = (int)n_out;
+  f.n_stream = (int)BH * f.d.splits;
+  return true;
+}
+bool decode_layer_once_ok(int B, int H, int d, int es, int t, int dim) {
+  LayerArgs f = {};
+  f.d.B = B; f.d.H = H; f.d.d = d; f.d.t = t;
+  f.in.M = f.out.M = B;
+  f.in.N = 6 * H * d; f.in.K = dim;
+  f.out.N = dim; f.out.K = H * d;
+  return layer_jobs(f, es);
+}
+
+// 1: the step does not go in one launch: by its sizes, with its row count on the device, or with views whose strides differ.
+int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, int dtype, hipStream_t stream) {
   const int es = dtype == 0 ? 4 : 2;
   LayerArgs f = {};
   f.d = d;
   f.in = {in.x, in.w, nullptr, in.M, in.N, in.K, in.ldx, in.ldw, 0, in.norm_w, in.eps, 0, nullptr, 0, 0, 0, nullptr, 0};
   f.out = {nullptr, out.w, out.y, out.M, out.N, out.K, 0, out.ldw, out.ldy, nullptr, 0.f, 0, out.res, out.ldr, 0, 0, nullptr, 0};
-  pick_job_tile(f.in);
-  pick_job_tile(f.out);
-  f.in_cols = (in.N + f.in.cols - 1) / f.in.cols;
-  f.out_cols = (out.N + f.out.cols - 1) / f.out.cols;
-  const int64_t n_in = (int64_t)f.in_cols * ((in.M + f.in.rows - 1) / f.in.rows), n_out = (int64_t)f.out_cols * ((out.M + f.out.rows - 1) / f.out.rows);
-  const int64_t BH = (int64_t)d.B * d.H;
-  const int rows = kThreads * 16 / (d.d * es) * (kEarly + 1);   // of a split: what it requests ahead of the token
-  f.d.splits = d.t * (kEarly + 1) <= rows ? 1 : (d.t + rows - 1) / rows + 1;
-  if (d.t_dev != nullptr || !views_alike(d) || 4 * BH * d.t * d.d * es > kLayerCacheBytes || f.d.splits > 64 || n_in + BH * f.d.splits > kLayerGroups * (int64_t)cus ||
-      n_in + BH * f.d.splits + n_out > kLayerJobs)
-    return 1;
-  f.n_in = (int)n_in;
-  f.n_out = (int)n_out;
-  f.n_stream = (int)BH * f.d.splits;
+  if (d.t_dev != nullptr || !views_alike(d) || !layer_jobs(f, es)) return 1;
   char* p = static_cast<char*>(control);
   f.control = reinterpret_cast<uint32_t*>(p);
   p += (kClaims + kLayerJobs) * 4;

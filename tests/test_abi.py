@@ -125,6 +125,26 @@ def test_products_refuse_operands_beyond_32_bit_offsets(lib):
     assert lib.castle_gemm_operand_ok(32767 - 192, 65536) and not lib.castle_gemm_operand_ok(32768 - 192, 65536)
 
 
+def test_layer_steps_go_in_one_launch_only_where_that_was_measured_ahead(lib):
+    ok = lib.castle_decode_layer_once_ok   # (B, H, d, dtype, t, dim)
+    f32, bf16, f16 = 0, 1, 2
+    for B, H, d, t, dim in ((1, 8, 64, 300, 512), (1, 16, 64, 300, 512), (4, 8, 64, 300, 512), (8, 8, 64, 300, 512), (16, 4, 64, 300, 512), (64, 2, 32, 100, 512),
+                            (1, 2, 64, 3000, 512), (1, 4, 128, 700, 512), (1, 1, 16, 0, 8)):
+        assert ok(B, H, d, bf16, t, dim) and ok(B, H, d, f16, t, dim)
+    assert ok(1, 4, 64, f32, 300, 256) and ok(2, 4, 64, f32, 300, 256) and ok(1, 4, 64, f32, 900, 256)
+    # contractions that a job reads in more than one round, also where the weights are few
+    for dtype, dim in ((bf16, 520), (bf16, 768), (f16, 1024), (bf16, 2048), (bf16, 4096), (f32, 260), (f32, 512)):
+        assert not ok(1, 4, 64, dtype, 300, dim)
+    # more than two jobs a CU before the output projection, two thirds of one in fp32
+    for B, H, dtype, t, dim in ((8, 16, bf16, 40, 512), (16, 8, bf16, 100, 512), (64, 4, bf16, 40, 512), (1, 32, bf16, 300, 512), (16, 4, f32, 100, 256), (1, 16, f32, 300, 256), (1, 5, f32, 600, 256)):
+        assert not ok(B, H, 64, dtype, t, dim)
+    # more than 10 MB of cached rows, more than 32 partial results of a head
+    assert not ok(8, 8, 64, bf16, 1000, 512) and ok(1, 1, 128, bf16, 32 * 48, 512) and not ok(1, 1, 128, bf16, 32 * 48 + 1, 512)
+    for B, H, d, dtype, t, dim in ((0, 8, 64, bf16, 1, 512), (1, 0, 64, bf16, 1, 512), (1, 8, 48, bf16, 1, 512), (1, 8, 64, 7, 1, 512), (1, 8, 64, bf16, -1, 512),
+                                   (1, 8, 64, bf16, 1, 0), (65536, 1, 64, bf16, 1, 512), (1 << 30, 1 << 30, 128, bf16, 1 << 30, 1 << 30)):
+        assert not ok(B, H, d, dtype, t, dim)
+
+
 def test_check_raises_with_message(lib):
     with pytest.raises(RuntimeError, match="unsupported shape"):
         N.check(-2, "castle_fwd")

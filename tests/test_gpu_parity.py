@@ -618,6 +618,7 @@ def test_layer_step_in_one_launch_passes_nan_on(dtype, t):
     rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
     rows, w_in, w_out = [rnd(B, Hh, t, d, std=0.6) for _ in range(4)], rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5)
     one, three = (LayerSteps(B, dim, Hh, d, dtype, rows, t + steps, w_in, w_out, None, once) for once in (True, False))
+    assert one.lib.castle_decode_layer_once_ok(B, Hh, d, one.code, t + steps, dim)
     for step in range(steps):
         x = rnd(B, 1, dim)
         if step == 1:
@@ -642,6 +643,7 @@ def test_layer_step_with_a_score_of_minus_infinity(t):
         if low and t > 1:   # every other cached row too: -1e20 times 1e20
             rows[2][:, :, ::2] = 1e20
         one, three = (LayerSteps(B, dim, Hh, d, dtype, rows, t + 2, w_in, w_out, None, once) for once in (True, False))
+        assert one.lib.castle_decode_layer_once_ok(B, Hh, d, one.code, t, dim)
         x = rnd(B, 1, dim)
         x[:, :, 0] = 1
         a, b = one.step(x), three.step(x)
@@ -656,54 +658,38 @@ def test_layer_step_with_a_score_of_minus_infinity(t):
             assert_close(y[0, 0], want, dtype, "layer step", 1e-4)
 
 
-@pytest.mark.parametrize("B,dim,Hh,d,t0,dtype,rotary", [(1, 96, 1, 16, 0, torch.float32, True), (2, 512, 3, 64, 30, torch.bfloat16, True), (3, 200, 2, 32, 189, torch.float16, False),
-                                                       (17, 264, 2, 64, 94, torch.bfloat16, False), (1, 136, 2, 128, 93, torch.bfloat16, True), (2, 1100, 2, 64, 700, torch.float32, False)])
-def test_layer_step_in_one_launch_equals_three(B, dim, Hh, d, t0, dtype, rotary):
-    """castle_decode_layer_once with its control words against castle_decode_layer over consecutive steps on caches of their own: around
-    whole iterations of a split (32 rows at d = 64 and 16 bit, three to a split) and with the write-back every fourth step.  Both
+@pytest.mark.parametrize("deferred", [True, False])
+@pytest.mark.parametrize("B,dim,Hh,d,t0,dtype,rotary,once", [
+    (1, 96, 1, 16, 0, torch.float32, True, True), (2, 512, 3, 64, 30, torch.bfloat16, True, True), (3, 200, 2, 32, 189, torch.float16, False, True),
+    (17, 264, 2, 64, 94, torch.bfloat16, False, True), (1, 136, 2, 128, 93, torch.bfloat16, True, True), (2, 256, 2, 64, 700, torch.float32, False, True), (1, 256, 2, 64, 1520, torch.float32, True, True),
+    (1, 136, 1, 128, 1100, torch.bfloat16, True, True), (1, 512, 1, 128, 1527, torch.float16, False, True),
+    (2, 1100, 2, 64, 700, torch.float32, False, False), (1, 520, 2, 64, 30, torch.bfloat16, False, False)])
+def test_layer_step_in_one_launch_equals_three(B, dim, Hh, d, t0, dtype, rotary, once, deferred):
+    """castle_decode_layer_once with its control words against the same without over consecutive steps on caches of their own: around
+    whole iterations of a split (32 rows at d = 64 and 16 bit, three to a split), up to 33 splits, and with the write-back every fourth step or in each.  Both
     round the projection and the attention output to the tensor type, so what differs is the order of 32-bit sums; a value of a 16-bit
-    tensor in between may then round the other way: two roundings of 2^-8 (bf16) through the output projection and the store."""
-    import ctypes
-
-    from lookahead_keys_attention_amd import _native as N, ops
-    from lookahead_keys_attention_amd.castle import _CacheStore
-
-    lib, steps = ctypes.CDLL(N.LIB_PATH), 9
-    lib.castle_decode_layer_control_bytes.restype = ctypes.c_int64
+    tensor in between may then round the other way: two roundings of 2^-8 (bf16) through the output projection and the store.  Only three
+    launches leave the projection in the scratch."""
+    steps = 9
     g = torch.Generator(device=DEV).manual_seed(B + dim)
     rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
     norm_w, res = 1 + rnd(dim, std=0.2), rnd(B, 1, dim)
     w_in, w_out = rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5)
-    code, u_half = N.DTYPE_CODES[dtype], dtype == torch.bfloat16
-    control = torch.zeros(lib.castle_decode_layer_control_bytes(B, Hh, d, code), dtype=torch.uint8, device=DEV)
-    stores = [_CacheStore(B, Hh, d, t0 + steps, dtype, torch.device(DEV)) for _ in range(2)]
-    for i in range(4):
-        rows = rnd(B, Hh, t0, d, std=0.6)
-        for store in stores:
-            store.buffers[i].zero_()
-            store.buffers[i][:, :, :t0] = rows.to(torch.float16).view(dtype) if i == 0 and u_half else rows
-    proj = torch.empty(B, 6 * Hh * d, dtype=dtype, device=DEV)
-    flags = (N.FLAG_ROTARY if rotary else 0) | (N.FLAG_U_HALF if u_half else 0)
-    vp, i64 = ctypes.c_void_p, ctypes.c_int64
+    rows = [rnd(B, Hh, t0, d, std=0.6) for _ in range(4)]
+    one, three = (LayerSteps(B, dim, Hh, d, dtype, rows, t0 + steps, w_in, w_out, norm_w, words, rotary, deferred) for words in (True, False))
     for step in range(steps):
-        x, ys = rnd(B, 1, dim), []
-        for store, words in zip(stores, (control, None)):
-            y = torch.empty(B, 1, dim, dtype=dtype, device=DEV)
-            views = [ctypes.byref(v) for v in store.views]
-            deferred = ops.make_deferred(store.rings[0], store.rings[1], t0)
-            rc = lib.castle_decode_layer_once(
-                *views, t0 + step, None, t0 + steps, vp(x.data_ptr()), i64(dim), dim, vp(norm_w.data_ptr()), ctypes.c_float(1e-5), vp(w_in.data_ptr()), i64(dim),
-                vp(w_out.data_ptr()), i64(Hh * d), vp(res.data_ptr()), i64(dim), vp(y.data_ptr()), i64(dim), vp(proj.data_ptr()), B, Hh, d, code,
-                ctypes.c_float(d ** -0.5), flags, ctypes.byref(deferred), vp(store.workspace.data_ptr()), i64(store.workspace.numel()),
-                vp(words.data_ptr() if words is not None else None), i64(words.numel() if words is not None else 0),
-                vp(torch.cuda.current_stream().cuda_stream))
-            assert rc == 0
-            ys.append(y.double())
+        assert one.lib.castle_decode_layer_once_ok(B, Hh, d, one.code, t0 + step, dim) == once
+        x = rnd(B, 1, dim)
+        for steps_of in (one, three):
+            steps_of.proj.fill_(7)
+        ys = [steps_of.step(x, res).double() for steps_of in (one, three)]
+        assert torch.all(one.proj == 7) == once and not torch.all(three.proj == 7)
         scale = ys[1].abs().max().item()
         assert (ys[0] - ys[1]).abs().max().item() <= scale * {torch.float32: 1e-4, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}[dtype], step
+    stores = (one.store, three.store)
     for a, b in zip(stores[0].buffers[1:], stores[1].buffers[1:]):
         assert_close(a.float(), b.float().cpu().double(), dtype, "cached rows", 1e-4)
-    if u_half:
+    if one.u_half:
         a, b = (store.buffers[0].view(torch.float16).float() for store in stores)
     else:
         a, b = (store.buffers[0].float() for store in stores)
