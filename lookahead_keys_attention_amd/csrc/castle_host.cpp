@@ -9,6 +9,7 @@
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
@@ -1025,10 +1026,14 @@ class StepPlan {
     const double e = norm_eps(eps);
     // the projection is scratch of the step like the workspace: kept with it, an allocation costs more than a microsecond
     if (!proj_.defined()) proj_ = at::empty({B, 6 * inner}, x.options().requires_grad(false));
-    if (!control_.defined() && !t_device) {   // for the step as one launch
+    // For the step as one launch, where it is one.  Not while a graph is recorded: the zeros would be there only once it is replayed, and
+    // steps outside of it use the words too.
+    const bool once = !t_device && castle_decode_layer_once_ok(s_.B, s_.H, s_.d, s_.dtype, (int)t, (int)dim);
+    if (once && !control_.defined() && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None) {
       const int64_t n = check(castle_decode_layer_control_bytes(s_.B, s_.H, s_.d, s_.dtype), "castle_decode_layer_control_bytes");
       control_ = at::zeros({n}, x.options().dtype(at::kByte).requires_grad(false));
     }
+    const bool words = once && control_.defined();
     used_on_current_stream();
     Tensor y = at::empty({B, 1, dim}, x.options());
     const castle_view4* c = views_;
@@ -1037,8 +1042,8 @@ class StepPlan {
                               nw.defined() ? nw.data_ptr() : nullptr, (float)e, w_qkv.data_ptr(), w_qkv.stride(0), w_out.data_ptr(),
                               w_out.stride(0), res.defined() ? res.data_ptr() : nullptr, res.defined() ? res.stride(0) : 0, y.data_ptr(), dim,
                               proj_.data_ptr(), s_.B, s_.H, s_.d, s_.dtype, (float)scale, flags_ | (rotary ? CASTLE_FLAG_ROTARY : 0),
-                              base >= 0 || base_device ? &def : nullptr, workspace_.data_ptr(), workspace_.numel(), t_device ? nullptr : control_.data_ptr(),
-                                   t_device ? 0 : control_.numel(), stream_of(x)),
+                              base >= 0 || base_device ? &def : nullptr, workspace_.data_ptr(), workspace_.numel(), words ? control_.data_ptr() : nullptr,
+                              words ? control_.numel() : 0, stream_of(x)),
           "castle_decode_layer_once");
     return y;
   }

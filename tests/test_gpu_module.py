@@ -345,6 +345,62 @@ def test_memory_of_a_dropped_cache_waits_for_a_step_on_another_stream():
     assert torch.equal(got, want)
 
 
+def test_first_cached_step_recorded_into_a_graph():
+    """A cache whose first step is recorded: steps outside the graph before its first replay, and replays between them, give what steps without a
+    graph give (the recorded step must not prepare memory that those steps rely on)."""
+    m = make(128, 2, 64, torch.bfloat16, prenorm=True).eval()
+    g = torch.Generator(device=DEV).manual_seed(3)
+    prompt, tokens = (torch.randn(2, n, 128, generator=g, device=DEV).bfloat16() for n in (20, 3))
+    tokens = [tokens[:, i:i + 1].contiguous() for i in range(3)]
+    with torch.no_grad():
+        _, cache = m(prompt, return_next_cache=True)
+        want = []
+        for token in tokens:
+            y, cache = m(token, cache=cache)
+            want.append(y)
+        _, cache = m(prompt, return_next_cache=True)
+        store = cache._store
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            recorded, _ = m(tokens[0], cache=cache)
+        store.length = 20   # recorded, not taken
+        cache = store.as_cache()
+        for i, token in enumerate(tokens):
+            y, cache = m(token, cache=cache)
+            assert torch.equal(y, want[i]) if i == 0 else True
+            bf16_close(y, want[i], f"step {i}")
+            if i < 2:   # (the step at 20 again; the lookahead keys are written at 23 only)
+                recorded.fill_(7)
+                graph.replay()
+                torch.cuda.synchronize()
+                bf16_close(recorded, want[0], f"replay {i}")
+
+
+def test_control_words_only_for_caches_whose_steps_go_in_one_launch():
+    """What a first step keeps for later ones: its projection, and control words where it is one launch."""
+    from lookahead_keys_attention_amd import _native as N
+
+    for B, heads, n in ((1, 8, 100), (16, 16, 40), (8, 8, 1000)):
+        m = make(512, heads, 64, torch.bfloat16).eval()
+        lib, inner = N.lib(), heads * 64
+        with torch.no_grad():
+            x = torch.randn(B, n, 512, device=DEV).bfloat16()
+            _, cache = m(x, return_next_cache=True)
+            cache._store.workspace
+            token = x[:, :1].contiguous()
+            y = m(token)   # whatever a first step of all allocates
+            y = None
+            before = torch.cuda.memory_allocated()
+            y, cache = m(token, cache=cache)
+            kept = torch.cuda.memory_allocated() - before
+        up = lambda n: (n + 511) // 512 * 512
+        once = lib.castle_decode_layer_once_ok(B, heads, 64, 1, n, 512)
+        assert once == (B == 1)
+        control = lib.castle_decode_layer_control_bytes(B, heads, 64, 1) if once else 0
+        assert kept == up(B * 6 * inner * 2) + up(y.numel() * 2) + up(control)
+
+
 def test_forward_mode_derivatives_of_a_layer_raise():
     from torch.autograd import forward_ad
 
