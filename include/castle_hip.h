@@ -67,6 +67,10 @@ extern "C" {
  * is 0; castle_bwd: the same place of the backward workspace holds partial maxima of |dout| (castle_gemm leaves them
  * there): a launch and a pass less.  Ignored for fp32. */
 #define CASTLE_FLAG_AMAX_READY 64
+/* castle_decode_layer_once in one launch, for tests of its waits: the jobs in reverse order and next to no patience, so that nearly all are done by
+ * workgroups that had waited for them; with _GIVE_UP these leave instead, and what they were to do is NaN as described there. */
+#define CASTLE_FLAG_STEP_TAKE_OVER 128
+#define CASTLE_FLAG_STEP_GIVE_UP 256
 #define CASTLE_AMAX_PARTIALS 256
 #define CASTLE_AMAX_OFFSET 256
 
@@ -243,8 +247,9 @@ int castle_decode_layer(const castle_view4* U, const castle_view4* qu_cache,
 /* The same in one launch where the host's work for three is what a step waits for: a few sequences, the row count from the host, up to 10 MB
  * of cached rows, caches of equal strides, and the sizes for which castle_decode_layer_once_ok says 1; otherwise in three.  `control`:
  * castle_decode_layer_control_bytes bytes, 256-byte aligned, zeroed once before the first such call and then left to these calls (NULL: three
- * launches); calls that share it must not overlap, as they must not on one cache.  Workgroups of the launch wait for each other's results, never for
- * one that has not started: the waits end whatever else runs on the GPU. */
+ * launches); calls that share it must not overlap, as they must not on one cache.  Workgroups of the launch wait for each other's results for a bounded
+ * time, then do themselves what no other has started: the waits end whatever else runs on the GPU.  Should results not come in some tens of seconds
+ * all the same, what depends on them is NaN: in y, and in a row of vc_cache of every head whose step is not complete. */
 int castle_decode_layer_once_ok(int B, int H, int d, int dtype, int t, int dim);
 int64_t castle_decode_layer_control_bytes(int B, int H, int d, int dtype);
 int castle_decode_layer_once(const castle_view4* U, const castle_view4* qu_cache,

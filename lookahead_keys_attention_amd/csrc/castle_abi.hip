@@ -24,7 +24,7 @@ int decode_pick_splits(int BH, int t, int rows_per_iteration, int cus);
 int decode_static_scratch(float** ptr);
 int64_t decode_layer_control_bytes(int B, int H, int d, int es);
 bool decode_layer_once_ok(int B, int H, int d, int es, int t, int dim);
-int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, int dtype, hipStream_t stream);
+int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, bool take_over, bool give_up, int dtype, hipStream_t stream);
 int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int K, int64_t ldx, int64_t ldw, int64_t ldy,
                         int dtype, const void* norm_w, float eps, int act, const void* res, int64_t ldr, hipStream_t stream, int* clear = nullptr, int clear_n = 0);
 int launch_sample(const void* logits, int64_t ld, const float* u, int rows, int V, int k, float inv_temperature, int64_t* out, int64_t out_ld,
@@ -453,7 +453,7 @@ static int decode_layer_common(const castle_view4* U, const castle_view4* qu_cac
     if (reinterpret_cast<uintptr_t>(control) % 256 != 0 || control_bytes < castle_decode_layer_control_bytes(B, H, d, dtype)) return CASTLE_ERR_WORKSPACE;
     const castle::DecodeLinear in = {x, w_in, nullptr, B, width, dim, ldx, ldw_in, 0, norm_weight, eps, nullptr, 0};
     const castle::DecodeLinear out = {nullptr, w_out, y, B, dim, inner, 0, ldw_out, ldy, nullptr, 0.f, residual, ldr};
-    rc = castle::launch_decode_layer(a, in, out, control, dtype, s);
+    rc = castle::launch_decode_layer(a, in, out, control, (flags & CASTLE_FLAG_STEP_TAKE_OVER) != 0, (flags & CASTLE_FLAG_STEP_GIVE_UP) != 0, dtype, s);
     if (rc != 1) return rc;
   }
   // the projection clears the arrival counts of the step, which then needs no launch to merge its splits

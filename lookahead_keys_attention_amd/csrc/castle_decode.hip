@@ -114,6 +114,7 @@ struct TokenWords {
   uint64_t* merged = nullptr;       // [B][H][d]
   uint64_t* part = nullptr;         // [B][H][splits][d + 2]: sums, maximum, sum of weights, a float each
   uint32_t tag = 0;
+  int patience = 1;                 // polls for words before this workgroup does something else
 };
 // LDS of the early rows: by iteration and tensor (qu, U, kc, vc, gates) 1 KB per wave
 constexpr int kEarly = 2;
@@ -137,11 +138,11 @@ template <typename T> __device__ __forceinline__ void put_word(uint64_t* row, in
     if (i % 2 == 0) store_word(row + i / 2, __builtin_bit_cast(uint32_t, vec<T, 2>{(T)v, (T)w}), tag);
   }
 }
-// N 16-byte pieces (four words each) per lane, zeros for a null pointer.  False if after some patience a word of the wave's lanes
-// still does not carry the tag.
-constexpr int kPatience = 64;   // polls, of about a microsecond
-template <typename T, int N> __device__ __forceinline__ bool wait_words(const uint64_t* const (&p)[N], uint32_t tag, vec<T, elem_traits<T>::vec16> (&x)[N]) {
-  for (int polls = 0; polls < kPatience; ++polls) {
+// N 16-byte pieces (four words each) per lane, zeros for a null pointer.  False if after `patience` polls (of about a microsecond, at least one) a word
+// of the wave's lanes still does not carry the tag.
+constexpr int kPatience = 64, kTries = 1 << 19;   // of a job whose operands do not come, polls each: some tens of seconds, where something else is broken
+template <typename T, int N> __device__ __forceinline__ bool wait_words(const uint64_t* const (&p)[N], uint32_t tag, int patience, vec<T, elem_traits<T>::vec16> (&x)[N]) {
+  for (int polls = 0; polls < patience; ++polls) {
     bool there = true;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
@@ -158,6 +159,11 @@ template <typename T, int N> __device__ __forceinline__ bool wait_words(const ui
     __builtin_amdgcn_s_sleep(1);
   }
   return false;
+}
+
+// rows of a split: whole iterations of a workgroup
+__device__ __forceinline__ int split_rows(int t, int splits, int rows_per_iteration) {
+  return ((t + splits - 1) / splits + rows_per_iteration - 1) / rows_per_iteration * rows_per_iteration;
 }
 
 // A group of LPR = d / V lanes owns one cache row per iteration.  (Workgroups of 16 waves, so that a head needs no
@@ -218,7 +224,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
   // rows of this workgroup: [r0, r1), whole iterations of RPI rows.  With WORDS the last split has none (unless it is the only
   // one): it has the appended row to see to, and the partial results of the others.
   const int with_rows = WORDS && a.splits > 1 ? a.splits - 1 : a.splits;
-  const int per = ((t + with_rows - 1) / with_rows + RPI - 1) / RPI * RPI;
+  const int per = split_rows(t, with_rows, RPI);
   const int r0 = split * per;
   const int r1 = min(t, r0 + per);
   // deferred write-back: how many tokens are pending, and whether this step writes U
@@ -278,7 +284,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
     const int64_t part = (int64_t)a.H * (HD / kPerWord<T>);
     vt got[6];
     const uint64_t* const need[6] = {w + part, w + 2 * part, w + 3 * part, owner ? w + 4 * part : nullptr, owner ? w : nullptr, owner ? w + 5 * part : nullptr};
-    if (!ready(wait_words<T>(need, words.tag, got))) return false;
+    if (!ready(wait_words<T>(need, words.tag, words.patience, got))) return false;
     tku = got[0]; tvu = got[1]; tqc = got[2];
     if (owner) { tkc = got[3]; tqu = got[4]; tvc = got[5]; }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the early rows are in LDS (requested in front of the words, they came first)
@@ -495,14 +501,15 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
       if (tid < 2) store_word(p + HD + tid, __builtin_bit_cast(uint32_t, tid == 0 ? M : lsum), words.tag);
       return true;
     }
-    // The last split's workgroup waits for the others (jobs in front of it) and merges: wave w takes every NW-th partial.
+    // The last split's workgroup waits for the others (jobs in front of it) and merges: wave w takes every NW-th partial.  What does not come makes the
+    // result NaN.
     constexpr int SU = 4;   // of them in flight
     float m_w = kLowest, l_w = 0.f, a_w[EPL];
 #pragma unroll
     for (int e = 0; e < EPL; ++e) a_w[e] = 0.f;
     for (int s0 = wave; s0 < a.splits - 1; s0 += SU * NW) {
       float v[SU][EPL + 2];
-      while (true) {
+      for (int polls = 0;; ++polls) {
         bool there = true;
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
@@ -521,6 +528,7 @@ __device__ __forceinline__ bool stream_job(const DecodeArgs& a, int split, int b
           }
         }
         if (__builtin_amdgcn_ballot_w64(!there) == 0) break;
+        if (polls == kPatience * kTries) { l_w = __builtin_nanf(""); break; }
         __builtin_amdgcn_s_sleep(1);
       }
 #pragma unroll
@@ -1071,9 +1079,11 @@ int launch_small_linear(const void* x, const void* w, void* y, int M, int N, int
 // start: every job is claimed before it writes anything (one word per job), jobs wait for jobs in front of them only, for a
 // bounded time, and a workgroup that has waited in vain claims and runs what nobody has claimed in front of its own job, first to
 // last, before it tries its own again.  The first of the unfinished jobs finds all it needs, so there is always one that
-// ends.  (The last split waits for the others without a bound, but only once all of them are claimed.)  A workgroup whose job was
+// ends.  (The last split waits for the others without taking over anything, but only once all of them are claimed.)  A workgroup whose job was
 // taken leaves.  The last workgroup to leave moves the tag on, so that no launch can take words or claims of another for
 // its own.
+// Every wait is bounded all the same (kTries).  A job that is given up at the end leaves NaN: in its words, in its part of y, and in a value row of
+// its head, so that neither this step nor a later one on the cache passes for a good one.
 constexpr int kExitGroups = 32, kLine = 32;   // words of a 128-byte line
 constexpr int kLayerJobs = 2048;
 constexpr int kLayerGroups = 3;   // workgroups of a CU
@@ -1095,13 +1105,14 @@ constexpr int kLayerFront16 = 512, kLayerFront32 = 176;         // jobs before t
 constexpr int kLayerSplits = 33;                                // 32 partial results, and the last split's own
 constexpr int64_t kLayerCacheBytes = 10 << 20;                  // of cached rows
 constexpr int layer_front(int es) { return es == 2 ? kLayerFront16 : kLayerFront32; }
-constexpr int kTries = 1 << 19;   // of a job whose operands do not come: some tens of seconds, where something else is broken
 struct LayerArgs {
   DecodeArgs d;
   LinearArgs in, out;
   uint32_t* control;   // tag of the last launch; workgroups gone, in all and by group, a line each; claims
   uint64_t *proj, *merged, *part;
   int n_in, n_stream, n_out, in_cols, out_cols;   // jobs; column tiles of the two products
+  int patience, tries;
+  bool reversed;   // the first workgroup has the last job
 };
 constexpr int kGone = kLine, kGoneGroup = 2 * kLine, kClaims = kGoneGroup + kExitGroups * kLine;
 
@@ -1142,7 +1153,7 @@ __device__ __forceinline__ LinearLds& linear_lds() {
 // One 16 x 16 tile (or part of one) of y = x w^T, the K split over the waves as in small_linear_kernel.  WORDS_IN: x comes as words, else
 // y leaves as words.  ready(whether the words came): a barrier that says whether the result may be written.
 template <typename T, bool WORDS_IN, typename G, typename F>
-__device__ __forceinline__ bool linear_job(const LinearArgs& a, int tile, int col_tiles, const uint64_t* xw, uint64_t* yw, uint32_t tag, G&& begin, F&& ready) {
+__device__ __forceinline__ bool linear_job(const LinearArgs& a, int tile, int col_tiles, const uint64_t* xw, uint64_t* yw, uint32_t tag, int patience, G&& begin, F&& ready) {
   constexpr int V = elem_traits<T>::vec16, DEPTH = 4 * V, MAXS = 4, W = kThreads / 64;
   typedef vec<T, V> vt;
   typedef vec<float, V> vf;
@@ -1182,7 +1193,7 @@ __device__ __forceinline__ bool linear_job(const LinearArgs& a, int tile, int co
       const uint64_t* const first[1] = {at(0)};
       const uint64_t* const rest[MAXS - 1] = {at(1), at(2), at(3)};
       vt x0[1], xr[MAXS - 1];
-      came = came && wait_words<T>(first, tag, x0) && wait_words<T>(rest, tag, xr);
+      came = came && wait_words<T>(first, tag, patience, x0) && wait_words<T>(rest, tag, patience, xr);
       fa[0] = x0[0];
 #pragma unroll
       for (int u = 1; u < MAXS; ++u) fa[u] = xr[u - 1];
@@ -1255,10 +1266,35 @@ __device__ __forceinline__ bool linear_job(const LinearArgs& a, int tile, int co
   return true;
 }
 
+// what a job that is given up leaves (those of the projection wait for nothing)
+template <typename T, int HD> __device__ __forceinline__ void give_up(const LayerArgs& f, int job, uint32_t tag) {
+  const T nan = (T)__builtin_nanf("");
+  const int tid = threadIdx.x, stream = job - f.n_in, out = stream - f.n_stream;
+  if (out >= 0) {
+    const int m = out / f.out_cols * f.out.rows + tid / 16, n = out % f.out_cols * f.out.cols + tid % 16;
+    if (tid / 16 < f.out.rows && tid % 16 < f.out.cols && m < f.out.M && n < f.out.N) static_cast<T*>(f.out.y)[(int64_t)m * f.out.ldy + n] = nan;
+    return;
+  }
+  const int bh = stream / f.d.splits, split = stream % f.d.splits;
+  const bool last = split == f.d.splits - 1;
+  if (last) {
+    uint32_t payload;
+    if constexpr (sizeof(T) == 4) payload = __builtin_bit_cast(uint32_t, nan);
+    else payload = __builtin_bit_cast(uint32_t, vec<T, 2>{nan, nan});
+    for (int i = tid; i < HD / kPerWord<T>; i += kThreads) store_word(f.merged + (int64_t)bh * (HD / kPerWord<T>) + i, payload, tag);
+  } else {
+    for (int i = tid; i < HD + 2; i += kThreads) store_word(f.part + (int64_t)stream * (HD + 2) + i, __builtin_bit_cast(uint32_t, __builtin_nanf("")), tag);
+  }
+  // of its own rows the first, of the last split the appended one
+  const int row = last ? f.d.t : split * split_rows(f.d.t, f.d.splits - 1, kThreads * elem_traits<T>::vec16 / HD);
+  if (last || row < f.d.t)
+    for (int e = tid; e < HD; e += kThreads) view_row<T>(f.d.vc_cache, bh / f.d.H, bh % f.d.H, row)[e] = nan;
+}
+
 template <typename T, int HD, bool UH>
 __global__ __launch_bounds__(kThreads, kLayerGroups) void decode_layer_kernel(LayerArgs args) {
   __shared__ int s_mine, s_came[kThreads / 64], s_job;
-  const int own = blockIdx.x;
+  const int own = args.reversed ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
   uint32_t* const claims = args.control + kClaims;
   const uint32_t tag = args.control[0] + 1;
   bool claimed = false, mine = true;   // mine, of thread 0: the claim's answer
@@ -1284,25 +1320,33 @@ __global__ __launch_bounds__(kThreads, kLayerGroups) void decode_layer_kernel(La
   auto run = [&](const LayerArgs& f, int job) __attribute__((always_inline)) {
     const int stream = job - f.n_in, out = stream - f.n_stream;
     if (stream < 0) {
-      linear_job<T, false>(f.in, job, f.in_cols, nullptr, f.proj, tag, begin, agree);
+      linear_job<T, false>(f.in, job, f.in_cols, nullptr, f.proj, tag, f.patience, begin, agree);
     } else if (out < 0) {
       const int split = stream % f.d.splits;
-      const TokenWords words = {f.proj, f.merged, f.part, tag};
+      const TokenWords words = {f.proj, f.merged, f.part, tag, f.patience};
       stream_job<T, HD, UH, false, true, true>(f.d, split, stream / f.d.splits, words, begin, [&](bool came) {
         // the last split waits for the others' partial results when its own rows are done: they have to be claimed by now
         if (split == f.d.splits - 1) came = came && jobs_claimed(claims + job - split, split, tag);
         return agree(came);
       });
     } else {
-      linear_job<T, true>(f.out, out, f.out_cols, f.merged, nullptr, tag, begin, agree);
+      linear_job<T, true>(f.out, out, f.out_cols, f.merged, nullptr, tag, f.patience, begin, agree);
     }
   };
   run(args, own);
   int job = own;
-  for (int tries = 0; (job != own || answer == kLater) && tries < kTries; ++tries) {
-    // The arguments are read where a job needs them: read ahead of the loop, 160 scalar and 80 vector registers spill.
+  // The arguments are read where a job needs them: read ahead of the loop, 160 scalar and 80 vector registers spill.
+  auto again = [] __attribute__((always_inline)) {
     const __attribute__((address_space(4))) LayerArgs* kernarg = (const __attribute__((address_space(4))) LayerArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(kernarg));
+    return (const LayerArgs*)kernarg;
+  };
+  for (int tries = 0; job != own || answer == kLater; ++tries) {
+    if (tries >= again()->tries) {
+      if (answer == kLater) give_up<T, HD>(*again(), job, tag);
+      if (job != own) give_up<T, HD>(*again(), own, tag);   // (its own waited for the one it took)
+      break;
+    }
     __syncthreads();   // what the last job kept in LDS is read
     if (job == own || answer != kLater) {   // (a job once taken is run until it is done)
       if (wave_id() == 0) {
@@ -1313,7 +1357,7 @@ __global__ __launch_bounds__(kThreads, kLayerGroups) void decode_layer_kernel(La
       job = __builtin_amdgcn_readfirstlane(s_job);
       if (job < 0) job = own;
     }
-    run(*(const LayerArgs*)kernarg, job);
+    run(*again(), job);
   }
   if (threadIdx.x == 0) {
     const int groups = min(kExitGroups, (int)gridDim.x), g = blockIdx.x % kExitGroups;
@@ -1395,13 +1439,16 @@ bool decode_layer_once_ok(int B, int H, int d, int es, int t, int dim) {
 }
 
 // 1: the step does not go in one launch: by its sizes, with its row count on the device, or with views whose strides differ.
-int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, int dtype, hipStream_t stream) {
+int launch_decode_layer(const DecodeArgs& d, const DecodeLinear& in, const DecodeLinear& out, void* control, bool take_over, bool give_up, int dtype, hipStream_t stream) {
   const int es = dtype == 0 ? 4 : 2;
   LayerArgs f = {};
   f.d = d;
   f.in = {in.x, in.w, nullptr, in.M, in.N, in.K, in.ldx, in.ldw, 0, in.norm_w, in.eps, 0, nullptr, 0, 0, 0, nullptr, 0};
   f.out = {nullptr, out.w, out.y, out.M, out.N, out.K, 0, out.ldw, out.ldy, nullptr, 0.f, 0, out.res, out.ldr, 0, 0, nullptr, 0};
   if (d.t_dev != nullptr || !views_alike(d) || !layer_jobs(f, es)) return 1;
+  f.patience = take_over || give_up ? 1 : kPatience;
+  f.tries = give_up ? 0 : kTries;
+  f.reversed = take_over || give_up;
   char* p = static_cast<char*>(control);
   f.control = reinterpret_cast<uint32_t*>(p);
   p += (kClaims + kLayerJobs) * 4;

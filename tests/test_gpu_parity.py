@@ -696,6 +696,54 @@ def test_layer_step_in_one_launch_equals_three(B, dim, Hh, d, t0, dtype, rotary,
     assert_close(a, b.cpu().double(), dtype, "lookahead keys", 1e-4)
 
 
+@pytest.mark.parametrize("B,dim,Hh,d,t0,dtype", [(1, 96, 1, 16, 0, torch.float32), (1, 512, 8, 64, 300, torch.bfloat16), (16, 512, 4, 64, 300, torch.bfloat16),
+                                                 (17, 264, 2, 64, 94, torch.float16), (1, 136, 1, 128, 1100, torch.bfloat16), (1, 256, 2, 64, 1520, torch.float32)])
+def test_layer_step_of_jobs_that_are_taken_over(B, dim, Hh, d, t0, dtype):
+    """Jobs in reverse order and next to no patience: workgroups do what they had waited for, and the step comes out with the same bits.  (That they wait in vain
+    in this order is what the next test sees.)"""
+    from lookahead_keys_attention_amd import _native as N
+
+    steps = 9
+    g = torch.Generator(device=DEV).manual_seed(B + dim)
+    rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
+    norm_w, w_in, w_out = 1 + rnd(dim, std=0.2), rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5)
+    rows = [rnd(B, Hh, t0, d, std=0.6) for _ in range(4)]
+    plain, taken = (LayerSteps(B, dim, Hh, d, dtype, rows, t0 + steps, w_in, w_out, norm_w, True, True) for _ in range(2))
+    for step in range(steps):
+        x = rnd(B, 1, dim)
+        taken.proj.fill_(7)
+        ys = plain.step(x), taken.step(x, flags=N.FLAG_STEP_TAKE_OVER)
+        assert torch.all(taken.proj == 7) and torch.isfinite(ys[0]).all() and torch.equal(*ys), step
+    for a, b in zip(plain.store.buffers, taken.store.buffers):
+        assert torch.equal(a[:, :, :t0 + steps].view(torch.uint8), b[:, :, :t0 + steps].view(torch.uint8))
+
+
+@pytest.mark.parametrize("B,dim,Hh,d,t0,dtype", [(2, 96, 1, 16, 0, torch.float32), (1, 512, 8, 64, 300, torch.bfloat16), (16, 512, 4, 64, 300, torch.bfloat16),
+                                                 (17, 264, 2, 64, 94, torch.float16), (3, 136, 1, 128, 200, torch.bfloat16)])
+def test_layer_step_that_is_given_up_does_not_pass_for_a_good_one(B, dim, Hh, d, t0, dtype):
+    """Workgroups that leave instead of taking over what they wait for: what is not there is NaN, in this step's output and, where the cache is not
+    complete, in every later one.  The control words serve the next step as before."""
+    from lookahead_keys_attention_amd import _native as N
+
+    g = torch.Generator(device=DEV).manual_seed(B + dim)
+    rnd = lambda *shape, std=1.0: (torch.randn(*shape, generator=g, device=DEV) * std).to(dtype)
+    w_in, w_out = rnd(6 * Hh * d, dim, std=dim ** -0.5), rnd(dim, Hh * d, std=(Hh * d) ** -0.5)
+    rows = [rnd(B, Hh, t0, d, std=0.6) for _ in range(4)]
+    good, bad, after = (LayerSteps(B, dim, Hh, d, dtype, rows, t0 + 6, w_in, w_out, None, True) for _ in range(3))
+    x = [rnd(B, 1, dim) for _ in range(6)]
+    want, got = good.step(x[0]), bad.step(x[0], flags=N.FLAG_STEP_GIVE_UP)
+    assert got.isnan().any() and torch.isfinite(want).all()
+    assert torch.all(got.isnan() | (got == want))
+    lost = bad.store.buffers[3][:, :, :t0 + 1].isnan().flatten(1).any(1)   # sequences
+    for token in x[1:]:
+        want, got = good.step(token), bad.step(token)
+        assert got[lost].isnan().all() and torch.equal(got[~lost], want[~lost])
+    after.control = bad.control
+    fresh = LayerSteps(B, dim, Hh, d, dtype, rows, t0 + 6, w_in, w_out, None, True)
+    for token in x:
+        assert torch.equal(after.step(token), fresh.step(token))
+
+
 @pytest.mark.parametrize("B,Hh,t0,steps,d,dtype,rotary", [(2, 2, 0, 23, 64, torch.float32, False), (1, 2, 101, 18, 32, torch.float32, True),
                                                         (2, 2, 203, 21, 64, torch.bfloat16, False), (1, 2, 130, 9, 128, torch.bfloat16, True)])
 def test_decode_with_deferred_write_back(B, Hh, t0, steps, d, dtype, rotary):
