@@ -624,7 +624,8 @@ int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns)
   return castle::gemm_amax_ok(M, N, K, es, column, column + columns);
 }
 
-// The kernel forms element offsets in 32 bits and runs ahead of the last row by up to three steps of the contraction.
+// The kernels form element offsets in 32 bits.  The first step of a range of the contraction, or of the second group of waves in it, may start up to two
+// steps (128 rows, 127 of them behind the last one) from the end; places further on are only stepped to, in unsigned numbers, and never read.
 int castle_gemm_operand_ok(int64_t rows, int64_t ld) { return rows >= 0 && ld >= 0 && ld < (int64_t)1 << 31 && rows < (int64_t)1 << 31 && (rows + 192) * ld < (int64_t)1 << 31; }
 
 int castle_gemm_norm_ok(int M, int N, int K, int dtype) {

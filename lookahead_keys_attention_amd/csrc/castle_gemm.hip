@@ -82,8 +82,9 @@ template <typename T, bool KC, int FREE, int BK, int G> struct Operand {
         if (k + (KC ? col_of(j) : row_of(j)) < k_end) r[slot][j] = *reinterpret_cast<const vt*>(p + at[j]);
       }
     }
+    // (behind the end of the contraction the place of a next step may lie beyond 31 bits: it wraps, and is not read)
 #pragma unroll
-    for (int j = 0; j < N; ++j) at[j] += KC ? G * BK : G * BK * ld;
+    for (int j = 0; j < N; ++j) at[j] = (int)((uint32_t)at[j] + (uint32_t)(KC ? G * BK : G * BK * ld));
   }
   __device__ __forceinline__ void store(int slot, T* lds) const {
 #pragma unroll

@@ -121,7 +121,7 @@ def test_products_refuse_operands_beyond_32_bit_offsets(lib):
         assert gemm(64, 0, ld, 1, M=64, K=40000) == -2
         assert gemm(ld, 1, 64, 1, M=64, K=40000) == -2
         assert not lib.castle_gemm_operand_ok(40000, ld)
-    # the last element at 2^31 and just inside, three steps of the contraction ahead
+    # the last element at 2^31 and just inside, with the room that the kernels' first steps want
     assert lib.castle_gemm_operand_ok(32767 - 192, 65536) and not lib.castle_gemm_operand_ok(32768 - 192, 65536)
 
 

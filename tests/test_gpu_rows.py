@@ -331,6 +331,26 @@ def test_product_of_normalised_rows(rows, n, k, dtype):
     assert torch.all((out[0][:, :n].double() - ref).abs() <= 1.01 * bound)
 
 
+@pytest.mark.parametrize("k", [1, 63, 129, 257, 321])
+def test_products_near_the_reach_of_32_bit_offsets(k):
+    """A contraction over rows as far apart as the products take: two groups of waves step up to 382 rows behind its end."""
+    import ctypes
+
+    from lookahead_keys_attention_amd import _native as N
+
+    ld, ok = ((1 << 31) // (k + 192) - 1) // 8 * 8, N.lib().castle_gemm_operand_ok
+    ok.argtypes = [ctypes.c_int64] * 2
+    assert ok(k, ld) and not ok(k, ld + 16)
+    g = torch.Generator(device=DEV).manual_seed(k)
+    a = torch.empty(k, ld, device=DEV, dtype=torch.bfloat16)[:, ld - 64:]
+    a.copy_(torch.randn(k, 64, generator=g, device=DEV))
+    b = torch.randn(k, 72, generator=g, device=DEV).bfloat16()
+    c = host().product(a, True, b, True, 0, None)
+    ref = a.double().t().contiguous() @ b.double()
+    bound = (k + 4) * 2.0 ** -24 * (a.double().abs().t().contiguous() @ b.double().abs()) + 2.0 ** -8 * ref.abs()
+    assert torch.all((c.double() - ref).abs() <= 1.01 * bound)
+
+
 def test_projection_of_rows_beyond_32_bit_offsets():
     """Rows that lie further apart than the products' offsets reach: 40000 of them, 65536 elements apart."""
     from lookahead_keys_attention_amd import Castle
