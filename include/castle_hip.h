@@ -334,6 +334,9 @@ int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const
 #define CASTLE_GEMM_GELU_SLOPE 2
 int castle_gemm_operand_ok(int64_t rows, int64_t ld);
 int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue);
+/* What castle_gemm makes of a product, for tests and measurements: rows and columns of a workgroup's tile, ranges of the contraction, groups of four waves
+ * that share a tile of 64 x 64. */
+int castle_gemm_plan(int M, int N, int K, int dtype, int epilogue, int* rows, int* columns, int* ranges, int* groups);
 /* amax != NULL: CASTLE_AMAX_PARTIALS partial maxima of |c| over `columns` columns from `column` on (whole 16-byte pieces), for
  * CASTLE_FLAG_AMAX_READY; status, if not NULL, is set to 0.  Only where castle_gemm_amax_ok says so. */
 typedef struct castle_amax {

@@ -55,6 +55,7 @@ EXPORTED_SYMBOLS = (
     "castle_small_linear_fused",
     "castle_gemm_operand_ok",
     "castle_gemm_workspace_bytes",
+    "castle_gemm_plan",
     "castle_gemm_amax_ok",
     "castle_gemm",
     "castle_gemm_norm_ok",

@@ -618,6 +618,16 @@ int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue
   return align_up(castle::gemm_workspace(M, N, K, es, epilogue != CASTLE_GEMM_PLAIN), 256);
 }
 
+int castle_gemm_plan(int M, int N, int K, int dtype, int epilogue, int* rows, int* columns, int* ranges, int* groups) {
+  const int64_t need = castle_gemm_workspace_bytes(M, N, K, dtype, epilogue);
+  if (need < 0) return (int)need;
+  if (rows == nullptr || columns == nullptr || ranges == nullptr || groups == nullptr) return CASTLE_ERR_ARG;
+  int out[4];
+  castle::gemm_plan(M, N, K, elem_size(dtype), epilogue != CASTLE_GEMM_PLAIN, out);
+  *rows = out[0]; *columns = out[1]; *ranges = out[2]; *groups = out[3];
+  return CASTLE_OK;
+}
+
 int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns) {
   const int es = elem_size(dtype);
   if (es == 0 || M <= 0 || N <= 0 || K <= 0 || column < 0 || columns <= 0 || column + columns > N || column % (16 / es) != 0 || columns % (16 / es) != 0) return 0;

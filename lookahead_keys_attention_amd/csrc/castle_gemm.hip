@@ -694,6 +694,11 @@ int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue) {
   return p.splits > 1 ? (int64_t)p.splits * M * N * 4 : 0;
 }
 
+void gemm_plan(int M, int N, int K, int elem_size, bool epilogue, int (&out)[4]) {
+  const Plan p = plan(M, N, K, !epilogue, elem_size);
+  out[0] = p.rows(); out[1] = p.columns(); out[2] = p.splits; out[3] = p.groups;
+}
+
 // the maximum is taken on the store: not for a contraction in ranges, nor for more tiles than there are slots
 bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to) {
   const Plan p = plan(M, N, K, true, elem_size);

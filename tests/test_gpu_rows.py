@@ -280,10 +280,57 @@ def test_products_of_two_groups(rows, n, k, dtype):
                                       (2112, 6144, 1024)])
 def test_products_of_wide_tiles(rows, n, k, dtype):
     """Tiles of 256 x 128 and 256 x 256 in each layout: last ones of 64 rows and columns and of odd eights, even and odd numbers of steps,
-    one tile a CU and several, ranges of the contraction."""
+    one tile a CU, ranges of the contraction."""
     test_products(rows, n, k, dtype)
     if dtype == torch.bfloat16 and n > k:
         test_product_leaves_partial_maxima(rows, n, k, 520, 256)
+
+
+def gemm_plan(M, N, K, dtype, epilogue):
+    """(rows, columns) of a tile, and how many of them a launch has."""
+    import ctypes
+
+    from lookahead_keys_attention_amd import _native
+
+    out = [ctypes.c_int() for _ in range(4)]
+    _native.check(_native.lib().castle_gemm_plan(M, N, K, _native.DTYPE_CODES[dtype], epilogue, *map(ctypes.byref, out)), "castle_gemm_plan")
+    rows, columns, ranges, _ = (v.value for v in out)
+    return (rows, columns), -(-M // rows) * -(-N // columns) * ranges
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,plain,fused", [(16456, 1032, 512, (256, 128), None), (8456, 1992, 256, (256, 128), None), (8456, 3064, 256, (256, 256), None),
+                                               (8456, 3064, 512, (256, 256), (256, 256)), (16456, 2040, 512, (256, 128), (256, 128)),
+                                               (16456, 3064, 256, (256, 128), (256, 128))])
+def test_products_of_several_wide_tiles_a_workgroup(M, N, K, plain, fused, dtype):
+    """More tiles of 256 rows than CUs, so that a workgroup goes on to the next while the last is being stored, between whole tiles and ones with remainders, in
+    each layout and with gelu, its slope and the maxima on the store.  Element by element: K products and sums of 2^-24 each, at most, and the roundings
+    to the type; gelu of the rounded product to 2^-20 before its own."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    a, b, u = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((M, K), (N, K), (M, N)))
+    ref, size, bits = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t(), {torch.bfloat16: 8, torch.float16: 11}[dtype]
+    error = (K + 4) * 2.0 ** -24 * size + 2.0 ** -bits * ref.abs()
+    layouts = [(a, False, b, False), (a, False, b.t().contiguous(), True), (a.t().contiguous(), True, b.t().contiguous(), True)]
+    tile, tiles = gemm_plan(M, N, K, dtype, 0)
+    assert tile == plain and tiles > 256
+    for operands in layouts:
+        assert torch.all((host().product(*operands, 0, None).double() - ref).abs() <= 1.01 * error)
+    if dtype == torch.bfloat16:
+        test_product_leaves_partial_maxima(M, N, K, 520, 256)
+    if fused is None:
+        return
+    tile, tiles = gemm_plan(M, N, K, dtype, 1)
+    assert tile == fused and tiles > 256
+    v = u.double()
+    slope = torch.special.ndtr(v) + v * torch.exp(-v * v / 2) / (2 * torch.pi) ** 0.5
+    for operands in layouts:
+        act = torch.empty_like(u)
+        up = host().product(*operands, 1, act)
+        assert torch.all((up.double() - ref).abs() <= 1.01 * error)
+        gelu = F.gelu(up.double())
+        assert torch.all((act.double() - gelu).abs() <= 1.01 * 2.0 ** -bits * gelu.abs() + 2.0 ** -20 * up.double().abs() + 2.0 ** -24)
+        got = host().product(*operands, 2, u).double()
+        assert torch.all((got - ref * slope).abs() <= 1.01 * (slope.abs() * error + 2.0 ** -bits * (ref * slope).abs()) + 2.0 ** -18 * ref.abs())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
