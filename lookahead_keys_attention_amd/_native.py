@@ -26,6 +26,7 @@ FLAG_ROTARY = 2          # rotary position embedding of qc, kc, qu, ku, vu insid
 FLAG_RECOMPUTE_SCORES = 4   # backward without the dS / dSu tile hand-over (less workspace, slower)
 FLAG_RECOMPUTE_STATE = 8    # backward re-runs the forward scan: the forward state buffer need not be kept
 FLAG_U_HALF = 16            # bf16 caches: the lookahead-key buffer holds fp16 bits of U / 64 (see castle_hip.h)
+FLAG_READ_ONCE = 32         # cached step: the loop it belongs to reads more than the last-level cache holds
 FLAG_STEP_TAKE_OVER = 128   # tests of a layer step in one launch: jobs in reverse order, taken over by those that wait for them
 FLAG_STEP_GIVE_UP = 256     # the same, given up instead
 U_HALF_UNSCALE = 64.0

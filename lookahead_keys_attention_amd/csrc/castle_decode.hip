@@ -727,9 +727,13 @@ static bool views_alike(const DecodeArgs& a) {
 }
 template <typename T, int HD, bool UH> static void launch_stream(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid(a.splits, a.B * a.H);
-  if (!views_alike(a)) hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, false, false>), grid, dim3(kThreads), 0, stream, a);
-  else if (a.read_once) hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, true, true>), grid, dim3(kThreads), 0, stream, a);
-  else hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, false, true>), grid, dim3(kThreads), 0, stream, a);
+  auto go = [&](auto once, auto alike) {
+    hipLaunchKernelGGL((decode_stream_kernel<T, HD, UH, decltype(once)::value, decltype(alike)::value>), grid, dim3(kThreads), 0, stream, a);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  if (views_alike(a)) a.read_once ? go(yes, yes) : go(no, yes);
+  else a.read_once ? go(yes, no) : go(no, no);
 }
 template <typename T, int HD> static int launch_decode_t(const DecodeArgs& a, hipStream_t stream) {
   {

@@ -446,10 +446,10 @@ def test_decode_step_ignores_what_lies_beyond_the_count(Hh, d, dtype, t):
     rnd = lambda *shape: (torch.randn(*shape, generator=g, device=DEV) * 0.6).to(dtype)
     rows, steps = [rnd(B, Hh, t, d) for _ in range(4)], [[rnd(B, Hh, 1, d) for _ in range(6)] for _ in range(3)]
     results = []
-    for kind in ("zero", "nan", "device", "strides"):
+    for kind in ("zero", "nan", "device", "strides", "strides, read once"):
         store = _CacheStore(B, Hh, d, cap, dtype, torch.device(DEV))
         fill = 0.0 if kind == "zero" else float("nan")
-        caches = [torch.full((B, Hh, cap, d + (16 * i if kind == "strides" else 0)), fill, dtype=dtype, device=DEV)[..., :d] for i in range(4)]
+        caches = [torch.full((B, Hh, cap, d + (16 * i if kind.startswith("strides") else 0)), fill, dtype=dtype, device=DEV)[..., :d] for i in range(4)]
         for cache, row in zip(caches, rows):
             cache[:, :, :t] = row
         for extra in store.rings:
@@ -463,13 +463,17 @@ def test_decode_step_ignores_what_lies_beyond_the_count(Hh, d, dtype, t):
                 N.check(N.lib().castle_decode_step_device_count(*[N.view4(c) for c in caches], count.data_ptr(), cap, *[N.view4(x) for x in token], B, Hh, d,
                                                                 N.dtype_code(dtype), d ** -0.5, N.FLAG_ROTARY, N.view4(out), deferred, store.workspace.data_ptr(),
                                                                 store.workspace.numel(), N.stream_ptr(out.device)), "castle_decode_step_device_count")
+            elif kind == "strides, read once":
+                N.check(N.lib().castle_decode_step(*[N.view4(c) for c in caches], t + i, cap, *[N.view4(x) for x in token], B, Hh, d, N.dtype_code(dtype),
+                                                   d ** -0.5, N.FLAG_ROTARY | N.FLAG_READ_ONCE, N.view4(out), deferred, store.workspace.data_ptr(),
+                                                   store.workspace.numel(), N.stream_ptr(out.device)), "castle_decode_step")
             else:
                 H().castle_decode_step_hip(*caches, t + i, *token, d ** -0.5, out, store.workspace, rotary=True, deferred=deferred)
             outs.append(out)
         results.append((torch.cat(outs, 2), torch.stack([c[:, :, :t + 3] for c in caches])))
     for out, cached in results:
         assert torch.isfinite(out.float()).all()
-    for (out, cached), kind in zip(results[1:], ("nan", "device", "strides")):
+    for (out, cached), kind in zip(results[1:], ("nan", "device", "strides", "strides, read once")):
         if kind == "device":   # (its splits are those of a full cache: sums in another order, roundings of the results)
             assert_close(out.float(), results[0][0].cpu().double(), dtype, kind, 1e-5)
         else:
