@@ -249,9 +249,7 @@ __global__ __launch_bounds__(kThreads, (scan_waves_per_simd<T, HD>())) void scan
 
 // ---------------------------------------------------------------------------
 // G: groups of four waves.  Two take alternate chunks of the keys of the same rows, each in LDS of its own, and are merged at the end: a
-// workgroup with a CU to itself then has the two waves per SIMD that the kernel needs, from its first chunk to its last.  Where the longest
-// row block is the time (d = 128; forward pass, one group / two: 2 x 16 heads x 2048 rows 276 / 264 us, 1 x 16 x 4096 482 / 458, 6 x 16 x 333 81 /
-// 75); a GPU that is full anyway does the same work faster in separate workgroups (3 x 16 x 2048 378 / 408).
+// workgroup with a CU to itself then has the two waves per SIMD that the kernel needs, from its first chunk to its last.
 template <typename T, typename TI, int HD, int G>
 __global__ __launch_bounds__(kThreads * G, sizeof(T) == 2 ? 2 : 1) void attn_kernel(FwdArgs a) {
   constexpr int KS = HD / 16;
@@ -276,7 +274,8 @@ __global__ __launch_bounds__(kThreads * G, sizeof(T) == 2 ? 2 : 1) void attn_ker
 
   if (G == 1) prio_by_band(blockIdx.x, a.s.cus);
   int rank, bh;
-  work_item(a.s.B * a.s.H, rank, bh);
+  if (G == 1 && (int)gridDim.x <= 2 * a.s.cus) work_item_snake(a.s.B * a.s.H, a.s.Lp / 128, a.s.cus, rank, bh);
+  else work_item(a.s.B * a.s.H, rank, bh);
   const int qb = a.s.Lp / 128 - 1 - rank;   // the last query block sees the most keys
   const int b = bh / a.s.H, h = bh % a.s.H;
   const int lane = lane_id(), wave = G == 1 ? wave_id() : wave_id() % 4, c = lane & 31, g = lane >> 5;
@@ -545,7 +544,13 @@ template <typename T, typename TI, int HD> static int launch_attn_t(const FwdArg
   ProfScope ps(kSlotAttn, stream);
   const dim3 grid(a.s.Lp / 128 * a.s.B * a.s.H);
   if constexpr (PAIRS) {
-    if ((int)grid.x <= 2 * a.s.cus) {   // as far as the longest row blocks and not their sum bound the launch
+    // As far as the longest row blocks and not their sum bound the launch: up to two workgroups a CU, and a half less where a head has few row blocks,
+    // whose second group has little to share and is merged all the same (forward pass of heads x rows, us, one group / two: 32 x 2048 270 / 259, 16 x
+    // 4096 476 / 455, 10 x 4000 441 / 390, 64 x 1024 166 / 166, 46 x 1408 220 / 217, 90 x 512 107 / 104, 60 x 768 129 / 115; 128 x 512 120 / 126, 85 x 768 151 / 158, 100 x
+    // 352 83 / 84, 170 x 352 113 / 122, 130 x 256 68 / 70, 512 x 128 84 / 95).  A GPU that is full anyway does the same work faster in separate
+    // workgroups (3 x 16 x 2048 378 / 408).
+    const int blocks = a.s.Lp / 128;
+    if ((int)grid.x <= 2 * a.s.cus && blocks >= 4 && (blocks >= 8 || (int)grid.x <= a.s.cus * 3 / 2)) {
       hipLaunchKernelGGL((attn_kernel<T, TI, HD, 2>), grid, dim3(2 * kThreads), 2 * attn_lds, stream, a);
       return hipGetLastError() == hipSuccess ? 0 : -3;
     }

@@ -110,10 +110,10 @@ def test_operator_with_long_walks_shared_by_eight_waves(B, Hh, L, d):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("Hh,L", [(300, 1), (257, 33), (512, 96), (257, 128), (130, 129), (100, 352), (40, 1000)])
+@pytest.mark.parametrize("Hh,L", [(300, 1), (257, 33), (512, 96), (257, 128), (130, 129), (100, 352), (40, 1000), (65, 385), (96, 500), (60, 705), (33, 961), (33, 993), (64, 1024)])
 def test_wide_heads_by_two_groups_of_waves(Hh, L, dtype):
-    """d = 128 at one and two row blocks a CU, where two groups of waves share the keys of a row, against the same heads among others: one
-    chunk, odd and even numbers of them, a last one that only the first group has."""
+    """d = 128 at one and two row blocks a CU, where two groups of waves share the keys of a row if a head has four row blocks or more, against the same heads
+    among others: odd and even numbers of chunks, a last one that only the first group has."""
     g = torch.Generator(device="cuda").manual_seed(L)
     six = [torch.randn(1, Hh, L, 128, generator=g, device="cuda").to(dtype) for _ in range(6)]
     blocks = Hh * ((L + 127) // 128)
@@ -131,7 +131,7 @@ def test_wide_heads_by_two_groups_of_waves(Hh, L, dtype):
 def test_wide_heads_with_scores_of_minus_infinity(first, last, dtype):
     """Keys whose scores are -inf have no weight, also where one of two groups of waves sees nothing else at first: what many heads, by one group, and
     the oracle give without them."""
-    Hh, L, d = 100, 352, 128
+    Hh, L, d = 65, 480, 128
     g = torch.Generator(device="cuda").manual_seed(first)
     six = [torch.randn(1, Hh, L, d, generator=g, device="cuda").to(dtype) for _ in range(6)]
     six[0][..., 0] = six[0][..., 0].abs() + 0.1
