@@ -61,8 +61,9 @@ template <typename T, bool KC, int FREE, int BK, int G> struct Operand {
   // data: those outputs are not stored.
   int at[N];
   vt r[2][N];
-  static __device__ __forceinline__ int row_of(int j) { return (threadIdx.x % kThreads + j * kThreads) / VPR; }
-  static __device__ __forceinline__ int col_of(int j) { return (threadIdx.x % kThreads + j * kThreads) % VPR * V; }
+  static __device__ __forceinline__ int thread() { return G == 1 ? threadIdx.x : threadIdx.x % kThreads; }
+  static __device__ __forceinline__ int row_of(int j) { return (thread() + j * kThreads) / VPR; }
+  static __device__ __forceinline__ int col_of(int j) { return (thread() + j * kThreads) % VPR * V; }
   __device__ __forceinline__ void start(int ld, int free0, int free_end, int k0) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
   constexpr int V = elem_traits<T>::vec16, LDC = BN + V;
   constexpr int kStage = 2 * (OpA::ELEMS + OpB::ELEMS), kOut = BM * LDC;
   __shared__ __attribute__((aligned(16))) T smem[G * kStage > kOut ? G * kStage : kOut];
-  const int lane = lane_id(), wave = wave_id() % 4, group = wave_id() / 4, c = lane & 31, g = lane >> 5;
+  const int lane = lane_id(), wave = G == 1 ? wave_id() : wave_id() % 4, group = G == 1 ? 0 : wave_id() / 4, c = lane & 31, g = lane >> 5;
   // Workgroups go round the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the tiles, so the rows of
   // `a` are read by one XCD, not by all (input gradient of 3000 rows x 1536 x 256: 13.5 -> 11.1 us).  A workgroup takes
   // several tiles where there are more than the CUs hold: the first steps of the next are requested before the
@@ -318,7 +319,7 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
       __shared__ float s_most[G * kThreads / 64];
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) most = fmaxf(most, __shfl_xor(most, o));
-      if (lane == 0) s_most[wave_id()] = most;
+      if (lane == 0) s_most[G == 1 ? wave : wave_id()] = most;
       __syncthreads();
       if (threadIdx.x == 0) {
 #pragma unroll
