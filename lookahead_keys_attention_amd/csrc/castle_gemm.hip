@@ -607,48 +607,57 @@ template <typename T, bool AK, bool BKC, int BN, bool FUSED> __global__ __launch
   }
 }
 
-// Tile, number of ranges of the contraction and groups of a workgroup, from what a launch takes (us, measured over 96 ... 16384 rows,
-// outputs of 128 ... 3072 columns and contractions of 128 ... 16384, with outputs that no cache holds): 2.3, and for each tile of a CU
-// so much a step and at its end, more at the end where gelu or its derivative rides on the store.  A second group takes a step of a
-// workgroup of 64 x 64 that has a CU to itself from 0.42 to 0.36, fp32 from 0.78 to 0.66, for 0.3 at the end (one range, one group / two:
-// 3000 rows of 1536 -> 256 12.7 / 9.9, 256 rows of fp32 512 -> 3072 15.1 / 13.1); at two workgroups a CU it gains where the contraction is
-// long (3000 rows of 3072 -> 512 29 / 26, of 512 -> 512 level), behind from three on.  A split adds a second launch, 2.5, and its partial
-// results, written and read.  Weight gradient of 3000 rows, 1536 x 256 out: 22.6 us in one range, 14.1 in two of two groups; 3008 rows
-// 512 -> 2048 17.6 on 64 x 64, 16.6 on 128 x 128, 14.2 on 256 x 128; 4096 rows 512 -> 3072 31.8, 26.2, 24.9 and 21.8 on 256 x 256.
+// Tile, number of ranges of the contraction and groups of a workgroup, from what a launch takes (us): a start (2.3 for tiles of 64 and 128 rows, where
+// gelu or its derivative rides on the store within the end of a tile), and for each tile of the fullest CU so much a step and at its end, more at the end where
+// gelu or its derivative rides on the store.  A second group takes a step of a workgroup of 64 x 64 that has a CU to itself from 0.42 to 0.36, fp32 from 0.78 to
+// 0.66, for 0.3 at the end, and pays from eight steps on, fp32 four (3000 rows of 1536 -> 256 12.7 with one, 9.9 with two, 1504 rows of 256 -> 512 5.3 and 6.1; 256
+// rows of fp32 512 -> 3072 15.1 and 13.1); at two workgroups a CU it gains where the contraction is long (3000 rows of 3072 -> 512 29 / 26, of 512 -> 512
+// level), behind from three on.  A split adds a second launch, 2.5, and its partial results, written and read, and tiles of 256 rows another start.
+// Weight gradient of 3000 rows, 1536 x 256 out: 22.6 in one range, 13.7 in two of two groups; 3008 rows 512 -> 2048 17.6 on 64 x 64, 16.6 on 128 x 128, 14.2 on
+// 256 x 128; 4096 rows 512 -> 3072 31.8, 26.2, 24.9 and 21.8 on 256 x 256; 8184 rows 64 -> 4096 20.0, 18.6, 15.8 and 15.3.  Over 2500 products of 96 ... 65536
+// rows, outputs of 64 ... 4096 columns and contractions of 64 ... 8184, in all layouts, each timed with every tile and up to 16 ranges, what this picks takes 1.5 %
+// more than the best of them on average.
 struct Plan {
   int tile, splits, groups;   // tile: 64, 128, or columns of a tile of 256 rows + 256
   int rows() const { return std::min(tile, kWideM); }
   int columns() const { return tile > kWideM ? tile - kWideM : tile; }
   int tiles(int M, int N) const { return ((M + rows() - 1) / rows()) * ((N + columns() - 1) / columns()); }
 };
+// workgroups of the fullest CU: tiles go to eight XCDs of 32 CUs each, so one of them may have work for 33 (weight gradient of 8184 rows, 640 x 320: 50 tiles in
+// five ranges 21.6 us, in four 16.9)
+int64_t on_a_cu(int64_t tiles, int splits) { return ((tiles + 7) / 8 * splits + 31) / 32; }
 Plan plan(int M, int N, int K, bool plain, int elem_size) {
   Plan best = {64, 1, 1};
   double best_cost = 1e30;
   auto take = [&](double cost, const Plan& p) {
     if (cost < best_cost) { best_cost = cost; best = p; }
   };
+  // Two tensors that no cache holds: stores of single lines cost more (gelu of 65536 rows 64 -> 1536 on 64 x 64 123, on 256 x 256 94), and 256 x 256 where rows do not
+  // start with lines (33000 rows 64 -> 3064 192, 256 x 128 103, 64 x 64 150).
+  const bool far = !plain && 4.0 * M * N > 2.5e8;
   for (int tile = 64; tile <= (elem_size == 2 ? 128 : 64); tile += 64) {
     const double alone = elem_size == 4 ? 0.78 : tile == 64 ? 0.42 : 0.85, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.29 : 0.6;
-    const double end = elem_size == 4 ? 0 : tile == 64 ? 0.25 : 2.3, fused = plain ? 0 : tile == 64 ? 0.5 : 2.6;
+    const double fused = plain ? 0 : tile == 128 ? 2.6 : far ? 1 : 0.5;
     const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
     const int steps = (K * elem_size + 127) / 128;   // 128 bytes of the contraction a step
     for (int s = 1; s <= (plain ? std::min(16, (steps + 1) / 2) : 1); ++s) {
-      const int64_t per_cu = (tiles * s + 255) / 256, n = (steps + s - 1) / s;
-      const int groups = tile == 64 && (per_cu == 1 ? n >= 4 : elem_size == 2 && s == 1 && per_cu == 2 && n >= 12) ? 2 : 1;
+      const int64_t per_cu = on_a_cu(tiles, s), n = (steps + s - 1) / s;
+      const double end = elem_size == 4 ? 0 : tile == 64 ? 0.25 : s > 1 ? 1 : 2.3;   // (partial results do not go through LDS)
+      const int groups = tile == 64 && (per_cu == 1 ? n >= (elem_size == 4 ? 4 : 8) : elem_size == 2 && s == 1 && per_cu == 2 && n >= 12) ? 2 : 1;
       double cost = groups == 2 ? 0.3 + n * (elem_size == 4 ? 0.66 : per_cu == 1 ? 0.36 : 0.55) : per_cu == 1 ? n * alone + end : per_cu * (n * shared + end);
       if (s > 1) cost += 2.5 + (double)s * M * N * 8 / 4e6;
-      take(cost + (per_cu == 1 ? 2 : per_cu) * fused, {tile, s, groups});
+      take((plain ? 2.3 : 0) + cost + (per_cu == 1 ? 2 : per_cu) * fused, {tile, s, groups});
     }
   }
   if (elem_size == 2 && K % kWideK == 0) {
     for (int columns = 128; columns <= 256; columns += 128) {
-      const double start = columns == 128 ? 1.6 : 2.6, end = columns == 128 ? (plain ? 3 : 8.8) : plain ? 6.5 : 16.5;
+      const double start = plain ? 3.5 : columns == 128 ? 1.6 : 2.6, end = columns == 128 ? (plain ? 1.8 : 8.8) : plain ? 4 : far && N % 64 != 0 ? 24.5 : 16.5;
       const int64_t tiles = (int64_t)((M + kWideM - 1) / kWideM) * ((N + columns - 1) / columns);
       const int steps = K / kWideK;
-      for (int s = 1; s <= (plain ? std::min(16, steps / 4) : 1); ++s) {
-        const int64_t per_cu = (tiles * s + 255) / 256, n = (steps + s - 1) / s;
+      for (int s = 1; s <= (plain ? std::min(16, std::max(1, steps / 4)) : 1); ++s) {
+        const int64_t per_cu = on_a_cu(tiles, s), n = (steps + s - 1) / s;
         const double busy = std::min(1., tiles * s / 256.), step = columns == 128 ? 0.75 + 0.27 * busy : 1.2 + 0.36 * busy;
-        take(start + per_cu * (n * step + end) + (s > 1 ? 2.5 + (double)s * M * N * 8 / 6e6 : 0), {kWideM + columns, s, 1});
+        take(start + per_cu * (n * step + end) + (s > 1 ? 4.8 + (double)s * M * N * 8 / 6e6 : 0), {kWideM + columns, s, 1});
       }
     }
   }
@@ -683,7 +692,8 @@ template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p,
       return hipGetLastError() == hipSuccess ? 0 : -3;
     }
   }
-  if (p.groups == 2) hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK, 2>), grid, dim3(2 * kThreads), 0, stream, a);
+  // (both operands contraction-strided at two workgroups a CU: one group, weight gradients of 1000 rows 512 x 3072 13.2 us and with two 14.2, of 3000 30.4 / 32.1)
+  if (p.groups == 2 && (AK || on_a_cu(tiles, p.splits) == 1)) hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK, 2>), grid, dim3(2 * kThreads), 0, stream, a);
   else hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK, 1>), grid, dim3(kThreads), 0, stream, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

@@ -464,19 +464,19 @@ Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epi
 // Own products where a call is short: the library's costs 18 us of host time, one here 4.  On the GPU they are level or
 // ahead up to the sizes below (us, own / library: input gradient of 1000 rows x 3072 x 512 15 / 16, 4096 x 3072 x 512 31 / 31, 8192 x 3072 x
 // 512 44 / 39; weight gradient of 3000 rows, 1536 x 256, 14 / 27, of 4096, 3072 x 512, 31 / 41; forward of 4096 rows 1024 -> 3072 31 / 30).
-// Contractions of 256 to 512 in whole steps of 64: ahead at every size measured up to 309 GFLOP (the line lies between that and 206), since a tile's start and end weigh more there than its
-// steps, and the store takes gelu and the maxima along (16384 rows 256 -> 3072 38 / 44, 448 -> 3072 57 / 59, 512 -> 2048 43 / 45, 512 -> 3072 60 / 64, 512 -> 512 14 /
-// 20, 65536 rows 512 -> 3072 227 / 246, 98304 rows 354 / 359, 131072 rows 478 / 473; input gradients 41 / 46, 56 / 62, -, 61 / 68, 14 / 20, 228 / 257, 361 / 379, 484 / 500).
-// Shorter ones are bound by the store of outputs that no cache holds, which is slower here (65536 rows, 64 -> 3072 138 / 100, 128 -> 3072 162 / 122, 192 -> 3072 173 /
-// 146; level at 16384: 29 / 29, 38 / 35, 39 / 38; input gradients of 16384 rows 128 -> 1024 16 / 19, 8192 of 128 -> 3072 22 / 24, 16384 37 / 36), longer ones are level at 16384 rows (forward 576 -> 3072 64 / 59, 640 68 / 64, 768 76 / 72).
+// Contractions of up to 512 in whole steps of 64: ahead at every size measured up to 309 GFLOP (the line lies between that and 206), since a tile's start
+// and end weigh more there than its steps, and the store takes gelu and the maxima along (forward / input gradient, 16384 rows 64 -> 3072 24 / 29 and
+// 24 / 30, 128 -> 3072 30 / 32 and 31 / 35, 256 -> 3072 38 / 43 and 38 / 45, 512 -> 3072 59 / 62 and 59 / 67, 512 -> 512 14 / 20 and 14 / 20; 65536 rows 64 -> 3072 81 /
+// 100 and 82 / 105, 128 -> 3072 103 / 126 and 105 / 129, 512 -> 3072 227 / 240 and 228 / 253; 98304 rows 354 / 359 and 361 / 379, 131072 rows 478 / 473 and 484 /
+// 500).  Longer ones are level at 16384 rows (forward 576 -> 3072 64 / 59, 640 68 / 64, 768 76 / 72).
 // In fp32 they are level up to the size below (256 rows, 512 <-> 3072: forward 13 / 13, input gradient 16 / 12,
 // weight gradient 15 / 16), where a layer's time is the host's; 2048 rows 60 / 53, 64 / 49, 72 / 55.
 bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16, double most_32) {
   return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
 }
-bool own_contraction(int64_t k) { return k >= 256 && k <= 512 && k % 64 == 0; }   // (others have no tiles of 256 rows)
+bool own_contraction(int64_t k) { return k <= 512 && k % 64 == 0; }   // (others have no tiles of 256 rows)
 double own_forward(int64_t k) { return own_contraction(k) ? 260e9 : 14e9; }
-double own_input_grad(int64_t k) { return own_contraction(k) ? 260e9 : k < 256 ? 7e9 : 4e9; }
+double own_input_grad(int64_t k) { return own_contraction(k) ? 260e9 : 4e9; }
 constexpr double kOwnWeightGrad = 40e9, kOwn32 = 1e9;
 constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 73 / 91
 
