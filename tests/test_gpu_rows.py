@@ -266,12 +266,14 @@ def test_products(rows, n, k, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,n,k", [(65, 72, 264), (130, 264, 328), (192, 64, 1000), (320, 512, 136)])
+@pytest.mark.parametrize("rows,n,k", [(65, 72, 264), (130, 264, 328), (192, 64, 1000), (320, 512, 136), (456, 584, 520), (511, 456, 584)])
 def test_products_of_two_groups(rows, n, k, dtype):
-    """One tile a CU and a contraction of four steps and more: even and odd numbers of steps, a last one that is partly filled, one that
-    only the first group has."""
+    """One tile a CU and a contraction of four steps and more (16-bit operands: eight): even and odd numbers of steps, a last one that is
+    partly filled, one that only the first group has."""
+    if rows > 400 and dtype == torch.bfloat16:   # in each layout; the others are so in some layouts, fp32 also in ranges of the contraction
+        assert all(gemm_plan(*sizes, dtype, 0, groups=True) == 2 for sizes in ((rows, n, k), (rows, k, n), (n, k, rows)))
     test_products(rows, n, k, dtype)
-    if dtype == torch.bfloat16 and 256 <= k < 512:   # (a longer contraction is split, and its maxima are not taken)
+    if dtype == torch.bfloat16 and (256 <= k < 512 or rows > 400):   # (split elsewhere, and no maxima are taken)
         test_product_leaves_partial_maxima(rows, n, k, 8, n - 16)
 
 
@@ -286,15 +288,17 @@ def test_products_of_wide_tiles(rows, n, k, dtype):
         test_product_leaves_partial_maxima(rows, n, k, 520, 256)
 
 
-def gemm_plan(M, N, K, dtype, epilogue):
-    """(rows, columns) of a tile, and how many of them a launch has."""
+def gemm_plan(M, N, K, dtype, epilogue, groups=False):
+    """(rows, columns) of a tile, and how many of them a launch has; or how many groups of waves share one."""
     import ctypes
 
     from lookahead_keys_attention_amd import _native
 
     out = [ctypes.c_int() for _ in range(4)]
     _native.check(_native.lib().castle_gemm_plan(M, N, K, _native.DTYPE_CODES[dtype], epilogue, *map(ctypes.byref, out)), "castle_gemm_plan")
-    rows, columns, ranges, _ = (v.value for v in out)
+    rows, columns, ranges, waves = (v.value for v in out)
+    if groups:
+        return waves
     return (rows, columns), -(-M // rows) * -(-N // columns) * ranges
 
 
