@@ -15,6 +15,10 @@ template <typename F> int by_type(int dtype, bool bf16_operands, F&& f) {
     default: return -1;
   }
 }
+template <typename F> int by_type16(int dtype, bool bf16_operands, F&& f) {   // 16-bit tensors only
+  if (dtype == 1) return bf16_operands ? f(bf16_t(), bf16_t()) : f(fp16_t(), bf16_t());
+  return dtype == 2 ? f(fp16_t(), fp16_t()) : -1;
+}
 // f(std::integral_constant<int, d>); fp32 kernels exist up to d = 64
 template <typename T, typename F> int by_head_dim(int d, F&& f) {
   switch (d) {

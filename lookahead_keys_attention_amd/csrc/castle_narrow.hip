@@ -8,9 +8,8 @@
 // (no barriers), and the partial results meet once at the end, in fp32 through LDS.  Every operand tile is copied as whole
 // lines into LDS that belongs to one wave, while the tile before it is worked on; the rows of the workgroup itself are
 // in LDS once, for all waves.  What bounds them is the wait for those tiles, two waves per SIMD at most (one at d = 128 and
-// fp32), and for fp32 the matrix instructions: operator forward and backward at 2 x 8 heads of 1024 rows 1426 -> 431 us
-// in fp32; 8 x 4 heads of 777 rows at d = 32 in fp16 269 -> 116 us (with the host path measured; the kernels took 193
-// of it and take 136 with the small kernels around them).
+// fp32): 8 x 4 heads of 777 rows at d = 32 in fp16 269 -> 116 us (operator forward and backward with the host path; the kernels took 193
+// of it and take 136 with the small kernels around them).  fp32 tensors run here below 128 rows only (see split_fp32).
 //
 //   scan_narrow    32 keys; the waves split the source blocks: every wave sums its own part first, then sweeps it
 //                  again from the sum of the parts before it, storing the snapshots (two gates per pair instead
@@ -36,25 +35,13 @@
 #include "castle_params.h"
 #include "castle_profile.h"
 #include "castle_tqv.h"
+#include "castle_waves.h"
 #include "castle_dispatch.h"
 #include "castle_narrow.h"
 
 namespace castle {
 
 extern __shared__ __attribute__((aligned(16))) unsigned char castle_smem[];
-
-// Waits out the longest matrix instruction (see the note on branches above): in front of the first reads of accumulators
-// whose last product sits in a loop or a branch that has just ended.
-__device__ __forceinline__ void settle() {
-  asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-// LDS traffic of one wave is in order; this keeps the compiler from moving it (and, where registers are short, from
-// requesting operands of the next stage early)
-template <bool STAGES = false> __device__ __forceinline__ void wave_lds_order() {
-  asm volatile("" ::: "memory");
-  if constexpr (STAGES) __builtin_amdgcn_sched_barrier(0);
-}
 
 // Two-phase copy of a 32 x COLS tile whose rows are contiguous in memory into a row-major LDS tile, by one wave: every
 // load covers 1 KB of consecutive addresses.  (MFMA fragments straight from global memory touch 32 lines per
@@ -107,67 +94,10 @@ template <typename T, int HD> __device__ __forceinline__ void put_rows32(T* tile
   for (int s = 0; s < HD / 16; ++s) *reinterpret_cast<frag_mem<T>*>(tile + c * LD + 16 * s + 8 * g) = f[s];
 }
 
-// Sums accumulator tiles over the W waves of a workgroup; wave w hands the quads q % W == w (four consecutive rows
-// n = 32 nt + 8 q + 4 g .. of the lane's column) to f(nt, q, sum)
-template <int W, int NT, typename F>
-__device__ __forceinline__ void reduce_waves(float* lds, const acc_t (&acc)[NT], int wave, int lane, F&& f) {
-  typedef vec<float, 4> v4;
-  v4* s = reinterpret_cast<v4*>(lds);
-  settle();
-  __syncthreads();   // whatever the memory held before is dead
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) s[(wave * NT * 4 + nt * 4 + q) * 64 + lane] = v4{acc[nt][4 * q], acc[nt][4 * q + 1], acc[nt][4 * q + 2], acc[nt][4 * q + 3]};
-  __syncthreads();
-#pragma unroll
-  for (int t = 0; t < NT * 4; ++t) {
-    if (t % W != wave) continue;
-    v4 sum = s[t * 64 + lane];
-#pragma unroll
-    for (int w = 1; w < W; ++w) sum += s[(w * NT * 4 + t) * 64 + lane];
-    f(t / 4, t % 4, sum);
-  }
-}
-
-// the sum of one accumulator tile over the waves, in every wave
-template <int W> __device__ __forceinline__ void total_of_waves(float* lds, acc_t& acc, int wave, int lane) {
-  typedef vec<float, 4> v4;
-  v4* s = reinterpret_cast<v4*>(lds);
-  settle();
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 4; ++q) s[(wave * 4 + q) * 64 + lane] = v4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    v4 sum = s[q * 64 + lane];
-#pragma unroll
-    for (int w = 1; w < W; ++w) sum += s[(w * 4 + q) * 64 + lane];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[4 * q + e] = sum[e];
-  }
-}
-
-// four consecutive columns n .. n + 3 of a gradient row, rotated back (pos >= 0) and scaled
-template <typename TI, int HD> __device__ __forceinline__ void store_quad(TI* row, int n, vec<float, 4> v, float mul, int pos) {
-  if (n >= HD) return;
-  if (pos >= 0) {
-    CASTLE_ROPE_PAIR(v[0], v[1], (float)pos, n / 2, HD, true);
-    CASTLE_ROPE_PAIR(v[2], v[3], (float)pos, n / 2 + 1, HD, true);
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] *= mul;
-  st4<TI>(row + n, __builtin_convertvector(v, vec<TI, 4>));
-}
-
-template <int HD> constexpr int narrow_nt() { return (HD < 32 ? 32 : HD) / 32; }
 template <typename T, int HD> constexpr int wave_tile_bytes() { return (int)sizeof(T) * 32 * lds_ld_tr<T>(HD); }
 template <typename T> constexpr int kLdT64 = lds_ld_tr<T>(kNB);              // of a tile of T' rows
 template <typename T> constexpr int t_tile_bytes() { return (int)sizeof(T) * 32 * kLdT64<T>; }
 template <typename T> constexpr int kLdX = 32 + 16 / (int)sizeof(T);   // leading dimension of a 32-column LDS tile
-template <int HD, int W> constexpr int reduce_bytes() { return W * narrow_nt<HD>() * 16 * 64 * 4; }
-constexpr int max2(int a, int b) { return a > b ? a : b; }
 // two waves per SIMD where the fragments of 16-bit operands leave room for it
 template <typename T, int HD> constexpr int narrow_waves() { return sizeof(T) == 2 && HD <= 64 ? 2 : 1; }
 template <typename T, int HD> __device__ __forceinline__ void narrow_item(int BH, int n, int cus, int& rank, int& bh) {

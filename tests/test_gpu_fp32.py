@@ -1,0 +1,82 @@
+"""fp32 tensors from 128 rows on run on pairs of fp16 numbers (csrc/castle_split.h): no less exact than fp32 sums, and in
+the range of fp32."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from oracle import castle_oracle as O
+
+DEV = "cuda:0"
+
+
+def H():
+    from lookahead_keys_attention_amd import ops
+
+    return ops
+
+
+def operands(B, Hh, L, d, seed, std=0.6):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, Hh, L, d, generator=g) * std for _ in range(6)], torch.randn(B, Hh, L, d, generator=g)
+
+
+def results(ops, dout, d):
+    leaves = [t.to(DEV).requires_grad_() for t in ops]
+    out, U = H().castle_attention_hip(*leaves, d ** -0.5, True)
+    out.backward(dout.to(DEV))
+    return [out.detach(), U] + [t.grad for t in leaves]
+
+
+def reference(ops, dout, d):
+    o64 = [t.double() for t in ops]
+    return list(O.parallel_core(*o64, d ** -0.5, want_U=True)) + list(O.closed_form_grads(*o64, d ** -0.5, dout.double()))
+
+
+def check(got, want, L):
+    # fp32 sums of L terms, through three contractions and an exponential: 4 sqrt(L) roundings of 2^-24 (measured: at most half of it)
+    for name, a, r in zip(("out", "U", "dqc", "dkc", "dvc", "dqu", "dku", "dvu"), got, want):
+        rel = ((a.cpu().double() - r).norm() / r.norm()).item()
+        assert rel <= 4 * L ** 0.5 * 2 ** -24, f"{name}: {rel:.2e}"
+
+
+@pytest.mark.parametrize("B,Hh,L,d", [(1, 2, 127, 64), (1, 2, 128, 64), (2, 2, 129, 32), (1, 3, 159, 16), (1, 2, 161, 64), (1, 1, 192, 64), (2, 1, 225, 32),
+                                      (1, 2, 257, 16), (1, 1, 511, 64), (1, 1, 1000, 64), (3, 45, 130, 32)])
+def test_results_at_tile_edges(B, Hh, L, d):
+    ops, dout = operands(B, Hh, L, d, seed=L + d)
+    check(results(ops, dout, d), reference(ops, dout, d), L)
+
+
+@pytest.mark.parametrize("flag", ["FLAG_RECOMPUTE_SCORES", "FLAG_RECOMPUTE_STATE"])
+def test_results_without_tiles_and_without_snapshots(flag, monkeypatch):
+    from lookahead_keys_attention_amd import _native
+
+    monkeypatch.setattr(H(), "DEFAULT_FLAGS", getattr(_native, flag))
+    ops, dout = operands(2, 2, 300, 64, seed=5)
+    check(results(ops, dout, 64), reference(ops, dout, 64), 300)
+
+
+def test_operands_of_any_magnitude():
+    """Heads, and tiles of 32 rows in a head, are scaled by themselves."""
+    ops, dout = operands(1, 3, 200, 64, seed=6)
+    size = torch.tensor([1e-8, 1.0, 1e8])[None, :, None, None]
+    ops[2] = ops[2] * size                                   # values
+    ops[0], ops[1] = ops[0] / size, ops[1] * size            # the scores stay
+    ops[4], ops[3] = ops[4] * size, ops[3] / size            # the gates stay
+    ops[5] = ops[5] * size                                   # the lookahead scores stay
+    dout = dout * torch.where(torch.arange(200) < 96, 1e-9, 1e3)[None, None, :, None]
+    got, want = results(ops, dout, 64), reference(ops, dout, 64)
+    for h in range(3):
+        check([t[:, h] for t in got], [t[:, h] for t in want], 200)
+    rows = slice(0, 96)   # their own gradient of the queries, not only beside that of the large rows
+    for h in range(3):
+        a, r = got[2][:, h, rows].cpu().double(), want[2][:, h, rows]
+        assert (a - r).norm() <= 4 * 200 ** 0.5 * 2 ** -24 * r.norm()
+
+
+@pytest.mark.parametrize("power", [-80, -30, 60])
+def test_gradients_are_linear_in_powers_of_two(power):
+    ops, dout = operands(1, 2, 200, 32, seed=7)
+    one, other = results(ops, dout, 32), results(ops, dout * 2.0 ** power, 32)
+    for a, b in zip(one[2:], other[2:]):
+        assert torch.equal(a * 2.0 ** power, b)
