@@ -71,6 +71,9 @@ extern "C" {
  * workgroups that had waited for them; with _GIVE_UP these leave instead, and what they were to do is NaN as described there. */
 #define CASTLE_FLAG_STEP_TAKE_OVER 128
 #define CASTLE_FLAG_STEP_GIVE_UP 256
+/* castle_fwd: no castle_bwd follows.  What lies in the workspace behind the status word and in the state is then undefined, and short sequences (up to
+ * 128 rows of 16-bit types, as long as there are few of them) take one launch. */
+#define CASTLE_FLAG_FORWARD_ONLY 512
 #define CASTLE_AMAX_PARTIALS 256
 #define CASTLE_AMAX_OFFSET 256
 
@@ -133,7 +136,7 @@ int64_t castle_fwd_state_bytes(int B, int H, int L, int d, int dtype);
  * written (any strides, e.g. those of a (B,L,H,d) buffer).  U: optional (NULL, or a view
  * with ptr == NULL, to skip) final lookahead keys for the decode cache
  * (lookahead_keys_attention.py:161-164).  d in {16,32,64,128}; fp32 needs d <= 64.
- * flags: any of CASTLE_FLAG_BF16_OPERANDS, CASTLE_FLAG_ROTARY, CASTLE_FLAG_U_HALF (format of U). */
+ * flags: any of CASTLE_FLAG_BF16_OPERANDS, CASTLE_FLAG_ROTARY, CASTLE_FLAG_U_HALF (format of U), CASTLE_FLAG_FORWARD_ONLY. */
 int castle_fwd(const castle_view4* qc, const castle_view4* kc, const castle_view4* vc,
                const castle_view4* qu, const castle_view4* ku, const castle_view4* vu,
                int B, int H, int L, int d, int dtype, float scale, int flags,

@@ -29,6 +29,7 @@ FLAG_U_HALF = 16            # bf16 caches: the lookahead-key buffer holds fp16 b
 FLAG_READ_ONCE = 32         # cached step: the loop it belongs to reads more than the last-level cache holds
 FLAG_STEP_TAKE_OVER = 128   # tests of a layer step in one launch: jobs in reverse order, taken over by those that wait for them
 FLAG_STEP_GIVE_UP = 256     # the same, given up instead
+FLAG_FORWARD_ONLY = 512     # forward pass: no backward pass will read what it leaves
 U_HALF_UNSCALE = 64.0
 
 EXPORTED_SYMBOLS = (

@@ -16,6 +16,7 @@
 namespace castle {
 int launch_fwd(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
+int launch_short(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_plain_state(const FwdArgs& a, hipStream_t stream);
 int launch_bwd(const BwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_decode(const DecodeArgs& a, int dtype, hipStream_t stream);
@@ -235,6 +236,10 @@ int castle_fwd(const castle_view4* qc, const castle_view4* kc, const castle_view
   a.u_half = (flags & CASTLE_FLAG_U_HALF) != 0;
   a.ws = carve(workspace, state, g);
   a.amax_ready = (flags & CASTLE_FLAG_AMAX_READY) != 0;
+  if (flags & CASTLE_FLAG_FORWARD_ONLY) {
+    rc = castle::launch_short(a, dtype, (flags & CASTLE_FLAG_BF16_OPERANDS) != 0, static_cast<hipStream_t>(stream));
+    if (rc != 1) return rc;
+  }
   return castle::launch_fwd(a, dtype, (flags & CASTLE_FLAG_BF16_OPERANDS) != 0, static_cast<hipStream_t>(stream));
 }
 

@@ -631,7 +631,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     }
     proj = proj.view({B, L, w_qkv.size(0)});
     const bool want_U = cache_rows > 0;
-    auto [merged, U, ws, state] = run_packed(proj, heads, scale, want_U, cache_rows, flags, want_graph && keep_state, prepared, into.empty() ? Tensor() : into[0]);
+    auto [merged, U, ws, state] = run_packed(proj, heads, scale, want_U, cache_rows, want_graph ? flags : flags | CASTLE_FLAG_FORWARD_ONLY, want_graph && keep_state, prepared, into.empty() ? Tensor() : into[0]);
     variable_list out{project(merged.view({B * L, merged.size(2)}), w_out).view({B, L, w_out.size(0)})};
     if (delta) out.push_back(n.sum.view({B, L, dim}));
     const size_t results = out.size();

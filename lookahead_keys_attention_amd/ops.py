@@ -192,7 +192,7 @@ def _check_range(ws):
 def castle_attention_hip(q, k, v, qu, ku, vu, scale, return_U_for_cache=False, rotary=False):
     """Drop-in for castle_attention_triton: returns out, or (out, U).  rotary=True applies the
     rotary position embedding (positions 0..L-1) to q, k, qu, ku, vu inside the kernels."""
-    flags = DEFAULT_FLAGS | (N.FLAG_ROTARY if rotary else 0)
+    flags = DEFAULT_FLAGS | (N.FLAG_ROTARY if rotary else 0) | (0 if torch.is_grad_enabled() else N.FLAG_FORWARD_ONLY)
     B, H, L, d = q.shape
     _check_dims(d, q.dtype)
     if N._host is None:
@@ -210,7 +210,8 @@ def castle_attention_packed(proj, heads, scale, return_U_for_cache=False, row_ca
     (reachable as U._base), which a decode cache can adopt as its U buffer without a copy.
     `u_half` (bf16 only): U comes back in the half-precision cache format (`decode_lookahead_keys`
     reads it), the format the cached step then keeps it in."""
-    flags = DEFAULT_FLAGS | (N.FLAG_ROTARY if rotary else 0) | (N.FLAG_U_HALF if u_half and return_U_for_cache else 0)
+    flags = (DEFAULT_FLAGS | (N.FLAG_ROTARY if rotary else 0) | (N.FLAG_U_HALF if u_half and return_U_for_cache else 0) |
+             (0 if torch.is_grad_enabled() else N.FLAG_FORWARD_ONLY))
     B, L, width = proj.shape
     _check_dims(width // (6 * int(heads)), proj.dtype)
     if N._host is None:
