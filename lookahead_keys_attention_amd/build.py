@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libcastle_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ("castle_fwd.hip", "castle_bwd.hip", "castle_narrow.hip", "castle_narrow32.hip", "castle_short.hip", "castle_decode.hip", "castle_rows.hip", "castle_gemm.hip", "castle_profile.hip", "castle_abi.hip")
+SOURCES = ("castle_fwd.hip", "castle_bwd.hip", "castle_narrow.hip", "castle_narrow32.hip", "castle_short.hip", "castle_decode.hip", "castle_rows.hip", "castle_gemm.hip", "castle_gemm32.hip", "castle_profile.hip", "castle_abi.hip")
 HOST_SOURCE = "castle_host.cpp"
 HOST_NAME = "_castle_host.so"
 ARCH = "gfx950"

@@ -31,6 +31,8 @@ bool gemm_norm_ok(int M, int N, int K, int elem_size);
 bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to);
 void gemm_plan(int M, int N, int K, int elem_size, bool epilogue, int (&out)[4]);
 int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue);
+// fp32, castle_gemm32.hip
+int launch_gemm32(const GemmArgs& a, bool a_kc, bool b_kc, int tile, int splits, int waves, hipStream_t stream);
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream);
 
 }  // namespace castle

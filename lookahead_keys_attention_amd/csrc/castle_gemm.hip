@@ -15,38 +15,14 @@
 #include "castle_tiles.h"
 #include "castle_dispatch.h"
 #include "castle_gemm.h"
+#include "castle_gelu.h"
+#include "castle_waves.h"
 #include <algorithm>
+#include <cmath>
 #include "castle_rows.h"
 
 namespace castle {
 namespace {
-
-// Phi(x) = erfc(-x / sqrt 2) / 2.  For 16-bit outputs from the Chebyshev fit of Numerical Recipes (erfcc, fractional error
-// below 1.2e-7 everywhere); the library's erff takes three times the instructions, which a store of 16384 x 2048 felt
-// with 8 us.
-template <typename T> __device__ __forceinline__ float normal_cdf(float x) {
-  if constexpr (sizeof(T) == 4) {
-    return 0.5f * (1.f + erff(x * 0.70710678f));
-  } else {
-    const float z = fabsf(x) * 0.70710678f, t = fast_rcp(__builtin_fmaf(0.5f, z, 1.f));
-    float p = 0.17087277f;
-    p = __builtin_fmaf(p, t, -0.82215223f);
-    p = __builtin_fmaf(p, t, 1.48851587f);
-    p = __builtin_fmaf(p, t, -1.13520398f);
-    p = __builtin_fmaf(p, t, 0.27886807f);
-    p = __builtin_fmaf(p, t, -0.18628806f);
-    p = __builtin_fmaf(p, t, 0.09678418f);
-    p = __builtin_fmaf(p, t, 0.37409196f);
-    p = __builtin_fmaf(p, t, 1.00002368f);
-    p = __builtin_fmaf(p, t, -1.26551223f);
-    const float e = 0.5f * t * fast_exp2(kLog2e * (p - z * z));
-    return x < 0.f ? e : 1.f - e;
-  }
-}
-template <typename T> __device__ __forceinline__ float gelu(float x) { return x * normal_cdf<T>(x); }
-template <typename T> __device__ __forceinline__ float gelu_slope(float x) {
-  return normal_cdf<T>(x) + x * 0.3989422804f * fast_exp2(-0.5f * kLog2e * x * x);
-}
 
 // A tile of FREE rows / columns and BK steps of the contraction: global -> registers -> LDS -> operand fragments.
 // KC: the operand is contraction-contiguous (LDS [FREE][BK]), else stored [contraction][free] (LDS [BK][FREE]).
@@ -351,11 +327,6 @@ template <int BN> struct Wide {
   static constexpr bool kOwnTurn = BN == 256;
   static constexpr int kLds = kStages * kStage + (kOwnTurn ? 4096 * kWideThreads / 64 : 4 * kWideThreads / 64);   // and a maximum of each wave
 };
-
-// the compiler waits for every load in flight at each read of LDS if it knows of loads into it: it is not told
-__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory", "m0");
-}
 template <typename T, bool KC, int FREE> struct WideOperand {
   static constexpr int N = FREE / 64;   // loads of a wave
   const T* at;
@@ -609,16 +580,18 @@ template <typename T, bool AK, bool BKC, int BN, bool FUSED> __global__ __launch
 
 // Tile, number of ranges of the contraction and groups of a workgroup, from what a launch takes (us): a start (2.3 for tiles of 64 and 128 rows, where
 // gelu or its derivative rides on the store within the end of a tile), and for each tile of the fullest CU so much a step and at its end, more at the end where
-// gelu or its derivative rides on the store.  A second group takes a step of a workgroup of 64 x 64 that has a CU to itself from 0.42 to 0.36, fp32 from 0.78 to
-// 0.66, for 0.3 at the end, and pays from eight steps on, fp32 four (3000 rows of 1536 -> 256 12.7 with one, 9.9 with two, 1504 rows of 256 -> 512 5.3 and 6.1; 256
-// rows of fp32 512 -> 3072 15.1 and 13.1); at two workgroups a CU it gains where the contraction is long (3000 rows of 3072 -> 512 29 / 26, of 512 -> 512
+// gelu or its derivative rides on the store.  A second group takes a step of a workgroup of 64 x 64 that has a CU to itself from 0.42 to 0.36,
+// for 0.3 at the end, and pays from eight steps on (3000 rows of 1536 -> 256 12.7 with one, 9.9 with two, 1504 rows of 256 -> 512 5.3 and 6.1);
+// at two workgroups a CU it gains where the contraction is long (3000 rows of 3072 -> 512 29 / 26, of 512 -> 512
 // level), behind from three on.  A split adds a second launch, 2.5, and its partial results, written and read, and tiles of 256 rows another start.
 // Weight gradient of 3000 rows, 1536 x 256 out: 22.6 in one range, 13.7 in two of two groups; 3008 rows 512 -> 2048 17.6 on 64 x 64, 16.6 on 128 x 128, 14.2 on
 // 256 x 128; 4096 rows 512 -> 3072 31.8, 26.2, 24.9 and 21.8 on 256 x 256; 8184 rows 64 -> 4096 20.0, 18.6, 15.8 and 15.3.  Over 2500 products of 96 ... 65536
 // rows, outputs of 64 ... 4096 columns and contractions of 64 ... 8184, in all layouts, each timed with every tile and up to 16 ranges, what this picks takes 1.5 %
 // more than the best of them on average.
+constexpr int kStep16 = 64;   // contraction steps in LDS
 struct Plan {
-  int tile, splits, groups;   // tile: 64, 128, or columns of a tile of 256 rows + 256
+  int tile, splits, groups;   // tile: 32 (fp32), 64, 128, or columns of a tile of 256 rows + 256; groups: of four waves
+  int waves = 0;   // fp32
   int rows() const { return std::min(tile, kWideM); }
   int columns() const { return tile > kWideM ? tile - kWideM : tile; }
   int tiles(int M, int N) const { return ((M + rows() - 1) / rows()) * ((N + columns() - 1) / columns()); }
@@ -626,7 +599,44 @@ struct Plan {
 // workgroups of the fullest CU: tiles go to eight XCDs of 32 CUs each, so one of them may have work for 33 (weight gradient of 8184 rows, 640 x 320: 50 tiles in
 // five ranges 21.6 us, in four 16.9)
 int64_t on_a_cu(int64_t tiles, int splits) { return ((tiles + 7) / 8 * splits + 31) / 32; }
+// fp32 (castle_gemm32.hip): tiles of 64 x 64 by one, two or four waves and of 32 x 32 by four or eight, `held` workgroups to a CU at once.  From what a launch takes (us): a
+// start, and for the workgroups of the fullest CU, so many at a time, so much for a wave's 32 steps and at the end (one by itself, and all of them); or so much for a MB that
+// the tiles read, and between the two where they are level; a split adds the sum of its ranges.  Fitted to 190000 timings of 9358 products of 16 ... 23000 rows, outputs of
+// 32 ... 4096 columns and contractions of 16 ... 23000, in all layouts.  What it picks takes 2 % more than the best of them on average, 8 % in one of ten, and 0.74 of what the
+// library takes, 1.02 in one of ten.
+Plan plan32(int M, int N, int K, bool plain) {
+  struct Kind { int tile, waves, held; float start, step, end, steps, ends, split, split_mb, read; };
+  constexpr Kind kinds[5] = {{64, 1, 8, 6.03f, 1.47f, 0.219f, 1.63f, 6.29f, 1.65f, 0.201f, 0.101f},
+                             {64, 2, 4, 4.28f, 1.51f, 1.62f, 3.33f, 3.03f, 1.72f, 0.218f, 0},
+                             {64, 4, 2, 4.07f, 1.61f, 1.58f, 2.51f, 2.33f, 1.93f, 0.213f, 0.097f},
+                             {32, 8, 2, 4.22f, 0.99f, 0, 1.61f, 0.304f, 2.03f, 0.25f, 0.078f},
+                             {32, 4, 4, 4.15f, 0.752f, 0.047f, 1.52f, 0.771f, 2.06f, 0.209f, 0.071f}};
+  Plan best = {64, 1, 1, 4};
+  float best_cost = 1e30f;
+  const auto tiles_of = [&](int tile) { return (int)std::min<int64_t>((int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile), 1 << 26); };
+  const int tiles64 = tiles_of(64), tiles32 = tiles_of(32);
+  const float mb = 8e-6f * M * N;
+  for (const int s : {1, 2, 3, 4, 6, 8, 12, 16}) {   // (a call looks at all this three times: no divisions and roots that can be spared)
+    if (s > 1 && (!plain || s > (K + 31) / 32 || tiles64 * s > 1024)) break;
+    const int stages = ((K + s - 1) / s + 31) / 32;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const Kind& kind = kinds[k];
+      const int tiles = kind.tile == 64 ? tiles64 : tiles32, per_cu = (int)on_a_cu(tiles, s), rounds = (stages + kind.waves - 1) / kind.waves;
+      const int rest = per_cu % kind.held;
+      const float full = rest > 1 ? (rest - 1.f) / (kind.held - 1) : 0.f;   // of the way from one by itself to all of them
+      float work = per_cu / kind.held * (rounds * kind.steps + kind.ends);
+      if (rest > 0) work += rounds * (kind.step + full * (kind.steps - kind.step)) + kind.end + full * (kind.ends - kind.end);
+      const float fixed = kind.start + (s > 1 ? kind.split + s * mb * kind.split_mb : 0.f);
+      if (fixed + work >= best_cost) continue;
+      const float read = 8e-6f * tiles * K * kind.tile * kind.read, w2 = work * work, r2 = read * read, cost = fixed + std::sqrt(std::sqrt(w2 * w2 + r2 * r2));
+      if (cost < best_cost) { best_cost = cost; best = {kind.tile, s, std::max(1, kind.waves / 4), kind.waves}; }
+    }
+  }
+  return best;
+}
 Plan plan(int M, int N, int K, bool plain, int elem_size) {
+  if (elem_size == 4) return plan32(M, N, K, plain);
   Plan best = {64, 1, 1};
   double best_cost = 1e30;
   auto take = [&](double cost, const Plan& p) {
@@ -635,21 +645,21 @@ Plan plan(int M, int N, int K, bool plain, int elem_size) {
   // Two tensors that no cache holds: stores of single lines cost more (gelu of 65536 rows 64 -> 1536 on 64 x 64 123, on 256 x 256 94), and 256 x 256 where rows do not
   // start with lines (33000 rows 64 -> 3064 192, 256 x 128 103, 64 x 64 150).
   const bool far = !plain && 4.0 * M * N > 2.5e8;
-  for (int tile = 64; tile <= (elem_size == 2 ? 128 : 64); tile += 64) {
-    const double alone = elem_size == 4 ? 0.78 : tile == 64 ? 0.42 : 0.85, shared = elem_size == 4 ? 0.62 : tile == 64 ? 0.29 : 0.6;
+  for (int tile = 64; tile <= 128; tile += 64) {
+    const double alone = tile == 64 ? 0.42 : 0.85, shared = tile == 64 ? 0.29 : 0.6;
     const double fused = plain ? 0 : tile == 128 ? 2.6 : far ? 1 : 0.5;
     const int64_t tiles = (int64_t)((M + tile - 1) / tile) * ((N + tile - 1) / tile);
-    const int steps = (K * elem_size + 127) / 128;   // 128 bytes of the contraction a step
+    const int steps = (K + kStep16 - 1) / kStep16;
     for (int s = 1; s <= (plain ? std::min(16, (steps + 1) / 2) : 1); ++s) {
       const int64_t per_cu = on_a_cu(tiles, s), n = (steps + s - 1) / s;
-      const double end = elem_size == 4 ? 0 : tile == 64 ? 0.25 : s > 1 ? 1 : 2.3;   // (partial results do not go through LDS)
-      const int groups = tile == 64 && (per_cu == 1 ? n >= (elem_size == 4 ? 4 : 8) : elem_size == 2 && s == 1 && per_cu == 2 && n >= 12) ? 2 : 1;
-      double cost = groups == 2 ? 0.3 + n * (elem_size == 4 ? 0.66 : per_cu == 1 ? 0.36 : 0.55) : per_cu == 1 ? n * alone + end : per_cu * (n * shared + end);
+      const double end = tile == 64 ? 0.25 : s > 1 ? 1 : 2.3;   // (partial results do not go through LDS)
+      const int groups = tile == 64 && (per_cu == 1 ? n >= 8 : s == 1 && per_cu == 2 && n >= 12) ? 2 : 1;
+      double cost = groups == 2 ? 0.3 + n * (per_cu == 1 ? 0.36 : 0.55) : per_cu == 1 ? n * alone + end : per_cu * (n * shared + end);
       if (s > 1) cost += 2.5 + (double)s * M * N * 8 / 4e6;
       take((plain ? 2.3 : 0) + cost + (per_cu == 1 ? 2 : per_cu) * fused, {tile, s, groups});
     }
   }
-  if (elem_size == 2 && K % kWideK == 0) {
+  if (K % kWideK == 0) {
     for (int columns = 128; columns <= 256; columns += 128) {
       const double start = plain ? 3.5 : columns == 128 ? 1.6 : 2.6, end = columns == 128 ? (plain ? 1.8 : 8.8) : plain ? 4 : far && N % 64 != 0 ? 24.5 : 16.5;
       const int64_t tiles = (int64_t)((M + kWideM - 1) / kWideM) * ((N + columns - 1) / columns);
@@ -663,8 +673,6 @@ Plan plan(int M, int N, int K, bool plain, int elem_size) {
   }
   return best;
 }
-constexpr int kStep16 = 64, kStep32 = 32;   // contraction steps in LDS, 16-bit and fp32
-
 template <typename T, bool AK, bool BKC, int BN, bool FUSED> int launch_wide(const GemmArgs& a, const Plan& p, hipStream_t stream) {
   static PerDeviceOnce once;
   bool& configured = once.flag();
@@ -677,20 +685,18 @@ template <typename T, bool AK, bool BKC, int BN, bool FUSED> int launch_wide(con
 }
 
 template <typename T, bool AK, bool BKC> int launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
-  constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
+  constexpr int BK = kStep16;
   const int tiles = p.tiles(a.M, a.N);
   // at most what the CUs hold at once: two workgroups of 128 x 128 tiles or four of 64 x 64
   const dim3 grid(std::min((tiles + 7) / 8 * 8, p.tile == 128 ? 512 : 1024), p.splits);
-  if constexpr (sizeof(T) == 2) {
-    if (p.tile > kWideM) {
-      const bool plain = a.epilogue == kGemmPlain;
-      if (p.columns() == 128) return plain ? launch_wide<T, AK, BKC, 128, false>(a, p, stream) : launch_wide<T, AK, BKC, 128, true>(a, p, stream);
-      return plain ? launch_wide<T, AK, BKC, 256, false>(a, p, stream) : launch_wide<T, AK, BKC, 256, true>(a, p, stream);
-    }
-    if (p.tile == 128) {
-      hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK, 1>), grid, dim3(kThreads), 0, stream, a);
-      return hipGetLastError() == hipSuccess ? 0 : -3;
-    }
+  if (p.tile > kWideM) {
+    const bool plain = a.epilogue == kGemmPlain;
+    if (p.columns() == 128) return plain ? launch_wide<T, AK, BKC, 128, false>(a, p, stream) : launch_wide<T, AK, BKC, 128, true>(a, p, stream);
+    return plain ? launch_wide<T, AK, BKC, 256, false>(a, p, stream) : launch_wide<T, AK, BKC, 256, true>(a, p, stream);
+  }
+  if (p.tile == 128) {
+    hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 128, 128, BK, 1>), grid, dim3(kThreads), 0, stream, a);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
   }
   // (both operands contraction-strided at two workgroups a CU: one group, weight gradients of 1000 rows 512 x 3072 13.2 us and with two 14.2, of 3000 30.4 / 32.1)
   if (p.groups == 2 && (AK || on_a_cu(tiles, p.splits) == 1)) hipLaunchKernelGGL((gemm_kernel<T, AK, BKC, 64, 64, BK, 2>), grid, dim3(2 * kThreads), 0, stream, a);
@@ -717,27 +723,26 @@ bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to
   return p.splits == 1 && (int64_t)((M + p.rows() - 1) / p.rows()) * per_row <= kAmaxBlocks;
 }
 
-// One tile per workgroup and a CU for each, so that a row is read for its factor where it costs nothing else; tile and groups of the product
+// One tile per workgroup and a CU for each (or for four of 32 rows), so that a row is read for its factor where it costs nothing else; tile and groups of the product
 // by itself, for the same bits.
 bool gemm_norm_ok(int M, int N, int K, int elem_size) {
   if ((int64_t)K * elem_size > kNormBytes) return false;
   const Plan p = plan(M, N, K, true, elem_size);
-  return p.tile == 64 && p.splits == 1 && p.tiles(M, N) <= 256;
+  return p.tile <= 64 && p.splits == 1 && p.tiles(M, N) * p.tile * p.tile <= 256 * 64 * 64 && (elem_size == 2 || p.waves >= 4);
 }
 
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream) {
-  const int es = dtype == 0 ? 4 : 2, step = dtype == 0 ? kStep32 : kStep16;
+  const int es = dtype == 0 ? 4 : 2, step = dtype == 0 ? 32 : kStep16;
   Plan p = plan(a.M, a.N, a.K, a.epilogue == kGemmPlain || a.amax != nullptr, es);   // (the slots of the maxima follow from the plain plan)
   a.k_per_split = ((a.K + p.splits - 1) / p.splits + step - 1) / step * step;
   p.splits = (a.K + a.k_per_split - 1) / a.k_per_split;   // rounding up may leave the last ones empty
   a.part = p.splits > 1 ? workspace : nullptr;
-  const int rc = by_type(dtype, true, [&](auto t, auto) {
+  const int rc = dtype == 0 ? launch_gemm32(a, a_kc, b_kc, p.tile, p.splits, p.waves, stream) : by_type16(dtype, true, [&](auto t, auto) {
     using T = decltype(t);
     if (a.norm_w != nullptr) {
-      constexpr int BK = sizeof(T) == 2 ? kStep16 : kStep32;
       const dim3 grid((p.tiles(a.M, a.N) + 7) / 8 * 8);
-      if (p.groups == 2) hipLaunchKernelGGL((gemm_kernel<T, true, true, 64, 64, BK, 2, true>), grid, dim3(2 * kThreads), 0, stream, a);
-      else hipLaunchKernelGGL((gemm_kernel<T, true, true, 64, 64, BK, 1, true>), grid, dim3(kThreads), 0, stream, a);
+      if (p.groups == 2) hipLaunchKernelGGL((gemm_kernel<T, true, true, 64, 64, kStep16, 2, true>), grid, dim3(2 * kThreads), 0, stream, a);
+      else hipLaunchKernelGGL((gemm_kernel<T, true, true, 64, 64, kStep16, 1, true>), grid, dim3(kThreads), 0, stream, a);
       return hipGetLastError() == hipSuccess ? 0 : -3;
     }
     if (a_kc && b_kc) return launch_t<T, true, true>(a, p, stream);

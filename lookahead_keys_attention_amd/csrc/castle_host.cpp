@@ -469,15 +469,15 @@ Tensor product(const Tensor& a, bool a_t, const Tensor& b, bool b_t, int64_t epi
 // 24 / 30, 128 -> 3072 30 / 32 and 31 / 35, 256 -> 3072 38 / 43 and 38 / 45, 512 -> 3072 59 / 62 and 59 / 67, 512 -> 512 14 / 20 and 14 / 20; 65536 rows 64 -> 3072 81 /
 // 100 and 82 / 105, 128 -> 3072 103 / 126 and 105 / 129, 512 -> 3072 227 / 240 and 228 / 253; 98304 rows 354 / 359 and 361 / 379, 131072 rows 478 / 473 and 484 /
 // 500).  Longer ones are level at 16384 rows (forward 576 -> 3072 64 / 59, 640 68 / 64, 768 76 / 72).
-// In fp32 they are level up to the size below (256 rows, 512 <-> 3072: forward 13 / 13, input gradient 16 / 12,
-// weight gradient 15 / 16), where a layer's time is the host's; 2048 rows 60 / 53, 64 / 49, 72 / 55.
-bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16, double most_32) {
-  return 2.0 * rows * n * k <= (a.scalar_type() == at::kFloat ? most_32 : most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
+// In fp32 they are ahead at nearly every size, up to the largest that was timed, 825 GFLOP (us, own / library: 16384 rows 2048 -> 12288 forward 4950 / 5530, input
+// gradient 4840 / 5350, weight gradient 4820 / 5360; 256 rows 512 -> 3072 11 / 13, 15 / 13 and 11 / 17).
+bool own_product(const Tensor& a, const Tensor& b, int64_t rows, int64_t n, int64_t k, double most_16) {
+  return (a.scalar_type() == at::kFloat || 2.0 * rows * n * k <= most_16) && n % 8 == 0 && k % 8 == 0 && product_rows(a) && product_rows(b);
 }
 bool own_contraction(int64_t k) { return k <= 512 && k % 64 == 0; }   // (others have no tiles of 256 rows)
 double own_forward(int64_t k) { return own_contraction(k) ? 260e9 : 14e9; }
 double own_input_grad(int64_t k) { return own_contraction(k) ? 260e9 : 4e9; }
-constexpr double kOwnWeightGrad = 40e9, kOwn32 = 1e9;
+constexpr double kOwnWeightGrad = 40e9;
 constexpr double kOwnGeluSlope = 40e9;   // the pass it saves over the hidden rows outweighs a slower product: 16384 x 512 x 2048 73 / 91
 
 // The attention kernels behind a product begin with the largest element of some of its columns (vu of a fused projection, all
@@ -498,7 +498,7 @@ Maxima maxima(const Tensor& like, int64_t rows, int64_t n, int64_t k, int64_t co
 }
 
 Tensor project(const Tensor& x, const Tensor& w) {   // (R, K), (N, K) -> (R, N)
-  if (own_product(x, w, x.size(0), w.size(0), x.size(1), own_forward(x.size(1)), kOwn32)) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
+  if (own_product(x, w, x.size(0), w.size(0), x.size(1), own_forward(x.size(1)))) return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(x, w.t());
 }
 // the fused projection, with the maxima of its vu part
@@ -507,7 +507,7 @@ Maxima packed_maxima(const Tensor& x, const Tensor& w, const Shape& s) {
   return maxima(x, x.size(0), w.size(0), x.size(1), 2 * part, part, check(castle_fwd_workspace_bytes(s.B, s.H, s.L, s.d, s.dtype), "castle_fwd_workspace_bytes"), true);
 }
 Tensor project_packed(const Tensor& x, const Tensor& w, const Shape& s, Tensor& prepared) {
-  if (!own_product(x, w, x.size(0), w.size(0), x.size(1), own_forward(x.size(1)), kOwn32)) return at::mm(x, w.t());
+  if (!own_product(x, w, x.size(0), w.size(0), x.size(1), own_forward(x.size(1)))) return at::mm(x, w.t());
   const Maxima m = packed_maxima(x, w, s);
   prepared = m.prepared;
   return product(x, false, w, false, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
@@ -517,7 +517,7 @@ bool norm_in_product(const Tensor& x, const Tensor& norm_w, const Tensor& w) {
   const int64_t R = x.size(0), D = x.size(1);
   return norm_w.defined() && norm_w.numel() == D && norm_w.is_contiguous() && norm_w.device() == x.device() && norm_w.scalar_type() == x.scalar_type() &&
          x.is_contiguous() && w.size(1) == D && w.device() == x.device() && w.scalar_type() == x.scalar_type() && castle_rms_norm_bwd_workspace_bytes(R, (int)D, dtype_code(x)) >= 0 &&
-         own_product(x, w, R, w.size(0), D, own_forward(D), kOwn32) && castle_gemm_norm_ok((int)R, (int)w.size(0), (int)D, dtype_code(x));
+         own_product(x, w, R, w.size(0), D, own_forward(D)) && castle_gemm_norm_ok((int)R, (int)w.size(0), (int)D, dtype_code(x));
 }
 // the same behind the norm; n.h and n.rstd are left where something will read them
 Tensor project_packed_of_norm(const Tensor& x, const Tensor& norm_w, std::optional<double> eps, const Tensor& w, const Shape& s, bool keep, Normed& n, Tensor& prepared) {
@@ -532,7 +532,7 @@ Tensor project_packed_of_norm(const Tensor& x, const Tensor& norm_w, std::option
   return c;
 }
 Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R, K)
-  if (own_product(dy, w, dy.size(0), w.size(0), w.size(1), own_input_grad(w.size(0)), kOwn32)) return product(dy, false, w, true, CASTLE_GEMM_PLAIN, std::nullopt);
+  if (own_product(dy, w, dy.size(0), w.size(0), w.size(1), own_input_grad(w.size(0)))) return product(dy, false, w, true, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(dy, w);
 }
 
@@ -557,7 +557,7 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (
           "castle_sum_parts");
     return dw;
   }
-  if (own_product(dy, x, rows, N, K, kOwnWeightGrad, kOwn32)) return product(dy, true, x, true, CASTLE_GEMM_PLAIN, std::nullopt);
+  if (own_product(dy, x, rows, N, K, kOwnWeightGrad)) return product(dy, true, x, true, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(dy.t(), x);
 }
 
@@ -692,7 +692,7 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
     const int64_t flags = ctx->saved_data["flags"].toInt();
     Tensor dmerged, prepared;
-    if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)), kOwn32)) {
+    if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)))) {
       const Maxima m = maxima(dy, B * L, w_out.size(1), w_out.size(0), 0, w_out.size(1), bwd_workspace_bytes(shape, flags, state), false);
       prepared = m.prepared;
       dmerged = product(dy, false, w_out, true, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
@@ -750,7 +750,7 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const int64_t R = x.numel() / x.size(-1);
     const Normed n = norm_rows(x.reshape({R, x.size(-1)}), delta.reshape({R, x.size(-1)}), norm_w, eps, want_graph);
     Tensor up, act;
-    if (own_product(n.h, w_up, R, w_up.size(0), w_up.size(1), own_forward(w_up.size(1)), kOwn32)) {   // GELU on the way out
+    if (own_product(n.h, w_up, R, w_up.size(0), w_up.size(1), own_forward(w_up.size(1)))) {   // GELU on the way out
       act = at::empty({R, w_up.size(0)}, n.h.options());
       up = product(n.h, false, w_up, false, CASTLE_GEMM_GELU, act);
     } else {
@@ -781,7 +781,7 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const Tensor dy = g[0].reshape({R, dim});
     if (ctx->needs_input_grad(4)) grads[4] = weight_grad(dy, act);
     if (!need_x && !need_norm && !need_up) return grads;
-    const Tensor dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnGeluSlope, kOwn32)
+    const Tensor dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnGeluSlope)
                            ? product(dy, false, w_down, true, CASTLE_GEMM_GELU_SLOPE, up)
                            : at::gelu_backward(at::mm(dy, w_down), up);
     if (need_up) grads[3] = weight_grad(dup, h);

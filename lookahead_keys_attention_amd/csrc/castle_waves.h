@@ -11,6 +11,10 @@ __device__ __forceinline__ void settle() {
   asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
+// the compiler waits for every load in flight at each read of LDS if it knows of loads into it: it is not told
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory", "m0");
+}
 // LDS traffic of one wave is in order; this keeps the compiler from moving it (and, where registers are short, from
 // requesting operands of the next stage early)
 template <bool STAGES = false> __device__ __forceinline__ void wave_lds_order() {
