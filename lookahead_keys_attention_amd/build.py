@@ -28,6 +28,11 @@ HIPCC_FLAGS = (
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 )
+# Kernels of one wave per SIMD have 256 accumulation registers beside the vector registers, and the compiler then lets every matrix
+# instruction write there, which costs a copy for each register that a vector instruction reads (a quarter of what the fp32 backward
+# kernels issued).  With this the results lie in vector registers and the other file takes what does not fit.
+VECTOR_RESULTS = ("-mllvm", "-amdgpu-mfma-vgpr-form=1")
+SOURCE_FLAGS = {"castle_narrow32.hip": VECTOR_RESULTS}
 
 
 def _hipcc() -> str:
@@ -64,7 +69,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
 
     def compile_one(src):
         obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        cmd = _host_compiler() if src == HOST_SOURCE else [hipcc, *HIPCC_FLAGS]
+        cmd = _host_compiler() if src == HOST_SOURCE else [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, ())]
         cmd = [*cmd, "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
