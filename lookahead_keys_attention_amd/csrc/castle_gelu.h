@@ -4,31 +4,36 @@
 
 namespace castle {
 
-// Phi(x) = erfc(-x / sqrt 2) / 2.  For 16-bit outputs from the Chebyshev fit of Numerical Recipes (erfcc, fractional error
-// below 1.2e-7 everywhere); the library's erff takes three times the instructions, which a store of 16384 x 2048 felt
-// with 8 us.
-template <typename T> __device__ __forceinline__ float normal_cdf(float x) {
-  if constexpr (sizeof(T) == 4) {
-    return 0.5f * (1.f + erff(x * 0.70710678f));
-  } else {
-    const float z = fabsf(x) * 0.70710678f, t = fast_rcp(__builtin_fmaf(0.5f, z, 1.f));
-    float p = 0.17087277f;
-    p = __builtin_fmaf(p, t, -0.82215223f);
-    p = __builtin_fmaf(p, t, 1.48851587f);
-    p = __builtin_fmaf(p, t, -1.13520398f);
-    p = __builtin_fmaf(p, t, 0.27886807f);
-    p = __builtin_fmaf(p, t, -0.18628806f);
-    p = __builtin_fmaf(p, t, 0.09678418f);
-    p = __builtin_fmaf(p, t, 0.37409196f);
-    p = __builtin_fmaf(p, t, 1.00002368f);
-    p = __builtin_fmaf(p, t, -1.26551223f);
-    const float e = 0.5f * t * fast_exp2(kLog2e * (p - z * z));
-    return x < 0.f ? e : 1.f - e;
+// Phi(-|x|) = t P(t) e, e = exp(-x^2 / 2), t = 1 / (1 + 0.305 |x|): P of the least largest fractional error for x in [0, 14], 7e-8 (a linear programme over 1800
+// points).  In fp32 within 5e-7 of Phi(-|x|) for |x| < 1, 3e-6 for |x| < 6, where the rounding of the exponent counts.  The library's erff takes three times the
+// instructions; with erfc as one exponential of a polynomial of degree 9 (Numerical Recipes' erfcc), a quarter more, and a second exponential for the slope:
+// products 16384 x 512 x 2048 with gelu on the store 71.8 -> 70.8 us, 16384 x 512 x 2048 with its slope 78.5 -> 75.0.
+template <typename T> struct Normal {
+  float cdf, e;   // Phi(x), exp(-x^2 / 2)
+  __device__ __forceinline__ explicit Normal(float x) {
+    const float w = 0.84932180f * x;
+    e = fast_exp2(-(w * w));
+    if constexpr (sizeof(T) == 4) {
+      cdf = 0.5f * (1.f + erff(x * 0.70710678f));
+    } else {
+      const float t = fast_rcp(__builtin_fmaf(0.305f, fabsf(x), 1.f));
+      float p = 0.0366340401f;
+      p = __builtin_fmaf(p, t, -0.152722267f);
+      p = __builtin_fmaf(p, t, 0.18528098f);
+      p = __builtin_fmaf(p, t, -0.0376090017f);
+      p = __builtin_fmaf(p, t, 0.12085099f);
+      p = __builtin_fmaf(p, t, 0.103463876f);
+      p = __builtin_fmaf(p, t, 0.122461473f);
+      p = __builtin_fmaf(p, t, 0.121639976f);
+      const float tail = p * t * e;
+      cdf = x < 0.f ? tail : 1.f - tail;
+    }
   }
-}
-template <typename T> __device__ __forceinline__ float gelu(float x) { return x * normal_cdf<T>(x); }
+};
+template <typename T> __device__ __forceinline__ float gelu(float x) { return x * Normal<T>(x).cdf; }
 template <typename T> __device__ __forceinline__ float gelu_slope(float x) {
-  return normal_cdf<T>(x) + x * 0.3989422804f * fast_exp2(-0.5f * kLog2e * x * x);
+  const Normal<T> n(x);
+  return __builtin_fmaf(x * 0.3989422804f, n.e, n.cdf);
 }
 
 }  // namespace castle
