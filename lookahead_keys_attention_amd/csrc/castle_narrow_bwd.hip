@@ -55,14 +55,14 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
     f.store(s_qu + t * 32 * LD, t == 0 ? -c1 : 1.f);
   }
   const int seg = (nblk - Iw + W - 1) / W;
+  // both gates of a block side by side, so that one chain of products fills the wait for the other (key pass of 16 heads x 1000 rows, d = 64: 41.5 -> 39.3 us);
+  // at d = 128, one wave to a SIMD, without room for a second tile of sources on its way, 3 % slower; fp32 was not tried
+  constexpr bool PAIRED = sizeof(T) == 2 && HD <= 64;
   const int lo = min(nblk, Iw + wave * seg), hi = min(nblk, lo + seg);
   // Edges need no branches: rows beyond the sequence are zero and have lse = inf, sources and queries in front of
   // the keys are masked; such tiles give zeros (and the tile arrays have room for them).
-  // gate A^T[j rows, k lanes] of source tile jt, whose Ku rows are in s_a
-  auto gate = [&](acc_t& aT, int jt) __attribute__((always_inline)) {
-    zero(aT);
-#pragma unroll
-    for (int s = 0; s < KS; ++s) mma(aT, ld_nat<T>(s_a, LD, c, 16 * s + 8 * g), ld_nat<T>(s_qu, LD, c, 16 * s + 8 * g));
+  // gate A^T[j rows, k lanes] of source tile jt from the product of its Ku rows
+  auto gate_of = [&](acc_t& aT, int jt) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) aT[r] = fast_rcp(1.f + fast_exp2(aT[r]));
     if (jt <= kt) {   // j > k only
@@ -70,6 +70,12 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
       for (int r = 0; r < 16; ++r)
         if (32 * (jt - kt) + acc_row(r, g) <= c) aT[r] = 0.f;
     }
+  };
+  auto gate = [&](acc_t& aT, int jt) __attribute__((always_inline)) {   // whose Ku rows are in s_a
+    zero(aT);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) mma(aT, ld_nat<T>(s_a, LD, c, 16 * s + 8 * g), ld_nat<T>(s_qu, LD, c, 16 * s + 8 * g));
+    gate_of(aT, jt);
   };
   // the next tiles, requested one step ahead
   Flat32<T, HD, SB> pa, pb;
@@ -92,6 +98,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
     };
     if (lo < hi) {
       pa.load(ku + (int64_t)lo * kNB * HD);
+      if (PAIRED) pb.load(ku + ((int64_t)lo * kNB + 32) * HD);
       sums(lo);
     }
     __syncthreads();   // the shared rows are there
@@ -102,22 +109,48 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
       sums(min(I + 1, nblk - 1));
       frag<T> fub[KS], fa[2][2];
       load_snap32<T, HD>(fub, I > Iw ? usnap + (usnap_off(I) + kw0) * HD : ku, c, g);
-#pragma unroll
-      for (int jtl = 0; jtl < 2; ++jtl) {
+      if constexpr (PAIRED) {
         wave_lds_order<STAGES>();
         pa.store(s_a);
+        pb.store(s_b);
         wave_lds_order<STAGES>();
-        if (jtl == 0) {
-          pa.load(ku + ((int64_t)I * kNB + 32) * HD);
-        } else {
-          pa.load(qc + (int64_t)I * kNB * HD);
-          pb.load(dout + (int64_t)I * kNB * HD);
-          pt.load(tb + (int64_t)I * kNB * kNB);
+        pa.load(qc + (int64_t)I * kNB * HD);
+        pb.load(dout + (int64_t)I * kNB * HD);
+        pt.load(tb + (int64_t)I * kNB * kNB);
+        acc_t a0, a1;
+        zero(a0);
+        zero(a1);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const frag<T> fq = ld_nat<T>(s_qu, LD, c, 16 * s + 8 * g);
+          mma(a0, ld_nat<T>(s_a, LD, c, 16 * s + 8 * g), fq);
+          mma(a1, ld_nat<T>(s_b, LD, c, 16 * s + 8 * g), fq);
         }
-        acc_t aT;
-        gate(aT, 2 * I + jtl);
-        fa[jtl][0] = chain<T>(aT, 0);
-        fa[jtl][1] = chain<T>(aT, 1);
+        gate_of(a0, 2 * I);
+        gate_of(a1, 2 * I + 1);
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+          fa[0][s2] = chain<T>(a0, s2);
+          fa[1][s2] = chain<T>(a1, s2);
+        }
+      } else {
+#pragma unroll
+        for (int jtl = 0; jtl < 2; ++jtl) {
+          wave_lds_order<STAGES>();
+          pa.store(s_a);
+          wave_lds_order<STAGES>();
+          if (jtl == 0) {
+            pa.load(ku + ((int64_t)I * kNB + 32) * HD);
+          } else {
+            pa.load(qc + (int64_t)I * kNB * HD);
+            pb.load(dout + (int64_t)I * kNB * HD);
+            pt.load(tb + (int64_t)I * kNB * kNB);
+          }
+          acc_t aT;
+          gate(aT, 2 * I + jtl);
+          fa[jtl][0] = chain<T>(aT, 0);
+          fa[jtl][1] = chain<T>(aT, 1);
+        }
       }
       if (I == Iw) {   // no state in front of the keys' own block
 #pragma unroll
@@ -149,6 +182,7 @@ __global__ __launch_bounds__(64 * W, (narrow_waves<T, HD>())) void key_narrow_ke
           if (!STAGES) pt.load(tb + ((int64_t)I * kNB + 32) * kNB);
         } else {
           pa.load(ku + (int64_t)min(I + 1, nblk - 1) * kNB * HD);
+          if (PAIRED) pb.load(ku + ((int64_t)min(I + 1, nblk - 1) * kNB + 32) * HD);
         }
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
