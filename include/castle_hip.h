@@ -331,14 +331,15 @@ int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const
  * epilogue: CASTLE_GEMM_GELU also writes gelu(c) (erf form) to aux, CASTLE_GEMM_GELU_SLOPE multiplies the product by the
  * derivative of gelu at aux; aux has c's shape and leading dimension.  A workspace of castle_gemm_workspace_bytes
  * (0 when the contraction is not split; then ldc may exceed N).  An operand of `rows` stored rows whose elements are further
- * than 2^31 from its start is refused (CASTLE_ERR_SHAPE): castle_gemm_operand_ok, 1 or 0. */
+ * than 2^31 from its start is refused (CASTLE_ERR_SHAPE): castle_gemm_operand_ok, 1 or 0.  fp32: an element goes to the 16-bit matrix instructions as three
+ * bf16 numbers, which hold all of it (below 2^-110 up to 2^-133); infinities and NaNs come out as fp32 instructions would have them. */
 #define CASTLE_GEMM_PLAIN 0
 #define CASTLE_GEMM_GELU 1
 #define CASTLE_GEMM_GELU_SLOPE 2
 int castle_gemm_operand_ok(int64_t rows, int64_t ld);
 int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue);
 /* What castle_gemm makes of a product, for tests and measurements: rows and columns of a workgroup's tile, ranges of the contraction, groups of four waves
- * that share a tile of 64 x 64. */
+ * that share a tile of 64 x 64 (fp32: of 32 x 32 or 64 x 64; 1 where fewer than four waves have one). */
 int castle_gemm_plan(int M, int N, int K, int dtype, int epilogue, int* rows, int* columns, int* ranges, int* groups);
 /* amax != NULL: CASTLE_AMAX_PARTIALS partial maxima of |c| over `columns` columns from `column` on (whole 16-byte pieces), for
  * CASTLE_FLAG_AMAX_READY; status, if not NULL, is set to 0.  Only where castle_gemm_amax_ok says so. */
