@@ -352,6 +352,15 @@ int castle_gemm_amax_ok(int M, int N, int K, int dtype, int column, int columns)
 int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b, int64_t ldb, int b_free_contiguous, void* c, int64_t ldc,
                 int M, int N, int K, int dtype, int epilogue, void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Both gradients of a projection y = x w^T in one launch: dw (N, K) = dy^T x and dx (R, K) = dy w, for dy (R, N), x (R, K) and w (N, K) with leading dimensions in
+ * elements; dw and dx are contiguous.  epilogue (CASTLE_GEMM_PLAIN or CASTLE_GEMM_GELU_SLOPE), aux and amax are those of castle_gemm for dx.  Only where the workspace's
+ * size is not negative: elsewhere two launches are ahead (N and K are multiples of 8).  _plan: for tests and measurements, a workgroup's tile and waves and the
+ * ranges of the two contractions. */
+int64_t castle_projection_grads_workspace_bytes(int R, int N, int K, int dtype, int epilogue, int with_amax);
+int castle_projection_grads_plan(int R, int N, int K, int dtype, int epilogue, int with_amax, int* tile, int* waves, int* dw_ranges, int* dx_ranges);
+int castle_projection_grads(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, const void* w, int64_t ld_w, void* dw, void* dx, int R, int N, int K,
+                            int dtype, int epilogue, const void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The same of normalised rows, castle_rms_norm without a summand and castle_gemm of two contraction-contiguous operands in one launch: c
  * = (a / sqrt(mean(a^2) + eps) * weight, rounded to the type) b^T.  h (M rows of K) and rstd (M floats) keep the normalised rows and their
  * factors, or are NULL; rstd needs h.  For few rows: only where castle_gemm_norm_ok says so. */

@@ -62,6 +62,9 @@ EXPORTED_SYMBOLS = (
     "castle_gemm",
     "castle_gemm_norm_ok",
     "castle_gemm_of_norm",
+    "castle_projection_grads_workspace_bytes",
+    "castle_projection_grads_plan",
+    "castle_projection_grads",
     "castle_rms_norm",
     "castle_rms_norm_bwd_workspace_bytes",
     "castle_rms_norm_bwd",

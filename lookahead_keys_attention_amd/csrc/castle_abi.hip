@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/castle_hip.h"
+#include <algorithm>
 #include <stdlib.h>
 #include <initializer_list>
 #include "castle_params.h"
@@ -720,6 +721,49 @@ int castle_gemm_of_norm(const void* a, int64_t lda, const castle_gemm_norm* norm
                         int dtype, const castle_amax* amax, void* stream) {
   if (norm == nullptr) return CASTLE_ERR_ARG;
   return gemm_common(norm, a, lda, 0, b, ldb, 0, c, ldc, M, N, K, dtype, CASTLE_GEMM_PLAIN, nullptr, amax, nullptr, 0, stream);
+}
+
+int64_t castle_projection_grads_workspace_bytes(int R, int N, int K, int dtype, int epilogue, int with_amax) {
+  const int es = elem_size(dtype);
+  if (es == 0) return CASTLE_ERR_DTYPE;
+  if (R <= 0 || N <= 0 || K <= 0 || N % 8 != 0 || K % 8 != 0 || (int64_t)(std::max(R, N) / 32 + 1) * (std::max(N, K) / 32 + 1) > (int64_t)1 << 30) return CASTLE_ERR_SHAPE;
+  if (epilogue != CASTLE_GEMM_PLAIN && epilogue != CASTLE_GEMM_GELU_SLOPE) return CASTLE_ERR_ARG;
+  const int64_t n = castle::grads_workspace(R, N, K, es, epilogue, with_amax != 0);
+  return n < 0 ? CASTLE_ERR_SHAPE : align_up(n, 256);
+}
+
+int castle_projection_grads_plan(int R, int N, int K, int dtype, int epilogue, int with_amax, int* tile, int* waves, int* dw_ranges, int* dx_ranges) {
+  const int64_t need = castle_projection_grads_workspace_bytes(R, N, K, dtype, epilogue, with_amax);
+  if (need < 0) return (int)need;
+  if (tile == nullptr || waves == nullptr || dw_ranges == nullptr || dx_ranges == nullptr) return CASTLE_ERR_ARG;
+  const castle::GradsPlan g = castle::grads_plan(R, N, K, elem_size(dtype), epilogue, with_amax != 0);
+  *tile = g.tile; *waves = g.waves; *dw_ranges = g.w_splits; *dx_ranges = g.x_splits;
+  return CASTLE_OK;
+}
+
+int castle_projection_grads(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, const void* w, int64_t ld_w, void* dw, void* dx, int R, int N, int K,
+                            int dtype, int epilogue, const void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t need = castle_projection_grads_workspace_bytes(R, N, K, dtype, epilogue, amax != nullptr);
+  if (need < 0) return (int)need;
+  const int v = 16 / elem_size(dtype);
+  if (!castle_gemm_operand_ok(R, ld_dy) || !castle_gemm_operand_ok(R, ld_x) || !castle_gemm_operand_ok(N, ld_w) || ld_dy < N || ld_x < K || ld_w < K || ld_dy % v != 0 ||
+      ld_x % v != 0 || ld_w % v != 0)
+    return CASTLE_ERR_SHAPE;
+  if (dy == nullptr || x == nullptr || w == nullptr || dw == nullptr || dx == nullptr || (epilogue != CASTLE_GEMM_PLAIN && aux == nullptr) || !aligned16({dy, x, w, dw, dx, aux}))
+    return CASTLE_ERR_ARG;
+  if (need > 0 && (workspace == nullptr || !aligned16({workspace}) || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
+  castle::GradsArgs p = {};
+  p.w = {dy, x, dw, nullptr, N, K, R, ld_dy, ld_x, K, castle::kGemmPlain, 0, nullptr, nullptr, nullptr, 0, 1, nullptr, 0.f, nullptr, nullptr};
+  p.x = {dy, w, dx, const_cast<void*>(aux), R, K, N, ld_dy, ld_w, K, epilogue, 0, nullptr, nullptr, nullptr, 0, 1, nullptr, 0.f, nullptr, nullptr};
+  if (amax != nullptr) {
+    if (amax->column < 0 || amax->columns <= 0 || amax->column + amax->columns > K || amax->column % v != 0 || amax->columns % v != 0) return CASTLE_ERR_SHAPE;
+    if (amax->partials == nullptr || reinterpret_cast<uintptr_t>(amax->partials) % 4 != 0 || reinterpret_cast<uintptr_t>(amax->status) % 4 != 0) return CASTLE_ERR_ARG;
+    p.x.amax = amax->partials;
+    p.x.amax_status = amax->status;
+    p.x.amax_from = amax->column;
+    p.x.amax_to = amax->column + amax->columns;
+  }
+  return castle::launch_grads(p, dtype, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
 }
 
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream) {

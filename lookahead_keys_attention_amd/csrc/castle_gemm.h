@@ -26,6 +26,12 @@ struct GemmArgs {
   void* h;
   float* rstd;
 };
+// Weight gradient w (both operands contraction-strided) and input gradient x (the second one) of a projection in one launch: w_groups workgroups in rows of w_row,
+// then x_groups in rows of x_row.
+struct GradsArgs {
+  GemmArgs w, x;
+  int w_groups, w_row, x_groups, x_row;
+};
 constexpr int kNormBytes = 2048;   // longest row that a product normalises
 bool gemm_norm_ok(int M, int N, int K, int elem_size);
 bool gemm_amax_ok(int M, int N, int K, int elem_size, int amax_from, int amax_to);
@@ -33,6 +39,11 @@ void gemm_plan(int M, int N, int K, int elem_size, bool epilogue, int (&out)[4])
 int64_t gemm_workspace(int M, int N, int K, int elem_size, bool epilogue);
 // fp32, castle_gemm32.hip
 int launch_gemm32(const GemmArgs& a, bool a_kc, bool b_kc, int tile, int splits, int waves, hipStream_t stream);
+int launch_grads32(const GradsArgs& p, int tile, int waves, hipStream_t stream);
+struct GradsPlan { int tile, waves, w_splits, x_splits; };   // tile 0: two launches
+GradsPlan grads_plan(int R, int N, int K, int elem_size, int epilogue, bool amax);
+int64_t grads_workspace(int R, int N, int K, int elem_size, int epilogue, bool amax);   // -1: two launches are ahead
+int launch_grads(GradsArgs p, int dtype, float* workspace, hipStream_t stream);
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream);
 
 }  // namespace castle

@@ -73,34 +73,38 @@ template <typename T, bool KC, int FREE, int BK, int G> struct Operand {
   }
 };
 
+constexpr int kStep16 = 64;   // contraction steps in LDS
 // G: groups of four waves.  Two take alternate steps of the contraction for the same tile, each in LDS of its own, and are summed at
 // the end: where the tiles leave a CU one workgroup, a second wave per SIMD works while the first waits for LDS and barrier.
 // NORM: the rows of `a` are normalised between memory and LDS, one tile per workgroup.  Every workgroup reads its 64 rows once for
 // their factors, with the first steps already on their way; that beats a launch in front of the product where the GPU is nearly empty.
-template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G, bool NORM = false>
-__global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(GemmArgs a) {
+template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G> constexpr int tile_elems() {
+  return max2(G * 2 * (Operand<T, AK, BM, BK, G>::ELEMS + Operand<T, BKC, BN, BK, G>::ELEMS), BM * (BN + elem_traits<T>::vec16));
+}
+// workgroup (bx, by) of (gx, ...), in `smem` of tile_elems
+template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G, bool NORM>
+__device__ __forceinline__ void gemm_tiles(const GemmArgs& a, T* smem, int bx, int by, int gx) {
   constexpr int WM = BM / 64, WN = BN / 64;   // 32-wide pieces of a wave's quarter
   typedef Operand<T, AK, BM, BK, G> OpA;
   typedef Operand<T, BKC, BN, BK, G> OpB;
   constexpr int V = elem_traits<T>::vec16, LDC = BN + V;
-  constexpr int kStage = 2 * (OpA::ELEMS + OpB::ELEMS), kOut = BM * LDC;
-  __shared__ __attribute__((aligned(16))) T smem[G * kStage > kOut ? G * kStage : kOut];
+  constexpr int kStage = 2 * (OpA::ELEMS + OpB::ELEMS);
   const int lane = lane_id(), wave = G == 1 ? wave_id() : wave_id() % 4, group = G == 1 ? 0 : wave_id() / 4, c = lane & 31, g = lane >> 5;
   // Workgroups go round the 8 XCDs, each with an L2 of its own: XCD x takes the x-th eighth of the tiles, so the rows of
   // `a` are read by one XCD, not by all (input gradient of 3000 rows x 1536 x 256: 13.5 -> 11.1 us).  A workgroup takes
   // several tiles where there are more than the CUs hold: the first steps of the next are requested before the
   // output of the last is written.
   const int tiles_n = (a.N + BN - 1) / BN, tiles = (a.M + BM - 1) / BM * tiles_n;
-  const int share = (tiles + 7) / 8, first = blockIdx.x % 8 * share, last = min(tiles, first + share);
+  const int share = (tiles + 7) / 8, first = bx % 8 * share, last = min(tiles, first + share);
   const int wm = wave / 2 * (BM / 2), wn = wave % 2 * (BN / 2);
-  const int k0 = blockIdx.y * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split);
+  const int k0 = by * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split);
   const int steps = ((k_end - k0 + BK - 1) / BK + G - 1) / G;   // of a group: its steps are G BK apart
   T* const stage = smem + group * kStage;
   const T *pa = static_cast<const T*>(a.a), *pb = static_cast<const T*>(a.b);
   OpA ra;
   OpB rb;
   acc_t acc[WM][WN];   // [n rows, m lanes]
-  int tile = first + blockIdx.x / 8;
+  int tile = first + bx / 8;
   auto request = [&]() __attribute__((always_inline)) {
     ra.start((int)a.lda, tile / tiles_n * BM, a.M, k0 + group * BK);
     rb.start((int)a.ldb, tile % tiles_n * BN, a.N, k0 + group * BK);
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
     }
   };
   const int amax_tile = a.amax_from / BN, amax_tiles = (a.amax_to - 1) / BN + 1 - amax_tile;   // of a row of tiles
-  if (a.amax != nullptr && blockIdx.x == 0) {
+  if (a.amax != nullptr && bx == 0) {
     for (int i = (a.M + BM - 1) / BM * amax_tiles + threadIdx.x; i < kAmaxBlocks; i += kThreads * G) a.amax[i] = 0.f;
     if (threadIdx.x == 0 && a.amax_status != nullptr) *a.amax_status = 0;
   }
@@ -213,7 +217,7 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
     }
     if constexpr (G == 2) {
       typedef vec<float, 4> v4;
-      static_assert(kThreads * WM * WN * 64 <= (int)sizeof(smem), "one group's sums");
+      static_assert(kThreads * WM * WN * 64 <= (int)sizeof(T) * tile_elems<T, AK, BKC, BM, BN, BK, G>(), "one group's sums");
       v4* sums = reinterpret_cast<v4*>(smem);
       asm volatile("s_nop 15\n\ts_nop 3" ::: "memory");   // the loop may end right behind a product
       __builtin_amdgcn_sched_barrier(0);
@@ -236,10 +240,10 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
           }
       }
     }
-    tile += gridDim.x / 8;
+    tile += gx / 8;
     if (tile < last) request();
     if (a.part != nullptr) {   // partial product of this range of the contraction
-      float* part = a.part + (int64_t)blockIdx.y * a.M * a.N;
+      float* part = a.part + (int64_t)by * a.M * a.N;
 #pragma unroll
       for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -304,6 +308,24 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
       }
     }
     __syncthreads();
+  }
+}
+template <typename T, bool AK, bool BKC, int BM, int BN, int BK, int G, bool NORM = false>
+__global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(GemmArgs a) {
+  __shared__ __attribute__((aligned(16))) T smem[tile_elems<T, AK, BKC, BM, BN, BK, G>()];
+  gemm_tiles<T, AK, BKC, BM, BN, BK, G, NORM>(a, smem, blockIdx.x, blockIdx.y, gridDim.x);
+}
+// Both gradients of a projection, which read the same dy and nothing of each other, in one launch: workgroups of the weight gradient
+// (w.k_per_split rows of the contraction each), then those of the input gradient.
+template <typename T, int G> __global__ __launch_bounds__(kThreads * G, 4) void grads_kernel(GradsArgs p) {
+  constexpr int kElems = max2(tile_elems<T, false, false, 64, 64, kStep16, G>(), tile_elems<T, true, false, 64, 64, kStep16, G>());
+  __shared__ __attribute__((aligned(16))) T smem[kElems];
+  int b = blockIdx.x;
+  if (b < p.w_groups) {
+    gemm_tiles<T, false, false, 64, 64, kStep16, G, false>(p.w, smem, b % p.w_row, b / p.w_row, p.w_row);
+  } else {
+    b -= p.w_groups;
+    gemm_tiles<T, true, false, 64, 64, kStep16, G, false>(p.x, smem, b % p.x_row, b / p.x_row, p.x_row);
   }
 }
 
@@ -588,10 +610,10 @@ template <typename T, bool AK, bool BKC, int BN, bool FUSED> __global__ __launch
 // 256 x 128; 4096 rows 512 -> 3072 31.8, 26.2, 24.9 and 21.8 on 256 x 256; 8184 rows 64 -> 4096 20.0, 18.6, 15.8 and 15.3.  Over 2500 products of 96 ... 65536
 // rows, outputs of 64 ... 4096 columns and contractions of 64 ... 8184, in all layouts, each timed with every tile and up to 16 ranges, what this picks takes 1.5 %
 // more than the best of them on average.
-constexpr int kStep16 = 64;   // contraction steps in LDS
 struct Plan {
   int tile, splits, groups;   // tile: 32 (fp32), 64, 128, or columns of a tile of 256 rows + 256; groups: of four waves
-  int waves = 0;   // fp32
+  int waves = 0;    // fp32
+  float cost = 0;   // us, roughly
   int rows() const { return std::min(tile, kWideM); }
   int columns() const { return tile > kWideM ? tile - kWideM : tile; }
   int tiles(int M, int N) const { return ((M + rows() - 1) / rows()) * ((N + columns() - 1) / columns()); }
@@ -630,7 +652,7 @@ Plan plan32(int M, int N, int K, bool plain) {
       const float fixed = kind.start + (s > 1 ? kind.split + s * mb * kind.split_mb : 0.f);
       if (fixed + work >= best_cost) continue;
       const float read = 8e-6f * tiles * K * kind.tile * kind.read, w2 = work * work, r2 = read * read, cost = fixed + std::sqrt(std::sqrt(w2 * w2 + r2 * r2));
-      if (cost < best_cost) { best_cost = cost; best = {kind.tile, s, std::max(1, kind.waves / 4), kind.waves}; }
+      if (cost < best_cost) { best_cost = cost; best = {kind.tile, s, std::max(1, kind.waves / 4), kind.waves, cost}; }
     }
   }
   return best;
@@ -640,7 +662,7 @@ Plan plan(int M, int N, int K, bool plain, int elem_size) {
   Plan best = {64, 1, 1};
   double best_cost = 1e30;
   auto take = [&](double cost, const Plan& p) {
-    if (cost < best_cost) { best_cost = cost; best = p; }
+    if (cost < best_cost) { best_cost = cost; best = p; best.cost = (float)cost; }
   };
   // Two tensors that no cache holds: stores of single lines cost more (gelu of 65536 rows 64 -> 1536 on 64 x 64 123, on 256 x 256 94), and 256 x 256 where rows do not
   // start with lines (33000 rows 64 -> 3064 192, 256 x 128 103, 64 x 64 150).
@@ -752,6 +774,79 @@ int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, h
   });
   if (rc != 0 || a.part == nullptr) return rc;
   return launch_part_sum(a.part, p.splits, (int64_t)a.M * a.N, a.c, dtype, stream);
+}
+
+// Both gradients of a projection in one launch, y = x w^T with R rows, N outputs, K inputs.  They are launches of a few us that leave CUs idle, each with a start,
+// a trip to memory and a last wave of its own.  What one launch of both takes (us): a start, and the 4-norm of the longest workgroup by itself, of the steps and ends
+// of all workgroups spread over the CUs, and of what the tiles read; ranges of a contraction add the launch that sums them and their partial results.  Fitted to 49000
+// timings of 2904 projections of 16 ... 8192 rows, widths of 64 ... 6144 and up to 40 GFLOP.  One launch is taken where this is clearly less than the plans of the two
+// by themselves, in four of five of those, 1.4 times as fast there in 16 bit and 1.3 in fp32 (all of them: 1.32 and 1.2; slower by more than 4 % in 0 and 0.4 %).  Two against
+// one, us: bf16 3000 rows 256 -> 1536 25.1 / 19.0, 256 -> 256 13.6 / 10.0, 199 rows 384 -> 384 9.9 / 6.0, fp32 256 rows 512 -> 3072 28.5 / 24.6, 512 -> 512 10.6 / 8.4;
+// bf16 977 rows 768 -> 4608, where one of the two has larger tiles, 42.3 / 52.6.
+GradsPlan grads_plan(int R, int N, int K, int elem_size, int epilogue, bool amax) {
+  struct Kind { int tile, waves, turns; float start, alone, shared, end, ends, split, split_mb, read; };   // turns: steps at a time
+  constexpr Kind kinds[2][3] = {{{64, 4, 4, 3.908f, 1.49f, 1.334f, 0.96f, 2.395f, 2.207f, 0.154f, 0.098f},
+                                 {32, 4, 4, 3.865f, 0.812f, 0.548f, 0, 0.604f, 2.135f, 0.118f, 0},
+                                 {32, 8, 8, 3.711f, 0.843f, 0.96f, 0, 0.898f, 1.991f, 0.138f, 0.065f}},
+                                {{64, 4, 1, 3.255f, 0.434f, 0.166f, 0, 1.09f, 2.431f, 0.167f, 0.064f},
+                                 {64, 8, 2, 3.183f, 0.581f, 0.404f, 0, 1.605f, 2.497f, 0.129f, 0.063f}}};
+  const bool plain = epilogue == kGemmPlain, half = elem_size == 2;
+  if ((int64_t)(N + R) * K > (int64_t)1 << 26) return {0, 0, 0, 0};
+  const int step = half ? kStep16 : 32;
+  GradsPlan best = {0, 0, 0, 0};
+  const Plan pw = plan(N, K, R, true, elem_size), px = plan(R, K, N, plain || amax, elem_size);
+  if (half && std::max(pw.tile, px.tile) > 64) return best;   // (larger tiles read less)
+  float best_cost = (half ? 0.96f : 0.88f) * (pw.cost + px.cost);
+  for (const Kind& kind : kinds[half]) {
+    if (kind.tile == 0) break;
+    const int tk = (K + kind.tile - 1) / kind.tile, tw = (N + kind.tile - 1) / kind.tile * tk, tx = (R + kind.tile - 1) / kind.tile * tk;
+    if (amax && tx > kAmaxBlocks) continue;
+    const float read = kind.read * 2e-6f * elem_size * kind.tile * ((float)tw * R + (float)tx * N), r2 = read * read;
+    for (const int w : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (w > 1 && (w * 64 > R || tw * w > 1100)) break;
+      const int nw = ((R + w - 1) / w + step - 1) / step;
+      for (const int x : {1, 2, 4, 8}) {
+        if (x > 1 && (!plain || amax || x * 128 > N || tx * x > 600)) break;
+        if (kind.tile == 32 && tw * w + tx * x > 1280) continue;   // (all tiles of 32 x 32 read twice what those of 64 x 64 do)
+        const int nx = ((N + x - 1) / x + step - 1) / step, tw_ = (nw + kind.turns - 1) / kind.turns, tx_ = (nx + kind.turns - 1) / kind.turns, longest = std::max(tw_, tx_);
+        const float groups_w = (tw + 7) / 8 * w * (1 / 32.f), groups_x = (tx + 7) / 8 * x * (1 / 32.f);
+        const float alone = kind.alone * longest + kind.end, all = kind.shared * std::max(groups_w * tw_ + groups_x * tx_, (float)longest) + kind.ends * std::ceil(groups_w + groups_x);
+        const float a2 = alone * alone, s2 = all * all;
+        const float cost = kind.start + std::sqrt(std::sqrt(a2 * a2 + s2 * s2 + r2 * r2)) + kind.split * ((w > 1) + (x > 1)) +
+                           kind.split_mb * 8e-6f * ((w > 1 ? (float)w * N * K : 0) + (x > 1 ? (float)x * R * K : 0));
+        if (cost < best_cost) { best_cost = cost; best = {kind.tile, kind.waves, w, x}; }
+      }
+    }
+  }
+  return best;
+}
+int64_t grads_workspace(int R, int N, int K, int elem_size, int epilogue, bool amax) {
+  const GradsPlan g = grads_plan(R, N, K, elem_size, epilogue, amax);
+  if (g.tile == 0) return -1;
+  return ((g.w_splits > 1 ? (int64_t)g.w_splits * N * K : 0) + (g.x_splits > 1 ? (int64_t)g.x_splits * R * K : 0)) * 4;
+}
+int launch_grads(GradsArgs p, int dtype, float* workspace, hipStream_t stream) {
+  const int step = dtype == 0 ? 32 : kStep16;
+  const GradsPlan g = grads_plan(p.x.M, p.x.K, p.x.N, dtype == 0 ? 4 : 2, p.x.epilogue, p.x.amax != nullptr);
+  auto place = [&](GemmArgs& a, int splits, int& groups, int& row) {
+    a.k_per_split = ((a.K + splits - 1) / splits + step - 1) / step * step;
+    splits = (a.K + a.k_per_split - 1) / a.k_per_split;   // rounding up may leave the last ones empty
+    a.part = splits > 1 ? workspace : nullptr;
+    if (splits > 1) workspace += (int64_t)splits * a.M * a.N;
+    row = (((a.M + g.tile - 1) / g.tile) * ((a.N + g.tile - 1) / g.tile) + 7) / 8 * 8;
+    groups = row * splits;
+  };
+  place(p.w, g.w_splits, p.w_groups, p.w_row);
+  place(p.x, g.x_splits, p.x_groups, p.x_row);
+  int rc = dtype == 0 ? launch_grads32(p, g.tile, g.waves, stream) : by_type16(dtype, true, [&](auto t, auto) {
+    using T = decltype(t);
+    if (g.waves == 8) hipLaunchKernelGGL((grads_kernel<T, 2>), dim3(p.w_groups + p.x_groups), dim3(2 * kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((grads_kernel<T, 1>), dim3(p.w_groups + p.x_groups), dim3(kThreads), 0, stream, p);
+    return hipGetLastError() == hipSuccess ? 0 : -3;
+  });
+  for (const GemmArgs* a : {&p.w, &p.x})
+    if (rc == 0 && a->part != nullptr) rc = launch_part_sum(a->part, (a->K + a->k_per_split - 1) / a->k_per_split, (int64_t)a->M * a->N, a->c, dtype, stream);
+  return rc;
 }
 
 }  // namespace castle

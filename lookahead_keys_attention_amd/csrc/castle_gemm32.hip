@@ -132,22 +132,21 @@ constexpr int kUnit32 = 66;
 template <int TILE> constexpr int wave_bytes() { return max2(TILE * TILE / 256 * kUnit32 * 16, 2 * TILE * kStep * 4); }
 // NORM: the rows of `a` are normalised on their way to the registers.
 template <bool AK, bool BKC, int TILE, int W, bool NORM>
-__global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void gemm32_kernel(GemmArgs a) {
+__device__ __forceinline__ void gemm32_tile(const GemmArgs& a, vec<float, 4>* s_sum, int bx, int by) {   // s_sum: of a wave, operands, then sums
   constexpr int V = 4, NT = 64 * W, BM = TILE, BN = TILE, F = TILE / 32, U = 4 * F * F;   // U: quads of accumulator registers
   typedef Operand32<AK, TILE> OpA;
   typedef Operand32<BKC, TILE> OpB;
   typedef vec<float, 4> v4;
   constexpr int kWave = wave_bytes<TILE>() / 16;
-  __shared__ __attribute__((aligned(16))) v4 s_sum[W * kWave];   // of a wave: operands, then sums
   const int lane = lane_id(), wave = wave_id(), c = lane & 31, g = lane >> 5;
   // XCD x takes the x-th eighth of the tiles, for its L2
   const int tiles_n = (a.N + BN - 1) / BN, tiles = (a.M + BM - 1) / BM * tiles_n, share = (tiles + 7) / 8;
-  const int tile = blockIdx.x % 8 * share + blockIdx.x / 8;
+  const int tile = bx % 8 * share + bx / 8;
   if (tile >= tiles) return;
   const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
-  const int k0 = blockIdx.y * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split), stages = (k_end - k0 + kStep - 1) / kStep;
+  const int k0 = by * a.k_per_split, k_end = min(a.K, k0 + a.k_per_split), stages = (k_end - k0 + kStep - 1) / kStep;
   const int amax_tile = a.amax_from / BN, amax_tiles = (a.amax_to - 1) / BN + 1 - amax_tile;   // of a row of tiles
-  if (a.amax != nullptr && blockIdx.x == 0) {
+  if (a.amax != nullptr && bx == 0) {
     for (int i = (a.M + BM - 1) / BM * amax_tiles + threadIdx.x; i < kAmaxBlocks; i += NT) a.amax[i] = 0.f;
     if (threadIdx.x == 0 && a.amax_status != nullptr) *a.amax_status = 0;
   }
@@ -307,7 +306,7 @@ __global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void gemm32_kernel(G
     v4 x = part[0];
     for (int w = 1; w < with; ++w) x += part[w * kWave];
     if (a.part != nullptr) {   // partial product of this range of the contraction
-      *reinterpret_cast<v4*>(a.part + (int64_t)blockIdx.y * a.M * a.N + (int64_t)m * a.N + n) = x;
+      *reinterpret_cast<v4*>(a.part + (int64_t)by * a.M * a.N + (int64_t)m * a.N + n) = x;
       continue;
     }
     const int64_t at = (int64_t)m * a.ldc + n;
@@ -341,6 +340,22 @@ __global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void gemm32_kernel(G
     }
   }
 }
+template <bool AK, bool BKC, int TILE, int W, bool NORM>
+__global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void gemm32_kernel(GemmArgs a) {
+  __shared__ __attribute__((aligned(16))) vec<float, 4> s_sum[W * wave_bytes<TILE>() / 16];
+  gemm32_tile<AK, BKC, TILE, W, NORM>(a, s_sum, blockIdx.x, blockIdx.y);
+}
+// both gradients of a projection: workgroups of the weight gradient, then those of the input gradient
+template <int TILE, int W> __global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void grads32_kernel(GradsArgs p) {
+  __shared__ __attribute__((aligned(16))) vec<float, 4> s_sum[W * wave_bytes<TILE>() / 16];
+  int b = blockIdx.x;
+  if (b < p.w_groups) {
+    gemm32_tile<false, false, TILE, W, false>(p.w, s_sum, b % p.w_row, b / p.w_row);
+  } else {
+    b -= p.w_groups;
+    gemm32_tile<true, false, TILE, W, false>(p.x, s_sum, b % p.x_row, b / p.x_row);
+  }
+}
 
 }  // namespace
 
@@ -362,6 +377,14 @@ int launch_gemm32(const GemmArgs& a, bool a_kc, bool b_kc, int tile, int splits,
   if (a.norm_w != nullptr) return go(yes, yes, yes);
   if (a_kc) return b_kc ? go(yes, yes, no) : go(yes, no, no);
   return b_kc ? -2 : go(no, no, no);
+}
+
+int launch_grads32(const GradsArgs& p, int tile, int waves, hipStream_t stream) {
+  const dim3 grid(p.w_groups + p.x_groups);
+  if (tile == 32 && waves == 8) hipLaunchKernelGGL((grads32_kernel<32, 8>), grid, dim3(512), 0, stream, p);
+  else if (tile == 32) hipLaunchKernelGGL((grads32_kernel<32, 4>), grid, dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((grads32_kernel<64, 4>), grid, dim3(256), 0, stream, p);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 }  // namespace castle

@@ -561,6 +561,34 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (
   return at::mm(dy.t(), x);
 }
 
+// Both gradients of a projection, in one launch where that is ahead (false: they are left to the functions above).  aux: dx is multiplied by the slope of gelu at
+// it; nbytes >= 0: the maxima of |dx| go to a workspace of that size, `prepared` (16-bit types).
+bool own_projection_grads(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& aux, int64_t nbytes, Tensor& dw, Tensor& dx, Tensor& prepared) {
+  const int64_t R = dy.size(0), N = dy.size(1), K = w.size(1);
+  const bool full = dy.scalar_type() == at::kFloat, with_amax = !full && nbytes >= 0;
+  if (x.dim() != 2 || x.size(0) != R || x.size(1) != K || w.size(0) != N || x.scalar_type() != dy.scalar_type() || w.scalar_type() != dy.scalar_type() || x.device() != dy.device() ||
+      w.device() != dy.device() || (!full && R >= kSplitWgradMinRows) || !own_product(dy, x, R, N, K, kOwnWeightGrad) ||
+      !own_product(dy, w, R, K, N, aux.defined() ? kOwnGeluSlope : own_input_grad(N)))
+    return false;
+  if (aux.defined() && !(aux.is_contiguous() && aux.dim() == 2 && aux.size(0) == R && aux.size(1) == K && aux.scalar_type() == dy.scalar_type() && aux.device() == dy.device() && aligned16(aux)))
+    return false;
+  const int dtype = dtype_code(dy), epilogue = aux.defined() ? CASTLE_GEMM_GELU_SLOPE : CASTLE_GEMM_PLAIN;
+  const int64_t need = castle_projection_grads_workspace_bytes((int)R, (int)N, (int)K, dtype, epilogue, with_amax);
+  if (need < 0) return false;
+  castle_amax where;
+  if (with_amax) {
+    prepared = bytes(nbytes, dy);
+    where = {reinterpret_cast<float*>(static_cast<char*>(prepared.data_ptr()) + CASTLE_AMAX_OFFSET), nullptr, 0, (int32_t)K};
+  }
+  const Tensor ws = need ? bytes(need, dy) : Tensor();
+  dw = at::empty({N, K}, dy.options());
+  dx = at::empty({R, K}, dy.options());
+  check(castle_projection_grads(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), dw.data_ptr(), dx.data_ptr(), (int)R, (int)N, (int)K, dtype,
+                                epilogue, aux.defined() ? aux.data_ptr() : nullptr, with_amax ? &where : nullptr, need ? ws.data_ptr() : nullptr, need, stream_of(dy)),
+        "castle_projection_grads");
+  return true;
+}
+
 // A projection as a registered operator, for callers that are traced.
 Tensor linear_op(const Tensor& x, const Tensor& weight) {
   const c10::DeviceGuard guard(x.device());
@@ -571,6 +599,8 @@ Tensor linear_op(const Tensor& x, const Tensor& weight) {
 std::tuple<Tensor, Tensor> linear_bwd_op(const Tensor& dy_, const Tensor& x, const Tensor& weight, bool need_x, bool need_w) {
   const c10::DeviceGuard guard(x.device());
   const Tensor dy = dy_.reshape({-1, weight.size(0)});
+  Tensor dw, dx, none;
+  if (need_x && need_w && own_projection_grads(dy, x.reshape({-1, x.size(-1)}), weight, Tensor(), -1, dw, dx, none)) return {dx.view(x.sizes()), dw};
   return {need_x ? input_grad(dy, weight).view(x.sizes()) : at::empty({0}, x.options()),
           need_w ? weight_grad(dy, x.reshape({-1, x.size(-1)})) : at::empty({0}, weight.options())};
 }
@@ -687,12 +717,19 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     auto rows = [&](const Tensor& t) { return t.defined() && t.dim() == 3 ? t.reshape({B * L, t.size(2)}) : t; };
     const size_t nn = rstd.defined() ? 1 : 0;
     const bool need_norm = nn && ctx->needs_input_grad(1 + nd), need_qkv = ctx->needs_input_grad(1 + nd + nn);
-    if (ctx->needs_input_grad(2 + nd + nn)) grads[4] = weight_grad(dy, merged.view({B * L, merged.size(2)}));
-    if (!need_x && !need_norm && !need_qkv) return grads;
+    const bool need_core = need_x || need_norm || need_qkv, need_out = ctx->needs_input_grad(2 + nd + nn);
+    const Tensor merged2 = merged.view({B * L, merged.size(2)});
+    if (!need_core) {
+      if (need_out) grads[4] = weight_grad(dy, merged2);
+      return grads;
+    }
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
     const int64_t flags = ctx->saved_data["flags"].toInt();
     Tensor dmerged, prepared;
-    if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)))) {
+    const bool both = need_out && own_projection_grads(dy, merged2, w_out, Tensor(), bwd_workspace_bytes(shape, flags, state), grads[4], dmerged, prepared);
+    if (need_out && !both) grads[4] = weight_grad(dy, merged2);
+    if (both) {
+    } else if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)))) {
       const Maxima m = maxima(dy, B * L, w_out.size(1), w_out.size(0), 0, w_out.size(1), bwd_workspace_bytes(shape, flags, state), false);
       prepared = m.prepared;
       dmerged = product(dy, false, w_out, true, CASTLE_GEMM_PLAIN, std::nullopt, m.get());
@@ -706,9 +743,11 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(), flags, d6, ws,
             state, prepared);
     const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
-    if (need_qkv) grads[3] = weight_grad(dp2, rows(s[4]));
+    Tensor dh, none;
+    const bool both_in = need_qkv && (need_x || need_norm) && own_projection_grads(dp2, rows(s[4]), w_qkv, Tensor(), -1, grads[3], dh, none);
+    if (need_qkv && !both_in) grads[3] = weight_grad(dp2, rows(s[4]));
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(input_grad(dp2, w_qkv), rows(s[0]), rstd, norm_w, rows(dsum), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(both_in ? dh : input_grad(dp2, w_qkv), rows(s[0]), rstd, norm_w, rows(dsum), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = dx.view({B, L, dx.size(1)});
       if (has_delta) grads[1] = grads[0];
@@ -779,14 +818,18 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const c10::DeviceGuard guard(h.device());
     const int64_t R = sum.size(0), dim = sum.size(1);
     const Tensor dy = g[0].reshape({R, dim});
-    if (ctx->needs_input_grad(4)) grads[4] = weight_grad(dy, act);
-    if (!need_x && !need_norm && !need_up) return grads;
-    const Tensor dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnGeluSlope)
-                           ? product(dy, false, w_down, true, CASTLE_GEMM_GELU_SLOPE, up)
-                           : at::gelu_backward(at::mm(dy, w_down), up);
-    if (need_up) grads[3] = weight_grad(dup, h);
+    const bool below = need_x || need_norm || need_up, need_down = ctx->needs_input_grad(4);
+    Tensor dup, dh, none;
+    const bool both = below && need_down && own_projection_grads(dy, act, w_down, up, -1, grads[4], dup, none);
+    if (need_down && !both) grads[4] = weight_grad(dy, act);
+    if (!below) return grads;
+    if (!both)
+      dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnGeluSlope) ? product(dy, false, w_down, true, CASTLE_GEMM_GELU_SLOPE, up)
+                                                                           : at::gelu_backward(at::mm(dy, w_down), up);
+    const bool both_up = need_up && (need_x || need_norm) && own_projection_grads(dup, h, w_up, Tensor(), -1, grads[3], dh, none);
+    if (need_up && !both_up) grads[3] = weight_grad(dup, h);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(input_grad(dup, w_up), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({R, dim}) : Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(both_up ? dh : input_grad(dup, w_up), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({R, dim}) : Tensor(), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = grads[1] = dx.view(g[0].sizes());
     }
@@ -820,9 +863,12 @@ struct HeadFn : torch::autograd::Function<HeadFn> {
     const c10::DeviceGuard guard(h.device());
     const Tensor dy = g[0].reshape({sum.size(0), w.size(0)});
     const bool need_x = ctx->needs_input_grad(0) || ctx->needs_input_grad(1), need_norm = ctx->needs_input_grad(2);
-    if (ctx->needs_input_grad(3)) grads[3] = weight_grad(dy, h);
+    const bool need_w = ctx->needs_input_grad(3);
+    Tensor dh, none;
+    const bool both = need_w && (need_x || need_norm) && own_projection_grads(dy, h, w, Tensor(), -1, grads[3], dh, none);
+    if (need_w && !both) grads[3] = weight_grad(dy, h);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(input_grad(dy, w), sum, rstd, norm_w, Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(both ? dh : input_grad(dy, w), sum, rstd, norm_w, Tensor(), need_x, need_norm);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = grads[1] = dx.view({g[0].size(0), g[0].size(1), sum.size(1)});
     }
