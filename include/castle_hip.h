@@ -318,11 +318,24 @@ int castle_gather_rows(const void* table, int64_t table_rows, int64_t ld, int wi
  * to `sum`) when delta != NULL.  rstd: NULL, or one float per row for the backward pass. */
 int castle_rms_norm(const void* x, const void* delta, const void* weight, void* sum, void* h, float* rstd, int64_t rows, int width, float eps,
                     int dtype, void* stream);
+/* A sum of partial results that a call has left, for castle_sums (up to CASTLE_MAX_SUMS of them, all of one type, in one launch): out[n] = sum over `parts` rows of
+ * part[parts][n]; columns: rather down the columns of a few, else n is a multiple of 8.  parts = 0: there is nothing to sum.  The workspace that `part` lies in is kept until then. */
+#define CASTLE_MAX_SUMS 4
+typedef struct castle_sum {
+  const float* part;
+  int64_t n;
+  void* out;
+  int32_t parts, columns;
+} castle_sum;
+int castle_sums(const castle_sum* sums, int count, int dtype, void* stream);
+
 /* dx = dres + d(norm)/dx dh (dres may be NULL), dweight = sum over rows; either result may be NULL.  The workspace is
- * only needed for dweight. */
+ * only needed for dweight.  _parts: the sum over rows is left to castle_sums. */
 int64_t castle_rms_norm_bwd_workspace_bytes(int64_t rows, int width, int dtype);
 int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
                         int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+int castle_rms_norm_bwd_parts(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight, castle_sum* dw_sum,
+                              int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* c[M, N] = the product of two matrices over K, in the type `dtype` with fp32 sums: the projections of a layer and their
  * gradients over hundreds to thousands of rows (nn.Linear at lookahead_keys_attention.py:75, 80, 99, 209).  An operand
@@ -354,12 +367,12 @@ int castle_gemm(const void* a, int64_t lda, int a_free_contiguous, const void* b
 
 /* Both gradients of a projection y = x w^T in one launch: dw (N, K) = dy^T x and dx (R, K) = dy w, for dy (R, N), x (R, K) and w (N, K) with leading dimensions in
  * elements; dw and dx are contiguous.  epilogue (CASTLE_GEMM_PLAIN or CASTLE_GEMM_GELU_SLOPE), aux and amax are those of castle_gemm for dx.  Only where the workspace's
- * size is not negative: elsewhere two launches are ahead (N and K are multiples of 8).  _plan: for tests and measurements, a workgroup's tile and waves and the
+ * size is not negative: elsewhere two launches are ahead (N and K are multiples of 8).  dw_sum != NULL: a dw that is formed in ranges is left to castle_sums.  _plan: for tests and measurements, a workgroup's tile and waves and the
  * ranges of the two contractions. */
 int64_t castle_projection_grads_workspace_bytes(int R, int N, int K, int dtype, int epilogue, int with_amax);
 int castle_projection_grads_plan(int R, int N, int K, int dtype, int epilogue, int with_amax, int* tile, int* waves, int* dw_ranges, int* dx_ranges);
 int castle_projection_grads(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, const void* w, int64_t ld_w, void* dw, void* dx, int R, int N, int K,
-                            int dtype, int epilogue, const void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream);
+                            int dtype, int epilogue, const void* aux, const castle_amax* amax, castle_sum* dw_sum, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The same of normalised rows, castle_rms_norm without a summand and castle_gemm of two contraction-contiguous operands in one launch: c
  * = (a / sqrt(mean(a^2) + eps) * weight, rounded to the type) b^T.  h (M rows of K) and rstd (M floats) keep the normalised rows and their

@@ -68,7 +68,9 @@ EXPORTED_SYMBOLS = (
     "castle_rms_norm",
     "castle_rms_norm_bwd_workspace_bytes",
     "castle_rms_norm_bwd",
+    "castle_rms_norm_bwd_parts",
     "castle_sum_parts",
+    "castle_sums",
     "castle_cross_entropy",
     "castle_cross_entropy_bwd",
     "castle_embedding_grad_workspace_bytes",

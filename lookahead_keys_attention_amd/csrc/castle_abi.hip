@@ -630,7 +630,7 @@ int64_t castle_rms_norm_bwd_workspace_bytes(int64_t rows, int width, int dtype) 
   return align_up((int64_t)castle::norm_bwd_groups(rows, width, es) * width * 4, 256);
 }
 
-int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
+static int norm_bwd_common(castle_sum* dw_sum, const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
                         int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   const int64_t need = castle_rms_norm_bwd_workspace_bytes(rows, width, dtype);
   if (need < 0) return (int)need;
@@ -640,7 +640,19 @@ int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const
     return CASTLE_ERR_ARG;
   if (dweight != nullptr && (workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < need)) return CASTLE_ERR_WORKSPACE;
   const castle::NormBwdArgs a = {dh, x, weight, dres, rstd, dx, dweight != nullptr ? static_cast<float*>(workspace) : nullptr, rows, width};
-  return castle::launch_norm_bwd(a, dweight, dtype, static_cast<hipStream_t>(stream));
+  castle::PartSum later = {};
+  const int rc = castle::launch_norm_bwd(a, dweight, dtype, dw_sum != nullptr ? &later : nullptr, static_cast<hipStream_t>(stream));
+  if (rc == 0 && dw_sum != nullptr) *dw_sum = {later.part, later.n, later.out, later.parts, later.columns};
+  return rc;
+}
+int castle_rms_norm_bwd(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight,
+                        int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  return norm_bwd_common(nullptr, dh, x, weight, rstd, dres, dx, dweight, rows, width, dtype, workspace, workspace_bytes, stream);
+}
+int castle_rms_norm_bwd_parts(const void* dh, const void* x, const void* weight, const float* rstd, const void* dres, void* dx, void* dweight, castle_sum* dw_sum,
+                              int64_t rows, int width, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (dw_sum == nullptr) return CASTLE_ERR_ARG;
+  return norm_bwd_common(dw_sum, dh, x, weight, rstd, dres, dx, dweight, rows, width, dtype, workspace, workspace_bytes, stream);
 }
 
 int64_t castle_gemm_workspace_bytes(int M, int N, int K, int dtype, int epilogue) {
@@ -742,7 +754,7 @@ int castle_projection_grads_plan(int R, int N, int K, int dtype, int epilogue, i
 }
 
 int castle_projection_grads(const void* dy, int64_t ld_dy, const void* x, int64_t ld_x, const void* w, int64_t ld_w, void* dw, void* dx, int R, int N, int K,
-                            int dtype, int epilogue, const void* aux, const castle_amax* amax, void* workspace, int64_t workspace_bytes, void* stream) {
+                            int dtype, int epilogue, const void* aux, const castle_amax* amax, castle_sum* dw_sum, void* workspace, int64_t workspace_bytes, void* stream) {
   const int64_t need = castle_projection_grads_workspace_bytes(R, N, K, dtype, epilogue, amax != nullptr);
   if (need < 0) return (int)need;
   const int v = 16 / elem_size(dtype);
@@ -763,7 +775,13 @@ int castle_projection_grads(const void* dy, int64_t ld_dy, const void* x, int64_
     p.x.amax_from = amax->column;
     p.x.amax_to = amax->column + amax->columns;
   }
-  return castle::launch_grads(p, dtype, static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+  castle::PartSum later;
+  const int rc = castle::launch_grads(p, dtype, static_cast<float*>(workspace), dw_sum != nullptr ? &later : nullptr, static_cast<hipStream_t>(stream));
+  if (rc == 0 && dw_sum != nullptr) {
+    if (later.parts > 0) *dw_sum = {later.part, later.n, later.out, later.parts, later.columns};
+    else *dw_sum = {nullptr, 0, nullptr, 0, 0};
+  }
+  return rc;
 }
 
 int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dtype, void* stream) {
@@ -771,6 +789,22 @@ int castle_sum_parts(const float* part, int parts, int64_t n, void* out, int dty
   if (parts <= 0 || n <= 0 || n % 8 != 0 || n / 8 > kMaxRows) return CASTLE_ERR_SHAPE;
   if (part == nullptr || out == nullptr || !aligned16({part, out})) return CASTLE_ERR_ARG;
   return castle::launch_part_sum(part, parts, n, out, dtype, static_cast<hipStream_t>(stream));
+}
+
+int castle_sums(const castle_sum* sums, int count, int dtype, void* stream) {
+  if (elem_size(dtype) == 0) return CASTLE_ERR_DTYPE;
+  static_assert(CASTLE_MAX_SUMS == castle::kMaxSums, "");
+  if (sums == nullptr || count <= 0 || count > CASTLE_MAX_SUMS) return CASTLE_ERR_ARG;
+  castle::PartSum jobs[CASTLE_MAX_SUMS];
+  for (int j = 0; j < count; ++j) {
+    const castle_sum& s = sums[j];
+    if (s.parts <= 0 || s.n <= 0 || s.n / 8 > kMaxRows || (s.columns ? s.n > 0x7ffffff : s.n % 8 != 0)) return CASTLE_ERR_SHAPE;
+    if (s.part == nullptr || s.out == nullptr || (s.columns ? reinterpret_cast<uintptr_t>(s.part) % 4 != 0 || reinterpret_cast<uintptr_t>(s.out) % elem_size(dtype) != 0
+                                                            : !aligned16({s.part, s.out})))
+      return CASTLE_ERR_ARG;
+    jobs[j] = {s.part, s.n, s.out, s.parts, s.columns};
+  }
+  return castle::launch_sums(jobs, count, dtype, static_cast<hipStream_t>(stream));
 }
 
 static int cross_entropy_args(castle::CrossEntropyArgs& a, const void* logits, const int64_t* target, int64_t target_n, int64_t target_ld, int64_t rows,

@@ -43,7 +43,8 @@ int launch_grads32(const GradsArgs& p, int tile, int waves, hipStream_t stream);
 struct GradsPlan { int tile, waves, w_splits, x_splits; };   // tile 0: two launches
 GradsPlan grads_plan(int R, int N, int K, int elem_size, int epilogue, bool amax);
 int64_t grads_workspace(int R, int N, int K, int elem_size, int epilogue, bool amax);   // -1: two launches are ahead
-int launch_grads(GradsArgs p, int dtype, float* workspace, hipStream_t stream);
+struct PartSum;
+int launch_grads(GradsArgs p, int dtype, float* workspace, PartSum* later, hipStream_t stream);   // later: dw's sum is left to launch_sums, if it has one (parts > 0)
 int launch_gemm(GemmArgs a, bool a_kc, bool b_kc, int dtype, float* workspace, hipStream_t stream);
 
 }  // namespace castle

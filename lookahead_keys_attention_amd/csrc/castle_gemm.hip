@@ -825,7 +825,7 @@ int64_t grads_workspace(int R, int N, int K, int elem_size, int epilogue, bool a
   if (g.tile == 0) return -1;
   return ((g.w_splits > 1 ? (int64_t)g.w_splits * N * K : 0) + (g.x_splits > 1 ? (int64_t)g.x_splits * R * K : 0)) * 4;
 }
-int launch_grads(GradsArgs p, int dtype, float* workspace, hipStream_t stream) {
+int launch_grads(GradsArgs p, int dtype, float* workspace, PartSum* later, hipStream_t stream) {
   const int step = dtype == 0 ? 32 : kStep16;
   const GradsPlan g = grads_plan(p.x.M, p.x.K, p.x.N, dtype == 0 ? 4 : 2, p.x.epilogue, p.x.amax != nullptr);
   auto place = [&](GemmArgs& a, int splits, int& groups, int& row) {
@@ -844,8 +844,16 @@ int launch_grads(GradsArgs p, int dtype, float* workspace, hipStream_t stream) {
     else hipLaunchKernelGGL((grads_kernel<T, 1>), dim3(p.w_groups + p.x_groups), dim3(kThreads), 0, stream, p);
     return hipGetLastError() == hipSuccess ? 0 : -3;
   });
-  for (const GemmArgs* a : {&p.w, &p.x})
-    if (rc == 0 && a->part != nullptr) rc = launch_part_sum(a->part, (a->K + a->k_per_split - 1) / a->k_per_split, (int64_t)a->M * a->N, a->c, dtype, stream);
+  PartSum sums[2];
+  int count = 0;
+  if (later != nullptr) later->parts = 0;
+  for (const GemmArgs* a : {&p.w, &p.x}) {
+    if (a->part == nullptr) continue;
+    const PartSum sum = {a->part, (int64_t)a->M * a->N, a->c, (a->K + a->k_per_split - 1) / a->k_per_split, 0};
+    if (a == &p.w && later != nullptr) *later = sum;
+    else sums[count++] = sum;
+  }
+  if (rc == 0 && count > 0) rc = launch_sums(sums, count, dtype, stream);
   return rc;
 }
 

@@ -368,8 +368,30 @@ Normed norm_rows(const Tensor& x_, const Tensor& delta_, const Tensor& w_, std::
   return {sum, h, rstd};
 }
 // dh -> (dres + gradient of the rows, gradient of the weight); rstd as norm_rows left it
+constexpr int64_t kSumsBytes = 64 << 20;
+// Sums of partial weight gradients that wait for the end of a backward pass, for one launch instead of one each (4 us each for a MB or two).
+struct Sums {
+  castle_sum sum[CASTLE_MAX_SUMS];
+  Tensor keep[2 * CASTLE_MAX_SUMS];   // what they read and write
+  int count = 0;
+  int64_t most = 0;   // bytes of partial results that are worth keeping; what is larger is not in a cache any more when it is read
+  bool takes(int64_t parts, int64_t n) const { return parts * n * 4 <= most && count < CASTLE_MAX_SUMS; }
+  void add(const castle_sum& s, const Tensor& part, const Tensor& out) {
+    if (s.parts == 0) return;
+    sum[count] = s;
+    keep[2 * count] = part;
+    keep[2 * count++ + 1] = out;
+  }
+  void flush() {
+    if (count == 0) return;
+    check(castle_sums(sum, count, dtype_code(keep[1]), stream_of(keep[1])), "castle_sums");
+    count = 0;
+    for (Tensor& t : keep) t = Tensor();
+  }
+};
+
 std::tuple<Tensor, Tensor> norm_rows_bwd(const Tensor& dh_, const Tensor& x_, const Tensor& rstd, const Tensor& w_, const Tensor& dres_, bool need_x,
-                                         bool need_w) {
+                                         bool need_w, Sums* sums = nullptr) {
   if (!w_.defined()) return {dres_.defined() ? dres_ + dh_ : dh_, Tensor()};
   const int64_t R = x_.size(0), D = x_.size(1);
   if (rstd.dim() != 1) {
@@ -379,6 +401,14 @@ std::tuple<Tensor, Tensor> norm_rows_bwd(const Tensor& dh_, const Tensor& x_, co
   const Tensor x = row_major(x_), dh = row_major(dh_), w = row_major(w_), dres = need_x && dres_.defined() ? row_major(dres_) : Tensor();
   const int64_t nbytes = need_w ? castle_rms_norm_bwd_workspace_bytes(R, (int)D, dtype_code(x)) : 0;
   Tensor dx = need_x ? at::empty_like(x) : Tensor(), dw = need_w ? at::empty_like(w) : Tensor(), ws = need_w ? bytes(nbytes, x) : Tensor();
+  if (sums != nullptr && need_w && sums->takes(1, nbytes / 4)) {
+    castle_sum sum;
+    check(castle_rms_norm_bwd_parts(dh.data_ptr(), x.data_ptr(), w.data_ptr(), static_cast<const float*>(rstd.data_ptr()), dres.defined() ? dres.data_ptr() : nullptr,
+                                    need_x ? dx.data_ptr() : nullptr, dw.data_ptr(), &sum, R, (int)D, dtype_code(x), ws.data_ptr(), nbytes, stream_of(x)),
+          "castle_rms_norm_bwd_parts");
+    sums->add(sum, ws, dw);
+    return {dx, dw};
+  }
   check(castle_rms_norm_bwd(dh.data_ptr(), x.data_ptr(), w.data_ptr(), static_cast<const float*>(rstd.data_ptr()), dres.defined() ? dres.data_ptr() : nullptr,
                             need_x ? dx.data_ptr() : nullptr, need_w ? dw.data_ptr() : nullptr, R, (int)D, dtype_code(x),
                             need_w ? ws.data_ptr() : nullptr, nbytes, stream_of(x)),
@@ -544,7 +574,7 @@ Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R
 // 6144 x 1024 214 / 187, 200, 231; 12288 x 2048 890 / 931, 884, 1000.
 constexpr int64_t kSplitWgradMinRows = 8192;
 
-Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (N, K)
+Tensor weight_grad(const Tensor& dy, const Tensor& x, Sums* sums = nullptr) {   // (R, N), (R, K) -> (N, K)
   const int64_t rows = x.size(0), N = dy.size(1), K = x.size(1);
   const int64_t tiles = ((N + 255) / 256) * ((K + 255) / 256), parts = tiles >= 192 ? 1 : tiles >= 96 ? 2 : tiles >= 48 ? 4 : 8;
   if (x.scalar_type() != at::kFloat && rows >= kSplitWgradMinRows && rows % parts == 0 && N * K % 8 == 0) {
@@ -553,6 +583,10 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (
     const Tensor a = dy.contiguous().view({parts, r, N}).transpose(1, 2);
     const Tensor part = at::bmm(a, x.contiguous().view({parts, r, K}), at::kFloat).contiguous();
     Tensor dw = at::empty({N, K}, x.options());
+    if (sums != nullptr && sums->takes(parts, N * K)) {
+      sums->add({static_cast<const float*>(part.data_ptr()), N * K, dw.data_ptr(), (int32_t)parts, 0}, part, dw);
+      return dw;
+    }
     check(castle_sum_parts(static_cast<const float*>(part.data_ptr()), (int)parts, N * K, dw.data_ptr(), dtype_code(x), stream_of(x)),
           "castle_sum_parts");
     return dw;
@@ -563,7 +597,7 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x) {   // (R, N), (R, K) -> (
 
 // Both gradients of a projection, in one launch where that is ahead (false: they are left to the functions above).  aux: dx is multiplied by the slope of gelu at
 // it; nbytes >= 0: the maxima of |dx| go to a workspace of that size, `prepared` (16-bit types).
-bool own_projection_grads(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& aux, int64_t nbytes, Tensor& dw, Tensor& dx, Tensor& prepared) {
+bool own_projection_grads(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& aux, int64_t nbytes, Tensor& dw, Tensor& dx, Tensor& prepared, Sums* sums = nullptr) {
   const int64_t R = dy.size(0), N = dy.size(1), K = w.size(1);
   const bool full = dy.scalar_type() == at::kFloat, with_amax = !full && nbytes >= 0;
   if (x.dim() != 2 || x.size(0) != R || x.size(1) != K || w.size(0) != N || x.scalar_type() != dy.scalar_type() || w.scalar_type() != dy.scalar_type() || x.device() != dy.device() ||
@@ -583,9 +617,12 @@ bool own_projection_grads(const Tensor& dy, const Tensor& x, const Tensor& w, co
   const Tensor ws = need ? bytes(need, dy) : Tensor();
   dw = at::empty({N, K}, dy.options());
   dx = at::empty({R, K}, dy.options());
+  castle_sum sum = {};
+  const bool later = sums != nullptr && sums->takes(1, need / 4);
   check(castle_projection_grads(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), dw.data_ptr(), dx.data_ptr(), (int)R, (int)N, (int)K, dtype,
-                                epilogue, aux.defined() ? aux.data_ptr() : nullptr, with_amax ? &where : nullptr, need ? ws.data_ptr() : nullptr, need, stream_of(dy)),
+                                epilogue, aux.defined() ? aux.data_ptr() : nullptr, with_amax ? &where : nullptr, later ? &sum : nullptr, need ? ws.data_ptr() : nullptr, need, stream_of(dy)),
         "castle_projection_grads");
+  if (later) sums->add(sum, ws, dw);
   return true;
 }
 
@@ -725,9 +762,11 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     }
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
     const int64_t flags = ctx->saved_data["flags"].toInt();
+    Sums sums;
+    sums.most = 4 << 20;   // (the attention's backward pass lies between)
     Tensor dmerged, prepared;
-    const bool both = need_out && own_projection_grads(dy, merged2, w_out, Tensor(), bwd_workspace_bytes(shape, flags, state), grads[4], dmerged, prepared);
-    if (need_out && !both) grads[4] = weight_grad(dy, merged2);
+    const bool both = need_out && own_projection_grads(dy, merged2, w_out, Tensor(), bwd_workspace_bytes(shape, flags, state), grads[4], dmerged, prepared, &sums);
+    if (need_out && !both) grads[4] = weight_grad(dy, merged2, &sums);
     if (both) {
     } else if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)))) {
       const Maxima m = maxima(dy, B * L, w_out.size(1), w_out.size(0), 0, w_out.size(1), bwd_workspace_bytes(shape, flags, state), false);
@@ -743,15 +782,17 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(), flags, d6, ws,
             state, prepared);
     const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
+    sums.most = kSumsBytes;
     Tensor dh, none;
-    const bool both_in = need_qkv && (need_x || need_norm) && own_projection_grads(dp2, rows(s[4]), w_qkv, Tensor(), -1, grads[3], dh, none);
-    if (need_qkv && !both_in) grads[3] = weight_grad(dp2, rows(s[4]));
+    const bool both_in = need_qkv && (need_x || need_norm) && own_projection_grads(dp2, rows(s[4]), w_qkv, Tensor(), -1, grads[3], dh, none, &sums);
+    if (need_qkv && !both_in) grads[3] = weight_grad(dp2, rows(s[4]), &sums);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(both_in ? dh : input_grad(dp2, w_qkv), rows(s[0]), rstd, norm_w, rows(dsum), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(both_in ? dh : input_grad(dp2, w_qkv), rows(s[0]), rstd, norm_w, rows(dsum), need_x, need_norm, &sums);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = dx.view({B, L, dx.size(1)});
       if (has_delta) grads[1] = grads[0];
     }
+    sums.flush();
     return grads;
   }
 };
@@ -819,20 +860,23 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const int64_t R = sum.size(0), dim = sum.size(1);
     const Tensor dy = g[0].reshape({R, dim});
     const bool below = need_x || need_norm || need_up, need_down = ctx->needs_input_grad(4);
+    Sums sums;
+    sums.most = kSumsBytes;
     Tensor dup, dh, none;
-    const bool both = below && need_down && own_projection_grads(dy, act, w_down, up, -1, grads[4], dup, none);
-    if (need_down && !both) grads[4] = weight_grad(dy, act);
+    const bool both = below && need_down && own_projection_grads(dy, act, w_down, up, -1, grads[4], dup, none, &sums);
+    if (need_down && !both) grads[4] = weight_grad(dy, act, below ? &sums : nullptr);
     if (!below) return grads;
     if (!both)
       dup = own_product(dy, w_down, R, dim, w_down.size(1), kOwnGeluSlope) ? product(dy, false, w_down, true, CASTLE_GEMM_GELU_SLOPE, up)
                                                                            : at::gelu_backward(at::mm(dy, w_down), up);
-    const bool both_up = need_up && (need_x || need_norm) && own_projection_grads(dup, h, w_up, Tensor(), -1, grads[3], dh, none);
-    if (need_up && !both_up) grads[3] = weight_grad(dup, h);
+    const bool both_up = need_up && (need_x || need_norm) && own_projection_grads(dup, h, w_up, Tensor(), -1, grads[3], dh, none, &sums);
+    if (need_up && !both_up) grads[3] = weight_grad(dup, h, &sums);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(both_up ? dh : input_grad(dup, w_up), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({R, dim}) : Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(both_up ? dh : input_grad(dup, w_up), sum, rstd, norm_w, dsum.defined() ? dsum.reshape({R, dim}) : Tensor(), need_x, need_norm, &sums);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = grads[1] = dx.view(g[0].sizes());
     }
+    sums.flush();
     return grads;
   }
 };
@@ -864,14 +908,17 @@ struct HeadFn : torch::autograd::Function<HeadFn> {
     const Tensor dy = g[0].reshape({sum.size(0), w.size(0)});
     const bool need_x = ctx->needs_input_grad(0) || ctx->needs_input_grad(1), need_norm = ctx->needs_input_grad(2);
     const bool need_w = ctx->needs_input_grad(3);
+    Sums sums;
+    sums.most = kSumsBytes;
     Tensor dh, none;
-    const bool both = need_w && (need_x || need_norm) && own_projection_grads(dy, h, w, Tensor(), -1, grads[3], dh, none);
-    if (need_w && !both) grads[3] = weight_grad(dy, h);
+    const bool both = need_w && (need_x || need_norm) && own_projection_grads(dy, h, w, Tensor(), -1, grads[3], dh, none, &sums);
+    if (need_w && !both) grads[3] = weight_grad(dy, h, &sums);
     if (need_x || need_norm) {
-      auto [dx, dn] = norm_rows_bwd(both ? dh : input_grad(dy, w), sum, rstd, norm_w, Tensor(), need_x, need_norm);
+      auto [dx, dn] = norm_rows_bwd(both ? dh : input_grad(dy, w), sum, rstd, norm_w, Tensor(), need_x, need_norm, &sums);
       if (need_norm) grads[2] = dn;
       if (need_x) grads[0] = grads[1] = dx.view({g[0].size(0), g[0].size(1), sum.size(1)});
     }
+    sums.flush();
     return grads;
   }
 };

@@ -28,7 +28,21 @@ struct NormBwdArgs {
   int D;
 };
 int norm_bwd_groups(int64_t rows, int D, int elem_size);
-int launch_norm_bwd(const NormBwdArgs& a, void* dw, int dtype, hipStream_t stream);
+// out[n] = sum over `parts` rows of part[parts][n]: eight columns a thread (n a multiple of 8), or with `columns` sixteen threads down a column of few
+struct PartSum {
+  const float* part;
+  int64_t n;
+  void* out;
+  int32_t parts, columns;
+};
+constexpr int kMaxSums = 4;
+struct SumsArgs {
+  PartSum job[kMaxSums];
+  int first[kMaxSums];   // workgroup
+};
+int launch_sums(const PartSum* sums, int count, int dtype, hipStream_t stream);
+// later: the sum of the weight's gradient is left to launch_sums
+int launch_norm_bwd(const NormBwdArgs& a, void* dw, int dtype, PartSum* later, hipStream_t stream);
 
 int launch_part_sum(const float* part, int parts, int64_t n, void* out, int dtype, hipStream_t stream);
 

@@ -138,9 +138,9 @@ template <typename T, int LPR, int NP> __global__ __launch_bounds__(kThreads) vo
 }
 
 // out[i] = sum over the G rows of part[G][D]: 16 columns of a workgroup, 16 threads down each of them
-template <typename T> __global__ __launch_bounds__(kThreads) void column_sum_kernel(const float* part, int G, int D, T* out) {
+template <typename T> __device__ __forceinline__ void column_sum(const float* part, int G, int D, T* out, int block) {
   __shared__ float s[16][17];
-  const int c = threadIdx.x % 16, r = threadIdx.x / 16, col = blockIdx.x * 16 + c;
+  const int c = threadIdx.x % 16, r = threadIdx.x / 16, col = block * 16 + c;
   float v = 0.f;
   if (col < D) {
 #pragma unroll 8
@@ -157,8 +157,8 @@ template <typename T> __global__ __launch_bounds__(kThreads) void column_sum_ker
 
 // out[i] = sum over P of part[P][n], n a multiple of 8: the partial products of a weight gradient.  8 parts of 512 x 512 ...
 // 3072 x 512: 6.7 us on average, 14 as a sum and a conversion of their own.
-template <typename T> __global__ __launch_bounds__(kThreads) void part_sum_kernel(const float* part, int P, int64_t n, T* out) {
-  const int64_t i = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 8;
+template <typename T> __device__ __forceinline__ void part_sum(const float* part, int P, int64_t n, T* out, int block) {
+  const int64_t i = ((int64_t)block * kThreads + threadIdx.x) * 8;
   if (i >= n) return;
   typedef vec<float, 4> v4;
   v4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
@@ -171,6 +171,20 @@ template <typename T> __global__ __launch_bounds__(kThreads) void part_sum_kerne
 #pragma unroll
   for (int e = 0; e < 4; ++e) { s[e] = a[e]; s[4 + e] = b[e]; }
   *reinterpret_cast<frag_mem<T>*>(out + i) = __builtin_convertvector(s, frag<T>);
+}
+
+// Several sums, each of the workgroups first[j] .. first[j + 1] - 1.  A sum by itself is a launch of 4 us for 1 to 3 MB, hardly more than its start.
+template <typename T> __global__ __launch_bounds__(kThreads) void sums_kernel(SumsArgs a) {
+  PartSum job = a.job[0];
+  int block = blockIdx.x;
+#pragma unroll
+  for (int j = 1; j < kMaxSums; ++j)
+    if ((int)blockIdx.x >= a.first[j]) {
+      job = a.job[j];
+      block = blockIdx.x - a.first[j];
+    }
+  if (job.columns) column_sum<T>(job.part, job.parts, (int)job.n, static_cast<T*>(job.out), block);
+  else part_sum<T>(job.part, job.parts, job.n, static_cast<T*>(job.out), block);
 }
 
 // Mean cross entropy of rows of logits against class numbers (torch's default ignore_index -100 does not count; a class
@@ -341,7 +355,7 @@ int norm_bwd_groups(int64_t rows, int D, int elem_size) {
   return (int)(g < 1 ? 1 : g > 1024 ? 1024 : g);
 }
 
-int launch_norm_bwd(const NormBwdArgs& a, void* dw, int dtype, hipStream_t stream) {
+int launch_norm_bwd(const NormBwdArgs& a, void* dw, int dtype, PartSum* later, hipStream_t stream) {
   return by_tensor_type(dtype, [&](auto t) {
     using T = decltype(t);
     const int groups = norm_bwd_groups(a.rows, a.D, (int)sizeof(T));
@@ -350,17 +364,31 @@ int launch_norm_bwd(const NormBwdArgs& a, void* dw, int dtype, hipStream_t strea
       return launched();
     });
     if (rc != 0 || a.dw_part == nullptr) return rc;
-    hipLaunchKernelGGL((column_sum_kernel<T>), dim3((a.D + 15) / 16), dim3(kThreads), 0, stream, a.dw_part, groups, a.D, static_cast<T*>(dw));
-    return launched();
+    const PartSum sum = {a.dw_part, a.D, dw, groups, 1};
+    if (later != nullptr) *later = sum;
+    return later != nullptr ? 0 : launch_sums(&sum, 1, dtype, stream);
   });
 }
 
-int launch_part_sum(const float* part, int parts, int64_t n, void* out, int dtype, hipStream_t stream) {
+int launch_sums(const PartSum* sums, int count, int dtype, hipStream_t stream) {
+  SumsArgs a = {};
+  int64_t blocks = 0;
+  for (int j = 0; j < kMaxSums; ++j) {
+    a.first[j] = j < count ? (int)blocks : 0x7fffffff;
+    if (j >= count) continue;
+    a.job[j] = sums[j];
+    const int64_t per = sums[j].columns ? 16 : 8 * kThreads;
+    blocks += (sums[j].n + per - 1) / per;
+    if (blocks > 0x7ffffff0) return -2;
+  }
   return by_tensor_type(dtype, [&](auto t) {
-    using T = decltype(t);
-    hipLaunchKernelGGL((part_sum_kernel<T>), dim3((unsigned)((n / 8 + kThreads - 1) / kThreads)), dim3(kThreads), 0, stream, part, parts, n, static_cast<T*>(out));
+    hipLaunchKernelGGL((sums_kernel<decltype(t)>), dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
     return launched();
   });
+}
+int launch_part_sum(const float* part, int parts, int64_t n, void* out, int dtype, hipStream_t stream) {
+  const PartSum sum = {part, n, out, parts, 0};
+  return launch_sums(&sum, 1, dtype, stream);
 }
 
 int cross_entropy_groups(int64_t rows) {

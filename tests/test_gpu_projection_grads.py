@@ -19,7 +19,7 @@ def entry():
 
     lib, i, i64, vp = N.lib(), ctypes.c_int, ctypes.c_int64, ctypes.c_void_p
     lib.castle_projection_grads_workspace_bytes.restype = i64
-    lib.castle_projection_grads.argtypes = [vp, i64, vp, i64, vp, i64, vp, vp, i, i, i, i, i, vp, vp, vp, i64, vp]
+    lib.castle_projection_grads.argtypes = [vp, i64, vp, i64, vp, i64, vp, vp, i, i, i, i, i, vp, vp, vp, vp, i64, vp]
     return N, lib
 
 
@@ -34,7 +34,7 @@ def run(dy, x, w, aux=None, amax=None):
     dw, dx = (torch.full(s, float("nan"), device=DEV, dtype=dy.dtype) for s in ((n, k), (R, k)))
     ws = torch.empty(max(need, 16), device=DEV, dtype=torch.uint8)
     N.check(lib.castle_projection_grads(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), dw.data_ptr(), dx.data_ptr(), R, n, k, code, slope,
-                                        None if aux is None else aux.data_ptr(), None if amax is None else ctypes.byref(amax), ws.data_ptr(), need,
+                                        None if aux is None else aux.data_ptr(), None if amax is None else ctypes.byref(amax), None, ws.data_ptr(), need,
                                         N.stream_ptr(dy.device)), "castle_projection_grads")
     return dw, dx, tuple(p.value for p in plan)
 
@@ -87,3 +87,23 @@ def test_slope_and_maxima(dtype, R, n, k):
     size = (dy.double().abs() @ w.double().abs()) * 1.13
     assert torch.all((got[1].double() - plain * v.grad).abs() <= 2.02 * ROUND[dtype] * (plain * v.grad).abs() + 2e-6 * plain.abs() + (n + 4) * 2.0 ** -24 * size)
     assert close(got[0], dy.double().t(), x.double(), dtype)
+
+
+class Sum(ctypes.Structure):
+    _fields_ = [("part", ctypes.c_void_p), ("n", ctypes.c_int64), ("out", ctypes.c_void_p), ("parts", ctypes.c_int32), ("columns", ctypes.c_int32)]
+
+
+# (parts, n, columns) of each sum: both kinds, one part and many, less than a workgroup and its edges
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sums", [[(1, 8, 0)], [(5, 2048, 0), (300, 257, 1)], [(3, 2056, 0), (1, 16, 1), (16, 4096, 0), (17, 1000, 1)]])
+def test_several_sums_in_one_launch(dtype, sums):
+    N, lib = entry()
+    g = torch.Generator(device=DEV).manual_seed(len(sums))
+    parts = [torch.randn(p, n, generator=g, device=DEV) for p, n, _ in sums]
+    outs = [torch.full((n,), float("nan"), device=DEV, dtype=dtype) for _, n, _ in sums]
+    jobs = (Sum * len(sums))(*[Sum(a.data_ptr(), n, o.data_ptr(), p, c) for a, o, (p, n, c) in zip(parts, outs, sums)])
+    lib.castle_sums.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    N.check(lib.castle_sums(ctypes.addressof(jobs), len(sums), N.DTYPE_CODES[dtype], N.stream_ptr(torch.device(DEV))), "castle_sums")
+    for a, o in zip(parts, outs):
+        ref = a.double().sum(0)
+        assert torch.all((o.double() - ref).abs() <= ROUND[dtype] * ref.abs() + a.shape[0] * 2.0 ** -24 * a.double().abs().sum(0))
