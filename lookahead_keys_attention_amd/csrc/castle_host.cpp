@@ -572,11 +572,23 @@ Tensor input_grad(const Tensor& dy, const Tensor& w) {   // (R, N), (N, K) -> (R
 // with fp32 partial results, then their sum; same rounding), as many as make about 256 tiles of 256 x 256: 16384 rows,
 // us as one product / with 2, 4, 8 ranges and their sum: 3072 x 512 123 / 80, 64, 63; 2048 x 2048 153 / 137, 139, 161;
 // 6144 x 1024 214 / 187, 200, 231; 12288 x 2048 890 / 931, 884, 1000.
+// Up to 32 GFLOP the framework's own product, which splits the rows by what fills the CUs, is ahead of that: over 2500 of 8192 ... 65536 rows, widths of 64 ... 6144
+// in bf16, partial products and their sum take 1.18 times as long below 1 GFLOP, 1.39 at 1 to 2, 1.55 at 2 to 8, 1.41 at 8 to 16, 1.28 at 16 to 32 (less than 0.97
+// times in 1 of 100 above 1 GFLOP), 1.16 at 32 to 40 with 1 of 13 behind, 1.00 from 64 on.  24000 rows 256 x 256 27.5 / 19.4, 16384 rows 768 x 128 25.1 / 18.8.  Rows that do not split
+// evenly leave the library one product: behind up to what was timed, 130 GFLOP (2.0 times at 40 to 64, 1.6 beyond).
 constexpr int64_t kSplitWgradMinRows = 8192;
+double own_weight_grad(const Tensor& x, int64_t rows, int64_t parts) {
+  return x.scalar_type() == at::kFloat || rows < kSplitWgradMinRows ? kOwnWeightGrad : rows % parts == 0 ? 32e9 : 130e9;
+}
+int64_t wgrad_parts(int64_t N, int64_t K) {
+  const int64_t tiles = ((N + 255) / 256) * ((K + 255) / 256);
+  return tiles >= 192 ? 1 : tiles >= 96 ? 2 : tiles >= 48 ? 4 : 8;
+}
 
 Tensor weight_grad(const Tensor& dy, const Tensor& x, Sums* sums = nullptr) {   // (R, N), (R, K) -> (N, K)
   const int64_t rows = x.size(0), N = dy.size(1), K = x.size(1);
-  const int64_t tiles = ((N + 255) / 256) * ((K + 255) / 256), parts = tiles >= 192 ? 1 : tiles >= 96 ? 2 : tiles >= 48 ? 4 : 8;
+  const int64_t parts = wgrad_parts(N, K);
+  if (own_product(dy, x, rows, N, K, own_weight_grad(x, rows, parts))) return product(dy, true, x, true, CASTLE_GEMM_PLAIN, std::nullopt);
   if (x.scalar_type() != at::kFloat && rows >= kSplitWgradMinRows && rows % parts == 0 && N * K % 8 == 0) {
     if (parts == 1) return at::mm(dy.t(), x);
     const int64_t r = rows / parts;
@@ -591,17 +603,17 @@ Tensor weight_grad(const Tensor& dy, const Tensor& x, Sums* sums = nullptr) {   
           "castle_sum_parts");
     return dw;
   }
-  if (own_product(dy, x, rows, N, K, kOwnWeightGrad)) return product(dy, true, x, true, CASTLE_GEMM_PLAIN, std::nullopt);
   return at::mm(dy.t(), x);
 }
 
+constexpr double kOwnLongGrads = 8e9;   // 16-bit: from kSplitWgradMinRows rows on both in one launch take 1/1.32 of two up to here, more of some from 12 GFLOP on
 // Both gradients of a projection, in one launch where that is ahead (false: they are left to the functions above).  aux: dx is multiplied by the slope of gelu at
 // it; nbytes >= 0: the maxima of |dx| go to a workspace of that size, `prepared` (16-bit types).
 bool own_projection_grads(const Tensor& dy, const Tensor& x, const Tensor& w, const Tensor& aux, int64_t nbytes, Tensor& dw, Tensor& dx, Tensor& prepared, Sums* sums = nullptr) {
   const int64_t R = dy.size(0), N = dy.size(1), K = w.size(1);
   const bool full = dy.scalar_type() == at::kFloat, with_amax = !full && nbytes >= 0;
   if (x.dim() != 2 || x.size(0) != R || x.size(1) != K || w.size(0) != N || x.scalar_type() != dy.scalar_type() || w.scalar_type() != dy.scalar_type() || x.device() != dy.device() ||
-      w.device() != dy.device() || (!full && R >= kSplitWgradMinRows) || !own_product(dy, x, R, N, K, kOwnWeightGrad) ||
+      w.device() != dy.device() || !own_product(dy, x, R, N, K, !full && R >= kSplitWgradMinRows ? kOwnLongGrads : kOwnWeightGrad) ||
       !own_product(dy, w, R, K, N, aux.defined() ? kOwnGeluSlope : own_input_grad(N)))
     return false;
   if (aux.defined() && !(aux.is_contiguous() && aux.dim() == 2 && aux.size(0) == R && aux.size(1) == K && aux.scalar_type() == dy.scalar_type() && aux.device() == dy.device() && aligned16(aux)))
