@@ -571,8 +571,8 @@ int launch_plain_state(const FwdArgs& a, hipStream_t stream) {
 // forward pass left) is also what the backward pass runs first when the forward snapshots were not kept.
 int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
   if (split_fp32(a.s, dtype)) return launch_scan_split(a, stream);
-  if (dtype == 0 || narrow_scan(a.s)) return launch_scan_narrow(a, dtype, bf16_operands, stream);
-  return by_type16(dtype, bf16_operands, [&](auto t, auto ti) {
+  if (narrow_scan(a.s)) return launch_scan_narrow(a, dtype, bf16_operands, stream);
+  return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
     return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_scan_t<T, TI, decltype(hd)::value>(a, stream); });
   });
@@ -587,8 +587,8 @@ int launch_fwd(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stre
   if (rc == 0) rc = launch_scan(a, dtype, bf16_operands, stream);
   if (rc != 0) return rc;
   if (split) return launch_attn_split(a, stream);
-  if (dtype == 0 || narrow_attn(a.s)) return launch_attn_narrow(a, dtype, bf16_operands, stream);
-  return by_type16(dtype, bf16_operands, [&](auto t, auto ti) {
+  if (narrow_attn(a.s)) return launch_attn_narrow(a, dtype, bf16_operands, stream);
+  return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
     return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_attn_t<T, TI, decltype(hd)::value>(a, stream); });
   });

@@ -47,6 +47,13 @@ def test_results_at_tile_edges(B, Hh, L, d):
     check(results(ops, dout, d), reference(ops, dout, d), L)
 
 
+# fewer rows than a tile's worth in so many heads that the scan, and from 513 on the attention, goes by 128 rows a workgroup
+@pytest.mark.parametrize("B,Hh,L,d", [(20, 16, 25, 64), (19, 31, 33, 32), (24, 24, 9, 16), (13, 41, 97, 64)])
+def test_many_heads_of_few_rows(B, Hh, L, d):
+    ops, dout = operands(B, Hh, L, d, seed=L + d)
+    check(results(ops, dout, d), reference(ops, dout, d), max(L, 64))   # (below 64 rows the head dimension has the longest sums)
+
+
 @pytest.mark.parametrize("flag", ["FLAG_RECOMPUTE_SCORES", "FLAG_RECOMPUTE_STATE"])
 def test_results_without_tiles_and_without_snapshots(flag, monkeypatch):
     from lookahead_keys_attention_amd import _native
