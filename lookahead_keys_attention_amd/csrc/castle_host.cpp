@@ -368,7 +368,7 @@ Normed norm_rows(const Tensor& x_, const Tensor& delta_, const Tensor& w_, std::
   return {sum, h, rstd};
 }
 // dh -> (dres + gradient of the rows, gradient of the weight); rstd as norm_rows left it
-constexpr int64_t kSumsBytes = 64 << 20;
+constexpr int64_t kSumsBytes = 4 << 20;
 // Sums of partial weight gradients that wait for the end of a backward pass, for one launch instead of one each (4 us each for a MB or two).
 struct Sums {
   castle_sum sum[CASTLE_MAX_SUMS];
