@@ -778,7 +778,6 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     sums.most = 4 << 20;   // (the attention's backward pass lies between)
     Tensor dmerged, prepared;
     const bool both = need_out && own_projection_grads(dy, merged2, w_out, Tensor(), bwd_workspace_bytes(shape, flags, state), grads[4], dmerged, prepared, &sums);
-    if (need_out && !both) grads[4] = weight_grad(dy, merged2, &sums);
     if (both) {
     } else if (own_product(dy, w_out, B * L, w_out.size(0), w_out.size(1), own_input_grad(w_out.size(0)))) {
       const Maxima m = maxima(dy, B * L, w_out.size(1), w_out.size(0), 0, w_out.size(1), bwd_workspace_bytes(shape, flags, state), false);
@@ -787,6 +786,8 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     } else {
       dmerged = at::mm(dy, w_out);
     }
+    // (behind the product above, whose reads of dy it shares: before it, that one took 22 us instead of 16 for 16384 rows of 512)
+    if (need_out && !both) grads[4] = weight_grad(dy, merged2, &sums);
     Tensor dproj = at::empty({B, L, 6 * merged.size(2)}, merged.options());
     castle_view4 d6[6];
     six_of_packed(dproj, shape, d6);
