@@ -374,8 +374,8 @@ struct Sums {
   castle_sum sum[CASTLE_MAX_SUMS];
   Tensor keep[2 * CASTLE_MAX_SUMS];   // what they read and write
   int count = 0;
-  int64_t most = 0;   // bytes of partial results that are worth keeping; what is larger is not in a cache any more when it is read
-  bool takes(int64_t parts, int64_t n) const { return parts * n * 4 <= most && count < CASTLE_MAX_SUMS; }
+  // what is larger is not in a cache any more when it is read (50 MB behind the input gradient of 16384 rows: 1 to 2 us lost, not won)
+  bool takes(int64_t parts, int64_t n) const { return parts * n * 4 <= kSumsBytes && count < CASTLE_MAX_SUMS; }
   void add(const castle_sum& s, const Tensor& part, const Tensor& out) {
     if (s.parts == 0) return;
     sum[count] = s;
@@ -775,7 +775,6 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     const Shape shape{(int)B, (int)heads, (int)L, (int)(merged.size(2) / heads), dtype_code(merged)};
     const int64_t flags = ctx->saved_data["flags"].toInt();
     Sums sums;
-    sums.most = 4 << 20;   // (the attention's backward pass lies between)
     Tensor dmerged, prepared;
     const bool both = need_out && own_projection_grads(dy, merged2, w_out, Tensor(), bwd_workspace_bytes(shape, flags, state), grads[4], dmerged, prepared, &sums);
     if (both) {
@@ -795,7 +794,6 @@ struct LayerFn : torch::autograd::Function<LayerFn> {
     run_bwd(d6, packed_view(merged, shape, 1, 0), packed_view(dmerged, shape, 1, 0), shape, ctx->saved_data["scale"].toDouble(), flags, d6, ws,
             state, prepared);
     const Tensor dp2 = dproj.view({B * L, dproj.size(2)});
-    sums.most = kSumsBytes;
     Tensor dh, none;
     const bool both_in = need_qkv && (need_x || need_norm) && own_projection_grads(dp2, rows(s[4]), w_qkv, Tensor(), -1, grads[3], dh, none, &sums);
     if (need_qkv && !both_in) grads[3] = weight_grad(dp2, rows(s[4]), &sums);
@@ -874,7 +872,6 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
     const Tensor dy = g[0].reshape({R, dim});
     const bool below = need_x || need_norm || need_up, need_down = ctx->needs_input_grad(4);
     Sums sums;
-    sums.most = kSumsBytes;
     Tensor dup, dh, none;
     const bool both = below && need_down && own_projection_grads(dy, act, w_down, up, -1, grads[4], dup, none, &sums);
     if (need_down && !both) grads[4] = weight_grad(dy, act, below ? &sums : nullptr);
@@ -922,7 +919,6 @@ struct HeadFn : torch::autograd::Function<HeadFn> {
     const bool need_x = ctx->needs_input_grad(0) || ctx->needs_input_grad(1), need_norm = ctx->needs_input_grad(2);
     const bool need_w = ctx->needs_input_grad(3);
     Sums sums;
-    sums.most = kSumsBytes;
     Tensor dh, none;
     const bool both = need_w && (need_x || need_norm) && own_projection_grads(dy, h, w, Tensor(), -1, grads[3], dh, none, &sums);
     if (need_w && !both) grads[3] = weight_grad(dy, h, &sums);
