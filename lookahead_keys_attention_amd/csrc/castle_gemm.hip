@@ -317,6 +317,8 @@ __global__ __launch_bounds__(kThreads * G, BM == 128 ? 2 : 4) void gemm_kernel(G
 }
 // Both gradients of a projection, which read the same dy and nothing of each other, in one launch: workgroups of the weight gradient
 // (w.k_per_split rows of the contraction each), then those of the input gradient.
+// Each by itself is bound by its start, trips to memory and CUs that stay idle; together they fill them (3000 rows 256 -> 1536, us: 16.8 and 11.4, both 19.0; the rule and
+// more figures at grads_plan).  Tiles of 64 x 64 for both, by one or two groups: larger ones do not leave a CU room for a workgroup of the other.
 template <typename T, int G> __global__ __launch_bounds__(kThreads * G, 4) void grads_kernel(GradsArgs p) {
   constexpr int kElems = max2(tile_elems<T, false, false, 64, 64, kStep16, G>(), tile_elems<T, true, false, 64, 64, kStep16, G>());
   __shared__ __attribute__((aligned(16))) T smem[kElems];

@@ -345,7 +345,8 @@ __global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void gemm32_kernel(G
   __shared__ __attribute__((aligned(16))) vec<float, 4> s_sum[W * wave_bytes<TILE>() / 16];
   gemm32_tile<AK, BKC, TILE, W, NORM>(a, s_sum, blockIdx.x, blockIdx.y);
 }
-// both gradients of a projection: workgroups of the weight gradient, then those of the input gradient
+// both gradients of a projection: workgroups of the weight gradient, then those of the input gradient (castle_gemm.hip; 256 rows 512 -> 3072, us: 12.9 and 16.1, both
+// 24.6, 512 -> 512 5.6 and 6.5, both 8.4)
 template <int TILE, int W> __global__ __launch_bounds__(64 * W, W / 4 < 2 ? 2 : W / 4) void grads32_kernel(GradsArgs p) {
   __shared__ __attribute__((aligned(16))) vec<float, 4> s_sum[W * wave_bytes<TILE>() / 16];
   int b = blockIdx.x;
