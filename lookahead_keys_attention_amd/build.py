@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libcastle_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
-SOURCES = ("castle_fwd.hip", "castle_bwd.hip", "castle_narrow.hip", "castle_narrow_bwd.hip", "castle_narrow32.hip", "castle_short.hip", "castle_decode.hip", "castle_rows.hip", "castle_gemm.hip", "castle_gemm32.hip", "castle_profile.hip", "castle_abi.hip")
+SOURCES = ("castle_fwd.hip", "castle_bwd.hip", "castle_narrow.hip", "castle_narrow_bwd.hip", "castle_short.hip", "castle_decode.hip", "castle_rows.hip", "castle_gemm.hip", "castle_gemm32.hip", "castle_profile.hip", "castle_abi.hip")
 HOST_SOURCE = "castle_host.cpp"
 HOST_NAME = "_castle_host.so"
 ARCH = "gfx950"
@@ -29,10 +29,10 @@ HIPCC_FLAGS = (
     "-Wno-unused-command-line-argument",
 )
 # Kernels of one wave per SIMD have 256 accumulation registers beside the vector registers, and the compiler then lets every matrix
-# instruction write there, which costs a copy for each register that a vector instruction reads (a quarter of what the fp32 backward
-# kernels issued).  With this the results lie in vector registers and the other file takes what does not fit.
+# instruction write there, which costs a copy for each register that a vector instruction reads.  With this the results lie in vector
+# registers and the other file takes what does not fit.
 VECTOR_RESULTS = ("-mllvm", "-amdgpu-mfma-vgpr-form=1")
-SOURCE_FLAGS = {"castle_narrow32.hip": VECTOR_RESULTS, "castle_narrow.hip": VECTOR_RESULTS}
+SOURCE_FLAGS = {"castle_narrow.hip": VECTOR_RESULTS}
 
 
 def _hipcc() -> str:

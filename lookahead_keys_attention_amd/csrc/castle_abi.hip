@@ -12,13 +12,11 @@
 #include "castle_profile.h"
 #include "castle_rows.h"
 #include "castle_tiles.h"
-#include "castle_narrow.h"
 
 namespace castle {
 int launch_fwd(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_short(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
-int launch_plain_state(const FwdArgs& a, hipStream_t stream);
 int launch_bwd(const BwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream);
 int launch_decode(const DecodeArgs& a, int dtype, hipStream_t stream);
 int launch_decode_flush(const DecodeArgs& a, int dtype, hipStream_t stream);
@@ -83,9 +81,7 @@ int64_t max_score_tile_bytes() {
 struct Geometry {
   int Lp, nblk;
   int64_t lse_bytes, tblk_bytes, snap_bytes, mat_bytes, op_bytes;
-  int64_t off_lse, off_t, off_tt, off_ttx, off_ops, off_op_mul, off_t_mul, total;
-  int64_t snap_mul, do_mul_bytes, ds_mul_bytes;   // fp32: where the multipliers of snapshots begin, sizes of others
-  bool plain_state;   // fp32 without room for the tiles: the backward pass makes unsplit copies, T' blocks and snapshots of its own
+  int64_t off_lse, off_t, off_tt, off_ttx, off_ops, total;
   int64_t bwd_total;
 };
 constexpr int64_t kHeaderBytes = 256 + 4 * castle::kAmaxBlocks;   // header + partial maxima, forward and backward alike
@@ -97,8 +93,7 @@ Geometry geometry(int B, int H, int L, int d, int es, int flags = 0) {
   const int64_t BH = (int64_t)B * H;
   g.lse_bytes = align_up(BH * g.Lp * 4, 256);
   g.tblk_bytes = align_up(BH * g.Lp * kNB * es, 256);
-  g.snap_mul = align_up(BH * castle::snap_rows(g.nblk) * d * es, 256);
-  g.snap_bytes = g.snap_mul + (es == 4 ? align_up(BH * g.nblk * (g.Lp / 32) * 4, 256) : 0);
+  g.snap_bytes = align_up(BH * castle::snap_rows(g.nblk) * d * es, 256);
   // dS / dSu tiles between the two backward kernels
   g.mat_bytes = align_up(BH * g.Lp * g.Lp * es, 256);
   // too long, or the caller asks for it: the query kernel recomputes the scores instead
@@ -109,15 +104,10 @@ Geometry geometry(int B, int H, int L, int d, int es, int flags = 0) {
   g.off_ttx = g.off_tt + g.tblk_bytes;
   g.op_bytes = align_up(BH * g.Lp * d * es, 256);   // one operand in the compute type, padded to Lp rows
   g.off_ops = g.off_ttx + g.tblk_bytes;
-  g.off_op_mul = g.off_ops + 6 * g.op_bytes;
-  g.do_mul_bytes = es == 4 ? align_up(BH * (g.Lp / 32) * 4, 256) : 0;
-  g.off_t_mul = g.off_op_mul + 6 * g.do_mul_bytes;
-  g.total = g.off_t_mul + (es == 4 ? align_up(BH * g.nblk * 4, 256) : 0);   // the snapshots live in their own buffer (g.snap_bytes)
-  g.ds_mul_bytes = es == 4 && g.mat_bytes != 0 ? align_up(BH * (g.Lp / 32) * (g.Lp / 32) * 4, 256) : 0;
-  g.plain_state = es == 4 && g.mat_bytes == 0 && L >= castle::kSplitMinRows;
+  g.total = g.off_ops + 6 * g.op_bytes;            // the snapshots live in their own buffer (g.snap_bytes)
   // header, reverse-state snapshots, delta, dO copy, dS / dSu tiles, and the forward snapshots when they are recomputed
-  g.bwd_total = kHeaderBytes + g.snap_bytes + g.lse_bytes + g.op_bytes + 2 * g.mat_bytes + g.do_mul_bytes + g.ds_mul_bytes +
-                (g.plain_state ? g.total : 0) + (g.plain_state || (flags & CASTLE_FLAG_RECOMPUTE_STATE) ? g.snap_bytes : 0);
+  g.bwd_total = kHeaderBytes + g.snap_bytes + g.lse_bytes + g.op_bytes + 2 * g.mat_bytes +
+                ((flags & CASTLE_FLAG_RECOMPUTE_STATE) ? g.snap_bytes : 0);
   return g;
 }
 
@@ -166,9 +156,6 @@ castle::FwdWorkspace carve(void* base, void* state, const Geometry& g) {
   w.qu_p = p + g.off_ops + 3 * g.op_bytes;
   w.ku_p = p + g.off_ops + 4 * g.op_bytes;
   w.vu_p = p + g.off_ops + 5 * g.op_bytes;
-  w.op_mul = reinterpret_cast<float*>(p + g.off_op_mul);
-  w.t_mul = reinterpret_cast<float*>(p + g.off_t_mul);
-  w.u_mul = reinterpret_cast<float*>(static_cast<char*>(state) + g.snap_mul);
   return w;
 }
 
@@ -288,7 +275,7 @@ int castle_bwd(const castle_view4* qc, const castle_view4* kc, const castle_view
   a.dqu = to_view(dqu); a.dku = to_view(dku); a.dvu = to_view(dvu);
   char* bw = static_cast<char*>(bwd_workspace);
   // forward snapshots: the caller's, or recomputed into the tail of this call's own workspace
-  void* state = recompute_state || g.plain_state ? bw + (g.bwd_total - g.snap_bytes) : const_cast<void*>(fwd_state);
+  void* state = recompute_state ? bw + (g.bwd_total - g.snap_bytes) : const_cast<void*>(fwd_state);
   a.ws = carve(const_cast<void*>(fwd_workspace), state, g);
   a.bhdr = reinterpret_cast<castle::BwdHeader*>(bw);
   a.amax_part = reinterpret_cast<float*>(bw + 256);
@@ -299,25 +286,12 @@ int castle_bwd(const castle_view4* qc, const castle_view4* kc, const castle_view
   a.dout_p = bw + g.snap_bytes + g.lse_bytes;
   a.ds_mat = g.mat_bytes ? bw + g.snap_bytes + g.lse_bytes + g.op_bytes : nullptr;
   a.dsu_mat = g.mat_bytes ? bw + g.snap_bytes + g.lse_bytes + g.op_bytes + g.mat_bytes : nullptr;
-  bw += g.snap_bytes + g.lse_bytes + g.op_bytes + 2 * g.mat_bytes;
-  a.g_mul = reinterpret_cast<float*>(static_cast<char*>(a.gsnap) + g.snap_mul);
-  a.do_mul = reinterpret_cast<float*>(bw);
-  a.ds_mul = reinterpret_cast<float*>(bw + g.do_mul_bytes);
-  if (recompute_state || g.plain_state) {   // the scan again, from the operand copies the forward pass left
+  if (recompute_state) {   // the scan again, from the operand copies the forward pass left
     castle::FwdArgs f;
     f.s = a.s;
     f.qc = a.qc; f.kc = a.kc; f.vc = a.vc; f.qu = a.qu; f.ku = a.ku; f.vu = a.vu;
     f.out = a.out;
     f.U = to_view(nullptr);
-    if (g.plain_state) {   // ... or from copies of its own; of the forward pass only the normalisers are read
-      const float* lse = a.ws.lse;
-      a.ws = carve(bw + g.do_mul_bytes + g.ds_mul_bytes, state, g);
-      f.ws = a.ws;
-      rc = castle::launch_plain_state(f, static_cast<hipStream_t>(stream));
-      if (rc != 0) return rc;
-      a.ws.lse = const_cast<float*>(lse);
-      return castle::launch_bwd(a, dtype, false, static_cast<hipStream_t>(stream));
-    }
     f.ws = a.ws;
     f.with_t = 0;
     rc = castle::launch_scan(f, dtype, (flags & CASTLE_FLAG_BF16_OPERANDS) != 0, static_cast<hipStream_t>(stream));

@@ -2427,7 +2427,6 @@ template <typename T, typename TI, int HD> static int launch_bwd_t(const BwdArgs
 // bf16 tensors use fp16 MFMA operands unless bf16_operands is set (must match the forward pass,
 // whose workspace holds operands in the compute type)
 int launch_bwd(const BwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
-  if (a.ds_mat != nullptr && split_fp32(a.s, dtype)) return launch_bwd_split(a, stream);
   const bool narrow = a.ds_mat != nullptr && narrow_bwd(a.s, dtype);
   const int rc = by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);

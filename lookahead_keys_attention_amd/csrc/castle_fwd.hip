@@ -559,18 +559,9 @@ template <typename T, typename TI, int HD> static int launch_attn_t(const FwdArg
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-// What the backward kernels of fp32 tensors without dS / dSu tiles work on: operand copies, T' blocks and snapshots in fp32
-int launch_plain_state(const FwdArgs& a, hipStream_t stream) {
-  return by_head_dim<float>(a.s.d, [&](auto hd) {
-    const int rc = launch_prep_t<float, float, decltype(hd)::value>(a, stream);
-    return rc != 0 ? rc : launch_scan_t<float, float, decltype(hd)::value>(a, stream);
-  });
-}
-
 // The scan alone (snapshots of the lookahead state into a.ws.usnap from the operand copies the
 // forward pass left) is also what the backward pass runs first when the forward snapshots were not kept.
 int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
-  if (split_fp32(a.s, dtype)) return launch_scan_split(a, stream);
   if (narrow_scan(a.s)) return launch_scan_narrow(a, dtype, bf16_operands, stream);
   return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
@@ -579,14 +570,12 @@ int launch_scan(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t str
 }
 
 int launch_fwd(const FwdArgs& a, int dtype, bool bf16_operands, hipStream_t stream) {
-  const bool split = split_fp32(a.s, dtype);
-  int rc = split ? launch_prep_split(a, stream) : by_type(dtype, bf16_operands, [&](auto t, auto ti) {
+  int rc = by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);
     return by_head_dim<T>(a.s.d, [&](auto hd) { return launch_prep_t<T, TI, decltype(hd)::value>(a, stream); });
   });
   if (rc == 0) rc = launch_scan(a, dtype, bf16_operands, stream);
   if (rc != 0) return rc;
-  if (split) return launch_attn_split(a, stream);
   if (narrow_attn(a.s)) return launch_attn_narrow(a, dtype, bf16_operands, stream);
   return by_type(dtype, bf16_operands, [&](auto t, auto ti) {
     using T = decltype(t); using TI = decltype(ti);

@@ -8,8 +8,9 @@
 // (no barriers), and the partial results meet once at the end, in fp32 through LDS.  Every operand tile is copied as whole
 // lines into LDS that belongs to one wave, while the tile before it is worked on; the rows of the workgroup itself are
 // in LDS once, for all waves.  What bounds them is the wait for those tiles, two waves per SIMD at most (one at d = 128 and
-// fp32): 8 x 4 heads of 777 rows at d = 32 in fp16 269 -> 116 us (operator forward and backward with the host path; the kernels took 193
-// of it and take 136 with the small kernels around them).  fp32 tensors run here below 128 rows only (see split_fp32).
+// fp32), and for fp32 the matrix instructions: operator forward and backward at 2 x 8 heads of 1024 rows 1426 -> 431 us
+// in fp32; 8 x 4 heads of 777 rows at d = 32 in fp16 269 -> 116 us (with the host path measured; the kernels took 193
+// of it and take 136 with the small kernels around them).
 //
 //   scan_narrow    32 keys; the waves split the source blocks: every wave sums its own part first, then sweeps it
 //                  again from the sum of the parts before it, storing the snapshots (two gates per pair instead

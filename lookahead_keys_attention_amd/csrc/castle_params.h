@@ -49,10 +49,6 @@ struct FwdWorkspace {
   // (written by the prep kernel; every other kernel reads these instead of the caller's tensors).
   // qc_p is pre-multiplied by scale * log2(e).
   void *qc_p, *kc_p, *vc_p, *qu_p, *ku_p, *vu_p;
-  // fp32 tensors: copies, T' blocks and snapshots hold pairs of fp16 numbers in tiles of 32 rows (castle_split.h).  What they are to be multiplied with:
-  float* op_mul;   // [6][B*H][Lp/32] the copies, in the order qc, kc, vc, qu, ku, vu
-  float* t_mul;    // [B*H][nblk] T' and its transpose
-  float* u_mul;    // [B*H][nblk][Lp/32] the snapshot tile of a block and 32 keys (behind the snapshots)
 };
 
 struct FwdArgs {
@@ -83,10 +79,6 @@ struct BwdArgs {
   void* dout_p;   // [B*H][Lp][d]  dO in the compute type, rows >= L zero (written by the delta kernel)
   void* ds_mat;   // dS
   void* dsu_mat;  // dSu
-  // fp32 tensors with tiles: dO copy, reverse states and tiles are pairs of fp16 numbers too
-  float* do_mul;  // [B*H][Lp/32]
-  float* g_mul;   // [B*H][nblk][Lp/32] (behind the reverse states)
-  float* ds_mul;  // [B*H][Lp/32][Lp/32] dS and dSu of a key and a query tile
 };
 
 // Half-precision cache format of the lookahead keys, for bf16 caches: the U buffer holds IEEE fp16

@@ -104,14 +104,10 @@ def _fake_state(B, H, L, d, like, keep_state):
 
 def state_bytes_formula(B, H, L, d, element_size) -> int:
     """castle_fwd_state_bytes in plain Python (64-row blocks over L rounded up to 128; one snapshot row
-    of d elements per key and later block, fp32 also a multiplier per block and 32 keys), for callers that
-    a tracing compiler looks into."""
+    of d elements per key and later block), for callers that a tracing compiler looks into."""
     nblk = (L + 127) // 128 * 2
     n = B * H * 64 * (nblk * (nblk - 1) // 2) * d * element_size
-    n = (n + 255) // 256 * 256
-    if element_size == 4:
-        n += (B * H * nblk * 2 * nblk * 4 + 255) // 256 * 256
-    return max(256, n)
+    return max(256, (n + 255) // 256 * 256)
 
 
 def keeps_state(B, H, L, d, dtype) -> bool:
