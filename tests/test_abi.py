@@ -55,6 +55,11 @@ def test_workspace_sizes(lib):
     assert lib.castle_bwd_workspace_bytes(4, 8, 4096, 64, 1, 0) == bwd
     assert lib.castle_bwd_workspace_bytes(4, 8, 4096, 64, 1, N.FLAG_RECOMPUTE_STATE) == bwd + snaps
     assert lib.castle_bwd_workspace_bytes(4, 8, 4096, 64, 1, N.FLAG_RECOMPUTE_SCORES) == bwd - 2 * BH * Lp * Lp * 2
+    # fp32 asks for nothing else, with and without its score tiles
+    bwd32 = header + 2 * snaps + BH * Lp * 4 + BH * Lp * 64 * 4
+    assert lib.castle_fwd_workspace_bytes(4, 8, 4096, 64, 0) == header + BH * Lp * 4 + 3 * BH * Lp * 64 * 4 + 6 * BH * Lp * 64 * 4
+    assert lib.castle_bwd_workspace_bytes(4, 8, 4096, 64, 0, 0) == bwd32 + 2 * BH * Lp * Lp * 4
+    assert lib.castle_bwd_workspace_bytes(4, 8, 4096, 64, 0, N.FLAG_RECOMPUTE_SCORES) == bwd32
     # ragged L rounds up to 128 rows
     assert lib.castle_fwd_workspace_bytes(1, 1, 129, 64, 0) == lib.castle_fwd_workspace_bytes(1, 1, 256, 64, 0)
     assert lib.castle_decode_workspace_bytes(32, 8, 64, 4096) > 0
