@@ -35,6 +35,17 @@ def test_header_symbols_are_exported(lib):
         assert hasattr(raw, name), f"{name} missing from libcastle_hip.so"
 
 
+def test_every_native_source_is_built():
+    """Nothing lies beside the sources that the build does not read."""
+    from lookahead_keys_attention_amd import build as B
+
+    files = set(os.listdir(B.CSRC))
+    headers = {f for f in files if f.endswith(".h")}
+    assert files - headers == {*B.SOURCES, B.HOST_SOURCE}
+    text = "".join(open(os.path.join(B.CSRC, f)).read() for f in files)
+    assert headers <= set(re.findall(r'#include "([^"/]+)"', text))
+
+
 def test_version_and_error_strings(lib):
     assert lib.castle_abi_version() == 5
     assert lib.castle_error_string(0) == b"ok"
