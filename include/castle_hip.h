@@ -72,7 +72,8 @@ extern "C" {
 #define CASTLE_FLAG_STEP_TAKE_OVER 128
 #define CASTLE_FLAG_STEP_GIVE_UP 256
 /* castle_fwd: no castle_bwd follows.  What lies in the workspace behind the status word and in the state is then undefined, and short sequences (up to
- * 128 rows of 16-bit types, as long as there are few of them) take one launch. */
+ * 128 rows of 16-bit types, as long as there are few of them) take one launch, whose roundings fall in other places: out and U are as exact as without the
+ * flag, not the same bits.  castle_bwd refuses it (CASTLE_ERR_ARG). */
 #define CASTLE_FLAG_FORWARD_ONLY 512
 #define CASTLE_AMAX_PARTIALS 256
 #define CASTLE_AMAX_OFFSET 256

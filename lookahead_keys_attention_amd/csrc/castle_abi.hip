@@ -253,6 +253,7 @@ int castle_bwd(const castle_view4* qc, const castle_view4* kc, const castle_view
   const castle_view4* in[] = {qc, kc, vc, qu, ku, vu, out, dout, dqc, dkc, dvc, dqu, dku, dvu};
   for (const castle_view4* v : in)
     if (!view_ok(v, es, true)) return CASTLE_ERR_ARG;
+  if (flags & CASTLE_FLAG_FORWARD_ONLY) return CASTLE_ERR_ARG;
   const Geometry g = geometry(B, H, L, d, es, flags);
   if (fwd_workspace == nullptr || reinterpret_cast<uintptr_t>(fwd_workspace) % 256 != 0 || fwd_workspace_bytes < g.total)
     return CASTLE_ERR_WORKSPACE;

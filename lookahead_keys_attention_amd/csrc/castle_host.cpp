@@ -206,7 +206,8 @@ Tensor attention_packed_bwd(const Tensor& proj, const Tensor& merged, const Tens
 // ---- autograd ----------------------------------------------------------------------------------------------------
 // U, the workspace and the state carry no gradient (lookahead_keys_attention_triton.py:513-515 for U), and
 // autograd does not materialise zeros for them (a fill of hundreds of MB per backward pass).  The formulas call
-// the backward operators through the dispatcher, so that they trace like any other operator.
+// the backward operators through the dispatcher, so that they trace like any other operator.  A graph that was traced without
+// gradients carries CASTLE_FLAG_FORWARD_ONLY in its arguments: where it runs with gradients, the flag is dropped.
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
@@ -250,6 +251,7 @@ struct AttentionFn : torch::autograd::Function<AttentionFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& qu,
                                const Tensor& ku, const Tensor& vu, double scale, bool want_U, int64_t flags, bool keep_state) {
     static const auto op = op_handle<decltype(attention)>("castle_hip::attention");
+    flags &= ~CASTLE_FLAG_FORWARD_ONLY;
     const at::AutoDispatchBelowADInplaceOrView below;
     auto [out, U, ws, state] = op.call(q, k, v, qu, ku, vu, scale, want_U, flags, keep_state);
     ctx->save_for_backward({q, k, v, qu, ku, vu, out, ws, state});
@@ -294,6 +296,7 @@ struct AttentionPackedFn : torch::autograd::Function<AttentionPackedFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& proj, int64_t heads, double scale, bool want_U, int64_t row_capacity,
                                int64_t flags, bool keep_state) {
     static const auto op = op_handle<decltype(attention_packed)>("castle_hip::attention_packed");
+    flags &= ~CASTLE_FLAG_FORWARD_ONLY;
     const at::AutoDispatchBelowADInplaceOrView below;
     auto [merged, U, ws, state] = op.call(proj, heads, scale, want_U, row_capacity, flags, keep_state);
     ctx->save_for_backward({proj, merged, ws, state});

@@ -110,6 +110,12 @@ def test_null_and_misaligned_views_are_rejected_on_the_host(lib):
     assert lib.castle_fwd(*a, *b) == -4
 
 
+def test_no_backward_pass_behind_a_forward_pass_by_itself(lib):
+    ok = N.View4(4096, 64, 64, 64)
+    for flags, code in ((N.FLAG_FORWARD_ONLY, -5), (0, -4)):   # (no workspace)
+        assert lib.castle_bwd(*[ok] * 8, 1, 1, 16, 64, 1, 0.125, flags, *[ok] * 6, None, 0, None, 0, None, 0, None) == code
+
+
 def test_small_linear_and_static_step_validate_on_the_host(lib):
     assert lib.castle_small_linear(4096, 4096, 4096, 4, 64, 30, 64, 64, 64, 1, None) == -2     # K % 8
     assert lib.castle_small_linear(4096, 4096, 4096, 4, 64, 32, 64, 64, 64, 0, None) == -1     # fp32 not offered

@@ -88,6 +88,38 @@ def test_forward_mode_derivatives_raise():
                     call()
 
 
+def test_a_graph_traced_without_gradients_can_be_differentiated():
+    """Flags are arguments: a graph that was traced under no_grad asks for a forward pass by itself wherever it runs.  One whose
+    backward pass is recorded must leave what that reads."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from lookahead_keys_attention_amd import _native as N
+
+    seen = []
+
+    class Record(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func.namespace == "castle_hip":
+                index = [a.name for a in func._schema.arguments].index("flags")
+                seen.append((func._opname, args[index]))
+            return func(*args, **(kwargs or {}))
+
+    with FakeTensorMode():
+        six = [torch.empty(1, 2, 40, 32, dtype=torch.bfloat16) for _ in range(6)]
+        proj = torch.empty(1, 40, 6 * 2 * 32, dtype=torch.bfloat16)
+        with torch.no_grad():
+            graphs = [(make_fx(lambda *t: ops.castle_attention_hip(*t, 0.1, rotary=True))(*six), six),
+                      (make_fx(lambda t: ops.castle_attention_packed(t, 2, 0.1, rotary=True))(proj), [proj])]
+        for graph, inputs in graphs:
+            with Record():
+                with torch.no_grad():
+                    graph(*inputs)
+                graph(*[t.requires_grad_() for t in inputs]).sum().backward()
+            assert [flags for _, flags in seen] == [N.FLAG_ROTARY | N.FLAG_FORWARD_ONLY, N.FLAG_ROTARY, N.FLAG_ROTARY], seen
+            seen.clear()
+
+
 def test_frozen_weights_cost_no_gradient_of_theirs():
     """The traced norm and projections form the gradients that are asked for, as the modules do."""
     from torch.utils._python_dispatch import TorchDispatchMode
