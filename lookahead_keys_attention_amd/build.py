@@ -30,7 +30,7 @@ HIPCC_FLAGS = (
 )
 # Kernels of one wave per SIMD have 256 accumulation registers beside the vector registers, and the compiler then lets every matrix
 # instruction write there, which costs a copy for each register that a vector instruction reads.  With this the results lie in vector
-# registers and the other file takes what does not fit.
+# registers and the other file takes what does not fit.  An internal option of the compiler: one that does not know it builds without.
 VECTOR_RESULTS = ("-mllvm", "-amdgpu-mfma-vgpr-form=1")
 SOURCE_FLAGS = {"castle_narrow.hip": VECTOR_RESULTS}
 
@@ -69,11 +69,18 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
 
     def compile_one(src):
         obj = os.path.join(objdir, os.path.splitext(src)[0] + ".o")
-        cmd = _host_compiler() if src == HOST_SOURCE else [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, ())]
+        cmd = _host_compiler() if src == HOST_SOURCE else [hipcc, *HIPCC_FLAGS]
         cmd = [*cmd, "-c", os.path.join(CSRC, src), "-o", obj]
+        extra = SOURCE_FLAGS.get(src, ())
         if verbose:
-            print(" ".join(cmd), flush=True)
-        _run(cmd)
+            print(" ".join((*cmd, *extra)), flush=True)
+        try:
+            _run([*cmd, *extra])
+        except RuntimeError as e:
+            if not extra or "Unknown command line argument" not in str(e):
+                raise
+            print(f"{src}: the compiler does not know {' '.join(extra)}, compiled without", file=sys.stderr, flush=True)
+            _run(cmd)
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as pool:

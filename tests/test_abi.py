@@ -46,6 +46,29 @@ def test_every_native_source_is_built():
     assert headers <= set(re.findall(r'#include "([^"/]+)"', text))
 
 
+@pytest.mark.parametrize("complaint, again", [("clang (LLVM option parsing): Unknown command line argument '{}'.", True), ("error: no such thing as {}", False)])
+def test_a_compiler_without_an_internal_option_builds_all_the_same(monkeypatch, complaint, again):
+    from lookahead_keys_attention_amd import build as B
+
+    option, commands = B.VECTOR_RESULTS[1], []
+
+    def run(cmd):
+        commands.append(cmd)
+        if option in cmd:
+            raise RuntimeError(complaint.format(option))
+        return ""
+
+    monkeypatch.setattr(B, "_run", run)
+    if not again:
+        with pytest.raises(RuntimeError):
+            B.build(jobs=1)
+        return
+    B.build(jobs=1)
+    for src in (*B.SOURCES, B.HOST_SOURCE):
+        tried = [c for c in commands if os.path.join(B.CSRC, src) in c]
+        assert option not in tried[-1] and len(tried) == 1 + (src in B.SOURCE_FLAGS)
+
+
 def test_version_and_error_strings(lib):
     assert lib.castle_abi_version() == 5
     assert lib.castle_error_string(0) == b"ok"
