@@ -40,6 +40,24 @@ def test_forward_without_a_graph(B, Hh, L, d, rotary, dtype):
         assert err <= 1.2 * allowed + 2.0 ** -(9 if dtype == torch.bfloat16 else 12), (err, allowed)
 
 
+# up to two tiles of 32 rows at any number of heads; beyond, up to 768 workgroups; the rows of four tiles do not fit into LDS at d = 128
+@pytest.mark.parametrize("B,Hh,L,d,one", [(1, 2, 1, 64, True), (1, 2, 33, 16, True), (2, 1, 65, 64, True), (1, 2, 96, 128, True), (1, 2, 97, 128, False), (5, 7, 128, 64, True),
+                                          (1, 2, 129, 64, False), (3, 64, 128, 16, True), (193, 1, 128, 16, False), (1, 256, 96, 32, True), (1, 257, 96, 32, False), (1, 800, 64, 16, True)])
+def test_which_calls_take_one_launch(B, Hh, L, d, one):
+    from lookahead_keys_attention_amd import _native as N
+
+    ops = [torch.zeros(B, Hh, L, d, device=DEV, dtype=torch.bfloat16) for _ in range(6)]
+    for records, want in ((False, ["attn"] if one else ["prep", "scan", "attn"]), (True, ["prep", "scan", "attn"])):
+        N.profile_enable(True)
+        try:
+            with torch.set_grad_enabled(records):
+                H().castle_attention_hip(*ops, d ** -0.5)
+            kernels = [name for name, _ in N.profile_read()]
+        finally:
+            N.profile_enable(False)
+        assert kernels == want, (records, kernels)
+
+
 @pytest.mark.parametrize("half", [False, True])
 def test_strided_operands_and_cache_rows(half):
     """The packed projection, and lookahead keys as the first rows of a cache buffer in either format."""
