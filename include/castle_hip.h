@@ -346,7 +346,7 @@ int castle_rms_norm_bwd_parts(const void* dh, const void* x, const void* weight,
  * derivative of gelu at aux; aux has c's shape and leading dimension.  A workspace of castle_gemm_workspace_bytes
  * (0 when the contraction is not split; then ldc may exceed N).  An operand of `rows` stored rows whose elements are further
  * than 2^31 from its start is refused (CASTLE_ERR_SHAPE): castle_gemm_operand_ok, 1 or 0.  fp32: an element goes to the 16-bit matrix instructions as three
- * bf16 numbers, which hold all of it (below 2^-110 up to 2^-133); infinities and NaNs come out as fp32 instructions would have them. */
+ * bf16 numbers, which hold all of it; where sums are below 2^-90, infinite or NaN the fp32 instruction forms them. */
 #define CASTLE_GEMM_PLAIN 0
 #define CASTLE_GEMM_GELU 1
 #define CASTLE_GEMM_GELU_SLOPE 2

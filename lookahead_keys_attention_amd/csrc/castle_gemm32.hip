@@ -4,7 +4,9 @@
 //   ac' + ca' + bb' + ab' + ba' + aa'
 // with fp32 sums: 192 cycles for a tile of 32 x 32 and 16 steps of the contraction, where the fp32 instruction takes 512 and rounds its sums four times as
 // often.  What is left out, bc' + cb' + cc', is below 2^-23 of a product, of either sign.  Infinities, NaNs and what bf16 rounds to infinity do not go by parts; they
-// leave no finite sum, and a wave that finds such a one goes over its steps again with the fp32 instruction.
+// leave no finite sum, and a wave that finds such a one goes over its steps again with the fp32 instruction.  So it does where a sum is below 2^-90 and not zero: of an
+// element below 2^-110, c is below what bf16 holds, 2^-133, an error of up to 2^-134.  In a sum of 2^-90 or more that is below 2^-24 of it, as long as the other operand's
+// elements add up to no more than 2^20.
 //
 // A workgroup has a tile of 64 x 64 or 32 x 32 of the output, and its waves take the contraction in turns, 32 steps each: every wave meets the whole tile, so an
 // element is converted once for it, six matrix instructions follow on two to four operands, and the operands go through LDS that belongs to the wave, with no barrier
@@ -129,6 +131,7 @@ template <bool KC, int F> struct Operand32 {   // F: 32 or 64
 
 // sums of a wave in LDS: pieces of 16 bytes from one quad of accumulator registers to the next, such that the readers' pieces of a row meet all banks
 constexpr int kUnit32 = 66;
+constexpr uint32_t kLeastBits = (127u - 90) << 23;   // 2^-90
 template <int TILE> constexpr int wave_bytes() { return max2(TILE * TILE / 256 * kUnit32 * 16, 2 * TILE * kStep * 4); }
 // NORM: the rows of `a` are normalised on their way to the registers.
 template <bool AK, bool BKC, int TILE, int W, bool NORM>
@@ -277,12 +280,21 @@ __device__ __forceinline__ void gemm32_tile(const GemmArgs& a, vec<float, 4>* s_
   };
   products(std::true_type());
   float most = 0.f;
-  bool finite = true;
+  // the place of |sum| above kLeast; smaller ones are beyond infinity
+  auto above = [&](bool zeros_count) __attribute__((always_inline)) {
+    uint32_t far = 0;
 #pragma unroll
-  for (int i = 0; i < F * F; ++i)
+    for (int i = 0; i < F * F; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) finite &= fabsf(acc[i / F][i % F][r]) < INFINITY;
-  if (__builtin_amdgcn_ballot_w64(!finite) != 0) {
+      for (int r = 0; r < 16; ++r) {
+        const float x = acc[i / F][i % F][r];   // (the bits of an element of a vector are taken from a copy: from the element itself they are the first one's)
+        const uint32_t w = 2 * __builtin_bit_cast(uint32_t, x);
+        far = max(far, (!zeros_count && w == 0 ? 2 * kLeastBits : w) - 2 * kLeastBits);
+      }
+    return far >= 2 * (0x7f800000u - kLeastBits);
+  };
+  // (zeros, of rows of zeros for instance, are looked at by themselves: that costs another instruction for each sum)
+  if (__builtin_amdgcn_ballot_w64(above(true)) != 0 && __builtin_amdgcn_ballot_w64(above(false)) != 0) {
     fetch(wave);
     products(std::false_type());
   }

@@ -58,3 +58,18 @@ def test_infinities_nans_and_the_ends_of_the_range(M, N, K):
         assert torch.all(got[over] == torch.sign(want[over]).float() * float("inf"))
         size = a.double().abs() @ b.double().abs().t()
         assert torch.all(((got.double() - want).abs() <= (K + 4) * 2.0 ** -24 * size)[finite])
+
+
+@pytest.mark.parametrize("M,N,K", [(72, 136, 40), (256, 512, 512), (4104, 1024, 264)])
+@pytest.mark.parametrize("power", [-105, -112, -118])
+def test_elements_near_the_smallest_normal_number(M, N, K, power):
+    """Rows of either operand whose third part, 2^-16 of an element, would be below what bf16 holds."""
+    g = torch.Generator(device=DEV).manual_seed(N)
+    a, b = (torch.randn(*s, generator=g, device=DEV) for s in ((M, K), (N, K)))
+    a[5:40] *= 2.0 ** power
+    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    for operands in layouts(a, b) + [(b, False, a, False)]:
+        got, ref, s = product(*operands, 0, None).double(), want, size
+        if operands[0] is b:
+            ref, s = want.t(), size.t()
+        assert torch.all((got - ref).abs() <= (K + 4) * 2.0 ** -24 * s + K * 2.0 ** -149)
